@@ -185,6 +185,52 @@ int ixh_gemm(const IxhPacked *packed, const int32_t *prefix, const uint16_t *x, 
 size_t ixh_gemm_workspace_bytes(const IxhPacked *packed, int32_t m);
 
 /*
+ * The lane layout: a second device form of a packed tensor for the products of few activation rows, made once when a
+ * layer is deployed.  The reference has no counterpart; it holds exactly the integers of the packed tensor, each at a
+ * fixed place and `bits` wide (3, 4, 5 or 8), in the order in which the lanes of the kernels multiply them, with the
+ * values that do not fit in a list (csrc/ixh_lanes.h has the layout).  Buffers are the caller's:
+ *   plane    plane_words = ixh_lanes_plane_words(out_f, in_f, bits) 32-bit words, 16-byte aligned
+ *   exc_off  ixh_lanes_cells(out_f, in_f) + 1 entries: first quad of listed elements of every cell (4 rows x 512 columns)
+ *   exc_pos, exc_val  4 * n_quads entries each, the elements with |value| > 2^(bits-1) - 1; n_quads: the cells' quads
+ *            together, rounded up to a multiple of 64, at least 64 (the rest zero: whole groups are read)
+ */
+typedef struct IxhLanes {
+    int32_t bits;
+    int64_t out_f;
+    int64_t in_f;
+    const uint32_t *plane;
+    uint64_t plane_words;
+    const uint32_t *exc_off;
+    const uint16_t *exc_pos;
+    const int8_t *exc_val;
+    uint64_t n_quads;
+    const uint16_t *scale;
+} IxhLanes;
+
+int64_t ixh_lanes_plane_words(int64_t out_f, int64_t in_f, int32_t bits);
+int64_t ixh_lanes_cells(int64_t out_f, int64_t in_f);
+
+/*
+ * Writing it, from the bf16 weights that ixh_decode makes of the packed tensor (out_f x in_f, dense; the integers come
+ * back exactly).  ixh_lanes_pack writes the plane and the number of quads of every cell to `counts` (ixh_lanes_cells
+ * entries); the caller turns those into exc_off (an exclusive running sum, the total behind the last), zeroes the list
+ * and ixh_lanes_list fills it in.  In both, `dst` names the buffers (written despite the const of its
+ * fields; ixh_lanes_pack uses plane and scale only).
+ */
+int ixh_lanes_pack(const uint16_t *w, const IxhLanes *dst, uint32_t *counts, ixh_stream_t stream);
+int ixh_lanes_list(const uint16_t *w, const IxhLanes *dst, ixh_stream_t stream);
+
+/*
+ * y[j, r] = bf16( sum_k f32(x[j, k]) * f32(w[r, k]) ) [ + bias[r], the sum rounded to bf16 again ], 1 <= m <= 16, as
+ * ixh_gemv computes it from the packed tensor.  bias may be NULL.  Partial sums go to `workspace`
+ * (ixh_lanes_gemv_workspace_bytes, may be 0).  Returns IXH_EUNSUPPORTED where the activations do not fit the kernels.
+ */
+int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
+                   int64_t ldy, void *workspace, size_t workspace_bytes, ixh_stream_t stream);
+
+size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m);
+
+/*
  * The encoder on the device, in two calls because the stream lengths depend on the data.
  * Together they replace int8x_quantize (ixrun/quantize.py:41-122, with pack_bits_stream
  * and pack_bitmap of ixrun/bitpack.py:13-61, :87-89) for a bf16 weight that is already in

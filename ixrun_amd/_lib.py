@@ -44,6 +44,21 @@ class IxhPacked(C.Structure):
     ]
 
 
+class IxhLanes(C.Structure):
+    _fields_ = [
+        ("bits", C.c_int32),
+        ("out_f", C.c_int64),
+        ("in_f", C.c_int64),
+        ("plane", C.c_void_p),
+        ("plane_words", C.c_uint64),
+        ("exc_off", C.c_void_p),
+        ("exc_pos", C.c_void_p),
+        ("exc_val", C.c_void_p),
+        ("n_quads", C.c_uint64),
+        ("scale", C.c_void_p),
+    ]
+
+
 class IxhError(RuntimeError):
     """A call into libixhip returned a negative code."""
 
@@ -59,6 +74,8 @@ EXPORTS = (
     "ixh_version", "ixh_last_error", "ixh_prefix_entries", "ixh_prefix_build", "ixh_decode",
     "ixh_gemv", "ixh_gemv_workspace_bytes", "ixh_gemv_noalloc", "ixh_gemm", "ixh_gemm_workspace_bytes",
     "ixh_encode_workspace_bytes", "ixh_encode_scan", "ixh_encode_pack", "ixh_decode_gs",
+    "ixh_lanes_plane_words", "ixh_lanes_cells", "ixh_lanes_pack", "ixh_lanes_list", "ixh_lanes_gemv",
+    "ixh_lanes_gemv_workspace_bytes",
 )
 TEST_EXPORTS = ("ixh_set_option",)
 
@@ -114,6 +131,19 @@ def lib() -> C.CDLL:
         ]
         L.ixh_encode_pack.restype = C.c_int
         L.ixh_encode_pack.argtypes = [C.c_void_p, C.POINTER(IxhPacked), C.c_void_p, C.c_void_p]
+        L.ixh_lanes_plane_words.restype = C.c_int64
+        L.ixh_lanes_plane_words.argtypes = [C.c_int64, C.c_int64, C.c_int32]
+        L.ixh_lanes_cells.restype = C.c_int64
+        L.ixh_lanes_cells.argtypes = [C.c_int64, C.c_int64]
+        L.ixh_lanes_pack.restype = C.c_int
+        L.ixh_lanes_pack.argtypes = [C.c_void_p, C.POINTER(IxhLanes), C.c_void_p, C.c_void_p]
+        L.ixh_lanes_list.restype = C.c_int
+        L.ixh_lanes_list.argtypes = [C.c_void_p, C.POINTER(IxhLanes), C.c_void_p]
+        L.ixh_lanes_gemv.restype = C.c_int
+        L.ixh_lanes_gemv.argtypes = [C.POINTER(IxhLanes), C.c_void_p, C.c_int64, C.c_void_p, C.c_int32, C.c_void_p,
+                                     C.c_int64, C.c_void_p, C.c_size_t, C.c_void_p]
+        L.ixh_lanes_gemv_workspace_bytes.restype = C.c_size_t
+        L.ixh_lanes_gemv_workspace_bytes.argtypes = [C.POINTER(IxhLanes), C.c_int32]
         _lib = L
     return _lib
 
@@ -319,6 +349,67 @@ class DevicePacked:
             workspace.data_ptr() if workspace is not None else None,
             workspace.numel() * workspace.element_size() if workspace is not None else 0,
             current_stream(self.device)))
+
+
+LANE_BITS = (3, 4, 5, 8)
+
+
+def lane_bits(level_bits, counts) -> int:
+    """The width of the lane layout that makes a tensor smallest: a listed element takes three bytes and a fifth more for
+    the uneven rows of its quads.  Their number follows from the level counts, for the widths the scheme has a level of."""
+    n = max(sum(counts), 1)
+    costs = [(b * n + 29 * sum(counts[i + 1:]), b) for i, b in enumerate(level_bits) if b in LANE_BITS]
+    return min(costs)[1]
+
+
+class LanePacked:
+    """The lane layout (``IxhLanes``) of a packed tensor, over device tensors that it keeps alive:
+    ``tensors`` = plane, first quads of the cells, positions and values of the listed elements."""
+
+    def __init__(self, out_f, in_f, tensors, scale):
+        for t in tensors:
+            _require_cuda(t, "lane layout")
+        L = lib()
+        self.tensors, self.scale = list(tensors), scale
+        plane, exc_off, exc_pos, exc_val = tensors
+        self.bits = plane.numel() // int(L.ixh_lanes_plane_words(out_f, in_f, 8) // 8)
+        if exc_off.numel() != L.ixh_lanes_cells(out_f, in_f) + 1 or exc_pos.numel() != exc_val.numel():
+            raise ValueError("the lane layout's tensors do not fit together")
+        self.struct = IxhLanes(self.bits, out_f, in_f, plane.data_ptr(), plane.numel(), exc_off.data_ptr(), exc_pos.data_ptr(),
+                               exc_val.data_ptr(), exc_pos.numel() // 4, scale.data_ptr())
+
+    @staticmethod
+    def estimate(dp: DevicePacked, counts):
+        """Bytes the layout of a packed tensor takes, to within the unevenness of its rows; None where it has none."""
+        bits = lane_bits(dp.level_bits, counts)
+        words = lib().ixh_lanes_plane_words(dp.out_f, dp.in_f, bits)
+        return None if words < 0 else 4 * words + 4 * sum(c for b, c in zip(dp.level_bits, counts) if b > bits)
+
+    @classmethod
+    def build(cls, dp: DevicePacked, table: torch.Tensor, unit: int, counts) -> "LanePacked":
+        """Lay out a packed tensor (through its bf16 weights; one synchronisation, for the length of the list)."""
+        dev, L = dp.device, lib()
+        words, cells = L.ixh_lanes_plane_words(dp.out_f, dp.in_f, lane_bits(dp.level_bits, counts)), L.ixh_lanes_cells(dp.out_f, dp.in_f)
+        with torch.cuda.device(dev):
+            w = torch.empty(dp.N, dtype=torch.bfloat16, device=dev)
+            dp.decode(table, unit, out_bf16=w)
+            plane = torch.empty(words, dtype=torch.int32, device=dev)
+            exc_off = torch.zeros(cells + 1, dtype=torch.int32, device=dev)
+            quads = torch.empty(cells, dtype=torch.int32, device=dev)
+            none = torch.zeros(256, dtype=torch.int16, device=dev)
+            stream = current_stream(dev)
+            first = cls(dp.out_f, dp.in_f, (plane, exc_off, none, none.to(torch.int8)), dp.tensors[-1])
+            check(L.ixh_lanes_pack(w.data_ptr(), C.byref(first.struct), quads.data_ptr(), stream))
+            torch.cumsum(quads, 0, dtype=torch.int32, out=exc_off[1:])
+            n_quads = max(-(-int(exc_off[-1]) // 64), 1) * 64
+            exc_pos = torch.zeros(4 * n_quads, dtype=torch.int16, device=dev)
+            exc_val = torch.zeros(4 * n_quads, dtype=torch.int8, device=dev)
+            whole = cls(dp.out_f, dp.in_f, (plane, exc_off, exc_pos, exc_val), dp.tensors[-1])
+            check(L.ixh_lanes_list(w.data_ptr(), C.byref(whole.struct), stream))
+        return whole
+
+    def gemv_workspace_bytes(self, m: int) -> int:
+        return int(lib().ixh_lanes_gemv_workspace_bytes(C.byref(self.struct), int(m)))
 
 
 def encode_device(weight: torch.Tensor, level_bits) -> tuple:

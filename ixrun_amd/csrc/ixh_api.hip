@@ -10,6 +10,7 @@
 #include "../../include/ixhip_test.h"
 #include "ixh_dev.h"
 #include "ixh_fast358.h"
+#include "ixh_lanes.h"
 #include "ixh_prefill358.h"
 
 namespace ixh {
@@ -492,6 +493,90 @@ int ixh_gemm(const IxhPacked *packed, const int32_t *prefix, const uint16_t *x, 
     else
         rc = launch_prefill(d, prefix, x, (uint32_t)m, ldx, y, ldy, (float *)workspace, (hipStream_t)stream);
     if (rc == IXH_ELAUNCH) set_error("gemm: launch failed");
+    return rc;
+}
+
+// ---- the lane layout ----
+static bool lanes_shape(int64_t out_f, int64_t in_f, uint64_t *tiles, uint64_t *cells) {
+    if (out_f <= 0 || in_f <= 0) return false;
+    *tiles = ((uint64_t)out_f + 3u) / 4u;
+    *cells = ((uint64_t)in_f + kLnCols - 1u) / kLnCols;
+    return *tiles * *cells < (1ull << 31) / kLnCell;  // flat indexes and cell * 2048 stay below 2^31
+}
+
+int64_t ixh_lanes_plane_words(int64_t out_f, int64_t in_f, int32_t bits) {
+    uint64_t t, c;
+    if (!lanes_shape(out_f, in_f, &t, &c) || (bits != 3 && bits != 4 && bits != 5 && bits != 8)) return -1;
+    return (int64_t)(t * c * 64u * (uint32_t)bits);
+}
+
+int64_t ixh_lanes_cells(int64_t out_f, int64_t in_f) {
+    uint64_t t, c;
+    return lanes_shape(out_f, in_f, &t, &c) ? (int64_t)(t * c) : -1;
+}
+
+static int to_lanes(const IxhLanes *p, LanesDev *out, bool whole) {
+    if (!p) { set_error("lanes is NULL"); return IXH_EINVAL; }
+    const int64_t words = ixh_lanes_plane_words(p->out_f, p->in_f, p->bits);
+    if (words < 0) {
+        set_error("lanes: %lld x %lld at %d bits is no lane layout", (long long)p->out_f, (long long)p->in_f, p->bits);
+        return IXH_EINVAL;
+    }
+    if (!p->plane || p->plane_words < (uint64_t)words || ((uintptr_t)p->plane & 15u)) {
+        set_error("lanes: the plane needs %lld words, 16-byte aligned", (long long)words);
+        return IXH_EINVAL;
+    }
+    if (!p->scale || (whole && !p->exc_off) || (whole && (!p->exc_pos || !p->exc_val || p->n_quads < 64))) {
+        set_error("lanes: scale, exc_off or the list is NULL, or the list holds fewer than 64 quads");
+        return IXH_EINVAL;
+    }
+    *out = LanesDev{p->plane, p->exc_off, p->exc_pos, p->exc_val, p->scale, (uint32_t)p->out_f, (uint32_t)p->in_f,
+                    (uint32_t)((p->out_f + 3) / 4), (uint32_t)((p->in_f + kLnCols - 1) / kLnCols), p->bits};
+    return IXH_OK;
+}
+
+int ixh_lanes_pack(const uint16_t *w, const IxhLanes *dst, uint32_t *counts, ixh_stream_t stream) {
+    LanesDev d;
+    int rc = to_lanes(dst, &d, false);
+    if (rc) return rc;
+    if (!w || !counts) { set_error("lanes_pack: w or counts is NULL"); return IXH_EINVAL; }
+    rc = launch_lanes_pack(w, d, const_cast<uint32_t *>(d.plane), counts, (hipStream_t)stream);
+    if (rc == IXH_ELAUNCH) set_error("lanes_pack: launch failed");
+    return rc;
+}
+
+int ixh_lanes_list(const uint16_t *w, const IxhLanes *dst, ixh_stream_t stream) {
+    LanesDev d;
+    int rc = to_lanes(dst, &d, true);
+    if (rc) return rc;
+    if (!w) { set_error("lanes_list: w is NULL"); return IXH_EINVAL; }
+    rc = launch_lanes_list(w, d, const_cast<uint16_t *>(d.exc_pos), const_cast<int8_t *>(d.exc_val), (hipStream_t)stream);
+    if (rc == IXH_ELAUNCH) set_error("lanes_list: launch failed");
+    return rc;
+}
+
+size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m) {
+    LanesDev d;
+    if (to_lanes(lanes, &d, true) || m < 1 || m > 16) return 0;
+    return lanes_gemv_workspace_bytes(d, m);
+}
+
+int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
+                   int64_t ldy, void *workspace, size_t workspace_bytes, ixh_stream_t stream) {
+    LanesDev d;
+    int rc = to_lanes(lanes, &d, true);
+    if (rc) return rc;
+    if (m < 1 || m > 16) { set_error("m = %d not in 1..16", m); return IXH_EINVAL; }
+    if (!x || !y) { set_error("x or y is NULL"); return IXH_EINVAL; }
+    if (m > 1 && (ldx < (int64_t)d.in_f || ldy < (int64_t)d.out_f)) { set_error("ldx or ldy shorter than a row"); return IXH_EINVAL; }
+    const size_t need = lanes_gemv_workspace_bytes(d, m);
+    if (need && (!workspace || workspace_bytes < need)) {
+        set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
+        return IXH_EWORKSPACE;
+    }
+    rc = launch_lanes_gemv(d, x, m, ldx, bias, y, ldy, (float *)workspace, (hipStream_t)stream);
+    if (rc == IXH_ELAUNCH) set_error("lanes_gemv: launch failed");
+    if (rc == IXH_EUNSUPPORTED) set_error("lanes_gemv: %d activation rows of %u do not fit", m, d.in_f);
     return rc;
 }
 

@@ -1,0 +1,849 @@
+// Products of few activation rows with weights in the lane layout (ixh_lanes.h), and the kernels that write it.
+#include "ixh_lanes.h"
+
+#include "ixh_fast358.h"
+
+namespace ixh {
+
+typedef uint32_t ln_u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t ln_u32x3 __attribute__((ext_vector_type(3)));
+typedef uint32_t ln_u32x2 __attribute__((ext_vector_type(2)));
+typedef short ln_s16x4 __attribute__((ext_vector_type(4)));
+typedef float ln_f32x4 __attribute__((ext_vector_type(4)));
+typedef float ln_f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 ln_bf16x2 __attribute__((ext_vector_type(2)));
+
+constexpr size_t kLnLds = 160 * 1024;
+
+#define LN_LDS(T) __attribute__((address_space(3))) T
+
+__device__ __forceinline__ uint32_t ln_pack(float lo, float hi) {
+    const ln_f32x2 v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, ln_bf16x2));
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// Pair tables.  A table of dequantised pairs (both weights as bf16) indexed by the 2 * BITS bits of a pair, in
+// 2^kCopies copies side by side so that the lanes of a wave, which read unrelated entries, spread over the banks.
+// A vector shift and an AND take half the issue time of a bit-field extract, a conversion or a packed operation
+// (measured: 2 against 4 clocks a wave instruction), so a pair costs 6 clocks of issue and one LDS read where
+// arithmetic (extract, convert, multiply, round) takes about 20.
+// ---------------------------------------------------------------------------------------------------------------
+template <int BITS, bool WIDE = true> struct LnPairs {
+    // log2: 32 copies of 64 entries never collide; 8 of 1024 leave about half of the collisions (5120 x 17408, 5 bits, one
+    // row: 21.9 us with one copy, 21.1 with eight).  The tile kernel has no LDS to spare for more than two.
+    static constexpr int kCopies = BITS == 3 ? 5 : WIDE ? (BITS == 4 ? 4 : 3) : 1;
+    static constexpr uint32_t kEntries = BITS == 8 ? 0u : 1u << (2 * BITS);
+    static constexpr uint32_t kLutBytes = kEntries << (kCopies + 2);
+    static constexpr uint32_t kMask = ((1u << (2 * BITS)) - 1u) << (kCopies + 2);
+};
+
+template <int BITS, bool WIDE>
+__device__ __forceinline__ void ln_build_lut(uint32_t lut, float scale, uint32_t tid, uint32_t n_threads) {
+    using P = LnPairs<BITS, WIDE>;
+    if constexpr (P::kEntries != 0) {
+        constexpr int T = (1 << (BITS - 1)) - 1;
+        constexpr uint32_t RUN = P::kCopies >= 2 ? 4u : 2u;  // copies a thread stores at a time
+        for (uint32_t e = tid * RUN; e < (P::kEntries << P::kCopies); e += n_threads * RUN) {
+            const uint32_t idx = e >> P::kCopies;
+            const uint32_t v = ln_pack((float)((int)(idx & ((1u << BITS) - 1u)) - T) * scale, (float)((int)(idx >> BITS) - T) * scale);
+            if constexpr (RUN == 4) *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(lut + e * 4u)) = ln_u32x4{v, v, v, v};
+            else *reinterpret_cast<LN_LDS(ln_u32x2) *>((uintptr_t)(lut + e * 4u)) = ln_u32x2{v, v};
+        }
+    }
+}
+
+template <int SH> __device__ __forceinline__ uint32_t ln_shift(uint32_t w) {
+    if constexpr (SH >= 0) return w >> SH;
+    else return w << -SH;
+}
+
+// the sixteen dequantised pairs of a lane's `BITS` dwords
+template <int BITS, bool WIDE>
+__device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lut_lane, float scale, uint32_t (&o)[16]) {
+    using P = LnPairs<BITS, WIDE>;
+    if constexpr (BITS == 8) {
+        // (c - 127) * scale as c * scale - 127 * scale: both products and the difference are exact in fp32
+        const float off = -127.0f * scale;
+#pragma unroll
+        for (int p = 0; p < 16; ++p) {
+            const uint32_t d = w[p >> 1] >> (16 * (p & 1));
+            o[p] = ln_pack(__fmaf_rn((float)(d & 255u), scale, off), __fmaf_rn((float)((d >> 8) & 255u), scale, off));
+        }
+    } else {
+        constexpr int PER = BITS == 4 ? 4 : BITS == 3 ? 5 : 3;  // whole pairs a dword
+        constexpr int FIRST = BITS == 4 ? 0 : 2;
+        constexpr int TO = P::kCopies + 2;
+        uint32_t a[16];
+#define LN_FIELD(d, f) (ln_shift<FIRST + 2 * BITS * (f) - TO>(w[d]) & P::kMask)
+#pragma unroll
+        for (int d = 0; d < BITS; ++d) {
+            a[PER * d] = LN_FIELD(d, 0);
+            a[PER * d + 1] = LN_FIELD(d, 1);
+            a[PER * d + 2] = LN_FIELD(d, 2);
+            if constexpr (PER > 3) a[PER * d + 3] = LN_FIELD(d, 3);
+            if constexpr (PER > 4) a[PER * d + 4] = LN_FIELD(d, 4);
+        }
+#undef LN_FIELD
+        if constexpr (BITS == 3 || BITS == 5) {
+            uint32_t last = 0;
+#pragma unroll
+            for (int d = 0; d < BITS; ++d) last |= (w[d] & 3u) << (TO + 2 * d);
+            a[15] = last;
+        }
+        if constexpr (BITS == 5) {
+            // The last whole pair of a dword by arithmetic, which evens out the LDS and the vector unit: the code next to
+            // the exponent of 1.0 reads as 1 + code / 32, and (1 + code / 32) * 32 scale - 47 scale is value * scale,
+            // every term exact in fp32.
+            const float s32 = 32.0f * scale, off = -47.0f * scale;
+#pragma unroll
+            for (int d = 0; d < 5; ++d) {
+                const float lo = __uint_as_float(((w[d] >> 4) & 0x7C0000u) | 0x3F800000u);
+                const float hi = __uint_as_float(((w[d] >> 9) & 0x7C0000u) | 0x3F800000u);
+                o[PER * d + 2] = ln_pack(__fmaf_rn(lo, s32, off), __fmaf_rn(hi, s32, off));
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < 16; ++p)
+            if (BITS != 5 || p == 15 || p % 3 != 2)
+                o[p] = *reinterpret_cast<const LN_LDS(uint32_t) *>((uintptr_t)(a[p] + lut_lane));
+    }
+}
+
+template <int BITS>
+__device__ __forceinline__ void ln_load_lane(const uint32_t *__restrict__ p, uint32_t lane, uint32_t (&w)[BITS]) {
+    if constexpr (BITS == 3) {
+        const ln_u32x3 v = *reinterpret_cast<const ln_u32x3 *>(p + lane * 3u);
+        w[0] = v[0]; w[1] = v[1]; w[2] = v[2];
+    } else {
+        const ln_u32x4 v = *reinterpret_cast<const ln_u32x4 *>(p + lane * 4u);
+        w[0] = v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
+        if constexpr (BITS == 5) w[4] = p[256u + lane];
+        if constexpr (BITS == 8) {
+            const ln_u32x4 u = *reinterpret_cast<const ln_u32x4 *>(p + 256u + lane * 4u);
+            w[4] = u[0]; w[5] = u[1]; w[6] = u[2]; w[7] = u[3];
+        }
+    }
+}
+
+template <int BITS>
+__device__ __forceinline__ void ln_load(const uint32_t *__restrict__ plane, uint32_t cell, uint32_t lane, uint32_t (&w)[BITS]) {
+    ln_load_lane<BITS>(plane + (size_t)cell * (64u * BITS), lane, w);
+}
+
+template <int CTRL> __device__ __forceinline__ float ln_dpp(float v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// k_lanes_gemv<BITS, MT>: up to MT activation rows, MT = 1, 2 or 4.
+//
+// Bound: HBM.  A workgroup owns whole row quads, so each output is made in one place (no workspace, no second
+// launch).  Its cells, in memory order, are dealt to its waves in contiguous shares; a wave keeps several cells of
+// loads in flight, whose addresses depend on nothing that is loaded.  The activations are copied to LDS once per
+// workgroup, 16-byte pieces of a 512-column cell at piece ^ (q << 2) so that the sixteen slices of a wave read from
+// different banks.  Products: v_mfma_f32_4x4x4_16b_bf16, one of its sixteen 4 x 4 blocks per slice (weight row = lane
+// % 4, activation row = lane % 4), so a weight costs no product instructions of its own.
+//
+// Listed elements lie in cell order, so those of a share are one run of quads.  They are taken 64 quads at a time, one
+// such group with every cell from the share's first on, fetched as far ahead as the cells: value times gathered
+// activation, added to the lane's sum of the row.
+// ---------------------------------------------------------------------------------------------------------------
+constexpr uint32_t kLnAhead = 4;
+constexpr uint32_t kLnXAhead = 3;  // 16-byte pieces of the activations a thread asks for before anything else
+
+template <int BITS, int MT>
+__global__ void __launch_bounds__(1024)
+k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
+             const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t all_tiles, uint32_t tiles_per_wg, uint32_t in_f,
+             const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, int m, int64_t ldx,
+             const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, uint32_t out_f, bool x_aligned) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t ln_smem[];
+    const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)ln_smem;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, n_threads = blockDim.x, n_waves = n_threads >> 6;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t t0 = blockIdx.x * tiles_per_wg, C = n_cells;
+    const uint32_t n_tiles = min(tiles_per_wg, all_tiles - t0);
+    const uint32_t n_seq = n_tiles * C, cell0 = t0 * C;
+    const uint32_t s0 = wave * n_seq / n_waves, s1 = (wave + 1) * n_seq / n_waves;
+    const uint32_t x_at = smem + LnPairs<BITS>::kLutBytes, x_row = C * 1024u, x_pieces = MT * C * 64u;
+    float *const parts = reinterpret_cast<float *>(ln_smem + LnPairs<BITS>::kLutBytes + MT * x_row);
+
+    auto x_piece = [&](uint32_t e) {
+        const uint32_t r = MT == 1 ? 0u : e / (C * 64u), col = (e - r * (C * 64u)) * 8u;
+        ln_u32x4 v = {0u, 0u, 0u, 0u};
+        if (r < (uint32_t)m && col < in_f) {
+            const uint16_t *src = x + (int64_t)r * ldx + col;
+            if (x_aligned && col + 8u <= in_f) {
+                v = *reinterpret_cast<const ln_u32x4 *>(src);
+            } else {
+                uint32_t h[8];
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k) h[k] = col + k < in_f ? src[k] : 0u;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = h[2 * k] | (h[2 * k + 1] << 16);
+            }
+        }
+        return v;
+    };
+    auto x_store = [&](uint32_t e, ln_u32x4 v) {
+        const uint32_t r = MT == 1 ? 0u : e / (C * 64u), piece = e - r * (C * 64u);
+        *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + r * x_row + lane_offset(piece * 8u))) = v;
+    };
+
+    // ---- everything that depends on nothing is asked for: activations, the first cells, the list's extent ----
+    // (Requests are never inside a branch: past the end they repeat the last cell, group or piece.  The compiler counts
+    // requests in flight, and one that may or may not have been made turns its counted waits into waits for all.)
+    ln_u32x4 xv[kLnXAhead];
+#pragma unroll
+    for (uint32_t p = 0; p < kLnXAhead; ++p) {
+        const uint32_t e = min(tid + p * n_threads, x_pieces - 1u), r = MT == 1 ? 0u : min(e / (C * 64u), (uint32_t)m - 1u);
+        // whole pieces of an aligned row only; the others are read below
+        const uint32_t col = min((e - e / (C * 64u) * (C * 64u)) * 8u, x_aligned ? (in_f & ~7u) - 8u : 0u);
+        xv[p] = x_aligned ? *reinterpret_cast<const ln_u32x4 *>(x + (int64_t)r * ldx + col) : ln_u32x4{0, 0, 0, 0};
+    }
+    uint32_t buf[kLnAhead][BITS];
+    const uint32_t cell_last = max(cell0 + s1, cell0 + 1u) - 1u;
+#pragma unroll
+    for (uint32_t p = 0; p < kLnAhead; ++p) ln_load<BITS>(plane, min(cell0 + s0 + p, cell_last), lane, buf[p]);
+    // the list's cursor: its range is the listed elements of one row quad within one segment of exc_pos
+    uint32_t l_tile = s0 / C, l_cell = s0 % C;
+    auto l_extent = [&](uint32_t at) { return min(min(s1 - at, C - l_cell), kLnSegCells - l_cell % kLnSegCells); };
+    uint32_t l_seq = s0, l_cells = l_extent(s0);
+    uint32_t r0 = exc_off[cell0 + s0], r1 = exc_off[cell0 + s0 + l_cells];
+    const uint32_t e_end = exc_off[cell0 + s1];  // behind the share's last listed element
+
+    // ---- pair table, activations and zeroed sums to LDS ----
+    const float scale = bf16_bits_to_f32(*scale_at);
+    ln_build_lut<BITS, true>(smem, scale, tid, n_threads);
+    for (uint32_t e = tid; e < n_tiles * n_waves * (MT * 8u); e += n_threads) parts[e] = 0.0f;
+    // the list's groups, one per cell from the share's first cell on
+    struct Group { ln_u32x2 pos; uint32_t val; } list[kLnAhead];
+    const uint32_t g_first = r0 >> 6, g_last = max((e_end + 63u) >> 6, g_first + 1u) - 1u;
+    const uint32_t n_groups = e_end > r0 ? g_last - g_first + 1u : 0u;
+    auto g_load = [&](uint32_t i) {
+        const uint32_t g = min(g_first + i, g_last);
+        return Group{*reinterpret_cast<const ln_u32x2 *>(exc_pos + (size_t)g * 256u + lane * 4u),
+                     *reinterpret_cast<const uint32_t *>(exc_val + (size_t)g * 256u + lane * 4u)};
+    };
+#pragma unroll
+    for (uint32_t p = 0; p < kLnAhead; ++p) list[p] = g_load(p);
+#pragma unroll
+    for (uint32_t p = 0; p < kLnXAhead; ++p) {
+        const uint32_t e = tid + p * n_threads, r = MT == 1 ? 0u : e / (C * 64u), col = (e - r * (C * 64u)) * 8u;
+        if (e < x_pieces && x_aligned && r < (uint32_t)m && col + 8u <= in_f) x_store(e, xv[p]);
+    }
+    for (uint32_t e = tid; e < x_pieces; e += n_threads) {  // what is not stored yet
+        const uint32_t r = MT == 1 ? 0u : e / (C * 64u), col = (e - r * (C * 64u)) * 8u;
+        if (e >= kLnXAhead * n_threads || !x_aligned || r >= (uint32_t)m || col + 8u > in_f) x_store(e, x_piece(e));
+    }
+    __syncthreads();
+
+    const uint32_t lut_lane = smem + ((lane & ((1u << LnPairs<BITS>::kCopies) - 1u)) << 2);
+    const uint32_t q = lane >> 4, kg = (lane >> 2) & 3u, am = min(lane & 3u, (uint32_t)MT - 1u);
+    uint32_t xa[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) xa[i] = x_at + am * x_row + q * 256u + ((i ^ q) << 6) + kg * 16u;
+
+    ln_f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
+
+    float ex[MT][4];
+#pragma unroll
+    for (int r = 0; r < MT; ++r)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) ex[r][k] = 0.0f;
+    // sums over the lanes of a row's products, to `parts`: lane l has row l % 4
+    auto put = [&](uint32_t tile, uint32_t half, int r, float v) {
+        v += ln_dpp<0x124>(v);
+        v += ln_dpp<0x128>(v);
+        v += __shfl_xor(v, 16);
+        v += __shfl_xor(v, 32);
+        if (lane < 4) parts[((tile * n_waves + wave) * 2u + half) * (MT * 4u) + (uint32_t)r * 4u + lane] = v;
+    };
+    // one group of listed elements, range by range
+    auto list_group = [&](const Group &in, uint32_t i) {
+        const uint32_t g0 = (g_first + i) << 6, quad = g0 + lane;
+        for (;;) {
+            uint32_t vals = in.val, p01 = in.pos[0], p23 = in.pos[1];
+            if (g0 < r0 || g0 + 64u > r1) {  // quads outside the range count as 0 * x[0]
+                const bool in_range = quad >= r0 && quad < r1;
+                vals = in_range ? vals : 0u;
+                p01 = in_range ? p01 : 0u;
+                p23 = in_range ? p23 : 0u;
+            }
+            const uint32_t x_seg = x_at + (l_cell / kLnSegCells) * (kLnSegCells * 1024u);
+            const uint32_t at[4] = {x_seg + (p01 & 0xFFFFu), x_seg + (p01 >> 16), x_seg + (p23 & 0xFFFFu), x_seg + (p23 >> 16)};
+            const uint32_t w01 = ln_pack((float)(int)(int8_t)vals * scale, (float)(int)(int8_t)(vals >> 8) * scale);
+            const uint32_t w23 = ln_pack((float)(int)(int8_t)(vals >> 16) * scale, (float)((int)vals >> 24) * scale);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t wk = k & 2 ? w23 : w01;
+                const float wv = __uint_as_float(k & 1 ? wk & 0xFFFF0000u : wk << 16);
+#pragma unroll
+                for (int r = 0; r < MT; ++r) {
+                    const uint32_t h = *reinterpret_cast<const LN_LDS(uint16_t) *>((uintptr_t)(at[k] + (uint32_t)r * x_row));
+                    ex[r][k] = __fmaf_rn(wv, __uint_as_float(h << 16), ex[r][k]);
+                }
+            }
+            if (g0 + 64u < r1) break;  // the range goes on in the next group
+            l_seq += l_cells;
+            l_cell += l_cells;
+            if (l_cell == C || l_seq == s1) {  // the row quad is complete
+#pragma unroll
+                for (int r = 0; r < MT; ++r) {
+                    // every lane gets the sum of row lane % 4 over its quad of lanes
+                    float own = 0.0f;
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        float v = ex[r][k];
+                        v += ln_dpp<0xB1>(v);
+                        v += ln_dpp<0x4E>(v);
+                        own = (lane & 3u) == k ? v : own;
+                        ex[r][k] = 0.0f;
+                    }
+                    put(l_tile, 1u, r, own);
+                }
+                l_cell = 0;
+                ++l_tile;
+            }
+            if (l_seq == s1) break;
+            l_cells = l_extent(l_seq);
+            r0 = r1;
+            r1 = exc_off[cell0 + l_seq + l_cells];
+            if (r0 >= g0 + 64u) break;
+        }
+    };
+
+    uint32_t c = s0 % C, tile = s0 / C;
+    for (uint32_t s = s0; s < s1; s += kLnAhead) {
+        // Left alone, the waves of a SIMD are served oldest first and the last one ends long after the first; a wave
+        // that has more cells to go takes precedence.
+        const uint32_t behind = (s1 - s) * 4u / (s1 - s0 + 1u);
+        if (behind >= 3u) __builtin_amdgcn_s_setprio(3);
+        else if (behind == 2u) __builtin_amdgcn_s_setprio(2);
+        else if (behind == 1u) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+        for (uint32_t p = 0; p < kLnAhead; ++p) {
+            if (s + p >= s1) break;
+            uint32_t o[16];
+            ln_decode<BITS, true>(buf[p], lut_lane, scale, o);
+            ln_load<BITS>(plane, min(cell0 + s + p + kLnAhead, cell_last), lane, buf[p]);
+            const uint32_t x_c = c * 1024u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const ln_u32x4 a = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(xa[i] + x_c));
+                acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(ln_s16x4, ln_u32x2{a[0], a[1]}),
+                                                             __builtin_bit_cast(ln_s16x4, ln_u32x2{o[4 * i], o[4 * i + 1]}), acc0, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(ln_s16x4, ln_u32x2{a[2], a[3]}),
+                                                             __builtin_bit_cast(ln_s16x4, ln_u32x2{o[4 * i + 2], o[4 * i + 3]}), acc1, 0, 0, 0);
+            }
+            if (s + p - s0 < n_groups) list_group(list[p], s + p - s0);
+            list[p] = g_load(s + p - s0 + kLnAhead);
+            ++c;
+            if (c == C || s + p + 1 == s1) {
+#pragma unroll
+                for (int r = 0; r < MT; ++r) put(tile, 0u, r, acc0[r] + acc1[r]);
+                acc0 = ln_f32x4{0, 0, 0, 0};
+                acc1 = ln_f32x4{0, 0, 0, 0};
+                c = 0;
+                ++tile;
+            }
+        }
+    }
+    // a list of more groups than cells
+    for (uint32_t i = s1 - s0; i < n_groups; ++i) list_group(g_load(i), i);
+    __syncthreads();
+
+    // ---- outputs: the waves' parts in wave order ----
+    for (uint32_t e = tid; e < n_tiles * 4u * (uint32_t)m; e += n_threads) {
+        const uint32_t r = e / (n_tiles * 4u), row = e - r * (n_tiles * 4u), at = t0 * 4u + row;
+        if (at >= out_f) continue;
+        float sum = 0.0f;
+        for (uint32_t w = 0; w < 2u * n_waves; ++w) sum += parts[((row >> 2) * n_waves * 2u + w) * (MT * 4u) + r * 4u + (row & 3u)];
+        uint32_t b = f32_to_bf16_bits(sum);
+        if (bias) b = f32_to_bf16_bits(bf16_bits_to_f32(b) + bf16_bits_to_f32(bias[at]));
+        y[(int64_t)r * ldy + at] = (uint16_t)b;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// k_lanes_tile<BITS>: 5 to 16 activation rows (fewer where those of a whole row do not fit k_lanes_gemv).
+//
+// Bound: LDS, close to HBM.  v_mfma_f32_16x16x32_bf16: sixteen weight rows (a block of four row quads) x sixteen
+// activation rows.  A workgroup owns a run of blocks and a slice of the columns, whose activations it copies to LDS in
+// operand order (read from global memory they would be sixteen rows apart, one 16-byte access per lane: 37 us instead of
+// the time below for sixteen rows).  A wave takes 16 x 128 weights at a time: it decodes them to its own 4 KB of
+// LDS in operand order, stores the listed elements over their places, and reads the operands back, each lane its own
+// eight weights.  Nothing is shared between the waves on the way, so there is no barrier in the loop; codes and list are
+// asked for one cell ahead.
+//
+// The cell columns (16 x 512) of a workgroup's blocks are dealt to its waves in contiguous shares, blocks first: a block that lies in
+// one share leaves from its wave, the others' sums meet in LDS and are added in wave order.  The slices' sums meet in
+// the workspace; k_lanes_reduce adds them in slice order.
+// ---------------------------------------------------------------------------------------------------------------
+typedef __bf16 ln_bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr uint32_t kLtWaves = 16;
+constexpr uint32_t kLtTileBytes = 4096;
+constexpr uint32_t kLtXBytes = 64 * 1024;  // activations of a slice at most
+
+__device__ __forceinline__ void ln_wave_order() {  // LDS accesses of the wave's lanes before this one come first
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int BITS>
+__global__ void __launch_bounds__(kLtWaves *kWave)
+k_lanes_tile(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
+             const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t n_tiles, uint32_t slices, uint32_t in_f,
+             const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, int m, int64_t ldx, uint32_t out_f,
+             bool x_aligned, float *__restrict__ ws, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t ln_smem[];
+    using P = LnPairs<BITS, false>;
+    const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)ln_smem;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, M = (uint32_t)m;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t n_blocks = (n_tiles + 3u) / 4u, groups = gridDim.x / slices;
+    const uint32_t slice = blockIdx.x % slices, group = blockIdx.x / slices;
+    const uint32_t c0 = slice * n_cells / slices, c1 = (slice + 1u) * n_cells / slices;
+    const uint32_t b0 = group * n_blocks / groups, b1 = (group + 1u) * n_blocks / groups;
+    const uint32_t block_len = c1 - c0, total = (b1 - b0) * block_len;  // cells of a block, of the workgroup
+    const uint32_t u0 = wave * total / kLtWaves, u1 = (wave + 1u) * total / kLtWaves;
+    const uint32_t tile_at = smem + P::kLutBytes + wave * kLtTileBytes;
+    // a wave's sums of the block that it begins in, [wave][activation row][weight row]; those of its last one: in its tile
+    float *const tiles = reinterpret_cast<float *>(ln_smem + P::kLutBytes);
+    float *const red = reinterpret_cast<float *>(ln_smem + P::kLutBytes + kLtWaves * kLtTileBytes);
+    const uint32_t x_at = smem + P::kLutBytes + kLtWaves * (kLtTileBytes + 1024u);
+
+    const uint32_t n = lane & 15u, kg = lane >> 4;
+    // Requests are made for cells past the share's end too (the last one again), and never inside a branch: the compiler
+    // counts what is in flight.
+    struct Cell { uint32_t block, c; };
+    const uint32_t v0 = min(u0, total - 1u);
+    Cell now{b0 + v0 / block_len, c0 + v0 % block_len};
+    uint32_t to_come = max(u1, u0 + 1u) - u0 - 1u;  // cells of the share behind the one asked for last
+    auto advance = [&](Cell &k) {
+        if (to_come == 0) return;
+        --to_come;
+        if (++k.c == c1) { k.c = c0; ++k.block; }
+    };
+    uint32_t w[4][BITS];
+    auto codes = [&](const Cell &k, uint32_t q) {
+        const uint32_t t = min(4u * k.block + (n >> 2), n_tiles - 1u);
+        const uint8_t *const cell = reinterpret_cast<const uint8_t *>(plane) + (t * n_cells + k.c) * (256u * BITS);  // (below 2^31)
+        ln_load_lane<BITS>(reinterpret_cast<const uint32_t *>(cell), 16u * q + 4u * kg + (n & 3u), w[q]);
+    };
+    // the list of row quad kg of the block in the cell; quads first + n, + 16 and + 32 are this lane's (at 5 % listed
+    // elements the fullest of four rows has 31 in 512 columns, 48 are five standard deviations away)
+    constexpr uint32_t ROUNDS = 3;
+    struct Extent { uint32_t first, end; };
+    auto extent = [&](const Cell &k) {
+        const uint32_t t = 4u * k.block + kg, cell = min(t, n_tiles - 1u) * n_cells + k.c;
+        const uint32_t a = exc_off[cell], b = exc_off[cell + 1u];
+        return Extent{a, t < n_tiles ? b : a};
+    };
+    struct Quads { ln_u32x2 pos[ROUNDS]; uint32_t val[ROUNDS]; };
+    auto quads = [&](const Extent &e) {
+        Quads l;
+#pragma unroll
+        for (uint32_t r = 0; r < ROUNDS; ++r) {
+            const uint32_t at = e.first + n + 16u * r < e.end ? e.first + n + 16u * r : 0u;
+            l.pos[r] = *reinterpret_cast<const ln_u32x2 *>(reinterpret_cast<const uint8_t *>(exc_pos) + at * 8u);
+            l.val[r] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(exc_val) + at * 4u);
+        }
+        return l;
+    };
+
+    // ---- first requests; activations (8 pieces x 8 rows a wave and turn) and pair table to LDS ----
+    const uint32_t pieces = (c1 - c0) * 64u, m_groups = (M + 7u) / 8u, chunks = (pieces / 8u) * m_groups;
+    Cell far = now;
+    Extent e_now = extent(far);
+    const uint32_t in_8 = in_f & ~7u;
+    if (x_aligned) {
+        for (uint32_t chunk = wave; chunk < chunks; chunk += 4u * kLtWaves) {
+            ln_u32x4 v[4];
+            uint32_t to[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                const uint32_t ch = min(chunk + k * kLtWaves, chunks - 1u), pg = ch / m_groups;
+                const uint32_t r = min((ch - pg * m_groups) * 8u + (lane & 7u), M - 1u), p = pg * 8u + (lane >> 3);
+                to[k] = x_at + (p * M + r) * 16u;
+                // (whole pieces of the row; what lies past them is written below)
+                v[k] = *reinterpret_cast<const ln_u32x4 *>(x + (int64_t)r * ldx + min(c0 * kLnCols + p * 8u, in_8 - 8u));
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)to[k]) = v[k];
+        }
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) codes(far, q);
+    Quads list = quads(e_now);
+    advance(far);
+    Extent e_next = extent(far);
+    const float scale = bf16_bits_to_f32(*scale_at);
+    ln_build_lut<BITS, false>(smem, scale, tid, kLtWaves * kWave);
+    __syncthreads();
+    {   // pieces that are no whole ones of an aligned row, element by element; zero past the row
+        const uint32_t from = x_aligned ? max(in_8, c0 * kLnCols) : c0 * kLnCols, to = c1 * kLnCols;
+        if (from < to) {
+            for (uint32_t e = tid; e < (to - from) / 8u * M; e += kLtWaves * kWave) {
+                const uint32_t piece = e / M, r = e - piece * M, col = from + piece * 8u;
+                uint32_t h[8];
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k) h[k] = col + k < in_f ? x[(int64_t)r * ldx + col + k] : 0u;
+                *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + ((col / 8u - c0 * 64u) * M + r) * 16u)) =
+                    ln_u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+            }
+            __syncthreads();
+        }
+    }
+    const uint32_t lut_lane = smem + ((lane & ((1u << P::kCopies) - 1u)) << 2);
+    const uint32_t xa = x_at + (kg * M + min(n, M - 1u)) * 16u;  // (rows past the last: any, their sums are not used)
+
+    auto out = [&](uint32_t row, uint32_t r, float sum) {
+        if (row >= out_f || r >= M) return;
+        if (slices > 1u) {
+            ws[((size_t)slice * M + r) * out_f + row] = sum;
+        } else {
+            uint32_t h = f32_to_bf16_bits(sum);
+            if (bias) h = f32_to_bf16_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(bias[row]));
+            y[(int64_t)r * ldy + row] = (uint16_t)h;
+        }
+    };
+
+    ln_f32x4 acc = {0, 0, 0, 0};
+    uint32_t block_first = u0;  // first of this wave's cells in the block
+    for (uint32_t u = u0; u < u1; ++u) {
+        // ---- listed elements: value (high half), where it goes in the tile of its quarter (bits 0..11; the tile's block i
+        // is at i ^ q, as the list has it), the quarter (bits 12..14; none of the four where there is no element) ----
+        uint32_t put[4 * ROUNDS];
+#pragma unroll
+        for (uint32_t r = 0; r < ROUNDS; ++r) {
+            const uint32_t val = e_now.first + n + 16u * r < e_now.end ? list.val[r] : 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                const uint32_t p = (k & 1) ? list.pos[r][k >> 1] >> 16 : list.pos[r][k >> 1];
+                const int v = (int)(val << (24 - 8 * k)) >> 24;
+                put[4 * r + k] = (ln_pack(0.0f, (float)v * scale) & 0xFFFF0000u) | (v != 0 ? (p & 0x300u) << 4 : 0x4000u) |
+                                 (((p & 0xF0u) << 4) + (p & 14u) + (kg << 6) + k * 16u);
+            }
+        }
+        bool any[ROUNDS];
+#pragma unroll
+        for (uint32_t r = 0; r < ROUNDS; ++r) any[r] = __any(e_now.first + 16u * r < e_now.end);
+        const bool more = __any(e_now.first + 16u * ROUNDS < e_now.end);
+        const Extent e_more = e_now;
+        e_now = e_next;
+        list = quads(e_now);
+        const Cell next = far;
+        advance(far);
+        e_next = extent(far);
+        const uint32_t x_c = xa + (now.c - c0) * 1024u * M;
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            uint32_t o[16];
+            ln_decode<BITS, false>(w[q], lut_lane, scale, o);
+            codes(next, q);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i)
+                *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(tile_at + ((i ^ q) << 10) + lane * 16u)) =
+                    ln_u32x4{o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]};
+            ln_wave_order();
+#pragma unroll
+            for (uint32_t r = 0; r < ROUNDS; ++r)
+                if (any[r])
+#pragma unroll
+                    for (uint32_t e = 4 * r; e < 4 * r + 4; ++e)
+                        if ((put[e] & 0x7000u) == (q << 12))
+                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + (put[e] & 0xFFFu))) = (uint16_t)(put[e] >> 16);
+            if (more) {  // rows with yet more listed elements in the cell
+                for (uint32_t f = e_more.first + n + 16u * ROUNDS; f < e_more.end; f += 16u)
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        const uint32_t p = exc_pos[(size_t)f * 4u + k];
+                        const int v = exc_val[(size_t)f * 4u + k];
+                        if (v != 0 && (p & 0x300u) == (q << 8))
+                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + (kg << 6) + k * 16u + ((p & 0xF0u) << 4) + (p & 14u))) =
+                                (uint16_t)(ln_pack((float)v * scale, 0.0f) & 0xFFFFu);
+                    }
+            }
+            ln_wave_order();
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                const ln_u32x4 b = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(tile_at + ((i ^ q) << 10) + lane * 16u));
+                const ln_u32x4 a = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(x_c + (q * 16u + i * 4u) * 16u * M));
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ln_bf16x8, a), __builtin_bit_cast(ln_bf16x8, b), acc, 0, 0, 0);
+            }
+            ln_wave_order();
+        }
+        if (u + 1u == u1 || now.c + 1u == c1) {  // this wave's part of the block is complete
+            const uint32_t from = (now.block - b0) * block_len;
+            const bool whole = block_first <= from && u + 1u == from + block_len;
+            float *const part = u + 1u == u1 ? tiles + wave * (kLtTileBytes / 4u) : red + wave * 256u;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                if (whole) out(now.block * 16u + n, 4u * kg + k, acc[k]);
+                else part[(4u * kg + k) * 16u + n] = acc[k];
+            }
+            acc = ln_f32x4{0, 0, 0, 0};
+            block_first = u + 1u;
+        }
+        if (++now.c == c1) { now.c = c0; ++now.block; }
+    }
+    __syncthreads();
+
+    // ---- blocks that lie in several shares: their waves' sums in wave order, a wave a block ----
+    for (uint32_t b = wave; b < b1 - b0; b += kLtWaves) {
+        const uint32_t from = b * block_len, to = from + block_len;
+        bool shared = true;
+        ln_f32x4 sum = {0, 0, 0, 0};
+#pragma unroll
+        for (uint32_t k = 0; k < kLtWaves; ++k) {
+            const uint32_t a0 = k * total / kLtWaves, a1 = (k + 1u) * total / kLtWaves;
+            if (a0 >= a1 || a1 <= from || a0 >= to) continue;
+            if (a0 <= from && a1 >= to) shared = false;
+            sum += *reinterpret_cast<const ln_f32x4 *>((a1 <= to ? tiles + k * (kLtTileBytes / 4u) : red + k * 256u) + lane * 4u);
+        }
+        if (shared)
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) out((b0 + b) * 16u + ((lane * 4u + k) & 15u), lane >> 2, sum[k]);
+    }
+}
+
+// outputs from the slices' sums, in slice order
+__global__ void __launch_bounds__(256)
+k_lanes_reduce(const float *__restrict__ ws, uint32_t slices, int m, uint32_t out_f, const uint16_t *__restrict__ bias,
+               uint16_t *__restrict__ y, int64_t ldy) {
+    const uint32_t row = blockIdx.x * 256u + threadIdx.x, r = blockIdx.y;
+    if (row >= out_f) return;
+    const float *p = ws + (size_t)r * out_f + row;
+    const size_t stride = (size_t)m * out_f;
+    float sum = 0.0f;
+    for (uint32_t g = 0; g < slices; g += 8) {
+        float v[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) v[k] = p[(size_t)min(g + k, slices - 1u) * stride];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            if (g + k < slices) sum += v[k];
+    }
+    uint32_t h = f32_to_bf16_bits(sum);
+    if (bias) h = f32_to_bf16_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(bias[row]));
+    y[(int64_t)r * ldy + row] = (uint16_t)h;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// Writing the layout from the decoded bf16 weights (deploy time): one wave per cell.  value = round(w / scale) gives
+// back the integer exactly (w is value * scale rounded to 8 significant bits, |value| <= 128).
+// ---------------------------------------------------------------------------------------------------------------
+template <int BITS>
+__device__ __forceinline__ void ln_cell_values(const uint16_t *__restrict__ w, const LanesDev &L, uint32_t cell,
+                                               uint32_t lane, int (&v)[32]) {
+    const uint32_t t = cell / L.n_cells, c = cell - t * L.n_cells;
+    const uint32_t row = 4u * t + (lane & 3u), col0 = kLnCols * c + 128u * (lane >> 4) + 8u * ((lane >> 2) & 3u);
+    const float scale = bf16_bits_to_f32(*L.scale);
+#pragma unroll
+    for (uint32_t e = 0; e < 32; ++e) {
+        const uint32_t col = col0 + 32u * (e >> 3) + (e & 7u);
+        v[e] = 0;
+        if (row < L.out_f && col < L.in_f)
+            v[e] = __float2int_rn(bf16_bits_to_f32(w[(size_t)row * L.in_f + col]) / scale);
+    }
+}
+
+template <int BITS> __device__ __forceinline__ bool ln_listed(int v) {
+    constexpr int T = (1 << (BITS - 1)) - 1;
+    return v > T || v < -T;
+}
+
+template <int BITS>
+__global__ void __launch_bounds__(256)
+k_lanes_pack(const uint16_t *__restrict__ w, LanesDev L, uint32_t *__restrict__ plane, uint32_t *__restrict__ counts) {
+    const uint32_t lane = threadIdx.x & 63u, cell = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (cell >= L.n_tiles * L.n_cells) return;
+    int v[32];
+    ln_cell_values<BITS>(w, L, cell, lane, v);
+    constexpr int T = (1 << (BITS - 1)) - 1;
+    uint32_t n = 0, code[32], d[BITS];
+#pragma unroll
+    for (int e = 0; e < 32; ++e) {
+        const bool listed = ln_listed<BITS>(v[e]);
+        n += listed;
+        code[e] = (uint32_t)((listed ? 0 : v[e]) + T);
+    }
+#pragma unroll
+    for (int k = 0; k < BITS; ++k) d[k] = 0;
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+        const uint32_t pair = code[2 * p] | (code[2 * p + 1] << BITS);
+        if constexpr (BITS == 8) d[p >> 1] |= pair << (16 * (p & 1));
+        else if constexpr (BITS == 4) d[p >> 2] |= pair << (8 * (p & 3));
+        else {
+            constexpr int PER = BITS == 3 ? 5 : 3;
+            if (p < 15) d[p / PER] |= pair << (2 + 2 * BITS * (p % PER));
+            else
+                for (int k = 0; k < BITS; ++k) d[k] |= (pair >> (2 * k)) & 3u;
+        }
+    }
+    uint32_t *out = plane + (size_t)cell * (64u * BITS);
+    constexpr int HEAD = BITS < 4 ? BITS : 4;
+#pragma unroll
+    for (int k = 0; k < BITS; ++k) {
+        if (k < HEAD) out[lane * HEAD + k] = d[k];
+        else out[64 * HEAD + lane * (BITS - HEAD) + (k - HEAD)] = d[k];
+    }
+    for (int o = 4; o < 64; o <<= 1) n += __shfl_xor(n, o);  // of the lane's row
+    n = max(n, (uint32_t)__shfl_xor(n, 1));
+    n = max(n, (uint32_t)__shfl_xor(n, 2));
+    if (lane == 0) counts[cell] = n;
+}
+
+template <int BITS>
+__global__ void __launch_bounds__(256)
+k_lanes_list(const uint16_t *__restrict__ w, LanesDev L, uint16_t *__restrict__ pos, int8_t *__restrict__ val) {
+    const uint32_t lane = threadIdx.x & 63u, cell = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (cell >= L.n_tiles * L.n_cells) return;
+    int v[32];
+    ln_cell_values<BITS>(w, L, cell, lane, v);
+    uint32_t n = 0;
+#pragma unroll
+    for (int e = 0; e < 32; ++e) n += ln_listed<BITS>(v[e]);
+    uint32_t before = n;  // listed elements of the row in the slices up to this one
+    for (int o = 4; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(before, o);
+        if (lane >= (uint32_t)o) before += u;
+    }
+    uint32_t at = L.exc_off[cell] + before - n;
+    const uint32_t end = L.exc_off[cell + 1];
+    const uint32_t col0 = (kLnCols * (cell % L.n_cells) + 128u * (lane >> 4) + 8u * ((lane >> 2) & 3u)) % (kLnSegCells * kLnCols);
+#pragma unroll
+    for (uint32_t e = 0; e < 32; ++e)
+        if (ln_listed<BITS>(v[e]) && at < end) {
+            pos[4u * at + (lane & 3u)] = (uint16_t)lane_offset(col0 + 32u * (e >> 3) + (e & 7u));
+            val[4u * at + (lane & 3u)] = (int8_t)v[e];
+            ++at;
+        }
+}
+
+static uint32_t ln_cus() {
+    static const uint32_t n = [] {
+        int dev = 0, v = 256;
+        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev);
+        return (uint32_t)v;
+    }();
+    return n;
+}
+
+int launch_lanes_pack(const uint16_t *w, const LanesDev &L, uint32_t *plane, uint32_t *counts, hipStream_t s) {
+    const dim3 grid((L.n_tiles * L.n_cells + 3u) / 4u), block(256);
+    switch (L.bits) {
+        case 3: hipLaunchKernelGGL(k_lanes_pack<3>, grid, block, 0, s, w, L, plane, counts); break;
+        case 4: hipLaunchKernelGGL(k_lanes_pack<4>, grid, block, 0, s, w, L, plane, counts); break;
+        case 5: hipLaunchKernelGGL(k_lanes_pack<5>, grid, block, 0, s, w, L, plane, counts); break;
+        default: hipLaunchKernelGGL(k_lanes_pack<8>, grid, block, 0, s, w, L, plane, counts); break;
+    }
+    return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
+}
+
+int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_t *val, hipStream_t s) {
+    const dim3 grid((L.n_tiles * L.n_cells + 3u) / 4u), block(256);
+    switch (L.bits) {
+        case 3: hipLaunchKernelGGL(k_lanes_list<3>, grid, block, 0, s, w, L, pos, val); break;
+        case 4: hipLaunchKernelGGL(k_lanes_list<4>, grid, block, 0, s, w, L, pos, val); break;
+        case 5: hipLaunchKernelGGL(k_lanes_list<5>, grid, block, 0, s, w, L, pos, val); break;
+        default: hipLaunchKernelGGL(k_lanes_list<8>, grid, block, 0, s, w, L, pos, val); break;
+    }
+    return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
+}
+
+template <int BITS, int MT>
+static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
+                             int64_t ldy, hipStream_t s) {
+    // Workgroups of 16, 8 or 4 waves, one, two or four to a CU: the split whose last round of row quads is fullest.
+    const size_t fixed = LnPairs<BITS>::kLutBytes + (size_t)MT * L.n_cells * 1024u;
+    auto lds_of = [&](uint32_t tiles, uint32_t waves) { return fixed + (size_t)tiles * waves * (MT * 32u); };
+    uint32_t best_waves = 0, best_tiles = 0;
+    uint64_t best_cost = ~0ull;
+    for (uint32_t per_cu = 1; per_cu <= 4; per_cu *= 2) {
+        const uint32_t waves = 16u / per_cu, slots = ln_cus() * per_cu;
+        const uint32_t tiles = (L.n_tiles + slots - 1) / slots;
+        if (lds_of(tiles, waves) * per_cu > kLnLds) break;
+        const uint64_t cost = (uint64_t)tiles * per_cu;  // row quads a CU works through
+        if (cost < best_cost) { best_cost = cost; best_waves = waves; best_tiles = tiles; }
+    }
+    if (!best_waves) return IXH_EUNSUPPORTED;
+    const uint32_t waves = min(best_waves, best_tiles * L.n_cells);
+    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemv<BITS, MT>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
+    if (!raised) return IXH_ELAUNCH;
+    const bool aligned = ((uintptr_t)x & 15u) == 0 && (m == 1 || ldx % 8 == 0);
+    hipLaunchKernelGGL((k_lanes_gemv<BITS, MT>), dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave * waves),
+                       lds_of(best_tiles, waves), s, L.plane, x, L.exc_off, L.scale, L.n_cells, L.n_tiles, best_tiles, L.in_f,
+                       L.exc_pos, L.exc_val, m, ldx, bias, y, ldy, L.out_f, aligned);
+    return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
+}
+
+// How the tile kernel's work is cut: `slices` of the columns, few enough for the activations of one to fit, and the
+// blocks of 16 rows in as many groups as leave a workgroup per CU.  Of all such cuts the one whose fullest wave has the
+// fewest cells, then whose workgroups have; a further slice counts as a cell, for its sums' way through memory.
+struct LtPlan { uint32_t slices, groups; };
+static LtPlan lt_plan(const LanesDev &L, int m) {
+    const uint32_t blocks = (L.n_tiles + 3u) / 4u, cus = ln_cus();
+    const uint32_t most_cells = max(kLtXBytes / (1024u * (uint32_t)m), 1u);
+    LtPlan best{1, 1};
+    uint64_t best_cost = ~0ull;
+    for (uint32_t s = (L.n_cells + most_cells - 1u) / most_cells; s <= min(L.n_cells, cus); ++s) {
+        const uint32_t groups = min(max(cus / s, 1u), blocks);
+        const uint32_t cells = ((blocks + groups - 1u) / groups) * ((L.n_cells + s - 1u) / s);
+        const uint64_t cost = (uint64_t)((cells + kLtWaves - 1u) / kLtWaves) * 64u + cells + s;
+        if (cost < best_cost) { best_cost = cost; best = {s, groups}; }
+    }
+    return best;
+}
+
+template <int BITS>
+static int lanes_tile_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
+                             int64_t ldy, float *ws, hipStream_t s) {
+    constexpr size_t fixed = LnPairs<BITS, false>::kLutBytes + kLtWaves * (kLtTileBytes + 1024u);
+    static_assert(fixed + kLtXBytes <= kLnLds, "LDS of a CU");
+    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_tile<BITS>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
+    if (!raised) return IXH_ELAUNCH;
+    const LtPlan p = lt_plan(L, m);
+    const uint32_t cells = (L.n_cells + p.slices - 1u) / p.slices;
+    const bool aligned = ((uintptr_t)x & 15u) == 0 && (m == 1 || ldx % 8 == 0);
+    hipLaunchKernelGGL(k_lanes_tile<BITS>, dim3(p.slices * p.groups), dim3(kLtWaves * kWave), fixed + (size_t)cells * 1024u * (uint32_t)m, s,
+                       L.plane, x, L.exc_off, L.scale, L.n_cells, L.n_tiles, p.slices, L.in_f, L.exc_pos, L.exc_val, m, ldx, L.out_f,
+                       aligned, ws, bias, y, ldy);
+    if (p.slices > 1)
+        hipLaunchKernelGGL(k_lanes_reduce, dim3((L.out_f + 255u) / 256u, m), dim3(256), 0, s, ws, p.slices, m, L.out_f, bias, y, ldy);
+    return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
+}
+
+template <int BITS>
+static int lanes_gemv_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
+                           int64_t ldy, float *ws, hipStream_t s) {
+    int rc = IXH_EUNSUPPORTED;
+    if (m == 1) rc = lanes_gemv_launch<BITS, 1>(L, x, m, ldx, bias, y, ldy, s);
+    else if (m == 2) rc = lanes_gemv_launch<BITS, 2>(L, x, m, ldx, bias, y, ldy, s);
+    else if (m <= 4) rc = lanes_gemv_launch<BITS, 4>(L, x, m, ldx, bias, y, ldy, s);
+    if (rc == IXH_EUNSUPPORTED) rc = lanes_tile_launch<BITS>(L, x, m, ldx, bias, y, ldy, ws, s);
+    return rc;
+}
+
+size_t lanes_gemv_workspace_bytes(const LanesDev &L, int m) {
+    const LtPlan p = lt_plan(L, m);
+    return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * L.out_f * sizeof(float) : 0;
+}
+
+int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
+                      int64_t ldy, float *ws, hipStream_t s) {
+    switch (L.bits) {
+        case 3: return lanes_gemv_rows<3>(L, x, m, ldx, bias, y, ldy, ws, s);
+        case 4: return lanes_gemv_rows<4>(L, x, m, ldx, bias, y, ldy, ws, s);
+        case 5: return lanes_gemv_rows<5>(L, x, m, ldx, bias, y, ldy, ws, s);
+        default: return lanes_gemv_rows<8>(L, x, m, ldx, bias, y, ldy, ws, s);
+    }
+}
+
+}  // namespace ixh

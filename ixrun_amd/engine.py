@@ -33,6 +33,7 @@ except AttributeError:  # pragma: no cover
     def _raw_stream(index):
         return torch.cuda.current_stream(index).cuda_stream
 
+LANE_BUFFERS = ("_lane_plane", "_lane_off", "_lane_pos", "_lane_val")
 MAX_FUSED_ROWS = 16  # activation rows served by the fused decode+GEMV kernel
 # With a decode buffer at hand, more rows than this go through decode + library GEMM.  Tensors that are almost all
 # level 1, MI355X: the pair takes 72-75 us on 17408 x 5120 and 5120 x 17408 at any M up to 32 and 34-50 us on
@@ -67,9 +68,16 @@ class StreamingLinear(nn.Module):
     (``ixh_prefix_build``); ``_q1``/``_q2`` and ``_b1_blk``/``_b2_blk`` are the
     reference-shaped views of them.  Any level scheme is accepted; bitmaps and
     streams beyond the third level are registered as ``_b3``, ``_l4`` and so on.
+
+    With ``lanes`` the same integers are kept in the lane layout as well
+    (``csrc/ixh_lanes.h``; 3.1 to 6.5 bits a weight for the mixes that take 4.0
+    to 5.5 packed), which the forwards of up to 16 rows read: one row of
+    5120 x 17408 takes 14 us from it instead of 17 (99 % of the weights in
+    level 1), 20 us instead of 48 (55 / 40 / 5 %), five levels 20 us instead of
+    86.  It is no part of the state dict.
     """
 
-    def __init__(self, packed: dict, bias=None):
+    def __init__(self, packed: dict, bias=None, lanes: bool = True):
         super().__init__()
         self.out_features = packed["out_f"]
         self.in_features = packed["in_f"]
@@ -83,6 +91,7 @@ class StreamingLinear(nn.Module):
         for i in range(n_levels):
             self.register_buffer(f"_l{i + 1}", packed["streams"][i].cuda())
         self.register_buffer("_scale", packed["scale"].reshape(()).cuda())
+        self.register_buffer("_bias", bias.detach().clone().cuda() if bias is not None else None)
         self._gemv_flags = 0  # extra IXH_GEMV_* flags of every fused call (comparisons: bench.py --gemv-flags)
         self._bind()
 
@@ -115,13 +124,30 @@ class StreamingLinear(nn.Module):
         self.register_buffer("_q2", q[1].contiguous() if n_levels > 2 else torch.zeros_like(q[0]))
         self._y32 = None
 
-        if bias is not None:
-            self.register_buffer("_bias", bias.detach().clone().cuda())
-        else:
-            self._bias = None
         self._w_buf = None  # set by the engine
+        if lanes:
+            self._make_lanes()
         # the shared scratch takes its final size now, not inside some later forward (or graph capture)
-        shared_workspace(self._scale.device, self._dp.gemv_workspace_bytes(self._unit, MAX_FUSED_ROWS))
+        need = self._dp.gemv_workspace_bytes(self._unit, MAX_FUSED_ROWS)
+        if self._lanes is not None:
+            need = max(need, self._lanes.gemv_workspace_bytes(MAX_FUSED_ROWS))
+        shared_workspace(self._scale.device, need)
+
+    def _make_lanes(self):
+        """Lay the weights out for the lanes of the fused kernels (``_lib.LanePacked``), unless that would leave less than
+        a quarter of the GPU's memory: then the forwards read the packed streams."""
+        self._lanes = None
+        n_bytes = _lib.LanePacked.estimate(self._dp, self.counts)
+        free, total = torch.cuda.mem_get_info(self._scale.device)
+        if self.N == 0 or n_bytes is None or free - n_bytes - 2 * self.N < total // 4:
+            for name in LANE_BUFFERS:
+                self.register_buffer(name, None, persistent=False)
+            self._bind()
+            return
+        lanes = _lib.LanePacked.build(self._dp, self._table, self._unit, self.counts)
+        for name, t in zip(LANE_BUFFERS, lanes.tensors):
+            self.register_buffer(name, t, persistent=False)
+        self._bind()
 
     def _fused_gemm_wins(self, rows: int) -> bool:
         """Whether ``ixh_gemm`` beats decode + library GEMM when a decode buffer is at hand.
@@ -145,9 +171,17 @@ class StreamingLinear(nn.Module):
         )
         # what every fused call passes unchanged (the table follows the module when it moves: see _apply)
         import ctypes
-        self._gemv_fn = _lib.lib().ixh_gemv
         self._struct_ref = ctypes.byref(self._dp.struct)
         self._table_ptr = self._table.data_ptr() if hasattr(self, "_table") else None
+        self._lanes = self._lane_ref = self._bias_ptr = None
+        if getattr(self, LANE_BUFFERS[0], None) is not None:
+            self._lanes = _lib.LanePacked(self.out_features, self.in_features, [getattr(self, b) for b in LANE_BUFFERS],
+                                          self._scale)
+            self._lane_ref = ctypes.byref(self._lanes.struct)
+            bias = self._bias
+            if bias is not None and bias.dtype is torch.bfloat16 and bias.is_cuda and bias.is_contiguous():
+                self._bias_ptr = bias.data_ptr()  # added by the kernel
+        self._gemv_fn = _lib.lib().ixh_lanes_gemv if self._lanes is not None else _lib.lib().ixh_gemv
         self._plans = {}
 
     def _apply(self, fn, recurse=True):
@@ -156,6 +190,11 @@ class StreamingLinear(nn.Module):
         if hasattr(self, "_scale") and self._scale.is_cuda:
             self._bind()
         return out
+
+    def _load_from_state_dict(self, *args, **kwargs):
+        super()._load_from_state_dict(*args, **kwargs)
+        if self._scale.is_cuda:
+            self._make_lanes()  # the packed streams may be others now
 
     def _set_shared_buf(self, w_buf):
         self._w_buf = w_buf
@@ -173,7 +212,8 @@ class StreamingLinear(nn.Module):
         two for 17 .. 32 rows on a large layer that is almost all level 1) with the scratch it needs, or False where
         the many-row paths take over.  Worked out once per row count; ``_set_shared_buf`` and ``_bind`` forget the
         answers."""
-        if self._w_buf is None:
+        lanes = self._lanes is not None and self._gemv_flags == 0
+        if self._w_buf is None or lanes:
             fused_rows = MAX_FUSED_ROWS
         elif self.counts[0] * 100 >= self.N * 97:
             fused_rows = MAX_FUSED_ROWS_WITH_BUFFER
@@ -182,14 +222,15 @@ class StreamingLinear(nn.Module):
         else:
             fused_rows = 1
         two_calls = (MAX_FUSED_ROWS < rows <= 2 * MAX_FUSED_ROWS and fused_rows == MAX_FUSED_ROWS
-                     and self.N >= SPLIT_FUSED_MIN_WEIGHTS and self.counts[0] * 100 >= self.N * 97)
+                     and self.N >= SPLIT_FUSED_MIN_WEIGHTS and (lanes or self.counts[0] * 100 >= self.N * 97))
         plan = False
         if 1 <= rows <= fused_rows or two_calls:
             calls = []
             for r0 in range(0, rows, MAX_FUSED_ROWS):
                 n = min(MAX_FUSED_ROWS, rows - r0)
-                calls.append((r0, n, self._dp.gemv_workspace_bytes(self._unit, n, self._gemv_flags)))
-            plan = tuple(calls)
+                calls.append((r0, n, self._lanes.gemv_workspace_bytes(n) if lanes
+                              else self._dp.gemv_workspace_bytes(self._unit, n, self._gemv_flags)))
+            plan = (lanes, tuple(calls))
         self._plans[rows] = plan
         return plan
 
@@ -209,16 +250,22 @@ class StreamingLinear(nn.Module):
                 y = torch.empty(x.shape[:-1] + (out_f,), dtype=torch.bfloat16, device=dev)
                 x_ptr, y_ptr = x.data_ptr(), y.data_ptr()
                 stream = _raw_stream(dev.index if dev.index is not None else torch.cuda.current_device())
-                for r0, n, ws_bytes in plan:  # one call, or two on the same stream and workspace
+                lanes, calls = plan
+                for r0, n, ws_bytes in calls:  # one call, or two on the same stream and workspace
                     ws = _workspaces.get(dev) if ws_bytes else None
                     if ws_bytes and (ws is None or ws.numel() * 4 < ws_bytes):
                         ws = shared_workspace(dev, ws_bytes)
-                    rc = self._gemv_fn(self._struct_ref, self._table_ptr, self._unit, x_ptr + r0 * in_f * 2, n, in_f,
-                                       y_ptr + r0 * out_f * 2, out_f, None, ws.data_ptr() if ws_bytes else None,
-                                       ws_bytes, self._gemv_flags, stream)
+                    if lanes:
+                        rc = self._gemv_fn(self._lane_ref, x_ptr + r0 * in_f * 2, in_f, self._bias_ptr, n, y_ptr + r0 * out_f * 2,
+                                           out_f, ws.data_ptr() if ws_bytes else None, ws_bytes, stream)
+                    else:
+                        gemv = self._gemv_fn if self._lanes is None else _lib.lib().ixh_gemv
+                        rc = gemv(self._struct_ref, self._table_ptr, self._unit, x_ptr + r0 * in_f * 2, n, in_f,
+                                  y_ptr + r0 * out_f * 2, out_f, None, ws.data_ptr() if ws_bytes else None,
+                                  ws_bytes, self._gemv_flags, stream)
                     if rc:
                         _lib.check(rc)
-                if self._bias is not None:
+                if self._bias is not None and not (lanes and self._bias_ptr):
                     y = y + self._bias.to(y.dtype)
                 return y
         rows = x.numel() // in_f if in_f else 0
@@ -416,7 +463,7 @@ class Int8XEngine:
         for name, mod in targets:
             packed = quantize_for_deploy(mod.weight.data, level_bits)
             bias = mod.bias.data if mod.bias is not None else None
-            sl = StreamingLinear(packed, bias=bias)
+            sl = StreamingLinear(packed, bias=bias, lanes=False)  # only its decode is used
             buf = torch.empty(packed["N"], dtype=torch.bfloat16, device="cuda")
             sl._set_shared_buf(buf)
             specs.append((name, sl, buf))

@@ -1,0 +1,154 @@
+"""The lane layout (``ixh_lanes_*``) through the C ABI: products of 1 to 16 activation rows against the fp64 oracle.
+
+Shapes sit at the edges of the layout (row quads, 16-row blocks, 512-column cells, the 32768-column segments of the
+list), mixes at every width of the plane, with no listed element, with rows of listed elements only, and with one row
+far fuller than the others of its quad."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import activations, bf16_bits, bits_to_bf16, int8_mix, packed_from_int8, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    return torch.device("cuda:0")
+
+
+def values(kind, out_f, in_f):
+    """(int8 values, scheme, width of the plane)"""
+    n = out_f * in_f
+    if kind == "narrow":
+        return int8_mix("only_l1", n, seed=1), (3, 5, 8), 3
+    if kind == "rare":
+        return int8_mix("rare_other", n, seed=1), (3, 5, 8), 3
+    if kind == "four":
+        v = int8_mix("only_l1", n, seed=2) * 2
+        v[::67] = 100
+        return v.astype(np.int8), (4, 8), 4
+    if kind == "real":
+        rng = np.random.default_rng(3)
+        v = rng.integers(-15, 16, size=n)
+        hit = rng.random(n) < 0.05
+        v[hit] = rng.integers(16, 128, size=n)[hit] * (rng.integers(0, 2, size=n)[hit] * 2 - 1)
+        return v.astype(np.int8), (3, 4, 5, 6, 8), 5
+    if kind == "full_row":  # a quad of rows one of which is listed throughout
+        v = int8_mix("no_l3", n, seed=4).reshape(out_f, in_f)
+        v[out_f // 2] = 77
+        return v.reshape(-1), (3, 5, 8), 5 if out_f >= 16 else 8  # (8: shorter than the list would be)
+    return int8_mix("only_l3", n, seed=5), (3, 5, 8), 8
+
+
+def lay_out(kind, out_f, in_f, dev):
+    from ixrun_amd import _lib
+    from ixrun_amd.fused import pick_unit
+
+    v, scheme, bits = values(kind, out_f, in_f)
+    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
+    dp = _lib.DevicePacked.from_dict(p, dev)
+    unit = pick_unit(in_f)
+    lanes = _lib.LanePacked.build(dp, dp.prefix_build(unit), unit, p["counts"])
+    assert lanes.bits == bits
+    return p, lanes
+
+
+def product(lanes, x, out_f, in_f, bias=None):
+    from ixrun_amd import _lib
+
+    m = x.shape[0]
+    need = lanes.gemv_workspace_bytes(m)
+    ws = torch.full((need // 4 + 1,), float("nan"), dtype=torch.float32, device=x.device)
+    y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=x.device)
+    _lib.check(_lib.lib().ixh_lanes_gemv(C.byref(lanes.struct), x.data_ptr(), x.stride(0), bias.data_ptr() if bias is not None else None,
+                                         m, y.data_ptr(), out_f, ws.data_ptr(), need, _lib.current_stream(x.device)))
+    return y
+
+
+def check(oracle, p, x, y, bias=None):
+    want = oracle.gemm_f64(oracle.decode_packed_bf16(p), bf16_bits(x)).astype(np.float32)
+    want = oracle.f32_to_bf16_bits(want)
+    if bias is not None:
+        want = oracle.f32_to_bf16_bits(oracle.bf16_bits_to_f32(want) + bias.float().cpu().numpy()[None, :])
+    got = oracle.bf16_bits_to_f32(bf16_bits(y)).astype(np.float64)
+    assert rel_l2(got, oracle.bf16_bits_to_f32(want)) <= 1e-3
+
+
+@pytest.mark.parametrize("kind", ["narrow", "rare", "four", "real", "full_row", "wide"])
+@pytest.mark.parametrize("out_f,in_f", [(16, 512), (5, 511), (67, 1003), (130, 2560), (33, 4104)])
+def test_products(oracle, dev, kind, out_f, in_f):
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    for m in (1, 2, 3, 4, 5, 8, 9, 16):
+        x = activations(m, in_f, seed=m)
+        y = product(lanes, x.to(dev), out_f, in_f)
+        check(oracle, p, x, y)
+        assert torch.equal(y, product(lanes, x.to(dev), out_f, in_f))  # the order of the sums is fixed
+
+
+@pytest.mark.parametrize("kind", ["rare", "real"])
+@pytest.mark.parametrize("out_f,in_f", [(6, 33800), (4100, 520)])
+def test_long_rows_and_many_rows(oracle, dev, kind, out_f, in_f):
+    """More columns than a segment of the list; more row blocks than a workgroup has waves."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    for m in (1, 2, 4, 16):
+        x = activations(m, in_f, seed=m)
+        check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
+
+
+@pytest.mark.parametrize("m", [1, 4, 7])
+def test_bias_and_unaligned_activations(oracle, dev, m):
+    out_f, in_f = 37, 1536
+    p, lanes = lay_out("real", out_f, in_f, dev)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    wide = activations(m, in_f + 9, seed=3).to(dev)
+    for x in (wide[:, :in_f], wide[:, 3 : 3 + in_f]):
+        check(oracle, p, x.cpu(), product(lanes, x, out_f, in_f, bias.to(dev)), bias)
+
+
+def test_one_hot_rows_are_decoded_columns(oracle, dev):
+    out_f, in_f = 24, 1100
+    p, lanes = lay_out("real", out_f, in_f, dev)
+    w = bits_to_bf16(oracle.decode_packed_bf16(p)).reshape(out_f, in_f)
+    cols = [0, 31, 511, 512, 639, 1023, 1024, 1099]
+    for m in (1, 8):
+        for c0 in range(0, len(cols), m):
+            x = torch.zeros((m, in_f), dtype=torch.bfloat16)
+            for j in range(m):
+                x[j, cols[c0 + j]] = 1
+            y = product(lanes, x.to(dev), out_f, in_f).cpu()
+            for j in range(m):
+                assert torch.equal(y[j], w[:, cols[c0 + j]])
+
+
+def test_layer_rebuilds_its_lanes_with_its_state(dev):
+    """The layout is no part of the state dict and follows the packed streams that are loaded."""
+    from ixrun_amd.engine import StreamingLinear
+
+    layers = []
+    for seed in (1, 2):
+        v = int8_mix("only_l1", 64 * 1024, seed=seed)  # equal level counts: streams of equal length
+        layers.append(StreamingLinear(packed_from_int8(v, 64, 1024)))
+    assert not any("lane" in k for k in layers[0].state_dict())
+    x = activations(1, 1024, seed=9).to(dev)
+    assert not torch.equal(layers[0](x), layers[1](x))
+    layers[0].load_state_dict(layers[1].state_dict())
+    assert torch.equal(layers[0](x), layers[1](x))
+
+
+def test_malformed_lanes_are_refused(dev):
+    from ixrun_amd import _lib
+
+    L = _lib.lib()
+    p, lanes = lay_out("rare", 8, 512, dev)
+    x, y = activations(1, 512).to(dev), torch.empty((1, 8), dtype=torch.bfloat16, device=dev)
+    call = lambda s, m=1: L.ixh_lanes_gemv(C.byref(s), x.data_ptr(), 512, None, m, y.data_ptr(), 8, None, 0, None)
+    for field, value in (("bits", 6), ("plane_words", 100), ("n_quads", 0), ("exc_off", None), ("scale", None)):
+        s = _lib.IxhLanes.from_buffer_copy(lanes.struct)
+        setattr(s, field, value)
+        assert call(s) == -1, field
+    assert call(lanes.struct, 0) == -1 and call(lanes.struct, 17) == -1
+    assert L.ixh_lanes_plane_words(8, 512, 7) == -1 and L.ixh_lanes_cells(0, 512) == -1
