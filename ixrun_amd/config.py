@@ -28,3 +28,6 @@ CPU = torch.device("cpu")
 # Flat elements per entry of the block-offset tables returned by
 # precompute_block_offsets (reference ixrun/config.py:51).
 TRITON_BLOCK = 1024
+
+# Flat elements per rank-table unit of the specialised kernels (reference ixrun/fused.py:24).
+FUSED_TILE = 512

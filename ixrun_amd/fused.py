@@ -15,10 +15,9 @@ import numpy as np
 import torch
 
 from . import _lib
+from .config import FUSED_TILE
 
 __all__ = ["fused_gemv", "compute_row_prefixes", "FUSED_TILE"]
-
-FUSED_TILE = 512  # flat elements per rank-table unit of the specialised kernel
 
 
 # --------------------------------------------------------------------------- #
