@@ -5,12 +5,8 @@
 //                        k_enc_scale (one wave) turns the partial results into the bf16 scale
 //   2. k_enc_count<L>    quantise, count every level per 512-element unit; the counts are then summed into
 //                        the rank table (k_enc_tile_sums, k_enc_scan), which is the table the decoders take
-//   3. k_enc_pack<L>     quantise again, one wave per unit: the table says at which bit of every stream the
-//                        unit starts.  The first level is packed eight elements per lane (a wave prefix sum
-//                        places each lane's codes); what the first level leaves is queued in LDS in flat
-//                        order and taken through the other levels 64 elements at a time, ranked by ballots.
-//                        Each stream's piece is assembled in LDS and written as whole words; the two words a
-//                        piece may share with its neighbours are OR-ed in (the streams are cleared first)
+//   3. k_enc_pack<L>     quantise again and pack; the table says at which bit of every stream a wave's elements
+//                        start.  Only the words that two waves share are cleared (k_enc_borders) and OR-ed in
 // Between passes 2 and 3 the caller reads the level totals (last table entries) and sizes the streams.
 #include "ixh_dev.h"
 
@@ -19,7 +15,6 @@ namespace ixh {
 constexpr uint32_t kEncUnit = 512;          // elements per wave and step: eight per lane
 constexpr int kEncWaves = 4;                // waves per workgroup
 constexpr uint32_t kEncParts = 256;         // partial maxima of pass 1 (one per workgroup of 1024 lanes)
-constexpr uint32_t kEncWindow = kEncUnit * 7 / 32 + 4;  // LDS words for one unit's piece of the widest stream
 constexpr uint32_t kScanTile = 8192;        // table entries per workgroup of the scan
 
 // Eight consecutive bf16 starting at element p, widened to fp32 (zero past n).  Vector load when the address
@@ -199,18 +194,6 @@ __global__ void __launch_bounds__(1024) k_enc_scan(int32_t *table, uint32_t n_un
     if (blockIdx.x == 0 && tid == 0) row[0] = 0;
 }
 
-// every stream that is assembled with OR, in one launch
-struct EncClear {
-    uint32_t *dst[2 * (IXH_MAX_LEVELS - 1)];
-    uint32_t words[2 * (IXH_MAX_LEVELS - 1)];
-    int n;
-};
-
-__global__ void __launch_bounds__(256) k_enc_clear(EncClear c) {
-    for (int k = 0; k < c.n; ++k)
-        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < c.words[k]; i += gridDim.x * 256u) c.dst[k][i] = 0u;
-}
-
 // Destination of the encoder: the same fields as Dev, writable.
 struct EncOut {
     uint32_t *bm[IXH_MAX_LEVELS - 1];
@@ -221,198 +204,340 @@ struct EncOut {
     uint32_t last_bytes;
 };
 
-// OR `nbits` <= 64 bits of `value` into the window at bit `off`
-__device__ __forceinline__ void window_or(uint32_t *win, uint32_t off, uint64_t value, uint32_t nbits) {
-    if (nbits == 0) return;
-    const uint32_t wi = off >> 5, sh = off & 31u;
-    const uint64_t low = value << sh;
-    const uint32_t w0 = (uint32_t)low, w1 = (uint32_t)(low >> 32);
-    const uint32_t w2 = sh ? (uint32_t)(value >> (64u - sh)) : 0u;
-    if (w0) atomicOr(&win[wi], w0);
-    if (w1) atomicOr(&win[wi + 1], w1);
-    if (w2) atomicOr(&win[wi + 2], w2);
-}
-
-// the same for a value of at most 8 bits
-__device__ __forceinline__ void window_or_small(uint32_t *win, uint32_t off, uint32_t value) {
-    const uint32_t wi = off >> 5, sh = off & 31u;
-    const uint32_t w0 = value << sh, w1 = sh ? value >> (32u - sh) : 0u;
-    if (w0) atomicOr(&win[wi], w0);
-    if (w1) atomicOr(&win[wi + 1], w1);
-}
-
 // LDS traffic of this wave so far is visible to all its lanes after this
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
 
-// Write the window's words for the stream bits [bit0, bit1) and clear the window again.  The first and the last
-// word may also hold bits of the neighbouring units and are OR-ed into the cleared stream; the words between
-// belong to this unit alone.
-__device__ __forceinline__ void window_flush(uint32_t *win, uint32_t *dst, uint32_t dst_words, uint64_t bit0,
-                                             uint64_t bit1, uint32_t lane) {
-    wave_lds_sync();
-    if (bit1 > bit0) {
-        const uint32_t w_first = (uint32_t)(bit0 >> 5);
-        const uint32_t n_words = (uint32_t)((bit1 - 1) >> 5) - w_first + 1;
-        for (uint32_t j = lane; j < n_words; j += kWave) {
-            const uint32_t val = win[j];
-            win[j] = 0u;
-            if (w_first + j < dst_words) {
-                if (j == 0 || j == n_words - 1) {
-                    if (val) atomicOr(&dst[w_first + j], val);
-                } else {
-                    dst[w_first + j] = val;
-                }
-            }
+// ---------------------------------------------------------------------------------------------------------------
+// k_enc_pack<L>: bound by vector issue: of 5120 x 17408 at levels 3, 5, 8 about 700 instructions a wave and span, 68 us
+// (heavy tails) to 74 us (55 / 40 / 5 %); the 240 MB that it moves take 47.
+//
+// A wave takes spans of four units, 2048 elements, 32 consecutive ones a lane, so one prefix sum over the lanes serves them
+// all and a lane's membership bits are a whole word of bitmap 0.  Every element goes to LDS as one byte, value + 128: those
+// of the level to its dense run, the others to a second one, in order; the next level splits that second run the same
+// way, 16 bytes a lane.  A dense run starts in LDS where its first code falls in the stream's groups of 32 codes, so a
+// lane turns 32 bytes into `bits` whole words of the stream at once.  Only the groups (and bitmap words) that a wave
+// shares with its neighbours are OR-ed into memory; k_enc_borders clears those beforehand.
+// (Before, a wave packed 512 elements with an LDS atomic per code and a flush per stream: 279 us.)
+// ---------------------------------------------------------------------------------------------------------------
+constexpr uint32_t kEncSpan = 2048, kEncSpanUnits = kEncSpan / kEncUnit;
+constexpr uint32_t kEncBuf = kEncSpan + 256;  // two runs with their margins
+constexpr uint32_t dense_at = 32u;            // where a dense run's groups start in it
+
+// Spans per wave: a wave that goes on hands its unfinished groups to its next span in registers, and only its first and last
+// cost atomics (one span each: 107 .. 175 us instead of 68 .. 74).  As many as leave the chip some 4096 waves, at most 8.
+constexpr uint32_t kEncMaxSpans = 8, kEncFill = 4096;
+
+// level i's rank at unit `u`, and the index of the unit's first element in bitmap i
+struct EncRanks {
+    const int32_t *table;
+    uint32_t entries, n;
+    __device__ __forceinline__ uint32_t rank(int i, uint32_t u) const { return (uint32_t)table[(size_t)i * entries + u]; }
+    __device__ __forceinline__ uint32_t space(int i, uint32_t u) const {
+        uint32_t at = min(u * kEncUnit, n);
+        for (int j = 0; j < i; ++j) at -= rank(j, u);
+        return at;
+    }
+};
+
+// what a value's magnitude has to stay below to round into a level of `bits`: the thresholds are odd, so a tie goes up to
+// the next level, but for one bit (threshold 0), where it goes down to 0
+__device__ __forceinline__ float edge_of(int bits) { return (float)threshold_of(bits) + (bits == 1 ? 0.50012207f : 0.5f); }
+
+// clears what neighbouring waves share: of every stream the group of 32 codes that a wave's first code falls into,
+// of every bitmap but the first the word of its first bit; and any words behind the last code
+__global__ void __launch_bounds__(256)
+k_enc_borders(EncLevels lv, const int32_t *__restrict__ table, uint32_t n, uint32_t n_units, uint32_t wave_units, EncOut out) {
+    const uint32_t s = blockIdx.x * 256u + threadIdx.x, u = min(s * wave_units, n_units);
+    const uint32_t n_waves = (n_units + wave_units - 1) / wave_units;
+    const EncRanks r{table, n_units + 1, n};
+    for (int i = 0; i < lv.n_levels - 1; ++i) {
+        for (uint32_t k = (r.space(i, n_units) + 31u) / 32u + s; k < out.bm_words[i]; k += gridDim.x * 256u) out.bm[i][k] = 0u;
+        const uint64_t used = ((uint64_t)r.rank(i, n_units) * (uint32_t)lv.bits[i] + 31u) / 32u;
+        for (uint64_t k = used + s; k < out.st_words[i]; k += gridDim.x * 256u) out.st[i][k] = 0u;
+        if (s > n_waves) continue;
+        const uint32_t b = (uint32_t)lv.bits[i], word = (r.rank(i, u) >> 5) * b;
+        for (uint32_t k = 0; k < b; ++k)
+            if (word + k < out.st_words[i]) out.st[i][word + k] = 0u;
+        if (i > 0) {
+            const uint32_t at = r.space(i, u) >> 5;
+            if (at < out.bm_words[i]) out.bm[i][at] = 0u;
         }
     }
-    wave_lds_sync();
 }
 
-constexpr uint32_t kEncBmWindow = kEncUnit / 32 + 4;  // LDS words for one unit's piece of a bitmap
+// 32 codes (bytes, bias too high) to B words: four bytes to 4 B bits at a time
+template <int B>
+__device__ __forceinline__ void enc_words(const uint32_t (&x)[8], uint32_t bias4, uint32_t (&w)[B]) {
+#pragma unroll
+    for (int k = 0; k < B; ++k) w[k] = 0u;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const uint32_t v = x[c] - bias4, pair = ((1u << (2 * B)) - 1u) * 0x10001u;
+        uint32_t four;
+        if (B <= 4) {  // a shifted byte leaves nothing of its neighbour below it
+            const uint32_t two = (v | (v >> (8 - B))) & pair;
+            four = (two | (two >> (16 - 2 * B))) & ((1u << (4 * B)) - 1u);
+        } else {
+            const uint32_t two = (v & 0x00ff00ffu) | ((v & 0xff00ff00u) >> (8 - B));
+            four = ((two >> 16) << (2 * B)) | (two & 0xffffu);
+        }
+        const int bit = 4 * B * c, d = bit >> 5, sh = bit & 31;
+        w[d] |= four << sh;
+        if (sh + 4 * B > 32) w[d + 1] |= four >> (32 - sh);
+    }
+}
+
+// `groups` groups of 32 codes (bytes in LDS at `run`) to the stream from group g0 on; `first` and `last` are the groups
+// that the wave shares with its neighbours
+template <int B>
+__device__ __forceinline__ void enc_store_run(const uint8_t *run, uint32_t g0, uint32_t groups, uint32_t first, uint32_t last,
+                                              uint32_t *dst, uint32_t dst_words, uint32_t lane) {
+    const uint32_t bias4 = (128u - ((1u << (B - 1)) - 1u)) * 0x01010101u;
+    const bool inside = g0 > first && g0 + groups <= last && (g0 + groups) * B <= dst_words;
+    for (uint32_t g = lane; g < groups; g += kWave) {
+        const uint4 lo = *reinterpret_cast<const uint4 *>(run + g * 32u), hi = *reinterpret_cast<const uint4 *>(run + g * 32u + 16u);
+        const uint32_t x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        uint32_t w[B];
+        enc_words<B>(x, bias4, w);
+        const uint32_t at = (g0 + g) * B;
+        if (inside) {
+#pragma unroll
+            for (int k = 0; k < B; ++k) dst[at + k] = w[k];
+        } else if (g0 + g == first || g0 + g == last) {
+#pragma unroll
+            for (int k = 0; k < B; ++k)
+                if (at + k < dst_words && w[k]) atomicOr(&dst[at + k], w[k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < B; ++k)
+                if (at + k < dst_words) dst[at + k] = w[k];
+        }
+    }
+}
+__device__ __forceinline__ void enc_store_run_of(uint32_t b, const uint8_t *run, uint32_t g0, uint32_t groups, uint32_t first,
+                                                 uint32_t last, uint32_t *dst, uint32_t dst_words, uint32_t lane) {
+    switch (b) {  // uniform
+        case 1: enc_store_run<1>(run, g0, groups, first, last, dst, dst_words, lane); break;
+        case 2: enc_store_run<2>(run, g0, groups, first, last, dst, dst_words, lane); break;
+        case 3: enc_store_run<3>(run, g0, groups, first, last, dst, dst_words, lane); break;
+        case 4: enc_store_run<4>(run, g0, groups, first, last, dst, dst_words, lane); break;
+        case 5: enc_store_run<5>(run, g0, groups, first, last, dst, dst_words, lane); break;
+        case 6: enc_store_run<6>(run, g0, groups, first, last, dst, dst_words, lane); break;
+        default: enc_store_run<7>(run, g0, groups, first, last, dst, dst_words, lane); break;
+    }
+}
+
+// bits = 2 * bits + in, one instruction (the compiler makes three of it)
+__device__ __forceinline__ void enc_shift_in(uint32_t &bits, uint64_t in) {
+    uint64_t carry;
+    asm("s_nop 1\n\tv_addc_co_u32_e64 %0, %1, %0, %0, %2" : "+v"(bits), "=&s"(carry) : "s"(in));
+}
+
+// One element's byte to the next place of its run, where `to1` and `to0` are the LDS addresses of the two runs' next bytes
+// less t: the one taken moves on, and both fall behind t by one.  (As above: three instructions for seven.)
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+__device__ __forceinline__ uint32_t lds_address(uint8_t *p) { return (uint32_t)(uintptr_t)(lds_u8 *)p; }
+__device__ __forceinline__ void enc_put(uint32_t &to1, uint32_t &to0, uint64_t in, int t, uint8_t byte) {
+    uint32_t to;
+    uint64_t carry;
+    asm("s_nop 1\n\tv_cndmask_b32_e64 %2, %1, %0, %4\n\tv_addc_co_u32_e64 %0, %3, -1, %0, %4\n\tv_subbrev_co_u32_e64 %1, %3, 0, %1, %4"
+        : "+v"(to1), "+v"(to0), "=&v"(to), "=&s"(carry) : "s"(in));
+    ((lds_u8 *)(uintptr_t)to)[t] = byte;
+}
+
+// 32 weights from element p on, as pairs; infinite past n, which is in no level but the last.  `whole`: all of the wave's are there, at a multiple of 16 bytes.
+__device__ __forceinline__ void load32(const uint16_t *__restrict__ w, uint32_t p, uint32_t n, bool whole, uint32_t (&d)[16]) {
+    if (whole) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint4 q = *reinterpret_cast<const uint4 *>(w + p + 8 * k);
+            d[4 * k] = q.x; d[4 * k + 1] = q.y; d[4 * k + 2] = q.z; d[4 * k + 3] = q.w;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            d[k] = p + 2 * k < n ? w[p + 2 * k] : 0x7f80u;
+            d[k] |= (p + 2 * k + 1 < n ? (uint32_t)w[p + 2 * k + 1] : 0x7f80u) << 16;
+        }
+    }
+}
 
 template <int L>
 __global__ void __launch_bounds__(kWave *kEncWaves)
-k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, const uint16_t *__restrict__ scale_in,
-           EncLevels lv, const int32_t *__restrict__ table, EncOut out) {
-    __shared__ uint32_t windows[kEncWaves][kEncWindow];
-    __shared__ uint32_t bm_windows[kEncWaves][kEncBmWindow];
-    __shared__ uint8_t queues[kEncWaves][kEncUnit];
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t *win = windows[wave], *bm_win = bm_windows[wave];
-    uint8_t *queue = queues[wave];
-    for (uint32_t j = lane; j < kEncWindow; j += kWave) win[j] = 0u;
-    if (lane < kEncBmWindow) bm_win[lane] = 0u;
-    const uint32_t u = blockIdx.x * kEncWaves + wave;
-    if (u >= n_units) return;
-    const float inv_scale = __fdiv_rn(1.0f, bf16_bits_to_f32(*scale_in));
+k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, uint32_t wave_units,
+           const uint16_t *__restrict__ scale_in, EncLevels lv, const int32_t *__restrict__ table, EncOut out) {
+    __shared__ __attribute__((aligned(32))) uint8_t bufs[kEncWaves][2][kEncBuf];
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t u_first = (blockIdx.x * kEncWaves + wave) * wave_units, u_end = min(u_first + wave_units, n_units);
+    if (u_first >= n_units) return;
+    const EncRanks ranks{table, n_units + 1, n};
     const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
-    const uint32_t entries = n_units + 1;
-    // the unit's first rank in every level and the next unit's: requested now, needed after the first level
-    uint32_t ranks0[L - 1], ranks1[L - 1];
+    const float inv_scale = __fdiv_rn(1.0f, bf16_bits_to_f32(*scale_in));
+    // r0, space[i]: ranks and bitmap index at the span's start; g_*, w_*: the groups and bitmap words shared with the
+    // neighbouring waves; carry, bm_carry: what the span before left of an unfinished group and bitmap word
+    uint32_t r0[L - 1], g_first[L - 1], g_last[L - 1], carry[L - 1], w_first[L - 1], w_last[L - 1], bm_carry[L - 1];
 #pragma unroll
     for (int i = 0; i < L - 1; ++i) {
-        ranks0[i] = (uint32_t)table[(size_t)i * entries + u];
-        ranks1[i] = (uint32_t)table[(size_t)i * entries + u + 1];
+        r0[i] = ranks.rank(i, u_first);
+        g_first[i] = r0[i] / 32u;
+        g_last[i] = ranks.rank(i, u_end) / 32u;
+        w_first[i] = ranks.space(i, u_first) / 32u;
+        w_last[i] = ranks.space(i, u_end) / 32u;
+        carry[i] = 128u - (uint32_t)threshold_of(lv.bits[i]);
+        bm_carry[i] = 0u;
     }
-    const uint32_t e0 = u * kEncUnit, e1 = min(e0 + kEncUnit, n);  // the unit's elements
-    const uint32_t p = e0 + lane * 8u;
-    float f[8];
-    load8(w, min(p, n), n, aligned, f);
-    const uint32_t n_valid = p < e1 ? min(8u, e1 - p) : 0u;
-    const uint32_t valid = (1u << n_valid) - 1u;
+    for (uint32_t u0 = u_first; u0 < u_end; u0 += kEncSpanUnits) {
+        const uint32_t u1 = min(u0 + kEncSpanUnits, n_units);
+        const bool final = u1 == u_end;
+        const uint32_t e0 = u0 * kEncUnit, e1 = min(e0 + kEncSpan, n);
+        uint32_t r1[L - 1];
+#pragma unroll
+        for (int i = 0; i < L - 1; ++i) r1[i] = ranks.rank(i, u1);
+        uint32_t left = e1 - e0;  // (the counts below come from the caller's table: held to the span)
 
-    // ---- first level, eight elements per lane ----
-    const uint32_t b0 = (uint32_t)lv.bits[0];
-    const int thr0 = threshold_of((int)b0);
-    int q[8];
-    uint32_t above = 0;  // bit t: element t is not in the first level
+        // ---- quantise ----
+        const uint32_t p = e0 + lane * 32u;
+        uint32_t d[16], member = 0;
+        load32(w, p, n, aligned && e0 + kEncSpan <= n, d);
+        // (see quantise: the sum with 3072 restores exact ties)
+        float v[32];
+        uint64_t in[32];
+        const float edge0 = edge_of(lv.bits[0]);
 #pragma unroll
-    for (int t = 7; t >= 0; --t) {
-        const float r = quantise(f[t], inv_scale);
-        q[t] = (int)r;
-        above = (above << 1) | (fabsf(r) > (float)thr0 ? 1u : 0u);
-    }
-    const uint32_t member = ~above & valid;  // elements past n were loaded as zero and are not above
-    // bitmap 0 is indexed by the flat element: the lane's byte, four lanes to a word, whole words to memory
-    reinterpret_cast<uint8_t *>(bm_win)[lane] = (uint8_t)member;
-    wave_lds_sync();
-    if (lane < kEncUnit / 32) {
-        const uint32_t word = bm_win[lane], at = e0 / 32 + lane;
-        bm_win[lane] = 0u;
-        if (at < (n + 31u) / 32u && at < out.bm_words[0]) out.bm[0][at] = word;
-    }
-    uint32_t n_codes = 0;
-    uint64_t codes = 0;
-    if (b0 <= 4) {  // eight codes fit one register
-        uint32_t c32 = 0, sh = 0;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const bool m = (member >> t) & 1u;
-            c32 |= (m ? (uint32_t)(q[t] + thr0) : 0u) << sh;
-            sh += m ? b0 : 0u;
+        for (int t = 0; t < 32; ++t) {
+            const float f = __uint_as_float(t & 1 ? d[t / 2] & 0xffff0000u : d[t / 2] << 16);
+            v[t] = __fmaf_rn(f, inv_scale, 3072.0f) - 3072.0f;
+            in[t] = __builtin_amdgcn_ballot_w64(fabsf(v[t]) < edge0);
+            enc_shift_in(member, in[t]);
         }
-        codes = c32;
-        n_codes = sh;
-    } else {  // four and four, joined once
-        uint32_t half[2] = {0, 0}, sh[2] = {0, 0};
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const bool m = (member >> t) & 1u;
-            half[t >> 2] |= (m ? (uint32_t)(q[t] + thr0) : 0u) << sh[t >> 2];
-            sh[t >> 2] += m ? b0 : 0u;
-        }
-        codes = (uint64_t)half[0] | ((uint64_t)half[1] << sh[0]);
-        n_codes = sh[0] + sh[1];
-    }  // n_codes: bits of this lane's codes
-    const uint32_t n_above = (uint32_t)__popc(above);
-    const uint32_t incl = wave_scan_inclusive(n_codes | (n_above << 16));
-    const uint32_t bits_before = (incl & 0xffffu) - n_codes, above_before = (incl >> 16) - n_above;
-    const uint32_t total_above = (uint32_t)__builtin_amdgcn_readlane((int)(incl >> 16), 63);
-    uint32_t rank0 = ranks0[0], rank1 = ranks1[0];
-    {
-        const uint64_t bit0 = (uint64_t)rank0 * b0, bit1 = (uint64_t)rank1 * b0;
-        window_or(win, ((uint32_t)bit0 & 31u) + bits_before, codes, n_codes);
-        window_flush(win, out.st[0], out.st_words[0], bit0, bit1, lane);
-    }
-    if (total_above == 0) return;  // the whole wave
+        member = __brev(member);  // bit t: element t is in the first level
+        if (p < e1 && p / 32u < out.bm_words[0]) out.bm[0][p / 32u] = member;
 
-    // ---- what the first level left, queued in flat order as v + 128 ----
-    {
-        uint32_t at = above_before;
+        // ---- first level: codes to the dense run in buffer 0, the rest behind it (what lies past the last element
+        // follows them and is overwritten by the margin) ----
+        uint8_t *buf = bufs[wave][0], *other = bufs[wave][1];
+        const uint32_t cnt = (uint32_t)__popc(member);
+        const uint32_t before = wave_scan_inclusive(cnt) - cnt;
+        uint32_t n_i = min(r1[0] - r0[0], left);
+        r1[0] = r0[0] + n_i;
+        left -= n_i;
+        uint32_t rest = ((dense_at + 31u + (r0[0] & 31u) + n_i) & ~31u) + 32u;  // the other run's start
+        uint32_t space0 = e0 - r0[0], space1 = space0 + left;                   // its elements' indexes in the next bitmap
+        {
+            uint32_t to1 = lds_address(buf) + dense_at + (r0[0] & 31u) + before;
+            uint32_t to0 = lds_address(buf) + rest + (space0 & 31u) + lane * 32u - before;
+            // adding 1.5 * 2^23 rounds half to even and leaves the integer in the low bits
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            if ((above >> t) & 1u) queue[at++] = (uint8_t)(q[t] + 128);
+            for (int t = 0; t < 32; ++t) enc_put(to1, to0, in[t], t, (uint8_t)__float_as_uint(v[t] + (12582912.0f + 128.0f)));
         }
-    }
-    wave_lds_sync();
-    // first index of this unit and of the next one in the index space of the current level's bitmap
-    uint32_t space0 = e0 - rank0, space1 = e1 - rank1;
-    int thr_below = thr0;
-#pragma unroll
-    for (int i = 1; i < L - 1; ++i) {
-        const uint32_t b = (uint32_t)lv.bits[i];
-        const int thr_i = threshold_of((int)b);
-        rank0 = ranks0[i];
-        rank1 = ranks1[i];
-        const uint64_t bit0 = (uint64_t)rank0 * b, bit1 = (uint64_t)rank1 * b;
-        uint32_t seen_alive = space0 & 31u, seen_codes = (uint32_t)bit0 & 31u;  // window positions, in bits
-        if (space1 > space0) {
-            for (uint32_t s = 0; s < total_above; s += kWave) {
-                const bool have = s + lane < total_above;
-                const int v = have ? (int)queue[s + lane] - 128 : 0;
-                const int a = v < 0 ? -v : v;
-                const bool alive = have && a > thr_below;
-                const bool mine = alive && a <= thr_i;
-                const uint64_t alive_mask = __ballot(alive), mine_mask = __ballot(mine);
-                if (mine) {
-                    window_or_small(bm_win, seen_alive + lanes_below(alive_mask), 1u);
-                    window_or_small(win, seen_codes + lanes_below(mine_mask) * b, (uint32_t)(v + thr_i));
-                }
-                seen_alive += (uint32_t)__popcll(alive_mask);
-                seen_codes += (uint32_t)__popcll(mine_mask) * b;
+        // In front of a dense run: the codes of its unfinished group; behind it code 0.  Around the other run: value 0, a
+        // member of every level.
+        auto margins = [&](uint8_t *b, uint32_t at, uint32_t first, uint32_t count, uint32_t front, uint32_t back) {
+            const uint32_t off = first & 31u;
+            if (lane < 32u) {
+                if (lane < off) b[at + lane] = (uint8_t)front;
+                b[at + off + count + lane] = (uint8_t)back;
             }
+        };
+        // a level's run to its stream, the unfinished group kept for the next span or, at the wave's end, stored
+        auto store_level = [&](int i, const uint8_t *b) {
+            const uint32_t whole = r1[i] / 32u - r0[i] / 32u;
+            enc_store_run_of((uint32_t)lv.bits[i], b + dense_at, r0[i] / 32u, final ? (r1[i] + 31u) / 32u - r0[i] / 32u : whole,
+                             g_first[i], g_last[i], out.st[i], out.st_words[i], lane);
+            carry[i] = b[dense_at + whole * 32u + (lane & 31u)];
+        };
+        margins(buf, dense_at, r0[0], n_i, carry[0], 128u - (uint32_t)threshold_of(lv.bits[0]));
+        margins(buf, rest, space0, left, 128u, 128u);
+        wave_lds_sync();
+        store_level(0, buf);
+
+        // ---- the other levels, 16 elements a lane and turn; margin elements pass as members in front of the first and
+        // behind the last code, where the run's own margins overwrite them ----
+#pragma unroll
+        for (int i = 1; i < L - 1; ++i) {
+            if (space1 == space0 && !final) {  // nothing came this far: what is unfinished stays so
+                r1[i] = r0[i];
+                continue;
+            }
+            const uint32_t off = space0 & 31u, end = off + (space1 - space0);
+            const uint32_t thr = (uint32_t)threshold_of(lv.bits[i]);
+            n_i = min(r1[i] - r0[i], left);
+            r1[i] = r0[i] + n_i;
+            left -= n_i;
+            const uint32_t rest_i = ((dense_at + 31u + (r0[i] & 31u) + n_i) & ~31u) + 32u;
+            const uint32_t next0 = space0 - r0[i], next1 = next0 + left;
+            uint32_t base1 = dense_at + (r0[i] & 31u) - off, base0 = rest_i + (next0 & 31u);
+            uint32_t unfinished = 0;
+            for (uint32_t s = 0; s < end; s += 1024u) {
+                const uint32_t at = s + 16u * lane;
+                uint32_t bits = 0, n_here = 0, x[4] = {0, 0, 0, 0}, m[4] = {0, 0, 0, 0};
+                if (at < end) {
+                    const uint4 q = *reinterpret_cast<const uint4 *>(buf + rest + at);
+                    x[0] = q.x; x[1] = q.y; x[2] = q.z; x[3] = q.w;
+                    n_here = 16u;
+                    // four bytes at a time: bit 7 of m set where 128 - threshold <= byte <= 128 + threshold
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const uint32_t low = x[k] & 0x7f7f7f7fu;
+                        m[k] = ((low + thr * 0x01010101u) | x[k]) & ~((low + (127u - thr) * 0x01010101u) & x[k]) & 0x80808080u;
+                    }
+                    bits = (__builtin_amdgcn_udot4(m[1], 0x80402010u, __builtin_amdgcn_udot4(m[0], 0x08040201u, 0u, false), false) >> 7) |
+                           (__builtin_amdgcn_udot4(m[3], 0x80402010u, __builtin_amdgcn_udot4(m[2], 0x08040201u, 0u, false), false) >> 7 << 8);
+                }
+                const uint32_t c1 = (uint32_t)__popc(bits), c0 = n_here - c1;
+                const uint32_t incl = wave_scan_inclusive(c1 | (c0 << 16));
+                if (at < end) {
+                    uint32_t to1 = lds_address(other) + base1 + (incl & 0xffffu) - c1;
+                    uint32_t to0 = lds_address(other) + base0 + (incl >> 16) - c0;
+#pragma unroll
+                    for (int t = 0; t < 16; ++t)
+                        enc_put(to1, to0, __builtin_amdgcn_ballot_w64((m[t / 4] & (0x80u << (8 * (t & 3)))) != 0), t,
+                                (uint8_t)(x[t / 4] >> (8 * (t & 3))));
+                }
+                const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+                base1 += total & 0xffffu;
+                base0 += total >> 16;
+                // bitmap i: the bits of this lane's elements that are the span's, two lanes to a word
+                uint32_t mine = at < end ? bits : 0u;
+                if (at < off) mine &= off - at < 16u ? ~0u << (off - at) : 0u;
+                if (at + 16u > end) mine &= at < end ? (1u << (end - at)) - 1u : 0u;
+                uint32_t word = (mine & 0xffffu) | ((uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0xB1, 0xf, 0xf, true) << 16);
+                if (at == 0) word |= bm_carry[i];
+                const uint32_t wi = space0 / 32u + (at >> 5);
+                const bool last_word = at >= (end & ~31u);
+                if ((end & ~31u) - s < 1024u)
+                    unfinished = (uint32_t)__builtin_amdgcn_readlane((int)word, (int)(((end & ~31u) - s) >> 4));
+                if ((lane & 1u) == 0 && at < end && wi < out.bm_words[i] && (final || !last_word)) {
+                    if (wi == w_first[i] || wi == w_last[i]) {
+                        if (word) atomicOr(&out.bm[i][wi], word);
+                    } else {
+                        out.bm[i][wi] = word;
+                    }
+                }
+            }
+            bm_carry[i] = unfinished;
+            margins(other, dense_at, r0[i], n_i, carry[i], 128u - (uint32_t)threshold_of(lv.bits[i]));
+            margins(other, rest_i, next0, left, 128u, 128u);
+            wave_lds_sync();
+            store_level(i, other);
+            uint8_t *const swap = buf;
+            buf = other;
+            other = swap;
+            rest = rest_i;
+            space0 = next0;
+            space1 = next1;
         }
-        window_flush(bm_win, out.bm[i], out.bm_words[i], space0, space1, lane);
-        window_flush(win, out.st[i], out.st_words[i], bit0, bit1, lane);
-        space0 -= rank0;
-        space1 -= rank1;
-        thr_below = thr_i;
-    }
-    // last level: one byte per element left over (quantize.py:84-86)
-    if (space1 > space0) {
-        uint32_t at = space0;
-        for (uint32_t s = 0; s < total_above; s += kWave) {
-            const bool have = s + lane < total_above;
-            const int v = have ? (int)queue[s + lane] - 128 : 0;
-            const bool mine = have && (v < 0 ? -v : v) > thr_below;
-            const uint64_t mine_mask = __ballot(mine);
-            const uint32_t dst = at + lanes_below(mine_mask);
-            if (mine && dst < out.last_bytes) out.last[dst] = (uint8_t)(v + 127);
-            at += (uint32_t)__popcll(mine_mask);
-        }
+        // ---- last level: one byte, value + 127, per element left over (quantize.py:84-86) ----
+        for (uint32_t k = lane; k < space1 - space0; k += kWave)
+            if (space0 + k < out.last_bytes)
+                out.last[space0 + k] = (uint8_t)(max((int)buf[rest + (space0 & 31u) + k], 1) - 1);
+#pragma unroll
+        for (int i = 0; i < L - 1; ++i) r0[i] = r1[i];
+        wave_lds_sync();
     }
 }
 
@@ -457,9 +582,10 @@ int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *b
 
 template <int L>
 static void pack_launch(const uint16_t *w, uint32_t n, uint32_t n_units, const uint16_t *scale, const EncLevels &lv,
-                        const int32_t *table, const EncOut &out, hipStream_t s) {
-    hipLaunchKernelGGL(k_enc_pack<L>, dim3((n_units + kEncWaves - 1) / kEncWaves), dim3(kWave * kEncWaves), 0, s, w, n,
-                       n_units, scale, lv, table, out);
+                        uint32_t wave_units, const int32_t *table, const EncOut &out, hipStream_t s) {
+    const uint32_t waves = (n_units + wave_units - 1) / wave_units;
+    hipLaunchKernelGGL(k_enc_pack<L>, dim3((waves + kEncWaves - 1) / kEncWaves), dim3(kWave * kEncWaves), 0, s, w, n, n_units,
+                       wave_units, scale, lv, table, out);
 }
 
 int launch_encode_pack(const uint16_t *w, const Dev &P, const int32_t *table, hipStream_t s) {
@@ -477,31 +603,19 @@ int launch_encode_pack(const uint16_t *w, const Dev &P, const int32_t *table, hi
     }
     out.last = const_cast<uint8_t *>(P.last);
     out.last_bytes = P.last_bytes;
-    EncClear clr;
-    clr.n = 0;
-    uint32_t most = 0;
-    for (int i = 0; i < P.n_levels - 1; ++i) {
-        if (out.bm_words[i] && i > 0) {  // bitmap 0 is written in whole words
-            clr.dst[clr.n] = out.bm[i];
-            clr.words[clr.n++] = out.bm_words[i];
-            most = max(most, out.bm_words[i]);
-        }
-        if (out.st_words[i]) {
-            clr.dst[clr.n] = out.st[i];
-            clr.words[clr.n++] = out.st_words[i];
-            most = max(most, out.st_words[i]);
-        }
-    }
-    if (clr.n) hipLaunchKernelGGL(k_enc_clear, dim3(min(2048u, (most + 255u) / 256u)), dim3(256), 0, s, clr);
+    const uint32_t spans = (n_units + kEncSpanUnits - 1) / kEncSpanUnits;
+    const uint32_t wave_units = max(1u, min(kEncMaxSpans, spans / kEncFill)) * kEncSpanUnits;
+    const uint32_t waves = (n_units + wave_units - 1) / wave_units;
+    hipLaunchKernelGGL(k_enc_borders, dim3((waves + 256u) / 256u), dim3(256), 0, s, lv, table, n, n_units, wave_units, out);
     if (n_units != 0) {
         switch (P.n_levels) {
-            case 2: pack_launch<2>(w, n, n_units, P.scale, lv, table, out, s); break;
-            case 3: pack_launch<3>(w, n, n_units, P.scale, lv, table, out, s); break;
-            case 4: pack_launch<4>(w, n, n_units, P.scale, lv, table, out, s); break;
-            case 5: pack_launch<5>(w, n, n_units, P.scale, lv, table, out, s); break;
-            case 6: pack_launch<6>(w, n, n_units, P.scale, lv, table, out, s); break;
-            case 7: pack_launch<7>(w, n, n_units, P.scale, lv, table, out, s); break;
-            default: pack_launch<8>(w, n, n_units, P.scale, lv, table, out, s); break;
+            case 2: pack_launch<2>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
+            case 3: pack_launch<3>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
+            case 4: pack_launch<4>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
+            case 5: pack_launch<5>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
+            case 6: pack_launch<6>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
+            case 7: pack_launch<7>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
+            default: pack_launch<8>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
         }
     }
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;

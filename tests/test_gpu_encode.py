@@ -183,3 +183,11 @@ def test_encode_full_size_layer(oracle, dev):
     w = student_t_weight(5120, 17408, seed=0)
     p, q = check_against_oracle(oracle, dev, w, (3, 5, 8))
     assert np.array_equal(decode_int8(p, device=dev).cpu().numpy().reshape(-1), q)
+
+
+@pytest.mark.parametrize("level_bits", [(3, 5, 8), (1, 8), (3, 4, 5, 6, 8), (1, 2, 3, 4, 5, 6, 7, 8)])
+@pytest.mark.parametrize("n", [2016, 2047, 2048, 2049, 2080, 8191, 8192, 8193, 12 * 2048 + 31])
+@pytest.mark.parametrize("kind", ["student_t", "half_steps", "zeros", "all_extreme"])
+def test_encode_span_edges(oracle, dev, n, level_bits, kind):
+    """Around the 2048 elements of a wave and the 8192 of a workgroup, runs that are full, empty or split anywhere."""
+    check_against_oracle(oracle, dev, make_weight(kind, 1, n), level_bits)
