@@ -231,7 +231,7 @@ int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
 size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m);
 
 /*
- * The encoder on the device, in two calls because the stream lengths depend on the data.
+ * The encoder on the device, in two steps because the stream lengths depend on the data.
  * Together they replace int8x_quantize (ixrun/quantize.py:41-122, with pack_bits_stream
  * and pack_bitmap of ixrun/bitpack.py:13-61, :87-89) for a bf16 weight that is already in
  * device memory, and write byte for byte what that CPU encoder writes; the rank table of
@@ -242,7 +242,7 @@ size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m);
  *   prefix       the chunk-512 rank table, (n_levels-1) rows of E = ixh_prefix_entries(N, 512)
  *                entries; the last entry of row i, prefix[i*E + E-1], is the number of level-i
  *                elements ("counts[i]"); the last level holds what is left of N
- * The caller reads those totals (its own synchronisation), then allocates, for i < n_levels-1,
+ * The caller reads those totals (its own synchronisation, or the pair below), then allocates, for i < n_levels-1,
  * bitmap i of ceil((N - counts[0] - .. - counts[i-1]) / 32) words and stream i of
  * ceil(counts[i] * level_bits[i] / 32) words, and counts[n_levels-1] bytes for the last level.
  *
@@ -255,6 +255,18 @@ size_t ixh_encode_workspace_bytes(int64_t out_f, int64_t in_f, int32_t n_levels)
 int ixh_encode_scan(const uint16_t *w, int64_t out_f, int64_t in_f, int32_t n_levels, const int32_t *level_bits,
                     uint16_t *scale, int32_t *prefix, void *workspace, size_t workspace_bytes,
                     ixh_stream_t stream);
+
+/*
+ * ixh_encode_scan_counts: the same, and the totals are also written to host_counts: n_levels-1
+ * entries of pinned host memory that the device can write, set to -1 before the launch.
+ * ixh_encode_wait: returns when all of them have arrived (sooner than the stream's completion
+ * would be seen), or with IXH_ELAUNCH when the stream fails or drains without them.  The only
+ * call here that waits.
+ */
+int ixh_encode_scan_counts(const uint16_t *w, int64_t out_f, int64_t in_f, int32_t n_levels,
+                           const int32_t *level_bits, uint16_t *scale, int32_t *prefix, void *workspace,
+                           size_t workspace_bytes, int64_t *host_counts, ixh_stream_t stream);
+int ixh_encode_wait(const int64_t *host_counts, int32_t n_counts, ixh_stream_t stream);
 
 int ixh_encode_pack(const uint16_t *w, const IxhPacked *dst, const int32_t *prefix, ixh_stream_t stream);
 

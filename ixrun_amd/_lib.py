@@ -73,7 +73,8 @@ _lib = None
 EXPORTS = (
     "ixh_version", "ixh_last_error", "ixh_prefix_entries", "ixh_prefix_build", "ixh_decode",
     "ixh_gemv", "ixh_gemv_workspace_bytes", "ixh_gemv_noalloc", "ixh_gemm", "ixh_gemm_workspace_bytes",
-    "ixh_encode_workspace_bytes", "ixh_encode_scan", "ixh_encode_pack", "ixh_decode_gs",
+    "ixh_encode_workspace_bytes", "ixh_encode_scan", "ixh_encode_scan_counts", "ixh_encode_wait", "ixh_encode_pack",
+    "ixh_decode_gs",
     "ixh_lanes_plane_words", "ixh_lanes_cells", "ixh_lanes_pack", "ixh_lanes_list", "ixh_lanes_gemv",
     "ixh_lanes_gemv_workspace_bytes",
 )
@@ -129,6 +130,10 @@ def lib() -> C.CDLL:
             C.c_void_p, C.c_int64, C.c_int64, C.c_int32, C.POINTER(C.c_int32), C.c_void_p, C.c_void_p,
             C.c_void_p, C.c_size_t, C.c_void_p,
         ]
+        L.ixh_encode_scan_counts.restype = C.c_int
+        L.ixh_encode_scan_counts.argtypes = L.ixh_encode_scan.argtypes[:-1] + [C.c_void_p, C.c_void_p]
+        L.ixh_encode_wait.restype = C.c_int
+        L.ixh_encode_wait.argtypes = [C.c_void_p, C.c_int32, C.c_void_p]
         L.ixh_encode_pack.restype = C.c_int
         L.ixh_encode_pack.argtypes = [C.c_void_p, C.POINTER(IxhPacked), C.c_void_p, C.c_void_p]
         L.ixh_lanes_plane_words.restype = C.c_int64
@@ -164,8 +169,15 @@ def set_option(name: str, value) -> None:
     check(lib().ixh_set_option(name.encode(), int(value)))
 
 
+try:  # the handle itself: no Stream object per call
+    _raw_stream = torch._C._cuda_getCurrentRawStream
+except AttributeError:  # a CPU-only torch build
+    def _raw_stream(index):
+        return torch.cuda.current_stream(index).cuda_stream
+
+
 def current_stream(device) -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return C.c_void_p(_raw_stream(device.index if device.index is not None else torch.cuda.current_device()))
 
 
 def _require_cuda(t: torch.Tensor, what: str) -> None:
@@ -196,17 +208,15 @@ class DevicePacked:
         self.device = self.tensors[0].device
         s = IxhPacked()
         s.n_levels = n_levels
-        for i, b in enumerate(level_bits):
-            s.level_bits[i] = b
+        s.level_bits[:n_levels] = level_bits
         s.out_f, s.in_f = self.out_f, self.in_f
-        for i in range(n_levels - 1):
-            bm, st = bitmaps[i], streams[i]
-            if bm.dtype != torch.int32 or st.dtype != torch.int32:
-                raise ValueError("bitmaps and packed streams must be torch.int32")
-            s.bitmaps[i] = bm.data_ptr() if bm.numel() else None
-            s.bitmap_words[i] = bm.numel()
-            s.streams[i] = st.data_ptr() if st.numel() else None
-            s.stream_words[i] = st.numel()
+        n_bitmaps, n_streams = [t.numel() for t in bitmaps], [t.numel() for t in streams[:-1]]
+        if any(t.dtype != torch.int32 for t in bitmaps) or any(t.dtype != torch.int32 for t in streams[:-1]):
+            raise ValueError("bitmaps and packed streams must be torch.int32")
+        s.bitmaps[: n_levels - 1] = [t.data_ptr() if n else None for t, n in zip(bitmaps, n_bitmaps)]
+        s.bitmap_words[: n_levels - 1] = n_bitmaps
+        s.streams[: n_levels - 1] = [t.data_ptr() if n else None for t, n in zip(streams, n_streams)]
+        s.stream_words[: n_levels - 1] = n_streams
         last = streams[-1]
         if last.dtype != torch.uint8:
             raise ValueError("the last stream must be torch.uint8")
@@ -413,11 +423,11 @@ class LanePacked:
 
 
 def encode_device(weight: torch.Tensor, level_bits) -> tuple:
-    """Encode a bf16 [out_f, in_f] device tensor with the library's two encoder calls.
+    """Encode a bf16 [out_f, in_f] device tensor with the library's encoder calls.
 
     Returns ``(DevicePacked, table512, counts)``: the packed tensors (device), the int32
     ``[n_levels-1, entries]`` rank table at unit 512 and the per-level element counts (host ints).  One
-    host synchronisation (reading the counts) sits between the two calls.
+    host synchronisation (the counts' arrival) sits between the scan and the pack.
     """
     _require_cuda(weight, "weight")
     if weight.dtype != torch.bfloat16 or weight.dim() != 2:
@@ -433,18 +443,22 @@ def encode_device(weight: torch.Tensor, level_bits) -> tuple:
     workspace = torch.empty(max(ws_bytes, 4), dtype=torch.uint8, device=dev)
     scale = torch.empty(1, dtype=torch.bfloat16, device=dev)
     table = torch.empty((max(n_levels - 1, 1), max(entries, 1)), dtype=torch.int32, device=dev)
+    arrived = torch.empty(max(n_levels - 1, 1), dtype=torch.int64, pin_memory=True)  # the counts, as the kernel writes them
     with torch.cuda.device(dev):
-        check(L.ixh_encode_scan(weight.data_ptr(), out_f, in_f, n_levels, bits, scale.data_ptr(), table.data_ptr(),
-                                workspace.data_ptr(), ws_bytes, current_stream(dev)))
-        counts = [int(c) for c in table[:, -1].cpu().tolist()]  # the one synchronisation
-        counts.append(out_f * in_f - sum(counts))
+        stream = current_stream(dev)
+        check(L.ixh_encode_scan_counts(weight.data_ptr(), out_f, in_f, n_levels, bits, scale.data_ptr(), table.data_ptr(),
+                                       workspace.data_ptr(), ws_bytes, arrived.data_ptr(), stream))
         left = out_f * in_f
-        bitmaps, streams = [], []
+        bitmaps, streams = [torch.empty((left + 31) // 32, dtype=torch.int32, device=dev)], []
+        check(L.ixh_encode_wait(arrived.data_ptr(), n_levels - 1, stream))  # the one synchronisation
+        counts = arrived.tolist()
+        counts.append(out_f * in_f - sum(counts))
         for i, b in enumerate(level_bits[:-1]):
-            bitmaps.append(torch.empty((left + 31) // 32, dtype=torch.int32, device=dev))
+            if i > 0:
+                bitmaps.append(torch.empty((left + 31) // 32, dtype=torch.int32, device=dev))
             streams.append(torch.empty((counts[i] * b + 31) // 32, dtype=torch.int32, device=dev))
             left -= counts[i]
         streams.append(torch.empty(counts[-1], dtype=torch.uint8, device=dev))
         dp = DevicePacked(level_bits, out_f, in_f, bitmaps, streams, scale)
-        check(L.ixh_encode_pack(weight.data_ptr(), C.byref(dp.struct), table.data_ptr(), current_stream(dev)))
+        check(L.ixh_encode_pack(weight.data_ptr(), C.byref(dp.struct), table.data_ptr(), stream))
     return dp, table, counts

@@ -600,9 +600,9 @@ size_t ixh_encode_workspace_bytes(int64_t out_f, int64_t in_f, int32_t n_levels)
     return encode_workspace_bytes(n, n_levels);
 }
 
-int ixh_encode_scan(const uint16_t *w, int64_t out_f, int64_t in_f, int32_t n_levels, const int32_t *level_bits,
-                    uint16_t *scale, int32_t *prefix, void *workspace, size_t workspace_bytes,
-                    ixh_stream_t stream) {
+static int encode_scan(const uint16_t *w, int64_t out_f, int64_t in_f, int32_t n_levels, const int32_t *level_bits,
+                       uint16_t *scale, int32_t *prefix, void *workspace, size_t workspace_bytes, int64_t *host_counts,
+                       ixh_stream_t stream) {
     int rc = encode_levels_ok(n_levels, level_bits);
     if (rc) return rc;
     if (out_f <= 0 || in_f <= 0) { set_error("encode: empty weight (the reference's max() raises on it too)"); return IXH_EINVAL; }
@@ -616,9 +616,45 @@ int ixh_encode_scan(const uint16_t *w, int64_t out_f, int64_t in_f, int32_t n_le
     }
     int bits[IXH_MAX_LEVELS];
     for (int i = 0; i < n_levels; ++i) bits[i] = level_bits[i];
-    rc = launch_encode_scan(w, (uint32_t)n, n_levels, bits, scale, prefix, workspace, (hipStream_t)stream);
+    rc = launch_encode_scan(w, (uint32_t)n, n_levels, bits, scale, prefix, workspace, host_counts, (hipStream_t)stream);
     if (rc == IXH_ELAUNCH) set_error("encode_scan: launch failed");
     return rc;
+}
+
+int ixh_encode_scan(const uint16_t *w, int64_t out_f, int64_t in_f, int32_t n_levels, const int32_t *level_bits,
+                    uint16_t *scale, int32_t *prefix, void *workspace, size_t workspace_bytes,
+                    ixh_stream_t stream) {
+    return encode_scan(w, out_f, in_f, n_levels, level_bits, scale, prefix, workspace, workspace_bytes, nullptr, stream);
+}
+
+int ixh_encode_scan_counts(const uint16_t *w, int64_t out_f, int64_t in_f, int32_t n_levels, const int32_t *level_bits,
+                           uint16_t *scale, int32_t *prefix, void *workspace, size_t workspace_bytes, int64_t *host_counts,
+                           ixh_stream_t stream) {
+    if (!host_counts) { set_error("encode: host_counts is NULL"); return IXH_EINVAL; }
+    for (int i = 0; i < n_levels - 1 && i < IXH_MAX_LEVELS - 1; ++i) __atomic_store_n(host_counts + i, (int64_t)-1, __ATOMIC_RELEASE);
+    return encode_scan(w, out_f, in_f, n_levels, level_bits, scale, prefix, workspace, workspace_bytes, host_counts, stream);
+}
+
+int ixh_encode_wait(const int64_t *host_counts, int32_t n_counts, ixh_stream_t stream) {
+    if (!host_counts || n_counts < 1 || n_counts >= IXH_MAX_LEVELS) { set_error("encode: host_counts is NULL or n_counts wrong"); return IXH_EINVAL; }
+    // The counts arrive a few microseconds before the stream's completion would; the stream is asked now and then, so that
+    // the wait ends when it has failed, or has drained without them.
+    auto arrived = [&] {
+        for (int i = 0; i < n_counts; ++i)
+            if (__atomic_load_n(host_counts + i, __ATOMIC_ACQUIRE) < 0) return false;
+        return true;
+    };
+    for (uint32_t spins = 1; !arrived(); ++spins) {
+        if (spins % 4096 == 0) {
+            const hipError_t e = hipStreamQuery((hipStream_t)stream);
+            if (e == hipErrorNotReady) continue;
+            if (e == hipSuccess && arrived()) break;
+            set_error("encode_wait: the counts did not arrive (%s)", hipGetErrorString(e));
+            return IXH_ELAUNCH;
+        }
+        __builtin_ia32_pause();
+    }
+    return IXH_OK;
 }
 
 int ixh_encode_pack(const uint16_t *w, const IxhPacked *dst, const int32_t *prefix, ixh_stream_t stream) {

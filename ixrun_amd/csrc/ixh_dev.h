@@ -63,11 +63,15 @@ __device__ __forceinline__ int threshold_of(int bits) { return (1 << (bits - 1))
 
 // inclusive sum over the lanes at or below this one (DPP: shifts inside the 16-lane rows, then the two
 // row broadcasts that carry the totals across rows)
-__device__ __forceinline__ uint32_t wave_scan_inclusive(uint32_t v) {
+__device__ __forceinline__ uint32_t row_scan_inclusive(uint32_t v) {
     v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);   // row_shr:1
     v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);   // row_shr:2
     v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);   // row_shr:4
     v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);   // row_shr:8
+    return v;
+}
+__device__ __forceinline__ uint32_t wave_scan_inclusive(uint32_t v) {
+    v = row_scan_inclusive(v);
     v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
     v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
     return v;
@@ -133,7 +137,7 @@ int launch_prefill(const Dev &P, const int32_t *prefix, const uint16_t *x, uint3
                    int64_t ldy, float *ws, hipStream_t s);
 size_t encode_workspace_bytes(uint64_t n, int n_levels);
 int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *bits, uint16_t *scale, int32_t *table,
-                       void *workspace, hipStream_t s);
+                       void *workspace, int64_t *host_totals, hipStream_t s);
 int launch_encode_pack(const uint16_t *w, const Dev &P, const int32_t *table, hipStream_t s);
 int launch_fill_u16(uint16_t *dst, uint32_t n, uint16_t value, hipStream_t s);
 void set_error(const char *fmt, ...);

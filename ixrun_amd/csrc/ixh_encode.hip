@@ -1,10 +1,9 @@
 // The INT8-X encoder on the device: bf16 weights -> scale, rank table, nested bitmaps and code streams,
 // byte for byte what the reference's CPU writer produces (ixrun/quantize.py:41-122 with the bit packing of
 // ixrun/bitpack.py:13-61, :87-89).  Three passes over the weights, all bound by HBM reads:
-//   1. k_enc_absmax      largest magnitude, one partial result per workgroup (no atomics, nothing to clear);
-//                        k_enc_scale (one wave) turns the partial results into the bf16 scale
-//   2. k_enc_count<L>    quantise, count every level per 512-element unit; the counts are then summed into
-//                        the rank table (k_enc_tile_sums, k_enc_scan), which is the table the decoders take
+//   1. k_enc_absmax      largest magnitude, one partial result per workgroup (no atomics, nothing to clear)
+//   2. k_enc_count<L>    the bf16 scale from the partial results, and the elements of every level per 512-element unit;
+//                        k_enc_scan sums the counts into the rank table, which is the table the decoders take
 //   3. k_enc_pack<L>     quantise again and pack; the table says at which bit of every stream a wave's elements
 //                        start.  Only the words that two waves share are cleared (k_enc_borders) and OR-ed in
 // Between passes 2 and 3 the caller reads the level totals (last table entries) and sizes the streams.
@@ -15,25 +14,8 @@ namespace ixh {
 constexpr uint32_t kEncUnit = 512;          // elements per wave and step: eight per lane
 constexpr int kEncWaves = 4;                // waves per workgroup
 constexpr uint32_t kEncParts = 256;         // partial maxima of pass 1 (one per workgroup of 1024 lanes)
-constexpr uint32_t kScanTile = 8192;        // table entries per workgroup of the scan
-
-// Eight consecutive bf16 starting at element p, widened to fp32 (zero past n).  Vector load when the address
-// allows it.
-__device__ __forceinline__ void load8(const uint16_t *__restrict__ w, uint32_t p, uint32_t n, bool aligned,
-                                      float (&f)[8]) {
-    if (aligned && p + 8 <= n) {
-        const uint4 v = *reinterpret_cast<const uint4 *>(w + p);
-        const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            f[2 * k] = __uint_as_float(d[k] << 16);
-            f[2 * k + 1] = __uint_as_float(d[k] & 0xffff0000u);
-        }
-    } else {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) f[t] = p + t < n ? bf16_bits_to_f32(w[p + t]) : 0.0f;
-    }
-}
+constexpr uint32_t kScanTile = 4096;        // table entries per workgroup of the scan
+constexpr int kEncAhead = 4;                // loads in flight per lane of pass 1
 
 __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
     for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off));
@@ -67,131 +49,201 @@ struct EncLevels {
     int bits[IXH_MAX_LEVELS];
 };
 
+// Elements p and p + 1, `fill` for one at or past n.  The loads are unconditional, so that they do not wait for one another.
+__device__ __forceinline__ uint32_t pair_or(const uint16_t *__restrict__ w, uint64_t p, uint32_t n, uint32_t fill) {
+    const uint32_t a = w[min(p, (uint64_t)n - 1)], b = w[min(p + 1, (uint64_t)n - 1)];
+    return (p < n ? a : fill) | (p + 1 < n ? b : fill) << 16;
+}
+
+// Pairs of weights from element p on, eight in all; zero past n.  kWhole: all eight are there, at a multiple of 16 bytes.
+template <bool kWhole>
+__device__ __forceinline__ uint4 load8(const uint16_t *__restrict__ w, uint64_t p, uint32_t n) {
+    if (kWhole) return *reinterpret_cast<const uint4 *>(w + p);
+    return make_uint4(pair_or(w, p, n, 0u), pair_or(w, p + 2, n, 0u), pair_or(w, p + 4, n, 0u), pair_or(w, p + 6, n, 0u));
+}
+
+// Bound by HBM (a read of 178 MB: 37 us, 4.8 TB/s; more loads in flight or more workgroups change nothing).
 __global__ void __launch_bounds__(1024) k_enc_absmax(const uint16_t *__restrict__ w, uint32_t n, uint32_t *parts) {
     const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
-    uint32_t m = 0;
-    const uint32_t stride = gridDim.x * 1024u * 8u;
-    for (uint64_t p = ((uint64_t)blockIdx.x * 1024u + threadIdx.x) * 8u; p < n; p += stride) {
-        float f[8];
-        load8(w, (uint32_t)p, n, aligned, f);
+    typedef uint16_t half2 __attribute__((ext_vector_type(2)));
+    half2 m = {0, 0};
+    auto take = [&](const uint4 &q) {
+        const uint32_t d[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-        for (int t = 0; t < 8; ++t) m = max(m, (__float_as_uint(f[t]) >> 16) & 0x7fffu);
+        for (int t = 0; t < 4; ++t) m = __builtin_elementwise_max(m, __builtin_bit_cast(half2, d[t] & 0x7fff7fffu));
+    };
+    const uint64_t stride = (uint64_t)gridDim.x * 1024u * 8u;
+    uint64_t base = (uint64_t)blockIdx.x * 1024u * 8u;
+    const uint32_t mine = threadIdx.x * 8u;
+    for (; aligned && base + (kEncAhead - 1) * stride + 1024u * 8u <= n; base += kEncAhead * stride) {
+        uint4 q[kEncAhead];
+#pragma unroll
+        for (int k = 0; k < kEncAhead; ++k) q[k] = load8<true>(w, base + k * stride + mine, n);
+#pragma unroll
+        for (int k = 0; k < kEncAhead; ++k) take(q[k]);
     }
+    for (; base < n; base += stride) take(load8<false>(w, base + mine, n));
     __shared__ uint32_t wave_m[16];
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) wave_m[threadIdx.x >> 6] = m;
+    uint32_t top = wave_max(max((uint32_t)m.x, (uint32_t)m.y));
+    if ((threadIdx.x & 63) == 0) wave_m[threadIdx.x >> 6] = top;
     __syncthreads();
     if (threadIdx.x < 16) {
-        m = wave_m[threadIdx.x];
-        for (int off = 8; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off));
-        if (threadIdx.x == 0) parts[blockIdx.x] = m;
+        top = wave_m[threadIdx.x];
+        for (int off = 8; off > 0; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off));
+        if (threadIdx.x == 0) parts[blockIdx.x] = top;
     }
 }
 
-__global__ void __launch_bounds__(kWave) k_enc_scale(const uint32_t *__restrict__ parts, uint16_t *scale_out) {
-    const uint32_t sbits = scale_bits_from_parts(parts, threadIdx.x);
-    if (threadIdx.x == 0) *scale_out = (uint16_t)sbits;
-}
+// table[i * entries + u + 1] = number of level-i elements of unit u (raw counts; the scan turns them into ranks), and
+// sums[i * groups + g] = that of a workgroup's kCountUnits units.
+//
+// Magnitudes order like their bf16 bits, so "|int8| above a level's threshold" is one comparison of 15-bit numbers, with a
+// cutoff that every wave finds by quantising the 64 bf16 values around (threshold + 1/2) * scale: the very arithmetic of
+// the pack.  (A level is "the thresholds below |v|", quantize.py:25-37: counting what is above each and taking
+// differences gives the levels.)  Two weights to a subtraction; a row of 16 lanes takes a unit, so that four DPP steps sum
+// four units.  Bound by its read, which the last-level cache serves in part: 5120 x 17408 in 28 us, 6.3 TB/s (35 when
+// every weight was quantised in fp32).
+constexpr uint32_t kCountUnits = 64;
 
-// table[i * entries + u + 1] = number of level-i elements of unit u (raw counts; the scan turns them into ranks).
-// A wave takes kCountUnits units in a row; a level is "the thresholds below |v|" (quantize.py:25-37), so the
-// kernel counts, per threshold, the values above it and takes differences.
-constexpr int kCountUnits = 4;
-
-template <int L>
-__global__ void __launch_bounds__(kWave *kEncWaves)
-k_enc_count(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, const uint16_t *__restrict__ scale_in,
-            EncLevels lv, int32_t *table) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t u0 = (blockIdx.x * kEncWaves + (threadIdx.x >> 6)) * kCountUnits;
-    if (u0 >= n_units) return;
-    const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
-    float thr[L - 1];
+template <int L, bool kWhole>
+__device__ __forceinline__ void
+count_units(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, const uint32_t *__restrict__ parts,
+            const EncLevels &lv, int32_t *table, uint32_t *sums, uint16_t *scale_out) {
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t u_first = blockIdx.x * kCountUnits + wave * (kCountUnits / kEncWaves);
+    constexpr int kTurns = kCountUnits / kEncWaves / 4;
+    auto place = [&](int turn, int k) {
+        return (uint64_t)(u_first + 4 * turn + (lane >> 4)) * kEncUnit + (lane & 15u) * 8u + 128u * k;
+    };
+    uint4 q[4];
+    if (kWhole) {
 #pragma unroll
-    for (int i = 0; i < L - 1; ++i) thr[i] = (float)threshold_of(lv.bits[i]);
-    float f[kCountUnits][8];
+        for (int k = 0; k < 4; ++k) q[k] = load8<true>(w, place(0, k), n);
+    }
+    const uint32_t sbits = scale_bits_from_parts(parts, lane);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = (uint16_t)sbits;
+    const float scale = bf16_bits_to_f32(sbits), inv_scale = __fdiv_rn(1.0f, scale);
+    uint32_t cut[L - 1];  // in both halves: the smallest magnitude above the level's threshold
 #pragma unroll
-    for (int k = 0; k < kCountUnits; ++k) load8(w, min((u0 + k) * kEncUnit + lane * 8u, n), n, aligned, f[k]);
-    const float inv_scale = __fdiv_rn(1.0f, bf16_bits_to_f32(*scale_in));
+    for (int i = 0; i < L - 1; ++i) {
+        const float thr = (float)threshold_of(lv.bits[i]);
+        const int around = (int)(__float_as_uint((thr + 0.5f) * scale) >> 16) - 32;
+        const int mag = min(max(around + (int)lane, 0), 0x7fff);
+        const uint64_t above = __ballot(fabsf(quantise(bf16_bits_to_f32((uint32_t)mag), inv_scale)) > thr);
+        // (all of them above: a scale that is not a number, where every weight is)
+        const uint32_t c = above == ~0ull ? 0u : (uint32_t)min(max(around + (int)__builtin_ctzll(above | 1ull << 63), 0), 0x7fff);
+        cut[i] = c * 0x10001u;
+    }
     const uint32_t entries = n_units + 1;
+    uint32_t total[L - 1] = {};
+#pragma unroll(kWhole ? kTurns : 1)
+    for (int turn = 0; turn < kTurns; ++turn) {
+        uint4 ahead[4];
+        if (kWhole && turn + 1 < kTurns) {
 #pragma unroll
-    for (int k = 0; k < kCountUnits; ++k) {
-        const uint32_t u = u0 + k;
-        if (u >= n_units) break;
-        // values above each threshold, 10-bit fields, three to a word: a wave holds at most 512 of anything
-        uint32_t above[L - 1] = {};
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const float a = fabsf(quantise(f[k][t], inv_scale));
-#pragma unroll
-            for (int i = 0; i < L - 1; ++i) above[i] += a > thr[i] ? 1u : 0u;
+            for (int k = 0; k < 4; ++k) ahead[k] = load8<true>(w, place(turn + 1, k), n);
         }
+        uint32_t above[L - 1] = {};
+#pragma unroll(kWhole ? 4 : 1)
+        for (int k = 0; k < 4; ++k) {
+            const uint4 c = kWhole ? q[k] : load8<false>(w, place(turn, k), n);
+            const uint32_t d[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < L - 1; ++i) above[i] += __popc(((d[t] | 0x80008000u) - cut[i]) & 0x80008000u);
+        }
+        // sums over the row's lanes, 10-bit fields, three to a word: at most 512 of anything
         uint32_t acc[(L + 1) / 3] = {};
 #pragma unroll
         for (int i = 0; i < L - 1; ++i) acc[i / 3] |= above[i] << (10 * (i % 3));
 #pragma unroll
-        for (int j = 0; j < (L + 1) / 3; ++j) acc[j] = wave_scan_inclusive(acc[j]);
-        // elements of the unit (those past n were loaded as zero and are above nothing)
-        uint32_t prev = min(kEncUnit, n - u * kEncUnit);
+        for (int j = 0; j < (L + 1) / 3; ++j) acc[j] = row_scan_inclusive(acc[j]);
+        const uint32_t u = u_first + 4 * turn + (lane >> 4);
+        if ((lane & 15u) == 15u && u < n_units) {
+            uint32_t prev = min(kEncUnit, n - u * kEncUnit);
 #pragma unroll
-        for (int i = 0; i < L - 1; ++i) {
-            const uint32_t ab = (acc[i / 3] >> (10 * (i % 3))) & 1023u;
-            if (lane == 63) table[(size_t)i * entries + u + 1] = (int32_t)(prev - ab);
-            prev = ab;
+            for (int i = 0; i < L - 1; ++i) {
+                const uint32_t ab = min((acc[i / 3] >> (10 * (i % 3))) & 1023u, prev);
+                table[(size_t)i * entries + u + 1] = (int32_t)(prev - ab);
+                total[i] += prev - ab;
+                prev = ab;
+            }
+        }
+        if (kWhole) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = ahead[k];
         }
     }
-}
-
-// sums[row * tiles + tile] = sum of the raw counts of one tile of one table row
-__global__ void __launch_bounds__(1024) k_enc_tile_sums(const int32_t *__restrict__ table, uint32_t n_units,
-                                                         uint32_t *sums) {
-    const int32_t *row = table + (size_t)blockIdx.y * (n_units + 1) + 1;
-    const uint32_t base = blockIdx.x * kScanTile;
-    uint32_t s = 0;
-    for (uint32_t k = threadIdx.x; k < kScanTile && base + k < n_units; k += 1024) s += (uint32_t)row[base + k];
-    __shared__ uint32_t wave_s[16];
-    s = wave_scan_inclusive(s);
-    if ((threadIdx.x & 63) == 63) wave_s[threadIdx.x >> 6] = s;
+    __shared__ uint32_t wave_t[kEncWaves][L - 1];
+#pragma unroll
+    for (int i = 0; i < L - 1; ++i) {
+        const uint32_t t = wave_scan_inclusive(total[i]);
+        if (lane == 63) wave_t[wave][i] = t;
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < L - 1) {
         uint32_t t = 0;
-        for (int i = 0; i < 16; ++i) t += wave_s[i];
-        sums[blockIdx.y * gridDim.x + blockIdx.x] = t;
+#pragma unroll
+        for (int k = 0; k < kEncWaves; ++k) t += wave_t[k][threadIdx.x];
+        sums[threadIdx.x * gridDim.x + blockIdx.x] = t;
     }
 }
 
-// In place, per row: row[0] = 0, row[u + 1] = counts of units 0 .. u.  Each thread takes eight consecutive entries.
-__global__ void __launch_bounds__(1024) k_enc_scan(int32_t *table, uint32_t n_units, const uint32_t *__restrict__ sums) {
+template <int L>
+__global__ void __launch_bounds__(kWave *kEncWaves)
+k_enc_count(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, const uint32_t *__restrict__ parts,
+            EncLevels lv, int32_t *table, uint32_t *sums, uint16_t *scale_out) {
+    const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
+    if (aligned && (uint64_t)(blockIdx.x + 1) * kCountUnits * kEncUnit <= n)
+        count_units<L, true>(w, n, n_units, parts, lv, table, sums, scale_out);
+    else
+        count_units<L, false>(w, n, n_units, parts, lv, table, sums, scale_out);
+}
+
+// In place, per row: row[0] = 0, row[u + 1] = counts of units 0 .. u.  Each thread takes four consecutive entries; what
+// the workgroups of k_enc_count in front of the tile counted comes first.  6 us, all of it latency (tiles twice as large,
+// eight entries a thread, and sums from a kernel of their own: 14).
+struct __attribute__((packed, aligned(4))) Int4 { int32_t v[4]; };
+__global__ void __launch_bounds__(1024)
+k_enc_scan(int32_t *table, uint32_t n_units, const uint32_t *__restrict__ sums, uint32_t groups, int64_t *host_totals) {
     int32_t *row = table + (size_t)blockIdx.y * (n_units + 1);
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ uint32_t wave_s[16], wave_c[16];
-    // ranks before this tile: the partial sums of the tiles in front of it
-    {
-        uint32_t c = 0;
-        const uint32_t *mine_sums = sums + (size_t)blockIdx.y * gridDim.x;
-        for (uint32_t t = tid; t < blockIdx.x; t += 1024) c += mine_sums[t];
-        c = wave_scan_inclusive(c);
-        if (lane == 63) wave_c[wave] = c;
-    }
-    const uint32_t first = blockIdx.x * kScanTile + tid * 8u;
-    uint32_t v[8];
-    uint32_t mine = 0;
+    const uint32_t first = blockIdx.x * kScanTile + tid * 4u;
+    uint32_t v[4];
+    if (first + 4 <= n_units) {
+        const Int4 q = *reinterpret_cast<const Int4 *>(row + first + 1);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        v[t] = first + t < n_units ? (uint32_t)row[first + t + 1] : 0u;
-        mine += v[t];
+        for (int t = 0; t < 4; ++t) v[t] = (uint32_t)q.v[t];
+    } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[t] = first + t < n_units ? (uint32_t)row[first + t + 1] : 0u;
     }
+    uint32_t c = 0;
+    const uint32_t *row_sums = sums + (size_t)blockIdx.y * groups;
+    for (uint32_t g = tid; g < blockIdx.x * (kScanTile / kCountUnits); g += 1024) c += row_sums[g];
+    c = wave_scan_inclusive(c);
+    if (lane == 63) wave_c[wave] = c;
+    const uint32_t mine = v[0] + v[1] + v[2] + v[3];
     const uint32_t incl = wave_scan_inclusive(mine);
     if (lane == 63) wave_s[wave] = incl;
     __syncthreads();
     uint32_t run = incl - mine;
     for (uint32_t k = 0; k < 16; ++k) run += wave_c[k] + (k < wave ? wave_s[k] : 0u);
+    Int4 q;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        run += v[t];
-        if (first + t < n_units) row[first + t + 1] = (int32_t)run;
+    for (int t = 0; t < 4; ++t) q.v[t] = (int32_t)(run += v[t]);
+    if (first + 4 <= n_units) {
+        *reinterpret_cast<Int4 *>(row + first + 1) = q;
+    } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (first + t < n_units) row[first + t + 1] = q.v[t];
     }
     if (blockIdx.x == 0 && tid == 0) row[0] = 0;
+    if (host_totals && blockIdx.x + 1 == gridDim.x && tid == 1023)
+        __hip_atomic_store(host_totals + blockIdx.y, (int64_t)run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Destination of the encoder: the same fields as Dev, writable.
@@ -358,10 +410,7 @@ __device__ __forceinline__ void load32(const uint16_t *__restrict__ w, uint32_t 
         }
     } else {
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            d[k] = p + 2 * k < n ? w[p + 2 * k] : 0x7f80u;
-            d[k] |= (p + 2 * k + 1 < n ? (uint32_t)w[p + 2 * k + 1] : 0x7f80u) << 16;
-        }
+        for (int k = 0; k < 16; ++k) d[k] = pair_or(w, p + 2 * k, n, 0x7f80u);
     }
 }
 
@@ -541,22 +590,22 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, uint32_
     }
 }
 
+// workspace: partial maxima (kEncParts), sums of k_enc_count's workgroups
+static uint32_t count_groups(uint64_t n) { return (uint32_t)((n + (uint64_t)kEncUnit * kCountUnits - 1) / ((uint64_t)kEncUnit * kCountUnits)); }
+
 size_t encode_workspace_bytes(uint64_t n, int n_levels) {
-    const uint64_t n_units = (n + kEncUnit - 1) / kEncUnit;
-    const uint64_t tiles = (n_units + kScanTile - 1) / kScanTile;
-    return (size_t)(kEncParts * 4u + (uint64_t)(n_levels - 1) * (tiles ? tiles : 1) * 4u);
+    return 4u * (kEncParts + (size_t)(n_levels - 1) * count_groups(n));
 }
 
 template <int L>
-static void scan_launch(const uint16_t *w, uint32_t n, uint32_t n_units, const EncLevels &lv, const uint16_t *scale,
-                        int32_t *table, hipStream_t s) {
-    const uint32_t per_block = kEncWaves * kCountUnits;
-    hipLaunchKernelGGL(k_enc_count<L>, dim3((n_units + per_block - 1) / per_block), dim3(kWave * kEncWaves), 0, s, w, n,
-                       n_units, scale, lv, table);
+static void scan_launch(const uint16_t *w, uint32_t n, uint32_t n_units, const EncLevels &lv, const uint32_t *parts,
+                        uint16_t *scale, int32_t *table, uint32_t *sums, hipStream_t s) {
+    hipLaunchKernelGGL(k_enc_count<L>, dim3(count_groups(n)), dim3(kWave * kEncWaves), 0, s, w, n, n_units, parts, lv, table,
+                       sums, scale);
 }
 
 int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *bits, uint16_t *scale, int32_t *table,
-                       void *workspace, hipStream_t s) {
+                       void *workspace, int64_t *host_totals, hipStream_t s) {
     const uint32_t n_units = (n + kEncUnit - 1) / kEncUnit;
     const uint32_t tiles = max(1u, (n_units + kScanTile - 1) / kScanTile);
     uint32_t *parts = static_cast<uint32_t *>(workspace);
@@ -565,18 +614,17 @@ int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *b
     lv.n_levels = n_levels;
     for (int i = 0; i < IXH_MAX_LEVELS; ++i) lv.bits[i] = i < n_levels ? bits[i] : 0;
     hipLaunchKernelGGL(k_enc_absmax, dim3(kEncParts), dim3(1024), 0, s, w, n, parts);
-    hipLaunchKernelGGL(k_enc_scale, dim3(1), dim3(kWave), 0, s, parts, scale);
     switch (n_levels) {
-        case 2: scan_launch<2>(w, n, n_units, lv, scale, table, s); break;
-        case 3: scan_launch<3>(w, n, n_units, lv, scale, table, s); break;
-        case 4: scan_launch<4>(w, n, n_units, lv, scale, table, s); break;
-        case 5: scan_launch<5>(w, n, n_units, lv, scale, table, s); break;
-        case 6: scan_launch<6>(w, n, n_units, lv, scale, table, s); break;
-        case 7: scan_launch<7>(w, n, n_units, lv, scale, table, s); break;
-        default: scan_launch<8>(w, n, n_units, lv, scale, table, s); break;
+        case 2: scan_launch<2>(w, n, n_units, lv, parts, scale, table, sums, s); break;
+        case 3: scan_launch<3>(w, n, n_units, lv, parts, scale, table, sums, s); break;
+        case 4: scan_launch<4>(w, n, n_units, lv, parts, scale, table, sums, s); break;
+        case 5: scan_launch<5>(w, n, n_units, lv, parts, scale, table, sums, s); break;
+        case 6: scan_launch<6>(w, n, n_units, lv, parts, scale, table, sums, s); break;
+        case 7: scan_launch<7>(w, n, n_units, lv, parts, scale, table, sums, s); break;
+        default: scan_launch<8>(w, n, n_units, lv, parts, scale, table, sums, s); break;
     }
-    hipLaunchKernelGGL(k_enc_tile_sums, dim3(tiles, n_levels - 1), dim3(1024), 0, s, table, n_units, sums);
-    hipLaunchKernelGGL(k_enc_scan, dim3(tiles, n_levels - 1), dim3(1024), 0, s, table, n_units, sums);
+    hipLaunchKernelGGL(k_enc_scan, dim3(tiles, n_levels - 1), dim3(1024), 0, s, table, n_units, sums, count_groups(n),
+                       host_totals);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
