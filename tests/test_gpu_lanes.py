@@ -152,3 +152,20 @@ def test_malformed_lanes_are_refused(dev):
         assert call(s) == -1, field
     assert call(lanes.struct, 0) == -1 and call(lanes.struct, 17) == -1
     assert L.ixh_lanes_plane_words(8, 512, 7) == -1 and L.ixh_lanes_cells(0, 512) == -1
+
+
+@pytest.mark.parametrize("out_f,in_f", [(7, 1000), (33, 513), (5, 4099)])
+def test_rows_of_other_lengths_decode_by_flat_units(oracle, dev, out_f, in_f):
+    """A layer whose rows are not whole units of 512 decodes by units counted over the row ends, also after another
+    layer's state has been loaded into it."""
+    from ixrun_amd.engine import StreamingLinear
+
+    v, scheme, _ = values("real", out_f, in_f)
+    packed = [packed_from_int8(w, out_f, in_f, level_bits=scheme) for w in (v, np.roll(v, 3))]
+    want = [oracle.decode_packed_bf16(p).reshape(-1) for p in packed]
+    layers = [StreamingLinear(p) for p in packed]
+    for layer, w in zip(layers, want):
+        layer._set_shared_buf(torch.empty(out_f * in_f, dtype=torch.bfloat16, device=dev))
+        assert np.array_equal(bf16_bits(layer._decode()).reshape(-1), w)
+    layers[0].load_state_dict(layers[1].state_dict())
+    assert np.array_equal(bf16_bits(layers[0]._decode()).reshape(-1), want[1])
