@@ -59,6 +59,16 @@ class IxhLanes(C.Structure):
     ]
 
 
+def host():
+    """The native host module (``csrc/ixh_host.cpp``); raises if it has not been built."""
+    try:
+        from . import _host
+    except ImportError as e:
+        raise RuntimeError(f"ixrun_amd/_host.so cannot be loaded ({e}): build it with ixrun_amd/csrc/build.sh; "
+                           "there is no fallback path") from e
+    return _host
+
+
 class IxhError(RuntimeError):
     """A call into libixhip returned a negative code."""
 

@@ -12,7 +12,16 @@ FLAGS="--offload-arch=gfx950 -O3 -std=c++17 -fPIC -Xclang -target-feature -Xclan
 PRELOAD_SRCS="${PRELOAD_SRCS-ixh_rows358.hip ixh_lanes.hip}"
 PRELOAD_FLAGS="-mllvm -amdgpu-kernarg-preload-count=14"
 mkdir -p build
+# the host module, against this interpreter's torch
+PYTHON="${PYTHON:-python3}"
+TORCH="$($PYTHON -c 'import os, importlib.util as u; print(os.path.dirname(u.find_spec("torch").origin))')"
+PYINC="$($PYTHON -c 'import sysconfig; print(sysconfig.get_paths()["include"])')"
+g++ -O2 -std=c++17 -fPIC -shared -fvisibility=hidden -Wall -Wno-unknown-pragmas -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 \
+    -I"$PYINC" -isystem "$TORCH/include" -isystem "$TORCH/include/torch/csrc/api/include" -isystem /opt/rocm/include \
+    ixh_host.cpp -o ../_host.so -L"$TORCH/lib" -lc10 -lc10_hip -ltorch_cpu -ltorch_python &
+HOST_PID=$!
 OBJS=""
 for s in $SRCS; do OBJS="$OBJS build/${s%.hip}.o"; done
 printf '%s\n' $SRCS | xargs -P "${JOBS:-8}" -I{} sh -c "rm -f build/\$(basename {} .hip).o; extra=; case ' $PRELOAD_SRCS ' in *' {} '*) extra='$PRELOAD_FLAGS';; esac; $HIPCC $FLAGS \$extra -c {} -o build/\$(basename {} .hip).o 2>&1 | grep -v 'packed-fp32-ops' >&2; test -f build/\$(basename {} .hip).o"
+wait $HOST_PID
 exec "$HIPCC" --offload-arch=gfx950 -shared -fPIC $OBJS -o libixhip.so

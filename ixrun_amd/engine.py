@@ -187,6 +187,16 @@ class StreamingLinear(nn.Module):
                 self._bias_ptr = bias.data_ptr()  # added by the kernel
         self._gemv_fn = _lib.lib().ixh_lanes_gemv if self._lanes is not None else _lib.lib().ixh_gemv
         self._plans = {}
+        # the forward of up to MAX_FUSED_ROWS rows from the lanes, in native code
+        self._native = self._native_fn = None
+        if self._lanes is not None and (self._bias is None or self._bias_ptr):
+            dev = self._scale.device
+            self._native_fn = self._gemv_fn
+            self._native = _lib.host().Forward(
+                ctypes.cast(self._gemv_fn, ctypes.c_void_p).value, ctypes.addressof(self._lanes.struct), self._bias_ptr or 0,
+                self.in_features, self.out_features, dev.index,
+                (0,) + tuple(self._lanes.gemv_workspace_bytes(n) for n in range(1, MAX_FUSED_ROWS + 1)),
+                (self._lanes, self._bias), _workspaces, dev, _lib.check)
 
     def _apply(self, fn, recurse=True):
         # .to()/.cuda() may move the buffers: point the kernel arguments at the new storage
@@ -245,6 +255,10 @@ class StreamingLinear(nn.Module):
         return plan
 
     def forward(self, x):
+        if self._native is not None and self._use_fused and not self._gemv_flags and self._gemv_fn is self._native_fn:
+            y = self._native(x)
+            if y is not None:
+                return y
         in_f = self.in_features
         if self._use_fused and x.dtype is torch.bfloat16 and x.is_cuda and in_f and x.shape[-1] == in_f:
             rows = x.numel() // in_f
@@ -252,7 +266,7 @@ class StreamingLinear(nn.Module):
             if plan is None:
                 plan = self._fused_plan(rows)
             if plan:
-                # the hot path of token generation: one ctypes call with the arguments that never change kept bound
+                # one ctypes call with the arguments that never change kept bound
                 out_f = self.out_features
                 if not x.is_contiguous():
                     x = x.contiguous()

@@ -169,3 +169,25 @@ def test_rows_of_other_lengths_decode_by_flat_units(oracle, dev, out_f, in_f):
         assert np.array_equal(bf16_bits(layer._decode()).reshape(-1), w)
     layers[0].load_state_dict(layers[1].state_dict())
     assert np.array_equal(bf16_bits(layers[0]._decode()).reshape(-1), want[1])
+
+
+def test_forward_in_native_code_takes_only_the_common_case(oracle, dev):
+    """Contiguous bf16 activations of 1 to 16 rows go through the native forward, with any leading dimensions; the rest
+    (views, other row lengths, other types, 17 rows) is left to the code behind it, which has to give the same."""
+    from ixrun_amd.engine import StreamingLinear
+
+    v, scheme, _ = values("real", 24, 1024)
+    p = packed_from_int8(v, 24, 1024, level_bits=scheme)
+    bias = torch.randn(24, generator=torch.Generator().manual_seed(1)).bfloat16()
+    layer = StreamingLinear(p, bias=bias)
+    layer._set_shared_buf(torch.empty(p["N"], dtype=torch.bfloat16, device=dev))
+    x = activations(16, 1024, seed=4).to(dev)
+    want = layer(x)
+    assert torch.equal(layer._native(x), want)
+    assert torch.equal(layer(x.view(2, 8, 1024)), want.view(2, 8, 24)) and torch.equal(layer(x[3]), layer(x[3:4])[0])
+    for other in (x.t().contiguous().t(), torch.cat([x, x])[::2], x[:, :512], x.float(), x.cpu(), torch.cat([x, x[:1]]), x[:0]):
+        assert layer._native(other) is None
+    assert torch.equal(layer(x.t().contiguous().t()), want)
+    assert layer(x[:0]).shape == (0, 24)
+    with pytest.raises(TypeError):
+        layer._native.__init__(1, 2)
