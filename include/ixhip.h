@@ -94,6 +94,14 @@ int64_t ixh_prefix_entries(int64_t n, int64_t chunk);
 int ixh_prefix_build(const IxhPacked *packed, int64_t chunk, int32_t *prefix, ixh_stream_t stream);
 
 /*
+ * The same table in fewer launches, with a workspace of ixh_prefix_workspace_bytes
+ * (4 bytes per level and 128 entries) for sums.
+ */
+size_t ixh_prefix_workspace_bytes(int64_t n, int64_t chunk, int32_t n_levels);
+int ixh_prefix_build_ws(const IxhPacked *packed, int64_t chunk, int32_t *prefix, void *workspace,
+                        size_t workspace_bytes, ixh_stream_t stream);
+
+/*
  * Full decode: out_i8[p] = int8 value of flat element p (nullable),
  * out_bf16[p] = bf16(f32(v) * f32(scale)) (nullable).  Replaces
  * _ix_decode_kernel / decode_weight_triton (ixrun/triton_kernels.py:68-177,

@@ -59,14 +59,23 @@ class IxhLanes(C.Structure):
     ]
 
 
+_native = None
+
+
 def host():
     """The native host module (``csrc/ixh_host.cpp``); raises if it has not been built."""
-    try:
-        from . import _host
-    except ImportError as e:
-        raise RuntimeError(f"ixrun_amd/_host.so cannot be loaded ({e}): build it with ixrun_amd/csrc/build.sh; "
-                           "there is no fallback path") from e
-    return _host
+    global _native
+    if _native is None:
+        try:
+            from . import _host
+        except ImportError as e:
+            raise RuntimeError(f"ixrun_amd/_host.so cannot be loaded ({e}): build it with ixrun_amd/csrc/build.sh; "
+                               "there is no fallback path") from e
+        L = lib()
+        _host.bind(*(C.cast(f, C.c_void_p).value for f in (
+            L.ixh_prefix_entries, L.ixh_prefix_workspace_bytes, L.ixh_prefix_build_ws, L.ixh_decode, L.ixh_decode_gs)), check)
+        _native = _host
+    return _native
 
 
 class IxhError(RuntimeError):
@@ -81,7 +90,8 @@ _lib = None
 
 # the product interface (include/ixhip.h) and the testing hook (include/ixhip_test.h)
 EXPORTS = (
-    "ixh_version", "ixh_last_error", "ixh_prefix_entries", "ixh_prefix_build", "ixh_decode",
+    "ixh_version", "ixh_last_error", "ixh_prefix_entries", "ixh_prefix_build", "ixh_prefix_build_ws",
+    "ixh_prefix_workspace_bytes", "ixh_decode",
     "ixh_gemv", "ixh_gemv_workspace_bytes", "ixh_gemv_noalloc", "ixh_gemm", "ixh_gemm_workspace_bytes",
     "ixh_encode_workspace_bytes", "ixh_encode_scan", "ixh_encode_scan_counts", "ixh_encode_wait", "ixh_encode_pack",
     "ixh_decode_gs",
@@ -109,6 +119,10 @@ def lib() -> C.CDLL:
         L.ixh_prefix_entries.argtypes = [C.c_int64, C.c_int64]
         L.ixh_prefix_build.restype = C.c_int
         L.ixh_prefix_build.argtypes = [C.POINTER(IxhPacked), C.c_int64, C.c_void_p, C.c_void_p]
+        L.ixh_prefix_workspace_bytes.restype = C.c_size_t
+        L.ixh_prefix_workspace_bytes.argtypes = [C.c_int64, C.c_int64, C.c_int32]
+        L.ixh_prefix_build_ws.restype = C.c_int
+        L.ixh_prefix_build_ws.argtypes = [C.POINTER(IxhPacked), C.c_int64, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]
         L.ixh_decode.restype = C.c_int
         L.ixh_decode.argtypes = [C.POINTER(IxhPacked), C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]
         L.ixh_decode_gs.restype = C.c_int
@@ -253,7 +267,10 @@ class DevicePacked:
         if entries < 1:
             raise ValueError(f"chunk {chunk} must be positive")
         table = torch.empty((len(self.level_bits) - 1, entries), dtype=torch.int32, device=self.device)
-        check(lib().ixh_prefix_build(C.byref(self.struct), int(chunk), table.data_ptr(), current_stream(self.device)))
+        ws = torch.empty(lib().ixh_prefix_workspace_bytes(self.N, int(chunk), len(self.level_bits)), dtype=torch.uint8,
+                         device=self.device)
+        check(lib().ixh_prefix_build_ws(C.byref(self.struct), int(chunk), table.data_ptr(), ws.data_ptr(), ws.numel(),
+                                        current_stream(self.device)))
         return table
 
     def decode(self, table: torch.Tensor, chunk: int, out_i8=None, out_bf16=None) -> None:

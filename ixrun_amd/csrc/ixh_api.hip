@@ -177,6 +177,28 @@ int ixh_prefix_build(const IxhPacked *packed, int64_t chunk, int32_t *prefix, ix
     return rc;
 }
 
+size_t ixh_prefix_workspace_bytes(int64_t n, int64_t chunk, int32_t n_levels) {
+    if (n < 0 || n >= (1ll << 31) || chunk <= 0 || chunk >= (1ll << 31) || n_levels < 2 || n_levels > IXH_MAX_LEVELS) return 0;
+    return prefix_workspace_bytes((uint64_t)n, (uint64_t)chunk, n_levels);
+}
+
+int ixh_prefix_build_ws(const IxhPacked *packed, int64_t chunk, int32_t *prefix, void *workspace, size_t workspace_bytes,
+                        ixh_stream_t stream) {
+    Dev d;
+    int rc = to_dev(packed, &d, false);
+    if (rc) return rc;
+    if (chunk <= 0 || chunk >= (1ll << 31)) { set_error("chunk %lld out of range", (long long)chunk); return IXH_EINVAL; }
+    if (!prefix) { set_error("prefix is NULL"); return IXH_EINVAL; }
+    const size_t need = prefix_workspace_bytes(d.n, (uint64_t)chunk, d.n_levels);
+    if (!workspace || workspace_bytes < need) {
+        set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
+        return IXH_EWORKSPACE;
+    }
+    rc = launch_prefix_build_ws(d, (uint32_t)chunk, prefix, workspace, (hipStream_t)stream);
+    if (rc) set_error("prefix_build: launch failed");
+    return rc;
+}
+
 static int decode_any(const IxhPacked *packed, const int32_t *prefix, int64_t chunk, int8_t *out_i8, uint16_t *out_bf16,
                       GroupScales gs, ixh_stream_t stream) {
     Dev d;

@@ -121,6 +121,8 @@ __device__ __forceinline__ int decode64(const Dev &P, uint32_t p0, bool alive, u
 
 // ---- host-side launchers (one per translation unit of kernels) ----
 int launch_prefix_build(const Dev &P, uint32_t chunk, int32_t *prefix, hipStream_t s);
+size_t prefix_workspace_bytes(uint64_t n, uint64_t chunk, int n_levels);
+int launch_prefix_build_ws(const Dev &P, uint32_t chunk, int32_t *table, void *workspace, hipStream_t s);
 int launch_decode(const Dev &P, const int32_t *prefix, uint32_t chunk, int8_t *o8, uint16_t *o16, GroupScales gs,
                   hipStream_t s);
 int launch_gemv_generic(const Dev &P, const int32_t *prefix, uint32_t chunk, const uint16_t *x, int m,

@@ -2,6 +2,8 @@
 // general fused decode+GEMV.  One wave64 owns a run of consecutive flat
 // elements and ranks them with ballots (decode64 in ixh_dev.h), so any number
 // of levels, any chunk size and ragged tails are handled by the same code.
+#include <algorithm>
+
 #include "ixh_dev.h"
 
 namespace ixh {
@@ -119,6 +121,102 @@ int launch_prefix_build(const Dev &P, uint32_t chunk, int32_t *prefix, hipStream
         }
         launch_scan_row(prefix + (size_t)i * entries, n_units, s);
     }
+    return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// The same table with a workspace for sums: one launch per level and one more, where counting a level and scanning it in
+// two or four launches each pays for every launch (2048 x 2048 at three levels: 4 launches and 24 us before, 3 and 8 us;
+// 17408 x 5120: 8 and 81, 3 and 14 us).  Bound by the latency of its chain: sums, the row in front, bitmap words.
+//
+// k_rank_level turns the local ranks of level - 1, which the launch before left per tile of kRankTile units, into final
+// ones (the tiles in front of it have left their sums in the workspace), so that it knows where its units start in
+// bitmap `level`; counts them there, four lanes to a unit; and leaves local ranks and its sum for the next launch.
+// ---------------------------------------------------------------------------------------------------------------
+constexpr uint32_t kRankTile = 128, kRankThreads = 4 * kRankTile;
+
+__global__ void __launch_bounds__(kRankThreads)
+k_rank_level(Dev P, int level, uint32_t chunk, uint32_t n_units, int32_t *table, uint32_t *sums) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t entries = n_units + 1, u0 = blockIdx.x * kRankTile, tiles = gridDim.x;
+    __shared__ uint32_t wave_s[kRankThreads / 64], start[kRankTile + 1], count[kRankTile];
+    uint32_t at = 0;  // index of unit u0 + tid's first element in bitmap `level`
+    if (tid <= kRankTile && u0 + tid <= n_units) {
+        at = (uint32_t)min((uint64_t)(u0 + tid) * chunk, (uint64_t)P.n);
+        for (int j = 0; j < level - 1; ++j) at -= (uint32_t)table[(size_t)j * entries + u0 + tid];
+    }
+    if (level > 0) {
+        int32_t *row = table + (size_t)(level - 1) * entries;
+        const bool mine = tid > 0 && tid <= kRankTile && u0 + tid <= n_units;
+        uint32_t rank = mine ? (uint32_t)row[u0 + tid] : 0u;
+        uint32_t front = 0;
+        for (uint32_t g = tid; g < blockIdx.x; g += kRankThreads) front += sums[(size_t)(level - 1) * tiles + g];
+        front = wave_scan_inclusive(front);
+        if (lane == 63) wave_s[wave] = front;
+        __syncthreads();
+        for (uint32_t k = 0; k < kRankThreads / 64; ++k) rank += wave_s[k];
+        if (mine) row[u0 + tid] = (int32_t)rank;
+        if (u0 + tid == 0) row[0] = 0;
+        at -= rank;
+    }
+    if (level == P.n_levels - 1) return;
+    if (tid <= kRankTile) start[tid] = at;
+    __syncthreads();
+    const uint32_t t = tid >> 2;
+    uint32_t c = 0;
+    const uint32_t words = P.bm_words[level];
+    if (u0 + t < n_units && words != 0) {
+        const uint32_t lo = start[t], hi = start[t + 1];
+        const uint32_t *bm = P.bm[level];
+        if (hi > lo) {
+            const uint32_t w_first = lo >> 5, w_last = min((hi - 1) >> 5, words - 1);
+            for (uint32_t base = w_first + (tid & 3u); base <= w_last; base += 20) {
+                uint32_t bits[5];
+#pragma unroll
+                for (int k = 0; k < 5; ++k) bits[k] = bm[min(base + 4 * k, w_last)];
+#pragma unroll
+                for (int k = 0; k < 5; ++k) {
+                    const uint32_t w = base + 4 * k;
+                    if (w == w_first) bits[k] &= ~0u << (lo & 31);
+                    if (w == (hi - 1) >> 5 && (hi & 31) != 0) bits[k] &= ~0u >> (32 - (hi & 31));
+                    c += w <= w_last ? __popc(bits[k]) : 0;
+                }
+            }
+        }
+    }
+    c += (uint32_t)__shfl_xor((int)c, 1);
+    c += (uint32_t)__shfl_xor((int)c, 2);
+    if ((tid & 3u) == 0) count[t] = c;
+    __syncthreads();
+    if (wave < kRankTile / 64) {
+        const uint32_t v = wave_scan_inclusive(count[tid]);
+        if (lane == 63) wave_s[wave] = v;
+        count[tid] = v;
+    }
+    __syncthreads();
+    if (tid < kRankTile) {
+        uint32_t rank = count[tid];
+        for (uint32_t k = 0; k < wave; ++k) rank += wave_s[k];
+        int32_t *row = table + (size_t)level * entries;
+        if (u0 + tid < n_units) row[u0 + tid + 1] = (int32_t)rank;
+        if (tid == kRankTile - 1) sums[(size_t)level * tiles + blockIdx.x] = rank;
+    }
+}
+
+static uint32_t rank_tiles(uint64_t n, uint64_t chunk) {
+    const uint64_t n_units = (n + chunk - 1) / chunk;
+    return (uint32_t)std::max<uint64_t>(1, (n_units + kRankTile - 1) / kRankTile);
+}
+
+size_t prefix_workspace_bytes(uint64_t n, uint64_t chunk, int n_levels) {
+    return (size_t)rank_tiles(n, chunk) * (size_t)(n_levels - 1) * 4u;
+}
+
+int launch_prefix_build_ws(const Dev &P, uint32_t chunk, int32_t *table, void *workspace, hipStream_t s) {
+    const uint32_t n_units = (uint32_t)(((uint64_t)P.n + chunk - 1) / chunk);
+    for (int i = 0; i < P.n_levels; ++i)
+        hipLaunchKernelGGL(k_rank_level, dim3(rank_tiles(P.n, chunk)), dim3(kRankThreads), 0, s, P, i, chunk, n_units, table,
+                           static_cast<uint32_t *>(workspace));
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 

@@ -120,6 +120,14 @@ def decode_weight_triton(packed: dict, device=None, dtype=torch.bfloat16) -> tor
 
     assert torch.cuda.is_available(), "the device decoder needs the GPU"
     device = torch.device(device) if device is not None else torch.device("cuda")
+    n = packed["N"]
+    if n and n == packed["out_f"] * packed["in_f"] and device.type == "cuda" and device.index in (None, torch.cuda.current_device()):
+        # in one native call, where every tensor is on the device already
+        w = _lib.host().decode((3, 5, 8), packed["out_f"], packed["in_f"], [packed["b1"], packed["b2"]],
+                               [packed["l1"], packed["l2"], packed["l3"]], None, None, packed["group_scales"],
+                               packed["group_size"])
+        if w is not None:
+            return w if dtype is torch.bfloat16 else w.to(dtype)
     mv = lambda t: t.to(device).contiguous()
     dp = _lib.DevicePacked((3, 5, 8), packed["out_f"], packed["in_f"], [mv(packed["b1"]), mv(packed["b2"])],
                            [mv(packed["l1"]), mv(packed["l2"]), mv(packed["l3"])], None)

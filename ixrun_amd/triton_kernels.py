@@ -59,6 +59,13 @@ def decode_weight_triton(packed: dict, device=None, dtype=torch.bfloat16) -> tor
         raise RuntimeError("decode_weight_triton runs the HIP kernel and needs the GPU; "
                            "decode_weight_scatter is the CPU decoder")
     device = torch.device(device) if device is not None else torch.device("cuda")
+    n = packed["N"]
+    if n and n == packed["out_f"] * packed["in_f"] and device.type == "cuda" and device.index in (None, torch.cuda.current_device()):
+        # in one native call, where every tensor is on the device already
+        w = _lib.host().decode(packed["level_bits"], packed["out_f"], packed["in_f"], packed["bitmaps"], packed["streams"],
+                               packed["scale"], packed.get("table512"), None, 0)
+        if w is not None:
+            return w if dtype is torch.bfloat16 else w.to(dtype)
     dp = _lib.DevicePacked.from_dict(packed, device)
     out = torch.empty(packed["N"], dtype=torch.bfloat16, device=device)
     if packed["N"]:

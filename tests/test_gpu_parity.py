@@ -838,3 +838,23 @@ def test_full_size_calibrated_layer(oracle, dev):
         y = sl(x.to(dev))
         y64 = oracle.gemm_f64(w_bits, bf16_bits(x))
         check_outputs(bf16_bits(y), y64, f"full-size calibrated m={m}")
+
+
+@pytest.mark.parametrize("n_units", [1, 127, 128, 129, 384, 1025])
+@pytest.mark.parametrize("level_bits,chunk", [((3, 5, 8), 512), ((2, 8), 5), ((3, 4, 5, 6, 8), 777), ((1, 2, 3, 4, 5, 6, 7, 8), 33)])
+def test_prefix_build_with_and_without_a_workspace(oracle, dev, n_units, level_bits, chunk):
+    """Both builders against the oracle, around the 128 units of a tile, with the last unit cut short."""
+    import ctypes as C
+
+    from ixrun_amd import _lib
+
+    n = n_units * chunk - chunk // 2
+    p = make_packed("student_t", 1, n, level_bits)
+    dp = device_packed(p, dev)
+    want = oracle.prefix(n, len(level_bits), [b.numpy().view(np.uint32) for b in p["bitmaps"]], chunk)
+    assert np.array_equal(dp.prefix_build(chunk).cpu().numpy(), want)
+    plain = torch.full_like(torch.from_numpy(want), -1).to(dev)
+    _lib.check(_lib.lib().ixh_prefix_build(C.byref(dp.struct), chunk, plain.data_ptr(), _lib.current_stream(dev)))
+    assert np.array_equal(plain.cpu().numpy(), want)
+    rc = _lib.lib().ixh_prefix_build_ws(C.byref(dp.struct), chunk, plain.data_ptr(), plain.data_ptr(), 0, None)
+    assert rc == -4, "a workspace that is too small"
