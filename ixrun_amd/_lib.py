@@ -73,7 +73,8 @@ def host():
                                "there is no fallback path") from e
         L = lib()
         _host.bind(*(C.cast(f, C.c_void_p).value for f in (
-            L.ixh_prefix_entries, L.ixh_prefix_workspace_bytes, L.ixh_prefix_build_ws, L.ixh_decode, L.ixh_decode_gs)), check)
+            L.ixh_prefix_entries, L.ixh_prefix_workspace_bytes, L.ixh_prefix_build_ws, L.ixh_decode, L.ixh_decode_gs,
+            L.ixh_encode_workspace_bytes, L.ixh_encode_scan_counts, L.ixh_encode_wait, L.ixh_encode_pack)), check)
         _native = _host
     return _native
 
@@ -225,12 +226,16 @@ class DevicePacked:
         self.N = self.out_f * self.in_f
         # scale None: the group-scale format, whose scales are an argument of its decode call
         self.tensors = list(bitmaps) + list(streams) + ([scale] if scale is not None else [])
+        self.struct = IxhPacked()
+        if host().describe(C.addressof(self.struct), level_bits, self.out_f, self.in_f, bitmaps, streams, scale):
+            self.device = self.tensors[0].device
+            return
         for i, t in enumerate(self.tensors):
             _require_cuda(t, f"packed tensor {i}")
         if scale is not None and (scale.dtype != torch.bfloat16 or scale.numel() != 1):
             raise ValueError("scale must be a one-element bf16 tensor")
         self.device = self.tensors[0].device
-        s = IxhPacked()
+        s = self.struct  # (tensors of several devices or other subclasses; or what has to raise)
         s.n_levels = n_levels
         s.level_bits[:n_levels] = level_bits
         s.out_f, s.in_f = self.out_f, self.in_f
@@ -247,7 +252,6 @@ class DevicePacked:
         s.last = last.data_ptr() if last.numel() else None
         s.last_bytes = last.numel()
         s.scale = scale.data_ptr() if scale is not None else None
-        self.struct = s
 
     @classmethod
     def from_dict(cls, packed: dict, device=None) -> "DevicePacked":
@@ -463,6 +467,11 @@ def encode_device(weight: torch.Tensor, level_bits) -> tuple:
     n_levels = len(level_bits)
     out_f, in_f = weight.shape
     dev = weight.device
+    if dev.index == torch.cuda.current_device():
+        done = host().encode(weight, level_bits)  # the steps below in one native call
+        if done is not None:
+            bitmaps, streams, scale, table, counts = done
+            return DevicePacked(level_bits, out_f, in_f, bitmaps, streams, scale), table, counts
     L = lib()
     bits = (C.c_int32 * n_levels)(*level_bits)
     entries = int(L.ixh_prefix_entries(out_f * in_f, 512))

@@ -10,6 +10,8 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/hip/HIPStream.h>
+#include <vector>
+
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -159,19 +161,41 @@ struct Library {
     decltype(&ixh_prefix_build_ws) prefix_build;
     decltype(&ixh_decode) decode;
     decltype(&ixh_decode_gs) decode_gs;
+    decltype(&ixh_encode_workspace_bytes) encode_workspace_bytes;
+    decltype(&ixh_encode_scan_counts) encode_scan;
+    decltype(&ixh_encode_wait) encode_wait;
+    decltype(&ixh_encode_pack) encode_pack;
     PyObject *check;
 } library;
 
-// bind(prefix_entries, prefix_workspace_bytes, prefix_build_ws, decode, decode_gs, check): addresses, and what raises for a negative code
+template <class F>
+void entry(F &slot, PyObject *address) {
+    slot = reinterpret_cast<F>(PyLong_AsUnsignedLongLong(address));
+}
+
+// raises what `check` makes of a negative code; false if it did
+bool checked(int rc) {
+    if (!rc) return true;
+    PyObject *r = PyObject_CallFunction(library.check, "i", rc);
+    Py_XDECREF(r);
+    return r != nullptr;
+}
+
+// bind(prefix_entries, prefix_workspace_bytes, prefix_build_ws, decode, decode_gs, encode_workspace_bytes,
+// encode_scan_counts, encode_wait, encode_pack, check): addresses, and what raises for a negative code
 PyObject *bind(PyObject *, PyObject *args) {
-    unsigned long long f[5];
-    PyObject *check;
-    if (!PyArg_ParseTuple(args, "KKKKKO", &f[0], &f[1], &f[2], &f[3], &f[4], &check)) return nullptr;
-    library.prefix_entries = reinterpret_cast<decltype(library.prefix_entries)>(f[0]);
-    library.prefix_workspace_bytes = reinterpret_cast<decltype(library.prefix_workspace_bytes)>(f[1]);
-    library.prefix_build = reinterpret_cast<decltype(library.prefix_build)>(f[2]);
-    library.decode = reinterpret_cast<decltype(library.decode)>(f[3]);
-    library.decode_gs = reinterpret_cast<decltype(library.decode_gs)>(f[4]);
+    PyObject *f[9], *check;
+    if (!PyArg_ParseTuple(args, "OOOOOOOOOO", &f[0], &f[1], &f[2], &f[3], &f[4], &f[5], &f[6], &f[7], &f[8], &check)) return nullptr;
+    entry(library.prefix_entries, f[0]);
+    entry(library.prefix_workspace_bytes, f[1]);
+    entry(library.prefix_build, f[2]);
+    entry(library.decode, f[3]);
+    entry(library.decode_gs, f[4]);
+    entry(library.encode_workspace_bytes, f[5]);
+    entry(library.encode_scan, f[6]);
+    entry(library.encode_wait, f[7]);
+    entry(library.encode_pack, f[8]);
+    if (PyErr_Occurred()) return nullptr;
     Py_INCREF(check);
     Py_XSETREF(library.check, check);
     Py_RETURN_NONE;
@@ -274,18 +298,123 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
             rc = scales ? library.decode_gs(&p, ranks, kUnit, static_cast<const uint16_t *>(scales->const_data_ptr()), group, out, stream)
                         : library.decode(&p, ranks, kUnit, nullptr, out, stream);
     }
-    if (rc) {
-        PyObject *r = PyObject_CallFunction(library.check, "i", rc);
-        Py_XDECREF(r);
-        if (!r) return nullptr;
-    }
+    if (!checked(rc)) return nullptr;
     return THPVariable_Wrap(std::move(w));
+    END_HANDLE_TH_ERRORS
+}
+
+// describe(address of an IxhPacked, level_bits, out_f, in_f, bitmaps, streams, scale): whether it was filled.  Of tensors on
+// one device.
+PyObject *describe_at(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    if (n_args != 7) {
+        PyErr_SetString(PyExc_TypeError, "describe: seven arguments");
+        return nullptr;
+    }
+    IxhPacked *p = reinterpret_cast<IxhPacked *>(PyLong_AsUnsignedLongLong(args[0]));
+    const long long out_f = PyLong_AsLongLong(args[2]), in_f = PyLong_AsLongLong(args[3]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!PyList_CheckExact(args[4]) || PyList_GET_SIZE(args[4]) == 0 || !THPVariable_CheckExact(PyList_GET_ITEM(args[4], 0)))
+        Py_RETURN_FALSE;
+    const at::Tensor &first = THPVariable_Unpack(PyList_GET_ITEM(args[4], 0));
+    if (!first.is_cuda()) Py_RETURN_FALSE;
+    IxhPacked filled;
+    if (!describe(args[1], out_f, in_f, args[4], args[5], args[6], first.get_device(), &filled)) Py_RETURN_FALSE;
+    *p = filled;
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+
+// encode(weight, level_bits): (bitmaps, streams, scale, table, counts) of a contiguous bf16 matrix on the current device.
+// Waits once, for the counts.  The host between the counts' arrival and the packing kernels is time that the GPU idles:
+// 4 us (13 from Python).
+PyObject *encode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    if (n_args != 2 || !library.check) {
+        PyErr_SetString(PyExc_TypeError, "encode: two arguments, after bind");
+        return nullptr;
+    }
+    const int64_t device = c10::hip::current_device();
+    const at::Tensor *w = plain(args[0], at::kBFloat16, device);
+    if (!w || w->dim() != 2 || !PyTuple_CheckExact(args[1])) Py_RETURN_NONE;
+    const int64_t out_f = w->size(0), in_f = w->size(1), n = w->numel();
+    const int levels = (int)PyTuple_GET_SIZE(args[1]);
+    if (n < 1 || levels < 2 || levels > IXH_MAX_LEVELS) Py_RETURN_NONE;
+    IxhPacked p{};
+    p.n_levels = levels;
+    p.out_f = out_f;
+    p.in_f = in_f;
+    for (int i = 0; i < levels; ++i) {
+        p.level_bits[i] = (int32_t)PyLong_AsLong(PyTuple_GET_ITEM(args[1], i));
+        if (PyErr_Occurred()) return nullptr;
+    }
+    const size_t bytes = library.encode_workspace_bytes(out_f, in_f, levels);
+    const int64_t entries = library.prefix_entries(n, 512);
+    std::vector<at::Tensor> bitmaps(levels - 1), streams(levels);
+    at::Tensor scale, table, arrived, scratch;
+    int64_t counts[IXH_MAX_LEVELS];
+    int rc;
+    {
+        pybind11::gil_scoped_release without_gil;
+        const auto options = at::TensorOptions().device(c10::Device(c10::kCUDA, (c10::DeviceIndex)device));
+        ixh_stream_t stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+        const uint16_t *src = static_cast<const uint16_t *>(w->const_data_ptr());
+        scratch = at::empty({(int64_t)bytes}, options.dtype(at::kByte));
+        scale = at::empty({1}, options.dtype(at::kBFloat16));
+        table = at::empty({levels - 1, entries}, options.dtype(at::kInt));
+        arrived = at::empty({levels - 1}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+        int32_t *ranks = static_cast<int32_t *>(table.data_ptr());
+        int64_t *host = static_cast<int64_t *>(arrived.data_ptr());
+        rc = library.encode_scan(src, out_f, in_f, levels, p.level_bits, static_cast<uint16_t *>(scale.data_ptr()), ranks,
+                                 scratch.data_ptr(), bytes, host, stream);
+        if (!rc) {
+            bitmaps[0] = at::empty({(n + 31) / 32}, options.dtype(at::kInt));
+            rc = library.encode_wait(host, levels - 1, stream);
+        }
+        if (!rc) {
+            int64_t left = n;
+            for (int i = 0; i < levels - 1; ++i) {
+                counts[i] = host[i];
+                if (i > 0) bitmaps[i] = at::empty({(left + 31) / 32}, options.dtype(at::kInt));
+                streams[i] = at::empty({(counts[i] * p.level_bits[i] + 31) / 32}, options.dtype(at::kInt));
+                p.bitmap_words[i] = (uint64_t)bitmaps[i].numel();
+                p.stream_words[i] = (uint64_t)streams[i].numel();
+                p.bitmaps[i] = bitmaps[i].numel() ? static_cast<const uint32_t *>(bitmaps[i].data_ptr()) : nullptr;
+                p.streams[i] = streams[i].numel() ? static_cast<const uint32_t *>(streams[i].data_ptr()) : nullptr;
+                left -= counts[i];
+            }
+            counts[levels - 1] = left;
+            streams[levels - 1] = at::empty({left}, options.dtype(at::kByte));
+            p.last_bytes = (uint64_t)left;
+            p.last = left ? static_cast<const uint8_t *>(streams[levels - 1].data_ptr()) : nullptr;
+            p.scale = static_cast<const uint16_t *>(scale.data_ptr());
+            rc = library.encode_pack(src, &p, ranks, stream);
+        }
+    }
+    if (!checked(rc)) return nullptr;
+    PyObject *bm = PyList_New(levels - 1), *st = PyList_New(levels), *cn = PyList_New(levels);
+    bool ok = bm && st && cn;
+    for (int i = 0; ok && i < levels; ++i) {
+        PyObject *s = THPVariable_Wrap(streams[i]), *c = PyLong_FromLongLong(counts[i]);
+        PyObject *b = i < levels - 1 ? THPVariable_Wrap(bitmaps[i]) : nullptr;
+        ok = s && c && (b || i == levels - 1);
+        if (s) PyList_SET_ITEM(st, i, s);
+        if (c) PyList_SET_ITEM(cn, i, c);
+        if (b) PyList_SET_ITEM(bm, i, b);
+    }
+    PyObject *result = ok ? Py_BuildValue("(OONNO)", bm, st, THPVariable_Wrap(scale), THPVariable_Wrap(table), cn) : nullptr;
+    Py_XDECREF(bm);
+    Py_XDECREF(st);
+    Py_XDECREF(cn);
+    return result;
     END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, "The library's entry points."},
     {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(decode)), METH_FASTCALL, "The bf16 weight of packed tensors, or None."},
+    {"describe", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(describe_at)), METH_FASTCALL, "Fills an IxhPacked."},
+    {"encode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(encode)), METH_FASTCALL, "Packed tensors of a bf16 weight, or None."},
     {nullptr, nullptr, 0, nullptr},
 };
 
