@@ -239,6 +239,16 @@ int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
 size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m);
 
 /*
+ * The same for 1 <= m <= 4096 rows, with the weights decoded on chip into matrix-core tiles once per 128 rows (meant for 17
+ * and more) and the bias added before the one rounding.  Returns IXH_EUNSUPPORTED unless in_f and ldx are multiples of 8, x is
+ * 16-byte aligned and m * ldx below 2^31.
+ */
+int ixh_lanes_gemm(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
+                   int64_t ldy, void *workspace, size_t workspace_bytes, ixh_stream_t stream);
+
+size_t ixh_lanes_gemm_workspace_bytes(const IxhLanes *lanes, int32_t m);
+
+/*
  * The encoder on the device, in two steps because the stream lengths depend on the data.
  * Together they replace int8x_quantize (ixrun/quantize.py:41-122, with pack_bits_stream
  * and pack_bitmap of ixrun/bitpack.py:13-61, :87-89) for a bf16 weight that is already in

@@ -97,7 +97,7 @@ EXPORTS = (
     "ixh_encode_workspace_bytes", "ixh_encode_scan", "ixh_encode_scan_counts", "ixh_encode_wait", "ixh_encode_pack",
     "ixh_decode_gs",
     "ixh_lanes_plane_words", "ixh_lanes_cells", "ixh_lanes_pack", "ixh_lanes_list", "ixh_lanes_gemv",
-    "ixh_lanes_gemv_workspace_bytes",
+    "ixh_lanes_gemv_workspace_bytes", "ixh_lanes_gemm", "ixh_lanes_gemm_workspace_bytes",
 )
 TEST_EXPORTS = ("ixh_set_option",)
 
@@ -174,6 +174,10 @@ def lib() -> C.CDLL:
                                      C.c_int64, C.c_void_p, C.c_size_t, C.c_void_p]
         L.ixh_lanes_gemv_workspace_bytes.restype = C.c_size_t
         L.ixh_lanes_gemv_workspace_bytes.argtypes = [C.POINTER(IxhLanes), C.c_int32]
+        L.ixh_lanes_gemm.restype = C.c_int
+        L.ixh_lanes_gemm.argtypes = L.ixh_lanes_gemv.argtypes
+        L.ixh_lanes_gemm_workspace_bytes.restype = C.c_size_t
+        L.ixh_lanes_gemm_workspace_bytes.argtypes = [C.POINTER(IxhLanes), C.c_int32]
         _lib = L
     return _lib
 
@@ -451,6 +455,18 @@ class LanePacked:
 
     def gemv_workspace_bytes(self, m: int) -> int:
         return int(lib().ixh_lanes_gemv_workspace_bytes(C.byref(self.struct), int(m)))
+
+    def gemm_workspace_bytes(self, m: int) -> int:
+        return int(lib().ixh_lanes_gemm_workspace_bytes(C.byref(self.struct), int(m)))
+
+    def gemm(self, x: torch.Tensor, y: torch.Tensor, bias: torch.Tensor = None):
+        """y[m, out_f] = x w^T (+ bias), 17 and more rows; the slices' sums go through memory allocated for the call."""
+        m, dev = x.shape[0], x.device
+        need = self.gemm_workspace_bytes(m)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+        with torch.cuda.device(dev):
+            check(lib().ixh_lanes_gemm(C.byref(self.struct), x.data_ptr(), x.stride(0), bias.data_ptr() if bias is not None else None,
+                                       m, y.data_ptr(), y.stride(0), ws.data_ptr() if need else None, need, current_stream(dev)))
 
 
 def encode_device(weight: torch.Tensor, level_bits) -> tuple:

@@ -602,6 +602,38 @@ int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
     return rc;
 }
 
+constexpr int32_t kLanesGemmMost = 4096;
+
+size_t ixh_lanes_gemm_workspace_bytes(const IxhLanes *lanes, int32_t m) {
+    LanesDev d;
+    if (to_lanes(lanes, &d, true) || m < 1 || m > kLanesGemmMost) return 0;
+    return lanes_gemm_workspace_bytes(d, m);
+}
+
+int ixh_lanes_gemm(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
+                   int64_t ldy, void *workspace, size_t workspace_bytes, ixh_stream_t stream) {
+    LanesDev d;
+    int rc = to_lanes(lanes, &d, true);
+    if (rc) return rc;
+    if (m < 1 || m > kLanesGemmMost) { set_error("m = %d not in 1..%d", m, kLanesGemmMost); return IXH_EINVAL; }
+    if (!x || !y) { set_error("x or y is NULL"); return IXH_EINVAL; }
+    if (m > 1 && (ldx < (int64_t)d.in_f || ldy < (int64_t)d.out_f)) { set_error("ldx or ldy shorter than a row"); return IXH_EINVAL; }
+    if (m == 1) ldx = d.in_f;
+    if (((uintptr_t)x & 15u) || d.in_f % 8u || ldx % 8 || ldx >= (1ll << 31) / m) {
+        set_error("lanes_gemm: x not 16-byte aligned, or rows of %u at a stride of %lld not whole 16-byte pieces within 4 GB",
+                  d.in_f, (long long)ldx);
+        return IXH_EUNSUPPORTED;
+    }
+    const size_t need = lanes_gemm_workspace_bytes(d, m);
+    if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15u))) {
+        set_error("workspace of %zu bytes needed, 16-byte aligned, %zu given", need, workspace ? workspace_bytes : (size_t)0);
+        return IXH_EWORKSPACE;
+    }
+    rc = launch_lanes_gemm(d, x, m, ldx, bias, y, ldy, (float *)workspace, (hipStream_t)stream);
+    if (rc == IXH_ELAUNCH) set_error("lanes_gemm: launch failed");
+    return rc;
+}
+
 static int encode_levels_ok(int32_t n_levels, const int32_t *level_bits) {
     if (n_levels < 2 || n_levels > IXH_MAX_LEVELS) { set_error("n_levels %d not in 2..%d", n_levels, IXH_MAX_LEVELS); return IXH_EINVAL; }
     if (!level_bits) { set_error("level_bits is NULL"); return IXH_EINVAL; }

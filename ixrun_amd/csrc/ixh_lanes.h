@@ -54,5 +54,9 @@ size_t lanes_gemv_workspace_bytes(const LanesDev &L, int m);
 // IXH_EUNSUPPORTED where the activations do not fit the kernels (the caller keeps the packed tensor's kernels)
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                       int64_t ldy, float *ws, hipStream_t s);
+// more rows (ixh_lanes_gemm.hip); x 16-byte aligned, in_f and ldx multiples of 8
+size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m);
+int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
+                      int64_t ldy, float *ws, hipStream_t s);
 
 }  // namespace ixh

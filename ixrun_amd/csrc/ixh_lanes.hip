@@ -1,130 +1,7 @@
 // Products of few activation rows with weights in the lane layout (ixh_lanes.h), and the kernels that write it.
-#include "ixh_lanes.h"
-
-#include "ixh_fast358.h"
+#include "ixh_lanes_dev.h"
 
 namespace ixh {
-
-typedef uint32_t ln_u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t ln_u32x3 __attribute__((ext_vector_type(3)));
-typedef uint32_t ln_u32x2 __attribute__((ext_vector_type(2)));
-typedef short ln_s16x4 __attribute__((ext_vector_type(4)));
-typedef float ln_f32x4 __attribute__((ext_vector_type(4)));
-typedef float ln_f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 ln_bf16x2 __attribute__((ext_vector_type(2)));
-
-constexpr size_t kLnLds = 160 * 1024;
-
-#define LN_LDS(T) __attribute__((address_space(3))) T
-
-__device__ __forceinline__ uint32_t ln_pack(float lo, float hi) {
-    const ln_f32x2 v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, ln_bf16x2));
-}
-
-// ---------------------------------------------------------------------------------------------------------------
-// Pair tables.  A table of dequantised pairs (both weights as bf16) indexed by the 2 * BITS bits of a pair, in
-// 2^kCopies copies side by side so that the lanes of a wave, which read unrelated entries, spread over the banks.
-// A vector shift and an AND take half the issue time of a bit-field extract, a conversion or a packed operation
-// (measured: 2 against 4 clocks a wave instruction), so a pair costs 6 clocks of issue and one LDS read where
-// arithmetic (extract, convert, multiply, round) takes about 20.
-// ---------------------------------------------------------------------------------------------------------------
-template <int BITS, bool WIDE = true> struct LnPairs {
-    // log2: 32 copies of 64 entries never collide; 8 of 1024 leave about half of the collisions (5120 x 17408, 5 bits, one
-    // row: 21.9 us with one copy, 21.1 with eight).  The tile kernel has no LDS to spare for more than two.
-    static constexpr int kCopies = BITS == 3 ? 5 : WIDE ? (BITS == 4 ? 4 : 3) : 1;
-    static constexpr uint32_t kEntries = BITS == 8 ? 0u : 1u << (2 * BITS);
-    static constexpr uint32_t kLutBytes = kEntries << (kCopies + 2);
-    static constexpr uint32_t kMask = ((1u << (2 * BITS)) - 1u) << (kCopies + 2);
-};
-
-template <int BITS, bool WIDE>
-__device__ __forceinline__ void ln_build_lut(uint32_t lut, float scale, uint32_t tid, uint32_t n_threads) {
-    using P = LnPairs<BITS, WIDE>;
-    if constexpr (P::kEntries != 0) {
-        constexpr int T = (1 << (BITS - 1)) - 1;
-        constexpr uint32_t RUN = P::kCopies >= 2 ? 4u : 2u;  // copies a thread stores at a time
-        for (uint32_t e = tid * RUN; e < (P::kEntries << P::kCopies); e += n_threads * RUN) {
-            const uint32_t idx = e >> P::kCopies;
-            const uint32_t v = ln_pack((float)((int)(idx & ((1u << BITS) - 1u)) - T) * scale, (float)((int)(idx >> BITS) - T) * scale);
-            if constexpr (RUN == 4) *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(lut + e * 4u)) = ln_u32x4{v, v, v, v};
-            else *reinterpret_cast<LN_LDS(ln_u32x2) *>((uintptr_t)(lut + e * 4u)) = ln_u32x2{v, v};
-        }
-    }
-}
-
-template <int SH> __device__ __forceinline__ uint32_t ln_shift(uint32_t w) {
-    if constexpr (SH >= 0) return w >> SH;
-    else return w << -SH;
-}
-
-// the sixteen dequantised pairs of a lane's `BITS` dwords
-template <int BITS, bool WIDE>
-__device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lut_lane, float scale, uint32_t (&o)[16]) {
-    using P = LnPairs<BITS, WIDE>;
-    if constexpr (BITS == 8) {
-        // (c - 127) * scale as c * scale - 127 * scale: both products and the difference are exact in fp32
-        const float off = -127.0f * scale;
-#pragma unroll
-        for (int p = 0; p < 16; ++p) {
-            const uint32_t d = w[p >> 1] >> (16 * (p & 1));
-            o[p] = ln_pack(__fmaf_rn((float)(d & 255u), scale, off), __fmaf_rn((float)((d >> 8) & 255u), scale, off));
-        }
-    } else {
-        constexpr int PER = BITS == 4 ? 4 : BITS == 3 ? 5 : 3;  // whole pairs a dword
-        constexpr int FIRST = BITS == 4 ? 0 : 2;
-        constexpr int TO = P::kCopies + 2;
-        uint32_t a[16];
-#define LN_FIELD(d, f) (ln_shift<FIRST + 2 * BITS * (f) - TO>(w[d]) & P::kMask)
-#pragma unroll
-        for (int d = 0; d < BITS; ++d) {
-            a[PER * d] = LN_FIELD(d, 0);
-            a[PER * d + 1] = LN_FIELD(d, 1);
-            a[PER * d + 2] = LN_FIELD(d, 2);
-            if constexpr (PER > 3) a[PER * d + 3] = LN_FIELD(d, 3);
-            if constexpr (PER > 4) a[PER * d + 4] = LN_FIELD(d, 4);
-        }
-#undef LN_FIELD
-        if constexpr (BITS == 3 || BITS == 5) {
-            uint32_t last = 0;
-#pragma unroll
-            for (int d = 0; d < BITS; ++d) last |= (w[d] & 3u) << (TO + 2 * d);
-            a[15] = last;
-        }
-        if constexpr (BITS == 5) {
-            // The last whole pair of a dword by arithmetic, which evens out the LDS and the vector unit: the code next to
-            // the exponent of 1.0 reads as 1 + code / 32, and (1 + code / 32) * 32 scale - 47 scale is value * scale,
-            // every term exact in fp32.
-            const float s32 = 32.0f * scale, off = -47.0f * scale;
-#pragma unroll
-            for (int d = 0; d < 5; ++d) {
-                const float lo = __uint_as_float(((w[d] >> 4) & 0x7C0000u) | 0x3F800000u);
-                const float hi = __uint_as_float(((w[d] >> 9) & 0x7C0000u) | 0x3F800000u);
-                o[PER * d + 2] = ln_pack(__fmaf_rn(lo, s32, off), __fmaf_rn(hi, s32, off));
-            }
-        }
-#pragma unroll
-        for (int p = 0; p < 16; ++p)
-            if (BITS != 5 || p == 15 || p % 3 != 2)
-                o[p] = *reinterpret_cast<const LN_LDS(uint32_t) *>((uintptr_t)(a[p] + lut_lane));
-    }
-}
-
-template <int BITS>
-__device__ __forceinline__ void ln_load_lane(const uint32_t *__restrict__ p, uint32_t lane, uint32_t (&w)[BITS]) {
-    if constexpr (BITS == 3) {
-        const ln_u32x3 v = *reinterpret_cast<const ln_u32x3 *>(p + lane * 3u);
-        w[0] = v[0]; w[1] = v[1]; w[2] = v[2];
-    } else {
-        const ln_u32x4 v = *reinterpret_cast<const ln_u32x4 *>(p + lane * 4u);
-        w[0] = v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
-        if constexpr (BITS == 5) w[4] = p[256u + lane];
-        if constexpr (BITS == 8) {
-            const ln_u32x4 u = *reinterpret_cast<const ln_u32x4 *>(p + 256u + lane * 4u);
-            w[4] = u[0]; w[5] = u[1]; w[6] = u[2]; w[7] = u[3];
-        }
-    }
-}
 
 template <int BITS>
 __device__ __forceinline__ void ln_load(const uint32_t *__restrict__ plane, uint32_t cell, uint32_t lane, uint32_t (&w)[BITS]) {
@@ -382,16 +259,9 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 // one share leaves from its wave, the others' sums meet in LDS and are added in wave order.  The slices' sums meet in
 // the workspace; k_lanes_reduce adds them in slice order.
 // ---------------------------------------------------------------------------------------------------------------
-typedef __bf16 ln_bf16x8 __attribute__((ext_vector_type(8)));
-
 constexpr uint32_t kLtWaves = 16;
 constexpr uint32_t kLtTileBytes = 4096;
 constexpr uint32_t kLtXBytes = 64 * 1024;  // activations of a slice at most
-
-__device__ __forceinline__ void ln_wave_order() {  // LDS accesses of the wave's lanes before this one come first
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 template <int BITS>
 __global__ void __launch_bounds__(kLtWaves *kWave)
@@ -612,12 +482,12 @@ k_lanes_tile(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 
 // outputs from the slices' sums, in slice order
 __global__ void __launch_bounds__(256)
-k_lanes_reduce(const float *__restrict__ ws, uint32_t slices, int m, uint32_t out_f, const uint16_t *__restrict__ bias,
-               uint16_t *__restrict__ y, int64_t ldy) {
+k_lanes_reduce(const float *__restrict__ ws, uint32_t slices, int m, uint32_t out_f, uint32_t ws_ld,
+               const uint16_t *__restrict__ bias, bool once, uint16_t *__restrict__ y, int64_t ldy) {
     const uint32_t row = blockIdx.x * 256u + threadIdx.x, r = blockIdx.y;
     if (row >= out_f) return;
-    const float *p = ws + (size_t)r * out_f + row;
-    const size_t stride = (size_t)m * out_f;
+    const float *p = ws + (size_t)r * ws_ld + row;
+    const size_t stride = (size_t)m * ws_ld;
     float sum = 0.0f;
     for (uint32_t g = 0; g < slices; g += 8) {
         float v[8];
@@ -628,8 +498,15 @@ k_lanes_reduce(const float *__restrict__ ws, uint32_t slices, int m, uint32_t ou
             if (g + k < slices) sum += v[k];
     }
     uint32_t h = f32_to_bf16_bits(sum);
-    if (bias) h = f32_to_bf16_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(bias[row]));
+    if (bias) h = f32_to_bf16_bits((once ? sum : bf16_bits_to_f32(h)) + bf16_bits_to_f32(bias[row]));
     y[(int64_t)r * ldy + row] = (uint16_t)h;
+}
+
+int launch_lanes_reduce(const float *ws, uint32_t slices, int m, uint32_t out_f, uint32_t ws_ld, const uint16_t *bias, bool once,
+                        uint16_t *y, int64_t ldy, hipStream_t s) {
+    hipLaunchKernelGGL(k_lanes_reduce, dim3((out_f + 255u) / 256u, m), dim3(256), 0, s, ws, slices, m, out_f, ws_ld, bias, once,
+                       y, ldy);
+    return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -725,15 +602,6 @@ k_lanes_list(const uint16_t *__restrict__ w, LanesDev L, uint16_t *__restrict__ 
         }
 }
 
-static uint32_t ln_cus() {
-    static const uint32_t n = [] {
-        int dev = 0, v = 256;
-        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev);
-        return (uint32_t)v;
-    }();
-    return n;
-}
-
 int launch_lanes_pack(const uint16_t *w, const LanesDev &L, uint32_t *plane, uint32_t *counts, hipStream_t s) {
     const dim3 grid((L.n_tiles * L.n_cells + 3u) / 4u), block(256);
     switch (L.bits) {
@@ -815,8 +683,7 @@ static int lanes_tile_launch(const LanesDev &L, const uint16_t *x, int m, int64_
     hipLaunchKernelGGL(k_lanes_tile<BITS>, dim3(p.slices * p.groups), dim3(kLtWaves * kWave), fixed + (size_t)cells * 1024u * (uint32_t)m, s,
                        L.plane, x, L.exc_off, L.scale, L.n_cells, L.n_tiles, p.slices, L.in_f, L.exc_pos, L.exc_val, m, ldx, L.out_f,
                        aligned, ws, bias, y, ldy);
-    if (p.slices > 1)
-        hipLaunchKernelGGL(k_lanes_reduce, dim3((L.out_f + 255u) / 256u, m), dim3(256), 0, s, ws, p.slices, m, L.out_f, bias, y, ldy);
+    if (p.slices > 1) return launch_lanes_reduce(ws, p.slices, m, L.out_f, L.out_f, bias, false, y, ldy, s);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 

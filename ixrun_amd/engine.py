@@ -2,8 +2,8 @@
 
 ``StreamingLinear`` keeps a layer's packed streams resident on the GPU and
 serves every forward from them: up to 16 activation rows go through the fused
-decode+GEMV kernel (the bf16 weight never reaches memory), larger batches are
-decoded into a shared bf16 buffer and multiplied with ``F.linear``.
+decode+GEMV kernel (the bf16 weight never reaches memory), prompts of up to 160
+to 512 rows through a fused decode+GEMM, larger ones are decoded into a shared bf16 buffer and multiplied with ``F.linear``.
 ``GraphLinear`` / ``Int8XEngine`` follow the reference's ``ixrun/engine.py``
 (``StreamingLinear`` ``:40-173``, ``GraphLinear`` ``:179-196``,
 ``ResourceScheduler`` ``:202-235``, ``Int8XEngine`` ``:241-516``) and keep its
@@ -18,6 +18,7 @@ import os
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib, gemm_tuning
 from .config import TRITON_BLOCK
@@ -51,12 +52,21 @@ MAX_FUSED_ROWS_WITH_BUFFER_DENSE = 16
 # layers: 5120 x 17408 at 17 / 24 / 32 rows 60 / 70 / 75 us in two calls against 118-120 us fused decode+GEMM and
 # 137 us decode + library GEMM; 17408 x 5120 54 / 60 / 64 us against 120-122 and 87 us.  On 5120 x 5120 the two
 # calls tie with the fused decode+GEMM (37-45 against 44-45 us) and lose to decode + library GEMM (34 us), and three
-# calls for 33 .. 48 rows gain nothing on any shape: large layers and up to 32 rows only.
+# calls for 33 .. 48 rows gain nothing on any shape: large layers and up to 32 rows only.  (A layer with lanes takes
+# them in one pass instead, 5120 x 17408 29-30 us, unless its rows are no whole 16-byte pieces: _lanes_gemm_wins.)
 SPLIT_FUSED_MIN_WEIGHTS = 40_000_000
 # More rows than that: with a shared decode buffer the layer decodes into it and calls the library GEMM
 # (5120 x 5120 five-level on MI355X: 60 us at 32 rows, 84 us at 512); without one it runs the fused
 # decode+GEMM, which keeps the bf16 weight out of HBM altogether but is slower (84 us and 194 us): its
 # decode shares the CU with the matrix-core tiles at two waves per SIMD, the stand-alone decode runs at six.
+
+
+def _plain_call(x) -> bool:
+    """Whether a product of ``x`` that is not torch's own is what the caller gets from ``F.linear``: no gradient, transform or
+    other result type is asked for."""
+    return (not (x.requires_grad and torch.is_grad_enabled()) and forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") is torch.bfloat16))
 
 
 class StreamingLinear(nn.Module):
@@ -114,7 +124,8 @@ class StreamingLinear(nn.Module):
         self._use_triton = True
 
         self._use_fused = True
-        self._gemm_ok = True
+        self._gemm_ok = True  # False: prompts are decoded and multiplied by the library
+        self._gemm_fits = True
         self._split_chunk = 0
         per_row = self.in_features // self._unit
         split = _pick_split(self.in_features) if self.out_features < self.in_features else 1
@@ -164,6 +175,22 @@ class StreamingLinear(nn.Module):
         outputs than inputs go back to the library from 257 rows on."""
         return (self.level_bits[0] == 3 and self.N > (1 << 24) and self.counts[0] * 100 >= self.N * 97
                 and (rows <= 256 or (rows <= 512 and self.in_features >= self.out_features)))
+
+    def _lanes_gemm_wins(self, rows: int) -> bool:
+        """Whether the lanes' decode into matrix-core tiles (``ixh_lanes_gemm``) is the fastest way for a prompt of so many rows.
+
+        MI355X, us, decode + library GEMM or, for tensors almost all level 1, ``ixh_gemm`` before, against this.  5 bits a
+        weight (55 / 40 / 5 %) at 64 / 100 / 160 / 256 rows: 10240 x 5120 61 / 64 / 72 / 82 against 34 / 45 / 59 / 91, 17408 x
+        5120 93 / 100 / 108 / 124 against 58 / 78 / 93 / 146.  3 bits at 64 / 100 / 200 / 256: 10240 x 5120 65 / 66 / 69 / 69
+        against 29 / 35 / 57 / 75, 17408 x 5120 92 / 97 / 107 / 110 against 48 / 55 / 88 / 124.  Below 2**24 weights the decode,
+        the GEMM and the host's way through both weigh more: 12000 x 768 at 256 rows 35 against 29 from a graph, 2048 x 2048
+        23 against 22 (eager: 30 against 22), and up to 2**20 weights 15 against 16 at 512 rows (eager 31 against 19).  Layers
+        of at most 2**18 weights keep decoding into their buffer (12 us against 8), which callers see there."""
+        n = self.N
+        return (self._lanes is not None and self._gemv_flags == 0 and self.in_features % 8 == 0 and n > 1 << 18
+                and rows * self.in_features < 1 << 31
+                and (rows <= 160 or (rows <= 224 and self._lanes.bits <= 4) or (rows <= 256 and n < 1 << 24)
+                     or (rows <= 512 and n <= 1 << 20)))
 
     def _bind(self):
         n_levels = len(self.level_bits)
@@ -242,7 +269,7 @@ class StreamingLinear(nn.Module):
         else:
             fused_rows = 1
         two_calls = (MAX_FUSED_ROWS < rows <= 2 * MAX_FUSED_ROWS and fused_rows == MAX_FUSED_ROWS
-                     and self.N >= SPLIT_FUSED_MIN_WEIGHTS and (lanes or self.counts[0] * 100 >= self.N * 97))
+                     and self.N >= SPLIT_FUSED_MIN_WEIGHTS and (not self._lanes_gemm_wins(rows) if lanes else self.counts[0] * 100 >= self.N * 97))
         plan = False
         if 1 <= rows <= fused_rows or two_calls:
             calls = []
@@ -293,7 +320,17 @@ class StreamingLinear(nn.Module):
                     y = y + self._bias.to(y.dtype)
                 return y
         rows = x.numel() // in_f if in_f else 0
-        if (self._use_fused and self._gemm_ok and x.dtype == torch.bfloat16 and x.is_cuda and rows > MAX_FUSED_ROWS
+        if (self._use_fused and self._gemm_ok and rows > MAX_FUSED_ROWS and x.dtype is torch.bfloat16 and x.is_cuda and x.shape[-1] == in_f
+                and self._lanes_gemm_wins(rows) and _plain_call(x)):
+            x2 = x.reshape(rows, in_f).contiguous()
+            if x2.data_ptr() % 16:
+                x2 = x2.clone()
+            y = torch.empty((rows, self.out_features), dtype=torch.bfloat16, device=x.device)
+            self._lanes.gemm(x2, y, self._bias if self._bias_ptr else None)
+            if self._bias is not None and not self._bias_ptr:
+                y = y + self._bias.to(y.dtype)
+            return y.view(x.shape[:-1] + (self.out_features,))
+        if (self._use_fused and self._gemm_ok and self._gemm_fits and x.dtype == torch.bfloat16 and x.is_cuda and rows > MAX_FUSED_ROWS
                 and x.shape[-1] == self.in_features and self._unit == 512
                 and (self._w_buf is None or self._fused_gemm_wins(rows))):
             # many rows: decode tiles on chip straight into the matrix-core GEMM, no bf16 weight in HBM
@@ -307,7 +344,7 @@ class StreamingLinear(nn.Module):
             except _lib.IxhError as e:
                 if e.code != _lib.IXH_EUNSUPPORTED:
                     raise
-                self._gemm_ok = False  # shape the fused GEMM does not take: decode + GEMM from here on
+                self._gemm_fits = False  # shape the fused GEMM does not take: decode + GEMM from here on
             else:
                 y = y.view(x.shape[:-1] + (self.out_features,))
                 if self._bias is not None:

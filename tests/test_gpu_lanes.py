@@ -69,10 +69,12 @@ def product(lanes, x, out_f, in_f, bias=None):
     return y
 
 
-def check(oracle, p, x, y, bias=None):
+def check(oracle, p, x, y, bias=None, once=False):
     want = oracle.gemm_f64(oracle.decode_packed_bf16(p), bf16_bits(x)).astype(np.float32)
+    if once and bias is not None:
+        want += bias.float().cpu().numpy()[None, :]
     want = oracle.f32_to_bf16_bits(want)
-    if bias is not None:
+    if bias is not None and not once:
         want = oracle.f32_to_bf16_bits(oracle.bf16_bits_to_f32(want) + bias.float().cpu().numpy()[None, :])
     got = oracle.bf16_bits_to_f32(bf16_bits(y)).astype(np.float64)
     assert rel_l2(got, oracle.bf16_bits_to_f32(want)) <= 1e-3
@@ -107,6 +109,73 @@ def test_bias_and_unaligned_activations(oracle, dev, m):
     wide = activations(m, in_f + 9, seed=3).to(dev)
     for x in (wide[:, :in_f], wide[:, 3 : 3 + in_f]):
         check(oracle, p, x.cpu(), product(lanes, x, out_f, in_f, bias.to(dev)), bias)
+
+
+@pytest.mark.parametrize("kind", ["narrow", "rare", "four", "real", "full_row", "wide"])
+@pytest.mark.parametrize("out_f,in_f", [(16, 512), (5, 520), (300, 1032), (67, 4104)])
+def test_many_rows(oracle, dev, kind, out_f, in_f):
+    """The decode into matrix-core tiles: edges of the blocks of 16 activation rows and of the groups of 128, of the blocks
+    of 16 weight rows, of the 128-column stages and of the cells."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    for m in (1, 17, 33, 48, 50, 79, 96, 97, 128, 129, 300):
+        wide = activations(m, in_f + 8, seed=m).to(dev)
+        x, b = wide[:, 8:], bias if m % 2 else None
+        y = [torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+        for t in y:
+            lanes.gemm(x, t, None if b is None else b.to(dev))
+        check(oracle, p, x.cpu(), y[0], b, once=True)
+        assert torch.equal(*y)  # the order of the sums is fixed
+
+
+@pytest.mark.parametrize("out_f,in_f,m", [(4100, 520, 20), (4500, 1536, 130), (20, 33800, 40)])
+def test_many_rows_of_larger_weights(oracle, dev, out_f, in_f, m):
+    """Workgroups with several rounds of blocks, and slices of several cells."""
+    p, lanes = lay_out("real", out_f, in_f, dev)
+    x = activations(m, in_f, seed=m)
+    y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
+    lanes.gemm(x.to(dev), y)
+    check(oracle, p, x, y)
+
+
+def test_prompts_of_a_layer_take_the_lanes_in_every_form(oracle, dev):
+    """What goes to the fused decode+GEMM comes out as from the layer without lanes, whatever the activations' form; what it
+    is not for (gradients, other types, more rows) still goes through the decode."""
+    from ixrun_amd.engine import StreamingLinear
+
+    out_f, in_f = 520, 1032
+    v, scheme, _ = values("real", out_f, in_f)
+    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    layer, plain = StreamingLinear(p, bias=bias), StreamingLinear(p, bias=bias, lanes=False)
+    bufs = [torch.zeros(p["N"], dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    for one, buf in zip((layer, plain), bufs):
+        one._set_shared_buf(buf)
+    wide = activations(160, in_f + 3, seed=5).to(dev)
+    flat = wide.reshape(-1)[3 : 3 + 40 * in_f]  # contiguous, 6 bytes off
+    forms = [wide[:17, :in_f], wide[:, 3:], wide[:33, :in_f].reshape(3, 11, in_f), flat.view(4, 10, in_f), wide[:1, :in_f].expand(20, in_f),
+             wide[:, :in_f].t().contiguous().t(), wide[::2, :in_f]]
+    for x in forms:
+        got, want = layer(x), plain(x)
+        assert got.shape == want.shape and got.dtype == want.dtype and got.is_contiguous()
+        # the library may round its product before it adds the bias: half a bf16 step more on either side
+        assert rel_l2(got.double().cpu().numpy(), want.double().cpu().numpy()) <= 2 ** -8
+        check(oracle, p, x.reshape(-1, in_f).cpu(), got.reshape(-1, out_f), bias, once=True)
+    assert not bool(bufs[0].any())
+    graph, x = torch.cuda.CUDAGraph(), wide[:50, :in_f].contiguous()
+    layer(x)
+    with torch.cuda.graph(graph):
+        y = layer(x)
+    for seed in (1, 2, 3):
+        x.copy_(activations(50, in_f, seed=seed))
+        graph.replay()
+        assert torch.equal(y, layer(x))
+    assert not bool(bufs[0].any())
+    x = wide[:40, :in_f].contiguous().requires_grad_()
+    assert layer(x).requires_grad and bool(bufs[0].any())
+    many = activations(600, in_f, seed=6).to(dev)
+    for x in (many, wide[:40, :in_f].float()):
+        assert rel_l2(layer(x).double().cpu().numpy(), plain(x).double().cpu().numpy()) <= 1e-3
 
 
 def test_one_hot_rows_are_decoded_columns(oracle, dev):
@@ -151,6 +220,11 @@ def test_malformed_lanes_are_refused(dev):
         setattr(s, field, value)
         assert call(s) == -1, field
     assert call(lanes.struct, 0) == -1 and call(lanes.struct, 17) == -1
+    many = lambda x, ldx, m, ws=0: L.ixh_lanes_gemm(C.byref(lanes.struct), x, ldx, None, m, y.data_ptr(), 8, None, ws, None)
+    assert many(x.data_ptr(), 512, 0) == -1 and many(x.data_ptr(), 512, 4097) == -1 and many(None, 512, 1) == -1
+    with pytest.raises(_lib.IxhError, match="16-byte"):
+        _lib.check(many(x.data_ptr() + 2, 512, 1))
+    assert many(x.data_ptr(), 516, 17) == _lib.IXH_EUNSUPPORTED
     assert L.ixh_lanes_plane_words(8, 512, 7) == -1 and L.ixh_lanes_cells(0, 512) == -1
 
 
