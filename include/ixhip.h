@@ -231,7 +231,7 @@ int ixh_lanes_list(const uint16_t *w, const IxhLanes *dst, ixh_stream_t stream);
 /*
  * y[j, r] = bf16( sum_k f32(x[j, k]) * f32(w[r, k]) ) [ + bias[r], the sum rounded to bf16 again ], 1 <= m <= 16, as
  * ixh_gemv computes it from the packed tensor.  bias may be NULL.  Partial sums go to `workspace`
- * (ixh_lanes_gemv_workspace_bytes, may be 0).  Returns IXH_EUNSUPPORTED where the activations do not fit the kernels.
+ * (ixh_lanes_gemv_workspace_bytes, may be 0).
  */
 int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
                    int64_t ldy, void *workspace, size_t workspace_bytes, ixh_stream_t stream);

@@ -580,7 +580,7 @@ int ixh_lanes_list(const uint16_t *w, const IxhLanes *dst, ixh_stream_t stream) 
 size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m) {
     LanesDev d;
     if (to_lanes(lanes, &d, true) || m < 1 || m > 16) return 0;
-    return lanes_gemv_workspace_bytes(d, m);
+    return lanes_gemm_workspace_bytes(d, m);
 }
 
 int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
@@ -591,14 +591,13 @@ int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
     if (m < 1 || m > 16) { set_error("m = %d not in 1..16", m); return IXH_EINVAL; }
     if (!x || !y) { set_error("x or y is NULL"); return IXH_EINVAL; }
     if (m > 1 && (ldx < (int64_t)d.in_f || ldy < (int64_t)d.out_f)) { set_error("ldx or ldy shorter than a row"); return IXH_EINVAL; }
-    const size_t need = lanes_gemv_workspace_bytes(d, m);
+    const size_t need = lanes_gemm_workspace_bytes(d, m);
     if (need && (!workspace || workspace_bytes < need)) {
         set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
         return IXH_EWORKSPACE;
     }
     rc = launch_lanes_gemv(d, x, m, ldx, bias, y, ldy, (float *)workspace, (hipStream_t)stream);
     if (rc == IXH_ELAUNCH) set_error("lanes_gemv: launch failed");
-    if (rc == IXH_EUNSUPPORTED) set_error("lanes_gemv: %d activation rows of %u do not fit", m, d.in_f);
     return rc;
 }
 
@@ -618,18 +617,17 @@ int ixh_lanes_gemm(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
     if (m < 1 || m > kLanesGemmMost) { set_error("m = %d not in 1..%d", m, kLanesGemmMost); return IXH_EINVAL; }
     if (!x || !y) { set_error("x or y is NULL"); return IXH_EINVAL; }
     if (m > 1 && (ldx < (int64_t)d.in_f || ldy < (int64_t)d.out_f)) { set_error("ldx or ldy shorter than a row"); return IXH_EINVAL; }
-    if (m == 1) ldx = d.in_f;
-    if (((uintptr_t)x & 15u) || d.in_f % 8u || ldx % 8 || ldx >= (1ll << 31) / m) {
+    if (!lanes_gemm_aligned(d, x, m, ldx)) {
         set_error("lanes_gemm: x not 16-byte aligned, or rows of %u at a stride of %lld not whole 16-byte pieces within 4 GB",
                   d.in_f, (long long)ldx);
         return IXH_EUNSUPPORTED;
     }
     const size_t need = lanes_gemm_workspace_bytes(d, m);
-    if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15u))) {
-        set_error("workspace of %zu bytes needed, 16-byte aligned, %zu given", need, workspace ? workspace_bytes : (size_t)0);
+    if (need && (!workspace || workspace_bytes < need)) {
+        set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
         return IXH_EWORKSPACE;
     }
-    rc = launch_lanes_gemm(d, x, m, ldx, bias, y, ldy, (float *)workspace, (hipStream_t)stream);
+    rc = launch_lanes_gemm(d, x, m, ldx, bias, true, y, ldy, (float *)workspace, (hipStream_t)stream);
     if (rc == IXH_ELAUNCH) set_error("lanes_gemm: launch failed");
     return rc;
 }

@@ -1,5 +1,5 @@
 // The lane layout: a second form of a packed tensor in which every code has a fixed place, made once when a layer is
-// deployed and read by the products of up to 16 activation rows (ixh_lanes.hip).
+// deployed and read by the products of up to 16 activation rows (ixh_lanes.hip) and of prompts (ixh_lanes_gemm.hip).
 //
 // The nested-bitmap streams locate a code by the number of codes before it, so a kernel that reads them spends most
 // of its time on ranks: prefix sums over bitmap words, windows at bit offsets that depend on them, a splice or a
@@ -50,13 +50,14 @@ struct LanesDev {
 
 int launch_lanes_pack(const uint16_t *w, const LanesDev &L, uint32_t *plane, uint32_t *counts, hipStream_t s);
 int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_t *val, hipStream_t s);
-size_t lanes_gemv_workspace_bytes(const LanesDev &L, int m);
-// IXH_EUNSUPPORTED where the activations do not fit the kernels (the caller keeps the packed tensor's kernels)
+// up to 16 rows
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                       int64_t ldy, float *ws, hipStream_t s);
-// more rows (ixh_lanes_gemm.hip); x 16-byte aligned, in_f and ldx multiples of 8
+// 5 and more rows (ixh_lanes_gemm.hip); IXH_EUNSUPPORTED for more than 16 unless lanes_gemm_aligned: x 16-byte aligned, in_f
+// and ldx multiples of 8, x within 4 GB.  once: the bias is added before the one rounding
+bool lanes_gemm_aligned(const LanesDev &L, const uint16_t *x, int m, int64_t ldx);
 size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m);
-int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
+int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once, uint16_t *y,
                       int64_t ldy, float *ws, hipStream_t s);
 
 }  // namespace ixh

@@ -244,242 +244,6 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     }
 }
 
-// ---------------------------------------------------------------------------------------------------------------
-// k_lanes_tile<BITS>: 5 to 16 activation rows (fewer where those of a whole row do not fit k_lanes_gemv).
-//
-// Bound: LDS, close to HBM.  v_mfma_f32_16x16x32_bf16: sixteen weight rows (a block of four row quads) x sixteen
-// activation rows.  A workgroup owns a run of blocks and a slice of the columns, whose activations it copies to LDS in
-// operand order (read from global memory they would be sixteen rows apart, one 16-byte access per lane: 37 us instead of
-// the time below for sixteen rows).  A wave takes 16 x 128 weights at a time: it decodes them to its own 4 KB of
-// LDS in operand order, stores the listed elements over their places, and reads the operands back, each lane its own
-// eight weights.  Nothing is shared between the waves on the way, so there is no barrier in the loop; codes and list are
-// asked for one cell ahead.
-//
-// The cell columns (16 x 512) of a workgroup's blocks are dealt to its waves in contiguous shares, blocks first: a block that lies in
-// one share leaves from its wave, the others' sums meet in LDS and are added in wave order.  The slices' sums meet in
-// the workspace; k_lanes_reduce adds them in slice order.
-// ---------------------------------------------------------------------------------------------------------------
-constexpr uint32_t kLtWaves = 16;
-constexpr uint32_t kLtTileBytes = 4096;
-constexpr uint32_t kLtXBytes = 64 * 1024;  // activations of a slice at most
-
-template <int BITS>
-__global__ void __launch_bounds__(kLtWaves *kWave)
-k_lanes_tile(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
-             const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t n_tiles, uint32_t slices, uint32_t in_f,
-             const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, int m, int64_t ldx, uint32_t out_f,
-             bool x_aligned, float *__restrict__ ws, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t ln_smem[];
-    using P = LnPairs<BITS, false>;
-    const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)ln_smem;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, M = (uint32_t)m;
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const uint32_t n_blocks = (n_tiles + 3u) / 4u, groups = gridDim.x / slices;
-    const uint32_t slice = blockIdx.x % slices, group = blockIdx.x / slices;
-    const uint32_t c0 = slice * n_cells / slices, c1 = (slice + 1u) * n_cells / slices;
-    const uint32_t b0 = group * n_blocks / groups, b1 = (group + 1u) * n_blocks / groups;
-    const uint32_t block_len = c1 - c0, total = (b1 - b0) * block_len;  // cells of a block, of the workgroup
-    const uint32_t u0 = wave * total / kLtWaves, u1 = (wave + 1u) * total / kLtWaves;
-    const uint32_t tile_at = smem + P::kLutBytes + wave * kLtTileBytes;
-    // a wave's sums of the block that it begins in, [wave][activation row][weight row]; those of its last one: in its tile
-    float *const tiles = reinterpret_cast<float *>(ln_smem + P::kLutBytes);
-    float *const red = reinterpret_cast<float *>(ln_smem + P::kLutBytes + kLtWaves * kLtTileBytes);
-    const uint32_t x_at = smem + P::kLutBytes + kLtWaves * (kLtTileBytes + 1024u);
-
-    const uint32_t n = lane & 15u, kg = lane >> 4;
-    // Requests are made for cells past the share's end too (the last one again), and never inside a branch: the compiler
-    // counts what is in flight.
-    struct Cell { uint32_t block, c; };
-    const uint32_t v0 = min(u0, total - 1u);
-    Cell now{b0 + v0 / block_len, c0 + v0 % block_len};
-    uint32_t to_come = max(u1, u0 + 1u) - u0 - 1u;  // cells of the share behind the one asked for last
-    auto advance = [&](Cell &k) {
-        if (to_come == 0) return;
-        --to_come;
-        if (++k.c == c1) { k.c = c0; ++k.block; }
-    };
-    uint32_t w[4][BITS];
-    auto codes = [&](const Cell &k, uint32_t q) {
-        const uint32_t t = min(4u * k.block + (n >> 2), n_tiles - 1u);
-        const uint8_t *const cell = reinterpret_cast<const uint8_t *>(plane) + (t * n_cells + k.c) * (256u * BITS);  // (below 2^31)
-        ln_load_lane<BITS>(reinterpret_cast<const uint32_t *>(cell), 16u * q + 4u * kg + (n & 3u), w[q]);
-    };
-    // the list of row quad kg of the block in the cell; quads first + n, + 16 and + 32 are this lane's (at 5 % listed
-    // elements the fullest of four rows has 31 in 512 columns, 48 are five standard deviations away)
-    constexpr uint32_t ROUNDS = 3;
-    struct Extent { uint32_t first, end; };
-    auto extent = [&](const Cell &k) {
-        const uint32_t t = 4u * k.block + kg, cell = min(t, n_tiles - 1u) * n_cells + k.c;
-        const uint32_t a = exc_off[cell], b = exc_off[cell + 1u];
-        return Extent{a, t < n_tiles ? b : a};
-    };
-    struct Quads { ln_u32x2 pos[ROUNDS]; uint32_t val[ROUNDS]; };
-    auto quads = [&](const Extent &e) {
-        Quads l;
-#pragma unroll
-        for (uint32_t r = 0; r < ROUNDS; ++r) {
-            const uint32_t at = e.first + n + 16u * r < e.end ? e.first + n + 16u * r : 0u;
-            l.pos[r] = *reinterpret_cast<const ln_u32x2 *>(reinterpret_cast<const uint8_t *>(exc_pos) + at * 8u);
-            l.val[r] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(exc_val) + at * 4u);
-        }
-        return l;
-    };
-
-    // ---- first requests; activations (8 pieces x 8 rows a wave and turn) and pair table to LDS ----
-    const uint32_t pieces = (c1 - c0) * 64u, m_groups = (M + 7u) / 8u, chunks = (pieces / 8u) * m_groups;
-    Cell far = now;
-    Extent e_now = extent(far);
-    const uint32_t in_8 = in_f & ~7u;
-    if (x_aligned) {
-        for (uint32_t chunk = wave; chunk < chunks; chunk += 4u * kLtWaves) {
-            ln_u32x4 v[4];
-            uint32_t to[4];
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) {
-                const uint32_t ch = min(chunk + k * kLtWaves, chunks - 1u), pg = ch / m_groups;
-                const uint32_t r = min((ch - pg * m_groups) * 8u + (lane & 7u), M - 1u), p = pg * 8u + (lane >> 3);
-                to[k] = x_at + (p * M + r) * 16u;
-                // (whole pieces of the row; what lies past them is written below)
-                v[k] = *reinterpret_cast<const ln_u32x4 *>(x + (int64_t)r * ldx + min(c0 * kLnCols + p * 8u, in_8 - 8u));
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)to[k]) = v[k];
-        }
-    }
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) codes(far, q);
-    Quads list = quads(e_now);
-    advance(far);
-    Extent e_next = extent(far);
-    const float scale = bf16_bits_to_f32(*scale_at);
-    ln_build_lut<BITS, false>(smem, scale, tid, kLtWaves * kWave);
-    __syncthreads();
-    {   // pieces that are no whole ones of an aligned row, element by element; zero past the row
-        const uint32_t from = x_aligned ? max(in_8, c0 * kLnCols) : c0 * kLnCols, to = c1 * kLnCols;
-        if (from < to) {
-            for (uint32_t e = tid; e < (to - from) / 8u * M; e += kLtWaves * kWave) {
-                const uint32_t piece = e / M, r = e - piece * M, col = from + piece * 8u;
-                uint32_t h[8];
-#pragma unroll
-                for (uint32_t k = 0; k < 8; ++k) h[k] = col + k < in_f ? x[(int64_t)r * ldx + col + k] : 0u;
-                *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + ((col / 8u - c0 * 64u) * M + r) * 16u)) =
-                    ln_u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
-            }
-            __syncthreads();
-        }
-    }
-    const uint32_t lut_lane = smem + ((lane & ((1u << P::kCopies) - 1u)) << 2);
-    const uint32_t xa = x_at + (kg * M + min(n, M - 1u)) * 16u;  // (rows past the last: any, their sums are not used)
-
-    auto out = [&](uint32_t row, uint32_t r, float sum) {
-        if (row >= out_f || r >= M) return;
-        if (slices > 1u) {
-            ws[((size_t)slice * M + r) * out_f + row] = sum;
-        } else {
-            uint32_t h = f32_to_bf16_bits(sum);
-            if (bias) h = f32_to_bf16_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(bias[row]));
-            y[(int64_t)r * ldy + row] = (uint16_t)h;
-        }
-    };
-
-    ln_f32x4 acc = {0, 0, 0, 0};
-    uint32_t block_first = u0;  // first of this wave's cells in the block
-    for (uint32_t u = u0; u < u1; ++u) {
-        // ---- listed elements: value (high half), where it goes in the tile of its quarter (bits 0..11; the tile's block i
-        // is at i ^ q, as the list has it), the quarter (bits 12..14; none of the four where there is no element) ----
-        uint32_t put[4 * ROUNDS];
-#pragma unroll
-        for (uint32_t r = 0; r < ROUNDS; ++r) {
-            const uint32_t val = e_now.first + n + 16u * r < e_now.end ? list.val[r] : 0u;
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) {
-                const uint32_t p = (k & 1) ? list.pos[r][k >> 1] >> 16 : list.pos[r][k >> 1];
-                const int v = (int)(val << (24 - 8 * k)) >> 24;
-                put[4 * r + k] = (ln_pack(0.0f, (float)v * scale) & 0xFFFF0000u) | (v != 0 ? (p & 0x300u) << 4 : 0x4000u) |
-                                 (((p & 0xF0u) << 4) + (p & 14u) + (kg << 6) + k * 16u);
-            }
-        }
-        bool any[ROUNDS];
-#pragma unroll
-        for (uint32_t r = 0; r < ROUNDS; ++r) any[r] = __any(e_now.first + 16u * r < e_now.end);
-        const bool more = __any(e_now.first + 16u * ROUNDS < e_now.end);
-        const Extent e_more = e_now;
-        e_now = e_next;
-        list = quads(e_now);
-        const Cell next = far;
-        advance(far);
-        e_next = extent(far);
-        const uint32_t x_c = xa + (now.c - c0) * 1024u * M;
-#pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-            uint32_t o[16];
-            ln_decode<BITS, false>(w[q], lut_lane, scale, o);
-            codes(next, q);
-#pragma unroll
-            for (uint32_t i = 0; i < 4; ++i)
-                *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(tile_at + ((i ^ q) << 10) + lane * 16u)) =
-                    ln_u32x4{o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]};
-            ln_wave_order();
-#pragma unroll
-            for (uint32_t r = 0; r < ROUNDS; ++r)
-                if (any[r])
-#pragma unroll
-                    for (uint32_t e = 4 * r; e < 4 * r + 4; ++e)
-                        if ((put[e] & 0x7000u) == (q << 12))
-                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + (put[e] & 0xFFFu))) = (uint16_t)(put[e] >> 16);
-            if (more) {  // rows with yet more listed elements in the cell
-                for (uint32_t f = e_more.first + n + 16u * ROUNDS; f < e_more.end; f += 16u)
-                    for (uint32_t k = 0; k < 4; ++k) {
-                        const uint32_t p = exc_pos[(size_t)f * 4u + k];
-                        const int v = exc_val[(size_t)f * 4u + k];
-                        if (v != 0 && (p & 0x300u) == (q << 8))
-                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + (kg << 6) + k * 16u + ((p & 0xF0u) << 4) + (p & 14u))) =
-                                (uint16_t)(ln_pack((float)v * scale, 0.0f) & 0xFFFFu);
-                    }
-            }
-            ln_wave_order();
-#pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) {
-                const ln_u32x4 b = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(tile_at + ((i ^ q) << 10) + lane * 16u));
-                const ln_u32x4 a = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(x_c + (q * 16u + i * 4u) * 16u * M));
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ln_bf16x8, a), __builtin_bit_cast(ln_bf16x8, b), acc, 0, 0, 0);
-            }
-            ln_wave_order();
-        }
-        if (u + 1u == u1 || now.c + 1u == c1) {  // this wave's part of the block is complete
-            const uint32_t from = (now.block - b0) * block_len;
-            const bool whole = block_first <= from && u + 1u == from + block_len;
-            float *const part = u + 1u == u1 ? tiles + wave * (kLtTileBytes / 4u) : red + wave * 256u;
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) {
-                if (whole) out(now.block * 16u + n, 4u * kg + k, acc[k]);
-                else part[(4u * kg + k) * 16u + n] = acc[k];
-            }
-            acc = ln_f32x4{0, 0, 0, 0};
-            block_first = u + 1u;
-        }
-        if (++now.c == c1) { now.c = c0; ++now.block; }
-    }
-    __syncthreads();
-
-    // ---- blocks that lie in several shares: their waves' sums in wave order, a wave a block ----
-    for (uint32_t b = wave; b < b1 - b0; b += kLtWaves) {
-        const uint32_t from = b * block_len, to = from + block_len;
-        bool shared = true;
-        ln_f32x4 sum = {0, 0, 0, 0};
-#pragma unroll
-        for (uint32_t k = 0; k < kLtWaves; ++k) {
-            const uint32_t a0 = k * total / kLtWaves, a1 = (k + 1u) * total / kLtWaves;
-            if (a0 >= a1 || a1 <= from || a0 >= to) continue;
-            if (a0 <= from && a1 >= to) shared = false;
-            sum += *reinterpret_cast<const ln_f32x4 *>((a1 <= to ? tiles + k * (kLtTileBytes / 4u) : red + k * 256u) + lane * 4u);
-        }
-        if (shared)
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) out((b0 + b) * 16u + ((lane * 4u + k) & 15u), lane >> 2, sum[k]);
-    }
-}
-
 // outputs from the slices' sums, in slice order
 __global__ void __launch_bounds__(256)
 k_lanes_reduce(const float *__restrict__ ws, uint32_t slices, int m, uint32_t out_f, uint32_t ws_ld,
@@ -624,6 +388,7 @@ int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
+// (fewer rows than five where those of whole rows do not fit k_lanes_gemv go to k_lanes_gemm as well)
 template <int BITS, int MT>
 static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                              int64_t ldy, hipStream_t s) {
@@ -651,42 +416,6 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
-// How the tile kernel's work is cut: `slices` of the columns, few enough for the activations of one to fit, and the
-// blocks of 16 rows in as many groups as leave a workgroup per CU.  Of all such cuts the one whose fullest wave has the
-// fewest cells, then whose workgroups have; a further slice counts as a cell, for its sums' way through memory.
-struct LtPlan { uint32_t slices, groups; };
-static LtPlan lt_plan(const LanesDev &L, int m) {
-    const uint32_t blocks = (L.n_tiles + 3u) / 4u, cus = ln_cus();
-    const uint32_t most_cells = max(kLtXBytes / (1024u * (uint32_t)m), 1u);
-    LtPlan best{1, 1};
-    uint64_t best_cost = ~0ull;
-    for (uint32_t s = (L.n_cells + most_cells - 1u) / most_cells; s <= min(L.n_cells, cus); ++s) {
-        const uint32_t groups = min(max(cus / s, 1u), blocks);
-        const uint32_t cells = ((blocks + groups - 1u) / groups) * ((L.n_cells + s - 1u) / s);
-        const uint64_t cost = (uint64_t)((cells + kLtWaves - 1u) / kLtWaves) * 64u + cells + s;
-        if (cost < best_cost) { best_cost = cost; best = {s, groups}; }
-    }
-    return best;
-}
-
-template <int BITS>
-static int lanes_tile_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
-                             int64_t ldy, float *ws, hipStream_t s) {
-    constexpr size_t fixed = LnPairs<BITS, false>::kLutBytes + kLtWaves * (kLtTileBytes + 1024u);
-    static_assert(fixed + kLtXBytes <= kLnLds, "LDS of a CU");
-    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_tile<BITS>),
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
-    if (!raised) return IXH_ELAUNCH;
-    const LtPlan p = lt_plan(L, m);
-    const uint32_t cells = (L.n_cells + p.slices - 1u) / p.slices;
-    const bool aligned = ((uintptr_t)x & 15u) == 0 && (m == 1 || ldx % 8 == 0);
-    hipLaunchKernelGGL(k_lanes_tile<BITS>, dim3(p.slices * p.groups), dim3(kLtWaves * kWave), fixed + (size_t)cells * 1024u * (uint32_t)m, s,
-                       L.plane, x, L.exc_off, L.scale, L.n_cells, L.n_tiles, p.slices, L.in_f, L.exc_pos, L.exc_val, m, ldx, L.out_f,
-                       aligned, ws, bias, y, ldy);
-    if (p.slices > 1) return launch_lanes_reduce(ws, p.slices, m, L.out_f, L.out_f, bias, false, y, ldy, s);
-    return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
-}
-
 template <int BITS>
 static int lanes_gemv_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                            int64_t ldy, float *ws, hipStream_t s) {
@@ -694,13 +423,7 @@ static int lanes_gemv_rows(const LanesDev &L, const uint16_t *x, int m, int64_t 
     if (m == 1) rc = lanes_gemv_launch<BITS, 1>(L, x, m, ldx, bias, y, ldy, s);
     else if (m == 2) rc = lanes_gemv_launch<BITS, 2>(L, x, m, ldx, bias, y, ldy, s);
     else if (m <= 4) rc = lanes_gemv_launch<BITS, 4>(L, x, m, ldx, bias, y, ldy, s);
-    if (rc == IXH_EUNSUPPORTED) rc = lanes_tile_launch<BITS>(L, x, m, ldx, bias, y, ldy, ws, s);
-    return rc;
-}
-
-size_t lanes_gemv_workspace_bytes(const LanesDev &L, int m) {
-    const LtPlan p = lt_plan(L, m);
-    return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * L.out_f * sizeof(float) : 0;
+    return rc == IXH_EUNSUPPORTED ? launch_lanes_gemm(L, x, m, ldx, bias, false, y, ldy, ws, s) : rc;
 }
 
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,

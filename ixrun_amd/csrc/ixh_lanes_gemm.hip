@@ -1,10 +1,11 @@
-// Products of 17 and more activation rows with weights in the lane layout (ixh_lanes.h).
+// Products of 5 and more activation rows with weights in the lane layout (ixh_lanes.h).
 #include "ixh_lanes_dev.h"
 
 namespace ixh {
 
 // ---------------------------------------------------------------------------------------------------------------
-// k_lanes_gemm<BITS, MB>: up to 16 * MB activation rows at a time, MB <= 8.
+// k_lanes_gemm<BITS, MB, NB, ALIGNED>: up to 16 * MB activation rows at a time, MB <= 8; NB blocks of 16 weight rows a wave (two from
+// MB = 4 on: an activation operand that is read serves both); activations that are no whole 16-byte pieces: MB = 1 only.
 //
 // Bound: LDS bandwidth (per 16 x 128 weights a wave reads 4 MB KB of activations, writes and reads 8 KB of weights and
 // looks up 4 KB of pairs; the matrix unit needs a third of that time).  A wave takes 16 weight rows x 128 columns a
@@ -16,6 +17,10 @@ namespace ixh {
 //
 // A workgroup owns a slice of the columns (whole cells) of a run of 16-row blocks, sixteen at most at a time; the slices' sums
 // meet in the workspace and launch_lanes_reduce adds them in slice order.
+//
+// 5 to 16 rows: a kernel of waves with 16 x 512 weights and columns of their own, without the barrier and with all activations of a
+// slice in LDS, took longer at every size: us of a layer in a graph at 8 rows 16.6 against 10.1 (288 x 8192, 5 bits), 20.7
+// against 16.5 (5120 x 5120), 37.2 against 35.6 (17408 x 5120), 3 bits 28.0 against 27.4 (5120 x 17408).
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kLgBlocks = 16;  // of 16 weight rows, in work at a time
 constexpr uint32_t kLgTileBytes = 4096;
@@ -23,12 +28,13 @@ constexpr uint32_t kLgMost = 8;  // blocks of 16 activation rows
 
 __device__ __forceinline__ void lg_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int BITS, int MB, int NB>
+template <int BITS, int MB, int NB, bool ALIGNED>
 __global__ void __launch_bounds__(kLgBlocks / NB *kWave)
 k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
              const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t n_tiles, uint32_t slices, uint32_t groups,
-             const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, uint32_t in_f, uint32_t m_all, uint32_t ldx,
-             uint32_t out_f, float *__restrict__ ws, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy) {
+             const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, uint32_t in_f, uint32_t m_all, int64_t ldx,
+             uint32_t out_f, float *__restrict__ ws, bool ws_aligned, const uint16_t *__restrict__ bias, bool once,
+             uint16_t *__restrict__ y, int64_t ldy) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lg_smem[];
     using P = LnPairs<BITS, false>;
     constexpr uint32_t kThreads = kLgBlocks / NB * kWave;
@@ -58,7 +64,16 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 #pragma unroll
         for (uint32_t k = 0; k < XP; ++k) {
             const uint32_t e = min(tid + k * kThreads, MB * 256u - 1u), row = min(row0 + (e >> 8) * 16u + (e & 15u), m_last);
-            r.v[k] = *reinterpret_cast<const ln_u32x4 *>(reinterpret_cast<const uint8_t *>(x) + 2u * (row * ldx + min(x_col(e, g), in_f - 8u)));
+            if constexpr (ALIGNED) {  // (the activations lie within 4 GB)
+                const uint32_t at = row * (uint32_t)ldx + min(x_col(e, g), in_f - 8u);
+                r.v[k] = *reinterpret_cast<const ln_u32x4 *>(reinterpret_cast<const uint8_t *>(x) + 2u * at);
+            } else {
+                uint32_t h[8];
+#pragma unroll
+                for (uint32_t i = 0; i < 8; ++i) h[i] = x_col(e, g) + i < in_f ? x[(int64_t)row * ldx + x_col(e, g) + i] : 0u;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r.v[k][i] = h[2 * i] | (h[2 * i + 1] << 16);
+            }
         }
         return r;
     };
@@ -102,7 +117,8 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         const uint8_t *const cell = reinterpret_cast<const uint8_t *>(plane) + (t * n_cells + k.c) * (256u * BITS);  // (below 2^31)
         ln_load_lane<BITS>(reinterpret_cast<const uint32_t *>(cell), 16u * q + 4u * kg + (n & 3u), w[j][q & 1u]);
     };
-    // the list of row quad kg of the block in the cell, as k_lanes_tile takes it
+    // the list of row quad kg of the block in the cell; quads first + n, + 16 and + 32 are this lane's (at 5 % listed
+    // elements the fullest of four rows has 31 in 512 columns, 48 are five standard deviations away)
     constexpr uint32_t ROUNDS = 3;
     struct Extent { uint32_t first, end; };
     auto extent = [&](const Cell &k, uint32_t j) {
@@ -148,7 +164,8 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 #pragma unroll
         for (int b = 0; b < MB; ++b) acc[j][b] = ln_f32x4{0, 0, 0, 0};
     for (uint32_t u = 0; u < total; ++u) {
-        // ---- listed elements, as in k_lanes_tile: value, place in the tile of its quarter, the quarter ----
+        // ---- listed elements: value (high half), where it goes in the tile of its quarter (bits 0..11; the tile's block i
+        // is at i ^ q, as the list has it), the quarter (bits 12..14; none of the four where there is no element) ----
         uint32_t put[NB][4 * ROUNDS];
         bool any[NB][ROUNDS], more[NB];
 #pragma unroll
@@ -257,13 +274,18 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
                 for (int b = 0; b < MB; ++b, r += 16u) {
                     if (mine && r < m_all) {
                         if (slices > 1u) {
-                            *reinterpret_cast<ln_f32x4 *>(ws + ((size_t)slice * m_all + r) * (n_blocks * 16u) + at) = acc[j][b];
+                            float *const to = ws + ((size_t)slice * m_all + r) * (n_blocks * 16u) + at;
+                            if (ws_aligned) *reinterpret_cast<ln_f32x4 *>(to) = acc[j][b];
+                            else
+#pragma unroll
+                                for (uint32_t k = 0; k < 4; ++k) to[k] = acc[j][b][k];
                         } else {
 #pragma unroll
                             for (uint32_t k = 0; k < 4; ++k) {
                                 if (at + k >= out_f) continue;
-                                const float sum = bias ? acc[j][b][k] + bf16_bits_to_f32(bias[at + k]) : acc[j][b][k];
-                                y[(int64_t)r * ldy + at + k] = (uint16_t)f32_to_bf16_bits(sum);
+                                uint32_t h = f32_to_bf16_bits(acc[j][b][k]);
+                                if (bias) h = f32_to_bf16_bits((once ? acc[j][b][k] : bf16_bits_to_f32(h)) + bf16_bits_to_f32(bias[at + k]));
+                                y[(int64_t)r * ldy + at + k] = (uint16_t)h;
                             }
                         }
                     }
@@ -276,7 +298,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     }
 }
 
-// How the work is cut: groups of 32 .. 128 activation rows, slices of the columns and groups of 16-row blocks, a workgroup
+// How the work is cut: groups of 16 .. 128 activation rows, slices of the columns and groups of 16-row blocks, a workgroup
 // per CU. Of all such cuts the one with the shortest estimate, in clocks. A stage takes 3000 + 400 MB from its first request
 // to its last product, whether 3 or 13 blocks share it (measured: 4.0 to 6.1 thousand for MB = 3, 7.0 to 8.4 thousand for MB
 // = 8), unless LDS, at 128 bytes a clock, is fuller than that; the slices' sums cost a launch and their way through memory.
@@ -286,8 +308,8 @@ static LgPlan lg_plan(const LanesDev &L, int m) {
     const uint32_t blocks = (L.n_tiles + 3u) / 4u, m_blocks = ((uint32_t)m + 15u) / 16u;
     LgPlan best{};
     uint64_t best_cost = ~0ull;
-    for (uint32_t m_groups = (m_blocks + kLgMost - 1u) / kLgMost; m_groups <= (m_blocks + 1u) / 2u; ++m_groups) {
-        const uint32_t mb = max((m_blocks + m_groups - 1u) / m_groups, 2u), cus = max(ln_cus() / m_groups, 1u);
+    for (uint32_t m_groups = (m_blocks + kLgMost - 1u) / kLgMost; m_groups <= max((m_blocks + 1u) / 2u, 1u); ++m_groups) {
+        const uint32_t mb = (m_blocks + m_groups - 1u) / m_groups, cus = max(ln_cus() / m_groups, 1u);
         for (uint32_t s = 1; s <= min(L.n_cells, cus); ++s) {
             const uint32_t groups = min(max(cus / s, 1u), blocks);
             const uint32_t share = (blocks + groups - 1u) / groups, rounds = (share + kLgBlocks - 1u) / kLgBlocks;
@@ -307,25 +329,31 @@ size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m) {
     return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * ((L.n_tiles + 3u) / 4u * 16u) * sizeof(float) : 0;
 }
 
-template <int BITS, int MB, int NB>
-static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias,
+template <int BITS, int MB, int NB, bool ALIGNED = true>
+static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once,
                        uint16_t *y, int64_t ldy, float *ws, hipStream_t s) {
     constexpr size_t lds = LnPairs<BITS, false>::kLutBytes + kLgBlocks * kLgTileBytes + 2u * MB * 4096u;
     static_assert(lds <= kLnLds, "LDS of a CU");
-    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemm<BITS, MB, NB>),
+    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemm<BITS, MB, NB, ALIGNED>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
-    hipLaunchKernelGGL((k_lanes_gemm<BITS, MB, NB>), dim3(p.slices * p.groups * p.m_groups), dim3(kLgBlocks / NB * kWave), lds, s, L.plane, x,
-                       L.exc_off, L.scale, L.n_cells, L.n_tiles, p.slices, p.groups, L.exc_pos, L.exc_val, L.in_f, (uint32_t)m, (uint32_t)ldx,
-                       L.out_f, ws, bias, y, ldy);
+    hipLaunchKernelGGL((k_lanes_gemm<BITS, MB, NB, ALIGNED>), dim3(p.slices * p.groups * p.m_groups), dim3(kLgBlocks / NB * kWave), lds, s, L.plane, x,
+                       L.exc_off, L.scale, L.n_cells, L.n_tiles, p.slices, p.groups, L.exc_pos, L.exc_val, L.in_f, (uint32_t)m, ldx,
+                       L.out_f, ws, ((uintptr_t)ws & 15u) == 0, bias, once, y, ldy);
     if (p.slices > 1)
-        return launch_lanes_reduce(ws, p.slices, m, L.out_f, (L.n_tiles + 3u) / 4u * 16u, bias, true, y, ldy, s);
+        return launch_lanes_reduce(ws, p.slices, m, L.out_f, (L.n_tiles + 3u) / 4u * 16u, bias, once, y, ldy, s);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
+bool lanes_gemm_aligned(const LanesDev &L, const uint16_t *x, int m, int64_t ldx) {
+    return ((uintptr_t)x & 15u) == 0 && L.in_f % 8u == 0 && (m == 1 || (ldx % 8 == 0 && ldx < (1ll << 31) / m));
+}
+
 template <int BITS, class... A>
-static int gemm_rows(const LanesDev &L, const LgPlan &p, A... a) {
+static int gemm_rows(const LanesDev &L, const LgPlan &p, bool aligned, A... a) {
+    if (!aligned) return p.mb == 1 ? gemm_launch<BITS, 1, 1, false>(L, p, a...) : IXH_EUNSUPPORTED;
     switch (p.mb) {
+        case 1: return gemm_launch<BITS, 1, 1>(L, p, a...);
         case 2: return gemm_launch<BITS, 2, 1>(L, p, a...);
         case 3: return gemm_launch<BITS, 3, 1>(L, p, a...);
         case 4: return gemm_launch<BITS, 4, 2>(L, p, a...);
@@ -336,14 +364,16 @@ static int gemm_rows(const LanesDev &L, const LgPlan &p, A... a) {
     }
 }
 
-int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
-                      int64_t ldy, float *ws, hipStream_t s) {
+int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once,
+                      uint16_t *y, int64_t ldy, float *ws, hipStream_t s) {
     const LgPlan p = lg_plan(L, m);
+    const bool aligned = lanes_gemm_aligned(L, x, m, ldx);
+    if (m == 1) ldx = L.in_f;
     switch (L.bits) {
-        case 3: return gemm_rows<3>(L, p, x, m, ldx, bias, y, ldy, ws, s);
-        case 4: return gemm_rows<4>(L, p, x, m, ldx, bias, y, ldy, ws, s);
-        case 5: return gemm_rows<5>(L, p, x, m, ldx, bias, y, ldy, ws, s);
-        default: return gemm_rows<8>(L, p, x, m, ldx, bias, y, ldy, ws, s);
+        case 3: return gemm_rows<3>(L, p, aligned, x, m, ldx, bias, once, y, ldy, ws, s);
+        case 4: return gemm_rows<4>(L, p, aligned, x, m, ldx, bias, once, y, ldy, ws, s);
+        case 5: return gemm_rows<5>(L, p, aligned, x, m, ldx, bias, once, y, ldy, ws, s);
+        default: return gemm_rows<8>(L, p, aligned, x, m, ldx, bias, once, y, ldy, ws, s);
     }
 }
 

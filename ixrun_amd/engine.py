@@ -145,7 +145,7 @@ class StreamingLinear(nn.Module):
         # the shared scratch takes its final size now, not inside some later forward (or graph capture)
         need = self._dp.gemv_workspace_bytes(self._unit, MAX_FUSED_ROWS)
         if self._lanes is not None:
-            need = max(need, self._lanes.gemv_workspace_bytes(MAX_FUSED_ROWS))
+            need = max(need, *(self._lanes.gemv_workspace_bytes(n) for n in range(1, MAX_FUSED_ROWS + 1)))
         shared_workspace(self._scale.device, need)
 
     def _make_lanes(self):
