@@ -33,7 +33,8 @@ __device__ __forceinline__ uint32_t ln_pack(float lo, float hi) {
 // ---------------------------------------------------------------------------------------------------------------
 template <int BITS, bool WIDE = true> struct LnPairs {
     // log2: 32 copies of 64 entries never collide; 8 of 1024 leave about half of the collisions (5120 x 17408, 5 bits, one
-    // row: 21.9 us with one copy, 21.1 with eight).  The tile kernel has no LDS to spare for more than two.
+    // row: 21.9 us with one copy, 21.1 with eight).  k_lanes_gemm gains nothing from four (5 bits) or
+    // sixteen (4 bits) instead of two: 10240 x 5120, 100 rows, 5 bits 47.3 and 47.8 us.
     static constexpr int kCopies = BITS == 3 ? 5 : WIDE ? (BITS == 4 ? 4 : 3) : 1;
     static constexpr uint32_t kEntries = BITS == 8 ? 0u : 1u << (2 * BITS);
     static constexpr uint32_t kLutBytes = kEntries << (kCopies + 2);

@@ -321,7 +321,7 @@ class StreamingLinear(nn.Module):
                 return y
         rows = x.numel() // in_f if in_f else 0
         if (self._use_fused and self._gemm_ok and rows > MAX_FUSED_ROWS and x.dtype is torch.bfloat16 and x.is_cuda and x.shape[-1] == in_f
-                and self._lanes_gemm_wins(rows) and _plain_call(x)):
+                and self._lanes_gemm_wins(rows) and x.device == self._scale.device and _plain_call(x)):
             x2 = x.reshape(rows, in_f).contiguous()
             if x2.data_ptr() % 16:
                 x2 = x2.clone()
