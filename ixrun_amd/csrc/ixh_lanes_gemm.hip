@@ -7,8 +7,10 @@ namespace ixh {
 // k_lanes_gemm<BITS, MB, NB, ALIGNED>: up to 16 * MB activation rows at a time, MB <= 8; NB blocks of 16 weight rows a wave (two from
 // MB = 4 on: an activation operand that is read serves both); activations that are no whole 16-byte pieces: MB = 1 only.
 //
-// Bound: LDS bandwidth (per 16 x 128 weights a wave reads 4 MB KB of activations, writes and reads 8 KB of weights and
-// looks up 4 KB of pairs; the matrix unit needs a third of that time).  A wave takes 16 weight rows x 128 columns a
+// Bound: a stage's latency (decode, list and products follow one another in a wave, and all waves meet at its end: 3 to 8
+// thousand clocks), then LDS (per 16 x 128 weights a wave reads 4 MB / NB KB of activations, writes and reads 8 KB of weights and
+// looks up 4 KB of pairs). 10240 x 5120 at 55 / 40 / 5 %, 100 rows: 44.5 us with the slices' sums, of which the products are
+// 11 and the listed elements 8; 74.3 for the decode to memory and the library's GEMM. A wave takes 16 weight rows x 128 columns a
 // stage: it decodes them to its own 4 KB of LDS in operand order, stores the listed elements over their places and
 // reads the operands back.  All waves of the workgroup are in the same 128 columns, whose activations one copy in LDS
 // serves (in operand order, two stages of it: the next one is fetched during the multiply), so a weight is decoded
