@@ -24,6 +24,7 @@
 //             in activations kept in the order of lane_offset() below, from column 32768 * (column / 32768) on.
 #pragma once
 #include "ixh_dev.h"
+#include "ixh_lanes_bounds.h"
 
 namespace ixh {
 
@@ -45,6 +46,7 @@ struct LanesDev {
     const int8_t *exc_val;
     const uint16_t *scale;
     uint32_t out_f, in_f, n_tiles, n_cells;
+    uint32_t list_groups;  // whole groups of 64 quads that the list holds
     int bits;
 };
 

@@ -34,7 +34,8 @@ __global__ void __launch_bounds__(1024)
 k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
              const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t all_tiles, uint32_t tiles_per_wg, uint32_t in_f,
              const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, int m, int64_t ldx,
-             const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, uint32_t out_f, bool x_aligned) {
+             const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, uint32_t out_f, bool x_aligned,
+             uint32_t list_groups) {
     extern __shared__ __attribute__((aligned(16))) uint8_t ln_smem[];
     const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)ln_smem;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, n_threads = blockDim.x, n_waves = n_threads >> 6;
@@ -96,10 +97,10 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     for (uint32_t e = tid; e < n_tiles * n_waves * (MT * 8u); e += n_threads) parts[e] = 0.0f;
     // the list's groups, one per cell from the share's first cell on
     struct Group { ln_u32x2 pos; uint32_t val; } list[kLnAhead];
-    const uint32_t g_first = r0 >> 6, g_last = max((e_end + 63u) >> 6, g_first + 1u) - 1u;
-    const uint32_t n_groups = e_end > r0 ? g_last - g_first + 1u : 0u;
+    const LnGroups groups = ln_groups(r0, e_end, list_groups);
+    const uint32_t g_first = groups.first, n_groups = groups.n;
     auto g_load = [&](uint32_t i) {
-        const uint32_t g = min(g_first + i, g_last);
+        const uint32_t g = min(g_first + i, groups.last);
         return Group{*reinterpret_cast<const ln_u32x2 *>(exc_pos + (size_t)g * 256u + lane * 4u),
                      *reinterpret_cast<const uint32_t *>(exc_val + (size_t)g * 256u + lane * 4u)};
     };
@@ -412,7 +413,7 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
     const bool aligned = ((uintptr_t)x & 15u) == 0 && (m == 1 || ldx % 8 == 0);
     hipLaunchKernelGGL((k_lanes_gemv<BITS, MT>), dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave * waves),
                        lds_of(best_tiles, waves), s, L.plane, x, L.exc_off, L.scale, L.n_cells, L.n_tiles, best_tiles, L.in_f,
-                       L.exc_pos, L.exc_val, m, ldx, bias, y, ldy, L.out_f, aligned);
+                       L.exc_pos, L.exc_val, m, ldx, bias, y, ldy, L.out_f, aligned, L.list_groups);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 

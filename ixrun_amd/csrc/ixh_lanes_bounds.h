@@ -1,0 +1,26 @@
+// What a wave of k_lanes_gemv (ixh_lanes.hip) asks for ahead of knowing whether it needs it.  Plain C++, so that the ranges
+// can be walked without a GPU.
+#pragma once
+#include <stdint.h>
+
+#ifdef __HIPCC__
+#define LN_BOTH __host__ __device__ __forceinline__
+#else
+#define LN_BOTH inline
+#endif
+
+namespace ixh {
+
+// The list's groups (64 quads each) of a share of cells whose listed quads are first_quad .. end_quad - 1, in a list of
+// `groups` groups (at least one).  The first group is asked for whether the share lists anything or not, and behind the
+// last listed quad of a full list there is none: `last` bounds every request, `n` is how many groups count.
+struct LnGroups {
+    uint32_t first, last, n;
+};
+LN_BOTH LnGroups ln_groups(uint32_t first_quad, uint32_t end_quad, uint32_t groups) {
+    const uint32_t first = first_quad >> 6, end = (end_quad + 63u) >> 6;
+    const uint32_t last = (end > first ? end : first + 1u) - 1u;
+    return {first, last < groups ? last : groups - 1u, end_quad > first_quad ? last - first + 1u : 0u};
+}
+
+}  // namespace ixh

@@ -44,15 +44,18 @@ def values(kind, out_f, in_f):
     return int8_mix("only_l3", n, seed=5), (3, 5, 8), 8
 
 
-def lay_out(kind, out_f, in_f, dev):
+def lay_out_values(p, out_f, in_f, dev):
     from ixrun_amd import _lib
     from ixrun_amd.fused import pick_unit
 
-    v, scheme, bits = values(kind, out_f, in_f)
-    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
     dp = _lib.DevicePacked.from_dict(p, dev)
     unit = pick_unit(in_f)
-    lanes = _lib.LanePacked.build(dp, dp.prefix_build(unit), unit, p["counts"])
+    return p, _lib.LanePacked.build(dp, dp.prefix_build(unit), unit, p["counts"])
+
+
+def lay_out(kind, out_f, in_f, dev):
+    v, scheme, bits = values(kind, out_f, in_f)
+    p, lanes = lay_out_values(packed_from_int8(v, out_f, in_f, level_bits=scheme), out_f, in_f, dev)
     assert lanes.bits == bits
     return p, lanes
 
@@ -176,6 +179,21 @@ def test_prompts_of_a_layer_take_the_lanes_in_every_form(oracle, dev):
     many = activations(600, in_f, seed=6).to(dev)
     for x in (many, wide[:40, :in_f].float()):
         assert rel_l2(layer(x).double().cpu().numpy(), plain(x).double().cpu().numpy()) <= 1e-3
+
+
+@pytest.mark.parametrize("listed", [0, 63, 64, 65, 128])
+def test_list_that_ends_on_a_whole_group(oracle, dev, listed):
+    """All listed elements in the first cells of a tensor: what is behind them starts at the list's end, which at 64 and 128
+    is the end of its last group as well."""
+    out_f, in_f = 260, 1536
+    v = int8_mix("only_l1", out_f * in_f, seed=6).reshape(out_f, in_f)
+    v[0, 7 : 7 + 2 * listed : 2] = 90
+    p = packed_from_int8(v.reshape(-1), out_f, in_f)
+    _, lanes = lay_out_values(p, out_f, in_f, dev)
+    assert lanes.bits == 3 and int(lanes.tensors[1][-1]) == listed and lanes.struct.n_quads == max(64, -(-listed // 64) * 64)
+    for m in (1, 2, 4, 8):
+        x = activations(m, in_f, seed=m)
+        check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
 
 
 def test_one_hot_rows_are_decoded_columns(oracle, dev):
