@@ -77,7 +77,7 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     for (uint32_t p = 0; p < kLnXAhead; ++p) {
         const uint32_t e = min(tid + p * n_threads, x_pieces - 1u), r = MT == 1 ? 0u : min(e / (C * 64u), (uint32_t)m - 1u);
         // whole pieces of an aligned row only; the others are read below
-        const uint32_t col = min((e - e / (C * 64u) * (C * 64u)) * 8u, x_aligned ? (in_f & ~7u) - 8u : 0u);
+        const uint32_t col = x_aligned ? ln_piece_column((e - e / (C * 64u) * (C * 64u)) * 8u, in_f) : 0u;
         xv[p] = x_aligned ? *reinterpret_cast<const ln_u32x4 *>(x + (int64_t)r * ldx + col) : ln_u32x4{0, 0, 0, 0};
     }
     uint32_t buf[kLnAhead][BITS];
@@ -410,7 +410,7 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
     static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemv<BITS, MT>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
-    const bool aligned = ((uintptr_t)x & 15u) == 0 && (m == 1 || ldx % 8 == 0);
+    const bool aligned = ln_whole_pieces((uintptr_t)x, L.in_f, m, ldx);
     hipLaunchKernelGGL((k_lanes_gemv<BITS, MT>), dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave * waves),
                        lds_of(best_tiles, waves), s, L.plane, x, L.exc_off, L.scale, L.n_cells, L.n_tiles, best_tiles, L.in_f,
                        L.exc_pos, L.exc_val, m, ldx, bias, y, ldy, L.out_f, aligned, L.list_groups);

@@ -23,4 +23,14 @@ LN_BOTH LnGroups ln_groups(uint32_t first_quad, uint32_t end_quad, uint32_t grou
     return {first, last < groups ? last : groups - 1u, end_quad > first_quad ? last - first + 1u : 0u};
 }
 
+// Activations: 16-byte pieces of whole rows are asked for before anything else where every row starts 16-byte aligned and
+// has a whole piece; of the pieces past a row's last whole one that one is asked for again.
+LN_BOTH bool ln_whole_pieces(uint64_t x, uint32_t in_f, int m, int64_t ldx) {
+    return (x & 15u) == 0 && in_f >= 8u && (m == 1 || ldx % 8 == 0);
+}
+LN_BOTH uint32_t ln_piece_column(uint32_t col, uint32_t in_f) {  // in_f >= 8
+    const uint32_t last = (in_f & ~7u) - 8u;
+    return col < last ? col : last;
+}
+
 }  // namespace ixh

@@ -181,6 +181,16 @@ def test_prompts_of_a_layer_take_the_lanes_in_every_form(oracle, dev):
         assert rel_l2(layer(x).double().cpu().numpy(), plain(x).double().cpu().numpy()) <= 1e-3
 
 
+@pytest.mark.parametrize("in_f", [1, 3, 7, 8, 9, 15])
+def test_rows_of_a_few_columns(oracle, dev, in_f):
+    """Rows shorter than, as long as and just longer than a 16-byte piece."""
+    out_f = 21
+    p, lanes = lay_out("rare", out_f, in_f, dev)
+    for m in (1, 2, 4, 6):
+        x = activations(m, in_f, seed=m)
+        check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
+
+
 @pytest.mark.parametrize("listed", [0, 63, 64, 65, 128])
 def test_list_that_ends_on_a_whole_group(oracle, dev, listed):
     """All listed elements in the first cells of a tensor: what is behind them starts at the list's end, which at 64 and 128
