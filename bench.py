@@ -623,7 +623,7 @@ def main():
         gemm_tuning.enable()
     for sl in layers:
         sl._gemv_flags = args.gemv_flags
-        sl._plans = {}
+        sl._forget_plans()
     x = x_host.to(dev)
     table_bytes = layers[0]._table.numel() * 4
     # algorithmic bytes of one step: the packed layer, the activations in, the outputs out

@@ -62,9 +62,10 @@ SPLIT_FUSED_MIN_WEIGHTS = 40_000_000
 
 
 def _plain_call(x) -> bool:
-    """Whether a product of ``x`` that is not torch's own is what the caller gets from ``F.linear``: no gradient, transform or
-    other result type is asked for."""
+    """Whether a product of ``x`` that is not torch's own is what the caller gets from ``F.linear``: no gradient, transform,
+    other result type or other kind of tensor is asked for."""
     return (not (x.requires_grad and torch.is_grad_enabled()) and forward_ad._current_level < 0
+            and not torch.overrides.has_torch_function_unary(x)
             and torch._C._functorch.peek_interpreter_stack() is None
             and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") is torch.bfloat16))
 
@@ -103,6 +104,7 @@ class StreamingLinear(nn.Module):
         self.register_buffer("_scale", packed["scale"].reshape(()).cuda())
         self.register_buffer("_bias", bias.detach().clone().cuda() if bias is not None else None)
         self._gemv_flags = 0  # extra IXH_GEMV_* flags of every fused call (comparisons: bench.py --gemv-flags)
+        self._w_buf = None  # set by the engine
         self._bind()
 
         # rank tables: the kernels' own (unit = 512 where rows allow it) and
@@ -139,7 +141,6 @@ class StreamingLinear(nn.Module):
         self.register_buffer("_q2", q[1].contiguous() if n_levels > 2 else torch.zeros_like(q[0]))
         self._y32 = None
 
-        self._w_buf = None  # set by the engine
         if lanes:
             self._make_lanes()
         # the shared scratch takes its final size now, not inside some later forward (or graph capture)
@@ -213,7 +214,7 @@ class StreamingLinear(nn.Module):
             if bias is not None and bias.dtype is torch.bfloat16 and bias.is_cuda and bias.is_contiguous():
                 self._bias_ptr = bias.data_ptr()  # added by the kernel
         self._gemv_fn = _lib.lib().ixh_lanes_gemv if self._lanes is not None else _lib.lib().ixh_gemv
-        self._plans = {}
+        self._forget_plans()
         # the forward of up to MAX_FUSED_ROWS rows from the lanes, in native code
         self._native = self._native_fn = None
         if self._lanes is not None and (self._bias is None or self._bias_ptr):
@@ -241,7 +242,12 @@ class StreamingLinear(nn.Module):
 
     def _set_shared_buf(self, w_buf):
         self._w_buf = w_buf
+        self._forget_plans()
+
+    def _forget_plans(self):
         self._plans = {}
+        # activations (elements) up to which a forward from the lanes takes calls that are not plain too: see _fused_plan
+        self._any_call = self._packed_rows() * self.in_features
 
     def _decode_table(self):
         """The rank table and unit of a decode of the whole weight."""
@@ -254,22 +260,26 @@ class StreamingLinear(nn.Module):
         self._dp.decode(*self._decode_table(), out_bf16=w_flat)
         return w_flat.view(self.out_features, self.in_features)
 
+    def _packed_rows(self) -> int:
+        """Most rows that one call of ``ixh_gemv`` on the packed streams is the fastest way for."""
+        if self._w_buf is None:
+            return MAX_FUSED_ROWS
+        if self.counts[0] * 100 >= self.N * 97:
+            return MAX_FUSED_ROWS_WITH_BUFFER
+        return MAX_FUSED_ROWS_WITH_BUFFER_DENSE if self.level_bits == (3, 5, 8) else 1
+
     def _fused_plan(self, rows):
         """How a forward of `rows` activation rows is served by the fused kernel: the row count of each call (one, or
         two for 17 .. 32 rows on a large layer that is almost all level 1) with the scratch it needs, or False where
-        the many-row paths take over.  Worked out once per row count; ``_set_shared_buf`` and ``_bind`` forget the
-        answers."""
+        the many-row paths take over; and whether that holds for plain calls only, because without lanes the rows would go
+        through decode + ``F.linear``, which serves gradients, transforms and autocast.  Worked out once per row count;
+        ``_set_shared_buf`` and ``_bind`` forget the answers."""
         lanes = self._lanes is not None and self._gemv_flags == 0
-        if self._w_buf is None or lanes:
-            fused_rows = MAX_FUSED_ROWS
-        elif self.counts[0] * 100 >= self.N * 97:
-            fused_rows = MAX_FUSED_ROWS_WITH_BUFFER
-        elif self.level_bits == (3, 5, 8):
-            fused_rows = MAX_FUSED_ROWS_WITH_BUFFER_DENSE
-        else:
-            fused_rows = 1
-        two_calls = (MAX_FUSED_ROWS < rows <= 2 * MAX_FUSED_ROWS and fused_rows == MAX_FUSED_ROWS
-                     and self.N >= SPLIT_FUSED_MIN_WEIGHTS and (not self._lanes_gemm_wins(rows) if lanes else self.counts[0] * 100 >= self.N * 97))
+        packed_rows = self._packed_rows()
+        fused_rows = MAX_FUSED_ROWS if lanes else packed_rows
+        two_calls = MAX_FUSED_ROWS < rows <= 2 * MAX_FUSED_ROWS and self.N >= SPLIT_FUSED_MIN_WEIGHTS
+        two_packed_calls = two_calls and packed_rows == MAX_FUSED_ROWS and self.counts[0] * 100 >= self.N * 97
+        two_calls = two_calls and not self._lanes_gemm_wins(rows) if lanes else two_packed_calls
         plan = False
         if 1 <= rows <= fused_rows or two_calls:
             calls = []
@@ -277,12 +287,13 @@ class StreamingLinear(nn.Module):
                 n = min(MAX_FUSED_ROWS, rows - r0)
                 calls.append((r0, n, self._lanes.gemv_workspace_bytes(n) if lanes
                               else self._dp.gemv_workspace_bytes(self._unit, n, self._gemv_flags)))
-            plan = (lanes, tuple(calls))
+            plan = (lanes, tuple(calls), rows > packed_rows and not two_packed_calls)
         self._plans[rows] = plan
         return plan
 
     def forward(self, x):
-        if self._native is not None and self._use_fused and not self._gemv_flags and self._gemv_fn is self._native_fn:
+        if (self._native is not None and self._use_fused and not self._gemv_flags and self._gemv_fn is self._native_fn
+                and (x.numel() <= self._any_call or (x.numel() <= MAX_FUSED_ROWS * self.in_features and _plain_call(x)))):
             y = self._native(x)
             if y is not None:
                 return y
@@ -292,7 +303,7 @@ class StreamingLinear(nn.Module):
             plan = self._plans.get(rows)
             if plan is None:
                 plan = self._fused_plan(rows)
-            if plan:
+            if plan and (not plan[2] or _plain_call(x)):
                 # one ctypes call with the arguments that never change kept bound
                 out_f = self.out_features
                 if not x.is_contiguous():
@@ -301,7 +312,7 @@ class StreamingLinear(nn.Module):
                 y = torch.empty(x.shape[:-1] + (out_f,), dtype=torch.bfloat16, device=dev)
                 x_ptr, y_ptr = x.data_ptr(), y.data_ptr()
                 stream = _raw_stream(dev.index if dev.index is not None else torch.cuda.current_device())
-                lanes, calls = plan
+                lanes, calls, _ = plan
                 for r0, n, ws_bytes in calls:  # one call, or two on the same stream and workspace
                     ws = _workspaces.get(dev) if ws_bytes else None
                     if ws_bytes and (ws is None or ws.numel() * 4 < ws_bytes):

@@ -206,6 +206,64 @@ def test_list_that_ends_on_a_whole_group(oracle, dev, listed):
         check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
 
 
+@pytest.mark.parametrize("in_f,rows", [(1024, 2), (1024, 16), (1004, 5), (1004, 20)])
+def test_calls_that_are_not_plain_keep_the_decode(monkeypatch, dev, in_f, rows):
+    """Gradients, forward mode, vmap, autocast and other kinds of tensors: a layer with a decode buffer whose rows went
+    through decode + F.linear before it had lanes (dense, not (3,5,8); 17 to 32 rows of a large dense layer) still serves them
+    that way, and only plain calls from the lanes."""
+    from torch.autograd import forward_ad
+
+    from ixrun_amd import engine
+
+    monkeypatch.setattr(engine, "SPLIT_FUSED_MIN_WEIGHTS", 0)
+    products = []
+
+    def linear(x, w, bias):  # in fp32: what is asked for here is who multiplies, and what the caller gets back
+        products.append(x.shape)
+        return torch.nn.functional.linear(x.float(), w.float(), bias).to(torch.float16 if torch.is_autocast_enabled("cuda") else x.dtype)
+
+    monkeypatch.setattr(engine.gemm_tuning, "linear", linear)
+    v, scheme, _ = values("real", 64, in_f)
+    p = packed_from_int8(v, 64, in_f, level_bits=scheme)
+    layer, plain = engine.StreamingLinear(p), engine.StreamingLinear(p, lanes=False)
+    for one in (layer, plain):
+        one._set_shared_buf(torch.zeros(p["N"], dtype=torch.bfloat16, device=dev))
+    x = activations(rows, in_f, seed=5).to(dev)
+
+    with torch.no_grad():
+        layer(x.clone().requires_grad_())
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        layer(x)
+    y = layer(x)
+    assert not products and not bool(layer._w_buf.any())
+
+    def gradient(one):
+        leaf = x.clone().requires_grad_()
+        one(leaf).sum().backward()
+        return leaf.grad
+
+    def tangent(one):
+        with forward_ad.dual_level():
+            return forward_ad.unpack_dual(one(forward_ad.make_dual(x, x.flip(0)))).tangent
+
+    def mapped(one):
+        return torch.vmap(one)(torch.stack([x, x.flip(0)]))
+
+    def cast(one):
+        with torch.autocast("cuda", dtype=torch.float16):
+            return one(x)
+
+    class Named(torch.Tensor):
+        pass
+
+    for call in (gradient, tangent, mapped, cast, lambda one: one(x.as_subclass(Named))):
+        del products[:]
+        got, n = call(layer), len(products)
+        want = call(plain)
+        assert n and len(products) == 2 * n and type(got) is type(want) and got.dtype == want.dtype and torch.equal(got, want)
+    assert rel_l2(y.double().cpu().numpy(), plain(x).double().cpu().numpy()) <= 2 ** -8
+
+
 def test_one_hot_rows_are_decoded_columns(oracle, dev):
     out_f, in_f = 24, 1100
     p, lanes = lay_out("real", out_f, in_f, dev)
