@@ -238,7 +238,8 @@ class StreamingLinear(nn.Module):
         if self._scale.is_cuda:  # the packed streams may be others now
             if self._flat_table is not None:
                 self._flat_table = self._dp.prefix_build(FUSED_TILE)
-            self._make_lanes()
+            if self._lanes is not None:  # a layer that was built without lanes stays without
+                self._make_lanes()
 
     def _set_shared_buf(self, w_buf):
         self._w_buf = w_buf

@@ -294,6 +294,19 @@ def test_layer_rebuilds_its_lanes_with_its_state(dev):
     assert torch.equal(layers[0](x), layers[1](x))
 
 
+def test_layer_without_lanes_stays_without_when_it_loads_a_state(dev):
+    from ixrun_amd.engine import StreamingLinear
+
+    p = [packed_from_int8(int8_mix("only_l1", 64 * 1024, seed=seed), 64, 1024) for seed in (1, 2)]
+    without, other = StreamingLinear(p[0], lanes=False), StreamingLinear(p[1])
+    without.load_state_dict(other.state_dict())
+    assert without._lanes is None and not any("lane" in name for name, b in without.named_buffers() if b is not None)
+    x = activations(3, 1024, seed=9).to(dev)
+    assert rel_l2(without(x).double().cpu().numpy(), other(x).double().cpu().numpy()) <= 1e-3
+    other.load_state_dict(without.state_dict())
+    assert other._lanes is not None
+
+
 def test_malformed_lanes_are_refused(dev):
     from ixrun_amd import _lib
 
