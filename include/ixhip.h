@@ -199,8 +199,8 @@ size_t ixh_gemm_workspace_bytes(const IxhPacked *packed, int32_t m);
  * values that do not fit in a list (csrc/ixh_lanes.h has the layout).  Buffers are the caller's:
  *   plane    plane_words = ixh_lanes_plane_words(out_f, in_f, bits) 32-bit words, 16-byte aligned
  *   exc_off  ixh_lanes_cells(out_f, in_f) + 1 entries: first quad of listed elements of every cell (4 rows x 512 columns)
- *   exc_pos, exc_val  4 * n_quads entries each, the elements with |value| > 2^(bits-1) - 1; n_quads: the cells' quads
- *            together, rounded up to a multiple of 64, at least 64 (the rest zero: whole groups are read)
+ *   exc_pos, exc_val  4 * n_quads entries each, the elements with |value| > 2^(bits-1) - 1; n_quads: a multiple
+ *            of 64, at least 64 and at least the cells' quads together (the rest zero: whole groups are read)
  */
 typedef struct IxhLanes {
     int32_t bits;

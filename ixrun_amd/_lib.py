@@ -431,8 +431,13 @@ class LanePacked:
         return None if words < 0 else 4 * words + 4 * sum(c for b, c in zip(dp.level_bits, counts) if b > bits)
 
     @classmethod
-    def build(cls, dp: DevicePacked, table: torch.Tensor, unit: int, counts) -> "LanePacked":
-        """Lay out a packed tensor (through its bf16 weights; one synchronisation, for the length of the list)."""
+    def build(cls, dp: DevicePacked, table: torch.Tensor, unit: int, counts, into: "LanePacked | None" = None) -> "LanePacked":
+        """Lay out a packed tensor (through its bf16 weights; one synchronisation, for the length of the list).
+
+        ``into``: an earlier layout of a tensor of the same shape and counts, written over and returned if its list holds
+        the new one.  A list is allocated 1/32 longer than needed (some 0.5 % of a layout), and one that replaces another at
+        least half as long again, so that this is the rule and a layout is not replaced often: a list has at most as many
+        quads as elements, four times the fewest."""
         dev, L = dp.device, lib()
         words, cells = L.ixh_lanes_plane_words(dp.out_f, dp.in_f, lane_bits(dp.level_bits, counts)), L.ixh_lanes_cells(dp.out_f, dp.in_f)
         with torch.cuda.device(dev):
@@ -446,10 +451,20 @@ class LanePacked:
             first = cls(dp.out_f, dp.in_f, (plane, exc_off, none, none.to(torch.int8)), dp.tensors[-1])
             check(L.ixh_lanes_pack(w.data_ptr(), C.byref(first.struct), quads.data_ptr(), stream))
             torch.cumsum(quads, 0, dtype=torch.int32, out=exc_off[1:])
-            n_quads = max(-(-int(exc_off[-1]) // 64), 1) * 64
-            exc_pos = torch.zeros(4 * n_quads, dtype=torch.int16, device=dev)
-            exc_val = torch.zeros(4 * n_quads, dtype=torch.int8, device=dev)
-            whole = cls(dp.out_f, dp.in_f, (plane, exc_off, exc_pos, exc_val), dp.tensors[-1])
+            n_quads = max(int(exc_off[-1]), 1)
+            if into is not None and into.bits == first.bits and n_quads <= into.struct.n_quads:
+                whole = into
+                for kept, t in zip(whole.tensors, (plane, exc_off)):
+                    kept.copy_(t)
+                for t in whole.tensors[2:]:
+                    t.zero_()
+            else:
+                n_quads += n_quads // 32
+                if into is not None:
+                    n_quads = max(n_quads, into.struct.n_quads * 3 // 2)
+                n_quads = -(-n_quads // 64) * 64
+                whole = cls(dp.out_f, dp.in_f, (plane, exc_off, torch.zeros(4 * n_quads, dtype=torch.int16, device=dev),
+                                                torch.zeros(4 * n_quads, dtype=torch.int8, device=dev)), dp.tensors[-1])
             check(L.ixh_lanes_list(w.data_ptr(), C.byref(whole.struct), stream))
         return whole
 

@@ -105,6 +105,7 @@ class StreamingLinear(nn.Module):
         self.register_buffer("_bias", bias.detach().clone().cuda() if bias is not None else None)
         self._gemv_flags = 0  # extra IXH_GEMV_* flags of every fused call (comparisons: bench.py --gemv-flags)
         self._w_buf = None  # set by the engine
+        self._replaced_lanes = []
         self._bind()
 
         # rank tables: the kernels' own (unit = 512 where rows allow it) and
@@ -237,9 +238,20 @@ class StreamingLinear(nn.Module):
         super()._load_from_state_dict(*args, **kwargs)
         if self._scale.is_cuda:  # the packed streams may be others now
             if self._flat_table is not None:
-                self._flat_table = self._dp.prefix_build(FUSED_TILE)
+                self._flat_table.copy_(self._dp.prefix_build(FUSED_TILE))
             if self._lanes is not None:  # a layer that was built without lanes stays without
-                self._make_lanes()
+                self._refresh_lanes()
+
+    def _refresh_lanes(self):
+        """Lay the weights out again, in place: a graph captured earlier serves the new ones, as it does from the packed
+        streams.  Where the new list does not fit into the old one's memory the layout is replaced as a whole and the old one
+        stays alive: such a graph goes on serving the old weights and has to be captured again."""
+        lanes = _lib.LanePacked.build(self._dp, *self._decode_table(), self.counts, into=self._lanes)
+        if lanes is not self._lanes:
+            self._replaced_lanes.append(self._lanes)
+            for name, t in zip(LANE_BUFFERS, lanes.tensors):
+                setattr(self, name, t)
+            self._bind()
 
     def _set_shared_buf(self, w_buf):
         self._w_buf = w_buf

@@ -4,6 +4,7 @@ Shapes sit at the edges of the layout (row quads, 16-row blocks, 512-column cell
 list), mixes at every width of the plane, with no listed element, with rows of listed elements only, and with one row
 far fuller than the others of its quad."""
 import ctypes as C
+import weakref
 
 import numpy as np
 import pytest
@@ -200,7 +201,9 @@ def test_list_that_ends_on_a_whole_group(oracle, dev, listed):
     v[0, 7 : 7 + 2 * listed : 2] = 90
     p = packed_from_int8(v.reshape(-1), out_f, in_f)
     _, lanes = lay_out_values(p, out_f, in_f, dev)
-    assert lanes.bits == 3 and int(lanes.tensors[1][-1]) == listed and lanes.struct.n_quads == max(64, -(-listed // 64) * 64)
+    assert lanes.bits == 3 and int(lanes.tensors[1][-1]) == listed
+    groups = max(-(-listed // 64), 1)
+    lanes.struct.n_quads = 64 * groups  # (no room behind the last group that the list needs)
     for m in (1, 2, 4, 8):
         x = activations(m, in_f, seed=m)
         check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
@@ -305,6 +308,48 @@ def test_layer_without_lanes_stays_without_when_it_loads_a_state(dev):
     assert rel_l2(without(x).double().cpu().numpy(), other(x).double().cpu().numpy()) <= 1e-3
     other.load_state_dict(without.state_dict())
     assert other._lanes is not None
+
+
+@pytest.mark.parametrize("in_f", [1024, 1000])
+@pytest.mark.parametrize("grows", [False, True])
+def test_graph_serves_the_state_that_is_loaded(dev, in_f, grows):
+    """A graph captured before load_state_dict: the layer's layout and tables are refreshed in place, and the replay gives the
+    new weights' products.  A list that has outgrown its memory takes a new layout, and the old one stays whole: the graph
+    gives the old products, and one captured again the new ones."""
+    from ixrun_amd.engine import StreamingLinear
+
+    out_f, names = 256, ("_lane_plane", "_lane_off", "_lane_pos", "_lane_val")
+    v = [int8_mix("only_l1", out_f * in_f, seed=seed).reshape(out_f, in_f) for seed in (1, 2)]
+    for i in range(256):  # as many listed elements: one a row (64 quads), or all in one row and cell (256)
+        v[0][i, 5] = 50
+        v[1][(0, i) if grows else (i, 7)] = 60
+    p = [packed_from_int8(w.reshape(-1), out_f, in_f) for w in v]
+    assert p[0]["counts"] == p[1]["counts"]
+    layer, other = StreamingLinear(p[0]), StreamingLinear(p[1])
+    assert (other._lanes.struct.n_quads > layer._lanes.struct.n_quads) == grows
+    xs = [activations(m, in_f, seed=9).to(dev) for m in (1, 8)]
+    old, new = [layer(x) for x in xs], [other(x) for x in xs]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ys = [layer(x) for x in xs]
+    kept = [weakref.ref(getattr(layer, n)) for n in names]
+    sizes = [t().shape for t in kept]
+    layer.load_state_dict(other.state_dict())
+    for _ in range(3):
+        junk = [torch.full(n, 3, dtype=t.dtype, device=dev) for n, t in zip(sizes, layer._lanes.tensors)]  # what freed buffers would be given to
+        graph.replay()
+        torch.cuda.synchronize()
+        for y, want in zip(ys, old if grows else new):
+            assert torch.equal(y, want)
+        del junk
+    for x, want in zip(xs, new):
+        assert torch.equal(layer(x), want)
+    assert [getattr(layer, n) is t() for n, t in zip(names, kept)] == [not grows] * 4
+    assert all(t() is not None for t in kept)
+    buf = torch.empty(out_f * in_f, dtype=torch.bfloat16, device=dev)
+    for one in (layer, other):
+        one._set_shared_buf(buf)
+    assert torch.equal(layer._decode().clone(), other._decode())
 
 
 def test_malformed_lanes_are_refused(dev):
