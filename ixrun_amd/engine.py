@@ -106,6 +106,7 @@ class StreamingLinear(nn.Module):
         self._gemv_flags = 0  # extra IXH_GEMV_* flags of every fused call (comparisons: bench.py --gemv-flags)
         self._w_buf = None  # set by the engine
         self._replaced_lanes = []
+        self._stale = False
         self._bind()
 
         # rank tables: the kernels' own (unit = 512 where rows allow it) and
@@ -232,15 +233,25 @@ class StreamingLinear(nn.Module):
         out = super()._apply(fn, recurse)
         if hasattr(self, "_scale") and self._scale.is_cuda:
             self._bind()
+            if self._stale:
+                self._follow_streams()
         return out
 
     def _load_from_state_dict(self, *args, **kwargs):
         super()._load_from_state_dict(*args, **kwargs)
-        if self._scale.is_cuda:  # the packed streams may be others now
-            if self._flat_table is not None:
-                self._flat_table.copy_(self._dp.prefix_build(FUSED_TILE))
-            if self._lanes is not None:  # a layer that was built without lanes stays without
-                self._refresh_lanes()
+        if self._scale.is_cuda:  # the packed streams may be others now (with assign=True, in other places)
+            self._bind()
+            self._follow_streams()
+        else:  # when the layer is back on the GPU
+            self._stale = True
+
+    def _follow_streams(self):
+        """Bring what is derived from the packed streams and is no part of the state dict in line with them."""
+        if self._flat_table is not None:
+            self._flat_table.copy_(self._dp.prefix_build(FUSED_TILE))
+        if self._lanes is not None:  # a layer that was built without lanes stays without
+            self._refresh_lanes()
+        self._stale = False
 
     def _refresh_lanes(self):
         """Lay the weights out again, in place: a graph captured earlier serves the new ones, as it does from the packed

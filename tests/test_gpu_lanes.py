@@ -73,6 +73,12 @@ def product(lanes, x, out_f, in_f, bias=None):
     return y
 
 
+def lib_gemv():
+    from ixrun_amd import _lib
+
+    return _lib.lib().ixh_gemv
+
+
 def check(oracle, p, x, y, bias=None, once=False):
     want = oracle.gemm_f64(oracle.decode_packed_bf16(p), bf16_bits(x)).astype(np.float32)
     if once and bias is not None:
@@ -295,6 +301,42 @@ def test_layer_rebuilds_its_lanes_with_its_state(dev):
     assert not torch.equal(layers[0](x), layers[1](x))
     layers[0].load_state_dict(layers[1].state_dict())
     assert torch.equal(layers[0](x), layers[1](x))
+
+
+@pytest.mark.parametrize("in_f", [1024, 1000])
+@pytest.mark.parametrize("way", ["moved", "assigned", "assigned on the host"])
+def test_layer_follows_a_state_loaded_elsewhere(dev, in_f, way):
+    """A state loaded while the layer is on the host, or taken over tensor by tensor: lanes, tables and decode are of the
+    new weights once the layer is on the GPU."""
+    from ixrun_amd.engine import StreamingLinear
+
+    p = [packed_from_int8(int8_mix("only_l1", 64 * in_f, seed=seed), 64, in_f) for seed in (1, 2)]
+    layer, other = StreamingLinear(p[0]), StreamingLinear(p[1])
+    if way == "moved":
+        layer.cpu()
+        layer.load_state_dict(other.state_dict())
+        layer.cuda()
+    else:
+        state = {k: t.to("cpu" if "host" in way else dev, copy=True) for k, t in other.state_dict().items()}
+        layer.load_state_dict(state, assign=True)
+        del state
+        layer.cuda()
+    junk = [torch.full((1 << 14,), 3, dtype=torch.int32, device=dev) for _ in range(8)]
+    buf = torch.empty(64 * in_f, dtype=torch.bfloat16, device=dev)
+    for one in (layer, other):
+        one._set_shared_buf(buf)
+    assert torch.equal(layer._decode().clone(), other._decode())
+    for m in (1, 3, 12):
+        x = activations(m, in_f, seed=9).to(dev)
+        want = other(x)
+        assert torch.equal(layer(x), want)
+        layer._lanes, lanes = None, layer._lanes  # and from the packed streams
+        layer._native, native, layer._gemv_fn, fn = None, layer._native, lib_gemv(), layer._gemv_fn
+        layer._forget_plans()
+        assert rel_l2(layer(x).double().cpu().numpy(), want.double().cpu().numpy()) <= 1e-3
+        layer._lanes, layer._native, layer._gemv_fn = lanes, native, fn
+        layer._forget_plans()
+    del junk
 
 
 def test_layer_without_lanes_stays_without_when_it_loads_a_state(dev):
