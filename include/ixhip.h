@@ -200,7 +200,7 @@ size_t ixh_gemm_workspace_bytes(const IxhPacked *packed, int32_t m);
  *   plane    plane_words = ixh_lanes_plane_words(out_f, in_f, bits) 32-bit words, 16-byte aligned
  *   exc_off  ixh_lanes_cells(out_f, in_f) + 1 entries: first quad of listed elements of every cell (4 rows x 512 columns)
  *   exc_pos, exc_val  4 * n_quads entries each, the elements with |value| > 2^(bits-1) - 1; n_quads: a multiple
- *            of 64, at least 64 and at least the cells' quads together (the rest zero: whole groups are read)
+ *            of 64, at least 64 and at least the cells' quads together (whole groups are read)
  */
 typedef struct IxhLanes {
     int32_t bits;
@@ -221,8 +221,8 @@ int64_t ixh_lanes_cells(int64_t out_f, int64_t in_f);
 /*
  * Writing it, from the bf16 weights that ixh_decode makes of the packed tensor (out_f x in_f, dense; the integers come
  * back exactly).  ixh_lanes_pack writes the plane and the number of quads of every cell to `counts` (ixh_lanes_cells
- * entries); the caller turns those into exc_off (an exclusive running sum, the total behind the last), zeroes the list
- * and ixh_lanes_list fills it in.  In both, `dst` names the buffers (written despite the const of its
+ * entries); the caller turns those into exc_off (an exclusive running sum, the total behind the last), zeroes exc_val
+ * and ixh_lanes_list fills both in, with positions of no effect where there is no element.  In both, `dst` names the buffers (written despite the const of its
  * fields; ixh_lanes_pack uses plane and scale only).
  */
 int ixh_lanes_pack(const uint16_t *w, const IxhLanes *dst, uint32_t *counts, ixh_stream_t stream);

@@ -456,14 +456,13 @@ class LanePacked:
                 whole = into
                 for kept, t in zip(whole.tensors, (plane, exc_off)):
                     kept.copy_(t)
-                for t in whole.tensors[2:]:
-                    t.zero_()
+                whole.tensors[3].zero_()
             else:
                 n_quads += n_quads // 32
                 if into is not None:
                     n_quads = max(n_quads, into.struct.n_quads * 3 // 2)
                 n_quads = -(-n_quads // 64) * 64
-                whole = cls(dp.out_f, dp.in_f, (plane, exc_off, torch.zeros(4 * n_quads, dtype=torch.int16, device=dev),
+                whole = cls(dp.out_f, dp.in_f, (plane, exc_off, torch.empty(4 * n_quads, dtype=torch.int16, device=dev),
                                                 torch.zeros(4 * n_quads, dtype=torch.int8, device=dev)), dp.tensors[-1])
             check(L.ixh_lanes_list(w.data_ptr(), C.byref(whole.struct), stream))
         return whole

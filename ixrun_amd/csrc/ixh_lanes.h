@@ -12,16 +12,18 @@
 //   lane l    row l % 4, slice s = l / 4 (q = s / 4, kg = s % 4) of the columns 128 q + 32 i + 8 kg + j, i < 4, j < 8:
 //             32 weights, in pairs p = 4 i + j / 2.
 //   dwords    the first min(bits, 4) of a lane are consecutive, lane after lane, so are the others behind them.
-//   codes     value + 2^(bits-1) - 1; a listed element has the code of 0, and so has the padding of the last row quad
-//             and of the last cell of a row.
+//   codes     value + 2^(bits-1) - 1; a listed element has the code of its sign, +1 or -1, which a kernel that adds the
+//             list to the plane's products takes off again: with the code of 0 an infinite activation there would give NaN.
+//             The padding of the last row quad and of the last cell of a row has the code of 0.
 //   pairs     2 * bits wide, first element in the low half.  bits = 4: pair p in byte p % 4 of dword p / 4.
 //             bits = 3: five pairs a dword from bit 2 on (p = 5 d + f at bit 2 + 6 f), the two low bits of the three
 //             dwords are pair 15.  bits = 5: three a dword from bit 2 on (p = 3 d + f), the two low bits of the five
 //             dwords are pair 15.  bits = 8: four bytes a dword, in element order.
 //   listed    in quads, one element of each of a cell's four rows: exc_pos[4 n + r], exc_val[4 n + r] belong to row r of
 //             quad n.  A cell has as many quads as its fullest row has listed elements (the others end in value 0 at
-//             position 0), from exc_off[cell] on (one more at the end).  exc_pos: the byte offset of the element's column
-//             in activations kept in the order of lane_offset() below, from column 32768 * (column / 32768) on.
+//             position lane_none()), from exc_off[cell] on (one more at the end).  exc_pos: the byte offset of the
+//             element's column in activations kept in the order of lane_offset() below, from column 32768 * (column /
+//             32768) on.
 #pragma once
 #include "ixh_dev.h"
 #include "ixh_lanes_bounds.h"
@@ -38,6 +40,11 @@ __host__ __device__ inline uint32_t lane_offset(uint32_t col) {
     const uint32_t b = 2u * col;
     return b ^ ((b >> 2) & 0xC0u);
 }
+
+// Where a quad's place without an element points: behind the row's last cell, where a kernel keeps an activation of 0 (value
+// 0 times an infinite activation is NaN).  Rows of 64 and more cells have no offset left for that: 0, and the kernel looks at
+// the value instead.
+__host__ __device__ inline uint32_t lane_none(uint32_t n_cells) { return n_cells < kLnSegCells ? n_cells * 2u * kLnCols : 0u; }
 
 struct LanesDev {
     const uint32_t *plane;

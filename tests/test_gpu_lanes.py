@@ -188,6 +188,36 @@ def test_prompts_of_a_layer_take_the_lanes_in_every_form(oracle, dev):
         assert rel_l2(layer(x).double().cpu().numpy(), plain(x).double().cpu().numpy()) <= 1e-3
 
 
+@pytest.mark.parametrize("kind,out_f,in_f", [(k, 67, 1000) for k in ("narrow", "rare", "four", "real", "full_row", "wide")] +
+                         [("real", 9, 511), ("rare", 6, 32000), ("real", 6, 33800)])
+def test_infinite_activations(oracle, dev, kind, out_f, in_f):
+    """An infinite activation gives an infinity of the right sign, or NaN where a row's own weight is zero or another
+    infinity meets it: where the list's padding points (column 0), in columns with listed elements and in others."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    w = bits_to_bf16(oracle.decode_packed_bf16(p)).reshape(out_f, in_f).double()
+    listed = w.abs().argmax(1)  # of each row: the columns its largest weights are in
+    for m in (1, 2, 3, 4, 8, 20):
+        if m > 16 and in_f % 8:
+            continue
+        x = activations(m, in_f, seed=m)
+        for j in range(m):
+            x[j, (0, int(listed[j % out_f]), in_f - 1, int(listed[(j + 1) % out_f]))[j % 4]] = float("inf") if j % 3 else -float("inf")
+        if m > 2:
+            x[2, int(listed[2])] = float("inf")  # a second one
+            x[m - 1, 5] = float("nan")
+        want = torch.stack([(w * x[j].double()).sum(1) for j in range(m)])
+        if m <= 16:
+            y = product(lanes, x.to(dev), out_f, in_f).cpu().double()
+        else:
+            y = torch.empty((m, out_f), dtype=torch.bfloat16, device=dev)
+            lanes.gemm(x.to(dev), y)
+            y = y.cpu().double()
+        assert bool(want.isinf().any())
+        assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y[y.isinf()], want[want.isinf()])
+        fine = want.isfinite()
+        assert rel_l2(y[fine].numpy(), want[fine].bfloat16().double().numpy()) <= 1e-3
+
+
 @pytest.mark.parametrize("in_f", [1, 3, 7, 8, 9, 15])
 def test_rows_of_a_few_columns(oracle, dev, in_f):
     """Rows shorter than, as long as and just longer than a 16-byte piece."""
