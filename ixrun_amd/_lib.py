@@ -512,11 +512,15 @@ def encode_device(weight: torch.Tensor, level_bits) -> tuple:
     arrived = torch.empty(max(n_levels - 1, 1), dtype=torch.int64, pin_memory=True)  # the counts, as the kernel writes them
     with torch.cuda.device(dev):
         stream = current_stream(dev)
-        check(L.ixh_encode_scan_counts(weight.data_ptr(), out_f, in_f, n_levels, bits, scale.data_ptr(), table.data_ptr(),
-                                       workspace.data_ptr(), ws_bytes, arrived.data_ptr(), stream))
         left = out_f * in_f
         bitmaps, streams = [torch.empty((left + 31) // 32, dtype=torch.int32, device=dev)], []
-        check(L.ixh_encode_wait(arrived.data_ptr(), n_levels - 1, stream))  # the one synchronisation
+        try:
+            check(L.ixh_encode_scan_counts(weight.data_ptr(), out_f, in_f, n_levels, bits, scale.data_ptr(), table.data_ptr(),
+                                           workspace.data_ptr(), ws_bytes, arrived.data_ptr(), stream))
+            check(L.ixh_encode_wait(arrived.data_ptr(), n_levels - 1, stream))  # the one synchronisation
+        except BaseException:  # (an interrupt too) the kernel has to be done with `arrived` before that is given back
+            torch.cuda.current_stream(dev).synchronize()
+            raise
         counts = arrived.tolist()
         counts.append(out_f * in_f - sum(counts))
         for i, b in enumerate(level_bits[:-1]):

@@ -363,14 +363,12 @@ PyObject *encode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
         scale = at::empty({1}, options.dtype(at::kBFloat16));
         table = at::empty({levels - 1, entries}, options.dtype(at::kInt));
         arrived = at::empty({levels - 1}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+        bitmaps[0] = at::empty({(n + 31) / 32}, options.dtype(at::kInt));
         int32_t *ranks = static_cast<int32_t *>(table.data_ptr());
         int64_t *host = static_cast<int64_t *>(arrived.data_ptr());
         rc = library.encode_scan(src, out_f, in_f, levels, p.level_bits, static_cast<uint16_t *>(scale.data_ptr()), ranks,
                                  scratch.data_ptr(), bytes, host, stream);
-        if (!rc) {
-            bitmaps[0] = at::empty({(n + 31) / 32}, options.dtype(at::kInt));
-            rc = library.encode_wait(host, levels - 1, stream);
-        }
+        if (!rc) rc = library.encode_wait(host, levels - 1, stream);  // (nothing that throws in between: the kernel writes to `arrived`)
         if (!rc) {
             int64_t left = n;
             for (int i = 0; i < levels - 1; ++i) {

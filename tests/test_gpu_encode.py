@@ -191,3 +191,85 @@ def test_encode_full_size_layer(oracle, dev):
 def test_encode_span_edges(oracle, dev, n, level_bits, kind):
     """Around the 2048 elements of a wave and the 8192 of a workgroup, runs that are full, empty or split anywhere."""
     check_against_oracle(oracle, dev, make_weight(kind, 1, n), level_bits)
+
+
+SCAN = "ixh_encode_scan_counts"
+
+
+@pytest.fixture(params=["native", "python"])
+def watched_encode(request, monkeypatch, dev):
+    """``encode_device`` by its native and its Python way, with what the scan's launch does on the way in ``launches``."""
+    import ctypes as C
+
+    from ixrun_amd import _lib
+
+    L, launches = _lib.lib(), []
+    scan = getattr(L, SCAN)
+    proto = C.CFUNCTYPE(C.c_int, *(C.c_void_p if t is C.POINTER(C.c_int32) else t for t in scan.argtypes))
+    raw = proto(C.cast(scan, C.c_void_p).value)
+
+    def watch(*args):
+        launches.append(SCAN)
+        return raw(*args)
+
+    if request.param == "native":
+        watched = proto(watch)
+        monkeypatch.setattr(_lib, "_native", None)
+        with monkeypatch.context() as during:
+            during.setattr(L, SCAN, watched)
+            _lib.host()
+    else:
+        real = _lib.host()
+
+        class Host:
+            describe = staticmethod(real.describe)
+            encode = staticmethod(lambda *a: None)
+
+        monkeypatch.setattr(_lib, "host", lambda: Host)
+        monkeypatch.setattr(L, SCAN, lambda *a: (launches.append(SCAN), scan(*a))[1])
+    yield request.param, launches
+    monkeypatch.undo()
+    _lib._native = None  # bound to the library's own entry points again at its next use
+    _lib.host()
+
+
+def test_memory_for_the_bitmap_is_found_before_anything_runs(watched_encode, dev):
+    """The scan writes the counts to pinned memory that an exception would give back: where memory is short for the first
+    bitmap, the call fails with nothing launched."""
+    from ixrun_amd import _lib
+
+    _, launches = watched_encode
+    w = torch.zeros(16384, 16384, dtype=torch.bfloat16, device=dev)  # bitmap 34 MB; rank table and scratch 4 MB
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 30 * 2 ** 20) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            _lib.encode_device(w, (3, 5, 8))
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert not launches
+    _, _, counts = _lib.encode_device(w, (3, 5, 8))
+    assert launches and counts == [w.numel(), 0, 0]
+
+
+@pytest.mark.parametrize("watched_encode", ["python"], indirect=True)
+def test_interrupt_waits_for_the_scan(monkeypatch, watched_encode, dev):
+    """An exception between the scan's launch and the counts' arrival (the Python way; the native one has no such place)
+    leaves only when the stream is done with the counts' memory."""
+    from ixrun_amd import _lib
+
+    _, launches = watched_encode
+
+    def interrupted(*args):
+        raise KeyboardInterrupt
+
+    monkeypatch.setattr(_lib.lib(), "ixh_encode_wait", interrupted)
+    w = outlier_weight(512, 2048, seed=1).to(dev)
+    torch.cuda.synchronize()
+    torch.cuda._sleep(50_000_000)  # some 20 ms of other work in front
+    assert not torch.cuda.current_stream().query()
+    with pytest.raises(KeyboardInterrupt):
+        _lib.encode_device(w, (3, 5, 8))
+    assert launches and torch.cuda.current_stream().query()
