@@ -424,11 +424,17 @@ class LanePacked:
                                exc_val.data_ptr(), exc_pos.numel() // 4, scale.data_ptr())
 
     @staticmethod
-    def estimate(dp: DevicePacked, counts):
+    def estimate(level_bits, out_f: int, in_f: int, counts):
         """Bytes the layout of a packed tensor takes, to within the unevenness of its rows; None where it has none."""
-        bits = lane_bits(dp.level_bits, counts)
-        words = lib().ixh_lanes_plane_words(dp.out_f, dp.in_f, bits)
-        return None if words < 0 else 4 * words + 4 * sum(c for b, c in zip(dp.level_bits, counts) if b > bits)
+        bits, L = lane_bits(level_bits, counts), lib()
+        words, cells = L.ixh_lanes_plane_words(out_f, in_f, bits), L.ixh_lanes_cells(out_f, in_f)
+        if words < 0:
+            return None
+        return 4 * words + 4 * (cells + 1) + max(4 * sum(c for b, c in zip(level_bits, counts) if b > bits), 64 * 12)
+
+    @property
+    def nbytes(self) -> int:
+        return sum(t.numel() * t.element_size() for t in self.tensors)
 
     @classmethod
     def build(cls, dp: DevicePacked, table: torch.Tensor, unit: int, counts, into: "LanePacked | None" = None) -> "LanePacked":

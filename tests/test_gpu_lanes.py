@@ -424,6 +424,25 @@ def test_graph_serves_the_state_that_is_loaded(dev, in_f, grows):
     assert torch.equal(layer._decode().clone(), other._decode())
 
 
+@pytest.mark.parametrize("kind", ["rare", "real"])
+@pytest.mark.parametrize("out_f,in_f,lanes", [(512, 64, False), (3, 700, True), (1, 1000, False), (256, 520, True), (300, 320, True)])
+def test_layout_is_not_larger_than_the_weight(oracle, dev, kind, out_f, in_f, lanes):
+    """The layout's padding (whole blocks of 4 rows x 512 columns) is bounded: where it would take more than the bf16
+    weight, the layer is served from the packed streams."""
+    from ixrun_amd.engine import StreamingLinear
+
+    v, scheme, _ = values(kind, out_f, in_f)
+    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
+    layer = StreamingLinear(p)
+    assert (layer._lanes is not None) == lanes
+    if lanes:
+        assert layer._lanes.nbytes <= 2 * p["N"] + 4096  # (a list holds 64 quads at least)
+    layer._set_shared_buf(torch.empty(p["N"], dtype=torch.bfloat16, device=dev))
+    for m in (1, 4, 16, 40):
+        x = activations(m, in_f, seed=m)
+        check(oracle, p, x, layer(x.to(dev)))
+
+
 def test_malformed_lanes_are_refused(dev):
     from ixrun_amd import _lib
 
