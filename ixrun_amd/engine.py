@@ -70,6 +70,13 @@ def _plain_call(x) -> bool:
             and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") is torch.bfloat16))
 
 
+def _lane_bytes(level_bits, out_f, in_f, counts) -> int:
+    """Bytes of a layer's lane layout, to within the unevenness of its rows; 0 where it would take more than the bf16 weight
+    (see ``StreamingLinear._make_lanes``)."""
+    n_bytes = _lib.LanePacked.estimate(level_bits, out_f, in_f, counts) or 0
+    return n_bytes if n_bytes <= 2 * out_f * in_f else 0
+
+
 class StreamingLinear(nn.Module):
     """GPU-resident packed weight, decoded inside every forward.
 
@@ -159,9 +166,9 @@ class StreamingLinear(nn.Module):
         it (16384 x 520, one token 8 us against 25), rows of 64 take 42 where bf16 takes 16 (16384 x 64, one token 7.0 us
         against 6.8, 100 rows 16 against 10)."""
         self._lanes = None
-        n_bytes = _lib.LanePacked.estimate(self.level_bits, self.out_features, self.in_features, self.counts)
+        n_bytes = _lane_bytes(self.level_bits, self.out_features, self.in_features, self.counts)
         free, total = torch.cuda.mem_get_info(self._scale.device)
-        if self.N == 0 or n_bytes is None or n_bytes > 2 * self.N or free - n_bytes - 2 * self.N < total // 4:
+        if not n_bytes or free - n_bytes - 2 * self.N < total // 4:
             for name in LANE_BUFFERS:
                 self.register_buffer(name, None, persistent=False)
             self._bind()
@@ -416,21 +423,27 @@ class GraphLinear(nn.Module):
 
 
 class ResourceScheduler:
-    """Memory estimates and a mode recommendation (reference ``ixrun/engine.py:202-235``)."""
+    """Memory estimates and a mode recommendation (reference ``ixrun/engine.py:202-235``).
+
+    A streaming deploy keeps ``packed_storage_MB``, ``lane_storage_MB`` (the layout that the forwards read; nothing with
+    ``lanes=False``) and ``shared_decode_buf_MB`` on the GPU."""
 
     @staticmethod
     @torch.no_grad()
     def estimate(model: nn.Module, level_bits=(3, 5, 8)) -> dict:
-        bf16_bytes = packed_bytes = n_elems = max_layer = 0
+        bf16_bytes = packed_bytes = lane_bytes = n_elems = max_layer = 0
         for _, mod in iter_quantizable_linears(model):
             w = mod.weight.data
-            packed_bytes += int8x_quantize(w, level_bits)["total_bytes"]
+            packed = int8x_quantize(w, level_bits)
+            packed_bytes += packed["total_bytes"]
+            lane_bytes += _lane_bytes(packed["level_bits"], packed["out_f"], packed["in_f"], packed["counts"])
             bf16_bytes += w.numel() * 2
             n_elems += w.numel()
             max_layer = max(max_layer, w.numel())
         return {
             "bf16_weight_MB": bf16_bytes / 1e6,
             "packed_storage_MB": packed_bytes / 1e6,
+            "lane_storage_MB": lane_bytes / 1e6,
             "compression": bf16_bytes / max(packed_bytes, 1),
             "max_layer_elems": max_layer,
             "shared_decode_buf_MB": max_layer * 2 / 1e6,
@@ -461,7 +474,7 @@ class Int8XEngine:
 
     @classmethod
     def from_pretrained(cls, model_path: str, mode: str = "cached", level_bits=(3, 5, 8),
-                        dtype=torch.bfloat16, verbose: bool = True, cache_path: str | None = None):
+                        dtype=torch.bfloat16, verbose: bool = True, cache_path: str | None = None, lanes: bool = True):
         from transformers import AutoModelForCausalLM, AutoTokenizer
 
         tokenizer = AutoTokenizer.from_pretrained(model_path, trust_remote_code=True)
@@ -472,7 +485,7 @@ class Int8XEngine:
         if not big:
             model = model.cuda()
         if mode == "streaming":
-            stats = cls._deploy_streaming(model, level_bits, verbose=verbose, cache_path=cache_path)
+            stats = cls._deploy_streaming(model, level_bits, verbose=verbose, cache_path=cache_path, lanes=lanes)
         elif mode == "graph":
             stats, replay = cls._deploy_graph(model, level_bits, verbose=verbose)
             return cls(model, tokenizer, stats, graph_replay=replay)
@@ -492,13 +505,18 @@ class Int8XEngine:
 
     @staticmethod
     @torch.no_grad()
-    def _deploy_streaming(model, level_bits, verbose=True, cache_path=None):
+    def _deploy_streaming(model, level_bits, verbose=True, cache_path=None, lanes=True):
         """Packed weights resident on the GPU plus one shared decode buffer
         (reference ``ixrun/engine.py:343-416``).  ``cache_path`` names a file of
         already packed layers, ``{"level_bits": ..., "layers": [(name, packed,
         bias), ...]}``, written on the first deploy and read on later ones; a
         cache built with other ``level_bits`` or for other layer names raises
-        ``ValueError`` as in the reference (``:360-370``)."""
+        ``ValueError`` as in the reference (``:360-370``).
+
+        With ``lanes`` every layer also keeps the lane layout that its forwards read, while a quarter of the GPU's memory
+        stays free: the layers deployed last may go without and are slower for it.  The statistics say how many have one
+        (``n_lane_layers``), its bytes (``lane_bytes``) and all that the layers hold on the GPU (``resident_bytes``: packed
+        streams, rank tables, lanes, biases); ``total_bytes`` are the packed streams, as in the reference."""
         targets = list(iter_quantizable_linears(model))
         layer_data = None
         if cache_path is not None and os.path.exists(cache_path):
@@ -531,7 +549,7 @@ class Int8XEngine:
         total_bytes = max_n = 0
         layers = []
         for name, packed, bias in layer_data:
-            layers.append((name, StreamingLinear(packed, bias=bias)))
+            layers.append((name, StreamingLinear(packed, bias=bias, lanes=lanes)))
             total_bytes += packed["total_bytes"]
             max_n = max(max_n, packed["N"])
         shared_w = torch.empty(max_n, dtype=torch.bfloat16, device="cuda")
@@ -541,10 +559,14 @@ class Int8XEngine:
         gc.collect()
         torch.cuda.empty_cache()
         shared_mb = shared_w.numel() * 2 / 1e6
+        laid_out = [sl._lanes.nbytes for _, sl in layers if sl._lanes is not None]
+        resident = sum(b.numel() * b.element_size() for _, sl in layers for b in sl.buffers())
         if verbose:
-            print(f"[engine][streaming] {len(layers)} layers | packed GPU-resident={total_bytes / 1e6:.0f}MB | "
+            print(f"[engine][streaming] {len(layers)} layers | packed={total_bytes / 1e6:.0f}MB | "
+                  f"lane layout={sum(laid_out) / 1e6:.0f}MB on {len(laid_out)} layers | GPU-resident={resident / 1e6:.0f}MB | "
                   f"shared decode buf={shared_mb:.1f}MB", flush=True)
-        return {"mode": "streaming", "n_layers": len(layers), "total_bytes": total_bytes, "shared_gpu_MB": shared_mb}
+        return {"mode": "streaming", "n_layers": len(layers), "total_bytes": total_bytes, "shared_gpu_MB": shared_mb,
+                "lane_bytes": sum(laid_out), "n_lane_layers": len(laid_out), "resident_bytes": resident}
 
     @staticmethod
     @torch.no_grad()

@@ -92,6 +92,28 @@ def test_deploy_modes(tmp_path, rows):
         assert close(graph_model(x), want)
 
 
+def test_deploy_reports_what_it_holds(capsys):
+    """A streaming deploy says what the layers keep on the GPU beside the packed streams, and can be asked to keep no lanes."""
+    from ixrun_amd.engine import Int8XEngine, ResourceScheduler
+
+    base = toy_model()
+    expected = ResourceScheduler.estimate(base)
+    x = torch.randn(3, 512, generator=torch.Generator().manual_seed(5)).bfloat16().cuda()
+    want = int8_reference(base)(x)
+    for lanes in (True, False):
+        model = copy.deepcopy(base)
+        stats = Int8XEngine._deploy_streaming(model, (3, 5, 8), lanes=lanes)
+        held = {n: b.numel() * b.element_size() for n, b in model.named_buffers() if n.startswith("proj")}
+        assert stats["resident_bytes"] == sum(held.values())
+        assert stats["lane_bytes"] == sum(v for n, v in held.items() if "lane" in n)
+        assert stats["n_lane_layers"] == (2 if lanes else 0) and (stats["lane_bytes"] > 0) == lanes
+        assert stats["total_bytes"] == round(expected["packed_storage_MB"] * 1e6) < stats["resident_bytes"]
+        assert f"GPU-resident={stats['resident_bytes'] / 1e6:.0f}MB" in capsys.readouterr().out
+        if lanes:  # the estimate is of the list's elements, not of its rows' unevenness
+            assert abs(stats["lane_bytes"] / 1e6 / expected["lane_storage_MB"] - 1) < 0.15
+        assert close(model.cuda()(x), want)
+
+
 def test_five_level_streaming_linear():
     from ixrun_amd.engine import StreamingLinear
     from ixrun_amd.quantize import int8x_quantize, decode_to_weight
