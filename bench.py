@@ -1,10 +1,12 @@
 #!/usr/bin/env python3
 """Headline benchmark: fused (3,5,8) decode + GEMV on the 5120x17408 batch-1 layer.
 
-One step = one fused decode+GEMV over one packed layer.  The timed region walks
-round-robin over COPIES distinct packed copies of the layer (together larger
-than the 256 MB last-level cache) so that every launch streams its packed bytes
-from HBM.  Inputs are resident on the GPU before the clock starts.
+One step = one fused decode+GEMV over one deployed layer (``StreamingLinear``), which
+reads its weights from the lane layout, or with ``--packed`` from the packed streams.  The
+timed region walks round-robin over COPIES distinct copies of the layer (together larger
+than the 256 MB last-level cache) so that every launch streams its bytes from HBM; the
+roofline divides the bytes of the form that is read.  Inputs are resident on the GPU before
+the clock starts.
 
 Prints one JSON line.  Extra workloads (--workload) time the other shapes of the
 hot path with the same harness; the many-row (prefill) workload runs the fused
@@ -33,7 +35,8 @@ MFMA_BF16_PEAK = 2.5e15  # FLOP/s dense bf16, MI355X published
 # x 2.0 and x 1.0); the counter summaries are kept under profiles/.  Each figure carries the hash of the kernel
 # sources it was measured on (kernel_sources_sha16) and is reported only while the sources still hash to it;
 # workloads without a counter run, or measured on other sources, report null.
-# (bytes per launch, the sources the kernel is compiled from, their kernel_sources_sha16 at the counter run)
+# (bytes per launch, the sources the kernel is compiled from, their kernel_sources_sha16 at the counter run); names that end
+# in _packed are --packed runs, of the kernels that read the packed streams
 _ROWS = ("ixh_rows358.hip", "ixh_rows_common.h", "ixh_dev.h", "build.sh")
 _TILES = ("ixh_tiles358.hip", "ixh_rows_common.h", "ixh_dev.h")
 _DENSE = ("ixh_dense358.hip", "ixh_dense_tiles.h", "ixh_dev.h")
@@ -42,15 +45,15 @@ _PREFILL = ("ixh_prefill358.hip", "ixh_prefill358.h", "ixh_rows_common.h", "ixh_
 _DECODE_ROWS = ("ixh_decode_rows358.hip", "ixh_rows_common.h", "ixh_dev.h")
 _OLD = ((), "measured-on-earlier-sources")  # figures kept for the record; reported as null
 MEASURED_TRAFFIC_BYTES = {
-    "down_proj_5120x17408_m1_student_t": (23032.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "3e8407b518bc293b"),
-    "gate_up_17408x5120_m1_student_t": (22936.0 * 2.0 * 1024 + 40.0 * 1024, _ROWS, "3e8407b518bc293b"),
-    "attn_proj_5120x5120_m1_student_t": (7135.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "3e8407b518bc293b"),
-    "down_proj_5120x17408_m1_calibrated": (33825.0 * 2.0 * 1024 + 40.0 * 1024, _DENSE, "711eef94d053feb1"),
-    "down_proj_5120x17408_m1_five_level_calibrated": (49708.0 * 2.0 * 1024 + 1338.0 * 1024, _DENSE5, "aaca19573f1ed2a1"),
-    "gate_up_17408x5120_m4_student_t": (28740.0 * 2.0 * 1024 + 160.0 * 1024, _TILES, "21f9d013a3b417ff"),
-    "gate_up_17408x5120_m16_student_t": (26687.0 * 2.0 * 1024 + 640.0 * 1024, _TILES, "21f9d013a3b417ff"),
-    "attn_proj_5120x5120_m16_student_t": (8657.0 * 2.0 * 1024 + 640.0 * 1024, _TILES, "21f9d013a3b417ff"),
-    "down_proj_5120x17408_m16_student_t": (27677.0 * 2.0 * 1024 + 960.0 * 1024, _TILES, "21f9d013a3b417ff"),
+    "down_proj_5120x17408_m1_student_t_packed": (23032.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "3e8407b518bc293b"),
+    "gate_up_17408x5120_m1_student_t_packed": (22936.0 * 2.0 * 1024 + 40.0 * 1024, _ROWS, "3e8407b518bc293b"),
+    "attn_proj_5120x5120_m1_student_t_packed": (7135.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "3e8407b518bc293b"),
+    "down_proj_5120x17408_m1_calibrated_packed": (33825.0 * 2.0 * 1024 + 40.0 * 1024, _DENSE, "711eef94d053feb1"),
+    "down_proj_5120x17408_m1_five_level_calibrated_packed": (49708.0 * 2.0 * 1024 + 1338.0 * 1024, _DENSE5, "aaca19573f1ed2a1"),
+    "gate_up_17408x5120_m4_student_t_packed": (28740.0 * 2.0 * 1024 + 160.0 * 1024, _TILES, "21f9d013a3b417ff"),
+    "gate_up_17408x5120_m16_student_t_packed": (26687.0 * 2.0 * 1024 + 640.0 * 1024, _TILES, "21f9d013a3b417ff"),
+    "attn_proj_5120x5120_m16_student_t_packed": (8657.0 * 2.0 * 1024 + 640.0 * 1024, _TILES, "21f9d013a3b417ff"),
+    "down_proj_5120x17408_m16_student_t_packed": (27677.0 * 2.0 * 1024 + 960.0 * 1024, _TILES, "21f9d013a3b417ff"),
     "decode_5120x17408_five_level_calibrated": (49719.0 * 2.0 * 1024 + 174080.0 * 1024, _DENSE5, "aaca19573f1ed2a1"),
     "prefill_5120x5120_m512_five_level": (50297.9 * 2.0 * 1024 + 30720.0 * 1024,) + _OLD,
     # the three kernels of a step: k_prefill_xtile + k_prefill358 + k_prefill358_reduce
@@ -73,10 +76,10 @@ MEASURED_TRAFFIC_BYTES = {
 # rocprofv3 --pmc run of this script, mean over the launches), gated by the hash of the kernel's sources like the
 # traffic figures.  Reported per weight: vector and LDS instructions x 64 lanes / weights, scalar instructions / weights.
 MEASURED_INSTRUCTIONS = {
-    "down_proj_5120x17408_m1_student_t": ((5734195.0, 4469166.0, 1360042.0), _ROWS, "3e8407b518bc293b"),
-    "gate_up_17408x5120_m1_student_t": ((6030194.0, 4450915.0, 1414314.0), _ROWS, "3e8407b518bc293b"),
-    "attn_proj_5120x5120_m1_student_t": ((3570752.0, 2281697.0, 593732.0), _ROWS, "3e8407b518bc293b"),
-    "down_proj_5120x17408_m1_level1_only": ((4881551.0, 4104235.0, 1254926.0), _ROWS, "3e8407b518bc293b"),
+    "down_proj_5120x17408_m1_student_t_packed": ((5734195.0, 4469166.0, 1360042.0), _ROWS, "3e8407b518bc293b"),
+    "gate_up_17408x5120_m1_student_t_packed": ((6030194.0, 4450915.0, 1414314.0), _ROWS, "3e8407b518bc293b"),
+    "attn_proj_5120x5120_m1_student_t_packed": ((3570752.0, 2281697.0, 593732.0), _ROWS, "3e8407b518bc293b"),
+    "down_proj_5120x17408_m1_level1_only_packed": ((4881551.0, 4104235.0, 1254926.0), _ROWS, "3e8407b518bc293b"),
 }
 
 WORKLOADS = {
@@ -403,7 +406,17 @@ def measured_instructions(workload, n_weights):
             "lds_per_weight": round(lds * 64.0 / n_weights, 3)}
 
 
-def build_layers(workload, dev, copies=0, unfused=False):
+def form_read(layer, packed, rows):
+    """(name, bytes) of the form of a deployed layer's weights that a forward of so many rows reads: the lane layout (plane,
+    offsets, listed elements; not the list's spare room) or the packed streams."""
+    plan = layer._fused_plan(rows)
+    if plan[0] if plan else layer._lanes is not None and layer._gemm_ok and layer._lanes_gemm_wins(rows):
+        plane, off = layer._lanes.tensors[:2]
+        return "lanes", plane.numel() * 4 + off.numel() * 4 + int(off[-1]) * 12
+    return "packed", packed["total_bytes"]
+
+
+def build_layers(workload, dev, copies=0, unfused=False, lanes=True):
     """The packed layer of a workload (CPU generator, CPU writer: the literal recipe), `copies` device copies of it
     as StreamingLinear modules, and its activations."""
     from ixrun_amd.engine import StreamingLinear
@@ -415,7 +428,7 @@ def build_layers(workload, dev, copies=0, unfused=False):
     packed = int8x_quantize(weight, level_bits)
     chained = workload.startswith("graph64")
     copies = copies or (64 if chained else max(2, -(-600_000_000 // packed["total_bytes"])))
-    layers = [StreamingLinear(packed) for _ in range(copies)]
+    layers = [StreamingLinear(packed, lanes=lanes) for _ in range(copies)]
     if unfused:
         shared = torch.empty(packed["N"], dtype=torch.bfloat16, device=dev)
         for sl in layers:
@@ -550,13 +563,14 @@ def also_block(dev, args):
                 flops = 2.0 * m * out_f * in_f
                 r["TFLOP_per_s"] = round(flops / (ms * 1e-3) / 1e12, 1)
                 r["frac_mfma"] = round(flops / (ms * 1e-3) / MFMA_BF16_PEAK, 4)
-                # the same step against the HBM roofline: packed layer + activations in + outputs out
-                alg_bytes = packed["total_bytes"] + m * in_f * 2 + m * out_f * 2
+                # the same step against the HBM roofline: weights as they are read + activations in + outputs out
+                alg_bytes = form_read(layers[0], packed, m)[1] + m * in_f * 2 + m * out_f * 2
                 r["frac_hbm"] = round(alg_bytes / (ms * 1e-3) / HBM_PEAK, 4)
                 r["traffic"] = measured_traffic(name if variant == "fused" else name + "_unfused")
                 out.setdefault(name, {})["ixh_gemm" if variant == "fused" else "decode_plus_tuned_library_gemm"] = r
             else:
-                alg_bytes = packed["total_bytes"] + m * in_f * 2 + m * out_f * 2
+                r["form"], form_bytes = ("packed", packed["total_bytes"]) if variant != "fused" else form_read(layers[0], packed, m)
+                alg_bytes = form_bytes + m * in_f * 2 + m * out_f * 2
                 r["frac_hbm"] = round(alg_bytes / (ms * 1e-3) / HBM_PEAK, 4)
                 r["level_fractions"] = [round(c / packed["N"], 5) for c in packed["counts"]]
                 r["bits_per_weight"] = round(packed["bits_per_weight"], 3)
@@ -586,6 +600,7 @@ def main():
     ap.add_argument("--eager", action="store_true", help="time eager launches instead of hipGraph replays")
     ap.add_argument("--unfused", action="store_true",
                     help="many-row workloads: decode the bf16 weight to HBM and call the library GEMM instead")
+    ap.add_argument("--packed", action="store_true", help="layers without the lane layout: the kernels of ixh_gemv and ixh_gemm")
     ap.add_argument("--tune-gemm", action="store_true",
                     help="with --unfused: let the library GEMM of the many-row path be chosen by measurement")
     ap.add_argument("--set-option", action="append", default=[], metavar="NAME=VALUE",
@@ -615,7 +630,7 @@ def main():
     level_bits = rest[0] if rest else (3, 5, 8)
     headline = args.workload == "down_proj_5120x17408_m1_student_t"
     t0 = time.perf_counter()
-    weight, packed, layers, x_host, chained = build_layers(args.workload, dev, args.copies, args.unfused)
+    weight, packed, layers, x_host, chained = build_layers(args.workload, dev, args.copies, args.unfused, not args.packed)
     copies = len(layers)
     prep_s = time.perf_counter() - t0
     if args.tune_gemm:
@@ -625,9 +640,11 @@ def main():
         sl._gemv_flags = args.gemv_flags
         sl._forget_plans()
     x = x_host.to(dev)
-    table_bytes = layers[0]._table.numel() * 4
-    # algorithmic bytes of one step: the packed layer, the activations in, the outputs out
-    alg_bytes = packed["total_bytes"] + m * in_f * 2 + m * out_f * 2
+    # algorithmic bytes of one step: the weights in the form that is read, the activations in, the outputs out
+    form, form_bytes = form_read(layers[0], packed, m)
+    alg_bytes = form_bytes + m * in_f * 2 + m * out_f * 2
+    table_bytes = layers[0]._table.numel() * 4 if form == "packed" else 0  # (the lanes need no rank table)
+    counted = args.workload + ("_packed" if form == "packed" and m <= 16 else "")
 
     if args.calibrate_copy:
         src = torch.ones(256 << 20, dtype=torch.uint8, device=dev)
@@ -665,14 +682,14 @@ def main():
             "workload": args.workload, "out_f": out_f, "in_f": in_f, "batch": m, "level_bits": list(level_bits),
             "weights": recipe, "level_fractions": [c / packed["N"] for c in packed["counts"]],
             "bits_per_weight": packed["bits_per_weight"], "packed_bytes": packed["total_bytes"],
-            "rank_table_bytes": table_bytes, "distinct_copies": copies,
+            "form": form, "form_bytes": form_bytes, "rank_table_bytes": table_bytes, "distinct_copies": copies,
         },
         "roofline": {
             "bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
-            "frac": achieved / HBM_PEAK, "traffic": measured_traffic(args.workload),
-            **measured_instructions(args.workload, out_f * in_f),
-            "note": "algorithmic bytes = packed layer + x + y per launch; time = HIP-event time of the timed region / "
-                    "steps; traffic = HBM bytes per launch from rocprofv3 FETCH_SIZE / WRITE_SIZE runs of this script; "
+            "frac": achieved / HBM_PEAK, "traffic": measured_traffic(counted),
+            **measured_instructions(counted, out_f * in_f),
+            "note": "algorithmic bytes = weights in the form that is read (config.form) + x + y per launch; time = HIP-event "
+                    "time of the timed region / steps; traffic = HBM bytes per launch from rocprofv3 FETCH_SIZE / WRITE_SIZE runs of this script; "
                     "valu / lds_per_weight = wave instructions x 64 lanes / weights, salu_per_weight = scalar "
                     "instructions / weights, from an SQ_INSTS_* run (all null when the kernel sources have changed "
                     "since those runs)",
@@ -694,7 +711,8 @@ def main():
             "note": "2*M*N*K flops per launch pair (GEMM + slice reduce); the kernel is bound by the VALU decode "
                     "that feeds the matrix cores, not by MFMA issue",
         }
-        out["path"] = "decode to HBM + library GEMM" if args.unfused else "fused decode + MFMA (ixh_gemm)"
+        out["path"] = ("decode to HBM + library GEMM" if args.unfused else "fused decode + MFMA (ixh_lanes_gemm)" if form == "lanes"
+                       else "fused decode + MFMA (ixh_gemm)")
         if args.unfused and args.tune_gemm:
             out["path"] += ", GEMM kernel chosen by measurement (torch.cuda.tunable)"
     del graph, step, layers

@@ -149,18 +149,41 @@ def test_missing_library_is_loud(monkeypatch):
         _lib.lib()
 
 
-def test_bench_tables_are_well_formed():
-    """bench.py's workload table (shape, rows, recipe[, level scheme]) and its table of measured HBM traffic, whose
-    entries name sources that exist and workloads that the first table holds."""
-    import os
+def load_bench():
     import sys
 
-    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    sys.path.insert(0, root)
+    sys.path.insert(0, ROOT)
     try:
         import bench
     finally:
-        sys.path.remove(root)
+        sys.path.remove(ROOT)
+    return bench
+
+
+def test_bench_counts_the_form_that_is_read():
+    """bench.py divides the bytes of what a forward reads: the lane layout where the rows go there (its listed elements, not
+    the list's spare room), the packed streams otherwise."""
+    from types import SimpleNamespace as Of
+
+    bench = load_bench()
+    packed = {"total_bytes": 44}
+    off = torch.tensor([0, 3, 7], dtype=torch.int32)
+    lanes = Of(tensors=(torch.zeros(640, dtype=torch.int32), off, torch.zeros(400, dtype=torch.int16), torch.zeros(400, dtype=torch.int8)))
+    layer = Of(_lanes=lanes, _gemm_ok=True, _fused_plan=lambda rows: (rows < 8, ((0, rows, 0),), False) if rows <= 16 else False,
+               _lanes_gemm_wins=lambda rows: rows < 100)
+    read = 640 * 4 + 3 * 4 + 7 * 12
+    assert [bench.form_read(layer, packed, m) for m in (1, 50)] == [("lanes", read)] * 2
+    assert [bench.form_read(layer, packed, m) for m in (8, 200)] == [("packed", 44)] * 2
+    layer._gemm_ok = False
+    assert bench.form_read(layer, packed, 50) == ("packed", 44)
+    layer._lanes = None
+    assert bench.form_read(layer, packed, 50) == ("packed", 44)
+
+
+def test_bench_tables_are_well_formed():
+    """bench.py's workload table (shape, rows, recipe[, level scheme]) and its table of measured HBM traffic, whose
+    entries name sources that exist and workloads that the first table holds."""
+    bench, root = load_bench(), ROOT
     for name, spec in bench.WORKLOADS.items():
         assert len(spec) in (4, 5), name
         out_f, in_f, m, recipe = spec[:4]
@@ -168,5 +191,6 @@ def test_bench_tables_are_well_formed():
         assert out_f > 0 and in_f > 0 and 0 <= m <= 512, name  # m = 0: decode and encode workloads
     for name, (nbytes, files, sha16) in bench.MEASURED_TRAFFIC_BYTES.items():
         assert nbytes > 0 and isinstance(sha16, str), name
+        assert name.removesuffix("_unfused").removesuffix("_packed") in bench.WORKLOADS, name
         for f in files:
             assert os.path.exists(os.path.join(root, "ixrun_amd", "csrc", f)), (name, f)
