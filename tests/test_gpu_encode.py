@@ -158,14 +158,15 @@ def test_encode_rejects_bad_arguments(dev):
         _lib.encode_device(w, (3, 9, 8))
 
 
-def test_encoded_layer_runs(oracle, dev):
+@pytest.mark.parametrize("lanes", [True, False])
+def test_encoded_layer_runs(oracle, dev, lanes):
     """Encoder output straight into the module: decode gives back the int8, the fused product matches."""
     from ixrun_amd.engine import StreamingLinear
     from ixrun_amd.quantize import int8x_quantize_device
 
     w = student_t_weight(192, 2048, seed=4)
     p, q = check_against_oracle(oracle, dev, w, (3, 5, 8))
-    layer = StreamingLinear(p)
+    layer = StreamingLinear(p, lanes=lanes)
     q_dev = torch.empty(p["N"], dtype=torch.int8, device=dev)
     layer._dp.decode(layer._table, layer._unit, out_i8=q_dev)
     assert np.array_equal(q_dev.cpu().numpy(), q)

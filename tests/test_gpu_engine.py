@@ -114,13 +114,14 @@ def test_deploy_reports_what_it_holds(capsys):
         assert close(model.cuda()(x), want)
 
 
-def test_five_level_streaming_linear():
+@pytest.mark.parametrize("lanes", [True, False])
+def test_five_level_streaming_linear(lanes):
     from ixrun_amd.engine import StreamingLinear
     from ixrun_amd.quantize import int8x_quantize, decode_to_weight
 
     w = outlier_weight(256, 768, seed=7)
     p = int8x_quantize(w, (3, 4, 5, 6, 8))
-    sl = StreamingLinear(p)
+    sl = StreamingLinear(p, lanes=lanes)
     sl._set_shared_buf(torch.empty(p["N"], dtype=torch.bfloat16, device="cuda"))
     assert torch.equal(sl._decode().cpu(), decode_to_weight(p))
     for rows in (1, 5, 64):
@@ -162,8 +163,9 @@ def test_tuned_library_gemm_on_the_many_row_path(oracle):
     assert np.array_equal(tuned, again)
 
 
+@pytest.mark.parametrize("lanes", [True, False])
 @pytest.mark.parametrize("rows,dense", [(8, False), (16, False), (17, False), (4, True), (16, True), (17, True)])
-def test_row_count_policy_with_a_decode_buffer(oracle, rows, dense):
+def test_row_count_policy_with_a_decode_buffer(oracle, rows, dense, lanes):
     """Up to 16 rows the fused kernels, for dense level mixes as well, beyond that decode + GEMM when the layer has a
     decode buffer: all within the many-row tolerance of the exact product."""
     from ixrun_amd.engine import StreamingLinear
@@ -181,8 +183,8 @@ def test_row_count_policy_with_a_decode_buffer(oracle, rows, dense):
     x = torch.randn(rows, 2048, generator=torch.Generator("cpu").manual_seed(rows)).bfloat16()
     w_deq = oracle.bf16_bits_to_f32(oracle.decode_packed_bf16(p)).astype(np.float64).reshape(128, 2048)
     want = torch.from_numpy(x.double().numpy() @ w_deq.T).bfloat16().double().numpy()
-    plain = StreamingLinear(p)
-    buffered = StreamingLinear(p)
+    plain = StreamingLinear(p, lanes=lanes)
+    buffered = StreamingLinear(p, lanes=lanes)
     buf = torch.full((p["N"],), 9.0, dtype=torch.bfloat16, device=dev)
     buffered._set_shared_buf(buf)
     for layer in (plain, buffered):
@@ -194,7 +196,8 @@ def test_row_count_policy_with_a_decode_buffer(oracle, rows, dense):
 
 @pytest.mark.parametrize("rows", [16, 17, 24, 32, 33])
 @pytest.mark.parametrize("buffered", [False, True])
-def test_two_fused_calls_for_17_to_32_rows(oracle, monkeypatch, rows, buffered):
+@pytest.mark.parametrize("lanes", [True, False])
+def test_two_fused_calls_for_17_to_32_rows(oracle, monkeypatch, rows, buffered, lanes):
     """17 .. 32 rows on a large layer that is almost all level 1 go through the fused kernel in two calls (16 rows and
     the rest), with or without a decode buffer (which then stays untouched); 33 rows and small layers keep the
     many-row paths.  The size limit is lowered for the test so that a small layer counts as large."""
@@ -209,12 +212,12 @@ def test_two_fused_calls_for_17_to_32_rows(oracle, monkeypatch, rows, buffered):
     want = torch.from_numpy(x.double().numpy() @ w_deq.T).bfloat16().double().numpy()
     for limit, two_calls in ((0, 16 < rows <= 32), (engine.SPLIT_FUSED_MIN_WEIGHTS, False)):
         monkeypatch.setattr(engine, "SPLIT_FUSED_MIN_WEIGHTS", limit)
-        layer = engine.StreamingLinear(p)
+        layer = engine.StreamingLinear(p, lanes=lanes)
         buf = torch.full((p["N"],), 9.0, dtype=torch.bfloat16, device=dev)
         if buffered:
             layer._set_shared_buf(buf)
         calls = []
-        real = layer._gemv_fn  # the bound ixh_gemv; its fifth argument is the row count of the call
+        real = layer._gemv_fn  # the bound ixh_gemv or ixh_lanes_gemv; their fifth argument is the row count of the call
         monkeypatch.setattr(layer, "_gemv_fn", lambda *a: (calls.append(a[4]), real(*a))[1])
         got = layer(x.to(dev)).float().cpu().numpy()
         assert np.linalg.norm(got - want) / np.linalg.norm(want) <= 1e-3

@@ -10,13 +10,13 @@ from helpers import activations, bf16_bits, outlier_weight, student_t_weight
 pytestmark = pytest.mark.gpu
 
 
-def build_chain(n_layers, width, dev, maker, level_bits=(3, 5, 8)):
+def build_chain(n_layers, width, dev, maker, level_bits=(3, 5, 8), lanes=True):
     from ixrun_amd.engine import StreamingLinear
     from ixrun_amd.quantize import int8x_quantize
 
     layers = []
     for k in range(n_layers):
-        sl = StreamingLinear(int8x_quantize(maker(width, width, seed=k), level_bits))
+        sl = StreamingLinear(int8x_quantize(maker(width, width, seed=k), level_bits), lanes=lanes)
         layers.append(sl)
     return layers
 
@@ -35,19 +35,20 @@ def run_chain(layers, x):
     return h
 
 
+@pytest.mark.parametrize("lanes", [True, False])
 @pytest.mark.parametrize("maker,m,level_bits", [
     (student_t_weight, 1, (3, 5, 8)), (outlier_weight, 1, (3, 5, 8)), (student_t_weight, 4, (3, 5, 8)),
     (outlier_weight, 16, (3, 5, 8)), (dense_weight, 1, (3, 4, 5, 6, 8)), (student_t_weight, 16, (3, 4, 5, 6, 8)),
     (dense_weight, 2, (3, 5, 8)), (dense_weight, 8, (3, 5, 8)), (dense_weight, 16, (3, 5, 8)), (student_t_weight, 8, (3, 5, 8)),
     (student_t_weight, -8, (3, 5, 8)), (student_t_weight, -16, (3, 4, 5, 6, 8))])
-def test_graph_replay_matches_eager(maker, m, level_bits, gemv_option):
+def test_graph_replay_matches_eager(maker, m, level_bits, lanes, gemv_option):
     dev = torch.device("cuda:0")
-    if m < 0:  # the tile kernel with two workgroups to a block of rows: two launches a layer, pieces in the shared scratch
+    if m < 0:  # (packed streams) the tile kernel with two workgroups to a block of rows: two launches a layer, pieces in the shared scratch
         m = -m
         gemv_option("gemv_tiles", 1)
         gemv_option("gemv_tile_cus", 8)
         gemv_option("gemv_tile_split", 2)
-    layers = build_chain(6, 1024, dev, maker, level_bits)
+    layers = build_chain(6, 1024, dev, maker, level_bits, lanes)
     x = activations(m, 1024, seed=3).to(dev)
     eager = run_chain(layers, x).clone()
     torch.cuda.synchronize()
@@ -78,10 +79,11 @@ def test_graph_replay_matches_eager(maker, m, level_bits, gemv_option):
     assert torch.equal(static_y, run_chain(layers, x2))
 
 
+@pytest.mark.parametrize("lanes", [True, False])
 @pytest.mark.parametrize("shared_buffer", [False, True])
-def test_graph_replay_many_rows(shared_buffer):
-    """48 activation rows: the fused decode + MFMA GEMM (no decode buffer) and the bf16 decode + library GEMM
-    (with one), captured and replayed; five-level and dense (3,5,8) layers alternate down the chain."""
+def test_graph_replay_many_rows(shared_buffer, lanes):
+    """48 activation rows: the lanes' GEMM, or without lanes the fused decode + MFMA GEMM (no decode buffer) and the bf16
+    decode + library GEMM (with one), captured and replayed; five-level and dense (3,5,8) layers alternate down the chain."""
     from helpers import calibrated_weight
     from ixrun_amd.engine import StreamingLinear
     from ixrun_amd.quantize import int8x_quantize
@@ -94,7 +96,7 @@ def test_graph_replay_many_rows(shared_buffer):
             packed = int8x_quantize(student_t_weight(width, width, seed=k), (3, 4, 5, 6, 8))
         else:
             packed = int8x_quantize(calibrated_weight(width, width, seed=k, scale=0.0123046875)[0])
-        layers.append(StreamingLinear(packed))
+        layers.append(StreamingLinear(packed, lanes=lanes))
     if shared_buffer:
         shared = torch.empty(width * width, dtype=torch.bfloat16, device=dev)
         for sl in layers:
@@ -135,7 +137,8 @@ def _capture(fn, static_x):
     return graph, static_y
 
 
-def test_graph_64_layers_of_5120x5120():
+@pytest.mark.parametrize("lanes", [True, False])
+def test_graph_64_layers_of_5120x5120(lanes):
     """BASELINE config 5b as stated: a sequence of 64 packed 5120 x 5120 layers (64 distinct device copies, 0.85 GB
     of packed bytes), every per-layer launch captured in one hipGraph.  Replays equal the eager pass bit for bit; the
     first and the last layer's outputs are checked against the fp64 oracle on the inputs they really saw."""
@@ -147,7 +150,7 @@ def test_graph_64_layers_of_5120x5120():
     dev = torch.device("cuda:0")
     width, n_layers, n_distinct = 5120, 64, 4
     packed = [int8x_quantize(student_t_weight(width, width, seed=k)) for k in range(n_distinct)]
-    layers = [StreamingLinear(packed[k % n_distinct]) for k in range(n_layers)]
+    layers = [StreamingLinear(packed[k % n_distinct], lanes=lanes) for k in range(n_layers)]
 
     def chain(x, keep=None):
         h = x
@@ -189,7 +192,8 @@ def test_graph_64_layers_of_5120x5120():
     assert torch.equal(static_y, chain(x2))
 
 
-def test_graph_survives_a_larger_workspace_request():
+@pytest.mark.parametrize("lanes", [True, False])
+def test_graph_survives_a_larger_workspace_request(lanes):
     """A graph captured while the shared scratch was small keeps working after a bigger layer made the scratch grow:
     the replaced buffer stays alive, so the replay neither reads freed memory nor writes into tensors allocated
     afterwards."""
@@ -199,21 +203,25 @@ def test_graph_survives_a_larger_workspace_request():
 
     dev = torch.device("cuda:0")
     fused._workspaces.pop(dev, None)  # start from no scratch, whatever earlier tests left
-    # five-level layers with a dense mix: the staged kernel, whose pieces of a row meet in the workspace
-    layers = [StreamingLinear(int8x_quantize(outlier_weight(256, 2048, seed=k), (3, 4, 5, 6, 8))) for k in range(2)]
-    layers.append(StreamingLinear(int8x_quantize(outlier_weight(2048, 256, seed=9), (3, 4, 5, 6, 8))))
+    # five-level layers with a dense mix: the staged kernel (three rows), whose pieces of a row meet in the workspace, or the
+    # lanes' kernel for more than four rows, whose column slices do
+    layers = [StreamingLinear(int8x_quantize(outlier_weight(256, 2048, seed=k), (3, 4, 5, 6, 8)), lanes=lanes) for k in range(2)]
+    layers.append(StreamingLinear(int8x_quantize(outlier_weight(2048, 256, seed=9), (3, 4, 5, 6, 8)), lanes=lanes))
+    rows = 7 if lanes else 3
+    if lanes:
+        assert layers[0]._lanes.gemv_workspace_bytes(rows) > 0
 
     def chain(x):
         return layers[1](layers[2](layers[0](x)))
 
-    x = activations(3, 2048, seed=3).to(dev)
+    x = activations(rows, 2048, seed=3).to(dev)
     eager = chain(x).clone()
     small = fused._workspaces[dev]
     static_x = x.clone()
     graph, static_y = _capture(chain, static_x)
     assert fused._workspaces[dev] is small  # the capture itself did not grow it
 
-    big = StreamingLinear(int8x_quantize(outlier_weight(4096, 8192, seed=5), (3, 4, 5, 6, 8)))
+    big = StreamingLinear(int8x_quantize(outlier_weight(4096, 8192, seed=5), (3, 4, 5, 6, 8)), lanes=lanes)
     big(activations(16, 8192, seed=1).to(dev))
     assert fused._workspaces[dev] is not small and any(t is small for t in fused._retired)
     del small

@@ -443,6 +443,21 @@ def test_layout_is_not_larger_than_the_weight(oracle, dev, kind, out_f, in_f, la
         check(oracle, p, x, layer(x.to(dev)))
 
 
+def test_layer_goes_without_lanes_where_memory_is_short(monkeypatch, oracle, dev):
+    """A layout that would leave less than a quarter of the GPU's memory is not made; the layer serves from the packed streams."""
+    from ixrun_amd.engine import StreamingLinear
+
+    v, scheme, _ = values("real", 64, 1024)
+    p = packed_from_int8(v, 64, 1024, level_bits=scheme)
+    for free, lanes in ((60, False), (1000, True)):
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (free << 20, 240 << 20))
+        layer = StreamingLinear(p)
+        assert (layer._lanes is not None) == lanes
+        for m in (1, 3, 16):
+            x = activations(m, 1024, seed=m)
+            check(oracle, p, x, layer(x.to(dev)))
+
+
 def test_malformed_lanes_are_refused(dev):
     from ixrun_amd import _lib
 

@@ -637,8 +637,9 @@ def test_gemv_is_reproducible(oracle, dev):
         assert np.array_equal(run_gemv(dp, 512, x, 4, dev), first)
 
 
+@pytest.mark.parametrize("lanes", [True, False])
 @pytest.mark.parametrize("shape", [(1536, 1536), (4608, 1536), (1536, 4608)])
-def test_reference_call_surface(oracle, dev, shape):
+def test_reference_call_surface(oracle, dev, shape, lanes):
     """fused_gemv / StreamingLinear called the way the reference's tests call them
     (tests/test_fused.py:24-33, tests/test_splitk.py:25-33), on the reference's weight recipe."""
     from ixrun_amd.engine import StreamingLinear
@@ -665,7 +666,7 @@ def test_reference_call_surface(oracle, dev, shape):
         check_outputs(y32.cpu().numpy().reshape(1, -1), y64, f"fused_gemv split {shape}")
 
     bias = torch.randn(out_f, generator=torch.Generator().manual_seed(3)).bfloat16()
-    sl = StreamingLinear(p, bias=bias)
+    sl = StreamingLinear(p, bias=bias, lanes=lanes)
     shared = torch.empty(p["N"], dtype=torch.bfloat16, device=dev)
     sl._set_shared_buf(shared)
     assert np.array_equal(sl._q1.cpu().numpy(), (compute_row_prefixes(p, sl._split_chunk) if sl._split_chunk
@@ -698,21 +699,21 @@ def test_gemv_many_rows_to_a_workgroup(oracle, dev, kind, level_bits):
         check_outputs(y, oracle.gemm_f64(w_bits, bf16_bits(x)), f"{kind} {level_bits} {out_f}x{in_f} m={m}")
 
 
-@pytest.fixture(scope="module")
-def gate_up_layer(oracle, dev):
-    """BASELINE config 4's layer, 17408 x 5120 Student-t, packed once for its four batch sizes."""
+@pytest.fixture(scope="module", params=[True, False], ids=["lanes", "packed"])
+def gate_up_layer(oracle, dev, request):
+    """17408 x 5120 Student-t, packed once for its batch sizes, with the lane layout and without."""
     from ixrun_amd.engine import StreamingLinear
 
     p = quantize(student_t_weight(17408, 5120, seed=0))
     w_bits = oracle.decode_packed_bf16(p)
-    return StreamingLinear(p), w_bits
+    return StreamingLinear(p, lanes=request.param), w_bits
 
 
 @pytest.mark.parametrize("m", [1, 2, 4, 8, 16])
 def test_full_size_config4_every_batch(oracle, dev, gate_up_layer, m):
     """BASELINE config 4 as stated: 17408 x 5120 with M in {2, 4, 8, 16} activation rows, and one row, each through the
-    kernel the library picks for it (1 and 2 rows: the row-block kernel, 68 rows to a workgroup; 4, 8 and 16 rows: the
-    tile kernel, at 16 rows with the activations in two column parts)."""
+    kernel the library picks for it (from the packed streams 1 and 2 rows: the row-block kernel, 68 rows to a workgroup;
+    4, 8 and 16 rows: the tile kernel, at 16 rows with the activations in two column parts)."""
     sl, w_bits = gate_up_layer
     x = activations(m, 5120, seed=1)
     y = sl(x.to(dev))
@@ -720,19 +721,19 @@ def test_full_size_config4_every_batch(oracle, dev, gate_up_layer, m):
     check_outputs(bf16_bits(y), oracle.gemm_f64(w_bits, bf16_bits(x)), f"config 4 m={m}")
 
 
-@pytest.fixture(scope="module")
-def down_proj_layer(oracle, dev):
-    """The headline layer, 5120 x 17408 Student-t, packed once for several batch sizes."""
+@pytest.fixture(scope="module", params=[True, False], ids=["lanes", "packed"])
+def down_proj_layer(oracle, dev, request):
+    """The headline layer, 5120 x 17408 Student-t, packed once for several batch sizes, with lanes and without."""
     from ixrun_amd.engine import StreamingLinear
 
     p = quantize(student_t_weight(5120, 17408, seed=0))
-    return StreamingLinear(p), oracle.decode_packed_bf16(p)
+    return StreamingLinear(p, lanes=request.param), oracle.decode_packed_bf16(p)
 
 
 @pytest.mark.parametrize("m", [3, 6, 8, 9, 10, 12, 16, 24])
 def test_full_size_down_proj_many_rows(oracle, dev, down_proj_layer, m):
-    """5120 x 17408 with 3..16 activation rows as the library plans them on the whole device: 20 rows to a workgroup
-    at one or two activation rows; from three rows on blocks of 40 to 124 rows shared by two to six workgroups, each
+    """5120 x 17408 with 3..16 activation rows as the library plans them on the whole device; from the packed streams
+    20 rows to a workgroup at one or two activation rows; from three rows on blocks of 40 to 124 rows shared by two to six workgroups, each
     with a run of the column blocks (their sums added by a second launch); 24 rows in two calls."""
     sl, w_bits = down_proj_layer
     x = activations(m, 17408, seed=m)
@@ -765,14 +766,15 @@ def test_full_size_split_k_contract(oracle, dev):
     assert np.array_equal(y32.cpu().numpy(), once + once)
 
 
-def test_headline_kernel_is_reproducible(oracle, dev):
-    """Repeat launches of the row-block kernel on a layer that is almost all level 1 (the headline workload's kernel,
-    5120 x 17408 Student-t) give the same bits, for one and for four activation rows."""
+@pytest.mark.parametrize("lanes", [True, False])
+def test_headline_kernel_is_reproducible(oracle, dev, lanes):
+    """Repeat launches on a layer that is almost all level 1 (the headline workload, 5120 x 17408 Student-t; without lanes
+    the row-block kernel) give the same bits, for one and for four activation rows."""
     from ixrun_amd.engine import StreamingLinear
 
     p = quantize(student_t_weight(5120, 17408, seed=0))
     assert p["counts"][0] >= 0.97 * p["N"]
-    sl = StreamingLinear(p)
+    sl = StreamingLinear(p, lanes=lanes)
     for m in (1, 4):
         x = activations(m, 17408, seed=5).to(dev)
         first = bf16_bits(sl(x))
@@ -780,8 +782,9 @@ def test_headline_kernel_is_reproducible(oracle, dev):
             assert np.array_equal(bf16_bits(sl(x)), first), m
 
 
+@pytest.mark.parametrize("lanes", [True, False])
 @pytest.mark.parametrize("shape,m", [((5120, 5120), 1), ((5120, 17408), 1), ((17408, 5120), 4)])
-def test_full_size_layers(oracle, dev, shape, m):
+def test_full_size_layers(oracle, dev, shape, m, lanes):
     """BASELINE configs 2, 3 and 4 at full size: decoded int8 bit-exact, outputs within tolerance."""
     from ixrun_amd.engine import StreamingLinear
 
@@ -789,7 +792,7 @@ def test_full_size_layers(oracle, dev, shape, m):
     w = student_t_weight(out_f, in_f, seed=0)
     p = quantize(w)
     q_want = oracle.decode_packed_i8(p)
-    sl = StreamingLinear(p)
+    sl = StreamingLinear(p, lanes=lanes)
     o8 = torch.empty(p["N"], dtype=torch.int8, device=dev)
     sl._dp.decode(sl._table, sl._unit, out_i8=o8)
     assert np.array_equal(o8.cpu().numpy(), q_want)
@@ -818,7 +821,8 @@ def test_full_size_five_level_decode(oracle, dev):
     assert np.array_equal(bf16_bits(o16), oracle.decode_packed_bf16(p).reshape(-1))
 
 
-def test_full_size_calibrated_layer(oracle, dev):
+@pytest.mark.parametrize("lanes", [True, False])
+def test_full_size_calibrated_layer(oracle, dev, lanes):
     """5120 x 17408 with the 55/40/5 level mix of real LLM weights: the any-scheme kernels on runs of more than
     eight table units per wave (GEMV pieces of 8-9 units, decode runs of 11), against the oracle."""
     from ixrun_amd.engine import StreamingLinear
@@ -826,12 +830,12 @@ def test_full_size_calibrated_layer(oracle, dev):
     out_f, in_f = 5120, 17408
     w, _ = calibrated_weight(out_f, in_f, seed=0, scale=0.0123046875)
     p = quantize(w)
-    sl = StreamingLinear(p)
+    sl = StreamingLinear(p, lanes=lanes)
     shared = torch.empty(p["N"], dtype=torch.bfloat16, device=dev)
     sl._set_shared_buf(shared)
     w_bits = oracle.decode_packed_bf16(p)
     assert np.array_equal(bf16_bits(sl._decode()), w_bits)
-    # two rows: weights gathered per wave; eight and sixteen: the matrix-pipe kernel (a row block's spans lie in two
+    # (without lanes) two rows: weights gathered per wave; eight and sixteen: the matrix-pipe kernel (a row block's spans lie in two
     # workgroups here: 320 blocks of 16 rows x 9 spans dealt to one workgroup per CU)
     for m in (2, 8, 16):
         x = activations(m, in_f, seed=m)

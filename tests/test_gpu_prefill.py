@@ -181,13 +181,14 @@ def test_gemm_rejects_what_it_cannot_take(oracle, dev):
     assert e.value.code == -4
 
 
-def test_streaming_linear_takes_the_fused_gemm(oracle, dev):
+@pytest.mark.parametrize("lanes", [True, False])
+def test_streaming_linear_takes_the_fused_gemm(oracle, dev, lanes):
     """Five-level layer, 48 rows: StreamingLinear.forward must not touch the decode buffer."""
     from ixrun_amd.engine import StreamingLinear
 
     out_f, in_f = 192, 5120
     p = quantize(student_t_weight(out_f, in_f, seed=5), (3, 4, 5, 6, 8))
-    sl = StreamingLinear(p)  # no shared buffer set: a decode would fail
+    sl = StreamingLinear(p, lanes=lanes)  # no shared buffer set: a decode would fail
     x = activations(48, in_f, seed=2)
     y = sl(x.to(dev).reshape(2, 24, in_f))
     assert y.shape == (2, 24, out_f) and y.dtype == torch.bfloat16
