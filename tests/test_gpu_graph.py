@@ -139,7 +139,7 @@ def _capture(fn, static_x):
 
 @pytest.mark.parametrize("lanes", [True, False])
 def test_graph_64_layers_of_5120x5120(lanes):
-    """BASELINE config 5b as stated: a sequence of 64 packed 5120 x 5120 layers (64 distinct device copies, 0.85 GB
+    """A sequence of 64 packed 5120 x 5120 layers (64 distinct device copies, 0.85 GB
     of packed bytes), every per-layer launch captured in one hipGraph.  Replays equal the eager pass bit for bit; the
     first and the last layer's outputs are checked against the fp64 oracle on the inputs they really saw."""
     from ixrun_amd.engine import StreamingLinear

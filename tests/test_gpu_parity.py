@@ -220,7 +220,7 @@ def test_decode_other_level_schemes(oracle, dev, level_bits):
 
 
 def test_decode_config1_2048(oracle, dev):
-    """BASELINE config 1: 2048x2048 Student-t, int8 round trip bit-exact, level fractions reported."""
+    """2048x2048 Student-t, int8 round trip bit-exact, level fractions reported."""
     from ixrun_amd.triton_kernels import decode_weight_triton, decode_int8
 
     w = student_t_weight(2048, 2048, seed=0)
@@ -235,7 +235,7 @@ def test_decode_config1_2048(oracle, dev):
 
 # ---------------------------------------------------------------- fused decode + GEMV
 def test_gemv_config1_2048(oracle, dev):
-    """BASELINE config 1 through the fused path: ixh_gemv on the 2048 x 2048 Student-t tensor, one activation row,
+    """The fused path: ixh_gemv on the 2048 x 2048 Student-t tensor, one activation row,
     against the fp64 oracle; once with the kernel the library picks for this mix, once with the (3,5,8) row-block
     kernels forced (IXH_GEMV_FORCE_358), bf16 output and the fp32 atomic mode."""
     from ixrun_amd import _lib
@@ -711,14 +711,14 @@ def gate_up_layer(oracle, dev, request):
 
 @pytest.mark.parametrize("m", [1, 2, 4, 8, 16])
 def test_full_size_config4_every_batch(oracle, dev, gate_up_layer, m):
-    """BASELINE config 4 as stated: 17408 x 5120 with M in {2, 4, 8, 16} activation rows, and one row, each through the
+    """17408 x 5120 with M in {2, 4, 8, 16} activation rows, and one row, each through the
     kernel the library picks for it (from the packed streams 1 and 2 rows: the row-block kernel, 68 rows to a workgroup;
     4, 8 and 16 rows: the tile kernel, at 16 rows with the activations in two column parts)."""
     sl, w_bits = gate_up_layer
     x = activations(m, 5120, seed=1)
     y = sl(x.to(dev))
     assert y.shape == (m, 17408)
-    check_outputs(bf16_bits(y), oracle.gemm_f64(w_bits, bf16_bits(x)), f"config 4 m={m}")
+    check_outputs(bf16_bits(y), oracle.gemm_f64(w_bits, bf16_bits(x)), f"17408x5120 m={m}")
 
 
 @pytest.fixture(scope="module", params=[True, False], ids=["lanes", "packed"])
@@ -785,7 +785,7 @@ def test_headline_kernel_is_reproducible(oracle, dev, lanes):
 @pytest.mark.parametrize("lanes", [True, False])
 @pytest.mark.parametrize("shape,m", [((5120, 5120), 1), ((5120, 17408), 1), ((17408, 5120), 4)])
 def test_full_size_layers(oracle, dev, shape, m, lanes):
-    """BASELINE configs 2, 3 and 4 at full size: decoded int8 bit-exact, outputs within tolerance."""
+    """The square, down and gate/up layers at full size: decoded int8 bit-exact, outputs within tolerance."""
     from ixrun_amd.engine import StreamingLinear
 
     out_f, in_f = shape

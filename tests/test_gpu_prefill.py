@@ -213,6 +213,6 @@ def test_full_size_prefill_square_layer(oracle, dev):
 
 
 def test_full_size_prefill_config5(oracle, dev):
-    """BASELINE config 5 as stated: W 5120 x 17408 in the five-level scheme (3,4,5,6,8), 512 activation rows, through
+    """W 5120 x 17408 in the five-level scheme (3,4,5,6,8), 512 activation rows, through
     ixh_gemm (decode into LDS tiles, bf16 MFMA, fp32 accumulate); 192 sampled output columns against the fp64 oracle."""
-    _full_size_prefill(oracle, dev, 5120, 17408, 512, "config 5: 5120x17408 five-level m=512")
+    _full_size_prefill(oracle, dev, 5120, 17408, 512, "5120x17408 five-level m=512")
