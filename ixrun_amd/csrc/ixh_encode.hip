@@ -263,8 +263,8 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// k_enc_pack<L>: bound by vector issue: of 5120 x 17408 at levels 3, 5, 8 about 700 instructions a wave and span, 68 us
-// (heavy tails) to 74 us (55 / 40 / 5 %); the 240 MB that it moves take 47.
+// k_enc_pack<L>: bound by vector issue: of 5120 x 17408 at levels 3, 5, 8 690 vector instructions a wave and span (heavy tails)
+// to 790 (55 / 40 / 5 %), 70 to 75 us; the 240 MB that it moves take 47.
 //
 // A wave takes spans of four units, 2048 elements, 32 consecutive ones a lane, so one prefix sum over the lanes serves them
 // all and a lane's membership bits are a whole word of bitmap 0.  Every element goes to LDS as one byte, value + 128: those
@@ -279,7 +279,7 @@ constexpr uint32_t kEncBuf = kEncSpan + 256;  // two runs with their margins
 constexpr uint32_t dense_at = 32u;            // where a dense run's groups start in it
 
 // Spans per wave: a wave that goes on hands its unfinished groups to its next span in registers, and only its first and last
-// cost atomics (one span each: 107 .. 175 us instead of 68 .. 74).  As many as leave the chip some 4096 waves, at most 8.
+// cost atomics (one span each: 107 .. 175 us instead of 70 .. 75).  As many as leave the chip some 4096 waves, at most 8.
 constexpr uint32_t kEncMaxSpans = 8, kEncFill = 4096;
 
 // level i's rank at unit `u`, and the index of the unit's first element in bitmap i

@@ -10,9 +10,10 @@ namespace ixh {
 // Bound: a stage's latency (decode, list and products follow one another in a wave, and all waves meet at its end: 3 to 8
 // thousand clocks), then LDS (per 16 x 128 weights a wave reads 4 MB / NB KB of activations, writes and reads 8 KB of weights and
 // looks up 4 KB of pairs). 10240 x 5120 at 55 / 40 / 5 %, 100 rows: 44.5 us with the slices' sums, of which the products are
-// 11 and the listed elements 8; 74.3 for the decode to memory and the library's GEMM. A wave takes 16 weight rows x 128 columns a
-// stage: it decodes them to its own 4 KB of LDS in operand order, stores the listed elements over their places and
-// reads the operands back.  All waves of the workgroup are in the same 128 columns, whose activations one copy in LDS
+// 11 and the listed elements 8 (the matrix unit is busy for 12 % of it); 74.3 for the decode to memory and the library's
+// GEMM. A wave takes 16 weight rows x 128 columns a stage: it decodes them to its own 4 KB of LDS in operand order, stores
+// the listed elements over their places and reads the operands back.  All waves of the workgroup are in the same 128
+// columns, whose activations one copy in LDS
 // serves (in operand order, two stages of it: the next one is fetched during the multiply), so a weight is decoded
 // once per 128 activation rows and never reaches memory.  One barrier a stage, which waits for LDS only: codes
 // and list are asked for one cell ahead.

@@ -3,7 +3,8 @@
 ``StreamingLinear`` keeps a layer's packed streams resident on the GPU and
 serves every forward from them: up to 16 activation rows go through the fused
 decode+GEMV kernel (the bf16 weight never reaches memory), prompts of up to 160
-to 512 rows through a fused decode+GEMM, larger ones are decoded into a shared bf16 buffer and multiplied with ``F.linear``.
+to 512 rows through a fused decode+GEMM, larger ones are decoded into a shared
+bf16 buffer and multiplied with ``F.linear``.
 ``GraphLinear`` / ``Int8XEngine`` follow the reference's ``ixrun/engine.py``
 (``StreamingLinear`` ``:40-173``, ``GraphLinear`` ``:179-196``,
 ``ResourceScheduler`` ``:202-235``, ``Int8XEngine`` ``:241-516``) and keep its
@@ -89,10 +90,10 @@ class StreamingLinear(nn.Module):
 
     With ``lanes`` the same integers are kept in the lane layout as well
     (``csrc/ixh_lanes.h``; 3.1 to 6.5 bits a weight for the mixes that take 4.0
-    to 5.5 packed), which the forwards of up to 16 rows read: one row of
-    5120 x 17408 takes 14 us from it instead of 17 (99 % of the weights in
-    level 1), 20 us instead of 48 (55 / 40 / 5 %), five levels 20 us instead of
-    86.  It is no part of the state dict.
+    to 5.5 packed), which the forwards of up to 16 rows and of most prompts
+    read: one row of 5120 x 17408 takes 14.6 us from it instead of 16.8 (99 %
+    of the weights in level 1), 18.7 instead of 48.7 (55 / 40 / 5 %), five
+    levels 18.7 instead of 86.  It is no part of the state dict.
     """
 
     def __init__(self, packed: dict, bias=None, lanes: bool = True):
@@ -199,7 +200,11 @@ class StreamingLinear(nn.Module):
         against 29 / 35 / 57 / 75, 17408 x 5120 92 / 97 / 107 / 110 against 48 / 55 / 88 / 124.  Below 2**24 weights the decode,
         the GEMM and the host's way through both weigh more: 12000 x 768 at 256 rows 35 against 29 from a graph, 2048 x 2048
         23 against 22 (eager: 30 against 22), and up to 2**20 weights 15 against 16 at 512 rows (eager 31 against 19).  Layers
-        of at most 2**18 weights keep decoding into their buffer (12 us against 8), which callers see there."""
+        of at most 2**18 weights keep decoding into their buffer (12 us against 8), which callers see there.  Planes of 8 bits
+        have no list and are ahead longer than those of 5, whose limits they share (64 / 100 / 160 / 256 rows: 10240 x 5120
+        57 / 61 / 68 / 82 against 27 / 36 / 49 / 72, 17408 x 5120 103 / 106 / 115 / 138 against 49 / 57 / 81 / 121, 4096 x
+        4096 28 / 30 / 38 / 34 against 17 / 22 / 25 / 32).  Rows of up to 256 columns are behind from some 80 rows on where no
+        host time counts (16384 x 256, 100 rows, 16 against 17 from a graph) and ahead eager (30 against 17)."""
         n = self.N
         return (self._lanes is not None and self._gemv_flags == 0 and self.in_features % 8 == 0 and n > 1 << 18
                 and rows * self.in_features < 1 << 31

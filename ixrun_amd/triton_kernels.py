@@ -69,8 +69,8 @@ def decode_weight_triton(packed: dict, device=None, dtype=torch.bfloat16) -> tor
     dp = _lib.DevicePacked.from_dict(packed, device)
     out = torch.empty(packed["N"], dtype=torch.bfloat16, device=device)
     if packed["N"]:
-        # units of 512: what the fast decoders take (17408 x 5120 at 55 / 40 / 5 %: 54 us; from units of 1024 the general
-        # decoder takes 330).  The device encoder leaves their table in the dictionary.
+        # units of 512: what the fast decoders take (17408 x 5120 at 55 / 40 / 5 %: 58 us; from units of 1024 the general
+        # decoder takes 402).  The device encoder leaves their table in the dictionary.
         table = packed.get("table512")
         if table is None or table.device != dp.device:
             table = dp.prefix_build(FUSED_TILE)
