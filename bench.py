@@ -37,49 +37,64 @@ MFMA_BF16_PEAK = 2.5e15  # FLOP/s dense bf16, MI355X published
 # workloads without a counter run, or measured on other sources, report null.
 # (bytes per launch, the sources the kernel is compiled from, their kernel_sources_sha16 at the counter run); names that end
 # in _packed are --packed runs, of the kernels that read the packed streams
+_LANES = ("ixh_lanes.hip", "ixh_lanes_gemm.hip", "ixh_lanes.h", "ixh_lanes_dev.h", "ixh_lanes_bounds.h", "ixh_fast358.h", "ixh_dev.h",
+          "build.sh")
 _ROWS = ("ixh_rows358.hip", "ixh_rows_common.h", "ixh_dev.h", "build.sh")
 _TILES = ("ixh_tiles358.hip", "ixh_rows_common.h", "ixh_dev.h")
 _DENSE = ("ixh_dense358.hip", "ixh_dense_tiles.h", "ixh_dev.h")
 _DENSE5 = ("ixh_dense5.hip", "ixh_dense_tiles.h", "ixh_dev.h")
 _PREFILL = ("ixh_prefill358.hip", "ixh_prefill358.h", "ixh_rows_common.h", "ixh_dev.h")
 _DECODE_ROWS = ("ixh_decode_rows358.hip", "ixh_rows_common.h", "ixh_dev.h")
+_ENCODE = ("ixh_encode.hip", "ixh_dev.h")
 _OLD = ((), "measured-on-earlier-sources")  # figures kept for the record; reported as null
 MEASURED_TRAFFIC_BYTES = {
-    "down_proj_5120x17408_m1_student_t_packed": (23032.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "3e8407b518bc293b"),
-    "gate_up_17408x5120_m1_student_t_packed": (22936.0 * 2.0 * 1024 + 40.0 * 1024, _ROWS, "3e8407b518bc293b"),
-    "attn_proj_5120x5120_m1_student_t_packed": (7135.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "3e8407b518bc293b"),
-    "down_proj_5120x17408_m1_calibrated_packed": (33825.0 * 2.0 * 1024 + 40.0 * 1024, _DENSE, "711eef94d053feb1"),
-    "down_proj_5120x17408_m1_five_level_calibrated_packed": (49708.0 * 2.0 * 1024 + 1338.0 * 1024, _DENSE5, "aaca19573f1ed2a1"),
-    "gate_up_17408x5120_m4_student_t_packed": (28740.0 * 2.0 * 1024 + 160.0 * 1024, _TILES, "21f9d013a3b417ff"),
-    "gate_up_17408x5120_m16_student_t_packed": (26687.0 * 2.0 * 1024 + 640.0 * 1024, _TILES, "21f9d013a3b417ff"),
-    "attn_proj_5120x5120_m16_student_t_packed": (8657.0 * 2.0 * 1024 + 640.0 * 1024, _TILES, "21f9d013a3b417ff"),
-    "down_proj_5120x17408_m16_student_t_packed": (27677.0 * 2.0 * 1024 + 960.0 * 1024, _TILES, "21f9d013a3b417ff"),
-    "decode_5120x17408_five_level_calibrated": (49719.0 * 2.0 * 1024 + 174080.0 * 1024, _DENSE5, "aaca19573f1ed2a1"),
+    # k_lanes_gemv; from eight rows on k_lanes_gemm + k_lanes_reduce
+    "down_proj_5120x17408_m1_student_t": (17304.1 * 2.0 * 1024 + 16.0 * 1024, _LANES, "7d30d618c9f315ad"),
+    "down_proj_5120x17408_m1_calibrated": (35836.2 * 2.0 * 1024 + 16.0 * 1024, _LANES, "7d30d618c9f315ad"),
+    "down_proj_5120x17408_m1_five_level_calibrated": (35841.6 * 2.0 * 1024 + 16.0 * 1024, _LANES, "7d30d618c9f315ad"),
+    "gate_up_17408x5120_m8_calibrated": ((53254.3 + 2734.0) * 2.0 * 1024 + (7385.3 + 272.0) * 1024, _LANES, "7d30d618c9f315ad"),
+    "down_proj_5120x17408_m16_student_t": ((23830.6 + 1934.0) * 2.0 * 1024 + (3840.0 + 160.0) * 1024, _LANES, "7d30d618c9f315ad"),
+    "down_proj_5120x17408_m1_student_t_packed": (23032.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "bb78197b94a98e49"),
+    "gate_up_17408x5120_m1_student_t_packed": (22936.0 * 2.0 * 1024 + 40.0 * 1024, _ROWS, "bb78197b94a98e49"),
+    "attn_proj_5120x5120_m1_student_t_packed": (7135.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "bb78197b94a98e49"),
+    "down_proj_5120x17408_m1_calibrated_packed": (33828.0 * 2.0 * 1024 + 40.0 * 1024, _DENSE, "931a9c677790f220"),
+    "down_proj_5120x17408_m1_five_level_calibrated_packed": (49709.0 * 2.0 * 1024 + 1339.0 * 1024, _DENSE5, "eb26928c946e5c46"),
+    "gate_up_17408x5120_m4_student_t_packed": (28730.0 * 2.0 * 1024 + 160.0 * 1024, _TILES, "d56530b1958e0076"),
+    "gate_up_17408x5120_m16_student_t_packed": (26680.0 * 2.0 * 1024 + 640.0 * 1024, _TILES, "d56530b1958e0076"),
+    "attn_proj_5120x5120_m16_student_t_packed": (8657.0 * 2.0 * 1024 + 640.0 * 1024, _TILES, "d56530b1958e0076"),
+    "down_proj_5120x17408_m16_student_t_packed": (27677.0 * 2.0 * 1024 + 960.0 * 1024, _TILES, "d56530b1958e0076"),
+    "decode_5120x17408_calibrated": (37327.0 * 2.0 * 1024 + 174080.0 * 1024, _DENSE, "931a9c677790f220"),
+    "decode_5120x17408_five_level_calibrated": (50960.0 * 2.0 * 1024 + 174080.0 * 1024, _DENSE5, "eb26928c946e5c46"),
     "prefill_5120x5120_m512_five_level": (50297.9 * 2.0 * 1024 + 30720.0 * 1024,) + _OLD,
     # the three kernels of a step: k_prefill_xtile + k_prefill358 + k_prefill358_reduce
-    "prefill_5120x17408_m512_five_level": ((8716.0 + 68452.0 + 30734.0) * 2.0 * 1024 + (17408.0 + 61606.0 + 5120.0) * 1024,
-                                           _PREFILL, "55862ec6d8c72acd"),
+    "prefill_5120x17408_m512_five_level": ((8716.0 + 68498.0 + 30734.0) * 2.0 * 1024 + (17408.0 + 61606.0 + 5120.0) * 1024,
+                                           _PREFILL, "63398a2e235eb8d3"),
     # k_decode358_rows<true> (x 2.0 / x 1.0 as above) + the operands and outputs of the library GEMM that
     # torch.cuda.tunable picked (bf16 weight, X, Y: its FETCH_SIZE, 158,001, is weighted for other request sizes than
     # our kernels' and fixes its reads only between 162 and 324 MB)
-    "prefill_5120x17408_m512_five_level_unfused": (23101.0 * 2.0 * 1024 + 179854.0 * 1024
+    "prefill_5120x17408_m512_five_level_unfused": (23079.0 * 2.0 * 1024 + 179701.0 * 1024
                                                    + 2.0 * (5120 * 17408 + 512 * 17408 + 512 * 5120),
-                                                   _DECODE_ROWS, "54f9e436740640ef"),
+                                                   _DECODE_ROWS, "075e833956492693"),
     "decode_5120x17408_student_t": (23268.0 * 2.0 * 1024 + 179524.0 * 1024,) + _OLD,
-    "decode_5120x17408_calibrated": (36308.0 * 2.0 * 1024 + 174080.0 * 1024,) + _OLD,
     "decode_gs_5120x17408_student_t": (33559.0 * 2.0 * 1024 + 174080.0 * 1024,) + _OLD,
-    # all kernels of one encode step together (absmax, count, scans, clear, pack)
-    "encode_5120x17408_student_t": ((87053 + 87092 + 1402 + 15 + 92442) * 2.0 * 1024 + (32 + 2040 + 1362 + 32694 + 63405) * 1024,) + _OLD,
+    # all kernels of one encode step together (absmax, count, scan, borders, pack)
+    "encode_5120x17408_student_t": ((87061.0 + 87111.3 + 783.4 + 698.7 + 89483.2) * 2.0 * 1024
+                                    + (8.0 + 2285.2 + 1362.7 + 321.2 + 46935.8) * 1024, _ENCODE, "1b65ebbfa9fe9a7f"),
+    "encode_5120x17408_calibrated": ((87061.0 + 87111.2 + 783.4 + 698.7 + 89659.6) * 2.0 * 1024
+                                     + (8.0 + 2291.0 + 1362.7 + 637.6 + 68649.1) * 1024, _ENCODE, "1b65ebbfa9fe9a7f"),
 }
 
 # Wave-level instruction counts per launch of the dominant kernel (SQ_INSTS_VALU, SQ_INSTS_SALU, SQ_INSTS_LDS from one
 # rocprofv3 --pmc run of this script, mean over the launches), gated by the hash of the kernel's sources like the
 # traffic figures.  Reported per weight: vector and LDS instructions x 64 lanes / weights, scalar instructions / weights.
 MEASURED_INSTRUCTIONS = {
-    "down_proj_5120x17408_m1_student_t_packed": ((5734195.0, 4469166.0, 1360042.0), _ROWS, "3e8407b518bc293b"),
-    "gate_up_17408x5120_m1_student_t_packed": ((6030194.0, 4450915.0, 1414314.0), _ROWS, "3e8407b518bc293b"),
-    "attn_proj_5120x5120_m1_student_t_packed": ((3570752.0, 2281697.0, 593732.0), _ROWS, "3e8407b518bc293b"),
-    "down_proj_5120x17408_m1_level1_only_packed": ((4881551.0, 4104235.0, 1254926.0), _ROWS, "3e8407b518bc293b"),
+    "down_proj_5120x17408_m1_student_t": ((4372386.0, 2184050.0, 943884.0), _LANES, "7d30d618c9f315ad"),
+    "down_proj_5120x17408_m1_calibrated": ((6395054.0, 2807327.0, 811260.0), _LANES, "7d30d618c9f315ad"),
+    "down_proj_5120x17408_m1_five_level_calibrated": ((6395054.0, 2807327.0, 811260.0), _LANES, "7d30d618c9f315ad"),
+    "down_proj_5120x17408_m1_student_t_packed": ((5734195.0, 4469166.0, 1360042.0), _ROWS, "bb78197b94a98e49"),
+    "gate_up_17408x5120_m1_student_t_packed": ((6030194.0, 4450915.0, 1414314.0), _ROWS, "bb78197b94a98e49"),
+    "attn_proj_5120x5120_m1_student_t_packed": ((3570752.0, 2281697.0, 593732.0), _ROWS, "bb78197b94a98e49"),
+    "down_proj_5120x17408_m1_level1_only_packed": ((4881551.0, 4104235.0, 1254926.0), _ROWS, "bb78197b94a98e49"),
 }
 
 WORKLOADS = {
