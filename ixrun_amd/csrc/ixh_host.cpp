@@ -31,11 +31,13 @@ struct Forward {
     const uint16_t *bias;
     int64_t in_f, out_f;
     long device;
+    long any_rows;  // more rows than these: plain calls only (no gradient, transform or other result type is asked for)
     size_t workspace_bytes[kMaxRows + 1];
     PyObject *owner;       // keeps `lanes` and what it points at alive
     PyObject *workspaces;  // dict: device -> scratch tensor
     PyObject *device_key;
     PyObject *check;       // raises for a negative code
+    PyObject *plain;       // whether a call with these activations is a plain one
 };
 
 // A token of a layer of 2.4 M weights: 5 us of host time a call (8 us from Python).
@@ -50,6 +52,13 @@ PyObject *forward_call(PyObject *self_, PyObject *const *args, size_t nargsf, Py
         Py_RETURN_NONE;
     const int64_t rows = x.numel() / self->in_f;
     if (rows < 1 || rows > kMaxRows) Py_RETURN_NONE;
+    if (rows > self->any_rows) {
+        PyObject *r = PyObject_CallOneArg(self->plain, args[0]);
+        const int yes = r ? PyObject_IsTrue(r) : -1;
+        Py_XDECREF(r);
+        if (yes < 0) return nullptr;
+        if (!yes) Py_RETURN_NONE;
+    }
     const size_t need = self->workspace_bytes[rows];
     void *scratch = nullptr;
     if (need) {
@@ -83,15 +92,16 @@ PyObject *forward_call(PyObject *self_, PyObject *const *args, size_t nargsf, Py
     END_HANDLE_TH_ERRORS
 }
 
-// Forward(gemv, lanes, bias, in_f, out_f, device, workspace_bytes, owner, workspaces, device_key, check); addresses as ints
+// Forward(gemv, lanes, bias, in_f, out_f, device, workspace_bytes, owner, workspaces, device_key, check, plain); addresses as
+// ints.  any_rows is 0 until it is set.
 int forward_init(PyObject *self_, PyObject *args, PyObject *) {
     Forward *self = reinterpret_cast<Forward *>(self_);
     unsigned long long gemv, lanes, bias;
     long long in_f, out_f;
     long device;
-    PyObject *bytes, *owner, *workspaces, *key, *check;
-    if (!PyArg_ParseTuple(args, "KKKLLlO!OO!OO", &gemv, &lanes, &bias, &in_f, &out_f, &device, &PyTuple_Type, &bytes, &owner,
-                          &PyDict_Type, &workspaces, &key, &check))
+    PyObject *bytes, *owner, *workspaces, *key, *check, *plain;
+    if (!PyArg_ParseTuple(args, "KKKLLlO!OO!OOO", &gemv, &lanes, &bias, &in_f, &out_f, &device, &PyTuple_Type, &bytes, &owner,
+                          &PyDict_Type, &workspaces, &key, &check, &plain))
         return -1;
     if (!gemv || !lanes || in_f < 1 || out_f < 1 || PyTuple_GET_SIZE(bytes) != kMaxRows + 1) {
         PyErr_SetString(PyExc_ValueError, "Forward: malformed arguments");
@@ -108,9 +118,9 @@ int forward_init(PyObject *self_, PyObject *args, PyObject *) {
     self->in_f = in_f;
     self->out_f = out_f;
     self->device = device;
-    PyObject **slots[] = {&self->owner, &self->workspaces, &self->device_key, &self->check};
-    PyObject *values[] = {owner, workspaces, key, check};
-    for (int i = 0; i < 4; ++i) {
+    PyObject **slots[] = {&self->owner, &self->workspaces, &self->device_key, &self->check, &self->plain};
+    PyObject *values[] = {owner, workspaces, key, check, plain};
+    for (int i = 0; i < 5; ++i) {
         Py_INCREF(values[i]);
         Py_XSETREF(*slots[i], values[i]);
     }
@@ -135,6 +145,7 @@ int forward_traverse(PyObject *self_, visitproc visit, void *arg) {
     Py_VISIT(self->workspaces);
     Py_VISIT(self->device_key);
     Py_VISIT(self->check);
+    Py_VISIT(self->plain);
     return 0;
 }
 
@@ -145,6 +156,7 @@ int forward_clear(PyObject *self_) {
     Py_CLEAR(self->workspaces);
     Py_CLEAR(self->device_key);
     Py_CLEAR(self->check);
+    Py_CLEAR(self->plain);
     return 0;
 }
 
@@ -416,6 +428,11 @@ PyMethodDef methods[] = {
     {nullptr, nullptr, 0, nullptr},
 };
 
+PyMemberDef forward_members[] = {
+    {"any_rows", T_LONG, offsetof(Forward, any_rows), 0, "Rows up to which calls that are not plain are taken too."},
+    {nullptr, 0, 0, 0, nullptr},
+};
+
 PyTypeObject forward_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Host side of the short calls.", -1, methods};
@@ -428,6 +445,7 @@ PyMODINIT_FUNC PyInit__host() {
     forward_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC | Py_TPFLAGS_HAVE_VECTORCALL;
     forward_type.tp_vectorcall_offset = offsetof(Forward, call);
     forward_type.tp_call = PyVectorcall_Call;
+    forward_type.tp_members = forward_members;
     forward_type.tp_new = forward_new;
     forward_type.tp_init = forward_init;
     forward_type.tp_traverse = forward_traverse;

@@ -232,7 +232,6 @@ class StreamingLinear(nn.Module):
             if bias is not None and bias.dtype is torch.bfloat16 and bias.is_cuda and bias.is_contiguous():
                 self._bias_ptr = bias.data_ptr()  # added by the kernel
         self._gemv_fn = _lib.lib().ixh_lanes_gemv if self._lanes is not None else _lib.lib().ixh_gemv
-        self._forget_plans()
         # the forward of up to MAX_FUSED_ROWS rows from the lanes, in native code
         self._native = self._native_fn = None
         if self._lanes is not None and (self._bias is None or self._bias_ptr):
@@ -242,7 +241,8 @@ class StreamingLinear(nn.Module):
                 ctypes.cast(self._gemv_fn, ctypes.c_void_p).value, ctypes.addressof(self._lanes.struct), self._bias_ptr or 0,
                 self.in_features, self.out_features, dev.index,
                 (0,) + tuple(self._lanes.gemv_workspace_bytes(n) for n in range(1, MAX_FUSED_ROWS + 1)),
-                (self._lanes, self._bias), _workspaces, dev, _lib.check)
+                (self._lanes, self._bias), _workspaces, dev, _lib.check, _plain_call)
+        self._forget_plans()
 
     def _apply(self, fn, recurse=True):
         # .to()/.cuda() may move the buffers: point the kernel arguments at the new storage
@@ -286,8 +286,8 @@ class StreamingLinear(nn.Module):
 
     def _forget_plans(self):
         self._plans = {}
-        # activations (elements) up to which a forward from the lanes takes calls that are not plain too: see _fused_plan
-        self._any_call = self._packed_rows() * self.in_features
+        if self._native is not None:  # rows up to which calls that are not plain go to the lanes too: see _fused_plan
+            self._native.any_rows = self._packed_rows()
 
     def _decode_table(self):
         """The rank table and unit of a decode of the whole weight."""
@@ -332,8 +332,7 @@ class StreamingLinear(nn.Module):
         return plan
 
     def forward(self, x):
-        if (self._native is not None and self._use_fused and not self._gemv_flags and self._gemv_fn is self._native_fn
-                and (x.numel() <= self._any_call or (x.numel() <= MAX_FUSED_ROWS * self.in_features and _plain_call(x)))):
+        if self._native is not None and self._use_fused and not self._gemv_flags and self._gemv_fn is self._native_fn:
             y = self._native(x)
             if y is not None:
                 return y
