@@ -253,13 +253,19 @@ class StreamingLinear(nn.Module):
                 self._follow_streams()
         return out
 
-    def _load_from_state_dict(self, *args, **kwargs):
-        super()._load_from_state_dict(*args, **kwargs)
-        if self._scale.is_cuda:  # the packed streams may be others now (with assign=True, in other places)
+    def _load_from_state_dict(self, state_dict, prefix, local_metadata, strict, missing_keys, unexpected_keys, error_msgs):
+        n_errors = len(error_msgs)
+        super()._load_from_state_dict(state_dict, prefix, local_metadata, strict, missing_keys, unexpected_keys, error_msgs)
+        if self._scale.is_cuda:  # (with assign=True the tensors are others)
             self._bind()
-            self._follow_streams()
-        else:  # when the layer is back on the GPU
-            self._stale = True
+        # What is derived follows a whole new set of streams only: a state of other lengths (which load_state_dict goes on to
+        # raise for) or a part of one leaves streams and tables that do not belong together, and no kernel may read those.
+        names = ["_table"] + [f"_b{i + 1}" for i in range(len(self.level_bits) - 1)] + [f"_l{i + 1}" for i in range(len(self.level_bits))]
+        if len(error_msgs) == n_errors and all(prefix + name in state_dict for name in names):
+            if self._scale.is_cuda:
+                self._follow_streams()
+            else:  # when the layer is back on the GPU
+                self._stale = True
 
     def _follow_streams(self):
         """Bring what is derived from the packed streams and is no part of the state dict in line with them."""

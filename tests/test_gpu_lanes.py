@@ -189,7 +189,7 @@ def test_prompts_of_a_layer_take_the_lanes_in_every_form(oracle, dev):
 
 
 @pytest.mark.parametrize("kind,out_f,in_f", [(k, 67, 1000) for k in ("narrow", "rare", "four", "real", "full_row", "wide")] +
-                         [("real", 9, 511), ("rare", 6, 32000), ("real", 6, 33800)])
+                         [("real", 9, 511), ("rare", 6, 32000), ("real", 6, 32768), ("real", 6, 33800)])
 def test_infinite_activations(oracle, dev, kind, out_f, in_f):
     """An infinite activation gives an infinity of the right sign, or NaN where a row's own weight is zero or another
     infinity meets it: where the list's padding points (column 0), in columns with listed elements and in others."""
@@ -331,6 +331,29 @@ def test_layer_rebuilds_its_lanes_with_its_state(dev):
     assert not torch.equal(layers[0](x), layers[1](x))
     layers[0].load_state_dict(layers[1].state_dict())
     assert torch.equal(layers[0](x), layers[1](x))
+
+
+def test_state_that_does_not_fit_is_not_followed(monkeypatch, dev):
+    """A state of other stream lengths raises, one that holds a part of the streams is loaded: neither has its tables and
+    streams decoded together.  The layer goes on with the layout it has, and takes a whole state afterwards."""
+    from ixrun_amd.engine import StreamingLinear
+
+    p = [packed_from_int8(int8_mix(kind, 64 * 1000, seed=seed), 64, 1000)
+         for kind, seed in (("only_l1", 1), ("no_l3", 2), ("only_l1", 3))]
+    layer, longer, other = (StreamingLinear(q) for q in p)
+    x = activations(3, 1000, seed=9).to(dev)
+    want = layer(x)
+    followed = []
+    real = StreamingLinear._follow_streams
+    monkeypatch.setattr(StreamingLinear, "_follow_streams", lambda self: (followed.append(self), real(self)))
+    with pytest.raises(RuntimeError, match="size mismatch"):
+        layer.load_state_dict(longer.state_dict())
+    state = {k: t.clone() for k, t in other.state_dict().items()}
+    layer.load_state_dict({k: state[k] for k in ("_b1", "_scale")}, strict=False)
+    layer.load_state_dict({}, strict=False)
+    assert not followed and torch.equal(layer(x), want)
+    layer.load_state_dict(state)
+    assert followed == [layer] and torch.equal(layer(x), other(x))
 
 
 @pytest.mark.parametrize("in_f", [1024, 1000])
