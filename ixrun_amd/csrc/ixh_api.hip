@@ -548,8 +548,8 @@ static int to_lanes(const IxhLanes *p, LanesDev *out, bool whole) {
         set_error("lanes: the plane needs %lld words, 16-byte aligned", (long long)words);
         return IXH_EINVAL;
     }
-    if (!p->scale || (whole && !p->exc_off) || (whole && (!p->exc_pos || !p->exc_val || p->n_quads < 64 || p->n_quads >= (1ull << 30)))) {
-        set_error("lanes: scale, exc_off or the list is NULL, or the list holds fewer than 64 quads or 2^30 of them");
+    if (!p->scale || (whole && !p->exc_off) || (whole && (!p->exc_pos || !p->exc_val || p->n_quads < 64 || p->n_quads % 64 || p->n_quads >= (1ull << 30)))) {
+        set_error("lanes: scale, exc_off or the list is NULL, or the list holds no whole groups of 64 quads, or 2^30 quads");
         return IXH_EINVAL;
     }
     *out = LanesDev{p->plane, p->exc_off, p->exc_pos, p->exc_val, p->scale, (uint32_t)p->out_f, (uint32_t)p->in_f,

@@ -194,3 +194,20 @@ def test_bench_tables_are_well_formed():
         assert name.removesuffix("_unfused").removesuffix("_packed") in bench.WORKLOADS, name
         for f in files:
             assert os.path.exists(os.path.join(root, "ixrun_amd", "csrc", f)), (name, f)
+
+
+def test_malformed_lane_layouts():
+    """Descriptors that a kernel could not read within its buffers are refused on the host: the list is whole groups of 64
+    quads, at least one."""
+    lib = _lib.lib()
+    words = lib.ixh_lanes_plane_words(8, 1024, 3)
+    assert words == 2 * 2 * 64 * 3 and lib.ixh_lanes_cells(8, 1024) == 4
+    good = lambda: _lib.IxhLanes(3, 8, 1024, 0x1000, words, 0x1000, 0x1000, 0x1000, 64, 0x1000)
+    assert lib.ixh_lanes_gemv_workspace_bytes(C.byref(good()), 16) >= 0
+    call = lambda s: lib.ixh_lanes_gemv(C.byref(s), 0x1000, 1024, None, 1, 0x1000, 8, None, 0, None)
+    for field, value, needle in (("n_quads", 0, "groups of 64"), ("n_quads", 63, "groups of 64"), ("n_quads", 65, "groups of 64"),
+                                 ("n_quads", 1 << 30, "2^30"), ("exc_pos", None, "NULL"), ("plane_words", words - 1, "plane"),
+                                 ("plane", 0x1004, "16-byte"), ("bits", 6, "no lane layout"), ("in_f", 1 << 31, "no lane layout")):
+        s = good()
+        setattr(s, field, value)
+        assert call(s) == -1 and needle in lib.ixh_last_error().decode(), (field, value, lib.ixh_last_error())

@@ -488,7 +488,7 @@ def test_malformed_lanes_are_refused(dev):
     p, lanes = lay_out("rare", 8, 512, dev)
     x, y = activations(1, 512).to(dev), torch.empty((1, 8), dtype=torch.bfloat16, device=dev)
     call = lambda s, m=1: L.ixh_lanes_gemv(C.byref(s), x.data_ptr(), 512, None, m, y.data_ptr(), 8, None, 0, None)
-    for field, value in (("bits", 6), ("plane_words", 100), ("n_quads", 0), ("exc_off", None), ("scale", None)):
+    for field, value in (("bits", 6), ("plane_words", 100), ("n_quads", 0), ("n_quads", 100), ("n_quads", 1 << 30), ("exc_off", None), ("scale", None)):
         s = _lib.IxhLanes.from_buffer_copy(lanes.struct)
         setattr(s, field, value)
         assert call(s) == -1, field
