@@ -19,11 +19,11 @@
 //             bits = 3: five pairs a dword from bit 2 on (p = 5 d + f at bit 2 + 6 f), the two low bits of the three
 //             dwords are pair 15.  bits = 5: three a dword from bit 2 on (p = 3 d + f), the two low bits of the five
 //             dwords are pair 15.  bits = 8: four bytes a dword, in element order.
-//   listed    in quads, one element of each of a cell's four rows: exc_pos[4 n + r], exc_val[4 n + r] belong to row r of
-//             quad n.  A cell has as many quads as its fullest row has listed elements (the others end in value 0 at
-//             position lane_none()), from exc_off[cell] on (one more at the end).  exc_pos: the byte offset of the
-//             element's column in activations kept in the order of lane_offset() below, from column 32768 * (column /
-//             32768) on.
+//   listed    in quads, one element of each of a cell's four rows; row r's of quad n is at lane_listed(n, r), so that a
+//             lane's four consecutive ones are of one row.  A cell has as many quads as its fullest row has listed elements
+//             (the others end in value 0 at position lane_none()), from exc_off[cell] on (one more at the end).  exc_pos:
+//             the byte offset of the element's column in activations kept in the order of lane_offset() below, from column
+//             32768 * (column / 32768) on.
 #pragma once
 #include "ixh_dev.h"
 #include "ixh_lanes_bounds.h"
@@ -40,6 +40,9 @@ __host__ __device__ inline uint32_t lane_offset(uint32_t col) {
     const uint32_t b = 2u * col;
     return b ^ ((b >> 2) & 0xC0u);
 }
+
+// Four quads are sixteen elements, four of each row in turn.
+__host__ __device__ inline uint32_t lane_listed(uint32_t quad, uint32_t row) { return (quad >> 2) * 16u + row * 4u + (quad & 3u); }
 
 // Where a quad's place without an element points: behind the row's last cell, where a kernel keeps an activation of 0 (value
 // 0 times an infinite activation is NaN).  Rows of 64 and more cells have no offset left for that: 0, and the kernel looks at
@@ -59,7 +62,7 @@ struct LanesDev {
 
 int launch_lanes_pack(const uint16_t *w, const LanesDev &L, uint32_t *plane, uint32_t *counts, hipStream_t s);
 int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_t *val, hipStream_t s);
-// 1 to 16 rows; five and more, and three or four too long for k_lanes_gemv, go on to launch_lanes_gemm
+// 1 to 16 rows; five and more, and fewer too long for k_lanes_gemv, go on to launch_lanes_gemm
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                       int64_t ldy, float *ws, hipStream_t s);
 // 5 and more rows (ixh_lanes_gemm.hip); IXH_EUNSUPPORTED for more than 16 unless lanes_gemm_aligned: x 16-byte aligned, in_f

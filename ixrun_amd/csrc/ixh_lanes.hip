@@ -13,49 +13,58 @@ template <int CTRL> __device__ __forceinline__ float ln_dpp(float v) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// k_lanes_gemv<BITS, MT>: up to MT activation rows, MT = 1, 2 or 4.
+// k_lanes_gemv<BITS, MT, WIDE>: up to MT activation rows, MT = 1, 2 or 4.
 //
-// Bound: HBM and a launch's start-up (5120 x 17408, one row, copies beyond the caches: 3 bits 14.6 us for 34.6 MB, 5 bits at
-// 55 / 40 / 5 % 18.7 us for 72 MB, some 4 us before the first product; the packed streams' kernels take 16.8 and 48.7; 5120 x
-// 5120 8.5 and 10.7 against 11.2 and 20.1).  A workgroup owns whole row quads, so each output is made in one place (no workspace, no second
-// launch).  Its cells, in memory order, are dealt to its waves in contiguous shares; a wave keeps several cells of
-// loads in flight, whose addresses depend on nothing that is loaded.  The activations are copied to LDS once per
+// Bound: a launch's start-up, HBM and the decode, which overlap in part (17408 x 5120 at 5 bits, 5 % listed, one row, 15.0 us: 10.7
+// without the decode and the list, 11.8 without the list and with all weights in the caches).  A workgroup owns whole row
+// quads, so each output is made in one place (no workspace, no second launch).  Its cells, in memory order, are dealt to its
+// waves in contiguous shares; addresses depend on nothing that is loaded.  The activations are copied to LDS once per
 // workgroup, 16-byte pieces of a 512-column cell at piece ^ (q << 2) so that the sixteen slices of a wave read from
 // different banks.  Products: v_mfma_f32_4x4x4_16b_bf16, one of its sixteen 4 x 4 blocks per slice (weight row = lane
 // % 4, activation row = lane % 4), so a weight costs no product instructions of its own.
 //
-// Listed elements lie in cell order, so those of a share are one run of quads.  They are taken 64 quads at a time, one
-// such group with every cell from the share's first on, fetched as far ahead as the cells: weight less what the plane
-// has there (its sign times the scale; the difference is exact in fp32) times gathered activation, added to the lane's sum of
-// the row. Taking the sign off costs two instructions an element, 17408 x 5120 at 5 % listed 17.3 us against 17.0; a plane
-// without it turns an infinite activation in a listed column into NaN.
+// A wave has two cells in flight, one of them before the activations are there, and the loop over its ten or so cells is short:
+// with four cells ahead and the loop four times as long the first requests kept the activations of the workgroup's later
+// waves waiting, nothing was multiplied for some 5 us, and much of what a launch fetches was instructions (us at 4 / 2 ahead,
+// one row: 17408 x 5120 5 bits 18.5 / 15.8, 4096 x 11008 13.0 / 10.2, 5120 x 5120 9.3 / 8.1, 5120 x 17408 3 bits 13.6 / 12.6;
+// one ahead 15.8, 10.1, 7.8, 12.5, but five layers from a graph 79 against 77).
+//
+// Listed elements lie in cell order, so those of a share are one run of quads.  They are taken 64 quads at a time, between the
+// cells so that the one's latencies run under the other's instructions (all behind the cells 17.2 us instead of 16.2): weight
+// less what the plane has there (its sign times the scale; the difference is exact in fp32) times gathered activation, added to
+// the lane's sum of its row. Taking the sign off costs two instructions an element; a plane without it turns an infinite
+// activation in a listed column into NaN.
 // ---------------------------------------------------------------------------------------------------------------
-constexpr uint32_t kLnAhead = 4;
-constexpr uint32_t kLnXAhead = 3;  // 16-byte pieces of the activations a thread asks for before anything else
-constexpr uint32_t kLnXPad = 256;  // bytes behind a row of activations in LDS: zeros (whole turns of the banks)
+constexpr uint32_t kLnAhead = 2;      // cells in flight
+constexpr uint32_t kLnFirst = 1;      // of these, asked for before the activations are there
+constexpr uint32_t kLnListAhead = 2;  // groups of the list in flight
+constexpr uint32_t kLnXAhead = 3;     // 16-byte pieces of the activations a thread asks for before anything else
+constexpr uint32_t kLnXPad = 256;     // bytes behind a row of activations in LDS: zeros (whole turns of the banks)
 
-template <int BITS, int MT>
+template <int BITS, int MT, bool WIDE>
 __global__ void __launch_bounds__(1024)
 k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
-             const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t all_tiles, uint32_t tiles_per_wg, uint32_t in_f,
-             const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, int m, int64_t ldx,
-             const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, uint32_t out_f, bool x_aligned,
-             uint32_t list_groups) {
+             const uint16_t *__restrict__ scale_at, uint32_t shape, uint32_t all_tiles, uint32_t tiles_per_wg, uint32_t in_f,
+             uint32_t inv_cells, uint32_t list_groups, const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val,
+             int64_t ldx, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, uint32_t out_f) {
     extern __shared__ __attribute__((aligned(16))) uint8_t ln_smem[];
     const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)ln_smem;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, n_threads = blockDim.x, n_waves = n_threads >> 6;
+    // (what the first requests need lies in the arguments that the hardware loads into registers)
+    const uint32_t C = shape & 0xFFFFFu, log_waves = (shape >> 20) & 7u, m = 1u + (shape >> 24);
+    const bool x_aligned = (shape >> 23) & 1u;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, n_waves = 1u << log_waves, n_threads = kWave << log_waves;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const uint32_t t0 = blockIdx.x * tiles_per_wg, C = n_cells;
+    const uint32_t t0 = blockIdx.x * tiles_per_wg;
     const uint32_t n_tiles = min(tiles_per_wg, all_tiles - t0);
     const uint32_t n_seq = n_tiles * C, cell0 = t0 * C;
-    const uint32_t s0 = wave * n_seq / n_waves, s1 = (wave + 1) * n_seq / n_waves;
-    const uint32_t x_at = smem + LnPairs<BITS>::kLutBytes, x_row = C * 1024u + kLnXPad, x_pieces = MT * C * 64u;
-    float *const parts = reinterpret_cast<float *>(ln_smem + LnPairs<BITS>::kLutBytes + MT * x_row);
+    const uint32_t s0 = (wave * n_seq) >> log_waves, s1 = ((wave + 1u) * n_seq) >> log_waves;
+    const uint32_t x_at = smem + LnPairs<BITS, WIDE>::kLutBytes, x_row = C * 1024u + kLnXPad, x_pieces = MT * C * 64u;
+    float *const parts = reinterpret_cast<float *>(ln_smem + LnPairs<BITS, WIDE>::kLutBytes + MT * x_row);
 
     auto x_piece = [&](uint32_t e) {
         const uint32_t r = MT == 1 ? 0u : e / (C * 64u), col = (e - r * (C * 64u)) * 8u;
         ln_u32x4 v = {0u, 0u, 0u, 0u};
-        if (r < (uint32_t)m && col < in_f) {
+        if (r < m && col < in_f) {
             const uint16_t *src = x + (int64_t)r * ldx + col;
             if (x_aligned && col + 8u <= in_f) {
                 v = *reinterpret_cast<const ln_u32x4 *>(src);
@@ -74,37 +83,60 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + r * x_row + lane_offset(piece * 8u))) = v;
     };
 
-    // ---- everything that depends on nothing is asked for: activations, the first cells, the list's extent ----
-    // (Requests are never inside a branch: past the end they repeat the last cell, group or piece.  The compiler counts
-    // requests in flight, and one that may or may not have been made turns its counted waits into waits for all.)
+    // ---- everything that depends on nothing is asked for: scale, activations, the first cells, the list's extent ----
+    // (Past the end requests repeat the last cell, group or piece.  The compiler counts requests in flight, and one that may or
+    // may not have been made turns its counted waits into waits for all that is older.)
+    const uint32_t scale_raw = *scale_at;
     ln_u32x4 xv[kLnXAhead];
+    if (x_aligned)
 #pragma unroll
-    for (uint32_t p = 0; p < kLnXAhead; ++p) {
-        const uint32_t e = min(tid + p * n_threads, x_pieces - 1u), r = MT == 1 ? 0u : min(e / (C * 64u), (uint32_t)m - 1u);
-        // whole pieces of an aligned row only; the others are read below
-        const uint32_t col = x_aligned ? ln_piece_column((e - e / (C * 64u) * (C * 64u)) * 8u, in_f) : 0u;
-        xv[p] = x_aligned ? *reinterpret_cast<const ln_u32x4 *>(x + (int64_t)r * ldx + col) : ln_u32x4{0, 0, 0, 0};
-    }
+        for (uint32_t p = 0; p < kLnXAhead; ++p) {
+            if (p * n_threads >= x_pieces) break;
+            const uint32_t e = min(tid + p * n_threads, x_pieces - 1u), row = MT == 1 ? 0u : e / (C * 64u);
+            // whole pieces of a row only; the others are read below
+            const uint32_t at = MT == 1 ? 0u : min(row, m - 1u) * (uint32_t)ldx;
+            xv[p] = *reinterpret_cast<const ln_u32x4 *>(x + (at + ln_piece_column((e - row * (C * 64u)) * 8u, in_f)));
+        }
     uint32_t buf[kLnAhead][BITS];
     const uint32_t cell_last = max(cell0 + s1, cell0 + 1u) - 1u;
 #pragma unroll
-    for (uint32_t p = 0; p < kLnAhead; ++p) ln_load<BITS>(plane, min(cell0 + s0 + p, cell_last), lane, buf[p]);
-    // the list's cursor: its range is the listed elements of one row quad within one segment of exc_pos
-    uint32_t l_tile = s0 / C, l_cell = s0 % C;
-    auto l_extent = [&](uint32_t at) { return min(min(s1 - at, C - l_cell), kLnSegCells - l_cell % kLnSegCells); };
-    uint32_t l_seq = s0, l_cells = l_extent(s0);
-    uint32_t r0 = exc_off[cell0 + s0], r1 = exc_off[cell0 + s0 + l_cells];
+    for (uint32_t p = 0; p < kLnFirst; ++p) ln_load<BITS>(plane, min(cell0 + s0 + p, cell_last), lane, buf[p]);
+    // the list's cursor: its range is the listed elements r0 .. r1 - 1 of one row quad within one segment of exc_pos; the end of
+    // the range after it, r2, is asked for a range ahead
+    struct Range { uint32_t seq, cell, cells; };
+    auto l_extent = [&](uint32_t seq, uint32_t cell) {
+        return Range{seq, cell, (uint32_t)min(min(s1 - seq, C - cell), kLnSegCells - cell % kLnSegCells)};
+    };
+    auto l_after = [&](const Range &r) { return l_extent(r.seq + r.cells, r.cell + r.cells == C ? 0u : r.cell + r.cells); };
+    uint32_t l_tile = C == 1 ? s0 : __umulhi(s0, inv_cells);
+    Range l_now = l_extent(s0, s0 - l_tile * C), l_next = l_after(l_now);
+    uint32_t r0 = exc_off[cell0 + s0], r1 = exc_off[cell0 + l_next.seq], r2 = exc_off[cell0 + l_next.seq + l_next.cells];
     const uint32_t e_end = exc_off[cell0 + s1];  // behind the share's last listed element
 
-    // ---- pair table, activations and zeroed sums to LDS ----
-    const float scale = bf16_bits_to_f32(*scale_at);
-    ln_build_lut<BITS, true>(smem, scale, tid, n_threads);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- pair table, zeroed sums and activations to LDS ----
+    const float scale = bf16_bits_to_f32(scale_raw);
+    ln_build_lut<BITS, WIDE>(smem, scale, tid, n_threads);
     for (uint32_t e = tid; e < n_tiles * n_waves * (MT * 8u); e += n_threads) parts[e] = 0.0f;
-    for (uint32_t e = tid; e < MT * (kLnXPad / 16u); e += n_threads)
-        *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + e / (kLnXPad / 16u) * x_row + C * 1024u + e % (kLnXPad / 16u) * 16u)) =
+    if (tid < MT * (kLnXPad / 16u))
+        *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + tid / (kLnXPad / 16u) * x_row + C * 1024u + tid % (kLnXPad / 16u) * 16u)) =
             ln_u32x4{0, 0, 0, 0};
-    // the list's groups, one per cell from the share's first cell on
-    struct Group { ln_u32x2 pos; uint32_t val; } list[kLnAhead];
+#pragma unroll
+    for (uint32_t p = 0; p < kLnXAhead; ++p) {
+        const uint32_t e = tid + p * n_threads, r = MT == 1 ? 0u : e / (C * 64u), col = (e - r * (C * 64u)) * 8u;
+        if (e < x_pieces && x_aligned && r < m && col + 8u <= in_f) x_store(e, xv[p]);
+    }
+    if (x_pieces > kLnXAhead * n_threads || !x_aligned || m < MT || in_f % kLnCols != 0)
+        for (uint32_t e = tid; e < x_pieces; e += n_threads) {  // what is not stored yet
+            const uint32_t r = MT == 1 ? 0u : e / (C * 64u), col = (e - r * (C * 64u)) * 8u;
+            if (e >= kLnXAhead * n_threads || !x_aligned || r >= m || col + 8u > in_f) x_store(e, x_piece(e));
+        }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (uint32_t p = kLnFirst; p < kLnAhead; ++p) ln_load<BITS>(plane, min(cell0 + s0 + p, cell_last), lane, buf[p]);
+    // the list's groups, 64 quads each
+    struct Group { ln_u32x2 pos; uint32_t val; } list[kLnListAhead];
     const LnGroups groups = ln_groups(r0, e_end, list_groups);
     const uint32_t g_first = groups.first, n_groups = groups.n;
     auto g_load = [&](uint32_t i) {
@@ -113,19 +145,10 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
                      *reinterpret_cast<const uint32_t *>(exc_val + (size_t)g * 256u + lane * 4u)};
     };
 #pragma unroll
-    for (uint32_t p = 0; p < kLnAhead; ++p) list[p] = g_load(p);
-#pragma unroll
-    for (uint32_t p = 0; p < kLnXAhead; ++p) {
-        const uint32_t e = tid + p * n_threads, r = MT == 1 ? 0u : e / (C * 64u), col = (e - r * (C * 64u)) * 8u;
-        if (e < x_pieces && x_aligned && r < (uint32_t)m && col + 8u <= in_f) x_store(e, xv[p]);
-    }
-    for (uint32_t e = tid; e < x_pieces; e += n_threads) {  // what is not stored yet
-        const uint32_t r = MT == 1 ? 0u : e / (C * 64u), col = (e - r * (C * 64u)) * 8u;
-        if (e >= kLnXAhead * n_threads || !x_aligned || r >= (uint32_t)m || col + 8u > in_f) x_store(e, x_piece(e));
-    }
-    __syncthreads();
+    for (uint32_t p = 0; p < kLnListAhead; ++p) list[p] = g_load(p);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-    const uint32_t lut_lane = smem + ((lane & ((1u << LnPairs<BITS>::kCopies) - 1u)) << 2);
+    const uint32_t lut_lane = smem + ((lane & ((1u << LnPairs<BITS, WIDE>::kCopies) - 1u)) << 2);
     const uint32_t q = lane >> 4, kg = (lane >> 2) & 3u, am = min(lane & 3u, (uint32_t)MT - 1u);
     uint32_t xa[4];
 #pragma unroll
@@ -133,36 +156,32 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 
     ln_f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
 
-    float ex[MT][4];
+    float ex[MT];  // of the lane's row
 #pragma unroll
-    for (int r = 0; r < MT; ++r)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) ex[r][k] = 0.0f;
+    for (int r = 0; r < MT; ++r) ex[r] = 0.0f;
     // sums over the lanes of a row's products, to `parts`: lane l has row l % 4
     auto put = [&](uint32_t tile, uint32_t half, int r, float v) {
         v += ln_dpp<0x124>(v);
         v += ln_dpp<0x128>(v);
-        v += __shfl_xor(v, 16);
-        v += __shfl_xor(v, 32);
+        const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+        const auto g = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(g[0]) + __uint_as_float(g[1]);
         if (lane < 4) parts[((tile * n_waves + wave) * 2u + half) * (MT * 4u) + (uint32_t)r * 4u + lane] = v;
     };
-    const uint32_t none = lane_none(C) * 0x10001u, scale_bits = __float_as_uint(scale) & 0x7FFFFFFFu;
-    // one group of listed elements, range by range
+    const uint32_t scale_bits = __float_as_uint(scale) & 0x7FFFFFFFu, x_none = x_at + C * 1024u;
+    // one group of listed elements, range by range: the lane has four of its row, quads quad .. quad + 3
     auto list_group = [&](const Group &in, uint32_t i) {
-        const uint32_t g0 = (g_first + i) << 6, quad = g0 + lane;
+        const uint32_t g0 = (g_first + i) << 6, quad = g0 + (lane & ~3u);
         for (;;) {
-            uint32_t vals = in.val, p01 = in.pos[0], p23 = in.pos[1];
-            if (g0 < r0 || g0 + 64u > r1) {  // quads outside the range count as if they held no element
-                const bool in_range = quad >= r0 && quad < r1;
-                vals = in_range ? vals : 0u;
-                p01 = in_range ? p01 : none;
-                p23 = in_range ? p23 : none;
-            }
-            const uint32_t x_seg = x_at + (l_cell / kLnSegCells) * (kLnSegCells * 1024u);
-            uint32_t at[4] = {x_seg + (p01 & 0xFFFFu), x_seg + (p01 >> 16), x_seg + (p23 & 0xFFFFu), x_seg + (p23 >> 16)};
+            const uint32_t vals = in.val, x_seg = x_at + (l_now.cell / kLnSegCells) * (kLnSegCells * 1024u);
+            uint32_t at[4] = {x_seg + (in.pos[0] & 0xFFFFu), x_seg + (in.pos[0] >> 16), x_seg + (in.pos[1] & 0xFFFFu), x_seg + (in.pos[1] >> 16)};
             if (C >= kLnSegCells)
 #pragma unroll
-                for (int k = 0; k < 4; ++k) at[k] = (vals >> (8 * k)) & 255u ? at[k] : x_at + C * 1024u;
+                for (int k = 0; k < 4; ++k) at[k] = (vals >> (8 * k)) & 255u ? at[k] : x_none;
+            if (g0 < r0 || g0 + 64u > r1)  // quads outside the range count as if they held no element
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) at[k] = quad + k - r0 < r1 - r0 ? at[k] : x_none;
             const uint32_t w01 = ln_pack((float)(int)(int8_t)vals * scale, (float)(int)(int8_t)(vals >> 8) * scale);
             const uint32_t w23 = ln_pack((float)(int)(int8_t)(vals >> 16) * scale, (float)((int)vals >> 24) * scale);
 #pragma unroll
@@ -173,40 +192,63 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 #pragma unroll
                 for (int r = 0; r < MT; ++r) {
                     const uint32_t h = *reinterpret_cast<const LN_LDS(uint16_t) *>((uintptr_t)(at[k] + (uint32_t)r * x_row));
-                    ex[r][k] = __fmaf_rn(wv, __uint_as_float(h << 16), ex[r][k]);
+                    ex[r] = __fmaf_rn(wv, __uint_as_float(h << 16), ex[r]);
                 }
             }
             if (g0 + 64u < r1) break;  // the range goes on in the next group
-            l_seq += l_cells;
-            l_cell += l_cells;
-            if (l_cell == C || l_seq == s1) {  // the row quad is complete
+            if (l_next.cell == 0 || l_next.seq == s1) {  // the row quad is complete
 #pragma unroll
                 for (int r = 0; r < MT; ++r) {
-                    // every lane gets the sum of row lane % 4 over its quad of lanes
-                    float own = 0.0f;
-#pragma unroll
-                    for (uint32_t k = 0; k < 4; ++k) {
-                        float v = ex[r][k];
-                        v += ln_dpp<0xB1>(v);
-                        v += ln_dpp<0x4E>(v);
-                        own = (lane & 3u) == k ? v : own;
-                        ex[r][k] = 0.0f;
-                    }
-                    put(l_tile, 1u, r, own);
+                    put(l_tile, 1u, r, ex[r]);
+                    ex[r] = 0.0f;
                 }
-                l_cell = 0;
                 ++l_tile;
             }
-            if (l_seq == s1) break;
-            l_cells = l_extent(l_seq);
+            if (l_next.seq == s1) break;
+            l_now = l_next;
+            l_next = l_after(l_now);
             r0 = r1;
-            r1 = exc_off[cell0 + l_seq + l_cells];
+            r1 = r2;
+            r2 = exc_off[cell0 + l_next.seq + l_next.cells];
             if (r0 >= g0 + 64u) break;
         }
     };
 
-    uint32_t c = s0 % C, tile = s0 / C;
-    for (uint32_t s = s0; s < s1; s += kLnAhead) {
+    uint32_t c = l_now.cell, tile = l_tile, s = s0, g = 0;
+    auto list_next = [&] {
+        list_group(list[0], g);
+#pragma unroll
+        for (uint32_t p = 1; p < kLnListAhead; ++p) list[p - 1] = list[p];
+        list[kLnListAhead - 1] = g_load(g + kLnListAhead);
+        ++g;
+    };
+    auto cell = [&](uint32_t (&w)[BITS], bool more) {
+        uint32_t o[16];
+        ln_decode<BITS, WIDE>(w, lut_lane, scale, o);
+        if (more) ln_load<BITS>(plane, min(cell0 + s + kLnAhead, cell_last), lane, w);
+        const uint32_t x_c = c * 1024u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const ln_u32x4 a = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(xa[i] + x_c));
+            acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(ln_s16x4, ln_u32x2{a[0], a[1]}),
+                                                         __builtin_bit_cast(ln_s16x4, ln_u32x2{o[4 * i], o[4 * i + 1]}), acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(ln_s16x4, ln_u32x2{a[2], a[3]}),
+                                                         __builtin_bit_cast(ln_s16x4, ln_u32x2{o[4 * i + 2], o[4 * i + 3]}), acc1, 0, 0, 0);
+        }
+        ++c;
+        ++s;
+        if (c == C || s == s1) {
+#pragma unroll
+            for (int r = 0; r < MT; ++r) put(tile, 0u, r, acc0[r] + acc1[r]);
+            acc0 = ln_f32x4{0, 0, 0, 0};
+            acc1 = ln_f32x4{0, 0, 0, 0};
+            c = 0;
+            ++tile;
+        }
+    };
+    // Whole turns of the buffers, without a way out in between: with one the compiler takes the last request made before it
+    // for the first buffer's and waits for all that is in flight at the top of every turn.
+    while (s + kLnAhead <= s1) {
         // Left alone, the waves of a SIMD are served oldest first and the last one ends long after the first; a wave
         // that has more cells to go takes precedence.
         const uint32_t behind = (s1 - s) * 4u / (s1 - s0 + 1u);
@@ -215,39 +257,25 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         else if (behind == 1u) __builtin_amdgcn_s_setprio(1);
         else __builtin_amdgcn_s_setprio(0);
 #pragma unroll
-        for (uint32_t p = 0; p < kLnAhead; ++p) {
-            if (s + p >= s1) break;
-            uint32_t o[16];
-            ln_decode<BITS, true>(buf[p], lut_lane, scale, o);
-            ln_load<BITS>(plane, min(cell0 + s + p + kLnAhead, cell_last), lane, buf[p]);
-            const uint32_t x_c = c * 1024u;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const ln_u32x4 a = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(xa[i] + x_c));
-                acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(ln_s16x4, ln_u32x2{a[0], a[1]}),
-                                                             __builtin_bit_cast(ln_s16x4, ln_u32x2{o[4 * i], o[4 * i + 1]}), acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(ln_s16x4, ln_u32x2{a[2], a[3]}),
-                                                             __builtin_bit_cast(ln_s16x4, ln_u32x2{o[4 * i + 2], o[4 * i + 3]}), acc1, 0, 0, 0);
-            }
-            if (s + p - s0 < n_groups) list_group(list[p], s + p - s0);
-            list[p] = g_load(s + p - s0 + kLnAhead);
-            ++c;
-            if (c == C || s + p + 1 == s1) {
-#pragma unroll
-                for (int r = 0; r < MT; ++r) put(tile, 0u, r, acc0[r] + acc1[r]);
-                acc0 = ln_f32x4{0, 0, 0, 0};
-                acc1 = ln_f32x4{0, 0, 0, 0};
-                c = 0;
-                ++tile;
-            }
-        }
+        for (uint32_t p = 0; p < kLnAhead; ++p) cell(buf[p], true);
+        // as large a part of the list as of the cells
+#pragma unroll 1
+        while (g * (s1 - s0) < n_groups * (s - s0)) list_next();
     }
-    // a list of more groups than cells
-    for (uint32_t i = s1 - s0; i < n_groups; ++i) list_group(g_load(i), i);
+#pragma unroll 1
+    while (s < s1) {
+        cell(buf[0], false);
+#pragma unroll
+        for (uint32_t p = 1; p < kLnAhead; ++p)
+#pragma unroll
+            for (int d = 0; d < BITS; ++d) buf[p - 1][d] = buf[p][d];
+    }
+#pragma unroll 1
+    while (g < n_groups) list_next();
     __syncthreads();
 
     // ---- outputs: the waves' parts in wave order ----
-    for (uint32_t e = tid; e < n_tiles * 4u * (uint32_t)m; e += n_threads) {
+    for (uint32_t e = tid; e < n_tiles * 4u * m; e += n_threads) {
         const uint32_t r = e / (n_tiles * 4u), row = e - r * (n_tiles * 4u), at = t0 * 4u + row;
         if (at >= out_f) continue;
         float sum = 0.0f;
@@ -374,8 +402,8 @@ k_lanes_list(const uint16_t *__restrict__ w, LanesDev L, uint16_t *__restrict__ 
 #pragma unroll
     for (uint32_t e = 0; e < 32; ++e)
         if (ln_listed<BITS>(v[e]) && at < end) {
-            pos[4u * at + (lane & 3u)] = (uint16_t)lane_offset(col0 + 32u * (e >> 3) + (e & 7u));
-            val[4u * at + (lane & 3u)] = (int8_t)v[e];
+            pos[lane_listed(at, lane & 3u)] = (uint16_t)lane_offset(col0 + 32u * (e >> 3) + (e & 7u));
+            val[lane_listed(at, lane & 3u)] = (int8_t)v[e];
             ++at;
         }
 }
@@ -404,12 +432,11 @@ int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
-// (fewer rows than five where those of whole rows do not fit k_lanes_gemv go to k_lanes_gemm as well)
-template <int BITS, int MT>
+template <int BITS, int MT, bool WIDE>
 static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                              int64_t ldy, hipStream_t s) {
     // Workgroups of 16, 8 or 4 waves, one, two or four to a CU: the split whose last round of row quads is fullest.
-    const size_t fixed = LnPairs<BITS>::kLutBytes + (size_t)MT * (L.n_cells * 1024u + kLnXPad);
+    const size_t fixed = LnPairs<BITS, WIDE>::kLutBytes + (size_t)MT * (L.n_cells * 1024u + kLnXPad);
     auto lds_of = [&](uint32_t tiles, uint32_t waves) { return fixed + (size_t)tiles * waves * (MT * 32u); };
     uint32_t best_waves = 0, best_tiles = 0;
     uint64_t best_cost = ~0ull;
@@ -420,15 +447,24 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
         const uint64_t cost = (uint64_t)tiles * per_cu;  // row quads a CU works through
         if (cost < best_cost) { best_cost = cost; best_waves = waves; best_tiles = tiles; }
     }
-    if (!best_waves) return IXH_EUNSUPPORTED;
-    const uint32_t waves = min(best_waves, best_tiles * L.n_cells);
-    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemv<BITS, MT>),
+    if (!best_waves) {  // rows too long beside the larger pair table: the smaller one, or not here
+        if constexpr (WIDE && MT <= 2 && (BITS == 4 || BITS == 5)) return lanes_gemv_launch<BITS, MT, false>(L, x, m, ldx, bias, y, ldy, s);
+        return IXH_EUNSUPPORTED;
+    }
+    uint32_t log_waves = 31u - (uint32_t)__builtin_clz(best_waves);
+    while ((1u << log_waves) > best_tiles * L.n_cells) --log_waves;
+    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemv<BITS, MT, WIDE>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
-    const bool aligned = ln_whole_pieces((uintptr_t)x, L.in_f, m, ldx);
-    hipLaunchKernelGGL((k_lanes_gemv<BITS, MT>), dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave * waves),
-                       lds_of(best_tiles, waves), s, L.plane, x, L.exc_off, L.scale, L.n_cells, L.n_tiles, best_tiles, L.in_f,
-                       L.exc_pos, L.exc_val, m, ldx, bias, y, ldy, L.out_f, aligned, L.list_groups);
+    // (the kernel's offsets of 16-byte pieces are 32 bits of elements)
+    const bool aligned = ln_whole_pieces((uintptr_t)x, L.in_f, m, ldx) && (m == 1 || ldx < (1ll << 30));
+    const uint32_t shape = L.n_cells | log_waves << 20 | (uint32_t)aligned << 23 | (uint32_t)(m - 1) << 24;
+    // quotients by n_cells as products with 2^32 / n_cells, rounded up: exact below 2^32 / n_cells, and LDS holds no rows of more
+    // than 160 cells
+    const uint32_t inv_cells = L.n_cells == 1 ? 0u : (uint32_t)(((1ull << 32) + L.n_cells - 1u) / L.n_cells);
+    hipLaunchKernelGGL((k_lanes_gemv<BITS, MT, WIDE>), dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave << log_waves),
+                       lds_of(best_tiles, 1u << log_waves), s, L.plane, x, L.exc_off, L.scale, shape, L.n_tiles, best_tiles, L.in_f,
+                       inv_cells, L.list_groups, L.exc_pos, L.exc_val, ldx, bias, y, ldy, L.out_f);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
@@ -436,9 +472,9 @@ template <int BITS>
 static int lanes_gemv_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                            int64_t ldy, float *ws, hipStream_t s) {
     int rc = IXH_EUNSUPPORTED;
-    if (m == 1) rc = lanes_gemv_launch<BITS, 1>(L, x, m, ldx, bias, y, ldy, s);
-    else if (m == 2) rc = lanes_gemv_launch<BITS, 2>(L, x, m, ldx, bias, y, ldy, s);
-    else if (m <= 4) rc = lanes_gemv_launch<BITS, 4>(L, x, m, ldx, bias, y, ldy, s);
+    if (m == 1) rc = lanes_gemv_launch<BITS, 1, true>(L, x, m, ldx, bias, y, ldy, s);
+    else if (m == 2) rc = lanes_gemv_launch<BITS, 2, true>(L, x, m, ldx, bias, y, ldy, s);
+    else if (m <= 4) rc = lanes_gemv_launch<BITS, 4, true>(L, x, m, ldx, bias, y, ldy, s);
     return rc == IXH_EUNSUPPORTED ? launch_lanes_gemm(L, x, m, ldx, bias, false, y, ldy, ws, s) : rc;
 }
 

@@ -31,11 +31,12 @@ __device__ __forceinline__ uint32_t ln_pack(float lo, float hi) {
 // (measured: 2 against 4 clocks a wave instruction), so a pair costs 6 clocks of issue and one LDS read where
 // arithmetic (extract, convert, multiply, round) takes about 20.
 // ---------------------------------------------------------------------------------------------------------------
-template <int BITS, bool WIDE = true> struct LnPairs {
-    // log2: 32 copies of 64 entries never collide; 8 of 1024 leave about half of the collisions (5120 x 17408, 5 bits, one
-    // row: 21.9 us with one copy, 21.1 with eight).  k_lanes_gemm gains nothing from four (5 bits) or
-    // sixteen (4 bits) instead of two: 10240 x 5120, 100 rows, 5 bits 47.3 and 47.8 us.
-    static constexpr int kCopies = BITS == 3 ? 5 : WIDE ? (BITS == 4 ? 4 : 3) : 1;
+template <int BITS, bool WIDE> struct LnPairs {
+    // log2: 32 copies of 64 entries never collide, nor do 16 of 256 or 1024 much (a look-up 4.0 clocks of the LDS, against 6.1 with 8
+    // copies of 1024 and 6.9 with one; 2.2 without collisions).  WIDE, where LDS has the room: 17408 x 5120, 5 bits, one row
+    // 15.9 us with 8 copies and every third pair by arithmetic, 15.2 with 16.  k_lanes_gemm gains nothing from four (5 bits)
+    // or sixteen (4 bits) instead of two: 10240 x 5120, 100 rows, 5 bits 47.3 and 47.8 us.
+    static constexpr int kCopies = BITS == 3 ? 5 : WIDE ? 4 : 1;
     static constexpr uint32_t kEntries = BITS == 8 ? 0u : 1u << (2 * BITS);
     static constexpr uint32_t kLutBytes = kEntries << (kCopies + 2);
     static constexpr uint32_t kMask = ((1u << (2 * BITS)) - 1u) << (kCopies + 2);
@@ -94,9 +95,9 @@ __device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lu
             for (int d = 0; d < BITS; ++d) last |= (w[d] & 3u) << (TO + 2 * d);
             a[15] = last;
         }
-        if constexpr (BITS == 5) {
-            // The last whole pair of a dword by arithmetic, which evens out the LDS and the vector unit: the code next to
-            // the exponent of 1.0 reads as 1 + code / 32, and (1 + code / 32) * 32 scale - 47 scale is value * scale,
+        if constexpr (BITS == 5 && !WIDE) {
+            // Two copies collide: the last whole pair of a dword by arithmetic, which evens out the LDS and the vector unit: the
+            // code next to the exponent of 1.0 reads as 1 + code / 32, and (1 + code / 32) * 32 scale - 47 scale is value * scale,
             // every term exact in fp32.
             const float s32 = 32.0f * scale, off = -47.0f * scale;
 #pragma unroll
@@ -108,7 +109,7 @@ __device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lu
         }
 #pragma unroll
         for (int p = 0; p < 16; ++p)
-            if (BITS != 5 || p == 15 || p % 3 != 2)
+            if (BITS != 5 || WIDE || p == 15 || p % 3 != 2)
                 o[p] = *reinterpret_cast<const LN_LDS(uint32_t) *>((uintptr_t)(a[p] + lut_lane));
     }
 }

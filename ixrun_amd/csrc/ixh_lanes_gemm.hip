@@ -9,8 +9,9 @@ namespace ixh {
 //
 // Bound: a stage's latency (decode, list and products follow one another in a wave, and all waves meet at its end: 3 to 8
 // thousand clocks), then LDS (per 16 x 128 weights a wave reads 4 MB / NB KB of activations, writes and reads 8 KB of weights and
-// looks up 4 KB of pairs). 10240 x 5120 at 55 / 40 / 5 %, 100 rows: 44.5 us with the slices' sums, of which the products are
-// 11 and the listed elements 8 (the matrix unit is busy for 12 % of it); 74.3 for the decode to memory and the library's
+// looks up 4 KB of pairs). 10240 x 5120 at 55 / 40 / 5 %, 100 rows: 38.9 us with the slices' sums (44.2 when a lane held an
+// element of each of four rows of the list, so that a store of listed elements went to a quarter of the banks), of which the
+// products are 11 (the matrix unit is busy for 12 % of it); 74.3 for the decode to memory and the library's
 // GEMM. A wave takes 16 weight rows x 128 columns a stage: it decodes them to its own 4 KB of LDS in operand order, stores
 // the listed elements over their places and reads the operands back.  All waves of the workgroup are in the same 128
 // columns, whose activations one copy in LDS
@@ -120,8 +121,8 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         const uint8_t *const cell = reinterpret_cast<const uint8_t *>(plane) + (t * n_cells + k.c) * (256u * BITS);  // (below 2^31)
         ln_load_lane<BITS>(reinterpret_cast<const uint32_t *>(cell), 16u * q + 4u * kg + (n & 3u), w[j][q & 1u]);
     };
-    // the list of row quad kg of the block in the cell; quads first + n, + 16 and + 32 are this lane's (at 5 % listed
-    // elements the fullest of four rows has 31 in 512 columns, 48 are five standard deviations away)
+    // the list of row quad kg of the block in the cell: of its row n % 4 this lane has four of every sixteen quads, three times
+    // (at 5 % listed elements the fullest of four rows has 31 in 512 columns, 45 are four standard deviations away)
     constexpr uint32_t ROUNDS = 3;
     struct Extent { uint32_t first, end; };
     auto extent = [&](const Cell &k, uint32_t j) {
@@ -129,14 +130,15 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         const uint32_t a = exc_off[cell], b = exc_off[cell + 1u];
         return Extent{a, t < n_tiles ? b : a};
     };
+    auto mine = [&](const Extent &e) { return (e.first & ~3u) + (n & ~3u); };
     struct Quads { ln_u32x2 pos[ROUNDS]; uint32_t val[ROUNDS]; };
     auto quads = [&](const Extent &e) {
         Quads l;
 #pragma unroll
         for (uint32_t r = 0; r < ROUNDS; ++r) {
-            const uint32_t at = e.first + n + 16u * r < e.end ? e.first + n + 16u * r : 0u;
-            l.pos[r] = *reinterpret_cast<const ln_u32x2 *>(reinterpret_cast<const uint8_t *>(exc_pos) + at * 8u);
-            l.val[r] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(exc_val) + at * 4u);
+            const uint32_t quad = mine(e) + 16u * r, at = quad < e.end ? lane_listed(quad, n & 3u) : 0u;
+            l.pos[r] = *reinterpret_cast<const ln_u32x2 *>(reinterpret_cast<const uint8_t *>(exc_pos) + at * 2u);
+            l.val[r] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(exc_val) + at);
         }
         return l;
     };
@@ -175,17 +177,17 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         for (uint32_t j = 0; j < NB; ++j) {
 #pragma unroll
             for (uint32_t r = 0; r < ROUNDS; ++r) {
-                const uint32_t val = e_now[j].first + n + 16u * r < e_now[j].end ? list[j].val[r] : 0u;
+                const uint32_t quad = mine(e_now[j]) + 16u * r;
 #pragma unroll
                 for (uint32_t k = 0; k < 4; ++k) {
                     const uint32_t p = (k & 1) ? list[j].pos[r][k >> 1] >> 16 : list[j].pos[r][k >> 1];
-                    const int v = (int)(val << (24 - 8 * k)) >> 24;
+                    const int v = quad + k - e_now[j].first < e_now[j].end - e_now[j].first ? (int)(list[j].val[r] << (24 - 8 * k)) >> 24 : 0;
                     put[j][4 * r + k] = (ln_pack(0.0f, (float)v * scale) & 0xFFFF0000u) | (v != 0 ? (p & 0x300u) << 4 : 0x4000u) |
-                                        (((p & 0xF0u) << 4) + (p & 14u) + (kg << 6) + k * 16u);
+                                        (((p & 0xF0u) << 4) + (p & 14u) + (kg << 6) + (n & 3u) * 16u);
                 }
-                any[j][r] = __any(e_now[j].first + 16u * r < e_now[j].end);
+                any[j][r] = __any((e_now[j].first & ~3u) + 16u * r < e_now[j].end);
             }
-            more[j] = __any(e_now[j].first + 16u * ROUNDS < e_now[j].end);
+            more[j] = __any((e_now[j].first & ~3u) + 16u * ROUNDS < e_now[j].end);
         }
 #pragma unroll
         for (uint32_t q = 0; q < 4; ++q) {
@@ -213,15 +215,14 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
                                 *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + j * kLgTileBytes + (put[j][e] & 0xFFFu))) =
                                     (uint16_t)(put[j][e] >> 16);
                 if (more[j]) {  // rows with yet more listed elements in the cell
-                    for (uint32_t f = e_now[j].first + n + 16u * ROUNDS; f < e_now[j].end; f += 16u)
-                        for (uint32_t k = 0; k < 4; ++k) {
-                            const uint32_t p = exc_pos[(size_t)f * 4u + k];
-                            const int v = exc_val[(size_t)f * 4u + k];
-                            if (v != 0 && (p & 0x300u) == (q << 8))
-                                *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + j * kLgTileBytes + (kg << 6) + k * 16u +
-                                                                                 ((p & 0xF0u) << 4) + (p & 14u))) =
-                                    (uint16_t)(ln_pack((float)v * scale, 0.0f) & 0xFFFFu);
-                        }
+                    for (uint32_t f = (e_now[j].first & ~3u) + 16u * ROUNDS + (n >> 2); f < e_now[j].end; f += 4u) {
+                        const uint32_t p = exc_pos[lane_listed(f, n & 3u)];
+                        const int v = exc_val[lane_listed(f, n & 3u)];
+                        if (v != 0 && (p & 0x300u) == (q << 8))
+                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + j * kLgTileBytes + (kg << 6) + (n & 3u) * 16u +
+                                                                             ((p & 0xF0u) << 4) + (p & 14u))) =
+                                (uint16_t)(ln_pack((float)v * scale, 0.0f) & 0xFFFFu);
+                    }
                 }
             }
             if (q == 3) {  // the list of the next cell, over the multiply
