@@ -581,7 +581,7 @@ int ixh_lanes_list(const uint16_t *w, const IxhLanes *dst, ixh_stream_t stream) 
 size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m) {
     LanesDev d;
     if (to_lanes(lanes, &d, true) || m < 1 || m > 16) return 0;
-    return lanes_gemm_workspace_bytes(d, m);
+    return lanes_rows_workspace_bytes(d, m);
 }
 
 int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
@@ -592,7 +592,7 @@ int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
     if (m < 1 || m > 16) { set_error("m = %d not in 1..16", m); return IXH_EINVAL; }
     if (!x || !y) { set_error("x or y is NULL"); return IXH_EINVAL; }
     if (m > 1 && (ldx < (int64_t)d.in_f || ldy < (int64_t)d.out_f)) { set_error("ldx or ldy shorter than a row"); return IXH_EINVAL; }
-    const size_t need = lanes_gemm_workspace_bytes(d, m);
+    const size_t need = lanes_rows_workspace_bytes(d, m);
     if (need && (!workspace || workspace_bytes < need)) {
         set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
         return IXH_EWORKSPACE;
@@ -628,7 +628,7 @@ int ixh_lanes_gemm(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
         set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
         return IXH_EWORKSPACE;
     }
-    rc = launch_lanes_gemm(d, x, m, ldx, bias, true, y, ldy, (float *)workspace, (hipStream_t)stream);
+    rc = launch_lanes_gemm(d, x, m, ldx, bias, y, ldy, (float *)workspace, (hipStream_t)stream);
     if (rc == IXH_ELAUNCH) set_error("lanes_gemm: launch failed");
     return rc;
 }

@@ -1,5 +1,6 @@
 // The lane layout: a second form of a packed tensor in which every code has a fixed place, made once when a layer is
-// deployed and read by the products of up to four activation rows (ixh_lanes.hip) and of more (ixh_lanes_gemm.hip).
+// deployed and read by the products of up to four activation rows (ixh_lanes.hip), of up to 16 (ixh_lanes_rows.hip) and of
+// more (ixh_lanes_gemm.hip).
 //
 // The nested-bitmap streams locate a code by the number of codes before it, so a kernel that reads them spends most
 // of its time on ranks: prefix sums over bitmap words, windows at bit offsets that depend on them, a splice or a
@@ -62,14 +63,17 @@ struct LanesDev {
 
 int launch_lanes_pack(const uint16_t *w, const LanesDev &L, uint32_t *plane, uint32_t *counts, hipStream_t s);
 int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_t *val, hipStream_t s);
-// 1 to 16 rows; five and more, and fewer too long for k_lanes_gemv, go on to launch_lanes_gemm
+// 1 to 16 rows; five and more, and fewer too long for k_lanes_gemv, go on to launch_lanes_rows
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                       int64_t ldy, float *ws, hipStream_t s);
-// 5 and more rows (ixh_lanes_gemm.hip); IXH_EUNSUPPORTED for more than 16 unless lanes_gemm_aligned: x 16-byte aligned, in_f
-// and ldx multiples of 8, x within 4 GB.  once: the bias is added before the one rounding
+size_t lanes_rows_workspace_bytes(const LanesDev &L, int m);
+int launch_lanes_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
+                      float *ws, hipStream_t s);
+// 17 and more rows (ixh_lanes_gemm.hip), the bias added before the one rounding; IXH_EUNSUPPORTED unless lanes_gemm_aligned:
+// x 16-byte aligned, in_f and ldx multiples of 8, x within 4 GB
 bool lanes_gemm_aligned(const LanesDev &L, const uint16_t *x, int m, int64_t ldx);
 size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m);
-int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once, uint16_t *y,
-                      int64_t ldy, float *ws, hipStream_t s);
+int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
+                      float *ws, hipStream_t s);
 
 }  // namespace ixh

@@ -8,10 +8,6 @@ __device__ __forceinline__ void ln_load(const uint32_t *__restrict__ plane, uint
     ln_load_lane<BITS>(plane + (size_t)cell * (64u * BITS), lane, w);
 }
 
-template <int CTRL> __device__ __forceinline__ float ln_dpp(float v) {
-    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
-}
-
 // ---------------------------------------------------------------------------------------------------------------
 // k_lanes_gemv<BITS, MT, WIDE>: up to MT activation rows, MT = 1, 2 or 4.
 //
@@ -475,7 +471,7 @@ static int lanes_gemv_rows(const LanesDev &L, const uint16_t *x, int m, int64_t 
     if (m == 1) rc = lanes_gemv_launch<BITS, 1, true>(L, x, m, ldx, bias, y, ldy, s);
     else if (m == 2) rc = lanes_gemv_launch<BITS, 2, true>(L, x, m, ldx, bias, y, ldy, s);
     else if (m <= 4) rc = lanes_gemv_launch<BITS, 4, true>(L, x, m, ldx, bias, y, ldy, s);
-    return rc == IXH_EUNSUPPORTED ? launch_lanes_gemm(L, x, m, ldx, bias, false, y, ldy, ws, s) : rc;
+    return rc == IXH_EUNSUPPORTED ? launch_lanes_rows(L, x, m, ldx, bias, y, ldy, ws, s) : rc;
 }
 
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,

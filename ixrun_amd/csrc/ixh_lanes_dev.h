@@ -19,6 +19,10 @@ constexpr size_t kLnLds = 160 * 1024;
 
 #define LN_LDS(T) __attribute__((address_space(3))) T
 
+template <int CTRL> __device__ __forceinline__ float ln_dpp(float v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+
 __device__ __forceinline__ uint32_t ln_pack(float lo, float hi) {
     const ln_f32x2 v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, ln_bf16x2));

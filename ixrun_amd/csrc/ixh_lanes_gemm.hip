@@ -4,8 +4,8 @@
 namespace ixh {
 
 // ---------------------------------------------------------------------------------------------------------------
-// k_lanes_gemm<BITS, MB, NB, ALIGNED>: up to 16 * MB activation rows at a time, MB <= 8; NB blocks of 16 weight rows a wave (two from
-// MB = 4 on: an activation operand that is read serves both); activations that are no whole 16-byte pieces: MB = 1 only.
+// k_lanes_gemm<BITS, MB, NB>: up to 16 * MB activation rows at a time, MB <= 8; NB blocks of 16 weight rows a wave (two from
+// MB = 4 on: an activation operand that is read serves both).
 //
 // Bound: a stage's latency (decode, list and products follow one another in a wave, and all waves meet at its end: 3 to 8
 // thousand clocks), then LDS (per 16 x 128 weights a wave reads 4 MB / NB KB of activations, writes and reads 8 KB of weights and
@@ -21,10 +21,6 @@ namespace ixh {
 //
 // A workgroup owns a slice of the columns (whole cells) of a run of 16-row blocks, sixteen at most at a time; the slices' sums
 // meet in the workspace and launch_lanes_reduce adds them in slice order.
-//
-// 5 to 16 rows: a kernel of waves with 16 x 512 weights and columns of their own, without the barrier and with all activations of a
-// slice in LDS, took longer at every size: us of a layer in a graph at 8 rows 16.6 against 10.1 (288 x 8192, 5 bits), 20.7
-// against 16.5 (5120 x 5120), 37.2 against 35.6 (17408 x 5120), 3 bits 28.0 against 27.4 (5120 x 17408).
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kLgBlocks = 16;  // of 16 weight rows, in work at a time
 constexpr uint32_t kLgTileBytes = 4096;
@@ -32,12 +28,12 @@ constexpr uint32_t kLgMost = 8;  // blocks of 16 activation rows
 
 __device__ __forceinline__ void lg_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int BITS, int MB, int NB, bool ALIGNED>
+template <int BITS, int MB, int NB>
 __global__ void __launch_bounds__(kLgBlocks / NB *kWave)
 k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
              const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t n_tiles, uint32_t slices, uint32_t groups,
              const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, uint32_t in_f, uint32_t m_all, int64_t ldx,
-             uint32_t out_f, float *__restrict__ ws, bool ws_aligned, const uint16_t *__restrict__ bias, bool once,
+             uint32_t out_f, float *__restrict__ ws, bool ws_aligned, const uint16_t *__restrict__ bias,
              uint16_t *__restrict__ y, int64_t ldy) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lg_smem[];
     using P = LnPairs<BITS, false>;
@@ -68,16 +64,8 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 #pragma unroll
         for (uint32_t k = 0; k < XP; ++k) {
             const uint32_t e = min(tid + k * kThreads, MB * 256u - 1u), row = min(row0 + (e >> 8) * 16u + (e & 15u), m_last);
-            if constexpr (ALIGNED) {  // (the activations lie within 4 GB)
-                const uint32_t at = row * (uint32_t)ldx + min(x_col(e, g), in_f - 8u);
-                r.v[k] = *reinterpret_cast<const ln_u32x4 *>(reinterpret_cast<const uint8_t *>(x) + 2u * at);
-            } else {
-                uint32_t h[8];
-#pragma unroll
-                for (uint32_t i = 0; i < 8; ++i) h[i] = x_col(e, g) + i < in_f ? x[(int64_t)row * ldx + x_col(e, g) + i] : 0u;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) r.v[k][i] = h[2 * i] | (h[2 * i + 1] << 16);
-            }
+            const uint32_t at = row * (uint32_t)ldx + min(x_col(e, g), in_f - 8u);  // (the activations lie within 4 GB)
+            r.v[k] = *reinterpret_cast<const ln_u32x4 *>(reinterpret_cast<const uint8_t *>(x) + 2u * at);
         }
         return r;
     };
@@ -288,7 +276,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
                             for (uint32_t k = 0; k < 4; ++k) {
                                 if (at + k >= out_f) continue;
                                 uint32_t h = f32_to_bf16_bits(acc[j][b][k]);
-                                if (bias) h = f32_to_bf16_bits((once ? acc[j][b][k] : bf16_bits_to_f32(h)) + bf16_bits_to_f32(bias[at + k]));
+                                if (bias) h = f32_to_bf16_bits(acc[j][b][k] + bf16_bits_to_f32(bias[at + k]));
                                 y[(int64_t)r * ldy + at + k] = (uint16_t)h;
                             }
                         }
@@ -333,19 +321,19 @@ size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m) {
     return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * ((L.n_tiles + 3u) / 4u * 16u) * sizeof(float) : 0;
 }
 
-template <int BITS, int MB, int NB, bool ALIGNED = true>
-static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once,
+template <int BITS, int MB, int NB>
+static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias,
                        uint16_t *y, int64_t ldy, float *ws, hipStream_t s) {
     constexpr size_t lds = LnPairs<BITS, false>::kLutBytes + kLgBlocks * kLgTileBytes + 2u * MB * 4096u;
     static_assert(lds <= kLnLds, "LDS of a CU");
-    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemm<BITS, MB, NB, ALIGNED>),
+    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemm<BITS, MB, NB>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
-    hipLaunchKernelGGL((k_lanes_gemm<BITS, MB, NB, ALIGNED>), dim3(p.slices * p.groups * p.m_groups), dim3(kLgBlocks / NB * kWave), lds, s, L.plane, x,
+    hipLaunchKernelGGL((k_lanes_gemm<BITS, MB, NB>), dim3(p.slices * p.groups * p.m_groups), dim3(kLgBlocks / NB * kWave), lds, s, L.plane, x,
                        L.exc_off, L.scale, L.n_cells, L.n_tiles, p.slices, p.groups, L.exc_pos, L.exc_val, L.in_f, (uint32_t)m, ldx,
-                       L.out_f, ws, ((uintptr_t)ws & 15u) == 0, bias, once, y, ldy);
+                       L.out_f, ws, ((uintptr_t)ws & 15u) == 0, bias, y, ldy);
     if (p.slices > 1)
-        return launch_lanes_reduce(ws, p.slices, m, L.out_f, (L.n_tiles + 3u) / 4u * 16u, bias, once, y, ldy, s);
+        return launch_lanes_reduce(ws, p.slices, m, L.out_f, (L.n_tiles + 3u) / 4u * 16u, bias, true, y, ldy, s);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
@@ -354,8 +342,7 @@ bool lanes_gemm_aligned(const LanesDev &L, const uint16_t *x, int m, int64_t ldx
 }
 
 template <int BITS, class... A>
-static int gemm_rows(const LanesDev &L, const LgPlan &p, bool aligned, A... a) {
-    if (!aligned) return p.mb == 1 ? gemm_launch<BITS, 1, 1, false>(L, p, a...) : IXH_EUNSUPPORTED;
+static int gemm_rows(const LanesDev &L, const LgPlan &p, A... a) {
     switch (p.mb) {
         case 1: return gemm_launch<BITS, 1, 1>(L, p, a...);
         case 2: return gemm_launch<BITS, 2, 1>(L, p, a...);
@@ -368,16 +355,16 @@ static int gemm_rows(const LanesDev &L, const LgPlan &p, bool aligned, A... a) {
     }
 }
 
-int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once,
-                      uint16_t *y, int64_t ldy, float *ws, hipStream_t s) {
+int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
+                      float *ws, hipStream_t s) {
+    if (!lanes_gemm_aligned(L, x, m, ldx)) return IXH_EUNSUPPORTED;
     const LgPlan p = lg_plan(L, m);
-    const bool aligned = lanes_gemm_aligned(L, x, m, ldx);
     if (m == 1) ldx = L.in_f;
     switch (L.bits) {
-        case 3: return gemm_rows<3>(L, p, aligned, x, m, ldx, bias, once, y, ldy, ws, s);
-        case 4: return gemm_rows<4>(L, p, aligned, x, m, ldx, bias, once, y, ldy, ws, s);
-        case 5: return gemm_rows<5>(L, p, aligned, x, m, ldx, bias, once, y, ldy, ws, s);
-        default: return gemm_rows<8>(L, p, aligned, x, m, ldx, bias, once, y, ldy, ws, s);
+        case 3: return gemm_rows<3>(L, p, x, m, ldx, bias, y, ldy, ws, s);
+        case 4: return gemm_rows<4>(L, p, x, m, ldx, bias, y, ldy, ws, s);
+        case 5: return gemm_rows<5>(L, p, x, m, ldx, bias, y, ldy, ws, s);
+        default: return gemm_rows<8>(L, p, x, m, ldx, bias, y, ldy, ws, s);
     }
 }
 

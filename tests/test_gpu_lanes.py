@@ -111,6 +111,19 @@ def test_long_rows_and_many_rows(oracle, dev, kind, out_f, in_f):
         check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
 
 
+@pytest.mark.parametrize("kind", ["rare", "real"])
+@pytest.mark.parametrize("out_f,in_f,m", [(16 * 257 + 3, 1030, 5), (40, 5120, 8), (40, 5121, 8), (40, 10240, 7), (37, 3584, 16), (37, 3586, 9),
+                                          (20, 17407, 6), (20, 17409, 12), (3, 520, 16)])
+def test_rows_at_the_edges_of_their_slices(oracle, dev, kind, out_f, in_f, m):
+    """5 to 16 rows: as many columns as LDS holds and just more, a block more than there are workgroups, waves without a step,
+    rows that no pair of columns divides."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    x = activations(m, in_f, seed=m).to(dev)
+    y = product(lanes, x, out_f, in_f)
+    check(oracle, p, x.cpu(), y)
+    assert torch.equal(y, product(lanes, x, out_f, in_f))
+
+
 @pytest.mark.parametrize("m", [1, 4, 7])
 def test_bias_and_unaligned_activations(oracle, dev, m):
     out_f, in_f = 37, 1536
