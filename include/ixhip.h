@@ -239,8 +239,8 @@ int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
 size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m);
 
 /*
- * The same for 1 <= m <= 4096 rows, with the weights decoded on chip into matrix-core tiles once per 128 rows (meant for 17
- * and more) and the bias added before the one rounding.  Returns IXH_EUNSUPPORTED unless in_f and ldx are multiples of 8, x is
+ * The same for 1 <= m <= 4096 rows, with the weights decoded on chip into matrix-core tiles once per 128 to 512 rows (meant
+ * for 17 and more) and the bias added before the one rounding.  Returns IXH_EUNSUPPORTED unless in_f and ldx are multiples of 8, x is
  * 16-byte aligned and m * ldx below 2^31.
  */
 int ixh_lanes_gemm(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,

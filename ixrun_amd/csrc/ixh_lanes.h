@@ -1,6 +1,6 @@
 // The lane layout: a second form of a packed tensor in which every code has a fixed place, made once when a layer is
 // deployed and read by the products of up to four activation rows (ixh_lanes.hip), of up to 16 (ixh_lanes_rows.hip) and of
-// more (ixh_lanes_gemm.hip).
+// more (ixh_lanes_gemm.hip, ixh_lanes_prompt.hip).
 //
 // The nested-bitmap streams locate a code by the number of codes before it, so a kernel that reads them spends most
 // of its time on ranks: prefix sums over bitmap words, windows at bit offsets that depend on them, a splice or a
@@ -75,5 +75,10 @@ bool lanes_gemm_aligned(const LanesDev &L, const uint16_t *x, int m, int64_t ldx
 size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m);
 int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
                       float *ws, hipStream_t s);
+// of them, those of many rows and large layers (ixh_lanes_prompt.hip): x as above, ws 16-byte aligned
+bool lanes_prompt_wins(const LanesDev &L, int m);
+size_t lanes_prompt_workspace_bytes(const LanesDev &L, int m);
+int launch_lanes_prompt(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
+                        float *ws, hipStream_t s);
 
 }  // namespace ixh

@@ -204,12 +204,18 @@ class StreamingLinear(nn.Module):
         have no list and are ahead longer than those of 5, whose limits they share (64 / 100 / 160 / 256 rows: 10240 x 5120
         57 / 61 / 68 / 82 against 27 / 36 / 49 / 72, 17408 x 5120 103 / 106 / 115 / 138 against 49 / 57 / 81 / 121, 4096 x
         4096 28 / 30 / 38 / 34 against 17 / 22 / 25 / 32).  Rows of up to 256 columns are behind from some 80 rows on where no
-        host time counts (16384 x 256, 100 rows, 16 against 17 from a graph) and ahead eager (30 against 17)."""
+        host time counts (16384 x 256, 100 rows, 16 against 17 from a graph) and ahead eager (30 against 17).
+
+        Above 3 * 2**23 weights and 128 rows the call takes tiles of up to 512 rows, whose decode the products hide: at 192 /
+        256 / 384 / 512 rows 5120 x 17408 (3 bits) 85 / 94 / 118 / 126 by the best other way against 57 / 64 / 81 / 100, 10240 x
+        5120 (5 bits) 80 / 81 / 82 / 92 against 51 / 59 / 69 / 84, 5120 x 5120 53 / 63 / 54 / 58 against 36 / 39 / 46 / 56; at
+        768 rows 10240 x 5120 is behind (103 against 116) and 12288 x 6144 ahead (138 against 128; 1024 rows 154 against 155),
+        5120 x 17408 at 1024 317 against 179."""
         n = self.N
         return (self._lanes is not None and self._gemv_flags == 0 and self.in_features % 8 == 0 and n > 1 << 18
                 and rows * self.in_features < 1 << 31
                 and (rows <= 160 or (rows <= 224 and self._lanes.bits <= 4) or (rows <= 256 and n < 1 << 24)
-                     or (rows <= 512 and n <= 1 << 20)))
+                     or (rows <= 512 and (n <= 1 << 20 or n > 3 << 23)) or (rows <= 1024 and n > 1 << 26)))
 
     def _bind(self):
         n_levels = len(self.level_bits)

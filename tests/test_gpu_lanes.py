@@ -151,6 +151,28 @@ def test_many_rows(oracle, dev, kind, out_f, in_f):
         assert torch.equal(*y)  # the order of the sums is fixed
 
 
+@pytest.mark.parametrize("kind,out_f,in_f", [("rare", 24600, 1032), ("real", 8200, 3080), ("full_row", 8200, 3080), ("four", 1000, 25400),
+                                             ("wide", 400, 66000)])
+def test_many_rows_of_the_largest_weights(oracle, dev, kind, out_f, in_f):
+    """Tiles of 128 weight rows: each width of the sums and a second group of rows; a workgroup with a whole tile, with a slice of
+    one and with the end of one and the start of the next; lists longer than are held; y's rows at odd multiples of 2 bytes."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    wide = activations(513, in_f + 8, seed=3).to(dev)
+    x = wide[:, 8:]
+    weight = bits_to_bf16(oracle.decode_packed_bf16(p)).to(dev).reshape(out_f, in_f).float()
+    exact = x.float() @ weight.t()
+    for m in (129, 200, 257, 500, 513):
+        b = bias if m % 2 else None
+        want = (exact[:m] if b is None else exact[:m] + b.to(dev).float()).bfloat16()
+        y = torch.full((2, m, out_f + m % 3), 7.0, dtype=torch.bfloat16, device=dev)
+        for t in y:
+            lanes.gemm(x[:m], t[:, :out_f], None if b is None else b.to(dev))
+        # both are one rounding to bf16 of sums whose fp32 errors are far below it: they differ where a sum is next to a tie
+        assert rel_l2(y[0, :, :out_f].float().cpu().numpy(), want.float().cpu().numpy()) <= 1e-3
+        assert torch.equal(y[0], y[1]) and (y[:, :, out_f:] == 7).all()
+
+
 @pytest.mark.parametrize("out_f,in_f,m", [(4100, 520, 20), (4500, 1536, 130), (20, 33800, 40)])
 def test_many_rows_of_larger_weights(oracle, dev, out_f, in_f, m):
     """Workgroups with several rounds of blocks, and slices of several cells."""
