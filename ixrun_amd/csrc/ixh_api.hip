@@ -628,7 +628,7 @@ int ixh_lanes_gemm(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
         set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
         return IXH_EWORKSPACE;
     }
-    rc = launch_lanes_gemm(d, x, m, ldx, bias, y, ldy, (float *)workspace, (hipStream_t)stream);
+    rc = launch_lanes_gemm(d, x, m, ldx, bias, true, y, ldy, (float *)workspace, (hipStream_t)stream);
     if (rc == IXH_ELAUNCH) set_error("lanes_gemm: launch failed");
     return rc;
 }

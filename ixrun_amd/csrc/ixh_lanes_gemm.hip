@@ -33,7 +33,7 @@ __global__ void __launch_bounds__(kLgBlocks / NB *kWave)
 k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
              const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t n_tiles, uint32_t slices, uint32_t groups,
              const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, uint32_t in_f, uint32_t m_all, int64_t ldx,
-             uint32_t out_f, float *__restrict__ ws, bool ws_aligned, const uint16_t *__restrict__ bias,
+             uint32_t out_f, float *__restrict__ ws, bool ws_aligned, const uint16_t *__restrict__ bias, bool once,
              uint16_t *__restrict__ y, int64_t ldy) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lg_smem[];
     using P = LnPairs<BITS, false>;
@@ -276,7 +276,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
                             for (uint32_t k = 0; k < 4; ++k) {
                                 if (at + k >= out_f) continue;
                                 uint32_t h = f32_to_bf16_bits(acc[j][b][k]);
-                                if (bias) h = f32_to_bf16_bits(acc[j][b][k] + bf16_bits_to_f32(bias[at + k]));
+                                if (bias) h = f32_to_bf16_bits((once ? acc[j][b][k] : bf16_bits_to_f32(h)) + bf16_bits_to_f32(bias[at + k]));
                                 y[(int64_t)r * ldy + at + k] = (uint16_t)h;
                             }
                         }
@@ -323,7 +323,7 @@ size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m) {
 }
 
 template <int BITS, int MB, int NB>
-static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias,
+static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once,
                        uint16_t *y, int64_t ldy, float *ws, hipStream_t s) {
     constexpr size_t lds = LnPairs<BITS, false>::kLutBytes + kLgBlocks * kLgTileBytes + 2u * MB * 4096u;
     static_assert(lds <= kLnLds, "LDS of a CU");
@@ -332,9 +332,9 @@ static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, in
     if (!raised) return IXH_ELAUNCH;
     hipLaunchKernelGGL((k_lanes_gemm<BITS, MB, NB>), dim3(p.slices * p.groups * p.m_groups), dim3(kLgBlocks / NB * kWave), lds, s, L.plane, x,
                        L.exc_off, L.scale, L.n_cells, L.n_tiles, p.slices, p.groups, L.exc_pos, L.exc_val, L.in_f, (uint32_t)m, ldx,
-                       L.out_f, ws, ((uintptr_t)ws & 15u) == 0, bias, y, ldy);
+                       L.out_f, ws, ((uintptr_t)ws & 15u) == 0, bias, once, y, ldy);
     if (p.slices > 1)
-        return launch_lanes_reduce(ws, p.slices, m, L.out_f, (L.n_tiles + 3u) / 4u * 16u, bias, true, y, ldy, s);
+        return launch_lanes_reduce(ws, p.slices, m, L.out_f, (L.n_tiles + 3u) / 4u * 16u, bias, once, y, ldy, s);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
@@ -356,17 +356,17 @@ static int gemm_rows(const LanesDev &L, const LgPlan &p, A... a) {
     }
 }
 
-int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
-                      float *ws, hipStream_t s) {
+int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once, uint16_t *y,
+                      int64_t ldy, float *ws, hipStream_t s) {
     if (!lanes_gemm_aligned(L, x, m, ldx)) return IXH_EUNSUPPORTED;
-    if (lanes_prompt_wins(L, m) && ((uintptr_t)ws & 15u) == 0) return launch_lanes_prompt(L, x, m, ldx, bias, y, ldy, ws, s);
+    if (once && lanes_prompt_wins(L, m) && ((uintptr_t)ws & 15u) == 0) return launch_lanes_prompt(L, x, m, ldx, bias, y, ldy, ws, s);
     const LgPlan p = lg_plan(L, m);
     if (m == 1) ldx = L.in_f;
     switch (L.bits) {
-        case 3: return gemm_rows<3>(L, p, x, m, ldx, bias, y, ldy, ws, s);
-        case 4: return gemm_rows<4>(L, p, x, m, ldx, bias, y, ldy, ws, s);
-        case 5: return gemm_rows<5>(L, p, x, m, ldx, bias, y, ldy, ws, s);
-        default: return gemm_rows<8>(L, p, x, m, ldx, bias, y, ldy, ws, s);
+        case 3: return gemm_rows<3>(L, p, x, m, ldx, bias, once, y, ldy, ws, s);
+        case 4: return gemm_rows<4>(L, p, x, m, ldx, bias, once, y, ldy, ws, s);
+        case 5: return gemm_rows<5>(L, p, x, m, ldx, bias, once, y, ldy, ws, s);
+        default: return gemm_rows<8>(L, p, x, m, ldx, bias, once, y, ldy, ws, s);
     }
 }
 

@@ -335,9 +335,12 @@ k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 }
 
 // How the work is cut: slices of the columns, workgroups of a slice, waves of a workgroup. Of a few cuts the one with the shortest
-// estimate, in clocks: 4000 to the first product and 40 for 128 columns of activations a wave turns round, then whichever is
-// longer, 1400 for a step of 16 x 256 weights in a wave or 160 + 6 MT in the CU; the slices' sums cost a launch and their way
-// through memory. (Shapes from 512 x 8192 to 17408 x 5120, all cuts timed: within 4 % of the shortest.)
+// estimate, in clocks: 4000 to the first product and 400 for each wave that has to be there, 20 or 30 (up to 8 or 16 rows) for 128
+// columns of activations a wave turns round, then whichever is longer, 2500 or 2000 for a step of 16 x 256 weights in a wave or 130
+// in the CU; the slices' sums cost a launch and their way through memory.  Fitted to all cuts, timed, of 32 shapes from 256 x 4096 to
+// 17408 x 5120: within 0.3 % of the shortest in the mean, 8 % at worst.  (Without the waves' 400, and the slices dearer, layers of few
+// rows had one slice of sixteen waves where several of four fill the CUs: 960 x 3072 at 11 rows 11.0 us against 8.9, 256 x 4096
+// 11.9 against 8.7, 5120 x 17408 at 7 rows 18.0 against 16.0.)
 struct LrPlan { uint32_t slices, groups, waves, x_rows; size_t lds; };
 
 template <int BITS, int MT>
@@ -348,7 +351,7 @@ static LrPlan lr_plan(const LanesDev &L) {
     constexpr size_t kPart = 64u * MT;  // bytes of a wave's part of a block
     const uint32_t most = (uint32_t)((kLnLds - kLrXAt<BITS, MT> - 24u * kPart) / (kLnCols * 2u * MT));  // cells of a slice
     const uint32_t s_min = (L.n_cells + most - 1u) / most;
-    for (uint32_t s = s_min; s <= min(L.n_cells, s_min + 7u); ++s) {
+    for (uint32_t s = s_min; s <= min(L.n_cells, s_min + 15u); ++s) {
         // (16 rows more: the zeros that places without an element point at)
         const uint32_t cells = (L.n_cells + s - 1u) / s, x_rows = cells * kLnCols + 16u;
         for (uint32_t waves = 16; waves >= 4; waves /= 2) {
@@ -363,9 +366,9 @@ static LrPlan lr_plan(const LanesDev &L) {
             const uint32_t per_cu = min((uint32_t)(kLnLds / lds), 16u / waves), rounds = (groups * s + cus * per_cu - 1u) / (cus * per_cu);
             const uint32_t steps = nb * cells * 2u, mine = (steps + waves - 1u) / waves;
             const uint32_t resident = min(per_cu, (groups * s + cus - 1u) / cus);
-            const uint64_t run = std::max<uint64_t>((uint64_t)mine * 1400u, (uint64_t)steps * resident * (160u + 6u * MT));
-            const uint64_t sums = s > 1 ? 6000u + (uint64_t)s * L.n_tiles * 4u * MT * 8u / 3400u : 0u;
-            const uint64_t cost = rounds * (4600u + (uint64_t)cells * 64u / waves * 40u + run) + sums;
+            const uint64_t run = std::max<uint64_t>((uint64_t)mine * (MT == 8 ? 2500u : 2000u), (uint64_t)steps * resident * 130u);
+            const uint64_t sums = s > 1 ? (MT == 8 ? 4000u : 2000u) + (uint64_t)s * L.n_tiles * 4u * MT * 8u / 3400u : 0u;
+            const uint64_t cost = rounds * (4000u + 400u * waves + (uint64_t)cells * 64u / waves * (MT == 8 ? 20u : 30u) + run) + sums;
             if (cost < best_cost) { best_cost = cost; best = {s, groups, waves, x_rows, lds}; }
         }
     }
@@ -382,9 +385,21 @@ static LrPlan lr_plan_of(const LanesDev &L, int m) {
     }
 }
 
+// Nine to sixteen rows of up to 20 * 2^20 weights: turning the activations round for the whole of a long slice, or starting up for
+// a single cell, takes longer than k_lanes_gemm's way, whose sixteen waves share a copy of 128 columns a stage.  us, this / that at
+// 16 rows, 5 bits: 512 rows x 512 columns 6.6 / 6.0, 512 x 1024 7.2 / 8.3, 512 x 2048 8.8 / 8.3, 2048 x 4096 10.4 / 9.4, 4096 x 4096
+// 12.3 / 11.4, 4288 x 4096 (a second block for some workgroups) 13.9 / 11.9, 8192 x 4096 14.7 / 15.6.  Three bits, whose pairs sit in LDS 32 times over here: 4096 x 2048 8.7 / 10.6, 2048 x 4096
+// 10.1 / 10.7, 4096 x 4096 11.5 / 10.5, 2048 x 8192 11.6 / 10.9, 4096 x 8192 13.8 / 14.5.
+static bool lr_gemm_wins(const LanesDev &L, int m) {
+    const uint64_t n = (uint64_t)L.out_f * L.in_f;
+    if (m <= 8 || n > 20u << 20) return false;
+    return L.bits == 3 ? n > 10u << 20 && L.in_f > 2560u : L.in_f <= kLnCols || L.in_f >= 2048u;
+}
+
 size_t lanes_rows_workspace_bytes(const LanesDev &L, int m) {
     const LrPlan p = lr_plan_of(L, m);
-    return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * L.n_tiles * 4u * sizeof(float) : 0;
+    const size_t sums = p.slices > 1 ? (size_t)p.slices * (uint32_t)m * L.n_tiles * 4u * sizeof(float) : 0;
+    return lr_gemm_wins(L, m) ? max(sums, lanes_gemm_workspace_bytes(L, m)) : sums;
 }
 
 template <int BITS, int MT>
@@ -406,6 +421,7 @@ static int rows_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx,
 
 int launch_lanes_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
                       float *ws, hipStream_t s) {
+    if (lr_gemm_wins(L, m) && lanes_gemm_aligned(L, x, m, ldx)) return launch_lanes_gemm(L, x, m, ldx, bias, false, y, ldy, ws, s);
 #define LR_ROWS(B) (m <= 8 ? rows_launch<B, 8>(L, x, m, ldx, bias, y, ldy, ws, s) : rows_launch<B, 16>(L, x, m, ldx, bias, y, ldy, ws, s))
     switch (L.bits) {
         case 3: return LR_ROWS(3);

@@ -118,10 +118,12 @@ def test_rows_at_the_edges_of_their_slices(oracle, dev, kind, out_f, in_f, m):
     """5 to 16 rows: as many columns as LDS holds and just more, a block more than there are workgroups, waves without a step,
     rows that no pair of columns divides."""
     p, lanes = lay_out(kind, out_f, in_f, dev)
-    x = activations(m, in_f, seed=m).to(dev)
-    y = product(lanes, x, out_f, in_f)
-    check(oracle, p, x.cpu(), y)
-    assert torch.equal(y, product(lanes, x, out_f, in_f))
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    for skip in (0, 1, 2):  # whole 16-byte pieces (nine rows and more may take another way then), pairs or neither
+        x = activations(m, in_f + 8, seed=m).to(dev)[:, skip : skip + in_f]
+        y = product(lanes, x, out_f, in_f, bias.to(dev))
+        check(oracle, p, x.cpu(), y, bias)
+        assert torch.equal(y, product(lanes, x, out_f, in_f, bias.to(dev)))
 
 
 @pytest.mark.parametrize("m", [1, 4, 7])
