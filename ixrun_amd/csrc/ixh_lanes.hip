@@ -443,10 +443,14 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
         const uint64_t cost = (uint64_t)tiles * per_cu;  // row quads a CU works through
         if (cost < best_cost) { best_cost = cost; best_waves = waves; best_tiles = tiles; }
     }
-    if (!best_waves) {  // rows too long beside the larger pair table: the smaller one, or not here
-        if constexpr (WIDE && MT <= 2 && (BITS == 4 || BITS == 5)) return lanes_gemv_launch<BITS, MT, false>(L, x, m, ldx, bias, y, ldy, s);
-        return IXH_EUNSUPPORTED;
+    // The smaller pair table where rows are too long beside the larger one, and for a few cells a CU, which gain less from it than
+    // its 64 KB take to write (5 bits, one row, larger / smaller: 512 x 512 6.6 / 4.2 us, 900 x 3072 with 6 cells a CU 5.0 / 4.4, 2000
+    // x 4096 with 16 5.7 / 5.6, 4000 x 3072 with 24 6.4 / 6.4, 5000 x 5120 with 50 7.8 / 8.1).
+    if constexpr (WIDE && (BITS == 4 || BITS == 5)) {
+        const bool few = best_waves && best_tiles * L.n_cells * (16u / best_waves) <= 16u;
+        if (few || (!best_waves && MT <= 2)) return lanes_gemv_launch<BITS, MT, false>(L, x, m, ldx, bias, y, ldy, s);
     }
+    if (!best_waves) return IXH_EUNSUPPORTED;
     uint32_t log_waves = 31u - (uint32_t)__builtin_clz(best_waves);
     while ((1u << log_waves) > best_tiles * L.n_cells) --log_waves;
     static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemv<BITS, MT, WIDE>),

@@ -6,7 +6,7 @@
 namespace ixh {
 
 // ---------------------------------------------------------------------------------------------------------------
-// k_lanes_rows<BITS, MT>: up to MT activation rows, MT = 8 or 16.
+// k_lanes_rows<BITS, MT, WIDE>: up to MT activation rows, MT = 8 or 16.
 //
 // Bound: a launch's start-up (some 5 us to the first product: the activations of a slice are turned round on the way to LDS),
 // then the decode's LDS look-ups and vector instructions; the busiest unit is busy for some 60 % of the rest. us a layer:
@@ -47,9 +47,9 @@ __device__ __forceinline__ lr_bf16x4 lr_turned(uint32_t at) {
 }
 
 // (the order of a cell's columns is worked out on the address bits of 128 rows)
-template <int BITS, int MT> constexpr uint32_t kLrXAt = (LnPairs<BITS, (MT == 8)>::kLutBytes + 4095u) & ~4095u;
+template <int BITS, bool WIDE> constexpr uint32_t kLrXAt = (LnPairs<BITS, WIDE>::kLutBytes + 4095u) & ~4095u;
 
-template <int BITS, int MT>
+template <int BITS, int MT, bool WIDE>
 __global__ void __launch_bounds__(1024)
 k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
              const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t n_tiles, uint32_t in_f, uint32_t shape,
@@ -57,7 +57,7 @@ k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
              int64_t ldx, uint32_t out_f, uint32_t x_rows, float *__restrict__ ws, const uint16_t *__restrict__ bias,
              uint16_t *__restrict__ y, int64_t ldy) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lr_smem[];
-    using P = LnPairs<BITS, (MT == 8)>;
+    using P = LnPairs<BITS, WIDE>;
     const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)lr_smem;
     const uint32_t m = shape & 31u, log_waves = (shape >> 5) & 7u;
     const bool x_pairs = (shape >> 8) & 1u;
@@ -74,8 +74,8 @@ k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     const uint32_t H = 2u * C, total = n_blocks * H;
     const uint32_t s0 = (wave * total) >> log_waves, n_steps = (((wave + 1u) * total) >> log_waves) - s0;
     constexpr uint32_t ROW = 2u * MT;
-    const uint32_t x_at = smem + kLrXAt<BITS, MT>;
-    float *const parts = reinterpret_cast<float *>(lr_smem + kLrXAt<BITS, MT> + x_rows * ROW);  // [wave + block][16][MT]
+    const uint32_t x_at = smem + kLrXAt<BITS, WIDE>;
+    float *const parts = reinterpret_cast<float *>(lr_smem + kLrXAt<BITS, WIDE> + x_rows * ROW);  // [wave + block][16][MT]
 
     const uint32_t scale_raw = *scale_at;
     // ---- asked for first: this wave's activations, its first units, the list's extent, the scale ----
@@ -172,7 +172,7 @@ k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     const float scale = bf16_bits_to_f32(scale_raw);
     __builtin_amdgcn_sched_barrier(0);
 
-    ln_build_lut<BITS, (MT == 8)>(smem, scale, tid, n_threads);
+    ln_build_lut<BITS, WIDE>(smem, scale, tid, n_threads);
     // the column that places without an element point at, and what shares its run of eight rows
     if (tid < 16u) *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + H * 256u * ROW + tid * 16u)) = ln_u32x4{0, 0, 0, 0};
     auto groups_of = [&](const Range &r) {  // of the row quad that has most
@@ -248,8 +248,8 @@ k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         else if (behind == 1u) __builtin_amdgcn_s_setprio(1);
         else __builtin_amdgcn_s_setprio(0);
         uint32_t o[2][16];
-        ln_decode<BITS, (MT == 8)>(w[0], lut_lane, scale, o[0]);
-        ln_decode<BITS, (MT == 8)>(w[1], lut_lane, scale, o[1]);
+        ln_decode<BITS, WIDE>(w[0], lut_lane, scale, o[0]);
+        ln_decode<BITS, WIDE>(w[1], lut_lane, scale, o[1]);
         load(w);
         go_on(s + 2u < n_steps);
         // (columns 128 q + 32 i of a cell lie at 128 q + 32 (i ^ q))
@@ -343,19 +343,19 @@ k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 // 11.9 against 8.7, 5120 x 17408 at 7 rows 18.0 against 16.0.)
 struct LrPlan { uint32_t slices, groups, waves, x_rows; size_t lds; };
 
-template <int BITS, int MT>
+template <int BITS, int MT, bool WIDE>
 static LrPlan lr_plan(const LanesDev &L) {
     LrPlan best{};
     uint64_t best_cost = ~0ull;
     const uint32_t cus = ln_cus(), blocks = (L.n_tiles + 3u) / 4u;
     constexpr size_t kPart = 64u * MT;  // bytes of a wave's part of a block
-    const uint32_t most = (uint32_t)((kLnLds - kLrXAt<BITS, MT> - 24u * kPart) / (kLnCols * 2u * MT));  // cells of a slice
+    const uint32_t most = (uint32_t)((kLnLds - kLrXAt<BITS, WIDE> - 24u * kPart) / (kLnCols * 2u * MT));  // cells of a slice
     const uint32_t s_min = (L.n_cells + most - 1u) / most;
     for (uint32_t s = s_min; s <= min(L.n_cells, s_min + 15u); ++s) {
         // (16 rows more: the zeros that places without an element point at)
         const uint32_t cells = (L.n_cells + s - 1u) / s, x_rows = cells * kLnCols + 16u;
         for (uint32_t waves = 16; waves >= 4; waves /= 2) {
-            const size_t fixed = kLrXAt<BITS, MT> + (size_t)x_rows * 2u * MT + waves * kPart;
+            const size_t fixed = kLrXAt<BITS, WIDE> + (size_t)x_rows * 2u * MT + waves * kPart;
             if (fixed + kPart > kLnLds) continue;
             // as many workgroups as CUs, or as it takes for the parts of a workgroup's blocks to fit
             const uint32_t fit = min((uint32_t)((kLnLds - fixed) / kPart), 255u);
@@ -375,7 +375,17 @@ static LrPlan lr_plan(const LanesDev &L) {
     return best;
 }
 
-template <int BITS> static LrPlan lr_plan_rows(const LanesDev &L, int m) { return m <= 8 ? lr_plan<BITS, 8>(L) : lr_plan<BITS, 16>(L); }
+// The larger pair table up to eight rows (LDS has the room beside their activations) and from some cells a CU on: below, what it
+// saves is less than its 64 KB take to write (5 bits, 8 rows, larger / smaller: 512 x 512 5.9 / 5.2 us, 2000 x 2048 with 8 cells a CU
+// 6.9 / 6.6, 4000 x 3072 with 24 8.9 / 8.6, 2000 x 8192 with 32 11.1 / 11.8, 5000 x 5120 with 50 12.7 / 12.8).
+template <int BITS> static bool lr_wide(const LanesDev &L, int m) {
+    return (BITS == 4 || BITS == 5) && m <= 8 && (uint64_t)L.n_tiles * L.n_cells > 24u * ln_cus();
+}
+
+template <int BITS> static LrPlan lr_plan_rows(const LanesDev &L, int m) {
+    if (lr_wide<BITS>(L, m)) return lr_plan<BITS, 8, true>(L);
+    return m <= 8 ? lr_plan<BITS, 8, false>(L) : lr_plan<BITS, 16, false>(L);
+}
 static LrPlan lr_plan_of(const LanesDev &L, int m) {
     switch (L.bits) {
         case 3: return lr_plan_rows<3>(L, m);
@@ -393,7 +403,7 @@ static LrPlan lr_plan_of(const LanesDev &L, int m) {
 static bool lr_gemm_wins(const LanesDev &L, int m) {
     const uint64_t n = (uint64_t)L.out_f * L.in_f;
     if (m <= 8 || n > 20u << 20) return false;
-    return L.bits == 3 ? n > 10u << 20 && L.in_f > 2560u : L.in_f <= kLnCols || L.in_f >= 2048u;
+    return L.bits == 3 ? n > 9u << 20 && L.in_f > 2560u : L.in_f <= kLnCols || L.in_f >= 2048u;
 }
 
 size_t lanes_rows_workspace_bytes(const LanesDev &L, int m) {
@@ -402,17 +412,17 @@ size_t lanes_rows_workspace_bytes(const LanesDev &L, int m) {
     return lr_gemm_wins(L, m) ? max(sums, lanes_gemm_workspace_bytes(L, m)) : sums;
 }
 
-template <int BITS, int MT>
+template <int BITS, int MT, bool WIDE>
 static int rows_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
                        float *ws, hipStream_t s) {
-    const LrPlan p = lr_plan<BITS, MT>(L);
-    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_rows<BITS, MT>),
+    const LrPlan p = lr_plan<BITS, MT, WIDE>(L);
+    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_rows<BITS, MT, WIDE>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
     const bool pairs = ((uintptr_t)x & 3u) == 0 && L.in_f % 2u == 0 && ldx % 2 == 0;
     const uint32_t blocks = (L.n_tiles + 3u) / 4u, log_waves = 31u - (uint32_t)__builtin_clz(p.waves);
     const uint32_t shape = (uint32_t)m | log_waves << 5 | (uint32_t)pairs << 8;
-    hipLaunchKernelGGL((k_lanes_rows<BITS, MT>), dim3(p.slices, p.groups), dim3(kWave * p.waves), p.lds, s, L.plane, x, L.exc_off,
+    hipLaunchKernelGGL((k_lanes_rows<BITS, MT, WIDE>), dim3(p.slices, p.groups), dim3(kWave * p.waves), p.lds, s, L.plane, x, L.exc_off,
                        L.scale, L.n_cells, L.n_tiles, L.in_f, shape, (L.n_cells / p.slices) << 20 | L.n_cells % p.slices,
                        (blocks / p.groups) << 24 | blocks % p.groups, L.exc_pos, L.exc_val, ldx, L.out_f, p.x_rows, ws, bias, y, ldy);
     if (p.slices > 1) return launch_lanes_reduce(ws, p.slices, m, L.out_f, L.n_tiles * 4u, bias, false, y, ldy, s);
@@ -422,7 +432,10 @@ static int rows_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx,
 int launch_lanes_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
                       float *ws, hipStream_t s) {
     if (lr_gemm_wins(L, m) && lanes_gemm_aligned(L, x, m, ldx)) return launch_lanes_gemm(L, x, m, ldx, bias, false, y, ldy, ws, s);
-#define LR_ROWS(B) (m <= 8 ? rows_launch<B, 8>(L, x, m, ldx, bias, y, ldy, ws, s) : rows_launch<B, 16>(L, x, m, ldx, bias, y, ldy, ws, s))
+#define LR_ROWS(B)                                                                                                              \
+    (lr_wide<B>(L, m) ? rows_launch<B, 8, (B == 4 || B == 5)>(L, x, m, ldx, bias, y, ldy, ws, s)                                 \
+     : m <= 8         ? rows_launch<B, 8, false>(L, x, m, ldx, bias, y, ldy, ws, s)                                              \
+                      : rows_launch<B, 16, false>(L, x, m, ldx, bias, y, ldy, ws, s))
     switch (L.bits) {
         case 3: return LR_ROWS(3);
         case 4: return LR_ROWS(4);

@@ -126,6 +126,16 @@ def test_rows_at_the_edges_of_their_slices(oracle, dev, kind, out_f, in_f, m):
         assert torch.equal(y, product(lanes, x, out_f, in_f, bias.to(dev)))
 
 
+@pytest.mark.parametrize("kind", ["four", "real"])
+@pytest.mark.parametrize("out_f,in_f", [(4131, 1500), (4131, 3080)])
+def test_both_tables_of_pairs(oracle, dev, kind, out_f, in_f):
+    """Planes of 4 and 5 bits with few and with many cells a CU: the smaller table of pairs (the other tests' too) and the larger."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    for m in (1, 2, 4, 7):
+        x = activations(m, in_f, seed=m)
+        check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
+
+
 @pytest.mark.parametrize("m", [1, 4, 7])
 def test_bias_and_unaligned_activations(oracle, dev, m):
     out_f, in_f = 37, 1536
