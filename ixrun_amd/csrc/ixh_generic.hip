@@ -125,81 +125,141 @@ int launch_prefix_build(const Dev &P, uint32_t chunk, int32_t *prefix, hipStream
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// The same table with a workspace for sums: one launch per level and one more, where counting a level and scanning it in
-// two or four launches each pays for every launch (2048 x 2048 at three levels: 4 launches and 24 us before, 3 and 8 us;
-// 17408 x 5120: 8 and 81, 3 and 14 us).  Bound by the latency of its chain: sums, the row in front, bitmap words.
+// The same table with a workspace for sums: two launches for any number of levels, where counting a level and scanning it in two or
+// four launches each pays for every launch (2048 x 2048 at three levels: 4 launches and 24 us; 17408 x 5120: 8 and 81).  Bound by the
+// latency of their chains: bitmap words; sums, words around the first unit, a unit's words, the last two once more a level.  (A launch
+// a level and one more, each waiting for the sums of the one before: 2048 x 2048 at three levels 12.5 us, now 10.4; 5120 x 17408 at
+// five 29.1, now 23.6.)
 //
-// k_rank_level turns the local ranks of level - 1, which the launch before left per tile of kRankTile units, into final
-// ones (the tiles in front of it have left their sums in the workspace), so that it knows where its units start in
-// bitmap `level`; counts them there, four lanes to a unit; and leaves local ranks and its sum for the next launch.
+// k_rank_count counts level 0 in units (their places are known), four lanes to a unit, and leaves ranks local to a tile of kRankTile
+// units and the tile's sum; and it counts the other bitmaps in blocks of words, wherever units lie in them.  k_rank_units
+// makes the ranks of a tile final: the tiles in front give where its units start in bitmap 1, the blocks in front and the words up to
+// there the rank of the first one, its own words the others', and so on through the levels.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kRankTile = 128, kRankThreads = 4 * kRankTile;
 
-__global__ void __launch_bounds__(kRankThreads)
-k_rank_level(Dev P, int level, uint32_t chunk, uint32_t n_units, int32_t *table, uint32_t *sums) {
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t entries = n_units + 1, u0 = blockIdx.x * kRankTile, tiles = gridDim.x;
-    __shared__ uint32_t wave_s[kRankThreads / 64], start[kRankTile + 1], count[kRankTile];
-    uint32_t at = 0;  // index of unit u0 + tid's first element in bitmap `level`
-    if (tid <= kRankTile && u0 + tid <= n_units) {
-        at = (uint32_t)min((uint64_t)(u0 + tid) * chunk, (uint64_t)P.n);
-        for (int j = 0; j < level - 1; ++j) at -= (uint32_t)table[(size_t)j * entries + u0 + tid];
-    }
-    if (level > 0) {
-        int32_t *row = table + (size_t)(level - 1) * entries;
-        const bool mine = tid > 0 && tid <= kRankTile && u0 + tid <= n_units;
-        uint32_t rank = mine ? (uint32_t)row[u0 + tid] : 0u;
-        uint32_t front = 0;
-        for (uint32_t g = tid; g < blockIdx.x; g += kRankThreads) front += sums[(size_t)(level - 1) * tiles + g];
-        front = wave_scan_inclusive(front);
-        if (lane == 63) wave_s[wave] = front;
-        __syncthreads();
-        for (uint32_t k = 0; k < kRankThreads / 64; ++k) rank += wave_s[k];
-        if (mine) row[u0 + tid] = (int32_t)rank;
-        if (u0 + tid == 0) row[0] = 0;
-        at -= rank;
-    }
-    if (level == P.n_levels - 1) return;
-    if (tid <= kRankTile) start[tid] = at;
-    __syncthreads();
-    const uint32_t t = tid >> 2;
+// words of a block: as many bits as a tile has elements, so that there are no more blocks than tiles
+__device__ __forceinline__ uint32_t rank_block(uint32_t chunk) { return min(chunk, 1u << 26) * (kRankTile / 32u); }
+
+// bits set in words [from, end), the last of them up to bit `to` of word `last`; a workgroup's share
+__device__ __forceinline__ uint32_t rank_words(const uint32_t *bm, uint32_t from, uint32_t end, uint32_t last, uint32_t to) {
     uint32_t c = 0;
-    const uint32_t words = P.bm_words[level];
-    if (u0 + t < n_units && words != 0) {
-        const uint32_t lo = start[t], hi = start[t + 1];
-        const uint32_t *bm = P.bm[level];
-        if (hi > lo) {
-            const uint32_t w_first = lo >> 5, w_last = min((hi - 1) >> 5, words - 1);
-            for (uint32_t base = w_first + (tid & 3u); base <= w_last; base += 20) {
-                uint32_t bits[5];
+    for (uint32_t w0 = from + threadIdx.x; w0 < end; w0 += 4u * kRankThreads) {
+        uint32_t bits[4];
 #pragma unroll
-                for (int k = 0; k < 5; ++k) bits[k] = bm[min(base + 4 * k, w_last)];
+        for (uint32_t k = 0; k < 4; ++k) bits[k] = bm[min(w0 + k * kRankThreads, end - 1u)];
 #pragma unroll
-                for (int k = 0; k < 5; ++k) {
-                    const uint32_t w = base + 4 * k;
-                    if (w == w_first) bits[k] &= ~0u << (lo & 31);
-                    if (w == (hi - 1) >> 5 && (hi & 31) != 0) bits[k] &= ~0u >> (32 - (hi & 31));
-                    c += w <= w_last ? __popc(bits[k]) : 0;
-                }
-            }
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t w = w0 + k * kRankThreads;
+            c += w < end ? __popc(w == last ? bits[k] & ((1u << to) - 1u) : bits[k]) : 0;
         }
     }
+    return c;
+}
+
+// set bits of bitmap `level` in [lo, hi), dealt to four lanes
+__device__ __forceinline__ uint32_t rank_bits(const Dev &P, int level, uint32_t lo, uint32_t hi, uint32_t lane) {
+    const uint32_t words = P.bm_words[level];
+    if (hi <= lo || words == 0) return 0;
+    const uint32_t *bm = P.bm[level];
+    const uint32_t w_first = lo >> 5, w_last = min((hi - 1) >> 5, words - 1);
+    uint32_t c = 0;
+    for (uint32_t base = w_first + lane; base <= w_last; base += 20) {
+        uint32_t bits[5];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) bits[k] = bm[min(base + 4 * k, w_last)];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            const uint32_t w = base + 4 * k;
+            if (w == w_first) bits[k] &= ~0u << (lo & 31);
+            if (w == (hi - 1) >> 5 && (hi & 31) != 0) bits[k] &= ~0u >> (32 - (hi & 31));
+            c += w <= w_last ? __popc(bits[k]) : 0;
+        }
+    }
+    return c;
+}
+
+// the sum of a workgroup's values, in every thread; sum_s is free again after the caller's next barrier
+__device__ __forceinline__ uint32_t rank_sum(uint32_t v, uint32_t *sum_s) {
+    v = wave_scan_inclusive(v);
+    if ((threadIdx.x & 63) == 63) sum_s[threadIdx.x >> 6] = v;
+    __syncthreads();
+    uint32_t sum = 0;
+    for (uint32_t k = 0; k < kRankThreads / 64; ++k) sum += sum_s[k];
+    return sum;
+}
+
+// what four lanes counted of each unit, summed up to and with unit tid (tid < kRankTile)
+__device__ __forceinline__ uint32_t rank_scan(uint32_t c, uint32_t *count, uint32_t *wave_s) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     c += (uint32_t)__shfl_xor((int)c, 1);
     c += (uint32_t)__shfl_xor((int)c, 2);
-    if ((tid & 3u) == 0) count[t] = c;
+    if ((tid & 3u) == 0) count[tid >> 2] = c;
     __syncthreads();
+    uint32_t v = 0;
     if (wave < kRankTile / 64) {
-        const uint32_t v = wave_scan_inclusive(count[tid]);
+        v = wave_scan_inclusive(count[tid]);
         if (lane == 63) wave_s[wave] = v;
-        count[tid] = v;
     }
     __syncthreads();
+    for (uint32_t k = 0; k < wave && k < kRankTile / 64; ++k) v += wave_s[k];
+    return v;
+}
+
+__global__ void __launch_bounds__(kRankThreads)
+k_rank_count(Dev P, uint32_t chunk, uint32_t n_units, uint32_t tiles, int32_t *table, uint32_t *sums) {
+    const uint32_t tid = threadIdx.x;
+    __shared__ uint32_t wave_s[kRankThreads / 64], count[kRankTile];
+    if (blockIdx.x >= tiles) {
+        const uint32_t block = blockIdx.x % tiles, bw = rank_block(chunk);
+        const int level = (int)(blockIdx.x / tiles);
+        const uint64_t from = (uint64_t)block * bw, end = min(from + bw, (uint64_t)P.bm_words[level]);
+        uint32_t c = from < end ? rank_words(P.bm[level], (uint32_t)from, (uint32_t)end, ~0u, 0u) : 0u;
+        c = rank_sum(c, wave_s);
+        if (tid == 0) sums[blockIdx.x] = c;
+        return;
+    }
+    const uint32_t u = blockIdx.x * kRankTile + (tid >> 2);
+    uint32_t c = 0;
+    if (u < n_units)
+        c = rank_bits(P, 0, (uint32_t)((uint64_t)u * chunk), (uint32_t)min((uint64_t)(u + 1u) * chunk, (uint64_t)P.n), tid & 3u);
+    const uint32_t rank = rank_scan(c, count, wave_s);
     if (tid < kRankTile) {
-        uint32_t rank = count[tid];
-        for (uint32_t k = 0; k < wave; ++k) rank += wave_s[k];
-        int32_t *row = table + (size_t)level * entries;
-        if (u0 + tid < n_units) row[u0 + tid + 1] = (int32_t)rank;
-        if (tid == kRankTile - 1) sums[(size_t)level * tiles + blockIdx.x] = rank;
+        if (blockIdx.x * kRankTile + tid < n_units) table[blockIdx.x * kRankTile + tid + 1] = (int32_t)rank;
+        if (tid == kRankTile - 1) sums[blockIdx.x] = rank;
+    }
+}
+
+__global__ void __launch_bounds__(kRankThreads)
+k_rank_units(Dev P, uint32_t chunk, uint32_t n_units, int32_t *table, const uint32_t *sums) {
+    const uint32_t tid = threadIdx.x, entries = n_units + 1, u0 = blockIdx.x * kRankTile, tiles = gridDim.x;
+    __shared__ uint32_t sum_s[kRankThreads / 64], wave_s[kRankThreads / 64], start[kRankTile + 1], count[kRankTile];
+    const bool mine = tid <= kRankTile && u0 + tid <= n_units;
+    const bool kept = mine && (tid > 0 || u0 == 0);  // (the first unit's rank is the last of the tile in front)
+    uint32_t rank = mine && tid > 0 ? (uint32_t)table[u0 + tid] : 0u, front = 0;
+    for (uint32_t g = tid; g < blockIdx.x; g += kRankThreads) front += sums[g];
+    rank += rank_sum(front, sum_s);
+    if (kept) table[u0 + tid] = (int32_t)rank;
+    // index of unit u0 + tid's first element in the bitmap of the next level
+    uint32_t at = mine ? (uint32_t)min((uint64_t)(u0 + tid) * chunk, (uint64_t)P.n) - rank : 0u;
+    for (int level = 1; level < P.n_levels - 1; ++level) {
+        if (tid <= kRankTile) start[tid] = at;
+        __syncthreads();
+        // the rank of the tile's first unit
+        const uint32_t words = P.bm_words[level], p0 = start[0], bw = rank_block(chunk), block = min(p0 >> 5, words) / bw;
+        const uint32_t *const of = sums + (uint32_t)level * tiles;
+        uint32_t c = rank_words(P.bm[level], block * bw, min((p0 >> 5) + 1u, words), p0 >> 5, p0 & 31u);
+        for (uint32_t g = tid; g < block; g += kRankThreads) c += of[g];
+        // and of its units
+        const uint32_t t = tid >> 2, mine_c = u0 + t < n_units ? rank_bits(P, level, start[t], start[t + 1], tid & 3u) : 0u;
+        const uint32_t base = rank_sum(c, sum_s), up_to = rank_scan(mine_c, count, wave_s);
+        if (tid < kRankTile) count[tid] = up_to;
+        __syncthreads();
+        if (mine) {
+            rank = base + (tid ? count[tid - 1] : 0u);
+            if (kept) table[(size_t)level * entries + u0 + tid] = (int32_t)rank;
+            at -= rank;
+        }
     }
 }
 
@@ -213,10 +273,11 @@ size_t prefix_workspace_bytes(uint64_t n, uint64_t chunk, int n_levels) {
 }
 
 int launch_prefix_build_ws(const Dev &P, uint32_t chunk, int32_t *table, void *workspace, hipStream_t s) {
-    const uint32_t n_units = (uint32_t)(((uint64_t)P.n + chunk - 1) / chunk);
-    for (int i = 0; i < P.n_levels; ++i)
-        hipLaunchKernelGGL(k_rank_level, dim3(rank_tiles(P.n, chunk)), dim3(kRankThreads), 0, s, P, i, chunk, n_units, table,
-                           static_cast<uint32_t *>(workspace));
+    const uint32_t n_units = (uint32_t)(((uint64_t)P.n + chunk - 1) / chunk), tiles = rank_tiles(P.n, chunk);
+    uint32_t *const sums = static_cast<uint32_t *>(workspace);
+    hipLaunchKernelGGL(k_rank_count, dim3(tiles * (uint32_t)(P.n_levels - 1)), dim3(kRankThreads), 0, s, P, chunk, n_units,
+                       tiles, table, sums);
+    hipLaunchKernelGGL(k_rank_units, dim3(tiles), dim3(kRankThreads), 0, s, P, chunk, n_units, table, sums);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
