@@ -236,6 +236,7 @@ int ixh_lanes_list(const uint16_t *w, const IxhLanes *dst, ixh_stream_t stream);
 int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
                    int64_t ldy, void *workspace, size_t workspace_bytes, ixh_stream_t stream);
 
+/* From five rows on enough for any m up to 16; a call asks for what its own m takes. */
 size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m);
 
 /*

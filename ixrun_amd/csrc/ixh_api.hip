@@ -581,7 +581,10 @@ int ixh_lanes_list(const uint16_t *w, const IxhLanes *dst, ixh_stream_t stream) 
 size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m) {
     LanesDev d;
     if (to_lanes(lanes, &d, true) || m < 1 || m > 16) return 0;
-    return lanes_rows_workspace_bytes(d, m);
+    // From five rows on, what any count up to 16 takes: a batch that grows makes no caller replace its buffer (a shared one that
+    // captured graphs hold is kept for them beside the new one).
+    return m <= 4 ? lanes_rows_workspace_bytes(d, m)
+                  : max(lanes_rows_workspace_bytes(d, m), max(lanes_rows_workspace_bytes(d, 8), lanes_rows_workspace_bytes(d, 16)));
 }
 
 int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
