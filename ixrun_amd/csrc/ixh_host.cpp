@@ -31,6 +31,9 @@ struct Forward {
     const uint16_t *bias;
     int64_t in_f, out_f;
     long device;
+    decltype(&ixh_lanes_gemm) gemm;
+    decltype(&ixh_lanes_gemm_workspace_bytes) gemm_workspace_bytes;
+    long many_rows;  // rows up to which `many` takes a call; 0 until it is set
     long any_rows;  // more rows than these: plain calls only (no gradient, transform or other result type is asked for)
     size_t workspace_bytes[kMaxRows + 1];
     PyObject *owner;       // keeps `lanes` and what it points at alive
@@ -92,18 +95,59 @@ PyObject *forward_call(PyObject *self_, PyObject *const *args, size_t nargsf, Py
     END_HANDLE_TH_ERRORS
 }
 
-// Forward(gemv, lanes, bias, in_f, out_f, device, workspace_bytes, owner, workspaces, device_key, check, plain); addresses as
-// ints.  any_rows is 0 until it is set.
+// many(x): 17 .. many_rows rows, plain calls only.  The slices' sums go through memory allocated for the call.  The host's way from
+// Python and through ctypes took longer than the kernels of layers of up to some 2^24 weights: 20 to 21 us a call whatever the rows;
+// now 2048 x 2048 at 17 / 100 / 192 rows 10.4 / 13.3 / 17.5, 4096 x 4096 (4 bits) at 32 rows 13.1, 5120 x 5120 at 32 rows 18.6, which
+// are the kernels, and 512 x 768 10.6.
+PyObject *forward_many(PyObject *self_, PyObject *arg) {
+    HANDLE_TH_ERRORS
+    Forward *self = reinterpret_cast<Forward *>(self_);
+    if (self->call != forward_call || !THPVariable_CheckExact(arg)) Py_RETURN_NONE;
+    const at::Tensor &x = THPVariable_Unpack(arg);
+    if (!x.is_cuda() || x.scalar_type() != at::kBFloat16 || x.dim() < 1 || x.size(-1) != self->in_f || x.get_device() != self->device ||
+        !x.is_contiguous() || c10::hip::current_device() != self->device)
+        Py_RETURN_NONE;
+    const int64_t rows = x.numel() / self->in_f;
+    if (rows <= kMaxRows || rows > self->many_rows || (reinterpret_cast<uintptr_t>(x.const_data_ptr()) & 15u) != 0) Py_RETURN_NONE;
+    PyObject *plain = PyObject_CallOneArg(self->plain, arg);
+    const int yes = plain ? PyObject_IsTrue(plain) : -1;
+    Py_XDECREF(plain);
+    if (yes < 0) return nullptr;
+    if (!yes) Py_RETURN_NONE;
+    c10::SmallVector<int64_t, 4> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = self->out_f;
+    at::Tensor y, sums;
+    int rc;
+    {
+        pybind11::gil_scoped_release without_gil;
+        y = at::empty(shape, x.options());
+        const size_t need = self->gemm_workspace_bytes(self->lanes, (int32_t)rows);
+        if (need) sums = at::empty({(int64_t)need}, x.options().dtype(at::kByte));
+        rc = self->gemm(self->lanes, static_cast<const uint16_t *>(x.const_data_ptr()), self->in_f, self->bias, (int32_t)rows,
+                        static_cast<uint16_t *>(y.data_ptr()), self->out_f, need ? sums.data_ptr() : nullptr, need,
+                        c10::hip::getCurrentHIPStream((c10::DeviceIndex)self->device).stream());
+    }
+    if (rc) {
+        PyObject *r = PyObject_CallFunction(self->check, "i", rc);
+        Py_XDECREF(r);
+        if (!r) return nullptr;
+    }
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+// Forward(gemv, lanes, bias, in_f, out_f, device, workspace_bytes, owner, workspaces, device_key, check, plain, gemm,
+// gemm_workspace_bytes); addresses as ints.  any_rows and many_rows are 0 until they are set.
 int forward_init(PyObject *self_, PyObject *args, PyObject *) {
     Forward *self = reinterpret_cast<Forward *>(self_);
-    unsigned long long gemv, lanes, bias;
+    unsigned long long gemv, lanes, bias, gemm, gemm_workspace_bytes;
     long long in_f, out_f;
     long device;
     PyObject *bytes, *owner, *workspaces, *key, *check, *plain;
-    if (!PyArg_ParseTuple(args, "KKKLLlO!OO!OOO", &gemv, &lanes, &bias, &in_f, &out_f, &device, &PyTuple_Type, &bytes, &owner,
-                          &PyDict_Type, &workspaces, &key, &check, &plain))
+    if (!PyArg_ParseTuple(args, "KKKLLlO!OO!OOOKK", &gemv, &lanes, &bias, &in_f, &out_f, &device, &PyTuple_Type, &bytes, &owner,
+                          &PyDict_Type, &workspaces, &key, &check, &plain, &gemm, &gemm_workspace_bytes))
         return -1;
-    if (!gemv || !lanes || in_f < 1 || out_f < 1 || PyTuple_GET_SIZE(bytes) != kMaxRows + 1) {
+    if (!gemv || !lanes || !gemm || !gemm_workspace_bytes || in_f < 1 || out_f < 1 || PyTuple_GET_SIZE(bytes) != kMaxRows + 1) {
         PyErr_SetString(PyExc_ValueError, "Forward: malformed arguments");
         return -1;
     }
@@ -113,6 +157,8 @@ int forward_init(PyObject *self_, PyObject *args, PyObject *) {
     }
     self->call = forward_call;
     self->gemv = reinterpret_cast<LanesGemv>(gemv);
+    self->gemm = reinterpret_cast<decltype(self->gemm)>(gemm);
+    self->gemm_workspace_bytes = reinterpret_cast<decltype(self->gemm_workspace_bytes)>(gemm_workspace_bytes);
     self->lanes = reinterpret_cast<const IxhLanes *>(lanes);
     self->bias = reinterpret_cast<const uint16_t *>(bias);
     self->in_f = in_f;
@@ -430,7 +476,13 @@ PyMethodDef methods[] = {
 
 PyMemberDef forward_members[] = {
     {"any_rows", T_LONG, offsetof(Forward, any_rows), 0, "Rows up to which calls that are not plain are taken too."},
+    {"many_rows", T_LONG, offsetof(Forward, many_rows), 0, "Rows up to which `many` takes a call."},
     {nullptr, 0, 0, 0, nullptr},
+};
+
+PyMethodDef forward_methods[] = {
+    {"many", forward_many, METH_O, "The forward of more rows than a call takes, or None."},
+    {nullptr, nullptr, 0, nullptr},
 };
 
 PyTypeObject forward_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
@@ -446,6 +498,7 @@ PyMODINIT_FUNC PyInit__host() {
     forward_type.tp_vectorcall_offset = offsetof(Forward, call);
     forward_type.tp_call = PyVectorcall_Call;
     forward_type.tp_members = forward_members;
+    forward_type.tp_methods = forward_methods;
     forward_type.tp_new = forward_new;
     forward_type.tp_init = forward_init;
     forward_type.tp_traverse = forward_traverse;

@@ -247,7 +247,11 @@ class StreamingLinear(nn.Module):
                 ctypes.cast(self._gemv_fn, ctypes.c_void_p).value, ctypes.addressof(self._lanes.struct), self._bias_ptr or 0,
                 self.in_features, self.out_features, dev.index,
                 (0,) + tuple(self._lanes.gemv_workspace_bytes(n) for n in range(1, MAX_FUSED_ROWS + 1)),
-                (self._lanes, self._bias), _workspaces, dev, _lib.check, _plain_call)
+                (self._lanes, self._bias), _workspaces, dev, _lib.check, _plain_call,
+                *(ctypes.cast(f, ctypes.c_void_p).value
+                  for f in (_lib.lib().ixh_lanes_gemm, _lib.lib().ixh_lanes_gemm_workspace_bytes)))
+            # (what _lanes_gemm_wins allows for a count of rows, it allows for fewer)
+            self._native.many_rows = max((rows for rows in (160, 224, 256, 512, 1024) if self._lanes_gemm_wins(rows)), default=0)
         self._forget_plans()
 
     def _apply(self, fn, recurse=True):
@@ -346,6 +350,8 @@ class StreamingLinear(nn.Module):
     def forward(self, x):
         if self._native is not None and self._use_fused and not self._gemv_flags and self._gemv_fn is self._native_fn:
             y = self._native(x)
+            if y is None and self._gemm_ok:
+                y = self._native.many(x)
             if y is not None:
                 return y
         in_f = self.in_features

@@ -292,6 +292,49 @@ def test_list_that_ends_on_a_whole_group(oracle, dev, listed):
         check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
 
 
+@pytest.mark.parametrize("kind", ["rare", "real"])
+def test_prompts_from_native_code(dev, kind):
+    """17 rows up to the last count that the lanes are the fastest way for: the same bits as by Python's way, and left to it where
+    they always were (more rows, views, odd addresses, gradients, autocast to another type, a switch turned off)."""
+    from ixrun_amd.engine import StreamingLinear
+
+    out_f, in_f = 1030, 1024
+    v, scheme, _ = values(kind, out_f, in_f)
+    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
+    layer, other = StreamingLinear(p, bias := torch.randn(out_f).bfloat16()), StreamingLinear(p, bias)
+    other._native = None
+    most = layer._native.many_rows
+    assert layer._lanes_gemm_wins(most) and not layer._lanes_gemm_wins(most + 1)
+    wide = activations(most + 2, in_f + 8, seed=3).to(dev)
+
+    def same(x, native):
+        assert (layer._native.many(x) is not None) == native
+        y = layer(x)
+        assert torch.equal(y, other(x)) and y.shape == x.shape[:-1] + (out_f,)
+
+    for rows in (16, 17, 33, most, most + 1):
+        same(wide[:rows, :in_f].contiguous(), 17 <= rows <= most)
+    x = wide[:40, :in_f].contiguous()
+    same(x.view(5, 8, in_f), True)
+    same(x.view(2, 20, 1, in_f).transpose(0, 1), False)
+    same(wide.view(-1)[1 : 1 + 40 * in_f].view(40, in_f), False)
+    assert layer._native.many(x.clone().requires_grad_()) is None and layer._native.many(x.float()) is None
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert layer._native.many(x) is None
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        y = layer(x)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(y, other(x))
+    layer._set_shared_buf(torch.zeros(p["N"], dtype=torch.bfloat16, device=dev))
+    layer(x)
+    assert not bool(layer._w_buf.any())
+    layer._gemm_ok = False
+    layer(x)
+    assert bool(layer._w_buf.any())
+
+
 @pytest.mark.parametrize("in_f,rows", [(1024, 2), (1024, 16), (1004, 5), (1004, 20)])
 def test_calls_that_are_not_plain_keep_the_decode(monkeypatch, dev, in_f, rows):
     """Gradients, forward mode, vmap, autocast and other kinds of tensors: a layer with a decode buffer whose rows went
