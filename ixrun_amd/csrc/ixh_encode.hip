@@ -264,7 +264,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 // ---------------------------------------------------------------------------------------------------------------
 // k_enc_pack<L>: bound by vector issue: of 5120 x 17408 at levels 3, 5, 8 690 vector instructions a wave and span (heavy tails)
-// to 790 (55 / 40 / 5 %), 70 to 75 us; the 240 MB that it moves take 47.
+// to 790 (55 / 40 / 5 %), 62 to 72 us; the 240 MB that it moves take 47.
 //
 // A wave takes spans of four units, 2048 elements, 32 consecutive ones a lane, so one prefix sum over the lanes serves them
 // all and a lane's membership bits are a whole word of bitmap 0.  Every element goes to LDS as one byte, value + 128: those
@@ -279,8 +279,16 @@ constexpr uint32_t kEncBuf = kEncSpan + 256;  // two runs with their margins
 constexpr uint32_t dense_at = 32u;            // where a dense run's groups start in it
 
 // Spans per wave: a wave that goes on hands its unfinished groups to its next span in registers, and only its first and last
-// cost atomics (one span each: 107 .. 175 us instead of 70 .. 75).  As many as leave the chip some 4096 waves, at most 8.
-constexpr uint32_t kEncMaxSpans = 8, kEncFill = 4096;
+// cost atomics (one span each: 107 .. 175 us instead of 70 .. 75).  The spans are dealt out evenly to as many waves as run at the
+// same time (three levels, 89 registers: five on each of a CU's four SIMDs), so that no CU is left with a workgroup more than another: 5120 x 17408
+// at 55 / 40 / 5 % 71.8 us, 76.7 with eight spans each (5.3 workgroups a CU), 74.4 with four waves a SIMD, 80.2 with six (a second
+// round); at five levels (four waves a SIMD) 145.1 -> 130.2.
+struct EncShare {
+    uint32_t waves, spans, more;  // the first `more` waves have a span more than the others
+    __device__ __forceinline__ uint32_t first_unit(uint32_t wave, uint32_t n_units) const {
+        return min((wave * spans + min(wave, more)) * kEncSpanUnits, n_units);
+    }
+};
 
 // level i's rank at unit `u`, and the index of the unit's first element in bitmap i
 struct EncRanks {
@@ -300,23 +308,33 @@ __device__ __forceinline__ float edge_of(int bits) { return (float)threshold_of(
 
 // clears what neighbouring waves share: of every stream the group of 32 codes that a wave's first code falls into,
 // of every bitmap but the first the word of its first bit; and any words behind the last code
+// (5.8 us with the ranks asked for level by level, 5.1 with all of them first, 5120 x 17408: a launch and their latency.)
+template <int L>
 __global__ void __launch_bounds__(256)
-k_enc_borders(EncLevels lv, const int32_t *__restrict__ table, uint32_t n, uint32_t n_units, uint32_t wave_units, EncOut out) {
-    const uint32_t s = blockIdx.x * 256u + threadIdx.x, u = min(s * wave_units, n_units);
-    const uint32_t n_waves = (n_units + wave_units - 1) / wave_units;
+k_enc_borders(EncLevels lv, const int32_t *__restrict__ table, uint32_t n, uint32_t n_units, EncShare share, EncOut out) {
+    const uint32_t s = blockIdx.x * 256u + threadIdx.x, u = share.first_unit(min(s, share.waves), n_units);
     const EncRanks r{table, n_units + 1, n};
-    for (int i = 0; i < lv.n_levels - 1; ++i) {
-        for (uint32_t k = (r.space(i, n_units) + 31u) / 32u + s; k < out.bm_words[i]; k += gridDim.x * 256u) out.bm[i][k] = 0u;
-        const uint64_t used = ((uint64_t)r.rank(i, n_units) * (uint32_t)lv.bits[i] + 31u) / 32u;
+    uint32_t all[L - 1], here[L - 1];
+#pragma unroll
+    for (int i = 0; i < L - 1; ++i) {
+        all[i] = r.rank(i, n_units);
+        here[i] = r.rank(i, u);
+    }
+    uint32_t bits = n, at = min(u * kEncUnit, n);  // of bitmap i in all, and those in front of the unit
+#pragma unroll
+    for (int i = 0; i < L - 1; ++i) {
+        for (uint32_t k = (bits + 31u) / 32u + s; k < out.bm_words[i]; k += gridDim.x * 256u) out.bm[i][k] = 0u;
+        const uint32_t b = (uint32_t)lv.bits[i];
+        const uint64_t used = ((uint64_t)all[i] * b + 31u) / 32u;
         for (uint64_t k = used + s; k < out.st_words[i]; k += gridDim.x * 256u) out.st[i][k] = 0u;
-        if (s > n_waves) continue;
-        const uint32_t b = (uint32_t)lv.bits[i], word = (r.rank(i, u) >> 5) * b;
-        for (uint32_t k = 0; k < b; ++k)
-            if (word + k < out.st_words[i]) out.st[i][word + k] = 0u;
-        if (i > 0) {
-            const uint32_t at = r.space(i, u) >> 5;
-            if (at < out.bm_words[i]) out.bm[i][at] = 0u;
+        if (s <= share.waves) {
+            const uint32_t word = (here[i] >> 5) * b;
+            for (uint32_t k = 0; k < b; ++k)
+                if (word + k < out.st_words[i]) out.st[i][word + k] = 0u;
+            if (i > 0 && (at >> 5) < out.bm_words[i]) out.bm[i][at >> 5] = 0u;
         }
+        bits -= all[i];
+        at -= here[i];
     }
 }
 
@@ -416,13 +434,14 @@ __device__ __forceinline__ void load32(const uint16_t *__restrict__ w, uint32_t 
 
 template <int L>
 __global__ void __launch_bounds__(kWave *kEncWaves)
-k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, uint32_t wave_units,
+k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShare share,
            const uint16_t *__restrict__ scale_in, EncLevels lv, const int32_t *__restrict__ table, EncOut out) {
     __shared__ __attribute__((aligned(32))) uint8_t bufs[kEncWaves][2][kEncBuf];
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t u_first = (blockIdx.x * kEncWaves + wave) * wave_units, u_end = min(u_first + wave_units, n_units);
-    if (u_first >= n_units) return;
+    const uint32_t mine = blockIdx.x * kEncWaves + wave;
+    if (mine >= share.waves) return;
+    const uint32_t u_first = share.first_unit(mine, n_units), u_end = share.first_unit(mine + 1u, n_units);
     const EncRanks ranks{table, n_units + 1, n};
     const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
     const float inv_scale = __fdiv_rn(1.0f, bf16_bits_to_f32(*scale_in));
@@ -439,19 +458,27 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, uint32_
         carry[i] = 128u - (uint32_t)threshold_of(lv.bits[i]);
         bm_carry[i] = 0u;
     }
+    // a span's weights and the ranks at its end are asked for while the span before is packed
+    uint32_t d[16], r1_next[L - 1];
+    auto ask = [&](uint32_t u) {
+        const uint32_t e = u * kEncUnit, to = min(u + kEncSpanUnits, n_units);
+        load32(w, e + lane * 32u, n, aligned && (uint64_t)e + kEncSpan <= n, d);
+#pragma unroll
+        for (int i = 0; i < L - 1; ++i) r1_next[i] = ranks.rank(i, to);
+    };
+    ask(u_first);
     for (uint32_t u0 = u_first; u0 < u_end; u0 += kEncSpanUnits) {
         const uint32_t u1 = min(u0 + kEncSpanUnits, n_units);
         const bool final = u1 == u_end;
         const uint32_t e0 = u0 * kEncUnit, e1 = min(e0 + kEncSpan, n);
         uint32_t r1[L - 1];
 #pragma unroll
-        for (int i = 0; i < L - 1; ++i) r1[i] = ranks.rank(i, u1);
+        for (int i = 0; i < L - 1; ++i) r1[i] = r1_next[i];
         uint32_t left = e1 - e0;  // (the counts below come from the caller's table: held to the span)
 
         // ---- quantise ----
         const uint32_t p = e0 + lane * 32u;
-        uint32_t d[16], member = 0;
-        load32(w, p, n, aligned && e0 + kEncSpan <= n, d);
+        uint32_t member = 0;
         // (see quantise: the sum with 3072 restores exact ties)
         float v[32];
         uint64_t in[32];
@@ -499,6 +526,7 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, uint32_
                              g_first[i], g_last[i], out.st[i], out.st_words[i], lane);
             carry[i] = b[dense_at + whole * 32u + (lane & 31u)];
         };
+        if (!final) ask(u1);
         margins(buf, dense_at, r0[0], n_i, carry[0], 128u - (uint32_t)threshold_of(lv.bits[0]));
         margins(buf, rest, space0, left, 128u, 128u);
         wave_lds_sync();
@@ -630,10 +658,19 @@ int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *b
 
 template <int L>
 static void pack_launch(const uint16_t *w, uint32_t n, uint32_t n_units, const uint16_t *scale, const EncLevels &lv,
-                        uint32_t wave_units, const int32_t *table, const EncOut &out, hipStream_t s) {
-    const uint32_t waves = (n_units + wave_units - 1) / wave_units;
-    hipLaunchKernelGGL(k_enc_pack<L>, dim3((waves + kEncWaves - 1) / kEncWaves), dim3(kWave * kEncWaves), 0, s, w, n, n_units,
-                       wave_units, scale, lv, table, out);
+                        const int32_t *table, const EncOut &out, hipStream_t s) {
+    static const uint32_t at_once = [] {
+        int dev = 0, cus = 256, groups = 5;
+        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&groups, k_enc_pack<L>, kWave * kEncWaves, 0);
+        return (uint32_t)(max(cus, 1) * max(groups, 1)) * kEncWaves;
+    }();
+    const uint32_t spans = (n_units + kEncSpanUnits - 1) / kEncSpanUnits, waves = min(spans, at_once);
+    const EncShare share{waves, waves ? spans / waves : 0u, waves ? spans % waves : 0u};
+    hipLaunchKernelGGL(k_enc_borders<L>, dim3((share.waves + 256u) / 256u), dim3(256), 0, s, lv, table, n, n_units, share, out);
+    if (n_units == 0) return;
+    hipLaunchKernelGGL(k_enc_pack<L>, dim3((share.waves + kEncWaves - 1) / kEncWaves), dim3(kWave * kEncWaves), 0, s, w, n, n_units,
+                       share, scale, lv, table, out);
 }
 
 int launch_encode_pack(const uint16_t *w, const Dev &P, const int32_t *table, hipStream_t s) {
@@ -651,20 +688,14 @@ int launch_encode_pack(const uint16_t *w, const Dev &P, const int32_t *table, hi
     }
     out.last = const_cast<uint8_t *>(P.last);
     out.last_bytes = P.last_bytes;
-    const uint32_t spans = (n_units + kEncSpanUnits - 1) / kEncSpanUnits;
-    const uint32_t wave_units = max(1u, min(kEncMaxSpans, spans / kEncFill)) * kEncSpanUnits;
-    const uint32_t waves = (n_units + wave_units - 1) / wave_units;
-    hipLaunchKernelGGL(k_enc_borders, dim3((waves + 256u) / 256u), dim3(256), 0, s, lv, table, n, n_units, wave_units, out);
-    if (n_units != 0) {
-        switch (P.n_levels) {
-            case 2: pack_launch<2>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
-            case 3: pack_launch<3>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
-            case 4: pack_launch<4>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
-            case 5: pack_launch<5>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
-            case 6: pack_launch<6>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
-            case 7: pack_launch<7>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
-            default: pack_launch<8>(w, n, n_units, P.scale, lv, wave_units, table, out, s); break;
-        }
+    switch (P.n_levels) {
+        case 2: pack_launch<2>(w, n, n_units, P.scale, lv, table, out, s); break;
+        case 3: pack_launch<3>(w, n, n_units, P.scale, lv, table, out, s); break;
+        case 4: pack_launch<4>(w, n, n_units, P.scale, lv, table, out, s); break;
+        case 5: pack_launch<5>(w, n, n_units, P.scale, lv, table, out, s); break;
+        case 6: pack_launch<6>(w, n, n_units, P.scale, lv, table, out, s); break;
+        case 7: pack_launch<7>(w, n, n_units, P.scale, lv, table, out, s); break;
+        default: pack_launch<8>(w, n, n_units, P.scale, lv, table, out, s); break;
     }
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }

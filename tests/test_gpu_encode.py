@@ -194,6 +194,14 @@ def test_encode_span_edges(oracle, dev, n, level_bits, kind):
     check_against_oracle(oracle, dev, make_weight(kind, 1, n), level_bits)
 
 
+@pytest.mark.parametrize("level_bits,waves", [((3, 5, 8), 20), ((3, 4, 5, 6, 8), 16), ((2, 8), 24)])
+@pytest.mark.parametrize("spans,more", [(1, 0), (1, 1), (2, -1999)])
+def test_encode_waves_of_more_than_a_span(oracle, dev, level_bits, waves, spans, more):
+    """As many spans of 2048 as waves run at the same time (so many on each CU), one element more, and nearly twice as many."""
+    n = spans * waves * torch.cuda.get_device_properties(dev).multi_processor_count * 2048 + more
+    check_against_oracle(oracle, dev, make_weight("calibrated_odd_scale", 1, n), level_bits)
+
+
 SCAN = "ixh_encode_scan_counts"
 
 
