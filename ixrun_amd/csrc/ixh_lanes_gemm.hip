@@ -291,13 +291,19 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 }
 
 // How the work is cut: groups of 16 .. 128 activation rows, slices of the columns and groups of 16-row blocks, a workgroup
-// per CU. Of all such cuts the one with the shortest estimate, in clocks. A stage takes 3000 + 400 MB from its first request
-// to its last product, whether 3 or 13 blocks share it (measured: 4.0 to 6.1 thousand for MB = 3, 7.0 to 8.4 thousand for MB
-// = 8), unless LDS, at 128 bytes a clock, is fuller than that; the slices' sums cost a launch and their way through memory.
-// (More and smaller row groups where the weights leave CUs idle: 1024 x 1024, 128 rows, 19 us in one group, 13 in four.)
+// per CU. Of all such cuts the one with the shortest estimate, in clocks, from all cuts, timed, of 19 shapes from 256 x 17408 to
+// 17408 x 5120 at 24 to 256 rows.  Weights of few columns or few rows, and up to 64 activation rows of more than 2^23 weights: a
+// stage takes 3500 from its first request to its last product, 200 for each 16 activation rows and 60 for each block of weights that
+// shares it, and the slices' sums cost a launch and their way through memory.  Elsewhere 3000 and 400 for each 16 rows, whether 3 or
+// 13 blocks share the stage, unless LDS, at 128 bytes a clock, is fuller than that, and a cheaper launch of the sums.  Those figures
+// slice few columns that are better taken whole by more groups of activation rows (us, with them and with the first ones: 8192 x 1024 at
+// 52 / 100 / 128 rows 13.7 / 20.2 / 21.5 and 12.5 / 16.5 / 16.7, 16384 x 512 at 80 rows 15.5 and 12.9, 256 x 17408 at 128 rows 18.7
+// and 15.5, 4096 x 4096 (4 bits) at 40 rows 17.7 and 14.2); the first ones take too few groups elsewhere (3072 x 3072 at 128 rows
+// 19.7 and 20.4, 2048 x 7168 (3 bits) at 80 rows 18.4 and 19.6, 2048 x 2048 at 40 rows 10.3 and 10.7).
 struct LgPlan { uint32_t m_groups, mb, slices, groups; };
 static LgPlan lg_plan(const LanesDev &L, int m) {
     const uint32_t blocks = (L.n_tiles + 3u) / 4u, m_blocks = ((uint32_t)m + 15u) / 16u;
+    const bool shared = L.n_cells <= 2u || blocks <= 64u || (m <= 64 && (uint64_t)L.n_tiles * L.n_cells > 4096u);
     LgPlan best{};
     uint64_t best_cost = ~0ull;
     for (uint32_t m_groups = (m_blocks + kLgMost - 1u) / kLgMost; m_groups <= max((m_blocks + 1u) / 2u, 1u); ++m_groups) {
@@ -306,8 +312,8 @@ static LgPlan lg_plan(const LanesDev &L, int m) {
             const uint32_t groups = min(max(cus / s, 1u), blocks);
             const uint32_t share = (blocks + groups - 1u) / groups, rounds = (share + kLgBlocks - 1u) / kLgBlocks;
             const uint32_t at_once = (share + rounds - 1u) / rounds, cells = (L.n_cells + s - 1u) / s;
-            const uint64_t stage = max(3000u + 400u * mb, at_once * (4u * mb + 24u) * 4u);
-            const uint64_t sums = s > 1 ? 8000u + (uint64_t)s * (uint32_t)m * blocks * 16u * 8u / 3400u : 0u;
+            const uint64_t stage = shared ? 3500u + 200u * mb + 60u * at_once : max(3000u + 400u * mb, at_once * (4u * mb + 24u) * 4u);
+            const uint64_t sums = s > 1 ? (shared ? 14000u : 8000u) + (uint64_t)s * (uint32_t)m * blocks * 16u * 8u / 3400u : 0u;
             const uint64_t cost = 4u * stage * rounds * cells + sums;
             if (cost < best_cost) { best_cost = cost; best = {m_groups, mb, s, groups}; }
         }
