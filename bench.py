@@ -37,7 +37,8 @@ MFMA_BF16_PEAK = 2.5e15  # FLOP/s dense bf16, MI355X published
 # workloads without a counter run, or measured on other sources, report null.
 # (bytes per launch, the sources the kernel is compiled from, their kernel_sources_sha16 at the counter run); names that end
 # in _packed are --packed runs, of the kernels that read the packed streams
-_LANES = ("ixh_lanes.hip", "ixh_lanes_gemm.hip", "ixh_lanes.h", "ixh_lanes_dev.h", "ixh_lanes_bounds.h", "ixh_fast358.h", "ixh_dev.h",
+_LANES = ("ixh_lanes.hip", "ixh_lanes_rows.hip", "ixh_lanes_gemm.hip", "ixh_lanes_prompt.hip", "ixh_lanes.h",
+          "ixh_lanes_dev.h", "ixh_lanes_bounds.h", "ixh_fast358.h", "ixh_dev.h",
           "build.sh")
 _ROWS = ("ixh_rows358.hip", "ixh_rows_common.h", "ixh_dev.h", "build.sh")
 _TILES = ("ixh_tiles358.hip", "ixh_rows_common.h", "ixh_dev.h")
@@ -48,7 +49,7 @@ _DECODE_ROWS = ("ixh_decode_rows358.hip", "ixh_rows_common.h", "ixh_dev.h")
 _ENCODE = ("ixh_encode.hip", "ixh_dev.h")
 _OLD = ((), "measured-on-earlier-sources")  # figures kept for the record; reported as null
 MEASURED_TRAFFIC_BYTES = {
-    # k_lanes_gemv; from eight rows on k_lanes_gemm + k_lanes_reduce
+    # k_lanes_gemv; eight rows k_lanes_rows, sixteen with k_lanes_reduce
     "down_proj_5120x17408_m1_student_t": (17304.1 * 2.0 * 1024 + 16.0 * 1024, _LANES, "7d30d618c9f315ad"),
     "down_proj_5120x17408_m1_calibrated": (35836.2 * 2.0 * 1024 + 16.0 * 1024, _LANES, "7d30d618c9f315ad"),
     "down_proj_5120x17408_m1_five_level_calibrated": (35841.6 * 2.0 * 1024 + 16.0 * 1024, _LANES, "7d30d618c9f315ad"),
