@@ -247,6 +247,9 @@ size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m);
 int ixh_lanes_gemm(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
                    int64_t ldy, void *workspace, size_t workspace_bytes, ixh_stream_t stream);
 
+/* The sums of column slices; from 129 rows of large layers on, the activations in the kernel's order and 256 KB for each part of
+ * 128 rows of weights that two or more workgroups share: 128 MiB of those at most on 256 CUs, whatever the layer, and none where
+ * each workgroup has whole ones. */
 size_t ixh_lanes_gemm_workspace_bytes(const IxhLanes *lanes, int32_t m);
 
 /*

@@ -77,7 +77,7 @@ bool lanes_gemm_aligned(const LanesDev &L, const uint16_t *x, int m, int64_t ldx
 size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m);
 int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once, uint16_t *y,
                       int64_t ldy, float *ws, hipStream_t s);
-// of them, those of many rows and large layers (ixh_lanes_prompt.hip): x as above, ws 16-byte aligned
+// of them, those of many rows and large layers (ixh_lanes_prompt.hip): x as above, the bias added once
 bool lanes_prompt_wins(const LanesDev &L, int m);
 size_t lanes_prompt_workspace_bytes(const LanesDev &L, int m);
 int launch_lanes_prompt(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,

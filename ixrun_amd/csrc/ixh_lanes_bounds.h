@@ -1,5 +1,5 @@
-// What a wave of k_lanes_gemv (ixh_lanes.hip) asks for ahead of knowing whether it needs it.  Plain C++, so that the ranges
-// can be walked without a GPU.
+// What a wave of k_lanes_gemv (ixh_lanes.hip) asks for ahead of knowing whether it needs it, and where the workgroups of
+// k_lanes_prompt (ixh_lanes_prompt.hip) leave their sums.  Plain C++, so that the ranges can be walked without a GPU.
 #pragma once
 #include <stdint.h>
 
@@ -31,6 +31,26 @@ LN_BOTH bool ln_whole_pieces(uint64_t x, uint32_t in_f, int m, int64_t ldx) {
 LN_BOTH uint32_t ln_piece_column(uint32_t col, uint32_t in_f) {  // in_f >= 8
     const uint32_t last = (in_f & ~7u) - 8u;
     return col < last ? col : last;
+}
+
+// `groups` workgroups share `tiles` tiles of `cells` cells each in runs that differ by one cell at most: workgroup g has the
+// cells lp_begin(g) .. lp_begin(g + 1) - 1, counted through the tiles.  tiles * cells * groups is below 2^32.
+LN_BOTH uint32_t lp_begin(uint32_t g, uint32_t groups, uint32_t tiles, uint32_t cells) { return g * (tiles * cells) / groups; }
+LN_BOTH uint32_t lp_group_of(uint32_t cell, uint32_t groups, uint32_t tiles, uint32_t cells) {
+    return ((cell + 1u) * groups - 1u) / (tiles * cells);
+}
+
+// Of a tile that it has a part of only, a workgroup leaves its sums in memory; a whole tile it finishes by itself.  A run begins
+// inside one tile at most and ends inside one other: part g is workgroup g's of the tile that its run begins in, and behind
+// those come the parts of tiles that a run ends in, by tile (the first one is never among them) or by workgroup, whichever are
+// fewer.  There are none of these where every tile has its own workgroups, and no parts at all where every workgroup has whole tiles.
+LN_BOTH uint32_t lp_part(uint32_t g, uint32_t tile, bool begins, uint32_t groups, uint32_t tiles) {
+    return begins ? g : groups + (tiles <= groups ? tile - 1u : g);
+}
+LN_BOTH uint32_t lp_parts(uint32_t groups, uint32_t tiles) {
+    if (tiles % groups == 0) return 0;
+    if (groups % tiles == 0) return groups;
+    return groups + (tiles < groups ? tiles : groups) - 1u;
 }
 
 }  // namespace ixh

@@ -328,9 +328,9 @@ static LgPlan lg_plan(const LanesDev &L, int m) {
 }
 
 size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m) {
+    if (lanes_prompt_wins(L, m)) return lanes_prompt_workspace_bytes(L, m);
     const LgPlan p = lg_plan(L, m);
-    const size_t sums = p.slices > 1 ? (size_t)p.slices * (uint32_t)m * ((L.n_tiles + 3u) / 4u * 16u) * sizeof(float) : 0;
-    return lanes_prompt_wins(L, m) ? max(sums, lanes_prompt_workspace_bytes(L, m)) : sums;
+    return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * ((L.n_tiles + 3u) / 4u * 16u) * sizeof(float) : 0;
 }
 
 template <int BITS, int MB, int NB>
@@ -370,7 +370,7 @@ static int gemm_rows(const LanesDev &L, const LgPlan &p, A... a) {
 int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once, uint16_t *y,
                       int64_t ldy, float *ws, hipStream_t s) {
     if (!lanes_gemm_aligned(L, x, m, ldx)) return IXH_EUNSUPPORTED;
-    if (once && lanes_prompt_wins(L, m) && ((uintptr_t)ws & 15u) == 0) return launch_lanes_prompt(L, x, m, ldx, bias, y, ldy, ws, s);
+    if (lanes_prompt_wins(L, m)) return launch_lanes_prompt(L, x, m, ldx, bias, y, ldy, ws, s);
     const LgPlan p = lg_plan(L, m);
     if (m == 1) ldx = L.in_f;
     switch (L.bits) {

@@ -11,15 +11,13 @@ constexpr uint32_t kLpTile = kLpRows * 128u * 2u;    // bytes of a stage's weigh
 constexpr uint32_t kLpRounds = 3;                    // groups of 16 quads of a cell's list that a wave holds
 
 __host__ __device__ constexpr uint32_t lp_tiles(uint32_t n_quads) { return (n_quads * 4u + kLpRows - 1u) / kLpRows; }
-// parts of tiles that `groups` workgroups make: workgroup g's part of tile t is part g + t, for each of the two grows by one from
-// a part to the next
-__host__ __device__ constexpr uint32_t lp_parts(uint32_t groups, uint32_t tiles) { return groups + tiles - 1u; }
 
 struct LpOut {
     const uint16_t *bias;
     uint16_t *y;
     int64_t ldy;
     uint32_t m, out_f, wide;  // wide: y and ldy allow stores of 8 bytes
+    uint32_t parts;           // lp_parts: of tiles, for each group of activation rows
 };
 // four weight rows' sums of activation row r: the bias is added before the one rounding
 __device__ __forceinline__ void lp_store(const LpOut &out, uint32_t r, uint32_t row, ln_f32x4 sum) {
@@ -91,9 +89,10 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
     const uint32_t scale_raw = *scale_at;
     const float scale = bf16_bits_to_f32(scale_raw);
     ln_build_lut<BITS, true>(smem, scale, tid, kLpThreads);
-    const uint32_t units = lp_tiles(n_tiles) * n_cells, u_end = (blockIdx.x + 1u) * units / gridDim.x;
+    const uint32_t u_end = lp_begin(blockIdx.x + 1u, gridDim.x, lp_tiles(n_tiles), n_cells);
+    bool begins = true;  // the run, in this tile
 #pragma unroll 1
-    for (uint32_t u = blockIdx.x * units / gridDim.x; u < u_end;) {
+    for (uint32_t u = lp_begin(blockIdx.x, gridDim.x, lp_tiles(n_tiles), n_cells); u < u_end; begins = false) {
         const uint32_t tile = u / n_cells, c0 = u - tile * n_cells, c1 = min(n_cells, c0 + u_end - u);
         u += c1 - c0;
 
@@ -321,7 +320,8 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
                     lp_store(out, (mb0 + i) * 16u + n, tile * kLpRows + (nw * NI + b) * 16u + 4u * kg, acc[i][b]);
             continue;
         }
-        ln_f32x4 *const to = ws + (((size_t)mg * lp_parts(gridDim.x, lp_tiles(n_tiles)) + blockIdx.x + tile) * kLpWaves + wave) * (MI * NI * 64u) + lane;
+        const uint32_t part = mg * out.parts + lp_part(blockIdx.x, tile, begins, gridDim.x, lp_tiles(n_tiles));
+        ln_f32x4 *const to = ws + ((size_t)part * kLpWaves + wave) * (MI * NI * 64u) + lane;
 #pragma unroll
         for (uint32_t i = 0; i < MI; ++i)
 #pragma unroll
@@ -332,18 +332,17 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
 // y from the sums of a tile's parts, in the columns' order
 __global__ void __launch_bounds__(256)
 k_lanes_prompt_reduce(const ln_f32x4 *__restrict__ ws, uint32_t groups, uint32_t tiles, uint32_t n_cells, uint32_t mi, uint32_t nw, LpOut out) {
-    const uint32_t ni = 8u / nw, mw = 8u / nw, part = kLpWaves * mi * ni * 64u;
+    const uint32_t ni = 8u / nw, mw = 8u / nw, size = kLpWaves * mi * ni * 64u;
     const uint32_t at = blockIdx.x * 256u + threadIdx.x, tile = blockIdx.y, mg = blockIdx.z;
-    const uint32_t units = tiles * n_cells;  // workgroup g has units g * units / groups and on
-    const uint32_t g0 = ((tile * n_cells + 1u) * groups - 1u) / units, g1 = ((tile + 1u) * n_cells * groups - 1u) / units;
-    if (g0 == g1) return;
+    const uint32_t u0 = tile * n_cells, g0 = lp_group_of(u0, groups, tiles, n_cells), g1 = lp_group_of(u0 + n_cells - 1u, groups, tiles, n_cells);
+    if (g0 == g1) return;  // its one workgroup wrote y
     const uint32_t lane = at & 63u, block = at >> 6, b = block % ni, i = block / ni % mi, wave = block / (ni * mi);
     const uint32_t r = ((mg * mw + wave % mw) * mi + i) * 16u + (lane & 15u), row = tile * kLpRows + ((wave / mw) * ni + b) * 16u + 4u * (lane >> 4);
     if (r >= out.m || row >= out.out_f) return;
-    const ln_f32x4 *from = ws + ((size_t)mg * lp_parts(groups, tiles) + g0 + tile) * part + at;
-    ln_f32x4 sum = *from;
+    const ln_f32x4 *const from = ws + (size_t)mg * out.parts * size + at;
+    ln_f32x4 sum = from[(size_t)lp_part(g0, tile, lp_begin(g0, groups, tiles, n_cells) == u0, groups, tiles) * size];
 #pragma unroll 4
-    for (uint32_t g = g0; g < g1; ++g) sum += *(from += part);
+    for (uint32_t g = g0 + 1u; g <= g1; ++g) sum += from[(size_t)g * size];
     lp_store(out, r, row, sum);
 }
 
@@ -366,7 +365,7 @@ static LpPlan lp_plan(const LanesDev &L, int m) {
 }
 
 static size_t lp_x_bytes(const LanesDev &L, const LpPlan &p) { return (size_t)L.n_cells * 16u * p.n_mblk * 1024u; }
-static uint32_t lp_part(const LpPlan &p) { return kLpWaves * p.mi * (8u / p.nw) * 64u; }  // 16-byte units
+static uint32_t lp_part_size(const LpPlan &p) { return kLpWaves * p.mi * (8u / p.nw) * 64u; }  // 16-byte units
 
 // Above 128 rows and 3 * 2^23 weights.  Fewer rows do not hide the decode behind their products, and fewer weights leave a workgroup a
 // few cells, which the pipeline's start and the sums' way through memory outweigh.  us, k_lanes_gemm against this: 5120 x 17408
@@ -378,9 +377,10 @@ bool lanes_prompt_wins(const LanesDev &L, int m) {
            (uint64_t)L.n_cells * 16u * (((uint32_t)m + 15u) / 16u) * 1024u < 1ull << 31;
 }
 
+// (15: to the next whole 16 bytes of whatever address is given)
 size_t lanes_prompt_workspace_bytes(const LanesDev &L, int m) {
     const LpPlan p = lp_plan(L, m);
-    return lp_x_bytes(L, p) + (size_t)p.m_groups * lp_parts(p.groups, lp_tiles(L.n_tiles)) * lp_part(p) * 16u;
+    return 15u + lp_x_bytes(L, p) + (size_t)p.m_groups * lp_parts(p.groups, lp_tiles(L.n_tiles)) * lp_part_size(p) * 16u;
 }
 
 template <int BITS, int MI, int NW>
@@ -405,11 +405,11 @@ static int prompt_rows(const LanesDev &L, const LpPlan &p, const ln_u32x4 *xt, l
 int launch_lanes_prompt(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
                         float *ws, hipStream_t s) {
     const LpPlan p = lp_plan(L, m);
-    ln_u32x4 *const xt = reinterpret_cast<ln_u32x4 *>(ws);
-    ln_f32x4 *const sums = reinterpret_cast<ln_f32x4 *>(reinterpret_cast<uint8_t *>(ws) + lp_x_bytes(L, p));
-    const uint32_t n_kb = L.n_cells * 16u;
+    ln_u32x4 *const xt = reinterpret_cast<ln_u32x4 *>(((uintptr_t)ws + 15u) & ~(uintptr_t)15u);
+    ln_f32x4 *const sums = reinterpret_cast<ln_f32x4 *>(reinterpret_cast<uint8_t *>(xt) + lp_x_bytes(L, p));
+    const uint32_t n_kb = L.n_cells * 16u, tiles = lp_tiles(L.n_tiles);
     hipLaunchKernelGGL(k_lanes_xtile, dim3(n_kb / 4u, (p.n_mblk + 1u) / 2u), dim3(256), 0, s, x, ldx, (uint32_t)m, L.in_f, n_kb, p.n_mblk, xt);
-    const LpOut out{bias, y, ldy, (uint32_t)m, L.out_f, ((uintptr_t)y & 7u) == 0 && ldy % 4 == 0};
+    const LpOut out{bias, y, ldy, (uint32_t)m, L.out_f, ((uintptr_t)y & 7u) == 0 && ldy % 4 == 0, lp_parts(p.groups, tiles)};
     int rc;
     switch (L.bits) {
         case 3: rc = prompt_rows<3>(L, p, xt, sums, out, s); break;
@@ -418,9 +418,8 @@ int launch_lanes_prompt(const LanesDev &L, const uint16_t *x, int m, int64_t ldx
         default: rc = prompt_rows<8>(L, p, xt, sums, out, s); break;
     }
     if (rc != IXH_OK) return rc;
-    const uint32_t tiles = lp_tiles(L.n_tiles);
-    if (p.groups != tiles)  // else each has a tile of its own
-        hipLaunchKernelGGL(k_lanes_prompt_reduce, dim3(lp_part(p) / 256u, tiles, p.m_groups), dim3(256), 0, s, sums, p.groups, tiles, L.n_cells,
+    if (out.parts)
+        hipLaunchKernelGGL(k_lanes_prompt_reduce, dim3(lp_part_size(p) / 256u, tiles, p.m_groups), dim3(256), 0, s, sums, p.groups, tiles, L.n_cells,
                            p.mi, p.nw, out);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }

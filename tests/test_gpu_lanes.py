@@ -185,6 +185,30 @@ def test_many_rows_of_the_largest_weights(oracle, dev, kind, out_f, in_f):
         assert torch.equal(y[0], y[1]) and (y[:, :, out_f:] == 7).all()
 
 
+@pytest.mark.parametrize("kind,out_f,in_f", [("rare", 65536, 520), ("four", 70000, 400), ("real", 8200, 3080), ("four", 1000, 25400)])
+def test_scratch_of_prompts_at_any_address(oracle, dev, kind, out_f, in_f):
+    """Two whole tiles a workgroup (no sums in memory), more tiles than workgroups and shared ones, fewer shared, and several
+    workgroups to a tile: as many bytes as are asked for, at an odd address, hold all that is written."""
+    from ixrun_amd import _lib
+
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    weight = bits_to_bf16(oracle.decode_packed_bf16(p)).to(dev).reshape(out_f, in_f).float()
+    for m in (130, 513):
+        x = activations(m, in_f, seed=m).to(dev)
+        need = lanes.gemm_workspace_bytes(m)
+        ws = torch.full((need + 256,), 0xA5, dtype=torch.uint8, device=dev)
+        y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
+        _lib.check(_lib.lib().ixh_lanes_gemm(C.byref(lanes.struct), x.data_ptr(), in_f, None, m, y.data_ptr(), out_f, ws.data_ptr() + 101,
+                                             need, _lib.current_stream(dev)))
+        assert bool((ws[:101] == 0xA5).all()) and bool((ws[101 + need :] == 0xA5).all())
+        want = (x.float() @ weight.t()).bfloat16()
+        # (see test_many_rows_of_the_largest_weights)
+        assert rel_l2(y.float().cpu().numpy(), want.float().cpu().numpy()) <= 1e-3
+        again = torch.empty_like(y)
+        lanes.gemm(x, again)
+        assert torch.equal(y, again)
+
+
 @pytest.mark.parametrize("out_f,in_f,m", [(4100, 520, 20), (4500, 1536, 130), (20, 33800, 40)])
 def test_many_rows_of_larger_weights(oracle, dev, out_f, in_f, m):
     """Workgroups with several rounds of blocks, and slices of several cells."""

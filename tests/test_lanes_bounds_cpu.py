@@ -1,5 +1,5 @@
-"""What the lane kernels ask for ahead of need stays inside their buffers: the ranges of ``csrc/ixh_lanes_bounds.h`` walked
-on the host (the header is plain C++)."""
+"""What the lane kernels ask for ahead of need stays inside their buffers, and what the prompts' workgroups leave in memory has
+places of its own: the ranges of ``csrc/ixh_lanes_bounds.h`` walked on the host (the header is plain C++)."""
 import ctypes as C
 import os
 import subprocess
@@ -15,6 +15,10 @@ extern "C" void groups(uint32_t first, uint32_t end, uint32_t n, uint32_t *out) 
 }
 extern "C" int whole(uint64_t x, uint32_t in_f, int m, int64_t ldx) { return ixh::ln_whole_pieces(x, in_f, m, ldx); }
 extern "C" uint32_t column(uint32_t col, uint32_t in_f) { return ixh::ln_piece_column(col, in_f); }
+extern "C" uint32_t begin(uint32_t g, uint32_t groups, uint32_t tiles, uint32_t cells) { return ixh::lp_begin(g, groups, tiles, cells); }
+extern "C" uint32_t group_of(uint32_t c, uint32_t groups, uint32_t tiles, uint32_t cells) { return ixh::lp_group_of(c, groups, tiles, cells); }
+extern "C" uint32_t part(uint32_t g, uint32_t tile, int begins, uint32_t groups, uint32_t tiles) { return ixh::lp_part(g, tile, begins, groups, tiles); }
+extern "C" uint32_t parts(uint32_t groups, uint32_t tiles) { return ixh::lp_parts(groups, tiles); }
 """
 
 
@@ -57,3 +61,62 @@ def test_requests_of_the_activations_stay_in_their_row(bounds, in_f):
         for col in range(0, -(-in_f // 512) * 512, 8):
             at = bounds.column(col, in_f)
             assert at % 8 == 0 and at + 8 <= in_f and (at == col or col + 8 > in_f)
+
+
+@pytest.mark.parametrize("cells", [1, 2, 3, 5, 34])
+def test_parts_of_shared_tiles_each_have_a_place(bounds, cells):
+    """Every part of a tile that a workgroup leaves in memory has a place of its own, all places that are asked for are taken but
+    those of runs that happen to begin or end with a tile, and the reader of a tile finds its parts in the order of the columns."""
+    for tiles in (1, 2, 3, 7, 8, 40, 136):
+        for groups in sorted({1, 2, 3, tiles, tiles + 1, 2 * tiles, 2 * tiles - 1, 3 * tiles - 2, 6 * tiles, tiles // 2, tiles // 3 + 1, 61} - {0}):
+            if groups > tiles * cells:
+                continue
+            parts, written, at_an_edge = bounds.parts(groups, tiles), {}, 0
+            of_tile = [[] for _ in range(tiles)]
+            assert bounds.begin(0, groups, tiles, cells) == 0 and bounds.begin(groups, groups, tiles, cells) == tiles * cells
+            for g in range(groups):
+                u0, end = (bounds.begin(k, groups, tiles, cells) for k in (g, g + 1))
+                assert end > u0
+                at_an_edge += u0 % cells == 0
+                u = u0
+                while u < end:
+                    tile, c0 = divmod(u, cells)
+                    c1 = min(cells, c0 + end - u)
+                    if c1 - c0 < cells:
+                        part = bounds.part(g, tile, u == u0, groups, tiles)
+                        assert part < parts and part not in written
+                        written[part] = g
+                        of_tile[tile].append(part)
+                    u += c1 - c0
+            assert parts <= 2 * groups and parts - len(written) <= 2 * at_an_edge
+            for tile, own in enumerate(of_tile):
+                g0, g1 = (bounds.group_of(tile * cells + c, groups, tiles, cells) for c in (0, cells - 1))
+                begins = bounds.begin(g0, groups, tiles, cells) == tile * cells
+                assert own == ([] if g0 == g1 else [bounds.part(g0, tile, begins, groups, tiles)] + list(range(g0 + 1, g1 + 1)))
+
+
+def prompt_bytes(out_f, in_f, rows):
+    """What ixh_lanes_gemm asks for (no memory is read for that)."""
+    from ixrun_amd import _lib
+
+    some = 1 << 12
+    s = _lib.IxhLanes(3, out_f, in_f, some, int(_lib.lib().ixh_lanes_plane_words(out_f, in_f, 3)), some, some, some, 64, some)
+    return int(_lib.lib().ixh_lanes_gemm_workspace_bytes(C.byref(s), rows))
+
+
+@pytest.mark.parametrize("out_f,in_f,rows,parts", [
+    (32768, 4096, 512, 0),  # as many tiles as workgroups
+    (131072, 5120, 512, 0), (131072, 5120, 1024, 0),  # whole tiles for each
+    (5120, 17408, 512, 240),  # six workgroups to a tile
+    (17408, 5120, 512, 256 + 135),  # 256 workgroups share 136 tiles
+    (40000, 5120, 512, 256 + 255),  # and 313
+])
+def test_scratch_of_prompts_is_what_is_written(out_f, in_f, rows, parts):
+    """The activations in the kernel's order and 256 KB for each part of a tile, nothing for tiles that one workgroup finishes
+    (256 CUs: without a GPU the library plans for as many)."""
+    import torch
+
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("figures of 256 CUs")
+    x = -(-in_f // 512) * 512 * rows * 2
+    assert prompt_bytes(out_f, in_f, rows) == 15 + x + parts * 512 * 128 * 4
