@@ -118,7 +118,7 @@ PyObject *forward_many(PyObject *self_, PyObject *arg) {
     shape.back() = self->out_f;
     at::Tensor y, sums;
     int rc;
-    {
+    try {
         pybind11::gil_scoped_release without_gil;
         y = at::empty(shape, x.options());
         const size_t need = self->gemm_workspace_bytes(self->lanes, (int32_t)rows);
@@ -126,6 +126,8 @@ PyObject *forward_many(PyObject *self_, PyObject *arg) {
         rc = self->gemm(self->lanes, static_cast<const uint16_t *>(x.const_data_ptr()), self->in_f, self->bias, (int32_t)rows,
                         static_cast<uint16_t *>(y.data_ptr()), self->out_f, need ? sums.data_ptr() : nullptr, need,
                         c10::hip::getCurrentHIPStream((c10::DeviceIndex)self->device).stream());
+    } catch (const c10::OutOfMemoryError &) {
+        Py_RETURN_NONE;  // nothing has been launched; the caller may have a way without the sums' memory
     }
     if (rc) {
         PyObject *r = PyObject_CallFunction(self->check, "i", rc);

@@ -394,7 +394,14 @@ class StreamingLinear(nn.Module):
             if x2.data_ptr() % 16:
                 x2 = x2.clone()
             y = torch.empty((rows, self.out_features), dtype=torch.bfloat16, device=x.device)
-            self._lanes.gemm(x2, y, self._bias if self._bias_ptr else None)
+            try:
+                self._lanes.gemm(x2, y, self._bias if self._bias_ptr else None)
+            except torch.OutOfMemoryError:
+                if self._w_buf is None:
+                    raise
+                # no room for the slices' sums (128 MiB and the activations at most): the decode buffer is there already
+                del x2, y
+                return self._decode_and_multiply(x)
             if self._bias is not None and not self._bias_ptr:
                 y = y + self._bias.to(y.dtype)
             return y.view(x.shape[:-1] + (self.out_features,))
@@ -418,6 +425,9 @@ class StreamingLinear(nn.Module):
                 if self._bias is not None:
                     y = y + self._bias.to(y.dtype)
                 return y
+        return self._decode_and_multiply(x)
+
+    def _decode_and_multiply(self, x):
         w = self._decode()
         bias = self._bias.to(x.dtype) if self._bias is not None else None
         return gemm_tuning.linear(x, w.to(x.dtype) if w.dtype != x.dtype else w, bias)
@@ -448,7 +458,9 @@ class ResourceScheduler:
     """Memory estimates and a mode recommendation (reference ``ixrun/engine.py:202-235``).
 
     A streaming deploy keeps ``packed_storage_MB``, ``lane_storage_MB`` (the layout that the forwards read; nothing with
-    ``lanes=False``) and ``shared_decode_buf_MB`` on the GPU."""
+    ``lanes=False``) and ``shared_decode_buf_MB`` on the GPU.  With lanes a prompt takes memory for its call besides: its
+    activations once more and, from 129 rows on large layers, up to 128 MiB of sums (less below); where there is no room for
+    them it goes through the decode buffer."""
 
     @staticmethod
     @torch.no_grad()

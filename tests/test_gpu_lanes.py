@@ -359,6 +359,46 @@ def test_prompts_from_native_code(dev, kind):
     assert bool(layer._w_buf.any())
 
 
+@pytest.mark.parametrize("native", [True, False])
+def test_prompts_without_room_for_their_sums_take_the_decode_buffer(oracle, dev, native):
+    """Where the allocator has no room for a prompt's sums (here: a limit on this process) a layer with a decode buffer is served
+    from that, and one without raises."""
+    from ixrun_amd.engine import StreamingLinear
+
+    out_f, in_f, rows = 1000, 25400, 400
+    v, scheme, _ = values("four", out_f, in_f)
+    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    layer = StreamingLinear(p, bias=bias)
+    if not native:
+        layer._native = None
+    layer._set_shared_buf(torch.zeros(p["N"], dtype=torch.bfloat16, device=dev))
+    x = activations(rows, in_f, seed=3).to(dev)
+    want = layer(x).clone()
+    assert not bool(layer._w_buf.any())
+    layer._gemm_ok = False
+    layer(x)  # (the library takes its workspace now)
+    layer._gemm_ok = True
+    layer._w_buf.zero_()
+    total = torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.empty_cache()
+    room = layer._lanes.gemm_workspace_bytes(rows) // 2
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + room) / total, dev)
+        got = layer(x)
+        assert bool(layer._w_buf.any())
+        # the library rounds its product at other places: half a bf16 step on either side
+        assert rel_l2(got.double().cpu().numpy(), want.double().cpu().numpy()) <= 2 ** -8
+        buf = layer._w_buf  # (whose memory would be room)
+        layer._set_shared_buf(None)
+        with pytest.raises(torch.OutOfMemoryError):
+            layer(x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    del buf
+    assert torch.equal(layer(x), want)
+
+
 @pytest.mark.parametrize("in_f,rows", [(1024, 2), (1024, 16), (1004, 5), (1004, 20)])
 def test_calls_that_are_not_plain_keep_the_decode(monkeypatch, dev, in_f, rows):
     """Gradients, forward mode, vmap, autocast and other kinds of tensors: a layer with a decode buffer whose rows went
