@@ -578,13 +578,19 @@ int ixh_lanes_list(const uint16_t *w, const IxhLanes *dst, ixh_stream_t stream) 
     return rc;
 }
 
+static int lanes_status(int rc, const LnScratch &ws, const char *name) {
+    if (rc == IXH_EWORKSPACE) set_error("workspace of %zu bytes needed, %zu given", ws.need, ws.at ? ws.bytes : (size_t)0);
+    if (rc == IXH_ELAUNCH) set_error("%s: launch failed", name);
+    return rc;
+}
+
 size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m) {
     LanesDev d;
     if (to_lanes(lanes, &d, true) || m < 1 || m > 16) return 0;
     // From five rows on, what any count up to 16 takes: a batch that grows makes no caller replace its buffer (a shared one that
     // captured graphs hold is kept for them beside the new one).
-    return m <= 4 ? lanes_rows_workspace_bytes(d, m)
-                  : max(lanes_rows_workspace_bytes(d, m), max(lanes_rows_workspace_bytes(d, 8), lanes_rows_workspace_bytes(d, 16)));
+    if (m <= 4) return lanes_gemv_takes(d, m) ? 0 : lanes_rows_workspace_bytes(d, m);
+    return max(lanes_rows_workspace_bytes(d, m), max(lanes_rows_workspace_bytes(d, 8), lanes_rows_workspace_bytes(d, 16)));
 }
 
 int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,
@@ -595,14 +601,8 @@ int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
     if (m < 1 || m > 16) { set_error("m = %d not in 1..16", m); return IXH_EINVAL; }
     if (!x || !y) { set_error("x or y is NULL"); return IXH_EINVAL; }
     if (m > 1 && (ldx < (int64_t)d.in_f || ldy < (int64_t)d.out_f)) { set_error("ldx or ldy shorter than a row"); return IXH_EINVAL; }
-    const size_t need = lanes_rows_workspace_bytes(d, m);
-    if (need && (!workspace || workspace_bytes < need)) {
-        set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
-        return IXH_EWORKSPACE;
-    }
-    rc = launch_lanes_gemv(d, x, m, ldx, bias, y, ldy, (float *)workspace, (hipStream_t)stream);
-    if (rc == IXH_ELAUNCH) set_error("lanes_gemv: launch failed");
-    return rc;
+    LnScratch ws{(float *)workspace, workspace_bytes, 0};
+    return lanes_status(launch_lanes_gemv(d, x, m, ldx, bias, y, ldy, ws, (hipStream_t)stream), ws, "lanes_gemv");
 }
 
 constexpr int32_t kLanesGemmMost = 4096;
@@ -626,14 +626,8 @@ int ixh_lanes_gemm(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const 
                   d.in_f, (long long)ldx);
         return IXH_EUNSUPPORTED;
     }
-    const size_t need = lanes_gemm_workspace_bytes(d, m);
-    if (need && (!workspace || workspace_bytes < need)) {
-        set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
-        return IXH_EWORKSPACE;
-    }
-    rc = launch_lanes_gemm(d, x, m, ldx, bias, true, y, ldy, (float *)workspace, (hipStream_t)stream);
-    if (rc == IXH_ELAUNCH) set_error("lanes_gemm: launch failed");
-    return rc;
+    LnScratch ws{(float *)workspace, workspace_bytes, 0};
+    return lanes_status(launch_lanes_gemm(d, x, m, ldx, bias, true, y, ldy, ws, (hipStream_t)stream), ws, "lanes_gemm");
 }
 
 static int encode_levels_ok(int32_t n_levels, const int32_t *level_bits) {

@@ -61,26 +61,38 @@ struct LanesDev {
     int bits;
 };
 
+// Scratch that a call was given; a launch that wants more sets `need`, starts nothing and returns IXH_EWORKSPACE.  How the work is
+// cut decides what is needed, and finding the cut takes the host 0.3 to 3 us: it is found once, by the launch that uses it.
+struct LnScratch {
+    float *at;
+    size_t bytes, need;
+    bool holds(size_t n) {
+        need = n;
+        return !n || (at && bytes >= n);
+    }
+};
+
 int launch_lanes_pack(const uint16_t *w, const LanesDev &L, uint32_t *plane, uint32_t *counts, hipStream_t s);
 int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_t *val, hipStream_t s);
-// 1 to 16 rows; five and more, and fewer too long for k_lanes_gemv, go on to launch_lanes_rows, and some of nine and more from there
-// to launch_lanes_gemm
+// 1 to 16 rows; five and more, and fewer too long for k_lanes_gemv (which takes no scratch), go on to launch_lanes_rows, and some of
+// nine and more from there to launch_lanes_gemm
+bool lanes_gemv_takes(const LanesDev &L, int m);
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
-                      int64_t ldy, float *ws, hipStream_t s);
+                      int64_t ldy, LnScratch &ws, hipStream_t s);
 size_t lanes_rows_workspace_bytes(const LanesDev &L, int m);
 int launch_lanes_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
-                      float *ws, hipStream_t s);
+                      LnScratch &ws, hipStream_t s);
 // 17 and more rows (ixh_lanes_gemm.hip), the bias added before the one rounding (once) or after one, then rounded again;
 // IXH_EUNSUPPORTED unless lanes_gemm_aligned:
 // x 16-byte aligned, in_f and ldx multiples of 8, x within 4 GB
 bool lanes_gemm_aligned(const LanesDev &L, const uint16_t *x, int m, int64_t ldx);
 size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m);
 int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once, uint16_t *y,
-                      int64_t ldy, float *ws, hipStream_t s);
+                      int64_t ldy, LnScratch &ws, hipStream_t s);
 // of them, those of many rows and large layers (ixh_lanes_prompt.hip): x as above, the bias added once
 bool lanes_prompt_wins(const LanesDev &L, int m);
 size_t lanes_prompt_workspace_bytes(const LanesDev &L, int m);
 int launch_lanes_prompt(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
-                        float *ws, hipStream_t s);
+                        LnScratch &ws, hipStream_t s);
 
 }  // namespace ixh

@@ -428,21 +428,29 @@ int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
-template <int BITS, int MT, bool WIDE>
-static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
-                             int64_t ldy, hipStream_t s) {
-    // Workgroups of 16, 8 or 4 waves, one, two or four to a CU: the split whose last round of row quads is fullest.
-    const size_t fixed = LnPairs<BITS, WIDE>::kLutBytes + (size_t)MT * (L.n_cells * 1024u + kLnXPad);
-    auto lds_of = [&](uint32_t tiles, uint32_t waves) { return fixed + (size_t)tiles * waves * (MT * 32u); };
-    uint32_t best_waves = 0, best_tiles = 0;
+// Workgroups of 16, 8 or 4 waves, one, two or four to a CU: the split whose last round of row quads is fullest.  No waves where LDS
+// holds none: its first pass, sixteen waves, decides that.
+struct LvSplit { uint32_t waves, tiles; };
+template <int BITS, int MT, bool WIDE> static size_t lv_lds(const LanesDev &L, uint32_t tiles, uint32_t waves) {
+    return LnPairs<BITS, WIDE>::kLutBytes + (size_t)MT * (L.n_cells * 1024u + kLnXPad) + (size_t)tiles * waves * (MT * 32u);
+}
+template <int BITS, int MT, bool WIDE> static LvSplit lv_split(const LanesDev &L) {
+    LvSplit best{};
     uint64_t best_cost = ~0ull;
     for (uint32_t per_cu = 1; per_cu <= 4; per_cu *= 2) {
         const uint32_t waves = 16u / per_cu, slots = ln_cus() * per_cu;
         const uint32_t tiles = (L.n_tiles + slots - 1) / slots;
-        if (lds_of(tiles, waves) * per_cu > kLnLds) break;
+        if (lv_lds<BITS, MT, WIDE>(L, tiles, waves) * per_cu > kLnLds) break;
         const uint64_t cost = (uint64_t)tiles * per_cu;  // row quads a CU works through
-        if (cost < best_cost) { best_cost = cost; best_waves = waves; best_tiles = tiles; }
+        if (cost < best_cost) { best_cost = cost; best = {waves, tiles}; }
     }
+    return best;
+}
+
+template <int BITS, int MT, bool WIDE>
+static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
+                             int64_t ldy, hipStream_t s) {
+    const auto [best_waves, best_tiles] = lv_split<BITS, MT, WIDE>(L);
     // The smaller pair table where rows are too long beside the larger one, and for a few cells a CU, which gain less from it than
     // its 64 KB take to write (5 bits, one row, larger / smaller: 512 x 512 6.6 / 4.2 us, 900 x 3072 with 6 cells a CU 5.0 / 4.4, 2000
     // x 4096 with 16 5.7 / 5.6, 4000 x 3072 with 24 6.4 / 6.4, 5000 x 5120 with 50 7.8 / 8.1).
@@ -463,14 +471,14 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
     // than 160 cells
     const uint32_t inv_cells = L.n_cells == 1 ? 0u : (uint32_t)(((1ull << 32) + L.n_cells - 1u) / L.n_cells);
     hipLaunchKernelGGL((k_lanes_gemv<BITS, MT, WIDE>), dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave << log_waves),
-                       lds_of(best_tiles, 1u << log_waves), s, L.plane, x, L.exc_off, L.scale, shape, L.n_tiles, best_tiles, L.in_f,
+                       (lv_lds<BITS, MT, WIDE>(L, best_tiles, 1u << log_waves)), s, L.plane, x, L.exc_off, L.scale, shape, L.n_tiles, best_tiles, L.in_f,
                        inv_cells, L.list_groups, L.exc_pos, L.exc_val, ldx, bias, y, ldy, L.out_f);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
 template <int BITS>
 static int lanes_gemv_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
-                           int64_t ldy, float *ws, hipStream_t s) {
+                           int64_t ldy, LnScratch &ws, hipStream_t s) {
     int rc = IXH_EUNSUPPORTED;
     if (m == 1) rc = lanes_gemv_launch<BITS, 1, true>(L, x, m, ldx, bias, y, ldy, s);
     else if (m == 2) rc = lanes_gemv_launch<BITS, 2, true>(L, x, m, ldx, bias, y, ldy, s);
@@ -478,8 +486,24 @@ static int lanes_gemv_rows(const LanesDev &L, const uint16_t *x, int m, int64_t 
     return rc == IXH_EUNSUPPORTED ? launch_lanes_rows(L, x, m, ldx, bias, y, ldy, ws, s) : rc;
 }
 
+// whether lanes_gemv_launch finds a split
+template <int BITS> static bool lanes_gemv_fits(const LanesDev &L, int m) {
+    constexpr bool SMALLER = BITS != 4 && BITS != 5;  // (a smaller table of pairs, up to two rows)
+    if (m == 1) return lv_split<BITS, 1, SMALLER>(L).waves != 0;
+    if (m == 2) return lv_split<BITS, 2, SMALLER>(L).waves != 0;
+    return m <= 4 && lv_split<BITS, 4, true>(L).waves != 0;
+}
+bool lanes_gemv_takes(const LanesDev &L, int m) {
+    switch (L.bits) {
+        case 3: return lanes_gemv_fits<3>(L, m);
+        case 4: return lanes_gemv_fits<4>(L, m);
+        case 5: return lanes_gemv_fits<5>(L, m);
+        default: return lanes_gemv_fits<8>(L, m);
+    }
+}
+
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
-                      int64_t ldy, float *ws, hipStream_t s) {
+                      int64_t ldy, LnScratch &ws, hipStream_t s) {
     switch (L.bits) {
         case 3: return lanes_gemv_rows<3>(L, x, m, ldx, bias, y, ldy, ws, s);
         case 4: return lanes_gemv_rows<4>(L, x, m, ldx, bias, y, ldy, ws, s);

@@ -327,10 +327,12 @@ static LgPlan lg_plan(const LanesDev &L, int m) {
     return best;
 }
 
-size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m) {
-    if (lanes_prompt_wins(L, m)) return lanes_prompt_workspace_bytes(L, m);
-    const LgPlan p = lg_plan(L, m);
+static size_t lg_bytes(const LanesDev &L, const LgPlan &p, int m) {
     return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * ((L.n_tiles + 3u) / 4u * 16u) * sizeof(float) : 0;
+}
+
+size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m) {
+    return lanes_prompt_wins(L, m) ? lanes_prompt_workspace_bytes(L, m) : lg_bytes(L, lg_plan(L, m), m);
 }
 
 template <int BITS, int MB, int NB>
@@ -368,16 +370,17 @@ static int gemm_rows(const LanesDev &L, const LgPlan &p, A... a) {
 }
 
 int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once, uint16_t *y,
-                      int64_t ldy, float *ws, hipStream_t s) {
+                      int64_t ldy, LnScratch &ws, hipStream_t s) {
     if (!lanes_gemm_aligned(L, x, m, ldx)) return IXH_EUNSUPPORTED;
     if (lanes_prompt_wins(L, m)) return launch_lanes_prompt(L, x, m, ldx, bias, y, ldy, ws, s);
     const LgPlan p = lg_plan(L, m);
+    if (!ws.holds(lg_bytes(L, p, m))) return IXH_EWORKSPACE;
     if (m == 1) ldx = L.in_f;
     switch (L.bits) {
-        case 3: return gemm_rows<3>(L, p, x, m, ldx, bias, once, y, ldy, ws, s);
-        case 4: return gemm_rows<4>(L, p, x, m, ldx, bias, once, y, ldy, ws, s);
-        case 5: return gemm_rows<5>(L, p, x, m, ldx, bias, once, y, ldy, ws, s);
-        default: return gemm_rows<8>(L, p, x, m, ldx, bias, once, y, ldy, ws, s);
+        case 3: return gemm_rows<3>(L, p, x, m, ldx, bias, once, y, ldy, ws.at, s);
+        case 4: return gemm_rows<4>(L, p, x, m, ldx, bias, once, y, ldy, ws.at, s);
+        case 5: return gemm_rows<5>(L, p, x, m, ldx, bias, once, y, ldy, ws.at, s);
+        default: return gemm_rows<8>(L, p, x, m, ldx, bias, once, y, ldy, ws.at, s);
     }
 }
 

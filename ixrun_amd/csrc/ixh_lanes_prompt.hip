@@ -378,10 +378,10 @@ bool lanes_prompt_wins(const LanesDev &L, int m) {
 }
 
 // (15: to the next whole 16 bytes of whatever address is given)
-size_t lanes_prompt_workspace_bytes(const LanesDev &L, int m) {
-    const LpPlan p = lp_plan(L, m);
+static size_t lp_bytes(const LanesDev &L, const LpPlan &p) {
     return 15u + lp_x_bytes(L, p) + (size_t)p.m_groups * lp_parts(p.groups, lp_tiles(L.n_tiles)) * lp_part_size(p) * 16u;
 }
+size_t lanes_prompt_workspace_bytes(const LanesDev &L, int m) { return lp_bytes(L, lp_plan(L, m)); }
 
 template <int BITS, int MI, int NW>
 static int prompt_launch(const LanesDev &L, const LpPlan &p, const ln_u32x4 *xt, ln_f32x4 *sums, const LpOut &out, hipStream_t s) {
@@ -403,9 +403,10 @@ static int prompt_rows(const LanesDev &L, const LpPlan &p, const ln_u32x4 *xt, l
 }
 
 int launch_lanes_prompt(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
-                        float *ws, hipStream_t s) {
+                        LnScratch &ws, hipStream_t s) {
     const LpPlan p = lp_plan(L, m);
-    ln_u32x4 *const xt = reinterpret_cast<ln_u32x4 *>(((uintptr_t)ws + 15u) & ~(uintptr_t)15u);
+    if (!ws.holds(lp_bytes(L, p))) return IXH_EWORKSPACE;
+    ln_u32x4 *const xt = reinterpret_cast<ln_u32x4 *>(((uintptr_t)ws.at + 15u) & ~(uintptr_t)15u);
     ln_f32x4 *const sums = reinterpret_cast<ln_f32x4 *>(reinterpret_cast<uint8_t *>(xt) + lp_x_bytes(L, p));
     const uint32_t n_kb = L.n_cells * 16u, tiles = lp_tiles(L.n_tiles);
     hipLaunchKernelGGL(k_lanes_xtile, dim3(n_kb / 4u, (p.n_mblk + 1u) / 2u), dim3(256), 0, s, x, ldx, (uint32_t)m, L.in_f, n_kb, p.n_mblk, xt);

@@ -406,16 +406,20 @@ static bool lr_gemm_wins(const LanesDev &L, int m) {
     return L.bits == 3 ? n > 9u << 20 && L.in_f > 2560u : L.in_f <= kLnCols || L.in_f >= 2048u;
 }
 
+static size_t lr_bytes(const LanesDev &L, const LrPlan &p, int m) {
+    return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * L.n_tiles * 4u * sizeof(float) : 0;
+}
+
 size_t lanes_rows_workspace_bytes(const LanesDev &L, int m) {
-    const LrPlan p = lr_plan_of(L, m);
-    const size_t sums = p.slices > 1 ? (size_t)p.slices * (uint32_t)m * L.n_tiles * 4u * sizeof(float) : 0;
+    const size_t sums = lr_bytes(L, lr_plan_of(L, m), m);
     return lr_gemm_wins(L, m) ? max(sums, lanes_gemm_workspace_bytes(L, m)) : sums;
 }
 
 template <int BITS, int MT, bool WIDE>
 static int rows_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
-                       float *ws, hipStream_t s) {
+                       LnScratch &ws, hipStream_t s) {
     const LrPlan p = lr_plan<BITS, MT, WIDE>(L);
+    if (!ws.holds(lr_bytes(L, p, m))) return IXH_EWORKSPACE;
     static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_rows<BITS, MT, WIDE>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
@@ -424,13 +428,13 @@ static int rows_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx,
     const uint32_t shape = (uint32_t)m | log_waves << 5 | (uint32_t)pairs << 8;
     hipLaunchKernelGGL((k_lanes_rows<BITS, MT, WIDE>), dim3(p.slices, p.groups), dim3(kWave * p.waves), p.lds, s, L.plane, x, L.exc_off,
                        L.scale, L.n_cells, L.n_tiles, L.in_f, shape, (L.n_cells / p.slices) << 20 | L.n_cells % p.slices,
-                       (blocks / p.groups) << 24 | blocks % p.groups, L.exc_pos, L.exc_val, ldx, L.out_f, p.x_rows, ws, bias, y, ldy);
-    if (p.slices > 1) return launch_lanes_reduce(ws, p.slices, m, L.out_f, L.n_tiles * 4u, bias, false, y, ldy, s);
+                       (blocks / p.groups) << 24 | blocks % p.groups, L.exc_pos, L.exc_val, ldx, L.out_f, p.x_rows, ws.at, bias, y, ldy);
+    if (p.slices > 1) return launch_lanes_reduce(ws.at, p.slices, m, L.out_f, L.n_tiles * 4u, bias, false, y, ldy, s);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
 int launch_lanes_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
-                      float *ws, hipStream_t s) {
+                      LnScratch &ws, hipStream_t s) {
     if (lr_gemm_wins(L, m) && lanes_gemm_aligned(L, x, m, ldx)) return launch_lanes_gemm(L, x, m, ldx, bias, false, y, ldy, ws, s);
 #define LR_ROWS(B)                                                                                                              \
     (lr_wide<B>(L, m) ? rows_launch<B, 8, (B == 4 || B == 5)>(L, x, m, ldx, bias, y, ldy, ws, s)                                 \

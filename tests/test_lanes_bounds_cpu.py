@@ -95,13 +95,55 @@ def test_parts_of_shared_tiles_each_have_a_place(bounds, cells):
                 assert own == ([] if g0 == g1 else [bounds.part(g0, tile, begins, groups, tiles)] + list(range(g0 + 1, g1 + 1)))
 
 
-def prompt_bytes(out_f, in_f, rows):
-    """What ixh_lanes_gemm asks for (no memory is read for that)."""
+def described(out_f, in_f, bits=3):
+    """A layout to ask sizes of (no memory is read for that)."""
     from ixrun_amd import _lib
 
     some = 1 << 12
-    s = _lib.IxhLanes(3, out_f, in_f, some, int(_lib.lib().ixh_lanes_plane_words(out_f, in_f, 3)), some, some, some, 64, some)
-    return int(_lib.lib().ixh_lanes_gemm_workspace_bytes(C.byref(s), rows))
+    return _lib.IxhLanes(bits, out_f, in_f, some, int(_lib.lib().ixh_lanes_plane_words(out_f, in_f, bits)), some, some, some, 64, some)
+
+
+def prompt_bytes(out_f, in_f, rows):
+    from ixrun_amd import _lib
+
+    return int(_lib.lib().ixh_lanes_gemm_workspace_bytes(C.byref(described(out_f, in_f)), rows))
+
+
+@pytest.mark.parametrize("bits", [3, 4, 5, 8])
+def test_few_rows_ask_for_no_scratch(bits):
+    """One to four rows whose activations fit into LDS whole are summed there; longer rows go in slices, which need scratch as 5 to
+    16 rows do."""
+    from ixrun_amd import _lib
+
+    def need(out_f, in_f, m):
+        return int(_lib.lib().ixh_lanes_gemv_workspace_bytes(C.byref(described(out_f, in_f, bits)), m))
+
+    for out_f, in_f in ((1536, 1536), (256, 17408), (5120, 17408), (17408, 5120)):
+        assert [need(out_f, in_f, m) for m in (1, 2)] == [0, 0]
+        assert need(out_f, in_f, 16) > 0
+    assert need(17408, 5120, 4) == need(1536, 1536, 3) == 0
+    assert all(need(64, 100000, m) > 0 for m in (1, 2, 3, 4))
+
+
+@pytest.mark.parametrize("rows,need", [(1, 0), (4, 0), (8, 1), (16, 1), (100, 1), (512, 1)])
+def test_too_little_scratch_is_refused(rows, need):
+    """With the bytes that the size call names less one, and with none: before anything is launched."""
+    from ixrun_amd import _lib
+
+    L, s, some = _lib.lib(), described(5120, 17408), 1 << 12
+    call, size = (L.ixh_lanes_gemv, L.ixh_lanes_gemv_workspace_bytes) if rows <= 4 else (L.ixh_lanes_gemm, L.ixh_lanes_gemm_workspace_bytes)
+    if 4 < rows <= 16:  # (the size call answers for any count up to sixteen: what this count takes is in the refusal)
+        call = L.ixh_lanes_gemv
+        assert call(C.byref(s), some, 17408, None, rows, some, 5120, None, 0, None) == -4
+        n = int(L.ixh_last_error().split(b" bytes needed")[0].split()[-1])
+        assert 0 < n <= int(L.ixh_lanes_gemv_workspace_bytes(C.byref(s), rows))
+    else:
+        n = int(size(C.byref(s), rows))
+    assert (n > 0) == bool(need)
+    if n:
+        for at, given in ((some, n - 1), (None, n), (None, 0)):
+            assert call(C.byref(s), some, 17408, None, rows, some, 5120, at, given, None) == -4
+            assert b"%d bytes needed, %d given" % (n, given if at else 0) in L.ixh_last_error()
 
 
 @pytest.mark.parametrize("out_f,in_f,rows,parts", [
