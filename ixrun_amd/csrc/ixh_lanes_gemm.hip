@@ -162,7 +162,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         // Rounds that no row has elements for are passed over where lists are short (3 bits, 5120 x 17408 Student-t at 17 / 80 / 128
         // rows 28.8 / 43.7 / 49.5 -> 27.5 / 39.7 / 47.8 us) or a wave has one block (5 bits at 5 % listed, 10240 x 5120 at 40 rows 28.5
         // -> 27.7); with two blocks of 5 bits the branches cost more (100 rows 39.9 -> 40.6).
-        constexpr bool SKIP = BITS <= 4 || NB == 1;
+        constexpr bool SKIP = (BITS <= 4 && MB != 6) || NB == 1;
         uint32_t put[NB][4 * ROUNDS];
         bool any[NB][ROUNDS], more[NB];
 #pragma unroll
