@@ -289,6 +289,56 @@ def test_infinite_activations(oracle, dev, kind, out_f, in_f):
         assert rel_l2(y[fine].numpy(), want[fine].bfloat16().double().numpy()) <= 1e-3
 
 
+def with_infinities(x, w):
+    """In two of three rows an infinity or two, in some a NaN: in columns where a weight row has its largest weight (a listed one, where it
+    has any), in the first and last column, and in the first and last rows of the blocks of 16."""
+    m, in_f = x.shape
+    for j in range(m):
+        if j % 3 == 1:
+            continue
+        largest = int(w[j % w.shape[0]].abs().argmax())
+        x[j, (0, largest, in_f - 1, in_f // 2)[j % 4]] = float("inf") if j % 5 else -float("inf")
+        if j % 4 == 2:
+            x[j, largest] = -float("inf")
+        if j % 7 == 3:
+            x[j, 5] = float("nan")
+    x[m - 1, in_f - 1] = float("inf")
+    return x
+
+
+def same_infinities(y, want):
+    y, want = y.double().cpu(), want.cpu()
+    assert bool(want.isinf().any()) and bool(want.isfinite().any())
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y[y.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    assert rel_l2(y[fine].numpy(), want[fine].bfloat16().double().numpy()) <= 1e-3
+
+
+@pytest.mark.parametrize("kind", ["narrow", "rare", "four", "real", "full_row", "wide"])
+@pytest.mark.parametrize("out_f,in_f", [(67, 1000), (37, 1900), (20, 8003)])
+def test_infinite_activations_of_nine_to_sixteen_rows(oracle, dev, kind, out_f, in_f):
+    """As test_infinite_activations, where the kernel keeps sixteen rows of a column together (rows of one cell's and a few cells'
+    columns, and longer ones of no whole pieces, which no other kernel takes)."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    w = bits_to_bf16(oracle.decode_packed_bf16(p)).reshape(out_f, in_f).double()
+    for m in (9, 16):
+        x = with_infinities(activations(m, in_f, seed=m), w)
+        same_infinities(product(lanes, x.to(dev), out_f, in_f), torch.stack([(w * row.double()).sum(1) for row in x]))
+
+
+@pytest.mark.parametrize("kind,out_f,in_f", [("rare", 24600, 1032), ("real", 8200, 3080), ("full_row", 8200, 3080), ("four", 1000, 25400),
+                                             ("wide", 400, 66000)])
+def test_infinite_activations_of_large_prompts(oracle, dev, kind, out_f, in_f):
+    """The same through the tiles of 128 weight rows: each width of the sums, and a second group of rows."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    w = bits_to_bf16(oracle.decode_packed_bf16(p)).to(dev).reshape(out_f, in_f).double()
+    for m in (129, 300, 520):
+        x = with_infinities(activations(m, in_f, seed=m).to(dev), w)
+        y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
+        lanes.gemm(x, y)
+        same_infinities(y, x.double() @ w.t())
+
+
 @pytest.mark.parametrize("in_f", [1, 3, 7, 8, 9, 15])
 def test_rows_of_a_few_columns(oracle, dev, in_f):
     """Rows shorter than, as long as and just longer than a 16-byte piece."""
@@ -357,6 +407,42 @@ def test_prompts_from_native_code(dev, kind):
     layer._gemm_ok = False
     layer(x)
     assert bool(layer._w_buf.any())
+
+
+@pytest.mark.parametrize("kind,out_f,in_f", [("rare", 24600, 1032), ("real", 8200, 3080)])
+def test_large_prompts_of_a_layer(oracle, dev, kind, out_f, in_f):
+    """Prompts of a layer large enough for tiles of 128 weight rows, with a bias: from native code, from Python, as views, and
+    replayed from a graph between eager calls; the decode buffer stays untouched."""
+    from ixrun_amd.engine import StreamingLinear
+
+    v, scheme, _ = values(kind, out_f, in_f)
+    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    layer, python = StreamingLinear(p, bias=bias), StreamingLinear(p, bias=bias)
+    python._native = None
+    buf = torch.zeros(p["N"], dtype=torch.bfloat16, device=dev)
+    layer._set_shared_buf(buf)
+    python._set_shared_buf(buf)
+    assert layer._native.many_rows == 512
+    weight = bits_to_bf16(oracle.decode_packed_bf16(p)).to(dev).reshape(out_f, in_f).float()
+    wide = activations(512, in_f + 8, seed=3).to(dev)
+    for rows in (129, 300, 512):
+        x = wide[:rows, :in_f].contiguous()
+        assert layer._native.many(x) is not None
+        y = layer(x)
+        # one rounding to bf16 of sums whose fp32 errors are far below it
+        assert rel_l2(y.float().cpu().numpy(), (x.float() @ weight.t() + bias.to(dev).float()).bfloat16().float().cpu().numpy()) <= 1e-3
+        assert torch.equal(y, python(x)) and torch.equal(y, layer(wide[:rows, :in_f]))
+        assert torch.equal(y, layer(x.view(1, rows, in_f))[0])
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            z = layer(x)
+        for seed in (1, 2, 3):
+            x.copy_(activations(rows, in_f, seed=seed))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(z, layer(x))
+    assert not bool(buf.any())
 
 
 @pytest.mark.parametrize("native", [True, False])
