@@ -7,7 +7,7 @@ namespace ixh {
 // k_lanes_gemm<BITS, MB, NB>: up to 16 * MB activation rows at a time, MB <= 8; NB blocks of 16 weight rows a wave (two from
 // MB = 4 on: an activation operand that is read serves both).
 //
-// Bound: a stage's latency (decode, list and products follow one another in a wave, and all waves meet at its end: 3 to 8
+// Bound: a stage's latency (decode, list and products follow one another in a wave, and all waves meet at its end: 4 to 6
 // thousand clocks), then LDS (per 16 x 128 weights a wave reads 4 MB / NB KB of activations, writes and reads 8 KB of weights and
 // looks up 4 KB of pairs). 10240 x 5120 at 55 / 40 / 5 %, 100 rows: 38.9 us with the slices' sums (44.2 when a lane held an
 // element of each of four rows of the list, so that a store of listed elements went to a quarter of the banks), of which the
@@ -161,7 +161,8 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         // is at i ^ q, as the list has it), the quarter (bits 12..14; none of the four where there is no element) ----
         // Rounds that no row has elements for are passed over where lists are short (3 bits, 5120 x 17408 Student-t at 17 / 80 / 128
         // rows 28.8 / 43.7 / 49.5 -> 27.5 / 39.7 / 47.8 us) or a wave has one block (5 bits at 5 % listed, 10240 x 5120 at 40 rows 28.5
-        // -> 27.7); with two blocks of 5 bits the branches cost more (100 rows 39.9 -> 40.6).
+        // -> 27.7); with two blocks of 5 bits the branches cost more (100 rows 39.9 -> 40.6), and so they do at six blocks of activation
+        // rows, which spill with them (3 bits, 96 rows: 10240 x 5120 32.9 -> 34.2, 17408 x 5120 51.2 -> 53.7; 4 bits the same).
         constexpr bool SKIP = (BITS <= 4 && MB != 6) || NB == 1;
         uint32_t put[NB][4 * ROUNDS];
         bool any[NB][ROUNDS], more[NB];

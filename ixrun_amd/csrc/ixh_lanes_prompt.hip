@@ -66,8 +66,10 @@ k_lanes_xtile(const uint16_t *__restrict__ x, int64_t ldx, uint32_t m, uint32_t 
 // activations come from the L2 straight to registers as operands (k_lanes_xtile), two or four steps ahead: they are shared by no other
 // wave of the workgroup, and through LDS they would take its time from the lookups and the weights.  MI x 16 rows by 128 / NW weight
 // rows of sums a wave: 128 registers at 512 rows, so the rest is kept small: operands of weights read one block ahead, listed elements
-// worked out once a cell and kept in LDS, places recomputed.  Requests are never inside a branch or past a way out, else they are all
-// waited for at the join (with the last stage peeled by conditions the same loop took 110 us at 512 rows, and 287 when it spilled).
+// worked out once a cell and kept in LDS, places recomputed.  All the same <BITS, 4, 1>, 385 to 512 rows, has all 256 registers in
+// use and 7 / 14 / 18 / 18 more (at 3 / 4 / 5 / 8 bits; 32 to 76 bytes a lane) in memory; the other forms spill none.  Requests are never
+// inside a branch or past a way out, else they are all waited for at the join (with the last stage peeled by conditions the same loop
+// took 110 us at 512 rows, and a form whose loop spilled its sums 287).
 //
 // Parts of a tile meet in the workspace and k_lanes_prompt_reduce adds them in the columns' order; a workgroup with the whole of a tile
 // writes y itself (32768 x 4096, 512 rows: 160 -> 130 us).
