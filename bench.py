@@ -66,10 +66,10 @@ MEASURED_TRAFFIC_BYTES = {
     "down_proj_5120x17408_m16_student_t_packed": (27677.0 * 2.0 * 1024 + 960.0 * 1024, _TILES, "d56530b1958e0076"),
     "decode_5120x17408_calibrated": (37327.0 * 2.0 * 1024 + 174080.0 * 1024, _DENSE, "931a9c677790f220"),
     "decode_5120x17408_five_level_calibrated": (50960.0 * 2.0 * 1024 + 174080.0 * 1024, _DENSE5, "eb26928c946e5c46"),
-    "prefill_5120x5120_m512_five_level": (50297.9 * 2.0 * 1024 + 30720.0 * 1024,) + _OLD,
+    "prefill_5120x5120_m512_five_level_packed": (50297.9 * 2.0 * 1024 + 30720.0 * 1024,) + _OLD,
     # the three kernels of a step: k_prefill_xtile + k_prefill358 + k_prefill358_reduce
-    "prefill_5120x17408_m512_five_level": ((8716.0 + 68498.0 + 30734.0) * 2.0 * 1024 + (17408.0 + 61606.0 + 5120.0) * 1024,
-                                           _PREFILL, "63398a2e235eb8d3"),
+    "prefill_5120x17408_m512_five_level_packed": ((8716.0 + 68498.0 + 30734.0) * 2.0 * 1024 + (17408.0 + 61606.0 + 5120.0) * 1024,
+                                                  _PREFILL, "63398a2e235eb8d3"),
     # k_decode358_rows<true> (x 2.0 / x 1.0 as above) + the operands and outputs of the library GEMM that
     # torch.cuda.tunable picked (bf16 weight, X, Y: its FETCH_SIZE, 158,001, is weighted for other request sizes than
     # our kernels' and fixes its reads only between 162 and 324 MB)
@@ -400,6 +400,11 @@ def kernel_sources_sha16(files=None):
     return h.hexdigest()[:16]
 
 
+def counted_as(workload, form, unfused=False):
+    """The name that a workload's counter runs are kept under: the kernels differ with the form of the weights that is read."""
+    return workload + ("_unfused" if unfused else "_packed" if form == "packed" else "")
+
+
 def measured_traffic(workload):
     """HBM bytes per launch from the committed counter runs, or None when the kernel's sources have changed since."""
     hit = MEASURED_TRAFFIC_BYTES.get(workload)
@@ -580,10 +585,12 @@ def also_block(dev, args):
                 r["TFLOP_per_s"] = round(flops / (ms * 1e-3) / 1e12, 1)
                 r["frac_mfma"] = round(flops / (ms * 1e-3) / MFMA_BF16_PEAK, 4)
                 # the same step against the HBM roofline: weights as they are read + activations in + outputs out
-                alg_bytes = form_read(layers[0], packed, m)[1] + m * in_f * 2 + m * out_f * 2
+                r["form"], form_bytes = form_read(layers[0], packed, m)
+                alg_bytes = form_bytes + m * in_f * 2 + m * out_f * 2
                 r["frac_hbm"] = round(alg_bytes / (ms * 1e-3) / HBM_PEAK, 4)
-                r["traffic"] = measured_traffic(name if variant == "fused" else name + "_unfused")
-                out.setdefault(name, {})["ixh_gemm" if variant == "fused" else "decode_plus_tuned_library_gemm"] = r
+                r["traffic"] = measured_traffic(counted_as(name, r["form"], variant == "unfused"))
+                path = "decode_plus_tuned_library_gemm" if variant == "unfused" else "ixh_lanes_gemm" if r["form"] == "lanes" else "ixh_gemm"
+                out.setdefault(name, {})[path] = r
             else:
                 r["form"], form_bytes = ("packed", packed["total_bytes"]) if variant != "fused" else form_read(layers[0], packed, m)
                 alg_bytes = form_bytes + m * in_f * 2 + m * out_f * 2
@@ -660,7 +667,7 @@ def main():
     form, form_bytes = form_read(layers[0], packed, m)
     alg_bytes = form_bytes + m * in_f * 2 + m * out_f * 2
     table_bytes = layers[0]._table.numel() * 4 if form == "packed" else 0  # (the lanes need no rank table)
-    counted = args.workload + ("_packed" if form == "packed" and m <= 16 else "")
+    counted = counted_as(args.workload, form)
 
     if args.calibrate_copy:
         src = torch.ones(256 << 20, dtype=torch.uint8, device=dev)
@@ -723,9 +730,10 @@ def main():
         out["roofline"] = {
             "bound": "mfma", "achieved": flops / (ms_per_step * 1e-3) / 1e12, "peak": MFMA_BF16_PEAK / 1e12,
             "unit": "TFLOP/s", "frac": flops / (ms_per_step * 1e-3) / MFMA_BF16_PEAK,
-            "traffic": None if args.unfused else measured_traffic(args.workload),
-            "note": "2*M*N*K flops per launch pair (GEMM + slice reduce); the kernel is bound by the VALU decode "
-                    "that feeds the matrix cores, not by MFMA issue",
+            "traffic": None if args.unfused else measured_traffic(counted),
+            "note": "2*M*N*K flops per step (all its launches); " + (
+                "weights looked up between the products of the tile before" if form == "lanes" else
+                "the kernel is bound by the VALU decode that feeds the matrix cores, not by MFMA issue"),
         }
         out["path"] = ("decode to HBM + library GEMM" if args.unfused else "fused decode + MFMA (ixh_lanes_gemm)" if form == "lanes"
                        else "fused decode + MFMA (ixh_gemm)")

@@ -196,6 +196,19 @@ def test_bench_tables_are_well_formed():
             assert os.path.exists(os.path.join(root, "ixrun_amd", "csrc", f)), (name, f)
 
 
+def test_bench_counter_runs_are_of_the_form_that_is_read():
+    """A product's counters are those of the lanes' kernels under its own name, and of the kernels that read the packed streams
+    under a name of theirs, whatever the number of rows."""
+    bench = load_bench()
+    assert [bench.counted_as("w", form) for form in ("lanes", "packed")] == ["w", "w_packed"]
+    assert bench.counted_as("w", "packed", unfused=True) == "w_unfused"
+    for table in (bench.MEASURED_TRAFFIC_BYTES, bench.MEASURED_INSTRUCTIONS):
+        for name, (_, files, _) in table.items():
+            base = name.removesuffix("_unfused").removesuffix("_packed")
+            if bench.WORKLOADS[base][2] and files:  # (0 rows: decode and encode)
+                assert (name == base) == any("lanes" in f for f in files), name
+
+
 def test_malformed_lane_layouts():
     """Descriptors that a kernel could not read within its buffers are refused on the host: the list is whole groups of 64
     quads, at least one."""
