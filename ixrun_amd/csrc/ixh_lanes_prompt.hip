@@ -36,7 +36,7 @@ __device__ __forceinline__ void lp_store(const LpOut &out, uint32_t r, uint32_t 
     }
 }
 
-// Bound: memory (5120 x 17408 at 512 rows: 36 MB in 7 us).  X [m][in_f] row-major -> operand order: block (kb, mb), 32 columns x 16 rows, is 1 KB, lane l's 16 bytes are row l % 16, columns
+// Bound: memory (5120 x 17408 at 512 rows: 36 MB in 9 us under the profiler).  X [m][in_f] row-major -> operand order: block (kb, mb), 32 columns x 16 rows, is 1 KB, lane l's 16 bytes are row l % 16, columns
 // 8 (l / 16) .. + 7; zeros past the last row and column.  A workgroup writes four column blocks of two row blocks, so that
 // whole lines are read.
 __global__ void __launch_bounds__(256)
@@ -56,9 +56,9 @@ k_lanes_xtile(const uint16_t *__restrict__ x, int64_t ldx, uint32_t m, uint32_t 
 // ---------------------------------------------------------------------------------------------------------------
 // k_lanes_prompt<BITS, MI, NW>: 128 MI / NW activation rows by 128 weight rows a workgroup, over a run of the cells of a tile.
 //
-// Bound: the matrix unit and what stands between two stages.  5120 x 17408 at 512 rows (3 bits): 90 us for the products, 7 for the
-// activations' reordering and 15 for the sums, of which the products alone would take 56 at the rate of a large library product and
-// the sums (64 MB written and read) 13; decode into memory and that library's product took 126.
+// Bound: the matrix unit and what stands between two stages.  5120 x 17408 at 512 rows (3 bits): 99 us a call; one after the other
+// under the profiler 90 to 96 for this kernel, 9 for the activations' reordering and 11 for adding the sums (63 MB read).  The
+// products would take 58 at the rate of a large library product; decode into memory and that library's product took 126.
 //
 // Eight waves decode 128 rows x 128 columns a stage to LDS in operand order, 16 rows each, while they multiply the stage before: the
 // pairs of a wave's next stage are looked up between the products of its first four operands (a decode of its own before the products
@@ -123,6 +123,8 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
                 }
             }
         };
+        // (The list's steps are those of k_lanes_gemm, each kernel with a form of its own: as functions of ixh_lanes_dev.h they left this
+        // one as it is, and k_lanes_gemm<5 | 8, 7 | 8, 2> with 10 to 21 registers in memory.)
         struct Extent { uint32_t first, end; };
         // the lane's place in a list, worked out where it is used: held over the loop it would cost registers that the sums need
         struct Place { uint32_t row, quad, kg; };
@@ -372,8 +374,9 @@ static uint32_t lp_part_size(const LpPlan &p) { return kLpWaves * p.mi * (8u / p
 // Above 128 rows and 3 * 2^23 weights.  Fewer rows do not hide the decode behind their products, and fewer weights leave a workgroup a
 // few cells, which the pipeline's start and the sums' way through memory outweigh.  us, k_lanes_gemm against this: 5120 x 17408
 // (3 bits) 49 / 50 at 128 rows, 71 / 55 at 144, 145 / 100 at 512; 5120 x 5120 28 / 30, 33 / 32, 63 / 53; 5120 x 4096 28 / 32 at 144
-// rows and 41 / 41 at 384; 4096 x 4096 (5 bits) 30 / 30 at 192 rows, 46 / 47 at 512; 2048 x 2048 29 / 36 at 512.  The bounds keep
-// offsets within 32 bits.
+// rows and 41 / 41 at 384; 4096 x 4096 (5 bits) 30 / 30 at 192 rows, 46 / 47 at 512; 2048 x 2048 29 / 36 at 512.  Planes of 4 and 8 bits at
+// 129 / 256 / 512 rows: 5120 x 5120 (4) 32 / 31, 39 / 35, 63 / 52, 17408 x 5120 (4) 79 / 60, 110 / 78, 200 / 115, 5120 x 5120 (8) 30 / 28,
+// 43 / 35, 66 / 52, 12288 x 6144 (8) 61 / 57, 85 / 73, 145 / 107.  The bounds keep offsets within 32 bits.
 bool lanes_prompt_wins(const LanesDev &L, int m) {
     return m > 128 && (uint64_t)L.out_f * L.in_f > 3u << 23 && (uint64_t)lp_tiles(L.n_tiles) * L.n_cells < 1u << 24 &&
            (uint64_t)L.n_cells * 16u * (((uint32_t)m + 15u) / 16u) * 1024u < 1ull << 31;

@@ -3,7 +3,7 @@
 ``StreamingLinear`` keeps a layer's packed streams resident on the GPU and
 serves every forward from them: up to 16 activation rows go through the fused
 decode+GEMV kernel (the bf16 weight never reaches memory), prompts of up to 160
-to 512 rows through a fused decode+GEMM, larger ones are decoded into a shared
+to 1024 rows through a fused decode+GEMM, larger ones are decoded into a shared
 bf16 buffer and multiplied with ``F.linear``.
 ``GraphLinear`` / ``Int8XEngine`` follow the reference's ``ixrun/engine.py``
 (``StreamingLinear`` ``:40-173``, ``GraphLinear`` ``:179-196``,
@@ -54,7 +54,7 @@ MAX_FUSED_ROWS_WITH_BUFFER_DENSE = 16
 # 137 us decode + library GEMM; 17408 x 5120 54 / 60 / 64 us against 120-122 and 87 us.  On 5120 x 5120 the two
 # calls tie with the fused decode+GEMM (37-45 against 44-45 us) and lose to decode + library GEMM (34 us), and three
 # calls for 33 .. 48 rows gain nothing on any shape: large layers and up to 32 rows only.  (A layer with lanes takes
-# them in one pass instead, 5120 x 17408 29-30 us, unless its rows are no whole 16-byte pieces: _lanes_gemm_wins.)
+# them in one pass instead, 5120 x 17408 27-28 us, unless its rows are no whole 16-byte pieces: _lanes_gemm_wins.)
 SPLIT_FUSED_MIN_WEIGHTS = 40_000_000
 # More rows than that: with a shared decode buffer the layer decodes into it and calls the library GEMM
 # (5120 x 5120 five-level on MI355X: 60 us at 32 rows, 84 us at 512); without one it runs the fused
@@ -91,9 +91,9 @@ class StreamingLinear(nn.Module):
     With ``lanes`` the same integers are kept in the lane layout as well
     (``csrc/ixh_lanes.h``; 3.1 to 6.5 bits a weight for the mixes that take 4.0
     to 5.5 packed), which the forwards of up to 16 rows and of most prompts
-    read: one row of 5120 x 17408 takes 14.6 us from it instead of 16.8 (99 %
-    of the weights in level 1), 18.7 instead of 48.7 (55 / 40 / 5 %), five
-    levels 18.7 instead of 86.  It is no part of the state dict.
+    read: one row of 5120 x 17408 takes 13.0 us from it instead of 16.8 (99 %
+    of the weights in level 1), 17.1 instead of 48.7 (55 / 40 / 5 %), five
+    levels 17.1 instead of 86.  It is no part of the state dict.
     """
 
     def __init__(self, packed: dict, bias=None, lanes: bool = True):
@@ -194,23 +194,26 @@ class StreamingLinear(nn.Module):
     def _lanes_gemm_wins(self, rows: int) -> bool:
         """Whether the lanes' decode into matrix-core tiles (``ixh_lanes_gemm``) is the fastest way for a prompt of so many rows.
 
-        MI355X, us, decode + library GEMM or, for tensors almost all level 1, ``ixh_gemm`` before, against this.  5 bits a
-        weight (55 / 40 / 5 %) at 64 / 100 / 160 / 256 rows: 10240 x 5120 61 / 64 / 72 / 82 against 34 / 45 / 59 / 91, 17408 x
-        5120 93 / 100 / 108 / 124 against 58 / 78 / 93 / 146.  3 bits at 64 / 100 / 200 / 256: 10240 x 5120 65 / 66 / 69 / 69
-        against 29 / 35 / 57 / 75, 17408 x 5120 92 / 97 / 107 / 110 against 48 / 55 / 88 / 124.  Below 2**24 weights the decode,
-        the GEMM and the host's way through both weigh more: 12000 x 768 at 256 rows 35 against 29 from a graph, 2048 x 2048
-        23 against 22 (eager: 30 against 22), and up to 2**20 weights 15 against 16 at 512 rows (eager 31 against 19).  Layers
-        of at most 2**18 weights keep decoding into their buffer (12 us against 8), which callers see there.  Planes of 8 bits
-        have no list and are ahead longer than those of 5, whose limits they share (64 / 100 / 160 / 256 rows: 10240 x 5120
-        57 / 61 / 68 / 82 against 27 / 36 / 49 / 72, 17408 x 5120 103 / 106 / 115 / 138 against 49 / 57 / 81 / 121, 4096 x
-        4096 28 / 30 / 38 / 34 against 17 / 22 / 25 / 32).  Rows of up to 256 columns are behind from some 80 rows on where no
-        host time counts (16384 x 256, 100 rows, 16 against 17 from a graph) and ahead eager (30 against 17).
+        MI355X, us from graphs, a layer without lanes (decode + library GEMM or, for tensors almost all level 1, ``ixh_gemm``)
+        against this.  5 bits a weight (55 / 40 / 5 %) at 64 / 100 / 128 / 160 / 256 rows: 10240 x 5120 62 / 64 / 66 / 71 / 84
+        against 35 / 41 / 42 / 50 / 57, 17408 x 5120 90 / 94 / 94 / 101 / 115 against 55 / 65 / 70 / 75 / 85.  3 bits at 64 / 100 /
+        200 / 256: 10240 x 5120 65 / 66 / 70 / 70 against 28 / 35 / 49 / 49, 17408 x 5120 96 / 101 / 111 / 115 against 46 / 53 / 76
+        / 77.  8 bits, which have no list, at 64 / 100 / 160: 10240 x 5120 62 / 62 / 71 against 28 / 35 / 45, 17408 x 5120 102 /
+        106 / 116 against 49 / 55 / 68, 4096 x 4096 30 / 31 / 39 against 17 / 23 / 24.  Below 2**24
+        weights the decode, the GEMM and the host's way through both weigh more: 12000 x 768 at 256 rows 35 against 29, 2048 x 2048
+        23 against 21 (eager: 31 against 20), and up to 2**20 weights 15 against 14 at 512 rows (eager 31 against 13).  Layers of at
+        most 2**18 weights keep decoding into their buffer (12 us at 100 rows; the lanes took 8), which callers see there.  Rows of
+        up to 256 columns: 16384 x 256 at 80 / 100 rows 17 / 17 against 13 / 15 (eager 32 / 31 against 11 / 14).
 
         Above 3 * 2**23 weights and 128 rows the call takes tiles of up to 512 rows, whose decode the products hide: at 192 /
-        256 / 384 / 512 rows 5120 x 17408 (3 bits) 85 / 94 / 118 / 126 by the best other way against 57 / 64 / 81 / 100, 10240 x
-        5120 (5 bits) 80 / 81 / 82 / 92 against 51 / 59 / 69 / 84, 5120 x 5120 53 / 63 / 54 / 58 against 36 / 39 / 46 / 56; at
-        768 rows 10240 x 5120 is behind (103 against 116) and 12288 x 6144 ahead (138 against 128; 1024 rows 154 against 155),
-        5120 x 17408 at 1024 317 against 179."""
+        256 / 384 / 512 rows 5120 x 17408 (3 bits) 88 / 93 / 117 / 125 without lanes against 59 / 69 / 82 / 101, 10240 x 5120 (5
+        bits) 80 / 84 / 81 / 92 against 52 / 56 / 66 / 84, 5120 x 5120 55 / 64 / 50 / 58 against 35 / 38 / 44 / 55.  Above 512 rows
+        only layers of more than 2**26 weights gain whatever the count: 768 / 1024 rows 12288 x 6144 163 / 174 against 136 / 172,
+        17408 x 5120 191 / 225 against 160 / 198, 5120 x 17408 250 / 298 against 157 / 198, 40000 x 2048 194 / 227 against 163 / 211
+        (10240 x 5120 at 768 109 / 107).  Planes of 4 and 8 bits, decode + library against this, at 129 / 256 / 512 rows: 5120 x 5120
+        (4 bits) 48 / 68 / 61 against 32 / 35 / 52, 17408 x 5120 (4 bits) 106 / 119 / 141 against 61 / 78 / 116, 10240 x 5120
+        (8 bits) 67 / 85 / 90 against 40 / 53 / 78, 5120 x 17408 (8 bits) 199 / 249 / 217 against 56 / 72 / 105; at 1024 rows
+        12288 x 6144 161 against 160 (4 bits) and 165 against 159 (8 bits)."""
         n = self.N
         return (self._lanes is not None and self._gemv_flags == 0 and self.in_features % 8 == 0 and n > 1 << 18
                 and rows * self.in_features < 1 << 31
