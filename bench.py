@@ -50,11 +50,14 @@ _ENCODE = ("ixh_encode.hip", "ixh_dev.h")
 _OLD = ((), "measured-on-earlier-sources")  # figures kept for the record; reported as null
 MEASURED_TRAFFIC_BYTES = {
     # k_lanes_gemv; eight rows k_lanes_rows, sixteen with k_lanes_reduce
-    "down_proj_5120x17408_m1_student_t": (17354.8 * 2.0 * 1024 + 16.0 * 1024, _LANES, "026916a4c68e445a"),
-    "down_proj_5120x17408_m1_calibrated": (36911.7 * 2.0 * 1024 + 16.0 * 1024, _LANES, "026916a4c68e445a"),
-    "down_proj_5120x17408_m1_five_level_calibrated": (36913.4 * 2.0 * 1024 + 16.0 * 1024, _LANES, "026916a4c68e445a"),
-    "gate_up_17408x5120_m8_calibrated": (36753.7 * 2.0 * 1024 + 272.0 * 1024, _LANES, "026916a4c68e445a"),
-    "down_proj_5120x17408_m16_student_t": ((20850.3 + 1134.0) * 2.0 * 1024 + (2240.0 + 160.0) * 1024, _LANES, "026916a4c68e445a"),
+    "down_proj_5120x17408_m1_student_t": (17351.2 * 2.0 * 1024 + 16.0 * 1024, _LANES, "d92f0562d9c074fd"),
+    "down_proj_5120x17408_m1_calibrated": (36908.1 * 2.0 * 1024 + 16.0 * 1024, _LANES, "d92f0562d9c074fd"),
+    "down_proj_5120x17408_m1_five_level_calibrated": (36911.6 * 2.0 * 1024 + 16.0 * 1024, _LANES, "d92f0562d9c074fd"),
+    "gate_up_17408x5120_m8_calibrated": (36758.6 * 2.0 * 1024 + 272.0 * 1024, _LANES, "d92f0562d9c074fd"),
+    "down_proj_5120x17408_m16_student_t": ((20848.0 + 1134.0) * 2.0 * 1024 + (2240.0 + 160.0) * 1024, _LANES, "d92f0562d9c074fd"),
+    # k_lanes_xtile, k_lanes_prompt and k_lanes_prompt_reduce
+    "prefill_5120x17408_m512_five_level": ((8714.5 + 56900.5 + 30743.5) * 2.0 * 1024 + (17408.0 + 64800.0 + 5126.5) * 1024,
+                                           _LANES, "d92f0562d9c074fd"),
     "down_proj_5120x17408_m1_student_t_packed": (23032.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "47283b312ef4bb79"),
     "gate_up_17408x5120_m1_student_t_packed": (22935.9 * 2.0 * 1024 + 40.0 * 1024, _ROWS, "47283b312ef4bb79"),
     "attn_proj_5120x5120_m1_student_t_packed": (7135.5 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "47283b312ef4bb79"),
@@ -89,9 +92,9 @@ MEASURED_TRAFFIC_BYTES = {
 # rocprofv3 --pmc run of this script, mean over the launches), gated by the hash of the kernel's sources like the
 # traffic figures.  Reported per weight: vector and LDS instructions x 64 lanes / weights, scalar instructions / weights.
 MEASURED_INSTRUCTIONS = {
-    "down_proj_5120x17408_m1_student_t": ((3880532.0, 1977733.0, 923404.0), _LANES, "026916a4c68e445a"),
-    "down_proj_5120x17408_m1_calibrated": ((5080919.0, 2689316.0, 1016572.0), _LANES, "026916a4c68e445a"),
-    "down_proj_5120x17408_m1_five_level_calibrated": ((5080919.0, 2689316.0, 1016572.0), _LANES, "026916a4c68e445a"),
+    "down_proj_5120x17408_m1_student_t": ((3880532.0, 1977733.0, 923404.0), _LANES, "d92f0562d9c074fd"),
+    "down_proj_5120x17408_m1_calibrated": ((5080919.0, 2689316.0, 1016572.0), _LANES, "d92f0562d9c074fd"),
+    "down_proj_5120x17408_m1_five_level_calibrated": ((5080919.0, 2689316.0, 1016572.0), _LANES, "d92f0562d9c074fd"),
     "down_proj_5120x17408_m1_student_t_packed": ((5734195.0, 4469166.0, 1360042.0), _ROWS, "47283b312ef4bb79"),
     "gate_up_17408x5120_m1_student_t_packed": ((6030194.0, 4450915.0, 1414314.0), _ROWS, "47283b312ef4bb79"),
     "attn_proj_5120x5120_m1_student_t_packed": ((3570752.0, 2281697.0, 593732.0), _ROWS, "47283b312ef4bb79"),
