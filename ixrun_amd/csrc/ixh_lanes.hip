@@ -11,38 +11,48 @@ __device__ __forceinline__ void ln_load(const uint32_t *__restrict__ plane, uint
 // ---------------------------------------------------------------------------------------------------------------
 // k_lanes_gemv<BITS, MT, WIDE>: up to MT activation rows, MT = 1, 2 or 4.
 //
-// Bound: a launch's start-up, HBM and the decode, which overlap in part (17408 x 5120 at 5 bits, 5 % listed, one row, 15.0 us: 10.7
-// without the decode and the list, 11.8 without the list and with all weights in the caches).  A workgroup owns whole row
-// quads, so each output is made in one place (no workspace, no second launch).  Its cells, in memory order, are dealt to its
-// waves in contiguous shares; addresses depend on nothing that is loaded.  The activations are copied to LDS once per
-// workgroup, 16-byte pieces of a 512-column cell at piece ^ (q << 2) so that the sixteen slices of a wave read from
-// different banks.  Products: v_mfma_f32_4x4x4_16b_bf16, one of its sixteen 4 x 4 blocks per slice (weight row = lane
-// % 4, activation row = lane % 4), so a weight costs no product instructions of its own.
+// Bound: a launch's start-up and tail (some 4 us), the memory, then LDS (look-ups, activations, the list's gathers). A workgroup owns
+// whole row quads, so each output is made in one place (no workspace, no second launch).  Its cells are dealt to its waves in runs
+// that go down the row quads column by column: addresses depend on nothing that is loaded, and a cell's activations, read from LDS,
+// serve the cells of a column (in memory order, where each cell read them anew, 5120 x 17408 at 3 bits took 11.5 us for 11.0).  The
+// activations are copied to LDS once per workgroup, 16-byte pieces of a 512-column cell at piece ^ (q << 2) so that the sixteen slices
+// of a wave read from different banks.
+//
+// Products: v_mfma_f32_16x16x32_bf16 with the weights as they lie in the lanes: its column 4 kg + row is a weight row's 8 columns kg of
+// each 32, and its row 4 r + kg is activation row r at the columns kg, so that a lane's sum of its own kg is one of its four results and
+// the twelve others (columns of one kg, activations of another) are thrown away.  A cell's sums over the four kg go to LDS; the row
+// quad's outputs add them up in column order.  Four matrix instructions a cell, up to four activation rows, and no sums in registers
+// over the loop.
 //
 // A wave has two cells in flight, one of them before the activations are there, and the loop over its ten or so cells is short:
-// with four cells ahead and the loop four times as long the first requests kept the activations of the workgroup's later
-// waves waiting, nothing was multiplied for some 5 us, and much of what a launch fetches was instructions (us at 4 / 2 ahead,
-// one row: 17408 x 5120 5 bits 18.5 / 15.8, 4096 x 11008 13.0 / 10.2, 5120 x 5120 9.3 / 8.1, 5120 x 17408 3 bits 13.6 / 12.6;
-// one ahead 15.8, 10.1, 7.8, 12.5, but five layers from a graph 79 against 77).
+// what is asked for early keeps the activations of the workgroup's later waves waiting, and much of what a launch fetches is
+// instructions (us, two / three ahead, one row: 17408 x 5120 5 bits 14.9 / 15.6, 4096 x 11008 9.4 / 9.9, 5120 x 5120 7.2 / 7.8,
+// 5120 x 17408 3 bits 10.4 / 10.2; both cells in front of the activations 2 to 6 % more).
 //
-// Listed elements lie in cell order, so those of a share are one run of quads.  They are taken 64 quads at a time, between the
-// cells so that the one's latencies run under the other's instructions (all behind the cells 17.2 us instead of 16.2): weight
-// less what the plane has there (its sign times the scale; the difference is exact in fp32) times gathered activation, added to
-// the lane's sum of its row. Taking the sign off costs two instructions an element; a plane without it turns an infinite
+// Listed elements: a workgroup's are one run of quads, taken 64 at a time between the cells (two thirds of their 2 us hide there) and
+// dealt to the waves by such groups, wherever the row quads begin in them: weight less what the plane has there (its sign times the
+// scale; the difference is exact in fp32) times gathered activation, once a group, added to the lane's sum of the row quad that the
+// element is of.  (Dealt as the list of the wave's cells, a share was a part of one or two groups on a tensor with few of them, and
+// every wave had some: 5120 x 17408 3 bits 11.0 -> 10.4 us, 17408 x 5120 with four rows 14.4 -> 13.4.)  One group ahead: two
+// ahead 17408 x 5120 5 bits 14.9 for 14.4.  Taking the sign off costs two instructions an element; a plane without it turns an infinite
 // activation in a listed column into NaN.
+//
+// us a layer before / now: 5120 x 17408 3 bits 11.5 / 10.4, 17408 x 5120 5 bits 14.6 / 13.7, 4096 x 11008 9.3 / 8.9, 5120 x 5120 7.8 / 7.3,
+// 17408 x 5120 with two rows at 5 bits 15.9 / 14.7, with four at 3 bits 15.3 / 13.4.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kLnAhead = 2;      // cells in flight
 constexpr uint32_t kLnFirst = 1;      // of these, asked for before the activations are there
-constexpr uint32_t kLnListAhead = 2;  // groups of the list in flight
+constexpr uint32_t kLnListAhead = 1;  // groups of the list in flight
 constexpr uint32_t kLnXAhead = 3;     // 16-byte pieces of the activations a thread asks for before anything else
-constexpr uint32_t kLnXPad = 256;     // bytes behind a row of activations in LDS: zeros (whole turns of the banks)
+constexpr uint32_t kLnXPad = 64;      // bytes behind a row of activations in LDS: zeros
 
 template <int BITS, int MT, bool WIDE>
 __global__ void __launch_bounds__(1024)
 k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
              const uint16_t *__restrict__ scale_at, uint32_t shape, uint32_t all_tiles, uint32_t tiles_per_wg, uint32_t in_f,
-             uint32_t inv_cells, uint32_t list_groups, const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val,
-             int64_t ldx, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, uint32_t out_f) {
+             uint32_t inv_cells, uint32_t inv_tiles, const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val,
+             uint32_t list_groups, int64_t ldx, const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy,
+             uint32_t out_f) {
     extern __shared__ __attribute__((aligned(16))) uint8_t ln_smem[];
     const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)ln_smem;
     // (what the first requests need lies in the arguments that the hardware loads into registers)
@@ -52,10 +62,12 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t t0 = blockIdx.x * tiles_per_wg;
     const uint32_t n_tiles = min(tiles_per_wg, all_tiles - t0);
-    const uint32_t n_seq = n_tiles * C, cell0 = t0 * C;
-    const uint32_t s0 = (wave * n_seq) >> log_waves, s1 = ((wave + 1u) * n_seq) >> log_waves;
+    const uint32_t n_seq = tiles_per_wg * C, cell0 = t0 * C;
+    const uint32_t s0 = ln_share(n_seq, wave, log_waves), s1 = ln_share(n_seq, wave + 1u, log_waves);
     const uint32_t x_at = smem + LnPairs<BITS, WIDE>::kLutBytes, x_row = C * 1024u + kLnXPad, x_pieces = MT * C * 64u;
     float *const parts = reinterpret_cast<float *>(ln_smem + LnPairs<BITS, WIDE>::kLutBytes + MT * x_row);
+    float *const list_parts = parts + n_seq * (MT * 4u);  // of wave w and row quad t at t + w
+    uint32_t *const list_waves = reinterpret_cast<uint32_t *>(list_parts + (tiles_per_wg + n_waves) * (MT * 4u));
 
     auto x_piece = [&](uint32_t e) {
         const uint32_t r = MT == 1 ? 0u : e / (C * 64u), col = (e - r * (C * 64u)) * 8u;
@@ -94,27 +106,35 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
             xv[p] = *reinterpret_cast<const ln_u32x4 *>(x + (at + ln_piece_column((e - row * (C * 64u)) * 8u, in_f)));
         }
     uint32_t buf[kLnAhead][BITS];
-    const uint32_t cell_last = max(cell0 + s1, cell0 + 1u) - 1u;
-#pragma unroll
-    for (uint32_t p = 0; p < kLnFirst; ++p) ln_load<BITS>(plane, min(cell0 + s0 + p, cell_last), lane, buf[p]);
-    // the list's cursor: its range is the listed elements r0 .. r1 - 1 of one row quad within one segment of exc_pos; the end of
-    // the range after it, r2, is asked for a range ahead
-    struct Range { uint32_t seq, cell, cells; };
-    auto l_extent = [&](uint32_t seq, uint32_t cell) {
-        return Range{seq, cell, (uint32_t)min(min(s1 - seq, C - cell), kLnSegCells - cell % kLnSegCells)};
+    // the share's cells, column by column
+    struct At { uint32_t c, t; };
+    auto at_of = [&](uint32_t s) {
+        const uint32_t c = tiles_per_wg == 1 ? s : __umulhi(s, inv_tiles);
+        return At{c, s - c * tiles_per_wg};
     };
-    auto l_after = [&](const Range &r) { return l_extent(r.seq + r.cells, r.cell + r.cells == C ? 0u : r.cell + r.cells); };
-    uint32_t l_tile = C == 1 ? s0 : __umulhi(s0, inv_cells);
-    Range l_now = l_extent(s0, s0 - l_tile * C), l_next = l_after(l_now);
-    uint32_t r0 = exc_off[cell0 + s0], r1 = exc_off[cell0 + l_next.seq], r2 = exc_off[cell0 + l_next.seq + l_next.cells];
-    const uint32_t e_end = exc_off[cell0 + s1];  // behind the share's last listed element
+    At ask = at_of(s0), now = ask;
+    auto load_next = [&](uint32_t (&w)[BITS]) {
+        ln_load<BITS>(plane, cell0 + min(ask.t, n_tiles - 1u) * C + ask.c, lane, w);
+        if (ask.t + 1u < tiles_per_wg) ++ask.t;
+        else if (ask.c + 1u < C) ask = At{ask.c + 1u, 0u};
+    };
+#pragma unroll
+    for (uint32_t p = 0; p < kLnFirst; ++p) load_next(buf[p]);
+    // where the list's ranges begin: a range is what is listed of a row quad within one segment of exc_pos; lane 63 has the end of
+    // the workgroup's last one.  (A vector load, which the barrier does not wait for.)
+    const uint32_t segs = (C + kLnSegCells - 1u) / kLnSegCells, n_ranges = n_tiles * segs;
+    auto ranges_from = [&](uint32_t first) {
+        const uint32_t k = min(first + lane, n_ranges), row = segs == 1u ? k : k / segs;
+        return exc_off[cell0 + (lane == 63u ? n_tiles * C : row * C + (k - row * segs) * kLnSegCells)];
+    };
+    uint32_t begins = ranges_from(0u);
 
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- pair table, zeroed sums and activations to LDS ----
     const float scale = bf16_bits_to_f32(scale_raw);
     ln_build_lut<BITS, WIDE>(smem, scale, tid, n_threads);
-    for (uint32_t e = tid; e < n_tiles * n_waves * (MT * 8u); e += n_threads) parts[e] = 0.0f;
+    for (uint32_t e = tid; e < n_tiles; e += n_threads) list_waves[e] = 0u;
     if (tid < MT * (kLnXPad / 16u))
         *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + tid / (kLnXPad / 16u) * x_row + C * 1024u + tid % (kLnXPad / 16u) * 16u)) =
             ln_u32x4{0, 0, 0, 0};
@@ -130,87 +150,114 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (uint32_t p = kLnFirst; p < kLnAhead; ++p) ln_load<BITS>(plane, min(cell0 + s0 + p, cell_last), lane, buf[p]);
-    // the list's groups, 64 quads each
+    for (uint32_t p = kLnFirst; p < kLnAhead; ++p) load_next(buf[p]);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // the list's groups, 64 quads each, whole ones dealt to the waves
     struct Group { ln_u32x2 pos; uint32_t val; } list[kLnListAhead];
-    const LnGroups groups = ln_groups(r0, e_end, list_groups);
-    const uint32_t g_first = groups.first, n_groups = groups.n;
+    auto begin_of = [&](uint32_t r) { return (uint32_t)__builtin_amdgcn_readlane((int)begins, (int)r); };
+    const uint32_t quads_end = begin_of(63u);
+    const LnGroups all = ln_groups(begin_of(0u), quads_end, list_groups);
+    const uint32_t g_first = all.first + ((wave * all.n) >> log_waves), n_groups = all.first + (((wave + 1u) * all.n) >> log_waves) - g_first;
+    // the range that the first group begins in, its row quad and segment
+    const uint32_t quad_first = max(g_first << 6, begin_of(0u));
+    uint32_t chunk = 0;
+    while (begin_of(62u) <= quad_first && chunk + 62u < n_ranges) {
+        chunk += 62u;
+        begins = ranges_from(chunk);
+    }
+    uint32_t range = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(begins <= quad_first) & 0x7FFFFFFFFFFFFFFEull);
+    uint32_t l_tile = segs == 1u ? chunk + range : (chunk + range) / segs, l_seg = chunk + range - l_tile * segs;
+    uint32_t r0 = begin_of(range), r1 = begin_of(range + 1u);
     auto g_load = [&](uint32_t i) {
-        const uint32_t g = min(g_first + i, groups.last);
+        const uint32_t g = min(g_first + i, all.last);
         return Group{*reinterpret_cast<const ln_u32x2 *>(exc_pos + (size_t)g * 256u + lane * 4u),
                      *reinterpret_cast<const uint32_t *>(exc_val + (size_t)g * 256u + lane * 4u)};
     };
 #pragma unroll
     for (uint32_t p = 0; p < kLnListAhead; ++p) list[p] = g_load(p);
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
     const uint32_t lut_lane = smem + ((lane & ((1u << LnPairs<BITS, WIDE>::kCopies) - 1u)) << 2);
-    const uint32_t q = lane >> 4, kg = (lane >> 2) & 3u, am = min(lane & 3u, (uint32_t)MT - 1u);
+    const uint32_t q = lane >> 4, kg = lane & 3u, am = min((lane >> 2) & 3u, (uint32_t)MT - 1u);
     uint32_t xa[4];
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) xa[i] = x_at + am * x_row + q * 256u + ((i ^ q) << 6) + kg * 16u;
-
-    ln_f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
 
     float ex[MT];  // of the lane's row
 #pragma unroll
     for (int r = 0; r < MT; ++r) ex[r] = 0.0f;
     // sums over the lanes of a row's products, to `parts`: lane l has row l % 4
-    auto put = [&](uint32_t tile, uint32_t half, int r, float v) {
+    auto row_sum = [&](float v) {
         v += ln_dpp<0x124>(v);
         v += ln_dpp<0x128>(v);
         const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
         v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
         const auto g = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
         v = __uint_as_float(g[0]) + __uint_as_float(g[1]);
-        if (lane < 4) parts[((tile * n_waves + wave) * 2u + half) * (MT * 4u) + (uint32_t)r * 4u + lane] = v;
+        return v;
     };
     const uint32_t scale_bits = __float_as_uint(scale) & 0x7FFFFFFFu, x_none = x_at + C * 1024u;
     // one group of listed elements, range by range: the lane has four of its row, quads quad .. quad + 3
     auto list_group = [&](const Group &in, uint32_t i) {
-        const uint32_t g0 = (g_first + i) << 6, quad = g0 + (lane & ~3u);
-        for (;;) {
-            const uint32_t vals = in.val, x_seg = x_at + (l_now.cell / kLnSegCells) * (kLnSegCells * 1024u);
-            uint32_t at[4] = {x_seg + (in.pos[0] & 0xFFFFu), x_seg + (in.pos[0] >> 16), x_seg + (in.pos[1] & 0xFFFFu), x_seg + (in.pos[1] >> 16)};
-            if (C >= kLnSegCells)
+        const uint32_t g0 = (g_first + i) << 6, quad = g0 + (lane & ~3u), vals = in.val;
+        float p[4][MT];
+        for (bool first = true;; first = false) {
+            if (first || C >= kLnSegCells) {  // (positions start over in the next segment)
+                const uint32_t x_seg = x_at + l_seg * (kLnSegCells * 1024u);
+                uint32_t at[4] = {x_seg + (in.pos[0] & 0xFFFFu), x_seg + (in.pos[0] >> 16), x_seg + (in.pos[1] & 0xFFFFu), x_seg + (in.pos[1] >> 16)};
+                if (C >= kLnSegCells)
 #pragma unroll
-                for (int k = 0; k < 4; ++k) at[k] = (vals >> (8 * k)) & 255u ? at[k] : x_none;
-            if (g0 < r0 || g0 + 64u > r1)  // quads outside the range count as if they held no element
+                    for (int k = 0; k < 4; ++k) at[k] = (vals >> (8 * k)) & 255u ? at[k] : x_none;
+                const uint32_t w01 = ln_pack((float)(int)(int8_t)vals * scale, (float)(int)(int8_t)(vals >> 8) * scale);
+                const uint32_t w23 = ln_pack((float)(int)(int8_t)(vals >> 16) * scale, (float)((int)vals >> 24) * scale);
 #pragma unroll
-                for (uint32_t k = 0; k < 4; ++k) at[k] = quad + k - r0 < r1 - r0 ? at[k] : x_none;
-            const uint32_t w01 = ln_pack((float)(int)(int8_t)vals * scale, (float)(int)(int8_t)(vals >> 8) * scale);
-            const uint32_t w23 = ln_pack((float)(int)(int8_t)(vals >> 16) * scale, (float)((int)vals >> 24) * scale);
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t wk = k & 2 ? w23 : w01;
+                    const uint32_t wb = k & 1 ? wk & 0xFFFF0000u : wk << 16;
+                    const float wv = __uint_as_float(wb) - __uint_as_float((wb & 0x80000000u) | scale_bits);  // (no element: times 0)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint32_t wk = k & 2 ? w23 : w01;
-                const uint32_t wb = k & 1 ? wk & 0xFFFF0000u : wk << 16;
-                const float wv = __uint_as_float(wb) - __uint_as_float((wb & 0x80000000u) | scale_bits);  // (no element: times 0)
-#pragma unroll
-                for (int r = 0; r < MT; ++r) {
-                    const uint32_t h = *reinterpret_cast<const LN_LDS(uint16_t) *>((uintptr_t)(at[k] + (uint32_t)r * x_row));
-                    ex[r] = __fmaf_rn(wv, __uint_as_float(h << 16), ex[r]);
+                    for (int r = 0; r < MT; ++r) {
+                        const uint32_t h = *reinterpret_cast<const LN_LDS(uint16_t) *>((uintptr_t)(at[k] + (uint32_t)r * x_row));
+                        p[k][r] = wv * __uint_as_float(h << 16);
+                    }
                 }
             }
-            if (g0 + 64u < r1) break;  // the range goes on in the next group
-            if (l_next.cell == 0 || l_next.seq == s1) {  // the row quad is complete
+            if (g0 < r0 || g0 + 64u > r1) {  // quads of other ranges among them
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int r = 0; r < MT; ++r) ex[r] += quad + k - r0 < r1 - r0 ? p[k][r] : 0.0f;
+            } else {
+#pragma unroll
+                for (int r = 0; r < MT; ++r) ex[r] += (p[0][r] + p[1][r]) + (p[2][r] + p[3][r]);
+            }
+            const bool goes_on = g0 + 64u < r1, row_ends = !goes_on && l_seg + 1u == segs;
+            // all that the wave has of the row quad (nothing may be listed in its other segments)
+            if (row_ends || (goes_on ? i + 1u == n_groups : r1 >= quads_end || (i + 1u == n_groups && r1 == g0 + 64u))) {
 #pragma unroll
                 for (int r = 0; r < MT; ++r) {
-                    put(l_tile, 1u, r, ex[r]);
+                    const float v = row_sum(ex[r]);
+                    if (lane < 4) list_parts[(l_tile + wave) * (MT * 4u) + (uint32_t)r * 4u + lane] = v;
                     ex[r] = 0.0f;
                 }
-                ++l_tile;
+                if (lane == 0) __hip_atomic_fetch_or(list_waves + l_tile, 1u << wave, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
-            if (l_next.seq == s1) break;
-            l_now = l_next;
-            l_next = l_after(l_now);
+            if (goes_on) break;
+            l_tile += row_ends;
+            l_seg = row_ends ? 0u : l_seg + 1u;
             r0 = r1;
-            r1 = r2;
-            r2 = exc_off[cell0 + l_next.seq + l_next.cells];
+            if (r0 >= quads_end) break;
+            if (++range < 62u) {
+                r1 = begin_of(range + 1u);
+            } else {
+                const uint32_t next = l_seg + 1u == segs ? (l_tile + 1u) * C : l_tile * C + (l_seg + 1u) * kLnSegCells;
+                r1 = exc_off[cell0 + next];
+                asm volatile("" : "+s"(r1));  // waited for here: none is in flight where the ways meet
+            }
             if (r0 >= g0 + 64u) break;
         }
     };
 
-    uint32_t c = l_now.cell, tile = l_tile, s = s0, g = 0;
+    uint32_t s = s0, g = 0;
     auto list_next = [&] {
         list_group(list[0], g);
 #pragma unroll
@@ -218,35 +265,40 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         list[kLnListAhead - 1] = g_load(g + kLnListAhead);
         ++g;
     };
+    // an activation operand serves the cells of a column
+    ln_u32x4 xc[4];
+    auto x_read = [&] {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xc[i] = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(xa[i] + now.c * 1024u));
+    };
+    x_read();
+    const bool kg0 = (lane & 4u) != 0, kg1 = (lane & 8u) != 0;
+    uint32_t part_at = (uint32_t)(uintptr_t)(LN_LDS(float) *)parts + s0 * (MT * 16u) + (lane >> 4) * 16u + (lane & 3u) * 4u;
     auto cell = [&](uint32_t (&w)[BITS], bool more) {
         uint32_t o[16];
         ln_decode<BITS, WIDE>(w, lut_lane, scale, o);
-        if (more) ln_load<BITS>(plane, min(cell0 + s + kLnAhead, cell_last), lane, w);
-        const uint32_t x_c = c * 1024u;
+        if (more) load_next(w);
+        ln_f32x4 d = {0, 0, 0, 0};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const ln_u32x4 a = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(xa[i] + x_c));
-            acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(ln_s16x4, ln_u32x2{a[0], a[1]}),
-                                                         __builtin_bit_cast(ln_s16x4, ln_u32x2{o[4 * i], o[4 * i + 1]}), acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(ln_s16x4, ln_u32x2{a[2], a[3]}),
-                                                         __builtin_bit_cast(ln_s16x4, ln_u32x2{o[4 * i + 2], o[4 * i + 3]}), acc1, 0, 0, 0);
-        }
-        ++c;
+        for (int i = 0; i < 4; ++i)
+            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ln_bf16x8, xc[i]),
+                                                        __builtin_bit_cast(ln_bf16x8, ln_u32x4{o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]}), d, 0, 0, 0);
         ++s;
-        if (c == C || s == s1) {
-#pragma unroll
-            for (int r = 0; r < MT; ++r) put(tile, 0u, r, acc0[r] + acc1[r]);
-            acc0 = ln_f32x4{0, 0, 0, 0};
-            acc1 = ln_f32x4{0, 0, 0, 0};
-            c = 0;
-            ++tile;
+        if (++now.t == tiles_per_wg) {
+            now = At{now.c + 1u < C ? now.c + 1u : now.c, 0u};
+            x_read();
         }
+        float v = kg1 ? (kg0 ? d[3] : d[2]) : (kg0 ? d[1] : d[0]);
+        v += ln_dpp<0x124>(v);
+        v += ln_dpp<0x128>(v);
+        if ((lane & 12u) == 0 && lane < MT * 16u) *reinterpret_cast<LN_LDS(float) *>((uintptr_t)part_at) = v;
+        part_at += MT * 16u;
     };
     // Whole turns of the buffers, without a way out in between: with one the compiler takes the last request made before it
     // for the first buffer's and waits for all that is in flight at the top of every turn.
     while (s + kLnAhead <= s1) {
-        // Left alone, the waves of a SIMD are served oldest first and the last one ends long after the first; a wave
-        // that has more cells to go takes precedence.
+        // Left alone, the waves of a SIMD are served oldest first; a wave that has more cells to go takes precedence (3 bits
+        // 10.4 us, 10.9 without; the shares are uneven as well, see ln_share).
         const uint32_t behind = (s1 - s) * 4u / (s1 - s0 + 1u);
         if (behind >= 3u) __builtin_amdgcn_s_setprio(3);
         else if (behind == 2u) __builtin_amdgcn_s_setprio(2);
@@ -270,15 +322,21 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     while (g < n_groups) list_next();
     __syncthreads();
 
-    // ---- outputs: the waves' parts in wave order ----
-    for (uint32_t e = tid; e < n_tiles * 4u * m; e += n_threads) {
-        const uint32_t r = e / (n_tiles * 4u), row = e - r * (n_tiles * 4u), at = t0 * 4u + row;
-        if (at >= out_f) continue;
-        float sum = 0.0f;
-        for (uint32_t w = 0; w < 2u * n_waves; ++w) sum += parts[((row >> 2) * n_waves * 2u + w) * (MT * 4u) + r * 4u + (row & 3u)];
-        uint32_t b = f32_to_bf16_bits(sum);
-        if (bias) b = f32_to_bf16_bits(bf16_bits_to_f32(b) + bf16_bits_to_f32(bias[at]));
-        y[(int64_t)r * ldy + at] = (uint16_t)b;
+    // ---- outputs: a row quad's sums over the columns and the waves' parts of the list ----
+    for (uint32_t t = wave; t < n_tiles; t += n_waves) {
+        const uint32_t part = lane >> 2, at = (t0 + t) * 4u + (lane & 3u);
+        const bool listed = (list_waves[t] >> part) & 1u;
+#pragma unroll
+        for (int r = 0; r < MT; ++r) {
+            float sum = listed ? list_parts[(t + part) * (MT * 4u) + (uint32_t)r * 4u + (lane & 3u)] : 0.0f;
+            for (uint32_t c = part; c < C; c += 16u) sum += parts[(c * tiles_per_wg + t) * (MT * 4u) + (uint32_t)r * 4u + (lane & 3u)];
+            sum = row_sum(sum);
+            if (lane < 4 && at < out_f && (uint32_t)r < m) {
+                uint32_t b = f32_to_bf16_bits(sum);
+                if (bias) b = f32_to_bf16_bits(bf16_bits_to_f32(b) + bf16_bits_to_f32(bias[at]));
+                y[(int64_t)r * ldy + at] = (uint16_t)b;
+            }
+        }
     }
 }
 
@@ -432,7 +490,7 @@ int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_
 // holds none: its first pass, sixteen waves, decides that.
 struct LvSplit { uint32_t waves, tiles; };
 template <int BITS, int MT, bool WIDE> static size_t lv_lds(const LanesDev &L, uint32_t tiles, uint32_t waves) {
-    return LnPairs<BITS, WIDE>::kLutBytes + (size_t)MT * (L.n_cells * 1024u + kLnXPad) + (size_t)tiles * waves * (MT * 32u);
+    return LnPairs<BITS, WIDE>::kLutBytes + (size_t)MT * (L.n_cells * 1024u + kLnXPad) + ((size_t)tiles * (L.n_cells + 1u) + waves) * (MT * 16u) + tiles * 4u;
 }
 template <int BITS, int MT, bool WIDE> static LvSplit lv_split(const LanesDev &L) {
     LvSplit best{};
@@ -470,9 +528,10 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
     // quotients by n_cells as products with 2^32 / n_cells, rounded up: exact below 2^32 / n_cells, and LDS holds no rows of more
     // than 160 cells
     const uint32_t inv_cells = L.n_cells == 1 ? 0u : (uint32_t)(((1ull << 32) + L.n_cells - 1u) / L.n_cells);
+    const uint32_t inv_tiles = best_tiles == 1 ? 0u : (uint32_t)(((1ull << 32) + best_tiles - 1u) / best_tiles);
     hipLaunchKernelGGL((k_lanes_gemv<BITS, MT, WIDE>), dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave << log_waves),
                        (lv_lds<BITS, MT, WIDE>(L, best_tiles, 1u << log_waves)), s, L.plane, x, L.exc_off, L.scale, shape, L.n_tiles, best_tiles, L.in_f,
-                       inv_cells, L.list_groups, L.exc_pos, L.exc_val, ldx, bias, y, ldy, L.out_f);
+                       inv_cells, inv_tiles, L.exc_pos, L.exc_val, L.list_groups, ldx, bias, y, ldy, L.out_f);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 

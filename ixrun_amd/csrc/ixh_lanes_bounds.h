@@ -23,6 +23,15 @@ LN_BOTH LnGroups ln_groups(uint32_t first_quad, uint32_t end_quad, uint32_t grou
     return {first, last < groups ? last : groups - 1u, end_quad > first_quad ? last - first + 1u : 0u};
 }
 
+// A workgroup's cells are dealt to its 2^log_waves waves in runs: wave w has the cells ln_share(n, w) .. ln_share(n, w + 1) - 1.  The
+// first of sixteen waves has 1.47 times the mean, the last one 0.53 times: a SIMD serves the oldest of its waves first, so the last ones
+// have their first cells 1.4 us after the first ones and in even shares end 1.6 to 2 us after them (us a layer, even shares /
+// 1.12 .. 0.88 / 1.23 .. 0.77 / 1.47 .. 0.53 / 1.6 .. 0.4 of the mean: 17408 x 5120 at 5 bits 14.4 / 14.2 / 14.0 / 13.8 / 14.1, 5120 x
+// 5120 7.3 / 7.2 / 7.3 / 7.0 / 7.1, 5120 x 17408 at 3 bits 10.4 / 10.5 / 10.2 / 10.5 / 10.8).
+LN_BOTH uint32_t ln_share(uint32_t n, uint32_t wave, uint32_t log_waves) {
+    return (n * wave * (32u + (1u << log_waves) - wave)) >> (log_waves + 5u);
+}
+
 // Activations: 16-byte pieces of whole rows are asked for before anything else where every row starts 16-byte aligned and
 // has a whole piece; of the pieces past a row's last whole one that one is asked for again.
 LN_BOTH bool ln_whole_pieces(uint64_t x, uint32_t in_f, int m, int64_t ldx) {

@@ -111,6 +111,38 @@ def test_long_rows_and_many_rows(oracle, dev, kind, out_f, in_f):
         check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
 
 
+@pytest.mark.parametrize("at", [5, 32767, 32768, 33799])
+@pytest.mark.parametrize("listed", [1, 16, 17, 33])
+def test_list_of_one_segment_of_long_rows(oracle, dev, at, listed):
+    """The other segment of the rows has nothing listed; the last group ends with the segment or behind it."""
+    out_f, in_f = 1028, 33800  # 257 row quads: two a workgroup
+    v = int8_mix("only_l1", out_f * in_f, seed=6).reshape(out_f, in_f)
+    first = min(at, in_f - 4 * listed) if at != 32767 else 32768 - 4 * listed
+    v[:, first : first + 4 * listed : 4] = 90
+    p, lanes = lay_out_values(packed_from_int8(v.reshape(-1), out_f, in_f), out_f, in_f, dev)
+    assert lanes.bits == 3
+    for m in (1, 2):
+        x = activations(m, in_f, seed=m)
+        check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
+
+
+@pytest.mark.parametrize("kind", ["rare", "real"])
+@pytest.mark.parametrize("out_f", [63488, 70000])
+def test_more_row_quads_than_a_wave_has_lanes(oracle, dev, kind, out_f):
+    """62 and 69 row quads a workgroup, whose lists begin in more places than a wave looks up at once; most have one group in many
+    row quads, or none."""
+    in_f = 40
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    for m in (1, 2, 4):
+        x = activations(m, in_f, seed=m)
+        check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
+    v = int8_mix("only_l1", out_f * in_f, seed=6).reshape(out_f, in_f)
+    v[-300:, 3] = 90  # all that is listed lies in a workgroup's last row quads
+    p, lanes = lay_out_values(packed_from_int8(v.reshape(-1), out_f, in_f), out_f, in_f, dev)
+    x = activations(1, in_f, seed=9)
+    check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
+
+
 @pytest.mark.parametrize("kind", ["rare", "real"])
 @pytest.mark.parametrize("out_f,in_f,m", [(16 * 257 + 3, 1030, 5), (40, 5120, 8), (40, 5121, 8), (40, 10240, 7), (37, 3584, 16), (37, 3586, 9),
                                           (20, 17407, 6), (20, 17409, 12), (3, 520, 16)])

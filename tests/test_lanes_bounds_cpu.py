@@ -15,6 +15,7 @@ extern "C" void groups(uint32_t first, uint32_t end, uint32_t n, uint32_t *out) 
 }
 extern "C" int whole(uint64_t x, uint32_t in_f, int m, int64_t ldx) { return ixh::ln_whole_pieces(x, in_f, m, ldx); }
 extern "C" uint32_t column(uint32_t col, uint32_t in_f) { return ixh::ln_piece_column(col, in_f); }
+extern "C" uint32_t share(uint32_t n, uint32_t wave, uint32_t log_waves) { return ixh::ln_share(n, wave, log_waves); }
 extern "C" uint32_t begin(uint32_t g, uint32_t groups, uint32_t tiles, uint32_t cells) { return ixh::lp_begin(g, groups, tiles, cells); }
 extern "C" uint32_t group_of(uint32_t c, uint32_t groups, uint32_t tiles, uint32_t cells) { return ixh::lp_group_of(c, groups, tiles, cells); }
 extern "C" uint32_t part(uint32_t g, uint32_t tile, int begins, uint32_t groups, uint32_t tiles) { return ixh::lp_part(g, tile, begins, groups, tiles); }
@@ -61,6 +62,16 @@ def test_requests_of_the_activations_stay_in_their_row(bounds, in_f):
         for col in range(0, -(-in_f // 512) * 512, 8):
             at = bounds.column(col, in_f)
             assert at % 8 == 0 and at + 8 <= in_f and (at == col or col + 8 > in_f)
+
+
+@pytest.mark.parametrize("log_waves", [0, 1, 2, 3, 4])
+def test_shares_of_the_cells_follow_one_another(bounds, log_waves):
+    """Each cell in one wave's run, in order, and no wave without one where all others have several."""
+    waves = 1 << log_waves
+    for n in list(range(1, 400)) + [5440, 65535, 5 << 20]:
+        ends = [bounds.share(n, w, log_waves) for w in range(waves + 1)]
+        assert ends[0] == 0 and ends[-1] == n and ends == sorted(ends)
+        assert n < 32 * waves or 0.5 * n <= waves * min(b - a for a, b in zip(ends, ends[1:]))
 
 
 @pytest.mark.parametrize("cells", [1, 2, 3, 5, 34])
