@@ -133,6 +133,14 @@ int ixh_decode_gs(const IxhPacked *packed, const int32_t *prefix, int64_t chunk,
                   int64_t group_size, uint16_t *out_bf16, ixh_stream_t stream);
 
 /*
+ * ixh_decode (group_scales NULL) or ixh_decode_gs of a (3,5,8) tensor of at most 2^22 weights without a rank table, in one
+ * launch: for callers that decode a tensor whose table they do not keep.  IXH_EUNSUPPORTED, and nothing done, for anything else: larger
+ * tensors, other schemes, groups that are no power of two from 32 up, an out_bf16 that is not 16-byte aligned.
+ */
+int ixh_decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, uint16_t *out_bf16,
+                        ixh_stream_t stream);
+
+/*
  * Fused decode + GEMV / skinny GEMM:
  *   y[m, r] = bf16( sum_k f32(x[m, k]) * f32(bf16(f32(v[r, k]) * f32(scale))) ),
  * fp32 accumulation, m < M <= 16; x is bf16 [M, ldx], y is bf16 [M, ldy].

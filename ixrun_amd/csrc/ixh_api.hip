@@ -246,6 +246,25 @@ int ixh_decode_gs(const IxhPacked *packed, const int32_t *prefix, int64_t chunk,
     return decode_any(packed, prefix, chunk, nullptr, out_bf16, GroupScales{group_scales, (uint32_t)group_size}, stream);
 }
 
+int ixh_decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, uint16_t *out_bf16,
+                        ixh_stream_t stream) {
+    Dev d;
+    int rc = to_dev(packed, &d, group_scales == nullptr);
+    if (rc) return rc;
+    if (group_scales && (group_size <= 0 || group_size >= (1ll << 31))) { set_error("group_size %lld out of range", (long long)group_size); return IXH_EINVAL; }
+    if (d.n == 0) return IXH_OK;
+    if (!out_bf16) { set_error("out_bf16 is NULL"); return IXH_EINVAL; }
+    const GroupScales gs{group_scales, group_scales ? (uint32_t)group_size : 0u};
+    const bool forced = g_opt_decode_kernel.load(std::memory_order_relaxed) != kDecodeAuto;  // (the kernels that tests name take a table)
+    if (forced || !decode_counted358_supports(d, out_bf16, gs)) {
+        set_error("decode_unranked: not (3,5,8), more than 2^22 weights, groups that are no power of two from 32 up, or out_bf16 not 16-byte aligned");
+        return IXH_EUNSUPPORTED;
+    }
+    rc = launch_decode_counted358(d, out_bf16, gs, (hipStream_t)stream);
+    if (rc == IXH_ELAUNCH) set_error("decode_unranked: launch failed");
+    return rc;
+}
+
 static int gemv_checks(const Dev &d, int64_t chunk, int32_t m) {
     if (m < 1 || m > 16) { set_error("m = %d not in 1..16", m); return IXH_EINVAL; }
     if (chunk <= 0 || chunk > (int64_t)d.in_f || d.in_f % chunk != 0) {

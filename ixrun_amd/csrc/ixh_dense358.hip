@@ -355,11 +355,16 @@ struct DnFlatSpans {
     }
 };
 
-template <bool GS, class Spans, class Sink, bool TAKE_TURNS = true>
+// ONE_SPAN: the wave has one span, whose ranks are `known`, and there is no table.  (The table is an argument of its own: in a struct
+// the compiler takes its entries by vector loads, and the full decode of 17408 x 5120 takes 95 us instead of 58.)
+struct DnRanks { uint32_t q1a, q1b, q2a, q2b; };  // of levels 1 and 2 at a span's start and end
+
+template <bool GS, class Spans, class Sink, bool TAKE_TURNS = true, bool ONE_SPAN = false>
 __device__ __forceinline__ void dn_walk_spans(const Dev &P, const int32_t *__restrict__ prefix, uint32_t entries,
                                               const uint16_t *__restrict__ group_scales, uint32_t group_shift,
                                               const uint32_t *lut, uint16_t *wc, float scale, uint32_t lane,
-                                              const Spans &spans, Sink &sink, uint32_t wave_turn) {
+                                              const Spans &spans, Sink &sink, uint32_t wave_turn,
+                                              const DnRanks &known = {}) {
     const float m15 = -15.0f * scale, m127 = -127.0f * scale;
     uint32_t *const wc32 = reinterpret_cast<uint32_t *>(wc);
     const uint32_t lut_lane = (lane & 31u) << 2;
@@ -376,15 +381,16 @@ __device__ __forceinline__ void dn_walk_spans(const Dev &P, const int32_t *__res
     // What a span needs from memory before any arithmetic: four table entries (scalars), the lane's bitmap word and
     // its window of each code stream.  They are fetched one span ahead (the table entries two), so that a wave's
     // chain table -> windows -> arithmetic does not wait on memory twice per span.
-    struct Ranks { uint32_t q1a, q1b, q2a, q2b; };
+    using Ranks = DnRanks;
     struct Loads { uint32_t w1; d_u32x4 l1a; uint32_t l1b; d_u32x4 l2a; d_u32x3 l2b; d_u32x4 l3a, l3b; d_u32x2 l3c; uint32_t group_scale; };
     struct Shape { uint32_t p0, n_el, e1, e2, e3; };
     // Codes of a level per lane: enough for all of them, and twice an odd number, so that the lanes' rows of the LDS
     // array start an odd number of dwords apart (no two of 32 neighbouring lanes on one bank).  2, 6, ... 34.
     auto codes_per_lane = [](uint32_t n) { return (((n + 63) / 64 + 1) & ~3u) + 2; };
     auto table_of = [&](const DnSpan &sp) {
-        return Ranks{(uint32_t)prefix[sp.u0], (uint32_t)prefix[sp.u1], (uint32_t)prefix[entries + sp.u0],
-                     (uint32_t)prefix[entries + sp.u1]};
+        if constexpr (ONE_SPAN) return known;
+        else return Ranks{(uint32_t)prefix[sp.u0], (uint32_t)prefix[sp.u1], (uint32_t)prefix[entries + sp.u0],
+                          (uint32_t)prefix[entries + sp.u1]};
     };
     auto shape_of = [&](const DnSpan &sp, const Ranks &q) {
         const uint32_t p0 = sp.p0, n_el = sp.n_el;
@@ -436,7 +442,7 @@ __device__ __forceinline__ void dn_walk_spans(const Dev &P, const int32_t *__res
             else if (pr == 1) __builtin_amdgcn_s_setprio(1);
             else __builtin_amdgcn_s_setprio(2);
         }
-        const Loads in_next = fetch(sp_next, q_next);
+        const Loads in_next = ONE_SPAN ? in_now : fetch(sp_next, q_next);
         const Ranks q_after = table_of(sp_after);
         sink.begin(sp_now);
         const Shape g = shape_of(sp_now, q_now);
@@ -650,6 +656,105 @@ k_decode358_dense(Dev P, const int32_t *__restrict__ prefix, uint32_t n_units, u
     const DnFlatSpans spans{n_units, n_spans, P.n, blockIdx.x * kDnWaves + wave, gridDim.x * kDnWaves};
     DnStoreSink sink{out, wc_all[wave], lane};
     dn_walk_spans<GS>(P, prefix, n_units + 1, group_scales, group_shift, lut, wc_all[wave], scale, lane, spans, sink, wave);
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// The same without a rank table, for tensors of up to 2^22 weights: a workgroup counts the bitmaps in front of its spans itself, at
+// most eight spans, one a wave.  Bound by the latency of its chain (bitmap 0 up to the spans, bitmap 1 up to there, the spans' codes); at
+// 2^22 weights a workgroup reads up to 512 KB of bitmap 0, from the caches, which takes as long as the table's two launches and ends the
+// rule: with group scales, us from a graph, table / without: 256 x 512 9.8 / 5.9, 512 x 1024 10.2 / 6.9, 1024 x 1024 10.6 / 7.2, 1400 x
+// 1500 11.4 / 9.0, 2048 x 2048 12.7 / 11.8 to 12.9; called one by one, where three launches take the host as long, 14.6 / 9.6 up to
+// 1400 x 1500 and 14.5 / 11.8 to 12.9 at 2048 x 2048.
+// ---------------------------------------------------------------------------------------------------------------
+constexpr uint32_t kDnCountedWaves = 16, kDnCountedSpans = 8;
+constexpr uint32_t kDnCountedMost = 256u * kDnCountedSpans * kDnSpan;  // weights
+
+struct DnOneSpan {
+    DnSpan span;
+    __device__ __forceinline__ bool first_span(DnSpan &sp) const { sp = span; return true; }
+    __device__ __forceinline__ bool next(const DnSpan &, DnSpan &) const { return false; }
+};
+template <bool GS>
+__global__ void __launch_bounds__(kWave *kDnCountedWaves)
+k_decode358_counted(Dev P, uint32_t n_spans, uint32_t spans_per_wg, uint16_t *__restrict__ out,
+                    const uint16_t *__restrict__ group_scales, uint32_t group_shift) {
+    __shared__ __attribute__((aligned(16))) uint32_t lut[kDnLutBytes / 4];
+    __shared__ __attribute__((aligned(16))) uint16_t wc_all[kDnCountedSpans][kDnSlots];
+    __shared__ uint32_t front[2][kDnCountedWaves], inside[2][kDnCountedWaves];  // bits in front of the workgroup, of a wave's span
+    constexpr uint32_t kThreads = kWave * kDnCountedWaves, kAhead = 8;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t s0 = blockIdx.x * spans_per_wg, s = s0 + wave, p0 = s * kDnSpan;
+    const bool mine = wave < spans_per_wg && s < n_spans;
+    const uint32_t n_el = mine ? min(kDnSpan, P.n - p0) : 0u;
+    auto rsrc_of = [](const uint32_t *words, uint32_t n) {  // (a word past the end reads as zero)
+        return __builtin_amdgcn_make_buffer_rsrc((void *)words, 0, (int)(min(n, kDnCountedMost / 32u) * 4u), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t b1 = rsrc_of(P.bm[0], P.bm_words[0]), b2 = rsrc_of(P.bm[1], P.bm_words[1]);
+    // set bits in the first `quads` runs of four words, a thread's part of them
+    auto count = [&](const __amdgpu_buffer_rsrc_t &bitmap, uint32_t quads) {
+        uint32_t c = 0;
+        for (uint32_t q = tid; q < quads; q += kThreads * kAhead) {
+            d_u32x4 w[kAhead];
+#pragma unroll
+            for (uint32_t k = 0; k < kAhead; ++k)
+                w[k] = __builtin_amdgcn_raw_buffer_load_b128(bitmap, (int)(q + k * kThreads < quads ? (q + k * kThreads) * 16u : 0x7FFFFFF0u), 0, 0);
+#pragma unroll
+            for (uint32_t k = 0; k < kAhead; ++k) c += __popc(w[k][0]) + __popc(w[k][1]) + __popc(w[k][2]) + __popc(w[k][3]);
+        }
+        return c;
+    };
+    auto wave_sum = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_inclusive(v), 63); };
+    // what the workgroup and its waves counted: bits in front of the wave's span
+    auto in_front = [&](int level) {
+        uint32_t v = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kDnCountedWaves; ++k) v += front[level][k] + (k < wave ? inside[level][k] : 0u);
+        return v;
+    };
+
+    uint32_t w1 = 32 * lane < n_el ? __builtin_amdgcn_raw_buffer_load_b32(b1, (int)((p0 >> 5) * 4u + lane * 4u), 0, 0) : 0u;
+    uint32_t c = count(b1, s0 * (kDnSpan / 128u));
+    const float scale = GS ? 1.0f : bf16_bits_to_f32(*P.scale);
+    for (uint32_t e = tid; e < 64 * 32; e += kThreads) {
+        const uint32_t idx = e >> 5;
+        lut[e] = dn_pack(dequant((int)(idx & 7u) - 3, scale), dequant((int)(idx >> 3) - 3, scale));
+    }
+    const uint32_t n_here = 32 * lane < n_el ? min(32u, n_el - 32 * lane) : 0u;
+    w1 &= (uint32_t)(0xFFFFFFFFull >> (32u - n_here));
+    const uint32_t n1 = wave_sum((uint32_t)__popc(w1));
+    c = wave_sum(c);
+    if (lane == 0) front[0][wave] = c, inside[0][wave] = n1;
+    __syncthreads();
+    const uint32_t q1a = in_front(0);
+
+    // bitmap 1 has a bit for each element that is not in the first level
+    uint32_t ahead = s0 * kDnSpan;
+#pragma unroll
+    for (uint32_t k = 0; k < kDnCountedWaves; ++k) ahead -= front[0][k];
+    c = count(b2, ahead >> 7);
+    if (tid < 4u) {  // the run of four words that the workgroup's first bit lies in
+        const uint32_t word = (ahead >> 7) * 4u + tid, bits = ahead > word * 32u ? min(ahead - word * 32u, 32u) : 0u;
+        c += __popc(__builtin_amdgcn_raw_buffer_load_b32(b2, (int)(word * 4u), 0, 0) & (uint32_t)(0xFFFFFFFFull >> (32u - bits)));
+    }
+    const uint32_t g = p0 - q1a, left = n_el - n1;
+    {
+        const d_u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(b2, (int)(((g >> 5) + lane) * 4u), 0, 0);
+        const uint32_t bits = left > 32u * lane ? min(left - 32u * lane, 32u) : 0u;
+        const uint32_t n2 = wave_sum((uint32_t)__popc(__builtin_amdgcn_alignbit(w[1], w[0], g & 31u) & (uint32_t)(0xFFFFFFFFull >> (32u - bits))));
+        c = wave_sum(c);
+        if (lane == 0) front[1][wave] = c, inside[1][wave] = n2;
+    }
+    __syncthreads();
+    if (!mine) return;
+    const uint32_t q2a = in_front(1);
+    const DnRanks ranks{q1a, q1a + n1, q2a, q2a + inside[1][wave]};
+    DnSpan span{};
+    span.p0 = p0;
+    span.n_el = n_el;
+    DnStoreSink sink{out, wc_all[wave], lane};
+    dn_walk_spans<GS, DnOneSpan, DnStoreSink, true, true>(P, nullptr, 0u, group_scales, group_shift, lut, wc_all[wave], scale, lane,
+                                                          DnOneSpan{span}, sink, wave, ranks);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -950,6 +1055,20 @@ int launch_decode_dense358(const Dev &P, const int32_t *prefix, uint16_t *o16, G
     else
         hipLaunchKernelGGL(k_decode358_dense<false>, dim3(blocks), dim3(kWave * kDnWaves), 0, s, P, prefix, n_units, n_spans, o16,
                            (const uint16_t *)nullptr, 0u);
+    return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
+}
+
+bool decode_counted358_supports(const Dev &P, const uint16_t *o16, GroupScales gs) {
+    return P.n <= kDnCountedMost && decode_dense358_supports(P, kFastChunk, nullptr, o16, gs);
+}
+
+int launch_decode_counted358(const Dev &P, uint16_t *o16, GroupScales gs, hipStream_t s) {
+    const uint32_t n_spans = (P.n + kDnSpan - 1) / kDnSpan, per_wg = (n_spans + 255u) / 256u;
+    const dim3 grid((n_spans + per_wg - 1u) / per_wg), block(kWave * kDnCountedWaves);
+    if (gs.fp16)
+        hipLaunchKernelGGL(k_decode358_counted<true>, grid, block, 0, s, P, n_spans, per_wg, o16, gs.fp16, (uint32_t)__builtin_ctz(gs.group));
+    else
+        hipLaunchKernelGGL(k_decode358_counted<false>, grid, block, 0, s, P, n_spans, per_wg, o16, (const uint16_t *)nullptr, 0u);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 

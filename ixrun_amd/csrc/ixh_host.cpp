@@ -221,6 +221,7 @@ struct Library {
     decltype(&ixh_prefix_build_ws) prefix_build;
     decltype(&ixh_decode) decode;
     decltype(&ixh_decode_gs) decode_gs;
+    decltype(&ixh_decode_unranked) decode_unranked;
     decltype(&ixh_encode_workspace_bytes) encode_workspace_bytes;
     decltype(&ixh_encode_scan_counts) encode_scan;
     decltype(&ixh_encode_wait) encode_wait;
@@ -241,20 +242,21 @@ bool checked(int rc) {
     return r != nullptr;
 }
 
-// bind(prefix_entries, prefix_workspace_bytes, prefix_build_ws, decode, decode_gs, encode_workspace_bytes,
+// bind(prefix_entries, prefix_workspace_bytes, prefix_build_ws, decode, decode_gs, decode_unranked, encode_workspace_bytes,
 // encode_scan_counts, encode_wait, encode_pack, check): addresses, and what raises for a negative code
 PyObject *bind(PyObject *, PyObject *args) {
-    PyObject *f[9], *check;
-    if (!PyArg_ParseTuple(args, "OOOOOOOOOO", &f[0], &f[1], &f[2], &f[3], &f[4], &f[5], &f[6], &f[7], &f[8], &check)) return nullptr;
+    PyObject *f[10], *check;
+    if (!PyArg_ParseTuple(args, "OOOOOOOOOOO", &f[0], &f[1], &f[2], &f[3], &f[4], &f[5], &f[6], &f[7], &f[8], &f[9], &check)) return nullptr;
     entry(library.prefix_entries, f[0]);
     entry(library.prefix_workspace_bytes, f[1]);
     entry(library.prefix_build, f[2]);
     entry(library.decode, f[3]);
     entry(library.decode_gs, f[4]);
-    entry(library.encode_workspace_bytes, f[5]);
-    entry(library.encode_scan, f[6]);
-    entry(library.encode_wait, f[7]);
-    entry(library.encode_pack, f[8]);
+    entry(library.decode_unranked, f[5]);
+    entry(library.encode_workspace_bytes, f[6]);
+    entry(library.encode_scan, f[7]);
+    entry(library.encode_wait, f[8]);
+    entry(library.encode_pack, f[9]);
     if (PyErr_Occurred()) return nullptr;
     Py_INCREF(check);
     Py_XSETREF(library.check, check);
@@ -311,7 +313,7 @@ bool describe(PyObject *level_bits, long long out_f, long long in_f, PyObject *b
 }
 
 // decode(level_bits, out_f, in_f, bitmaps, streams, scale, table, group_scales, group_size): the bf16 weight, by units of
-// 512; without a rank table one is built, with group scales (fp16, in place of `scale`) they are used.  Of tensors on the
+// 512; without a rank table small (3,5,8) tensors do without and for others one is built, with group scales (fp16, in place of `scale`) they are used.  Of tensors on the
 // current device.
 // 2048 x 2048 with a table: 9 us of host time (17 from Python).
 PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
@@ -346,17 +348,22 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
         const auto options = at::TensorOptions().device(c10::Device(c10::kCUDA, (c10::DeviceIndex)device));
         ixh_stream_t stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
         w = at::empty({out_f, in_f}, options.dtype(at::kBFloat16));
-        if (!given) {
+        uint16_t *out = static_cast<uint16_t *>(w.data_ptr());
+        const uint16_t *of_groups = scales ? static_cast<const uint16_t *>(scales->const_data_ptr()) : nullptr;
+        rc = given ? IXH_EUNSUPPORTED : library.decode_unranked(&p, of_groups, group, out, stream);
+        const bool ranked = rc == IXH_EUNSUPPORTED;
+        if (ranked) rc = IXH_OK;
+        if (ranked && !given) {
             const size_t bytes = library.prefix_workspace_bytes(n, kUnit, p.n_levels);
             table = at::empty({rows * entries + (int64_t)bytes / 4}, options.dtype(at::kInt));  // and the scratch
             int32_t *ranks = static_cast<int32_t *>(table.data_ptr());
             rc = library.prefix_build(&p, kUnit, ranks, ranks + rows * entries, bytes, stream);
         }
-        const int32_t *ranks = static_cast<const int32_t *>((given ? *given : table).const_data_ptr());
-        uint16_t *out = static_cast<uint16_t *>(w.data_ptr());
-        if (!rc)
-            rc = scales ? library.decode_gs(&p, ranks, kUnit, static_cast<const uint16_t *>(scales->const_data_ptr()), group, out, stream)
+        if (ranked && !rc) {
+            const int32_t *ranks = static_cast<const int32_t *>((given ? *given : table).const_data_ptr());
+            rc = scales ? library.decode_gs(&p, ranks, kUnit, of_groups, group, out, stream)
                         : library.decode(&p, ranks, kUnit, nullptr, out, stream);
+        }
     }
     if (!checked(rc)) return nullptr;
     return THPVariable_Wrap(std::move(w));

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import bf16_bits
+from helpers import bf16_bits, int8_mix, packed_from_int8
 from test_ixgs_cpu import heavy_tail
 
 pytestmark = pytest.mark.gpu
@@ -82,6 +82,67 @@ def test_decode_hand_built_tiers(oracle, dev, decoder, mix, shape, group):
     p = packed_from_ints(oracle, q, scales, shape[0], shape[1], group)
     got = ixgs.decode_weight_triton(p, dev)
     assert np.array_equal(bf16_bits(got).reshape(-1), oracle.gs_dequant_bf16(q, scales, group))
+
+
+def on_device(p, dev):
+    return {k: v.to(dev) if isinstance(v, torch.Tensor) else v for k, v in p.items()}
+
+
+@pytest.mark.parametrize("mix", ["only_tier1", "only_tier2", "only_tier3", "all_tiers", "tier2_first"])
+@pytest.mark.parametrize("n", [1, 31, 32, 2047, 2048, 2049, 2048 * 256, 2048 * 256 + 1, 2048 * 1500 + 77, (1 << 22) - 5, 1 << 22])
+def test_decode_without_a_table(oracle, dev, mix, n):
+    """One launch, whose workgroups count the bitmaps in front of them: the edges of a word, a span, a span a workgroup, and the
+    largest size; bitmap 1 empty, full and of its own density."""
+    from ixrun_amd import _lib, ixgs
+    import ctypes as C
+
+    rng = np.random.default_rng(n)
+    q = {"only_tier1": rng.integers(-3, 5, size=n), "only_tier2": rng.choice([-15, -4, 5, 16], size=n),
+         "only_tier3": rng.choice([-127, -16, 17, 128], size=n), "all_tiers": rng.integers(-3, 5, size=n),
+         "tier2_first": rng.integers(-3, 5, size=n)}[mix].astype(np.int16)
+    if mix == "all_tiers":
+        r = rng.random(n)
+        q[r < 0.45] = rng.integers(-15, 17, size=int((r < 0.45).sum()))
+        q[r < 0.05] = rng.integers(-127, 129, size=int((r < 0.05).sum()))
+    if mix == "tier2_first":
+        q[: n // 3] = 16
+        q[n // 3 : n // 3 + 5] = 128
+    scales = (rng.random(-(-n // 64)).astype(np.float32) * 0.01 + 1e-4).astype(np.float16).view(np.uint16)
+    p = on_device(packed_from_ints(oracle, q, scales, 1, n, 64), dev)
+    want = oracle.gs_dequant_bf16(q, scales, 64)
+    dp = _lib.DevicePacked((3, 5, 8), 1, n, [p["b1"], p["b2"]], [p["l1"], p["l2"], p["l3"]], None)
+    out = torch.full((n + 8,), 7.0, dtype=torch.bfloat16, device=dev)
+    _lib.check(_lib.lib().ixh_decode_unranked(C.byref(dp.struct), p["group_scales"].data_ptr(), 64, out.data_ptr(), _lib.current_stream(dev)))
+    assert np.array_equal(bf16_bits(out)[:n], want) and bool((out[n:] == 7.0).all())
+    assert np.array_equal(bf16_bits(ixgs.decode_weight_triton(p)).reshape(-1), want)
+
+
+@pytest.mark.parametrize("kind", ["only_l1", "no_l3", "no_l2", "only_l3", "rare_other"])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 683), (33, 1000), (700, 1031)])
+def test_per_tensor_decode_without_a_table(oracle, dev, kind, shape):
+    from ixrun_amd import _lib, decode_weight_triton
+    import ctypes as C
+
+    out_f, in_f = shape
+    p = packed_from_int8(int8_mix(kind, out_f * in_f, seed=3), out_f, in_f)
+    want = oracle.decode_packed_bf16(p).reshape(-1)
+    dp = _lib.DevicePacked.from_dict(p, dev)
+    out = torch.empty(out_f * in_f, dtype=torch.bfloat16, device=dev)
+    _lib.check(_lib.lib().ixh_decode_unranked(C.byref(dp.struct), None, 0, out.data_ptr(), _lib.current_stream(dev)))
+    assert np.array_equal(bf16_bits(out), want)
+    assert np.array_equal(bf16_bits(decode_weight_triton(p)).reshape(-1), want)
+
+
+@pytest.mark.parametrize("n,group,code", [((1 << 22) + 1, 64, -2), (4096, 48, -2), (4096, 16, -2), (4096, 0, -1)])
+def test_decode_without_a_table_refuses_the_rest(oracle, dev, n, group, code):
+    from ixrun_amd import _lib
+    import ctypes as C
+
+    p = on_device(packed_from_ints(oracle, np.zeros(n, dtype=np.int16), np.ones(n, dtype=np.uint16), 1, n, group), dev)
+    dp = _lib.DevicePacked((3, 5, 8), 1, n, [p["b1"], p["b2"]], [p["l1"], p["l2"], p["l3"]], None)
+    out = torch.full((n,), 7.0, dtype=torch.bfloat16, device=dev)
+    assert _lib.lib().ixh_decode_unranked(C.byref(dp.struct), p["group_scales"].data_ptr(), group, out.data_ptr(), _lib.current_stream(dev)) == code
+    assert bool((out == 7.0).all())
 
 
 def test_linear_and_deploy(oracle, dev):
