@@ -7,23 +7,27 @@ namespace ixh {
 // k_lanes_gemm<BITS, MB, NB>: up to 16 * MB activation rows at a time, MB <= 8; NB blocks of 16 weight rows a wave (two from
 // MB = 4 on: an activation operand that is read serves both).
 //
-// Bound: a stage's latency (decode, list and products follow one another in a wave, and all waves meet at its end: 4 to 6
-// thousand clocks), then LDS (per 16 x 128 weights a wave reads 4 MB / NB KB of activations, writes and reads 8 KB of weights and
-// looks up 4 KB of pairs). 10240 x 5120 at 55 / 40 / 5 %, 100 rows: 38.9 us with the slices' sums (44.2 when a lane held an
-// element of each of four rows of the list, so that a store of listed elements went to a quarter of the banks), of which the
-// products are 11 (the matrix unit is busy for 12 % of it); 74.3 for the decode to memory and the library's
-// GEMM. A wave takes 16 weight rows x 128 columns a stage: it decodes them to its own 4 KB of LDS in operand order, stores
-// the listed elements over their places and reads the operands back.  All waves of the workgroup are in the same 128
-// columns, whose activations one copy in LDS
-// serves (in operand order, two stages of it: the next one is fetched during the multiply), so a weight is decoded
-// once per 128 activation rows and never reaches memory.  One barrier a stage, which waits for LDS only: codes
-// and list are asked for one cell ahead.
+// Bound: a stage's parts, which follow one another in a wave, while all waves meet at its end, and LDS under them.  10240 x 5120 at 55 /
+// 40 / 5 %, 100 rows, clocks a stage of a wave before listed elements were stored as they are now: decode and its stores 2000, listed
+// elements 2000, activations to LDS 500, products 1500, barrier 1000, of a stage's list 500; 6000 before the first stage and 6000 for
+// the sums behind the last; no unit of the CU is busy for more than half of it (LDS 4000 of 7900 a stage).  37.6 us with the slices'
+// sums (44.2 when a lane held an element of each of four rows of the list, so that a store of listed elements went to a quarter of the
+// banks, 39.0 with a branch around each such store); 74.3 for the decode to memory and the library's GEMM.  Looking up the next stage's
+// weights between the products of this one changes nothing, nor do two workgroups of half the size on a CU; activations straight from
+// the L2 as operands take twice as long.  A wave takes 16 weight rows x 128 columns a stage: it decodes them to its own 4 KB of LDS in
+// operand order, stores the listed elements over their places and reads the operands back.  All waves of the workgroup are in the same
+// 128 columns, whose activations one copy in LDS serves (in operand order, two stages of it: the next one is fetched during the
+// multiply), so a weight is decoded once per 128 activation rows and never reaches memory.  One barrier a stage, which waits for LDS
+// only: codes and list are asked for one cell ahead.
 //
 // A workgroup owns a slice of the columns (whole cells) of a run of 16-row blocks, sixteen at most at a time; the slices' sums
 // meet in the workspace and launch_lanes_reduce adds them in slice order.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kLgBlocks = 16;  // of 16 weight rows, in work at a time
-constexpr uint32_t kLgTileBytes = 4096;
+constexpr uint32_t kLgTile = 4096;
+// whether a store of a listed element has a branch around it; otherwise what is not to be stored goes to a dword a lane behind the tile
+template <int BITS, int MB> constexpr bool kLgBranch = MB == (BITS <= 4 ? 6 : 5);
+template <int BITS, int MB> constexpr uint32_t kLgTileBytes = kLgTile + (kLgBranch<BITS, MB> ? 0u : 256u);
 constexpr uint32_t kLgMost = 8;  // blocks of 16 activation rows
 
 __device__ __forceinline__ void lg_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -37,6 +41,8 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
              uint16_t *__restrict__ y, int64_t ldy) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lg_smem[];
     using P = LnPairs<BITS, false>;
+    constexpr bool BRANCH = kLgBranch<BITS, MB>;
+    constexpr uint32_t kTile = kLgTileBytes<BITS, MB>;
     constexpr uint32_t kThreads = kLgBlocks / NB * kWave;
     const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)lg_smem;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, n = lane & 15u, kg = lane >> 4;
@@ -49,10 +55,10 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     const uint32_t rounds = (b1 - b0 + kLgBlocks - 1u) / kLgBlocks;
     const uint32_t at_once = (b1 - b0 + rounds - 1u) / rounds;  // blocks of a round (the last one may have fewer)
     const uint32_t total = rounds * len;
-    const uint32_t tile_at = smem + P::kLutBytes + wave * (NB * kLgTileBytes);
+    const uint32_t tile_at = smem + P::kLutBytes + wave * (NB * kTile);
     // (base registers that the compiler takes as they are, the rest in the accesses' offset fields)
-    uint32_t tile_lane = tile_at + lane * 16u, x_lane = smem + P::kLutBytes + kLgBlocks * kLgTileBytes + lane * 16u;
-    uint32_t x_to = smem + P::kLutBytes + kLgBlocks * kLgTileBytes + tid * 16u;
+    uint32_t tile_lane = tile_at + lane * 16u, x_lane = smem + P::kLutBytes + kLgBlocks * kTile + lane * 16u;
+    uint32_t x_to = smem + P::kLutBytes + kLgBlocks * kTile + tid * 16u;
     asm("" : "+v"(tile_lane), "+v"(x_lane), "+v"(x_to));
 
     // ---- activations of the 128 columns from 128 g on: 16-byte pieces in operand order ----
@@ -165,11 +171,17 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         // rows, which spill with them (3 bits, 96 rows: 10240 x 5120 32.9 -> 34.2, 17408 x 5120 51.2 -> 53.7; 4 bits the same).
         constexpr bool SKIP = (BITS <= 4 && MB != 6) || NB == 1;
         uint32_t put[NB][4 * ROUNDS];
-        bool any[NB][ROUNDS], more[NB];
+        // A round's stores in each quarter that any lane has elements of, without branches around them: a lane's elements of other
+        // quarters go behind the tile.  (5 bits at 5 % listed, 10240 x 5120 at 17 / 64 / 100 / 128 rows 24.5 / 32.2 / 39.0 / 41.5 -> 23.6 /
+        // 30.5 / 37.6 / 40.2.)  Where that takes more registers than there are, each store has a branch of its own, in every quarter.
+        uint32_t in_q[NB][ROUNDS];  // bit q: the lane has elements of quarter q in the round
+        bool any[NB][ROUNDS];
+        bool more[NB];
 #pragma unroll
         for (uint32_t j = 0; j < NB; ++j) {
 #pragma unroll
             for (uint32_t r = 0; r < ROUNDS; ++r) {
+                in_q[j][r] = 0;
                 any[j][r] = __any((e_now[j].first & ~3u) + 16u * r < e_now[j].end);
                 if (SKIP && !any[j][r]) continue;
                 const uint32_t quad = mine(e_now[j]) + 16u * r;
@@ -179,6 +191,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
                     const int v = quad + k - e_now[j].first < e_now[j].end - e_now[j].first ? (int)(list[j].val[r] << (24 - 8 * k)) >> 24 : 0;
                     put[j][4 * r + k] = (ln_pack(0.0f, (float)v * scale) & 0xFFFF0000u) | (v != 0 ? (p & 0x300u) << 4 : 0x4000u) |
                                         (((p & 0xF0u) << 4) + (p & 14u) + (kg << 6) + (n & 3u) * 16u);
+                    if constexpr (!BRANCH) in_q[j][r] |= 1u << ((put[j][4 * r + k] >> 12) & 7u);
                 }
             }
             more[j] = __any((e_now[j].first & ~3u) + 16u * ROUNDS < e_now[j].end);
@@ -190,30 +203,38 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 #pragma unroll
             for (uint32_t j = 0; j < NB; ++j) {
                 uint32_t o[16];
-                ln_decode<BITS, false>(w[j][q & 1u], lut_lane, scale, o);
+                ln_decode<BITS, false, NB == 1 ? 2 : 1>(w[j][q & 1u], lut_lane, scale, o);
                 codes(q < 2 ? now : next, j, q ^ 2u);
 #pragma unroll
                 for (uint32_t i = 0; i < 4; ++i)
-                    *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(tile_lane + j * kLgTileBytes + ((i ^ q) << 10))) =
+                    *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(tile_lane + j * kTile + ((i ^ q) << 10))) =
                         ln_u32x4{o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]};
             }
             ln_wave_order();
 #pragma unroll
             for (uint32_t j = 0; j < NB; ++j) {
 #pragma unroll
-                for (uint32_t r = 0; r < ROUNDS; ++r)
-                    if (any[j][r])
+                for (uint32_t r = 0; r < ROUNDS; ++r) {
+                    if constexpr (BRANCH) {
+                        if (any[j][r])
+#pragma unroll
+                            for (uint32_t e = 4 * r; e < 4 * r + 4; ++e)
+                                if ((put[j][e] & 0x7000u) == (q << 12))
+                                    *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + j * kTile + (put[j][e] & 0xFFFu))) =
+                                        (uint16_t)(put[j][e] >> 16);
+                    } else if (__any(in_q[j][r] & (1u << q))) {
 #pragma unroll
                         for (uint32_t e = 4 * r; e < 4 * r + 4; ++e)
-                            if ((put[j][e] & 0x7000u) == (q << 12))
-                                *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + j * kLgTileBytes + (put[j][e] & 0xFFFu))) =
-                                    (uint16_t)(put[j][e] >> 16);
+                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + j * kTile + min((put[j][e] ^ (q << 12)) & 0x7FFFu, kLgTile + 4u * lane))) =
+                                (uint16_t)(put[j][e] >> 16);
+                    }
+                }
                 if (more[j]) {  // rows with yet more listed elements in the cell
                     for (uint32_t f = (e_now[j].first & ~3u) + 16u * ROUNDS + (n >> 2); f < e_now[j].end; f += 4u) {
                         const uint32_t p = exc_pos[lane_listed(f, n & 3u)];
                         const int v = exc_val[lane_listed(f, n & 3u)];
                         if (v != 0 && (p & 0x300u) == (q << 8))
-                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + j * kLgTileBytes + (kg << 6) + (n & 3u) * 16u +
+                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(tile_at + j * kTile + (kg << 6) + (n & 3u) * 16u +
                                                                              ((p & 0xF0u) << 4) + (p & 14u))) =
                                 (uint16_t)(ln_pack((float)v * scale, 0.0f) & 0xFFFFu);
                     }
@@ -234,7 +255,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
             for (uint32_t j = 0; j < NB; ++j)
 #pragma unroll
                 for (uint32_t i = 0; i < 4; ++i)
-                    a[j][i] = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(tile_lane + j * kLgTileBytes + ((i ^ q) << 10)));
+                    a[j][i] = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(tile_lane + j * kTile + ((i ^ q) << 10)));
 // activations one step ahead, and no further: all of them at once take more registers than there are
             constexpr bool AHEAD = NB == 2;
             constexpr uint32_t STEP = !AHEAD || BITS < 5 || MB == 4 ? 4u : 2u;  // pieces of 32 columns
@@ -339,7 +360,7 @@ size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m) {
 template <int BITS, int MB, int NB>
 static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once,
                        uint16_t *y, int64_t ldy, float *ws, hipStream_t s) {
-    constexpr size_t lds = LnPairs<BITS, false>::kLutBytes + kLgBlocks * kLgTileBytes + 2u * MB * 4096u;
+    constexpr size_t lds = LnPairs<BITS, false>::kLutBytes + kLgBlocks * kLgTileBytes<BITS, MB> + 2u * MB * 4096u;
     static_assert(lds <= kLnLds, "LDS of a CU");
     static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemm<BITS, MB, NB>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
