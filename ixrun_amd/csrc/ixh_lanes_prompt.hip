@@ -58,7 +58,12 @@ k_lanes_xtile(const uint16_t *__restrict__ x, int64_t ldx, uint32_t m, uint32_t 
 //
 // Bound: the matrix unit and what stands between two stages.  5120 x 17408 at 512 rows (3 bits): 99 us a call; one after the other
 // under the profiler 90 to 96 for this kernel, 9 for the activations' reordering and 11 for adding the sums (63 MB read).  The
-// products would take 58 at the rate of a large library product; decode into memory and that library's product took 126.
+// products would take 58 at the rate of a large library product; decode into memory and that library's product took 126.  Clocks a stage
+// of a wave, 7500 in all, of which its products are 2048 (and its neighbour's on the SIMD as many): first operand with the decode
+// 1750, the others 700 to 1050 each, listed elements 700, a stage's share of a cell's list 700, barrier 1150.  A cell's list is worked
+// out in the rounds that have elements, and stored in the stages that a round has any in: 3 bits at 192 / 256 / 384 / 512 rows 53.9 / 61.0 /
+// 77.6 / 98.5 -> 51.6 / 58.8 / 76.0 / 95.6, 9120 x 9216 at 5 bits 57.5 / 65.0 / 79.4 / 98.9 -> 55.0 / 62.8 / 77.4 / 96.8.  Operands of
+// weights two or three blocks ahead change nothing.
 //
 // Eight waves decode 128 rows x 128 columns a stage to LDS in operand order, 16 rows each, while they multiply the stage before: the
 // pairs of a wave's next stage are looked up between the products of its first four operands (a decode of its own before the products
@@ -67,7 +72,7 @@ k_lanes_xtile(const uint16_t *__restrict__ x, int64_t ldx, uint32_t m, uint32_t 
 // wave of the workgroup, and through LDS they would take its time from the lookups and the weights.  MI x 16 rows by 128 / NW weight
 // rows of sums a wave: 128 registers at 512 rows, so the rest is kept small: operands of weights read one block ahead, listed elements
 // worked out once a cell and kept in LDS, places recomputed.  All the same <BITS, 4, 1>, 385 to 512 rows, has all 256 registers in
-// use and 7 / 14 / 18 / 18 more (at 3 / 4 / 5 / 8 bits; 32 to 76 bytes a lane) in memory; the other forms spill none.  Requests are never
+// use and 11 / 14 / 16 / 18 more (at 3 / 4 / 5 / 8 bits; 48 to 76 bytes a lane) in memory; the other forms spill none.  Requests are never
 // inside a branch or past a way out, else they are all waited for at the join (with the last stage peeled by conditions the same loop
 // took 110 us at 512 rows, and a form whose loop spilled its sums 287).
 //
@@ -173,7 +178,8 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
         const uint32_t store_at = smem + P::kLutBytes + wave * 4096u;
         const LN_LDS(ln_u32x4) *const w_at = reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(smem + P::kLutBytes + nw * (NI * 4096u) + lane * 16u));
         LN_LDS(ln_u32x4) *const put_at = reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(smem + P::kLutBytes + 2u * kLpTile + tid * (16u * kLpRounds)));
-        bool any[kLpRounds], more;
+        uint32_t in_stage[kLpRounds];  // bit q: the block has elements of the cell's stage q in the round
+        bool any[kLpRounds], more;    // (8 bits list next to nothing: whether it has any, which takes fewer registers)
         uint32_t c_put;
         // listed elements of a cell: value (high half), where it goes in the wave's part of a stage's tile (bits 0 .. 11), the stage of
         // the cell (bits 12 .. 14; none of the four where there is no element)
@@ -182,17 +188,26 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
             const Place me = place();
 #pragma unroll
             for (uint32_t r = 0; r < kLpRounds; ++r) {
+                if constexpr (BITS != 8) {
+                    in_stage[r] = 0;
+                    if (!__any((e_now.first & ~3u) + 16u * r < e_now.end)) continue;
+                }
                 const uint32_t quad = (e_now.first & ~3u) + me.quad + 16u * r;
                 ln_u32x4 put;
+                uint32_t stages = 0;
 #pragma unroll
                 for (uint32_t k = 0; k < 4; ++k) {
                     const uint32_t p = (k & 1) ? list.pos[r][k >> 1] >> 16 : list.pos[r][k >> 1];
                     const int v = quad + k - e_now.first < e_now.end - e_now.first ? (int)(list.val[r] << (24 - 8 * k)) >> 24 : 0;
                     put[k] = (ln_pack(0.0f, (float)v * scale) & 0xFFFF0000u) | (v != 0 ? (p & 0x300u) << 4 : 0x4000u) |
                                      (((p & 0xF0u) << 4) + (p & 14u) + (me.kg << 6) + me.row * 16u);
+                    if constexpr (BITS != 8) stages |= 1u << ((put[k] >> 12) & 7u);
                 }
                 put_at[r] = put;
-                any[r] = __any((e_now.first & ~3u) + 16u * r < e_now.end);
+                if constexpr (BITS == 8) any[r] = __any((e_now.first & ~3u) + 16u * r < e_now.end);
+                else
+#pragma unroll
+                    for (uint32_t q = 0; q < 4; ++q) in_stage[r] |= (uint32_t)(__any(stages & (1u << q)) != 0) << q;
             }
             more = __any((e_now.first & ~3u) + 16u * kLpRounds < e_now.end);
             e_now = extent(c + 1u);
@@ -211,12 +226,22 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
             ln_wave_order();
 #pragma unroll
             for (uint32_t r = 0; r < kLpRounds; ++r)
-                if (any[r]) {
+                if (BITS == 8 ? any[r] : (in_stage[r] & (1u << q)) != 0) {
                     const ln_u32x4 put = put_at[r];
+                    if constexpr (MI == 4) {
 #pragma unroll
-                    for (uint32_t e = 0; e < 4; ++e)
-                        if ((put[e] & 0x7000u) == (q << 12))
-                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(base + (put[e] & 0xFFFu))) = (uint16_t)(put[e] >> 16);
+                        for (uint32_t e = 0; e < 4; ++e)
+                            if ((put[e] & 0x7000u) == (q << 12))
+                                *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(base + (put[e] & 0xFFFu))) = (uint16_t)(put[e] >> 16);
+                    } else {  // (elements of other stages go aside, a dword a lane: where there are the registers, shorter than a branch each)
+                        const Place me = place();
+                        const uint32_t aside = smem + P::kLutBytes + 2u * kLpTile + kLpThreads * (16u * kLpRounds) + (me.kg * 16u + me.quad + me.row) * 4u;
+#pragma unroll
+                        for (uint32_t e = 0; e < 4; ++e) {
+                            const uint32_t to = (put[e] ^ (q << 12)) & 0x7FFFu;
+                            *reinterpret_cast<LN_LDS(uint16_t) *>((uintptr_t)(to < 4096u ? base + to : aside)) = (uint16_t)(put[e] >> 16);
+                        }
+                    }
                 }
             if (more) {  // rows with yet more listed elements in the cell
                 const Extent e_put = extent(c_put);
@@ -293,7 +318,8 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
                         for (uint32_t i = 0; i < MI; ++i)
                             acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ln_bf16x8, v[b & 1u]),
                                                                                 __builtin_bit_cast(ln_bf16x8, a[t % AHEAD][i]), acc[i][b], 0, 0, 0);
-                        if (NI == 8 || j == 0) __builtin_amdgcn_sched_barrier(0);
+                        // (at 512 rows left to the compiler, 98.5 -> 95.4 us; at 384 62.4 -> 63.3)
+                        if ((NI == 8 && (MI != 4 || BITS == 8)) || j == 0) __builtin_amdgcn_sched_barrier(0);
                     }
                     if (j == 0) piece(3);
                     x_load(t + AHEAD < 16u ? c : c_next, (t + AHEAD) & 15u);
@@ -390,7 +416,7 @@ size_t lanes_prompt_workspace_bytes(const LanesDev &L, int m) { return lp_bytes(
 
 template <int BITS, int MI, int NW>
 static int prompt_launch(const LanesDev &L, const LpPlan &p, const ln_u32x4 *xt, ln_f32x4 *sums, const LpOut &out, hipStream_t s) {
-    constexpr size_t lds = LnPairs<BITS, true>::kLutBytes + 2u * kLpTile + 16u * kLpRounds * kLpThreads;
+    constexpr size_t lds = LnPairs<BITS, true>::kLutBytes + 2u * kLpTile + 16u * kLpRounds * kLpThreads + kWave * 4u;
     static_assert(lds <= kLnLds, "LDS of a CU");
     static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_prompt<BITS, MI, NW>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
