@@ -95,7 +95,10 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
     const uint32_t mb0 = (mg * MW + mw) * MI;  // the wave's first block of activation rows
     const uint32_t scale_raw = *scale_at;
     const float scale = bf16_bits_to_f32(scale_raw);
-    ln_build_lut<BITS, true>(smem, scale, tid, kLpThreads);
+    // The table of pairs behind the first tile's requests (0.4 us of 49 to 76); at 512 rows in front of them, where that leaves eight
+    // registers fewer in memory (0.9 us of 96).
+    constexpr bool LUT_FIRST = MI == 4 && NW == 1;
+    if constexpr (LUT_FIRST) ln_build_lut<BITS, true>(smem, scale, tid, kLpThreads);
     const uint32_t u_end = lp_begin(blockIdx.x + 1u, gridDim.x, lp_tiles(n_tiles), n_cells);
     bool begins = true;  // the run, in this tile
 #pragma unroll 1
@@ -172,6 +175,7 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
         };
 #pragma unroll
         for (uint32_t t = 0; t < AHEAD; ++t) x_load(c0, t);
+        if (!LUT_FIRST && begins) ln_build_lut<BITS, true>(smem, scale, tid, kLpThreads);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
         const uint32_t lut_lane = smem + ((lane & ((1u << P::kCopies) - 1u)) << 2);
