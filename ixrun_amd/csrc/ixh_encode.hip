@@ -62,6 +62,16 @@ __device__ __forceinline__ uint4 load8(const uint16_t *__restrict__ w, uint64_t 
     return make_uint4(pair_or(w, p, n, 0u), pair_or(w, p + 2, n, 0u), pair_or(w, p + 4, n, 0u), pair_or(w, p + 6, n, 0u));
 }
 
+// The smallest magnitude, as bf16 bits, that quantises above the threshold of a level of `bits`: every wave finds it by quantising the
+// 64 bf16 values around (threshold + 1/2) * scale.  (All of them above: a scale that is not a number, where every weight is.)
+__device__ __forceinline__ uint32_t enc_cut(int bits, float scale, float inv_scale, uint32_t lane) {
+    const float thr = (float)threshold_of(bits);
+    const int around = (int)(__float_as_uint((thr + 0.5f) * scale) >> 16) - 32;
+    const int mag = min(max(around + (int)lane, 0), 0x7fff);
+    const uint64_t above = __ballot(fabsf(quantise(bf16_bits_to_f32((uint32_t)mag), inv_scale)) > thr);
+    return above == ~0ull ? 0u : (uint32_t)min(max(around + (int)__builtin_ctzll(above | 1ull << 63), 0), 0x7fff);
+}
+
 // Bound by HBM (a read of 178 MB: 37 us, 4.8 TB/s; more loads in flight or more workgroups change nothing).
 __global__ void __launch_bounds__(1024) k_enc_absmax(const uint16_t *__restrict__ w, uint32_t n, uint32_t *parts) {
     const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
@@ -126,13 +136,7 @@ count_units(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, const 
     uint32_t cut[L - 1];  // in both halves: the smallest magnitude above the level's threshold
 #pragma unroll
     for (int i = 0; i < L - 1; ++i) {
-        const float thr = (float)threshold_of(lv.bits[i]);
-        const int around = (int)(__float_as_uint((thr + 0.5f) * scale) >> 16) - 32;
-        const int mag = min(max(around + (int)lane, 0), 0x7fff);
-        const uint64_t above = __ballot(fabsf(quantise(bf16_bits_to_f32((uint32_t)mag), inv_scale)) > thr);
-        // (all of them above: a scale that is not a number, where every weight is)
-        const uint32_t c = above == ~0ull ? 0u : (uint32_t)min(max(around + (int)__builtin_ctzll(above | 1ull << 63), 0), 0x7fff);
-        cut[i] = c * 0x10001u;
+        cut[i] = enc_cut(lv.bits[i], scale, inv_scale, lane) * 0x10001u;
     }
     const uint32_t entries = n_units + 1;
     uint32_t total[L - 1] = {};
@@ -263,8 +267,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// k_enc_pack<L>: bound by vector issue: of 5120 x 17408 at levels 3, 5, 8 690 vector instructions a wave and span (heavy tails)
-// to 790 (55 / 40 / 5 %), 62 to 72 us; the 240 MB that it moves take 47.
+// k_enc_pack<L>: bound by vector issue: of 5120 x 17408 at 55 / 40 / 5 % and levels 3, 5, 8 695 vector instructions a wave and span, 49
+// us of 66 (789 and 71 before a level's cutoff was compared with the weights as they are, codes were packed by dot products and a group
+// left in one store); the rest is the launch, first loads and the write-back of the caches.  The 240 MB that it moves take 47.
 //
 // A wave takes spans of four units, 2048 elements, 32 consecutive ones a lane, so one prefix sum over the lanes serves them
 // all and a lane's membership bits are a whole word of bitmap 0.  Every element goes to LDS as one byte, value + 128: those
@@ -302,10 +307,6 @@ struct EncRanks {
     }
 };
 
-// what a value's magnitude has to stay below to round into a level of `bits`: the thresholds are odd, so a tie goes up to
-// the next level, but for one bit (threshold 0), where it goes down to 0
-__device__ __forceinline__ float edge_of(int bits) { return (float)threshold_of(bits) + (bits == 1 ? 0.50012207f : 0.5f); }
-
 // clears what neighbouring waves share: of every stream the group of 32 codes that a wave's first code falls into,
 // of every bitmap but the first the word of its first bit; and any words behind the last code
 // (5.8 us with the ranks asked for level by level, 5.1 with all of them first, 5120 x 17408: a launch and their latency.)
@@ -338,22 +339,24 @@ k_enc_borders(EncLevels lv, const int32_t *__restrict__ table, uint32_t n, uint3
     }
 }
 
-// 32 codes (bytes, bias too high) to B words: four bytes to 4 B bits at a time
+// Four codes (bytes, `bias` too high) to 4 B bits.  Dot products of the bytes with powers of two put as many codes side by side as a
+// factor of a byte can move, and the bias comes off in what they start from (for three bits the last code is shifted there).
 template <int B>
-__device__ __forceinline__ void enc_words(const uint32_t (&x)[8], uint32_t bias4, uint32_t (&w)[B]) {
+__device__ __forceinline__ uint32_t enc_four(uint32_t x, uint32_t bias) {
+    constexpr uint32_t k1 = 1u << B, k2 = 1u << (2 * B), k3 = 1u << (3 * B);
+    if constexpr (B <= 2) return __builtin_amdgcn_udot4(x, 1u | k1 << 8 | k2 << 16 | k3 << 24, 0u - bias * (1u + k1 + k2 + k3), false);
+    if constexpr (B == 3) return __builtin_amdgcn_udot4(x, 1u | k1 << 8 | k2 << 16, ((x >> 24) << 9) - bias * (1u + k1 + k2 + k3), false);
+    const uint32_t low = __builtin_amdgcn_udot4(x, 1u | k1 << 8, 0u - bias * (1u + k1), false);
+    return (__builtin_amdgcn_udot4(x, (1u | k1 << 8) << 16, 0u - bias * (1u + k1), false) << (2 * B)) | low;
+}
+// 32 codes to B words
+template <int B>
+__device__ __forceinline__ void enc_words(const uint32_t (&x)[8], uint32_t bias, uint32_t (&w)[B]) {
 #pragma unroll
     for (int k = 0; k < B; ++k) w[k] = 0u;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-        const uint32_t v = x[c] - bias4, pair = ((1u << (2 * B)) - 1u) * 0x10001u;
-        uint32_t four;
-        if (B <= 4) {  // a shifted byte leaves nothing of its neighbour below it
-            const uint32_t two = (v | (v >> (8 - B))) & pair;
-            four = (two | (two >> (16 - 2 * B))) & ((1u << (4 * B)) - 1u);
-        } else {
-            const uint32_t two = (v & 0x00ff00ffu) | ((v & 0xff00ff00u) >> (8 - B));
-            four = ((two >> 16) << (2 * B)) | (two & 0xffffu);
-        }
+        const uint32_t four = enc_four<B>(x[c], bias);
         const int bit = 4 * B * c, d = bit >> 5, sh = bit & 31;
         w[d] |= four << sh;
         if (sh + 4 * B > 32) w[d + 1] |= four >> (32 - sh);
@@ -365,17 +368,19 @@ __device__ __forceinline__ void enc_words(const uint32_t (&x)[8], uint32_t bias4
 template <int B>
 __device__ __forceinline__ void enc_store_run(const uint8_t *run, uint32_t g0, uint32_t groups, uint32_t first, uint32_t last,
                                               uint32_t *dst, uint32_t dst_words, uint32_t lane) {
-    const uint32_t bias4 = (128u - ((1u << (B - 1)) - 1u)) * 0x01010101u;
+    constexpr uint32_t bias = 128u - ((1u << (B - 1)) - 1u);
     const bool inside = g0 > first && g0 + groups <= last && (g0 + groups) * B <= dst_words;
     for (uint32_t g = lane; g < groups; g += kWave) {
         const uint4 lo = *reinterpret_cast<const uint4 *>(run + g * 32u), hi = *reinterpret_cast<const uint4 *>(run + g * 32u + 16u);
         const uint32_t x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         uint32_t w[B];
-        enc_words<B>(x, bias4, w);
+        enc_words<B>(x, bias, w);
         const uint32_t at = (g0 + g) * B;
         if (inside) {
+            struct __attribute__((packed, aligned(4))) Words { uint32_t v[B]; } all;
 #pragma unroll
-            for (int k = 0; k < B; ++k) dst[at + k] = w[k];
+            for (int k = 0; k < B; ++k) all.v[k] = w[k];
+            *reinterpret_cast<Words *>(dst + at) = all;
         } else if (g0 + g == first || g0 + g == last) {
 #pragma unroll
             for (int k = 0; k < B; ++k)
@@ -433,7 +438,7 @@ __device__ __forceinline__ void load32(const uint16_t *__restrict__ w, uint32_t 
 }
 
 template <int L>
-__global__ void __launch_bounds__(kWave *kEncWaves)
+__global__ void __launch_bounds__(kWave *kEncWaves, L <= 3 ? 5 : 4)
 k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShare share,
            const uint16_t *__restrict__ scale_in, EncLevels lv, const int32_t *__restrict__ table, EncOut out) {
     __shared__ __attribute__((aligned(32))) uint8_t bufs[kEncWaves][2][kEncBuf];
@@ -444,7 +449,8 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
     const uint32_t u_first = share.first_unit(mine, n_units), u_end = share.first_unit(mine + 1u, n_units);
     const EncRanks ranks{table, n_units + 1, n};
     const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
-    const float inv_scale = __fdiv_rn(1.0f, bf16_bits_to_f32(*scale_in));
+    const float scale = bf16_bits_to_f32(*scale_in), inv_scale = __fdiv_rn(1.0f, scale);
+    const float cut0 = bf16_bits_to_f32(enc_cut(lv.bits[0], scale, inv_scale, lane));
     // r0, space[i]: ranks and bitmap index at the span's start; g_*, w_*: the groups and bitmap words shared with the
     // neighbouring waves; carry, bm_carry: what the span before left of an unfinished group and bitmap word
     uint32_t r0[L - 1], g_first[L - 1], g_last[L - 1], carry[L - 1], w_first[L - 1], w_last[L - 1], bm_carry[L - 1];
@@ -479,15 +485,13 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
         // ---- quantise ----
         const uint32_t p = e0 + lane * 32u;
         uint32_t member = 0;
-        // (see quantise: the sum with 3072 restores exact ties)
         float v[32];
         uint64_t in[32];
-        const float edge0 = edge_of(lv.bits[0]);
 #pragma unroll
         for (int t = 0; t < 32; ++t) {
             const float f = __uint_as_float(t & 1 ? d[t / 2] & 0xffff0000u : d[t / 2] << 16);
-            v[t] = __fmaf_rn(f, inv_scale, 3072.0f) - 3072.0f;
-            in[t] = __builtin_amdgcn_ballot_w64(fabsf(v[t]) < edge0);
+            v[t] = __fmaf_rn(f, inv_scale, 3072.0f);
+            in[t] = __builtin_amdgcn_ballot_w64(fabsf(f) < cut0);
             enc_shift_in(member, in[t]);
         }
         member = __brev(member);  // bit t: element t is in the first level
@@ -506,9 +510,10 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
         {
             uint32_t to1 = lds_address(buf) + dense_at + (r0[0] & 31u) + before;
             uint32_t to0 = lds_address(buf) + rest + (space0 & 31u) + lane * 32u - before;
-            // adding 1.5 * 2^23 rounds half to even and leaves the integer in the low bits
+            // 1.5 * 2^23 rounds half to even and leaves the integer in the low bits; the 3072 comes off with the same sum, which is
+            // exact up to its rounding
 #pragma unroll
-            for (int t = 0; t < 32; ++t) enc_put(to1, to0, in[t], t, (uint8_t)__float_as_uint(v[t] + (12582912.0f + 128.0f)));
+            for (int t = 0; t < 32; ++t) enc_put(to1, to0, in[t], t, (uint8_t)__float_as_uint(v[t] + (12582912.0f + 128.0f - 3072.0f)));
         }
         // In front of a dense run: the codes of its unfinished group; behind it code 0.  Around the other run: value 0, a
         // member of every level.
@@ -572,7 +577,7 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
                     uint32_t to0 = lds_address(other) + base0 + (incl >> 16) - c0;
 #pragma unroll
                     for (int t = 0; t < 16; ++t)
-                        enc_put(to1, to0, __builtin_amdgcn_ballot_w64((m[t / 4] & (0x80u << (8 * (t & 3)))) != 0), t,
+                        enc_put(to1, to0, __builtin_amdgcn_ballot_w64(((m[t / 4] >> (8 * (t & 3))) & 0xffu) != 0), t,
                                 (uint8_t)(x[t / 4] >> (8 * (t & 3))));
                 }
                 const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
