@@ -31,9 +31,9 @@ __device__ __forceinline__ uint32_t ln_pack(float lo, float hi) {
 // ---------------------------------------------------------------------------------------------------------------
 // Pair tables.  A table of dequantised pairs (both weights as bf16) indexed by the 2 * BITS bits of a pair, in
 // 2^kCopies copies side by side so that the lanes of a wave, which read unrelated entries, spread over the banks.
-// A vector shift and an AND take half the issue time of a bit-field extract, a conversion or a packed operation
-// (measured: 2 against 4 clocks a wave instruction), so a pair costs 6 clocks of issue and one LDS read where
-// arithmetic (extract, convert, multiply, round) takes about 20.
+// A shift right, an AND, an add, a product and a multiply-add in fp32 take half the issue time of a shift left, a bit-field
+// extract, a conversion or a packed operation (measured: 2.5 against 4.7 clocks a wave instruction), so a pair costs 5 clocks of issue
+// and one LDS read where arithmetic (extract, convert, multiply, round) takes about 20.
 // ---------------------------------------------------------------------------------------------------------------
 template <int BITS, bool WIDE> struct LnPairs {
     // log2: 32 copies of 64 entries never collide, nor do 16 of 256 or 1024 much (a look-up 4.0 clocks of the LDS, against 6.1 with 8
@@ -61,15 +61,34 @@ __device__ __forceinline__ void ln_build_lut(uint32_t lut, float scale, uint32_t
     }
 }
 
+// at + v * 2^SH for whole numbers below 2^24, as the bits of floats of which they are multiples of the smallest: exact, and two clocks of
+// issue where a shift left takes four and an add two more.  (Denormals are kept: the compiler's default here.)
+template <int SH> __device__ __forceinline__ uint32_t ln_shift_add(uint32_t v, uint32_t at) {
+    constexpr float by = SH >= 0 ? (float)(1 << (SH >= 0 ? SH : 0)) : 1.0f / (float)(1 << (SH < 0 ? -SH : 0));
+    return __float_as_uint(__fmaf_rn(__uint_as_float(v), by, __uint_as_float(at)));
+}
 template <int SH> __device__ __forceinline__ uint32_t ln_shift(uint32_t w) {
     if constexpr (SH >= 0) return w >> SH;
     else return w << -SH;
+}
+// Where copies of a table do not collide: 5120 x 17408 (3 bits) at 1 / 8 / 16 / 64 rows 12.2 / 16.3 / 19.5 / 35.6 us with shifts, 11.8 /
+// 15.8 / 18.8 / 34.9 so, 10240 x 5120 (5 bits) at 1 / 8 rows 11.1 / 16.3 and 10.8 / 15.5.  With two copies the look-ups are what a wave waits
+// for: 1536 x 3072 (4 bits) at 12 / 32 rows 8.3 / 9.1 with shifts, 8.5 / 9.3 so, 10240 x 5120 (5 bits) at 128 rows 41.0 and 41.7.
+template <class P> constexpr bool ln_float_shifts = P::kCopies > 1;
+// the address of the pair whose code begins at bit OFF of a dword (without FLOAT less lut_lane)
+template <class P, int BITS, int OFF, bool FLOAT> __device__ __forceinline__ uint32_t ln_pair_at(uint32_t w, uint32_t lut_lane) {
+    constexpr int TO = P::kCopies + 2;
+    constexpr uint32_t kField = (1u << (2 * BITS)) - 1u;
+    if constexpr (!FLOAT) return ln_shift<OFF - TO>(w) & P::kMask;
+    else if constexpr (OFF + 2 * BITS <= 24) return ln_shift_add<TO - OFF>(w & kField << OFF, lut_lane);
+    else if constexpr (OFF + 2 * BITS == 32) return ln_shift_add<TO>(w >> OFF, lut_lane);
+    else return ((w >> (OFF - TO)) & P::kMask) + lut_lane;
 }
 
 // the sixteen dequantised pairs of a lane's `BITS` dwords; at 5 bits in the smaller table ARITH of the three whole pairs of a dword by
 // arithmetic (k_lanes_gemm with a block of weights a wave, whose waves all look up at the same time: two; 10240 x 5120 at 17 / 32 / 48
 // rows 23.7 / 24.4 / 26.8 us with one, 22.7 / 23.5 / 26.0 with two)
-template <int BITS, bool WIDE, int ARITH = 1>
+template <int BITS, bool WIDE, int ARITH = 1, bool FLOAT = ln_float_shifts<LnPairs<BITS, WIDE>>>
 __device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lut_lane, float scale, uint32_t (&o)[16]) {
     using P = LnPairs<BITS, WIDE>;
     if constexpr (BITS == 8) {
@@ -83,9 +102,8 @@ __device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lu
     } else {
         constexpr int PER = BITS == 4 ? 4 : BITS == 3 ? 5 : 3;  // whole pairs a dword
         constexpr int FIRST = BITS == 4 ? 0 : 2;
-        constexpr int TO = P::kCopies + 2;
         uint32_t a[16];
-#define LN_FIELD(d, f) (ln_shift<FIRST + 2 * BITS * (f) - TO>(w[d]) & P::kMask)
+#define LN_FIELD(d, f) ln_pair_at<P, BITS, FIRST + 2 * BITS * (f), FLOAT>(w[d], lut_lane)
 #pragma unroll
         for (int d = 0; d < BITS; ++d) {
             a[PER * d] = LN_FIELD(d, 0);
@@ -96,10 +114,18 @@ __device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lu
         }
 #undef LN_FIELD
         if constexpr (BITS == 3 || BITS == 5) {
-            uint32_t last = 0;
+            constexpr int TO = P::kCopies + 2;
+            if constexpr (FLOAT) {
+                a[15] = ln_shift_add<TO>(w[0] & 3u, lut_lane);
+                a[15] = ln_shift_add<TO + 2>(w[1] & 3u, a[15]);
+                a[15] = ln_shift_add<TO + 4>(w[2] & 3u, a[15]);
+                if constexpr (BITS == 5) a[15] += ln_shift_add<TO + 8>(w[4] & 3u, ln_shift_add<TO + 6>(w[3] & 3u, 0u));
+            } else {
+                uint32_t last = 0;
 #pragma unroll
-            for (int d = 0; d < BITS; ++d) last |= (w[d] & 3u) << (TO + 2 * d);
-            a[15] = last;
+                for (int d = 0; d < BITS; ++d) last |= (w[d] & 3u) << (TO + 2 * d);
+                a[15] = last;
+            }
         }
         if constexpr (BITS == 5 && !WIDE) {
             // Two copies collide: the last whole pairs of a dword by arithmetic, which evens out the LDS and the vector unit: the
@@ -121,7 +147,7 @@ __device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lu
 #pragma unroll
         for (int p = 0; p < 16; ++p)
             if (BITS != 5 || WIDE || p == 15 || p % 3 < 3 - ARITH)
-                o[p] = *reinterpret_cast<const LN_LDS(uint32_t) *>((uintptr_t)(a[p] + lut_lane));
+                o[p] = *reinterpret_cast<const LN_LDS(uint32_t) *>((uintptr_t)(FLOAT ? a[p] : a[p] + lut_lane));
     }
 }
 

@@ -98,6 +98,7 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
     // The table of pairs behind the first tile's requests (0.4 us of 49 to 76); at 512 rows in front of them, where that leaves eight
     // registers fewer in memory (0.9 us of 96).
     constexpr bool LUT_FIRST = MI == 4 && NW == 1;
+    constexpr bool FLOAT = !LUT_FIRST;  // (its spilled registers: 96.4 us with shifts, 97.3 so; 256 rows 56.8 and 56.1)
     if constexpr (LUT_FIRST) ln_build_lut<BITS, true>(smem, scale, tid, kLpThreads);
     const uint32_t u_end = lp_begin(blockIdx.x + 1u, gridDim.x, lp_tiles(n_tiles), n_cells);
     bool begins = true;  // the run, in this tile
@@ -219,7 +220,7 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
         auto store = [&](uint32_t q) {  // stage q of the cell, to its half of the tile
             const uint32_t base = store_at + (q & 1u) * kLpTile;
             uint32_t o[16];
-            ln_decode<BITS, true>(w[q % CODES], lut_lane, scale, o);
+            ln_decode<BITS, true, 1, FLOAT>(w[q % CODES], lut_lane, scale, o);
 #pragma unroll
             for (uint32_t k = 0; k < 4; ++k)
                 *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(base + ((k ^ q) << 10) + lane * 16u)) =
@@ -313,7 +314,7 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
                         if (j == 0) {
                             if (b && b * PER % 4 == 0) piece(b * PER / 4 - 1);
                             uint32_t d[16];
-                            ln_decode<BITS, true>(w[p % CODES], lut_lane, scale, d);
+                            ln_decode<BITS, true, 1, FLOAT>(w[p % CODES], lut_lane, scale, d);
 #pragma unroll
                             for (uint32_t k = b * PER; k < b * PER + PER; ++k) o[k] = d[k];
                             __builtin_amdgcn_sched_barrier(0);
