@@ -36,21 +36,25 @@ __device__ __forceinline__ void lp_store(const LpOut &out, uint32_t r, uint32_t 
     }
 }
 
-// Bound: memory (5120 x 17408 at 512 rows: 36 MB in 9 us under the profiler).  X [m][in_f] row-major -> operand order: block (kb, mb), 32 columns x 16 rows, is 1 KB, lane l's 16 bytes are row l % 16, columns
+constexpr uint32_t kLpXBlocks = 2;  // row blocks of a workgroup of k_lanes_xtile
+
+// Bound: memory (5120 x 17408 at 512 rows: 36 MB in 7.9 us under the profiler; 9.1 with a branch around each request, 8.0 to 9.4 with one,
+// four or eight row blocks a workgroup, or with half or four times its column blocks).  X [m][in_f] row-major -> operand order: block (kb, mb), 32 columns x 16 rows, is 1 KB, lane l's 16 bytes are row l % 16, columns
 // 8 (l / 16) .. + 7; zeros past the last row and column.  A workgroup writes four column blocks of two row blocks, so that
-// whole lines are read.
+// whole lines are read; rows past the last are the last one's (no result has part in them).
 __global__ void __launch_bounds__(256)
 k_lanes_xtile(const uint16_t *__restrict__ x, int64_t ldx, uint32_t m, uint32_t in_f, uint32_t n_kb, uint32_t n_mblk,
               ln_u32x4 *__restrict__ xt) {
-    const uint32_t lane = threadIdx.x & 63u, sub = threadIdx.x >> 6;
-    const uint32_t kb = blockIdx.x * 4u + sub;
+    const uint32_t lane = threadIdx.x & 63u, kb = blockIdx.x * 4u + (threadIdx.x >> 6), col = kb * 32u + (lane >> 4) * 8u;
+    const uint16_t *const from = x + min(col, in_f - 8u);
+    ln_u32x4 v[kLpXBlocks];
 #pragma unroll
-    for (uint32_t j = 0; j < 2; ++j) {
-        const uint32_t mb = blockIdx.y * 2u + j, row = mb * 16u + (lane & 15u), col = kb * 32u + (lane >> 4) * 8u;
-        ln_u32x4 v = {0u, 0u, 0u, 0u};
-        if (row < m && col < in_f) v = *reinterpret_cast<const ln_u32x4 *>(x + (int64_t)row * ldx + col);
-        if (kb < n_kb && mb < n_mblk) xt[((size_t)kb * n_mblk + mb) * 64u + lane] = v;
-    }
+    for (uint32_t j = 0; j < kLpXBlocks; ++j)
+        v[j] = *reinterpret_cast<const ln_u32x4 *>(from + (int64_t)min((blockIdx.y * kLpXBlocks + j) * 16u + (lane & 15u), m - 1u) * ldx);
+    ln_u32x4 *const to = xt + ((size_t)kb * n_mblk + blockIdx.y * kLpXBlocks) * 64u + lane;
+#pragma unroll
+    for (uint32_t j = 0; j < kLpXBlocks; ++j)
+        if (blockIdx.y * kLpXBlocks + j < n_mblk) to[j * 64u] = col < in_f ? v[j] : ln_u32x4{0u, 0u, 0u, 0u};
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -445,7 +449,7 @@ int launch_lanes_prompt(const LanesDev &L, const uint16_t *x, int m, int64_t ldx
     ln_u32x4 *const xt = reinterpret_cast<ln_u32x4 *>(((uintptr_t)ws.at + 15u) & ~(uintptr_t)15u);
     ln_f32x4 *const sums = reinterpret_cast<ln_f32x4 *>(reinterpret_cast<uint8_t *>(xt) + lp_x_bytes(L, p));
     const uint32_t n_kb = L.n_cells * 16u, tiles = lp_tiles(L.n_tiles);
-    hipLaunchKernelGGL(k_lanes_xtile, dim3(n_kb / 4u, (p.n_mblk + 1u) / 2u), dim3(256), 0, s, x, ldx, (uint32_t)m, L.in_f, n_kb, p.n_mblk, xt);
+    hipLaunchKernelGGL(k_lanes_xtile, dim3(n_kb / 4u, (p.n_mblk + kLpXBlocks - 1u) / kLpXBlocks), dim3(256), 0, s, x, ldx, (uint32_t)m, L.in_f, n_kb, p.n_mblk, xt);
     const LpOut out{bias, y, ldy, (uint32_t)m, L.out_f, ((uintptr_t)y & 7u) == 0 && ldy % 4 == 0, lp_parts(p.groups, tiles)};
     int rc;
     switch (L.bits) {
