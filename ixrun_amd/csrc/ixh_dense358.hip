@@ -32,6 +32,33 @@ typedef uint32_t d_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t d_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t d_u32x3 __attribute__((ext_vector_type(3)));
 typedef uint16_t dn_u16x2 __attribute__((ext_vector_type(2)));
+
+// The walk over a lane's 32 positions, two at a time in the halves of a word (t and 16 + t): each half holds the slots (LDS byte address
+// / 2) of its next element in the three levels' arrays, and `flags` its bitmap 1, bit 0 the next element's that is not in level 1.
+// The arrays lie one behind the other, so that no sum or difference of slots leaves its half, and all but a shift and two selections are
+// 32-bit operations, of half a packed one's issue time.  k_decode358_dense, 17408 x 5120 at 55 / 40 / 5 %: 57.1 -> 54.4 us under the
+// profiler, 58.4 -> 56.8 the call; k_gemv358_dense on the same tensor 53.2 -> 46.8, k_gemv358_dense_rows (two rows) 62.2 -> 57.2, _tiles (eight)
+// 76.3 -> 72.8; before, fourteen packed operations for two positions.
+struct DnWalk {
+    uint32_t s1, s2, s3, flags, not1;
+    __device__ __forceinline__ uint32_t step(int t) {
+        auto halves = [](uint32_t v) { return __builtin_bit_cast(dn_u16x2, v); };
+        const uint32_t out1 = (not1 >> t) & 0x00010001u, in2 = flags & out1, in3 = out1 ^ in2;
+        const uint32_t at = __builtin_bit_cast(uint32_t, halves(s1) + halves(s2 - s1) * halves(out1) + halves(s3 - s2) * halves(in3));
+        s1 += out1 ^ 0x00010001u;
+        s2 += in2;
+        s3 += in3;
+        flags = __builtin_bit_cast(uint32_t, halves(flags) >> halves(out1));
+        return at;
+    }
+};
+// the LDS addresses of a step's two slots (a slot below 2^16 is a multiple of the smallest float: its sum with itself takes half the time
+// of a shift left)
+__device__ __forceinline__ uint32_t dn_low_at(uint32_t at) {
+    const float low = __uint_as_float(at & 0xffffu);
+    return __float_as_uint(low + low);
+}
+__device__ __forceinline__ uint32_t dn_high_at(uint32_t at) { return (at >> 15) & 0x1fffeu; }
 typedef __bf16 d_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float d_f32x2 __attribute__((ext_vector_type(2)));
 
@@ -201,38 +228,26 @@ k_gemv358_dense(Dev P, const int32_t *__restrict__ prefix, uint32_t n_chunks, ui
         const uint32_t first3 = first_a - first2;
 
         // ---- scatter the lane's 32 activations to their levels' arrays ----
-        // Two elements per step, t and t + 16, with their counters in the two halves of one register (packed
-        // 16-bit arithmetic): each half holds "LDS byte address / 2" of the next slot of its level, which fits
-        // 16 bits.  The second half starts where the first one will end: behind the level counts of the lane's
-        // first 16 elements.  in1 / in2 / in3 are 0 or 1 per half; the slot is picked by multiply-add.
+        // Two elements per step, t and t + 16 (DnWalk).  The second half starts where the first one will end: behind the level
+        // counts of the lane's first 16 elements.
         {
             const uint32_t xc_half = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)xc >> 1;
             const uint32_t low1 = (uint32_t)__popc(w1 & 0xffffu);               // level-1 elements among the first 16
             const uint32_t low_a = valid ? 16u - low1 : 0u;                       // elements above level 1 among them
             const uint32_t low2 = (uint32_t)__popc(bits2 & ((1u << low_a) - 1u));  // of which level 2
             const uint32_t a1 = xc_half + first1, a2 = xc_half + base2 + first2, a3 = xc_half + base3 + first3;
-            dn_u16x2 s1 = __builtin_bit_cast(dn_u16x2, a1 | ((a1 + low1) << 16));
-            dn_u16x2 s2 = __builtin_bit_cast(dn_u16x2, a2 | ((a2 + low2) << 16));
-            dn_u16x2 s3 = __builtin_bit_cast(dn_u16x2, a3 | ((a3 + low_a - low2) << 16));
-            // the level-2 flags each half walks through: bits2 from bit 0, and from bit low_a
-            const dn_u16x2 flags = __builtin_bit_cast(dn_u16x2, (bits2 & 0xffffu) | ((bits2 >> low_a) << 16));
-            dn_u16x2 ja = {0, 0};
-            const dn_u16x2 one = {1, 1};
+            // (the level-2 flags each half walks through: bits2 from bit 0, and from bit low_a)
+            DnWalk walk{a1 | ((a1 + low1) << 16), a2 | ((a2 + low2) << 16), a3 | ((a3 + low_a - low2) << 16),
+                        (bits2 & 0xffffu) | ((bits2 >> low_a) << 16), ~w1};
 #pragma unroll
             for (int t = 0; t < 16; ++t) {
-                const dn_u16x2 in1 = __builtin_bit_cast(dn_u16x2, (w1 >> t) & 0x00010001u);
-                const dn_u16x2 out1 = in1 ^ one;
-                const dn_u16x2 in2 = (flags >> ja) & out1;
-                const dn_u16x2 in3 = out1 ^ in2;
-                const dn_u16x2 at = in1 * (s1 - s3) + (in2 * (s2 - s3) + s3);
-                const uint32_t at32 = __builtin_bit_cast(uint32_t, at);
+                const uint32_t at = walk.step(t);
                 const uint32_t x_lo = xr[t >> 1], x_hi = xr[8 + (t >> 1)];
                 // lanes past the span scatter zeros behind the last array's entries
-                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)((at32 & 0xffffu) << 1)) =
+                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)dn_low_at(at)) =
                     (uint16_t)((t & 1) ? x_lo >> 16 : x_lo);
-                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)((at32 >> 16) << 1)) =
+                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)dn_high_at(at)) =
                     (uint16_t)((t & 1) ? x_hi >> 16 : x_hi);
-                s1 += in1; s2 += in2; s3 += in3; ja += out1;
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -554,22 +569,14 @@ __device__ __forceinline__ void dn_walk_spans(const Dev &P, const int32_t *__res
             const uint32_t low_a = min(n_here, 16u) - low1;
             const uint32_t low2 = (uint32_t)__popc(bits2 & ((1u << low_a) - 1u));
             const uint32_t a1 = wc_half + first1, a2 = wc_half + base2 + first2, a3 = wc_half + base3 + first3;
-            // Two positions at a time, in the halves of a word.  The arrays lie one behind the other, so that no sum or difference of
-            // slots leaves its half, and all but a shift and two selections are 32-bit operations, of half a packed one's issue time
-            // (and so is a sum of floats where a shift left would double: a slot below 2^16 is a multiple of the smallest float).
-            // 17408 x 5120 at 55 / 40 / 5 %: 57.1 -> 54.4 us under the profiler, 58.4 -> 56.8 the call.
-            uint32_t s1 = a1 | ((a1 + low1) << 16), s2 = a2 | ((a2 + low2) << 16), s3 = a3 | ((a3 + low_a - low2) << 16);
-            uint32_t flags = (bits2 & 0xffffu) | ((bits2 >> low_a) << 16);  // bit 0: the next position's that is not in level 1
-            const uint32_t not1 = ~w1;
-            auto halves = [](uint32_t v) { return __builtin_bit_cast(dn_u16x2, v); };
+            DnWalk walk{a1 | ((a1 + low1) << 16), a2 | ((a2 + low2) << 16), a3 | ((a3 + low_a - low2) << 16),
+                        (bits2 & 0xffffu) | ((bits2 >> low_a) << 16), ~w1};
 #pragma unroll
             for (int t = 0; t < 16; ++t) {
-                const uint32_t out1 = (not1 >> t) & 0x00010001u, in2 = flags & out1, in3 = out1 ^ in2;
-                const uint32_t at = __builtin_bit_cast(uint32_t, halves(s1) + halves(s2 - s1) * halves(out1) + halves(s3 - s2) * halves(in3));
+                const uint32_t at = walk.step(t);
                 // positions past the end of the tensor walk on through the last array; what they read is not stored
-                const float low = __uint_as_float(at & 0xffffu);
-                const uint32_t va = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)__float_as_uint(low + low));
-                const uint32_t vb = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)((at >> 15) & 0x1fffeu));
+                const uint32_t va = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)dn_low_at(at));
+                const uint32_t vb = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)dn_high_at(at));
                 if (t & 1) {
                     o[t >> 1] |= va << 16;
                     o[8 + (t >> 1)] |= vb << 16;
@@ -577,10 +584,6 @@ __device__ __forceinline__ void dn_walk_spans(const Dev &P, const int32_t *__res
                     o[t >> 1] = va;
                     o[8 + (t >> 1)] = vb;
                 }
-                s1 += out1 ^ 0x00010001u;
-                s2 += in2;
-                s3 += in3;
-                flags = __builtin_bit_cast(uint32_t, halves(flags) >> halves(out1));
             }
         }
         if (GS) {
