@@ -267,9 +267,10 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// k_enc_pack<L>: bound by vector issue: of 5120 x 17408 at 55 / 40 / 5 % and levels 3, 5, 8 695 vector instructions a wave and span, 49
-// us of 66 (789 and 71 before a level's cutoff was compared with the weights as they are, codes were packed by dot products and a group
-// left in one store); the rest is the launch, first loads and the write-back of the caches.  The 240 MB that it moves take 47.
+// k_enc_pack<L>: bound by vector issue; 5120 x 17408 at 55 / 40 / 5 % and levels 3, 5, 8: 789 vector instructions a wave and span, 71 us;
+// 695 and 66 since a level's cutoff is compared with the weights as they are, codes are packed by dot products and a group leaves in one store;
+// 62 since two elements at a time are put in their runs.  The launch, first loads and the write-back of the caches are some ten of it, and the
+// 240 MB that it moves take 47.
 //
 // A wave takes spans of four units, 2048 elements, 32 consecutive ones a lane, so one prefix sum over the lanes serves them
 // all and a lane's membership bits are a whole word of bitmap 0.  Every element goes to LDS as one byte, value + 128: those
@@ -411,17 +412,26 @@ __device__ __forceinline__ void enc_shift_in(uint32_t &bits, uint64_t in) {
     asm("s_nop 1\n\tv_addc_co_u32_e64 %0, %1, %0, %0, %2" : "+v"(bits), "=&s"(carry) : "s"(in));
 }
 
-// One element's byte to the next place of its run, where `to1` and `to0` are the LDS addresses of the two runs' next bytes
-// less t: the one taken moves on, and both fall behind t by one.  (As above: three instructions for seven.)
+// Elements' bytes to the next places of their runs, two elements at a time in the halves of a word: bit t and bit 16 + t of `not1` say which
+// run each goes to, and each half of to1 and to0 holds the LDS address of its run's next byte, the second half's where the first half's
+// elements will end.  The other run lies behind the dense one, so that no sum or difference leaves its half, and all but the selection are
+// 32-bit operations, which take half the time of packed ones and of those that use or make a carry (an element at a time, by v_cndmask,
+// v_addc and v_subb under masks in scalar registers, more of them than there are: 66.5 -> 62.0 us for the first level's, 5120 x 17408).
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
+typedef uint16_t enc_u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t lds_address(uint8_t *p) { return (uint32_t)(uintptr_t)(lds_u8 *)p; }
-__device__ __forceinline__ void enc_put(uint32_t &to1, uint32_t &to0, uint64_t in, int t, uint8_t byte) {
-    uint32_t to;
-    uint64_t carry;
-    asm("s_nop 1\n\tv_cndmask_b32_e64 %2, %1, %0, %4\n\tv_addc_co_u32_e64 %0, %3, -1, %0, %4\n\tv_subbrev_co_u32_e64 %1, %3, 0, %1, %4"
-        : "+v"(to1), "+v"(to0), "=&v"(to), "=&s"(carry) : "s"(in));
-    ((lds_u8 *)(uintptr_t)to)[t] = byte;
-}
+struct EncPut {
+    uint32_t to1, to0, not1;
+    __device__ __forceinline__ void two(int t, uint8_t first, uint8_t second) {
+        auto halves = [](uint32_t x) { return __builtin_bit_cast(enc_u16x2, x); };
+        const uint32_t out = (not1 >> t) & 0x00010001u;
+        const uint32_t at = __builtin_bit_cast(uint32_t, halves(to1) + halves(to0 - to1) * halves(out));
+        to1 += out ^ 0x00010001u;
+        to0 += out;
+        *(lds_u8 *)(uintptr_t)(at & 0xffffu) = first;
+        *(lds_u8 *)(uintptr_t)(at >> 16) = second;
+    }
+};
 
 // 32 weights from element p on, as pairs; infinite past n, which is in no level but the last.  `whole`: all of the wave's are there, at a multiple of 16 bytes.
 __device__ __forceinline__ void load32(const uint16_t *__restrict__ w, uint32_t p, uint32_t n, bool whole, uint32_t (&d)[16]) {
@@ -486,13 +496,11 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
         const uint32_t p = e0 + lane * 32u;
         uint32_t member = 0;
         float v[32];
-        uint64_t in[32];
 #pragma unroll
         for (int t = 0; t < 32; ++t) {
             const float f = __uint_as_float(t & 1 ? d[t / 2] & 0xffff0000u : d[t / 2] << 16);
             v[t] = __fmaf_rn(f, inv_scale, 3072.0f);
-            in[t] = __builtin_amdgcn_ballot_w64(fabsf(f) < cut0);
-            enc_shift_in(member, in[t]);
+            enc_shift_in(member, __builtin_amdgcn_ballot_w64(fabsf(f) < cut0));
         }
         member = __brev(member);  // bit t: element t is in the first level
         if (p < e1 && p / 32u < out.bm_words[0]) out.bm[0][p / 32u] = member;
@@ -508,12 +516,15 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
         uint32_t rest = ((dense_at + 31u + (r0[0] & 31u) + n_i) & ~31u) + 32u;  // the other run's start
         uint32_t space0 = e0 - r0[0], space1 = space0 + left;                   // its elements' indexes in the next bitmap
         {
-            uint32_t to1 = lds_address(buf) + dense_at + (r0[0] & 31u) + before;
-            uint32_t to0 = lds_address(buf) + rest + (space0 & 31u) + lane * 32u - before;
+            const uint32_t low = (uint32_t)__popc(member & 0xffffu);
+            const uint32_t to1 = lds_address(buf) + dense_at + (r0[0] & 31u) + before;
+            const uint32_t to0 = lds_address(buf) + rest + (space0 & 31u) + lane * 32u - before;
+            EncPut put{to1 | (to1 + low) << 16, to0 | (to0 + 16u - low) << 16, ~member};
             // 1.5 * 2^23 rounds half to even and leaves the integer in the low bits; the 3072 comes off with the same sum, which is
             // exact up to its rounding
+            auto byte = [&](int t) { return (uint8_t)__float_as_uint(v[t] + (12582912.0f + 128.0f - 3072.0f)); };
 #pragma unroll
-            for (int t = 0; t < 32; ++t) enc_put(to1, to0, in[t], t, (uint8_t)__float_as_uint(v[t] + (12582912.0f + 128.0f - 3072.0f)));
+            for (int t = 0; t < 16; ++t) put.two(t, byte(t), byte(16 + t));
         }
         // In front of a dense run: the codes of its unfinished group; behind it code 0.  Around the other run: value 0, a
         // member of every level.
@@ -573,12 +584,12 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
                 const uint32_t c1 = (uint32_t)__popc(bits), c0 = n_here - c1;
                 const uint32_t incl = wave_scan_inclusive(c1 | (c0 << 16));
                 if (at < end) {
-                    uint32_t to1 = lds_address(other) + base1 + (incl & 0xffffu) - c1;
-                    uint32_t to0 = lds_address(other) + base0 + (incl >> 16) - c0;
+                    const uint32_t low = (uint32_t)__popc(bits & 0xffu);
+                    uint32_t to1 = lds_address(other) + base1 + (incl & 0xffffu) - c1, to0 = lds_address(other) + base0 + (incl >> 16) - c0;
+                    EncPut put{to1 | (to1 + low) << 16, to0 | (to0 + 8u - low) << 16, ~((bits & 0xffu) | bits >> 8 << 16)};
 #pragma unroll
-                    for (int t = 0; t < 16; ++t)
-                        enc_put(to1, to0, __builtin_amdgcn_ballot_w64(((m[t / 4] >> (8 * (t & 3))) & 0xffu) != 0), t,
-                                (uint8_t)(x[t / 4] >> (8 * (t & 3))));
+                    for (int t = 0; t < 8; ++t)
+                        put.two(t, (uint8_t)(x[t / 4] >> (8 * (t & 3))), (uint8_t)(x[2 + t / 4] >> (8 * (t & 3))));
                 }
                 const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
                 base1 += total & 0xffffu;
