@@ -37,8 +37,8 @@ __device__ __forceinline__ void ln_load(const uint32_t *__restrict__ plane, uint
 // ahead 17408 x 5120 5 bits 14.9 for 14.4.  Taking the sign off costs two instructions an element; a plane without it turns an infinite
 // activation in a listed column into NaN.
 //
-// us a layer before / now: 5120 x 17408 3 bits 11.5 / 10.4, 17408 x 5120 5 bits 14.6 / 13.7, 4096 x 11008 9.3 / 8.9, 5120 x 5120 7.8 / 7.3,
-// 17408 x 5120 with two rows at 5 bits 15.9 / 14.7, with four at 3 bits 15.3 / 13.4.
+// us a layer before / now: 5120 x 17408 3 bits 11.5 / 9.9 (10.5 before the look-ups' addresses took two instructions), 17408 x 5120 5 bits
+// 14.6 / 13.8, 4096 x 11008 9.3 / 8.9, 5120 x 5120 7.8 / 7.3, 17408 x 5120 with two rows at 5 bits 15.9 / 14.7, with four at 3 bits 15.3 / 13.1.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kLnAhead = 2;      // cells in flight
 constexpr uint32_t kLnFirst = 1;      // of these, asked for before the activations are there

@@ -60,8 +60,10 @@ k_lanes_xtile(const uint16_t *__restrict__ x, int64_t ldx, uint32_t m, uint32_t 
 // ---------------------------------------------------------------------------------------------------------------
 // k_lanes_prompt<BITS, MI, NW>: 128 MI / NW activation rows by 128 weight rows a workgroup, over a run of the cells of a tile.
 //
-// Bound: the matrix unit and what stands between two stages.  5120 x 17408 at 512 rows (3 bits): 99 us a call; one after the other
-// under the profiler 90 to 96 for this kernel, 9 for the activations' reordering and 11 for adding the sums (63 MB read).  The
+// Bound: the matrix unit and what stands between two stages.  5120 x 17408 at 512 rows (3 bits): 97 us a call; one after the other
+// under the profiler 86 to 96 for this kernel, 8 for the activations' reordering and 12 for adding the sums (63 MB read).  (Which blocks share
+// an XCD's L2 matters little: all of an XCD on the same columns 2 to 4 % slower, on neighbouring runs up to 3 %.  Operands straight from
+// row-major activations: 126 instead of 88.)  The
 // products would take 58 at the rate of a large library product; decode into memory and that library's product took 126.  Clocks a stage
 // of a wave, 7500 in all, of which its products are 2048 (and its neighbour's on the SIMD as many): first operand with the decode
 // 1750, the others 700 to 1050 each, listed elements 700, a stage's share of a cell's list 700, barrier 1150.  A cell's list is worked

@@ -10,7 +10,7 @@ namespace ixh {
 //
 // Bound: a launch's start-up (some 5 us to the first product: the activations of a slice are turned round on the way to LDS),
 // then the decode's LDS look-ups and vector instructions; the busiest unit is busy for some 60 % of the rest. us a layer:
-// 17408 x 5120 at 55 / 40 / 5 %, 8 rows 32.6 -> 20.2, 5120 x 17408 at 3 bits, 16 rows 25.1 -> 18.6, 1536 x 2048, 8 rows
+// 17408 x 5120 at 55 / 40 / 5 %, 8 rows 32.6 -> 19.1, 5120 x 17408 at 3 bits, 16 rows 25.1 -> 17.9, 1536 x 2048, 8 rows
 // 9.7 -> 6.8, against k_lanes_gemm, which decodes to LDS, stores the listed elements over their places, reads the operands
 // back and meets at a barrier every 128 columns.
 //
