@@ -195,18 +195,18 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         v = __uint_as_float(g[0]) + __uint_as_float(g[1]);
         return v;
     };
-    const uint32_t scale_bits = __float_as_uint(scale) & 0x7FFFFFFFu, x_none = x_at + C * 1024u;
+    const uint32_t scale_bits = __float_as_uint(scale) & 0x7FFFFFFFu;
     // one group of listed elements, range by range: the lane has four of its row, quads quad .. quad + 3
     auto list_group = [&](const Group &in, uint32_t i) {
         const uint32_t g0 = (g_first + i) << 6, quad = g0 + (lane & ~3u), vals = in.val;
         float p[4][MT];
         for (bool first = true;; first = false) {
             if (first || C >= kLnSegCells) {  // (positions start over in the next segment)
-                const uint32_t x_seg = x_at + l_seg * (kLnSegCells * 1024u);
-                uint32_t at[4] = {x_seg + (in.pos[0] & 0xFFFFu), x_seg + (in.pos[0] >> 16), x_seg + (in.pos[1] & 0xFFFFu), x_seg + (in.pos[1] >> 16)};
+                uint32_t at[4] = {x_at + (in.pos[0] & 0xFFFFu), x_at + (in.pos[0] >> 16), x_at + (in.pos[1] & 0xFFFFu), x_at + (in.pos[1] >> 16)};
                 if (C >= kLnSegCells)
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) at[k] = (vals >> (8 * k)) & 255u ? at[k] : x_none;
+                    for (uint32_t k = 0; k < 4; ++k)
+                        at[k] = x_at + ln_listed_at(at[k] - x_at, (vals >> (8 * k)) & 255u, quad + k - r0 < r1 - r0, l_seg, C);
                 const uint32_t w01 = ln_pack((float)(int)(int8_t)vals * scale, (float)(int)(int8_t)(vals >> 8) * scale);
                 const uint32_t w23 = ln_pack((float)(int)(int8_t)(vals >> 16) * scale, (float)((int)vals >> 24) * scale);
 #pragma unroll

@@ -23,6 +23,13 @@ LN_BOTH LnGroups ln_groups(uint32_t first_quad, uint32_t end_quad, uint32_t grou
     return {first, last < groups ? last : groups - 1u, end_quad > first_quad ? last - first + 1u : 0u};
 }
 
+// Byte offset, in a row of `cells` cells of activations, of a listed element at position `pos` of segment `seg` (64 cells each), for rows
+// of a whole segment and more: a position of another segment's quad may lie behind the row, and a place without an element (value
+// 0) holds position 0: both go to the zeros behind the last cell.  `in_range`: the quad is of the row quad and segment in work.
+LN_BOTH uint32_t ln_listed_at(uint32_t pos, uint32_t value, bool in_range, uint32_t seg, uint32_t cells) {
+    return value && in_range ? seg * 65536u + pos : cells * 1024u;
+}
+
 // A workgroup's cells are dealt to its 2^log_waves waves in runs: wave w has the cells ln_share(n, w) .. ln_share(n, w + 1) - 1.  The
 // first of sixteen waves has 1.47 times the mean, the last one 0.53 times: a SIMD serves the oldest of its waves first, so the last ones
 // have their first cells 1.4 us after the first ones and in even shares end 1.6 to 2 us after them (us a layer, even shares /

@@ -16,6 +16,9 @@ extern "C" void groups(uint32_t first, uint32_t end, uint32_t n, uint32_t *out) 
 extern "C" int whole(uint64_t x, uint32_t in_f, int m, int64_t ldx) { return ixh::ln_whole_pieces(x, in_f, m, ldx); }
 extern "C" uint32_t column(uint32_t col, uint32_t in_f) { return ixh::ln_piece_column(col, in_f); }
 extern "C" uint32_t share(uint32_t n, uint32_t wave, uint32_t log_waves) { return ixh::ln_share(n, wave, log_waves); }
+extern "C" uint32_t listed_at(uint32_t pos, uint32_t value, int in_range, uint32_t seg, uint32_t cells) {
+    return ixh::ln_listed_at(pos, value, in_range, seg, cells);
+}
 extern "C" uint32_t begin(uint32_t g, uint32_t groups, uint32_t tiles, uint32_t cells) { return ixh::lp_begin(g, groups, tiles, cells); }
 extern "C" uint32_t group_of(uint32_t c, uint32_t groups, uint32_t tiles, uint32_t cells) { return ixh::lp_group_of(c, groups, tiles, cells); }
 extern "C" uint32_t part(uint32_t g, uint32_t tile, int begins, uint32_t groups, uint32_t tiles) { return ixh::lp_part(g, tile, begins, groups, tiles); }
@@ -62,6 +65,20 @@ def test_requests_of_the_activations_stay_in_their_row(bounds, in_f):
         for col in range(0, -(-in_f // 512) * 512, 8):
             at = bounds.column(col, in_f)
             assert at % 8 == 0 and at + 8 <= in_f and (at == col or col + 8 > in_f)
+
+
+@pytest.mark.parametrize("cells", [64, 65, 67, 70, 127, 128, 129, 150])
+def test_listed_elements_of_long_rows_are_gathered_from_their_row(bounds, cells):
+    """A group of the list holds quads of several segments of a row, whose positions start over in each: those of the segment in
+    work have their own activation, all others the zeros behind the row."""
+    segments = -(-cells // 64)
+    for seg in range(segments):
+        for of in range(segments):
+            end = min(65536, cells * 1024 - of * 65536)
+            for pos in [*range(0, min(end, 64), 2), *range(1024, end, 1024), end - 2]:
+                at = bounds.listed_at(pos, 90, of == seg, seg, cells)
+                assert at == (seg * 65536 + pos if of == seg else cells * 1024) and at + 2 <= cells * 1024 + 64
+        assert bounds.listed_at(0, 0, True, seg, cells) == cells * 1024
 
 
 @pytest.mark.parametrize("log_waves", [0, 1, 2, 3, 4])
