@@ -135,8 +135,11 @@ int ixh_decode_gs(const IxhPacked *packed, const int32_t *prefix, int64_t chunk,
 /*
  * ixh_decode (group_scales NULL) or ixh_decode_gs of a (3,5,8) tensor of at most 2^22 weights without a rank table, in one
  * launch: for callers that decode a tensor whose table they do not keep.  IXH_EUNSUPPORTED, and nothing done, for anything else: larger
- * tensors, other schemes, groups that are no power of two from 32 up, an out_bf16 that is not 16-byte aligned.
+ * tensors, other schemes, groups that are no power of two from 32 up, a last stream that is not 4-byte aligned, an out_bf16 that is not
+ * 16-byte aligned, and any tensor while the testing hook (ixhip_test.h) names a decoder.  ixh_decode_unranked_takes: 1 if none of these
+ * holds, else 0, for callers that go on to build a table; it validates nothing else and leaves ixh_last_error as it was.
  */
+int ixh_decode_unranked_takes(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, const uint16_t *out_bf16);
 int ixh_decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, uint16_t *out_bf16,
                         ixh_stream_t stream);
 

@@ -73,8 +73,9 @@ def host():
                                "there is no fallback path") from e
         L = lib()
         _host.bind(*(C.cast(f, C.c_void_p).value for f in (
-            L.ixh_prefix_entries, L.ixh_prefix_workspace_bytes, L.ixh_prefix_build_ws, L.ixh_decode, L.ixh_decode_gs, L.ixh_decode_unranked,
-            L.ixh_encode_workspace_bytes, L.ixh_encode_scan_counts, L.ixh_encode_wait, L.ixh_encode_pack)), check)
+            L.ixh_prefix_entries, L.ixh_prefix_workspace_bytes, L.ixh_prefix_build_ws, L.ixh_decode, L.ixh_decode_gs,
+            L.ixh_decode_unranked_takes, L.ixh_decode_unranked, L.ixh_encode_workspace_bytes, L.ixh_encode_scan_counts,
+            L.ixh_encode_wait, L.ixh_encode_pack)), check)
         _native = _host
     return _native
 
@@ -95,7 +96,7 @@ EXPORTS = (
     "ixh_prefix_workspace_bytes", "ixh_decode",
     "ixh_gemv", "ixh_gemv_workspace_bytes", "ixh_gemv_noalloc", "ixh_gemm", "ixh_gemm_workspace_bytes",
     "ixh_encode_workspace_bytes", "ixh_encode_scan", "ixh_encode_scan_counts", "ixh_encode_wait", "ixh_encode_pack",
-    "ixh_decode_gs", "ixh_decode_unranked",
+    "ixh_decode_gs", "ixh_decode_unranked", "ixh_decode_unranked_takes",
     "ixh_lanes_plane_words", "ixh_lanes_cells", "ixh_lanes_pack", "ixh_lanes_list", "ixh_lanes_gemv",
     "ixh_lanes_gemv_workspace_bytes", "ixh_lanes_gemm", "ixh_lanes_gemm_workspace_bytes",
 )
@@ -131,6 +132,8 @@ def lib() -> C.CDLL:
                                     C.c_void_p]
         L.ixh_decode_unranked.restype = C.c_int
         L.ixh_decode_unranked.argtypes = [C.POINTER(IxhPacked), C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p]
+        L.ixh_decode_unranked_takes.restype = C.c_int
+        L.ixh_decode_unranked_takes.argtypes = [C.POINTER(IxhPacked), C.c_void_p, C.c_int64, C.c_void_p]
         L.ixh_gemv.restype = C.c_int
         L.ixh_gemv.argtypes = [
             C.POINTER(IxhPacked), C.c_void_p, C.c_int64, C.c_void_p, C.c_int32, C.c_int64, C.c_void_p,

@@ -246,6 +246,21 @@ int ixh_decode_gs(const IxhPacked *packed, const int32_t *prefix, int64_t chunk,
     return decode_any(packed, prefix, chunk, nullptr, out_bf16, GroupScales{group_scales, (uint32_t)group_size}, stream);
 }
 
+// why ixh_decode_unranked does not take a call; nullptr if it does
+static const char *unranked_refuses(const IxhPacked &p, const uint16_t *group_scales, int64_t group_size, const uint16_t *out) {
+    if (p.n_levels != 3 || p.level_bits[0] != 3 || p.level_bits[1] != 5 || p.level_bits[2] != 8) return "levels other than (3,5,8)";
+    if (p.out_f > kDnCountedMost || p.in_f > kDnCountedMost || p.out_f * p.in_f > kDnCountedMost) return "more than 2^22 weights";
+    if (group_scales && (group_size < 32 || (group_size & (group_size - 1)) != 0)) return "groups that are no power of two from 32 up";
+    if (((uintptr_t)p.last & 3u) != 0) return "the last stream is not 4-byte aligned";
+    if (((uintptr_t)out & 15u) != 0) return "out_bf16 is not 16-byte aligned";
+    if (g_opt_decode_kernel.load(std::memory_order_relaxed) != kDecodeAuto) return "a decoder that takes a rank table is named";
+    return nullptr;
+}
+
+int ixh_decode_unranked_takes(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, const uint16_t *out_bf16) {
+    return packed && !unranked_refuses(*packed, group_scales, group_size, out_bf16);
+}
+
 int ixh_decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, uint16_t *out_bf16,
                         ixh_stream_t stream) {
     Dev d;
@@ -255,9 +270,8 @@ int ixh_decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, i
     if (d.n == 0) return IXH_OK;
     if (!out_bf16) { set_error("out_bf16 is NULL"); return IXH_EINVAL; }
     const GroupScales gs{group_scales, group_scales ? (uint32_t)group_size : 0u};
-    const bool forced = g_opt_decode_kernel.load(std::memory_order_relaxed) != kDecodeAuto;  // (the kernels that tests name take a table)
-    if (forced || !decode_counted358_supports(d, out_bf16, gs)) {
-        set_error("decode_unranked: not (3,5,8), more than 2^22 weights, groups that are no power of two from 32 up, or out_bf16 not 16-byte aligned");
+    if (const char *why = unranked_refuses(*packed, group_scales, group_size, out_bf16)) {
+        set_error("decode_unranked: %s", why);
         return IXH_EUNSUPPORTED;
     }
     rc = launch_decode_counted358(d, out_bf16, gs, (hipStream_t)stream);

@@ -672,7 +672,7 @@ k_decode358_dense(Dev P, const int32_t *__restrict__ prefix, uint32_t n_units, u
 // 1400 x 1500 and 14.5 / 11.8 to 12.9 at 2048 x 2048.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kDnCountedWaves = 16, kDnCountedSpans = 8;
-constexpr uint32_t kDnCountedMost = 256u * kDnCountedSpans * kDnSpan;  // weights
+static_assert(kDnCountedMost == 256u * kDnCountedSpans * kDnSpan, "up to 256 workgroups");
 
 struct DnOneSpan {
     DnSpan span;
@@ -1061,10 +1061,6 @@ int launch_decode_dense358(const Dev &P, const int32_t *prefix, uint16_t *o16, G
         hipLaunchKernelGGL(k_decode358_dense<false>, dim3(blocks), dim3(kWave * kDnWaves), 0, s, P, prefix, n_units, n_spans, o16,
                            (const uint16_t *)nullptr, 0u);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
-}
-
-bool decode_counted358_supports(const Dev &P, const uint16_t *o16, GroupScales gs) {
-    return P.n <= kDnCountedMost && decode_dense358_supports(P, kFastChunk, nullptr, o16, gs);
 }
 
 int launch_decode_counted358(const Dev &P, uint16_t *o16, GroupScales gs, hipStream_t s) {

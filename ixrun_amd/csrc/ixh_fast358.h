@@ -50,8 +50,8 @@ bool decode_rows358_supports(const Dev &P, uint32_t chunk, const int8_t *o8, con
 int launch_decode_rows358(const Dev &P, const int32_t *prefix, uint16_t *o16, hipStream_t s);
 bool decode_dense358_supports(const Dev &P, uint32_t chunk, const int8_t *o8, const uint16_t *o16, GroupScales gs);
 int launch_decode_dense358(const Dev &P, const int32_t *prefix, uint16_t *o16, GroupScales gs, hipStream_t s);
-// the same without a rank table, up to 2^22 weights
-bool decode_counted358_supports(const Dev &P, const uint16_t *o16, GroupScales gs);
+// the same without a rank table, up to kDnCountedMost weights
+constexpr uint32_t kDnCountedMost = 1u << 22;
 int launch_decode_counted358(const Dev &P, uint16_t *o16, GroupScales gs, hipStream_t s);
 int launch_reduce_chunks(const float *ws, uint32_t n_chunks, int m, uint32_t out_f, uint16_t *y, int64_t ldy,
                          hipStream_t s);

@@ -221,6 +221,7 @@ struct Library {
     decltype(&ixh_prefix_build_ws) prefix_build;
     decltype(&ixh_decode) decode;
     decltype(&ixh_decode_gs) decode_gs;
+    decltype(&ixh_decode_unranked_takes) decode_unranked_takes;
     decltype(&ixh_decode_unranked) decode_unranked;
     decltype(&ixh_encode_workspace_bytes) encode_workspace_bytes;
     decltype(&ixh_encode_scan_counts) encode_scan;
@@ -242,21 +243,22 @@ bool checked(int rc) {
     return r != nullptr;
 }
 
-// bind(prefix_entries, prefix_workspace_bytes, prefix_build_ws, decode, decode_gs, decode_unranked, encode_workspace_bytes,
-// encode_scan_counts, encode_wait, encode_pack, check): addresses, and what raises for a negative code
+// bind(prefix_entries, prefix_workspace_bytes, prefix_build_ws, decode, decode_gs, decode_unranked_takes, decode_unranked,
+// encode_workspace_bytes, encode_scan_counts, encode_wait, encode_pack, check): addresses, and what raises for a negative code
 PyObject *bind(PyObject *, PyObject *args) {
-    PyObject *f[10], *check;
-    if (!PyArg_ParseTuple(args, "OOOOOOOOOOO", &f[0], &f[1], &f[2], &f[3], &f[4], &f[5], &f[6], &f[7], &f[8], &f[9], &check)) return nullptr;
+    PyObject *f[11], *check;
+    if (!PyArg_ParseTuple(args, "OOOOOOOOOOOO", &f[0], &f[1], &f[2], &f[3], &f[4], &f[5], &f[6], &f[7], &f[8], &f[9], &f[10], &check)) return nullptr;
     entry(library.prefix_entries, f[0]);
     entry(library.prefix_workspace_bytes, f[1]);
     entry(library.prefix_build, f[2]);
     entry(library.decode, f[3]);
     entry(library.decode_gs, f[4]);
-    entry(library.decode_unranked, f[5]);
-    entry(library.encode_workspace_bytes, f[6]);
-    entry(library.encode_scan, f[7]);
-    entry(library.encode_wait, f[8]);
-    entry(library.encode_pack, f[9]);
+    entry(library.decode_unranked_takes, f[5]);
+    entry(library.decode_unranked, f[6]);
+    entry(library.encode_workspace_bytes, f[7]);
+    entry(library.encode_scan, f[8]);
+    entry(library.encode_wait, f[9]);
+    entry(library.encode_pack, f[10]);
     if (PyErr_Occurred()) return nullptr;
     Py_INCREF(check);
     Py_XSETREF(library.check, check);
@@ -350,10 +352,10 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
         w = at::empty({out_f, in_f}, options.dtype(at::kBFloat16));
         uint16_t *out = static_cast<uint16_t *>(w.data_ptr());
         const uint16_t *of_groups = scales ? static_cast<const uint16_t *>(scales->const_data_ptr()) : nullptr;
-        rc = given ? IXH_EUNSUPPORTED : library.decode_unranked(&p, of_groups, group, out, stream);
-        const bool ranked = rc == IXH_EUNSUPPORTED;
-        if (ranked) rc = IXH_OK;
-        if (ranked && !given) {
+        const bool ranked = given || !library.decode_unranked_takes(&p, of_groups, group, out);
+        if (!ranked) {
+            rc = library.decode_unranked(&p, of_groups, group, out, stream);
+        } else if (!given) {
             const size_t bytes = library.prefix_workspace_bytes(n, kUnit, p.n_levels);
             table = at::empty({rows * entries + (int64_t)bytes / 4}, options.dtype(at::kInt));  // and the scratch
             int32_t *ranks = static_cast<int32_t *>(table.data_ptr());

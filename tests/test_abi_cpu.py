@@ -96,6 +96,39 @@ def test_malformed_packed_is_refused(mutate, needle):
     assert rc == -1 and needle in lib.ixh_last_error().decode()
 
 
+@pytest.mark.parametrize("change,group,out,needle", [
+    ({}, 64, 0x1000, None),
+    ({}, None, 0x1000, None),
+    ({"level_bits": (3, 4, 5, 6, 8)}, None, 0x1000, "(3,5,8)"),
+    ({"in_f": (1 << 11) + 1}, None, 0x1000, "2^22"),
+    ({"out_f": 1, "in_f": (1 << 22) + 1}, None, 0x1000, "2^22"),
+    ({"last": 0x1002}, None, 0x1000, "last stream"),
+    ({}, None, 0x1008, "16-byte"),
+    ({}, 16, 0x1000, "power of two"),
+    ({}, 96, 0x1000, "power of two"),
+    ({"named": 3}, None, 0x1000, "named"),
+])
+def test_decode_without_a_table_says_what_it_does_not_take(change, group, out, needle):
+    """Each call that is refused is refused with its own reason, before any launch; asking first leaves the last error as it was."""
+    lib = _lib.lib()
+    change = dict(change)
+    named, last = change.pop("named", 0), change.pop("last", 0x1000)
+    s = _packed(**{"out_f": 1 << 11, "in_f": 1 << 11, "bm0_words": (1 << 17) + 64, **change})
+    s.last, s.last_bytes = last, 4
+    scales = 0x1000 if group else None
+    assert lib.ixh_set_option(b"decode_kernel", named) == 0
+    try:
+        assert lib.ixh_decode_unranked(None, None, 0, 0x1000, None) == -1
+        before = lib.ixh_last_error()
+        assert lib.ixh_decode_unranked_takes(C.byref(s), scales, group or 0, out) == (needle is None)
+        assert lib.ixh_last_error() == before
+        if needle:
+            assert lib.ixh_decode_unranked(C.byref(s), scales, group or 0, out, None) == -2
+            assert needle in lib.ixh_last_error().decode()
+    finally:
+        lib.ixh_set_option(b"decode_kernel", 0)
+
+
 def test_malformed_gemv_arguments():
     lib = _lib.lib()
     s = _packed(out_f=4, in_f=1024, bm0_words=128)

@@ -133,6 +133,24 @@ def test_per_tensor_decode_without_a_table(oracle, dev, kind, shape):
     assert np.array_equal(bf16_bits(decode_weight_triton(p)).reshape(-1), want)
 
 
+@pytest.mark.parametrize("levels,shape", [((3, 4, 5, 6, 8), (33, 1000)), ((3, 5, 8), (2049, 2048))])
+def test_a_decode_that_succeeds_leaves_no_error(oracle, dev, levels, shape):
+    """Tensors that need a table are not first refused without one."""
+    from ixrun_amd import _lib, decode_weight_triton
+    from ixrun_amd.quantize import int8x_quantize_device
+
+    w = (torch.randn(shape, generator=torch.Generator().manual_seed(5)) * 0.02).bfloat16().to(dev)
+    p = int8x_quantize_device(w, levels)
+    p.pop("table512", None)
+    assert _lib.lib().ixh_set_option(b"no such option", 0) == -1
+    before = _lib.lib().ixh_last_error()
+    got = decode_weight_triton(p)
+    assert _lib.lib().ixh_last_error() == before
+    on_host = lambda v: v.cpu() if isinstance(v, torch.Tensor) else [on_host(e) for e in v] if isinstance(v, list) else v
+    host = {k: on_host(v) for k, v in p.items()}
+    assert np.array_equal(bf16_bits(got), oracle.decode_packed_bf16(host).reshape(shape))
+
+
 @pytest.mark.parametrize("n,group,code", [((1 << 22) + 1, 64, -2), (4096, 48, -2), (4096, 16, -2), (4096, 0, -1)])
 def test_decode_without_a_table_refuses_the_rest(oracle, dev, n, group, code):
     from ixrun_amd import _lib
