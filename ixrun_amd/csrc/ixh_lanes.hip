@@ -8,6 +8,38 @@ __device__ __forceinline__ void ln_load(const uint32_t *__restrict__ plane, uint
     ln_load_lane<BITS>(plane + (size_t)cell * (64u * BITS), lane, w);
 }
 
+// sums over the lanes l, l + 16, l + 32 and l + 48, in each of them; over the lanes of a weight row, l + 4 k
+__device__ __forceinline__ float lv_sum_of_rows(float v) {
+    const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    const auto g = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(g[0]) + __uint_as_float(g[1]);
+}
+__device__ __forceinline__ float lv_row_sum(float v) {
+    v += ln_dpp<0x124>(v);
+    v += ln_dpp<0x128>(v);
+    return lv_sum_of_rows(v);
+}
+
+// products of a lane's four listed elements (places: two words of two byte offsets; four values) with the activations of MT rows
+template <int MT>
+__device__ __forceinline__ void lv_listed(const uint32_t (&at)[4], uint32_t vals, float scale, uint32_t x_row, float (&p)[4][MT]) {
+    const uint32_t scale_bits = __float_as_uint(scale) & 0x7FFFFFFFu;
+    const uint32_t w01 = ln_pack((float)(int)(int8_t)vals * scale, (float)(int)(int8_t)(vals >> 8) * scale);
+    const uint32_t w23 = ln_pack((float)(int)(int8_t)(vals >> 16) * scale, (float)((int)vals >> 24) * scale);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t wk = k & 2 ? w23 : w01;
+        const uint32_t wb = k & 1 ? wk & 0xFFFF0000u : wk << 16;
+        const float wv = __uint_as_float(wb) - __uint_as_float((wb & 0x80000000u) | scale_bits);  // (no element: times 0)
+#pragma unroll
+        for (int r = 0; r < MT; ++r) {
+            const uint32_t h = *reinterpret_cast<const LN_LDS(uint16_t) *>((uintptr_t)(at[k] + (uint32_t)r * x_row));
+            p[k][r] = wv * __uint_as_float(h << 16);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // k_lanes_gemv<BITS, MT, WIDE>: up to MT activation rows, MT = 1, 2 or 4.
 //
@@ -189,17 +221,6 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     float ex[MT];  // of the lane's row
 #pragma unroll
     for (int r = 0; r < MT; ++r) ex[r] = 0.0f;
-    // sums over the lanes of a row's products, to `parts`: lane l has row l % 4
-    auto row_sum = [&](float v) {
-        v += ln_dpp<0x124>(v);
-        v += ln_dpp<0x128>(v);
-        const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-        const auto g = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(g[0]) + __uint_as_float(g[1]);
-        return v;
-    };
-    const uint32_t scale_bits = __float_as_uint(scale) & 0x7FFFFFFFu;
     // one group of listed elements, range by range: the lane has four of its row, quads quad .. quad + 3
     auto list_group = [&](const Group &in, uint32_t i) {
         const uint32_t g0 = (g_first + i) << 6, quad = g0 + (lane & ~3u), vals = in.val;
@@ -211,19 +232,7 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 #pragma unroll
                     for (uint32_t k = 0; k < 4; ++k)
                         at[k] = x_at + ln_listed_at(at[k] - x_at, (vals >> (8 * k)) & 255u, quad + k - r0 < r1 - r0, l_seg, C);
-                const uint32_t w01 = ln_pack((float)(int)(int8_t)vals * scale, (float)(int)(int8_t)(vals >> 8) * scale);
-                const uint32_t w23 = ln_pack((float)(int)(int8_t)(vals >> 16) * scale, (float)((int)vals >> 24) * scale);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const uint32_t wk = k & 2 ? w23 : w01;
-                    const uint32_t wb = k & 1 ? wk & 0xFFFF0000u : wk << 16;
-                    const float wv = __uint_as_float(wb) - __uint_as_float((wb & 0x80000000u) | scale_bits);  // (no element: times 0)
-#pragma unroll
-                    for (int r = 0; r < MT; ++r) {
-                        const uint32_t h = *reinterpret_cast<const LN_LDS(uint16_t) *>((uintptr_t)(at[k] + (uint32_t)r * x_row));
-                        p[k][r] = wv * __uint_as_float(h << 16);
-                    }
-                }
+                lv_listed<MT>(at, vals, scale, x_row, p);
             }
             if (g0 < r0 || g0 + 64u > r1) {  // quads of other ranges among them
 #pragma unroll
@@ -239,7 +248,7 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
             if (row_ends || (goes_on ? i + 1u == n_groups : r1 >= quads_end || (i + 1u == n_groups && r1 == g0 + 64u))) {
 #pragma unroll
                 for (int r = 0; r < MT; ++r) {
-                    const float v = row_sum(ex[r]);
+                    const float v = lv_row_sum(ex[r]);
                     if (lane < 4) list_parts[(l_tile + wave) * (MT * 4u) + (uint32_t)r * 4u + lane] = v;
                     ex[r] = 0.0f;
                 }
@@ -334,12 +343,160 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         for (int r = 0; r < MT; ++r) {
             float sum = listed ? list_parts[(t + part) * (MT * 4u) + (uint32_t)r * 4u + (lane & 3u)] : 0.0f;
             for (uint32_t c = part; c < C; c += 16u) sum += parts[(c * tiles_per_wg + t) * (MT * 4u) + (uint32_t)r * 4u + (lane & 3u)];
-            sum = row_sum(sum);
+            sum = lv_row_sum(sum);
             if (lane < 4 && at < out_f && (uint32_t)r < m) {
                 uint32_t b = f32_to_bf16_bits(sum);
                 if (bias) b = f32_to_bf16_bits(bf16_bits_to_f32(b) + bf16_bits_to_f32(bias[at]));
                 y[(int64_t)r * ldy + at] = (uint16_t)b;
             }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// k_lanes_gemv_few<BITS, MT, N>: the same where a wave has one cell, or two (N).
+//
+// Bound: a launch, its instructions' way from the caches (3 to 7 KB of them; k_lanes_gemv has 9 to 14, of which such a layer runs through
+// all but its loop) and one chain of requests: scale, activations, cells and where their lists lie, then the lists.  All of them are made
+// before anything is waited for.  A cell's part of the list is in one segment and one row quad, so nothing is dealt or searched, and
+// its sums join the cell's.  The smaller pair table: the larger one takes longer to write than it saves.  us from a graph, k_lanes_gemv / this:
+// one row 256 x 512 4.52 / 3.40, 1536 x 1536 (3 bits) 4.42 / 3.28, 4096 x 1024 (5) 4.43 / 3.52; four rows 1536 x 1536 (3) 5.84 / 3.92; two cells: 3000 x
+// 3000 (5) 5.40 / 4.89, 8192 x 2048 (3) 5.94 / 5.42, (5) 6.85 / 6.65, 4096 x 4096 at 4 bits 6.40 / 6.49, four rows 8.70 / 8.35 (5).
+// ---------------------------------------------------------------------------------------------------------------
+template <int BITS, int MT, int N>
+__global__ void __launch_bounds__(1024)
+k_lanes_gemv_few(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
+                 const uint16_t *__restrict__ scale_at, const uint16_t *__restrict__ bias, uint32_t shape, uint32_t inv_cells,
+                 uint32_t out_f, uint32_t in_f, const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val,
+                 int64_t ldx, uint16_t *__restrict__ y, int64_t ldy) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t ln_smem[];
+    using P = LnPairs<BITS, false>;
+    const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)ln_smem;
+    const uint32_t C = shape & 255u, tiles_per_wg = (shape >> 8) & 255u, n_waves = 1u << ((shape >> 16) & 7u), m = 1u + (shape >> 20);
+    const bool x_aligned = (shape >> 19) & 1u;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t t0 = blockIdx.x * tiles_per_wg, cell0 = t0 * C, n_here = min(tiles_per_wg, ((out_f + 3u) >> 2) - t0) * C;
+    const uint32_t x_at = smem + P::kLutBytes, x_row = C * 1024u + kLnXPad;
+    float *const parts = reinterpret_cast<float *>(ln_smem + P::kLutBytes + MT * x_row);
+
+    // ---- all requests (for cells that a wave does not have, the last one's) ----
+    uint32_t bias_raw[N];
+#pragma unroll
+    for (uint32_t n = 0; n < N; ++n) bias_raw[n] = *(bias ? bias + min((t0 + wave + n * n_waves) * 4u + (lane & 3u), out_f - 1u) : scale_at);
+    const uint32_t scale_raw = *scale_at, col = tid * 8u;
+    ln_u32x4 xv[MT];
+    if (x_aligned)
+#pragma unroll
+        for (uint32_t r = 0; r < MT; ++r)
+            xv[r] = *reinterpret_cast<const ln_u32x4 *>(x + (int64_t)min(r, m - 1u) * ldx + ln_piece_column(col, in_f));
+    uint32_t w[N][BITS], e0[N], e1[N];
+#pragma unroll
+    for (uint32_t n = 0; n < N; ++n) {
+        const uint32_t cell = cell0 + min(wave + n * n_waves, n_here - 1u);
+        ln_load<BITS>(plane, cell, lane, w[n]);
+        e0[n] = exc_off[cell], e1[n] = exc_off[cell + 1u];
+    }
+    asm volatile("" ::"s"(y), "s"(ldy));  // (arguments that are read from memory: with these, not at the end)
+    // 64 quads of the list from a multiple of four on: the lane has four of its row
+    struct Listed { ln_u32x2 pos; uint32_t val; };
+    auto list_load = [&](uint32_t from, uint32_t end) {
+        const uint32_t at = min((from >> 2) + (lane >> 2), (max(end, 1u) - 1u) >> 2) * 16u + (lane & 3u) * 4u;
+        return Listed{*reinterpret_cast<const ln_u32x2 *>(exc_pos + at), *reinterpret_cast<const uint32_t *>(exc_val + at)};
+    };
+    Listed in[N];
+#pragma unroll
+    for (uint32_t n = 0; n < N; ++n) in[n] = list_load(e0[n] & ~3u, e1[n]);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- pair table and activations to LDS: a thread has the same piece of each row ----
+    const float scale = bf16_bits_to_f32(scale_raw);
+    ln_build_lut<BITS, false>(smem, scale, tid, n_waves * kWave);
+    if (tid < MT * (kLnXPad / 16u))
+        *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + tid / (kLnXPad / 16u) * x_row + C * 1024u + tid % (kLnXPad / 16u) * 16u)) =
+            ln_u32x4{0, 0, 0, 0};
+    if (tid < C * 64u) {
+#pragma unroll
+        for (uint32_t r = 0; r < MT; ++r) {
+            ln_u32x4 v = {0u, 0u, 0u, 0u};
+            if (x_aligned && col + 8u <= in_f) {
+                if (r < m) v = xv[r];
+            } else if (r < m) {
+                const uint16_t *const src = x + (int64_t)r * ldx;
+                uint32_t h[8];
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k) h[k] = src[min(col + k, in_f - 1u)];
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k)
+                    v[k] = (col + 2u * k < in_f ? h[2 * k] : 0u) | (col + 2u * k + 1u < in_f ? h[2 * k + 1] << 16 : 0u);
+            }
+            *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + r * x_row + lane_offset(col))) = v;
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+    const uint32_t lut_lane = smem + ((lane & ((1u << P::kCopies) - 1u)) << 2);
+    const uint32_t q = lane >> 4, kg = lane & 3u, am = min((lane >> 2) & 3u, (uint32_t)MT - 1u), x_lane = x_at + am * x_row + q * 256u + kg * 16u;
+    const bool kg0 = (lane & 4u) != 0, kg1 = (lane & 8u) != 0;
+#pragma unroll
+    for (uint32_t n = 0; n < N; ++n) {
+        // ---- the cell's products (see k_lanes_gemv) ----
+        if (n && wave + n * n_waves >= n_here) break;
+        const uint32_t cell = wave + n * n_waves, x_cell = x_lane + (cell - ((cell * inv_cells) >> 16) * C) * 1024u;
+        uint32_t o[16];
+        ln_decode<BITS, false>(w[n], lut_lane, scale, o);
+        ln_f32x4 d = {0, 0, 0, 0};
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const ln_u32x4 a = *reinterpret_cast<const LN_LDS(ln_u32x4) *>((uintptr_t)(x_cell + ((i ^ q) << 6)));
+            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ln_bf16x8, a),
+                                                        __builtin_bit_cast(ln_bf16x8, ln_u32x4{o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]}), d, 0, 0, 0);
+        }
+        float v = kg1 ? (kg0 ? d[3] : d[2]) : (kg0 ? d[1] : d[0]);
+        v += ln_dpp<0x124>(v);
+        v += ln_dpp<0x128>(v);
+        // ---- its listed elements (a first group also where there are none: behind a branch it would not be asked for before it) ----
+        float ex[MT];
+#pragma unroll
+        for (int r = 0; r < MT; ++r) ex[r] = 0.0f;
+        uint32_t from = e0[n] & ~3u;
+#pragma unroll 1
+        for (;;) {
+            const uint32_t at[4] = {x_at + (in[n].pos[0] & 0xFFFFu), x_at + (in[n].pos[0] >> 16), x_at + (in[n].pos[1] & 0xFFFFu), x_at + (in[n].pos[1] >> 16)};
+            float p[4][MT];
+            lv_listed<MT>(at, in[n].val, scale, x_row, p);
+            const uint32_t quad = from + (lane & ~3u) - e0[n];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+#pragma unroll
+                for (int r = 0; r < MT; ++r) ex[r] += quad + k < e1[n] - e0[n] ? p[k][r] : 0.0f;
+            from += 64u;
+            if (from >= e1[n]) break;
+            in[n] = list_load(from, e1[n]);
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < MT; ++r) {
+            const float sum = lv_row_sum(ex[r]);
+            v += lane >> 4 == r ? sum : 0.0f;
+        }
+        if (cell < n_here && (lane & 12u) == 0 && lane < MT * 16u) parts[cell * (MT * 4u) + (lane >> 4) * 4u + (lane & 3u)] = v;
+    }
+    __syncthreads();
+
+    // ---- outputs: a row quad's sums over the columns ----
+#pragma unroll
+    for (uint32_t n = 0; n < N; ++n) {
+        const uint32_t t = wave + n * n_waves, at = lane & (MT * 4u - 1u), out_row = (t0 + t) * 4u + (lane & 3u), r = lane >> 2;
+        if (t * C >= n_here) break;
+        float sum = 0.0f;
+        for (uint32_t k = lane / (MT * 4u); k < C; k += 64u / (MT * 4u)) sum += parts[(t * C + k) * (MT * 4u) + at];
+        if (MT == 1) sum += ln_dpp<0x124>(sum);
+        if (MT <= 2) sum += ln_dpp<0x128>(sum);
+        sum = lv_sum_of_rows(sum);
+        if (r < m && out_row < out_f) {
+            uint32_t b = f32_to_bf16_bits(sum);
+            if (bias) b = f32_to_bf16_bits(bf16_bits_to_f32(b) + bf16_bits_to_f32(bias_raw[n]));
+            y[(int64_t)r * ldy + out_row] = (uint16_t)b;
         }
     }
 }
@@ -509,17 +666,37 @@ template <int BITS, int MT, bool WIDE> static LvSplit lv_split(const LanesDev &L
     return best;
 }
 
+// row quads by `tiles` to a workgroup of `waves`, N cells a wave
+template <int BITS, int MT, int N>
+static int lanes_gemv_few_launch(const LanesDev &L, uint32_t tiles, uint32_t waves, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias,
+                                 uint16_t *y, int64_t ldy, hipStream_t s) {
+    const size_t lds = LnPairs<BITS, false>::kLutBytes + MT * (L.n_cells * 1024u + kLnXPad) + tiles * L.n_cells * (MT * 16u);
+    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemv_few<BITS, MT, N>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
+    if (!raised) return IXH_ELAUNCH;
+    const bool aligned = ln_whole_pieces((uintptr_t)x, L.in_f, m, ldx);
+    const uint32_t shape = L.n_cells | tiles << 8 | (uint32_t)__builtin_ctz(waves) << 16 | (uint32_t)aligned << 19 | (uint32_t)(m - 1) << 20;
+    // (a cell / n_cells as a product with 2^16 / n_cells, rounded up: exact for the 32 cells that there are at most)
+    hipLaunchKernelGGL((k_lanes_gemv_few<BITS, MT, N>), dim3((L.n_tiles + tiles - 1u) / tiles), dim3(kWave * waves), lds, s, L.plane, x, L.exc_off,
+                       L.scale, bias, shape, 65536u / L.n_cells + 1u, L.out_f, L.in_f, L.exc_pos, L.exc_val, ldx, y, ldy);
+    return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
+}
+
 template <int BITS, int MT, bool WIDE>
 static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                              int64_t ldy, hipStream_t s) {
     const auto [best_waves, best_tiles] = lv_split<BITS, MT, WIDE>(L);
-    // The smaller pair table where rows are too long beside the larger one, and for a few cells a CU, which gain less from it than
-    // its 64 KB take to write (5 bits, one row, larger / smaller: 512 x 512 6.6 / 4.2 us, 900 x 3072 with 6 cells a CU 5.0 / 4.4, 2000
-    // x 4096 with 16 5.7 / 5.6, 4000 x 3072 with 24 6.4 / 6.4, 5000 x 5120 with 50 7.8 / 8.1).
-    if constexpr (WIDE && (BITS == 4 || BITS == 5)) {
-        const bool few = best_waves && best_tiles * L.n_cells * (16u / best_waves) <= 16u;
-        if (few || (!best_waves && MT <= 2)) return lanes_gemv_launch<BITS, MT, false>(L, x, m, ldx, bias, y, ldy, s);
+    // A cell or two a wave: up to two cells a wave k_lanes_gemv is slower or even, see there.  (A thread takes one piece of a row of activations:
+    // no more cells in a row than waves.)
+    if (best_waves && L.n_cells <= best_waves && best_tiles * L.n_cells <= 2u * best_waves) {
+        uint32_t waves = best_waves;
+        while (waves / 2u >= best_tiles * L.n_cells) waves /= 2u;
+        if (best_tiles * L.n_cells <= waves) return lanes_gemv_few_launch<BITS, MT, 1>(L, best_tiles, waves, x, m, ldx, bias, y, ldy, s);
+        return lanes_gemv_few_launch<BITS, MT, 2>(L, best_tiles, waves, x, m, ldx, bias, y, ldy, s);
     }
+    // the smaller pair table where rows are too long beside the larger one
+    if constexpr (WIDE && (BITS == 4 || BITS == 5) && MT <= 2)
+        if (!best_waves) return lanes_gemv_launch<BITS, MT, false>(L, x, m, ldx, bias, y, ldy, s);
     if (!best_waves) return IXH_EUNSUPPORTED;
     uint32_t log_waves = 31u - (uint32_t)__builtin_clz(best_waves);
     while ((1u << log_waves) > best_tiles * L.n_cells) --log_waves;

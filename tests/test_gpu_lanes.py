@@ -126,6 +126,17 @@ def test_list_of_one_segment_of_long_rows(oracle, dev, at, listed):
         check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
 
 
+@pytest.mark.parametrize("kind", ["rare", "four", "real", "full_row", "wide"])
+@pytest.mark.parametrize("out_f,in_f", [(4096, 2048), (4093, 2041), (17 * 1024 - 3, 512), (8192, 2048), (8185, 2040), (8200, 2048), (40, 8192), (40, 8200)])
+def test_a_cell_or_two_a_wave(oracle, dev, kind, out_f, in_f):
+    """16, 17, 32 and 36 cells a workgroup, its last row quads incomplete or missing; rows of as many cells as waves and of one more."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    for m in (1, 2, 3, 4):
+        x = activations(m, in_f + 8, seed=m)[:, 8 * (m % 2) :][:, :in_f]
+        check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f, bias.to(dev) if m > 1 else None), bias if m > 1 else None)
+
+
 @pytest.mark.parametrize("kind", ["rare", "real"])
 @pytest.mark.parametrize("out_f", [63488, 70000])
 def test_more_row_quads_than_a_wave_has_lanes(oracle, dev, kind, out_f):
@@ -292,7 +303,7 @@ def test_prompts_of_a_layer_take_the_lanes_in_every_form(oracle, dev):
 
 
 @pytest.mark.parametrize("kind,out_f,in_f", [(k, 67, 1000) for k in ("narrow", "rare", "four", "real", "full_row", "wide")] +
-                         [("real", 9, 511), ("rare", 6, 32000), ("real", 6, 32768), ("real", 6, 33800)])
+                         [("real", 9, 511), ("real", 6000, 1032), ("rare", 6, 32000), ("real", 6, 32768), ("real", 6, 33800)])
 def test_infinite_activations(oracle, dev, kind, out_f, in_f):
     """An infinite activation gives an infinity of the right sign, or NaN where a row's own weight is zero or another
     infinity meets it: where the list's padding points (column 0), in columns with listed elements and in others."""

@@ -39,22 +39,25 @@ def spilled(tmp_path):
     return found
 
 
-def denormal_modes(code):
-    """{kernel: its descriptor's mode for fp32 denormals}: 3 where they are kept, 0 where they are flushed."""
+def symbols(code):
+    """(name, its bytes' place in the code object, their number) of all symbols that have a place."""
     sections, section_size, n_sections = struct.unpack_from("<Q10xHH", code, 0x28)[0], *struct.unpack_from("<HH", code, 0x3A)
     headers = [struct.unpack_from("<IIQQQQIIQQ", code, sections + i * section_size) for i in range(n_sections)]
-    found = {}
     for _, kind, _, _, offset, size, link, _, _, _ in headers:
         if kind != 2:  # the symbol table
             continue
         names = headers[link][4]
         for at in range(offset, offset + size, 24):
             name_at, _, _, section, value, length = struct.unpack_from("<IBBHQQ", code, at)
-            name = code[names + name_at : code.index(b"\0", names + name_at)].decode()
-            if name.endswith(".kd") and length == 64:
-                start = value - headers[section][3] + headers[section][4]
-                found[name[:-3]] = (struct.unpack_from("<I", code, start + 48)[0] >> 16) & 3
-    return found
+            if section and section < n_sections:
+                name = code[names + name_at : code.index(b"\0", names + name_at)].decode()
+                yield name, value - headers[section][3] + headers[section][4], length
+
+
+def denormal_modes(code):
+    """{kernel: its descriptor's mode for fp32 denormals}: 3 where they are kept, 0 where they are flushed."""
+    return {name[:-3]: (struct.unpack_from("<I", code, at + 48)[0] >> 16) & 3 for name, at, length in symbols(code)
+            if name.endswith(".kd") and length == 64}
 
 
 @pytest.mark.skipif(READELF is None or not os.path.exists(LIB), reason="needs the built library and llvm-readelf")
@@ -72,6 +75,17 @@ def test_kernels_keep_denormals():
         found.update(denormal_modes(code))
     assert sum("k_lanes_" in name or "dense" in name for name in found) > 50
     assert [name for name, mode in found.items() if mode != 3] == []
+
+
+@pytest.mark.skipif(not os.path.exists(LIB), reason="needs the built library")
+def test_kernels_of_small_layers_are_short():
+    """A launch fetches its instructions anew, and a small layer of a graph waits for little else: its kernel has at most half of
+    k_lanes_gemv's."""
+    size = {name: length for code in code_objects(open(LIB, "rb").read()) for name, _, length in symbols(code) if "k_lanes_gemv" in name and not name.endswith(".kd")}
+    of = lambda *parts: next(length for name, length in size.items() if all(p in name for p in parts))
+    for bits in (3, 4, 5, 8):
+        for rows in (1, 2, 4):
+            assert of("k_lanes_gemv_fewI", f"ILi{bits}ELi{rows}ELi1E") <= 0.5 * of("k_lanes_gemvI", f"ILi{bits}ELi{rows}ELb1E")
 
 
 @pytest.mark.skipif(shutil.which(HIPCC) is None, reason="needs hipcc")
