@@ -34,9 +34,10 @@ LN_BOTH uint32_t ln_listed_at(uint32_t pos, uint32_t value, bool in_range, uint3
 // first of sixteen waves has 1.47 times the mean, the last one 0.53 times: a SIMD serves the oldest of its waves first, so the last ones
 // have their first cells 1.4 us after the first ones and in even shares end 1.6 to 2 us after them (us a layer, even shares /
 // 1.12 .. 0.88 / 1.23 .. 0.77 / 1.47 .. 0.53 / 1.6 .. 0.4 of the mean: 17408 x 5120 at 5 bits 14.4 / 14.2 / 14.0 / 13.8 / 14.1, 5120 x
-// 5120 7.3 / 7.2 / 7.3 / 7.0 / 7.1, 5120 x 17408 at 3 bits 10.4 / 10.5 / 10.2 / 10.5 / 10.8).
+// 5120 7.3 / 7.2 / 7.3 / 7.0 / 7.1, 5120 x 17408 at 3 bits 10.4 / 10.5 / 10.2 / 10.5 / 10.8).  That lead does not grow with the layer: from
+// 256 cells on the first wave has 7.5 more than the mean (8192 x 65536 at 3 bits with 0.53 to 1.47 of it 52.3, so 47.1).
 LN_BOTH uint32_t ln_share(uint32_t n, uint32_t wave, uint32_t log_waves) {
-    return (n * wave * (32u + (1u << log_waves) - wave)) >> (log_waves + 5u);
+    return (32u * n * wave + (n < 256u ? n : 256u) * wave * ((1u << log_waves) - wave)) >> (log_waves + 5u);
 }
 
 // Activations: 16-byte pieces of whole rows are asked for before anything else where every row starts 16-byte aligned and

@@ -89,6 +89,7 @@ def test_shares_of_the_cells_follow_one_another(bounds, log_waves):
         ends = [bounds.share(n, w, log_waves) for w in range(waves + 1)]
         assert ends[0] == 0 and ends[-1] == n and ends == sorted(ends)
         assert n < 32 * waves or 0.5 * n <= waves * min(b - a for a, b in zip(ends, ends[1:]))
+        assert all(abs(b - a - n / waves) < 9 for a, b in zip(ends, ends[1:]))  # (a lead of some cells, however many there are)
 
 
 @pytest.mark.parametrize("cells", [1, 2, 3, 5, 34])
