@@ -653,8 +653,18 @@ struct LvSplit { uint32_t waves, tiles; };
 template <int BITS, int MT, bool WIDE> static size_t lv_lds(const LanesDev &L, uint32_t tiles, uint32_t waves) {
     return LnPairs<BITS, WIDE>::kLutBytes + (size_t)MT * (L.n_cells * 1024u + kLnXPad) + ((size_t)tiles * (L.n_cells + 1u) + waves) * (MT * 16u) + tiles * 4u;
 }
+// Several rows of layers of many row quads a CU and few cells to each: k_lanes_rows, which has 16 weight rows to a wave's sums, is faster (us from
+// graphs, k_lanes_gemv / k_lanes_rows, at 3 / 4 / 5 bits: four rows 24576 x 5120 18.7 / 21.3 / 23.7 and 17.9 / 21.4 / 24.3, 32768 x 4096 19.9 / 22.1 / 24.9
+// and 16.9 / 21.3 / 24.0, 131072 x 1024 28.8 / 29.3 / 32.5 and 18.3 / 22.3 / 25.4; two rows 32768 x 1024 10.9 / 11.5 / 12.0 and 10.4 / 11.2 / 12.3, 65536 x
+// 2048 19.7 / 21.5 / 23.2 and 17.2 / 21.1 / 23.8, 248320 x 1024 36.7 / 45.1 / 51.3 and 28.8 / 43.4 / 50.9; 128256 x 4096 at 3 and 5 bits 51.7 / 84.3 and before
+// k_lanes_gemv had the room 57.5 / 92.3).
+template <int MT> static bool lv_rows_win(const LanesDev &L) {
+    const uint32_t tiles = (L.n_tiles + ln_cus() - 1) / ln_cus();
+    return MT == 4 ? tiles > 30u && tiles * L.n_cells > 32u : MT == 2 && tiles > 60u && L.n_cells <= 4u;
+}
 template <int BITS, int MT, bool WIDE> static LvSplit lv_split(const LanesDev &L) {
     LvSplit best{};
+    if (lv_rows_win<MT>(L)) return best;
     uint64_t best_cost = ~0ull;
     for (uint32_t per_cu = 1; per_cu <= 4; per_cu *= 2) {
         const uint32_t waves = 16u / per_cu, slots = ln_cus() * per_cu;

@@ -257,3 +257,17 @@ def test_malformed_lane_layouts():
         s = good()
         setattr(s, field, value)
         assert call(s) == -1 and needle in lib.ixh_last_error().decode(), (field, value, lib.ixh_last_error())
+
+
+def test_several_rows_of_many_row_quads_are_not_the_gemv_kernels():
+    """Three and four rows of layers of more than 30 row quads a CU go to the kernel of 16 weight rows a wave (told by the scratch that it
+    takes on a layer of this size, where the one-row kernel takes none)."""
+    lib = _lib.lib()
+
+    def need(out_f, in_f, bits, rows):
+        words = lib.ixh_lanes_plane_words(out_f, in_f, bits)
+        s = _lib.IxhLanes(bits, out_f, in_f, 0x1000, words, 0x1000, 0x1000, 0x1000, 64, 0x1000)
+        return lib.ixh_lanes_gemv_workspace_bytes(C.byref(s), rows)
+
+    assert need(65536, 5120, 5, 3) > 0 and need(65536, 5120, 5, 4) > 0
+    assert need(65536, 5120, 5, 1) == 0 and need(17408, 5120, 5, 4) == 0
