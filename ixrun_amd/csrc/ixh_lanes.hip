@@ -54,7 +54,7 @@ __device__ __forceinline__ void lv_listed(const uint32_t (&at)[4], uint32_t vals
 // each 32, and its row 4 r + kg is activation row r at the columns kg, so that a lane's sum of its own kg is one of its four results and
 // the twelve others (columns of one kg, activations of another) are thrown away.  A cell's sums over the four kg go to LDS; the row
 // quad's outputs add them up in column order.  Four matrix instructions a cell, up to four activation rows, and no sums in registers
-// over the loop.
+// over the loop.  (k_lanes_gemv_by_wave: a wave adds the cells of a row quad up in LDS, in their order, where cells are too many for a place each.)
 //
 // A wave has two cells in flight, one of them before the activations are there, and the loop over its ten or so cells is short:
 // what is asked for early keeps the activations of the workgroup's later waves waiting, and much of what a launch fetches is
@@ -78,12 +78,12 @@ constexpr uint32_t kLnListAhead = 1;  // groups of the list in flight
 constexpr uint32_t kLnXAhead = 3;     // 16-byte pieces of the activations a thread asks for before anything else
 constexpr uint32_t kLnXPad = 64;      // bytes behind a row of activations in LDS: zeros
 
-template <int BITS, int MT, bool WIDE>
-__global__ void __launch_bounds__(1024)
-k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
-             const uint16_t *__restrict__ scale_at, uint32_t shape, uint32_t all_tiles, uint32_t tiles_per_wg, uint32_t in_f,
-             uint32_t inv_tiles, uint32_t list_groups, const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, int64_t ldx,
-             const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, uint32_t out_f) {
+#define LV_ARGUMENTS                                                                                                                     \
+    const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,                            \
+        const uint16_t *__restrict__ scale_at, uint32_t shape, uint32_t all_tiles, uint32_t tiles_per_wg, uint32_t in_f,                 \
+        uint32_t inv_tiles, uint32_t list_groups, const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, int64_t ldx, \
+        const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, uint32_t out_f
+template <int BITS, int MT, bool WIDE, bool BY_WAVE> __device__ __forceinline__ void lv_gemv(LV_ARGUMENTS) {
     extern __shared__ __attribute__((aligned(16))) uint8_t ln_smem[];
     const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)ln_smem;
     // (what the first requests need lies in the arguments that the hardware loads into registers)
@@ -97,7 +97,7 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     const uint32_t s0 = ln_share(n_seq, wave, log_waves), s1 = ln_share(n_seq, wave + 1u, log_waves);
     const uint32_t x_at = smem + LnPairs<BITS, WIDE>::kLutBytes, x_row = C * 1024u + kLnXPad, x_pieces = MT * C * 64u;
     float *const parts = reinterpret_cast<float *>(ln_smem + LnPairs<BITS, WIDE>::kLutBytes + MT * x_row);
-    float *const list_parts = parts + n_seq * (MT * 4u);  // of wave w and row quad t at t + w
+    float *const list_parts = parts + (BY_WAVE ? tiles_per_wg << log_waves : n_seq) * (MT * 4u);  // of wave w and row quad t at t + w
     uint32_t *const list_waves = reinterpret_cast<uint32_t *>(list_parts + (tiles_per_wg + n_waves) * (MT * 4u));
 
     auto x_piece = [&](uint32_t e) {
@@ -166,6 +166,8 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     const float scale = bf16_bits_to_f32(scale_raw);
     ln_build_lut<BITS, WIDE>(smem, scale, tid, n_threads);
     for (uint32_t e = tid; e < n_tiles; e += n_threads) list_waves[e] = 0u;
+    if constexpr (BY_WAVE)
+        for (uint32_t e = tid; e < (tiles_per_wg << log_waves) * (MT * 4u); e += n_threads) parts[e] = 0.0f;
     if (tid < MT * (kLnXPad / 16u))
         *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(x_at + tid / (kLnXPad / 16u) * x_row + C * 1024u + tid % (kLnXPad / 16u) * 16u)) =
             ln_u32x4{0, 0, 0, 0};
@@ -286,9 +288,12 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     };
     x_read();
     const bool kg0 = (lane & 4u) != 0, kg1 = (lane & 8u) != 0;
-    uint32_t part_at = (uint32_t)(uintptr_t)(LN_LDS(float) *)parts + s0 * (MT * 16u) + (lane >> 4) * 16u + (lane & 3u) * 4u;
+    uint32_t part_at = (uint32_t)(uintptr_t)(LN_LDS(float) *)parts + (BY_WAVE ? wave * tiles_per_wg : s0) * (MT * 16u) + (lane >> 4) * 16u + (lane & 3u) * 4u;
     auto cell = [&](uint32_t (&w)[BITS], bool more) {
         uint32_t o[16];
+        float before = 0.0f;
+        const uint32_t to = BY_WAVE ? part_at + now.t * (MT * 16u) : part_at;
+        if constexpr (BY_WAVE) before = *reinterpret_cast<const LN_LDS(float) *>((uintptr_t)to);
         ln_decode<BITS, WIDE>(w, lut_lane, scale, o);
         if (more) load_next(w);
         ln_f32x4 d = {0, 0, 0, 0};
@@ -304,8 +309,8 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         float v = kg1 ? (kg0 ? d[3] : d[2]) : (kg0 ? d[1] : d[0]);
         v += ln_dpp<0x124>(v);
         v += ln_dpp<0x128>(v);
-        if ((lane & 12u) == 0 && lane < MT * 16u) *reinterpret_cast<LN_LDS(float) *>((uintptr_t)part_at) = v;
-        part_at += MT * 16u;
+        if ((lane & 12u) == 0 && lane < MT * 16u) *reinterpret_cast<LN_LDS(float) *>((uintptr_t)to) = BY_WAVE ? before + v : v;
+        if constexpr (!BY_WAVE) part_at += MT * 16u;
     };
     // Whole turns of the buffers, without a way out in between: with one the compiler takes the last request made before it
     // for the first buffer's and waits for all that is in flight at the top of every turn.
@@ -342,7 +347,7 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 #pragma unroll
         for (int r = 0; r < MT; ++r) {
             float sum = listed ? list_parts[(t + part) * (MT * 4u) + (uint32_t)r * 4u + (lane & 3u)] : 0.0f;
-            for (uint32_t c = part; c < C; c += 16u) sum += parts[(c * tiles_per_wg + t) * (MT * 4u) + (uint32_t)r * 4u + (lane & 3u)];
+            for (uint32_t c = part; c < (BY_WAVE ? n_waves : C); c += 16u) sum += parts[(c * tiles_per_wg + t) * (MT * 4u) + (uint32_t)r * 4u + (lane & 3u)];
             sum = lv_row_sum(sum);
             if (lane < 4 && at < out_f && (uint32_t)r < m) {
                 uint32_t b = f32_to_bf16_bits(sum);
@@ -352,6 +357,16 @@ k_lanes_gemv(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
         }
     }
 }
+
+#define LV_PASSED plane, x, exc_off, scale_at, shape, all_tiles, tiles_per_wg, in_f, inv_tiles, list_groups, exc_pos, exc_val, ldx, bias, y, ldy, out_f
+template <int BITS, int MT, bool WIDE> __global__ void __launch_bounds__(1024) k_lanes_gemv(LV_ARGUMENTS) {
+    lv_gemv<BITS, MT, WIDE, false>(LV_PASSED);
+}
+template <int BITS, int MT, bool WIDE> __global__ void __launch_bounds__(1024) k_lanes_gemv_by_wave(LV_ARGUMENTS) {
+    lv_gemv<BITS, MT, WIDE, true>(LV_PASSED);
+}
+#undef LV_ARGUMENTS
+#undef LV_PASSED
 
 // ---------------------------------------------------------------------------------------------------------------
 // k_lanes_gemv_few<BITS, MT, N>: the same where a wave has one cell, or two (N).
@@ -650,8 +665,8 @@ int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_
 // Workgroups of 16, 8 or 4 waves, one, two or four to a CU: the split whose last round of row quads is fullest.  No waves where LDS
 // holds none: its first pass, sixteen waves, decides that.
 struct LvSplit { uint32_t waves, tiles; };
-template <int BITS, int MT, bool WIDE> static size_t lv_lds(const LanesDev &L, uint32_t tiles, uint32_t waves) {
-    return LnPairs<BITS, WIDE>::kLutBytes + (size_t)MT * (L.n_cells * 1024u + kLnXPad) + ((size_t)tiles * (L.n_cells + 1u) + waves) * (MT * 16u) + tiles * 4u;
+template <int BITS, int MT, bool WIDE, bool BY_WAVE> static size_t lv_lds(const LanesDev &L, uint32_t tiles, uint32_t waves) {
+    return LnPairs<BITS, WIDE>::kLutBytes + (size_t)MT * (L.n_cells * 1024u + kLnXPad) + ((size_t)tiles * ((BY_WAVE ? waves : L.n_cells) + 1u) + waves) * (MT * 16u) + tiles * 4u;
 }
 // Several rows of layers of many row quads a CU and few cells to each: k_lanes_rows, which has 16 weight rows to a wave's sums, is faster (us from
 // graphs, k_lanes_gemv / k_lanes_rows, at 3 / 4 / 5 bits: four rows 24576 x 5120 18.7 / 21.3 / 23.7 and 17.9 / 21.4 / 24.3, 32768 x 4096 19.9 / 22.1 / 24.9
@@ -662,14 +677,14 @@ template <int MT> static bool lv_rows_win(const LanesDev &L) {
     const uint32_t tiles = (L.n_tiles + ln_cus() - 1) / ln_cus();
     return MT == 4 ? tiles > 30u && tiles * L.n_cells > 32u : MT == 2 && tiles > 60u && L.n_cells <= 4u;
 }
-template <int BITS, int MT, bool WIDE> static LvSplit lv_split(const LanesDev &L) {
+template <int BITS, int MT, bool WIDE, bool BY_WAVE = false> static LvSplit lv_split(const LanesDev &L) {
     LvSplit best{};
     if (lv_rows_win<MT>(L)) return best;
     uint64_t best_cost = ~0ull;
     for (uint32_t per_cu = 1; per_cu <= 4; per_cu *= 2) {
         const uint32_t waves = 16u / per_cu, slots = ln_cus() * per_cu;
         const uint32_t tiles = (L.n_tiles + slots - 1) / slots;
-        if (lv_lds<BITS, MT, WIDE>(L, tiles, waves) * per_cu > kLnLds) break;
+        if (lv_lds<BITS, MT, WIDE, BY_WAVE>(L, tiles, waves) * per_cu > kLnLds) break;
         const uint64_t cost = (uint64_t)tiles * per_cu;  // row quads a CU works through
         if (cost < best_cost) { best_cost = cost; best = {waves, tiles}; }
     }
@@ -692,10 +707,10 @@ static int lanes_gemv_few_launch(const LanesDev &L, uint32_t tiles, uint32_t wav
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
-template <int BITS, int MT, bool WIDE>
+template <int BITS, int MT, bool WIDE, bool BY_WAVE = false>
 static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                              int64_t ldy, hipStream_t s) {
-    const auto [best_waves, best_tiles] = lv_split<BITS, MT, WIDE>(L);
+    const auto [best_waves, best_tiles] = lv_split<BITS, MT, WIDE, BY_WAVE>(L);
     // A cell or two a wave: up to two cells a wave k_lanes_gemv is slower or even, see there.  (A thread takes one piece of a row of activations:
     // no more cells in a row than waves.)
     if (best_waves && L.n_cells <= best_waves && best_tiles * L.n_cells <= 2u * best_waves) {
@@ -704,13 +719,25 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
         if (best_tiles * L.n_cells <= waves) return lanes_gemv_few_launch<BITS, MT, 1>(L, best_tiles, waves, x, m, ldx, bias, y, ldy, s);
         return lanes_gemv_few_launch<BITS, MT, 2>(L, best_tiles, waves, x, m, ldx, bias, y, ldy, s);
     }
+    // Sums by wave where there is no room for sums by cell, which save an LDS read a cell (us from graphs, k_lanes_rows or the smaller
+    // pair table in their place / so: two rows 65536 x 20480 at 5 bits 227 / 203, 20480 x 30720 108 / 100, 16384 x 32768 at 3 bits 54.4 / 51.8, 4096 x 36864
+    // 20.4 / 21.5; one row 20480 x 40960 at 5 bits 129.6 / 125.8).
+    if constexpr (!BY_WAVE && MT <= 2)
+        if (!best_waves && L.n_cells > 16u) {
+            const int rc = lanes_gemv_launch<BITS, MT, WIDE, true>(L, x, m, ldx, bias, y, ldy, s);
+            if (rc != IXH_EUNSUPPORTED) return rc;
+        }
     // the smaller pair table where rows are too long beside the larger one
-    if constexpr (WIDE && (BITS == 4 || BITS == 5) && MT <= 2)
+    if constexpr (!BY_WAVE && WIDE && (BITS == 4 || BITS == 5) && MT <= 2)
         if (!best_waves) return lanes_gemv_launch<BITS, MT, false>(L, x, m, ldx, bias, y, ldy, s);
     if (!best_waves) return IXH_EUNSUPPORTED;
     uint32_t log_waves = 31u - (uint32_t)__builtin_clz(best_waves);
     while ((1u << log_waves) > best_tiles * L.n_cells) --log_waves;
-    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemv<BITS, MT, WIDE>),
+    const auto kernel = [] {
+        if constexpr (BY_WAVE) return k_lanes_gemv_by_wave<BITS, MT, WIDE>;
+        else return k_lanes_gemv<BITS, MT, WIDE>;
+    }();
+    static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
     // (the kernel's offsets of 16-byte pieces are 32 bits of elements)
@@ -719,8 +746,8 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
     // quotients by best_tiles as products with 2^32 / best_tiles, rounded up: exact for the cells of a workgroup, n_cells * best_tiles,
     // while these times best_tiles are below 2^32; each has 16 bytes of LDS
     const uint32_t inv_tiles = best_tiles == 1 ? 0u : (uint32_t)(((1ull << 32) + best_tiles - 1u) / best_tiles);
-    hipLaunchKernelGGL((k_lanes_gemv<BITS, MT, WIDE>), dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave << log_waves),
-                       (lv_lds<BITS, MT, WIDE>(L, best_tiles, 1u << log_waves)), s, L.plane, x, L.exc_off, L.scale, shape, L.n_tiles, best_tiles, L.in_f,
+    hipLaunchKernelGGL(kernel, dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave << log_waves),
+                       (lv_lds<BITS, MT, WIDE, BY_WAVE>(L, best_tiles, 1u << log_waves)), s, L.plane, x, L.exc_off, L.scale, shape, L.n_tiles, best_tiles, L.in_f,
                        inv_tiles, L.list_groups, L.exc_pos, L.exc_val, ldx, bias, y, ldy, L.out_f);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
@@ -738,8 +765,8 @@ static int lanes_gemv_rows(const LanesDev &L, const uint16_t *x, int m, int64_t 
 // whether lanes_gemv_launch finds a split
 template <int BITS> static bool lanes_gemv_fits(const LanesDev &L, int m) {
     constexpr bool SMALLER = BITS != 4 && BITS != 5;  // (a smaller table of pairs, up to two rows)
-    if (m == 1) return lv_split<BITS, 1, SMALLER>(L).waves != 0;
-    if (m == 2) return lv_split<BITS, 2, SMALLER>(L).waves != 0;
+    if (m == 1) return lv_split<BITS, 1, SMALLER>(L).waves != 0 || (L.n_cells > 16u && lv_split<BITS, 1, SMALLER, true>(L).waves != 0);
+    if (m == 2) return lv_split<BITS, 2, SMALLER>(L).waves != 0 || (L.n_cells > 16u && lv_split<BITS, 2, SMALLER, true>(L).waves != 0);
     return m <= 4 && lv_split<BITS, 4, true>(L).waves != 0;
 }
 bool lanes_gemv_takes(const LanesDev &L, int m) {

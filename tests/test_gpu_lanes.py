@@ -126,6 +126,16 @@ def test_list_of_one_segment_of_long_rows(oracle, dev, at, listed):
         check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
 
 
+@pytest.mark.parametrize("kind", ["rare", "real"])
+@pytest.mark.parametrize("out_f,in_f,m", [(1028, 37888, 2), (1025, 37380, 2), (1028, 75776, 1), (1028, 75771, 1)])
+def test_rows_that_leave_no_room_for_sums_of_cells(oracle, dev, kind, out_f, in_f, m):
+    """Two row quads a workgroup of as many cells as LDS holds the activations of: the waves' sums are kept instead."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    assert lanes.gemv_workspace_bytes(m) == 0
+    x = activations(m, in_f, seed=m)
+    check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
+
+
 @pytest.mark.parametrize("kind", ["rare", "four", "real", "full_row", "wide"])
 @pytest.mark.parametrize("out_f,in_f", [(4096, 2048), (4093, 2041), (17 * 1024 - 3, 512), (8192, 2048), (8185, 2040), (8200, 2048), (40, 8192), (40, 8200)])
 def test_a_cell_or_two_a_wave(oracle, dev, kind, out_f, in_f):
