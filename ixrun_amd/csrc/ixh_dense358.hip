@@ -52,13 +52,6 @@ struct DnWalk {
         return at;
     }
 };
-// the LDS addresses of a step's two slots (a slot below 2^16 is a multiple of the smallest float: its sum with itself takes half the time
-// of a shift left)
-__device__ __forceinline__ uint32_t dn_low_at(uint32_t at) {
-    const float low = __uint_as_float(at & 0xffffu);
-    return __float_as_uint(low + low);
-}
-__device__ __forceinline__ uint32_t dn_high_at(uint32_t at) { return (at >> 15) & 0x1fffeu; }
 typedef __bf16 d_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float d_f32x2 __attribute__((ext_vector_type(2)));
 
@@ -244,9 +237,9 @@ k_gemv358_dense(Dev P, const int32_t *__restrict__ prefix, uint32_t n_chunks, ui
                 const uint32_t at = walk.step(t);
                 const uint32_t x_lo = xr[t >> 1], x_hi = xr[8 + (t >> 1)];
                 // lanes past the span scatter zeros behind the last array's entries
-                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)dn_low_at(at)) =
+                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)slot_low_at(at)) =
                     (uint16_t)((t & 1) ? x_lo >> 16 : x_lo);
-                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)dn_high_at(at)) =
+                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)slot_high_at(at)) =
                     (uint16_t)((t & 1) ? x_hi >> 16 : x_hi);
             }
         }
@@ -575,8 +568,8 @@ __device__ __forceinline__ void dn_walk_spans(const Dev &P, const int32_t *__res
             for (int t = 0; t < 16; ++t) {
                 const uint32_t at = walk.step(t);
                 // positions past the end of the tensor walk on through the last array; what they read is not stored
-                const uint32_t va = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)dn_low_at(at));
-                const uint32_t vb = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)dn_high_at(at));
+                const uint32_t va = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)slot_low_at(at));
+                const uint32_t vb = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)slot_high_at(at));
                 if (t & 1) {
                     o[t >> 1] |= va << 16;
                     o[8 + (t >> 1)] |= vb << 16;

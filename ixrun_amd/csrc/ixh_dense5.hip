@@ -49,12 +49,6 @@ struct D5Walk {
         return at;
     }
 };
-// the LDS addresses of a step's two slots (the first one's as a sum of floats: a shift left takes twice its time)
-__device__ __forceinline__ uint32_t d5_low_at(uint32_t at) {
-    const float low = __uint_as_float(at & 0xffffu);
-    return __float_as_uint(low + low);
-}
-__device__ __forceinline__ uint32_t d5_high_at(uint32_t at) { return (at >> 15) & 0x1fffeu; }
 typedef __bf16 e_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float e_f32x2 __attribute__((ext_vector_type(2)));
 
@@ -331,9 +325,9 @@ k_gemv34568_dense(Dev P, const int32_t *__restrict__ prefix, uint32_t n_chunks, 
                 const uint32_t at = walk.step(t);
                 const uint32_t x_lo = xr[t >> 1], x_hi = xr[8 + (t >> 1)];
                 // lanes past the span scatter zeros behind the last array's entries
-                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)d5_low_at(at)) =
+                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)slot_low_at(at)) =
                     (uint16_t)((t & 1) ? x_lo >> 16 : x_lo);
-                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)d5_high_at(at)) =
+                *reinterpret_cast<__attribute__((address_space(3))) uint16_t *>((uintptr_t)slot_high_at(at)) =
                     (uint16_t)((t & 1) ? x_hi >> 16 : x_hi);
             }
         }
@@ -652,8 +646,8 @@ k_decode34568_dense(Dev P, const int32_t *__restrict__ prefix, uint32_t n_units,
             for (int t = 0; t < 16; ++t) {
                 const uint32_t at = walk.step(t);
                 // positions past the end of the tensor walk on through the last array; what they read is not stored
-                const uint32_t va = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)d5_low_at(at));
-                const uint32_t vb = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)d5_high_at(at));
+                const uint32_t va = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)slot_low_at(at));
+                const uint32_t vb = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>((uintptr_t)slot_high_at(at));
                 if (t & 1) {
                     o[t >> 1] |= va << 16;
                     o[8 + (t >> 1)] |= vb << 16;

@@ -59,6 +59,14 @@ __device__ __forceinline__ float scale_of(const GroupScales &g, float tensor_sca
     return g.fp16 ? fp16_bits_to_f32(g.fp16[p / g.group]) : tensor_scale;
 }
 
+// LDS addresses from the slots (address / 2) in the halves of a word.  (A slot below 2^16 is a multiple of the smallest float: its sum with
+// itself takes half the time of a shift left.  Denormals are kept, build.sh.)
+__device__ __forceinline__ uint32_t slot_low_at(uint32_t slots) {
+    const float low = __uint_as_float(slots & 0xffffu);
+    return __float_as_uint(low + low);
+}
+__device__ __forceinline__ uint32_t slot_high_at(uint32_t slots) { return (slots >> 15) & 0x1fffeu; }
+
 __device__ __forceinline__ int threshold_of(int bits) { return (1 << (bits - 1)) - 1; }
 
 // inclusive sum over the lanes at or below this one (DPP: shifts inside the 16-lane rows, then the two

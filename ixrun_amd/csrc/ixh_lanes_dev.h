@@ -62,7 +62,7 @@ __device__ __forceinline__ void ln_build_lut(uint32_t lut, float scale, uint32_t
 }
 
 // at + v * 2^SH for whole numbers below 2^24, as the bits of floats of which they are multiples of the smallest: exact, and two clocks of
-// issue where a shift left takes four and an add two more.  (Denormals are kept: the compiler's default here.)
+// issue where a shift left takes four and an add two more.  (Denormals are kept, build.sh.)
 template <int SH> __device__ __forceinline__ uint32_t ln_shift_add(uint32_t v, uint32_t at) {
     constexpr float by = SH >= 0 ? (float)(1 << (SH >= 0 ? SH : 0)) : 1.0f / (float)(1 << (SH < 0 ? -SH : 0));
     return __float_as_uint(__fmaf_rn(__uint_as_float(v), by, __uint_as_float(at)));
