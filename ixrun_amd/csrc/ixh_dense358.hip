@@ -659,10 +659,12 @@ k_decode358_dense(Dev P, const int32_t *__restrict__ prefix, uint32_t n_units, u
 // ---------------------------------------------------------------------------------------------------------------
 // The same without a rank table, for tensors of up to 2^22 weights: a workgroup counts the bitmaps in front of its spans itself, at
 // most eight spans, one a wave.  Bound by the latency of its chain (bitmap 0 up to the spans, bitmap 1 up to there, the spans' codes); at
-// 2^22 weights a workgroup reads up to 512 KB of bitmap 0, from the caches, which takes as long as the table's two launches and ends the
-// rule: with group scales, us from a graph, table / without: 256 x 512 9.8 / 5.9, 512 x 1024 10.2 / 6.9, 1024 x 1024 10.6 / 7.2, 1400 x
-// 1500 11.4 / 9.0, 2048 x 2048 12.7 / 11.8 to 12.9; called one by one, where three launches take the host as long, 14.6 / 9.6 up to
-// 1400 x 1500 and 14.5 / 11.8 to 12.9 at 2048 x 2048.
+// 2^22 weights a workgroup reads up to 512 KB of bitmap 0, from the caches, which takes nearly as long as the table's two launches.  The
+// rule ends there, with a span a wave in 256 workgroups; above it neither was timed.  us from a graph, table / without, with group scales: 256 x
+// 512 9.8 / 5.9, 512 x 1024 10.2 / 6.9, 1024 x 1024 10.6 / 7.2, 1400 x 1500 11.4 / 9.0, 2048 x 2048 12.7 / 11.8 to 12.9; of tensors with a
+// scale of their own, almost all in the first level (k_decode358_rows with the table) / at 55 / 40 / 5 %: 256 x 512 10.2 / 6.1 and 10.2 / 6.1, 1024 x
+// 1024 11.3 / 7.4 and 11.3 / 7.4, 1400 x 1500 12.1 / 9.5 and 12.3 / 9.8, 2048 x 2048 14.6 / 12.7 and 14.8 / 13.7; called one by one, where three
+// launches take the host as long, 16 / 8 to 9 up to 1400 x 1500 and 16 / 11.4 to 12.1 at 2048 x 2048.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kDnCountedWaves = 16, kDnCountedSpans = 8;
 static_assert(kDnCountedMost == 256u * kDnCountedSpans * kDnSpan, "up to 256 workgroups");

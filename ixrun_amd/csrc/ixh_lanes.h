@@ -74,8 +74,8 @@ struct LnScratch {
 
 int launch_lanes_pack(const uint16_t *w, const LanesDev &L, uint32_t *plane, uint32_t *counts, hipStream_t s);
 int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_t *val, hipStream_t s);
-// 1 to 16 rows; five and more, and fewer too long for k_lanes_gemv (which takes no scratch), go on to launch_lanes_rows, and some of
-// nine and more from there to launch_lanes_gemm
+// 1 to 16 rows; five and more, fewer too long for k_lanes_gemv (which takes no scratch), and two to four of very many row quads go on to
+// launch_lanes_rows, and some of nine and more from there to launch_lanes_gemm
 bool lanes_gemv_takes(const LanesDev &L, int m);
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                       int64_t ldy, LnScratch &ws, hipStream_t s);

@@ -69,8 +69,8 @@ __device__ __forceinline__ void lv_listed(const uint32_t (&at)[4], uint32_t vals
 // ahead 17408 x 5120 5 bits 14.9 for 14.4.  Taking the sign off costs two instructions an element; a plane without it turns an infinite
 // activation in a listed column into NaN.
 //
-// us a layer before / now: 5120 x 17408 3 bits 11.5 / 9.9 (10.5 before the look-ups' addresses took two instructions), 17408 x 5120 5 bits
-// 14.6 / 13.8, 4096 x 11008 9.3 / 8.9, 5120 x 5120 7.8 / 7.3, 17408 x 5120 with two rows at 5 bits 15.9 / 14.7, with four at 3 bits 15.3 / 13.1.
+// us a call where the last-level cache has the weights / from a graph over copies that it cannot hold, one row: 5120 x 17408 3 bits 9.9 / 12.7,
+// 17408 x 5120 5 bits 13.6 / 16.2, 4096 x 11008 8.7 / 11.2, 5120 x 5120 - / 7.65; at 5 bits 17408 x 5120 with two rows - / 18.0, with four - / 19.2.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kLnAhead = 2;      // cells in flight
 constexpr uint32_t kLnFirst = 1;      // of these, asked for before the activations are there
@@ -123,8 +123,11 @@ template <int BITS, int MT, bool WIDE, bool BY_WAVE> __device__ __forceinline__ 
     };
 
     // ---- everything that depends on nothing is asked for: scale, activations, the first cells, the list's extent ----
-    // (Past the end requests repeat the last cell, group or piece.  The compiler counts requests in flight, and one that may or
-    // may not have been made turns its counted waits into waits for all that is older.)
+    // (Past the end requests repeat the last group or piece.  The compiler counts requests in flight, and one that may or may not have been
+    // made turns its counted waits into waits for all that is older.  Requests for cells run on past a wave's share, up to two of them, the next
+    // wave's, and repeat only the workgroup's last column: row quad at most n_tiles - 1, column at most C - 1.  That is 7 to 10 % more
+    // bytes; turns that leave a share's last two cells to the loop behind them, and with that no request too many for an even share, took
+    // between 4.5 % less and 4.5 % more over 45 layers and rows, in the mean as long.)
     const uint32_t scale_raw = *scale_at;
     ln_u32x4 xv[kLnXAhead];
     if (x_aligned)

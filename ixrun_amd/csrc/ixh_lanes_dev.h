@@ -71,8 +71,8 @@ template <int SH> __device__ __forceinline__ uint32_t ln_shift(uint32_t w) {
     if constexpr (SH >= 0) return w >> SH;
     else return w << -SH;
 }
-// Where copies of a table do not collide: 5120 x 17408 (3 bits) at 1 / 8 / 16 / 64 rows 12.2 / 16.3 / 19.5 / 35.6 us with shifts, 11.8 /
-// 15.8 / 18.8 / 34.9 so, 10240 x 5120 (5 bits) at 1 / 8 rows 11.1 / 16.3 and 10.8 / 15.5.  With two copies the look-ups are what a wave waits
+// Where copies of a table do not collide: 5120 x 17408 (3 bits), from graphs over copies beyond the last-level cache, at 1 / 8 / 16 / 64 rows
+// 12.2 / 16.3 / 19.5 / 35.6 us with shifts, 11.8 / 15.8 / 18.8 / 34.9 so (one layer over and over, one row: 10.5 and 9.9), 10240 x 5120 (5 bits) at 1 / 8 rows 11.1 / 16.3 and 10.8 / 15.5.  With two copies the look-ups are what a wave waits
 // for: 1536 x 3072 (4 bits) at 12 / 32 rows 8.3 / 9.1 with shifts, 8.5 / 9.3 so, 10240 x 5120 (5 bits) at 128 rows 41.0 and 41.7.
 template <class P> constexpr bool ln_float_shifts = P::kCopies > 1;
 // the address of the pair whose code begins at bit OFF of a dword (without FLOAT less lut_lane)

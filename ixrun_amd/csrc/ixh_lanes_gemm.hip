@@ -7,12 +7,10 @@ namespace ixh {
 // k_lanes_gemm<BITS, MB, NB>: up to 16 * MB activation rows at a time, MB <= 8; NB blocks of 16 weight rows a wave (two from
 // MB = 4 on: an activation operand that is read serves both).
 //
-// Bound: a stage's parts, which follow one another in a wave, while all waves meet at its end, and LDS under them.  10240 x 5120 at 55 /
-// 40 / 5 %, 100 rows, clocks a stage of a wave before listed elements were stored as they are now: decode and its stores 2000, listed
-// elements 2000, activations to LDS 500, products 1500, barrier 1000, of a stage's list 500; 6000 before the first stage and 6000 for
-// the sums behind the last; no unit of the CU is busy for more than half of it (LDS 4000 of 7900 a stage).  37.6 us with the slices'
-// sums (44.2 when a lane held an element of each of four rows of the list, so that a store of listed elements went to a quarter of the
-// banks, 39.0 with a branch around each such store); 74.3 for the decode to memory and the library's GEMM.  Looking up the next stage's
+// Bound: a stage's parts (decode and its stores, listed elements, products), which follow one another in a wave, while all waves meet at its
+// end, and LDS under them; no unit of the CU is busy for more than half of a stage, the matrix unit for 12 %.  10240 x 5120 at 55 / 40 / 5 %,
+// 100 rows: 37.4 us with the slices' sums (44.2 when a lane held an element of each of four rows of the list, so that a store of listed elements
+// went to a quarter of the banks, 39.0 with a branch around each such store); 74.3 for the decode to memory and the library's GEMM.  Looking up the next stage's
 // weights between the products of this one changes nothing, nor do two workgroups of half the size on a CU; activations straight from
 // the L2 as operands take twice as long.  A wave takes 16 weight rows x 128 columns a stage: it decodes them to its own 4 KB of LDS in
 // operand order, stores the listed elements over their places and reads the operands back.  All waves of the workgroup are in the same

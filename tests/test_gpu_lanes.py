@@ -150,8 +150,8 @@ def test_a_cell_or_two_a_wave(oracle, dev, kind, out_f, in_f):
 @pytest.mark.parametrize("kind", ["rare", "real"])
 @pytest.mark.parametrize("out_f", [63488, 70000])
 def test_more_row_quads_than_a_wave_has_lanes(oracle, dev, kind, out_f):
-    """62 and 69 row quads a workgroup, whose lists begin in more places than a wave looks up at once; most have one group in many
-    row quads, or none."""
+    """62 and 69 row quads a workgroup, whose lists begin in more places than a wave looks up at once (one row; two and four of such layers
+    are the other kernel's); most have one group in many row quads, or none."""
     in_f = 40
     p, lanes = lay_out(kind, out_f, in_f, dev)
     for m in (1, 2, 4):
