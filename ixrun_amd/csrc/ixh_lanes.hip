@@ -419,7 +419,7 @@ k_lanes_gemv_few(const uint32_t *__restrict__ plane, const uint16_t *__restrict_
     // 64 quads of the list from a multiple of four on: the lane has four of its row
     struct Listed { ln_u32x2 pos; uint32_t val; };
     auto list_load = [&](uint32_t from, uint32_t end) {
-        const uint32_t at = min((from >> 2) + (lane >> 2), (max(end, 1u) - 1u) >> 2) * 16u + (lane & 3u) * 4u;
+        const uint32_t at = ln_four_quads(from, lane, end) * 16u + (lane & 3u) * 4u;
         return Listed{*reinterpret_cast<const ln_u32x2 *>(exc_pos + at), *reinterpret_cast<const uint32_t *>(exc_val + at)};
     };
     Listed in[N];

@@ -1,4 +1,4 @@
-// What a wave of k_lanes_gemv (ixh_lanes.hip) asks for ahead of knowing whether it needs it, and where the workgroups of
+// What a wave of k_lanes_gemv and k_lanes_gemv_few (ixh_lanes.hip) asks for ahead of knowing whether it needs it, and where the workgroups of
 // k_lanes_prompt (ixh_lanes_prompt.hip) leave their sums.  Plain C++, so that the ranges can be walked without a GPU.
 #pragma once
 #include <stdint.h>
@@ -21,6 +21,13 @@ LN_BOTH LnGroups ln_groups(uint32_t first_quad, uint32_t end_quad, uint32_t grou
     const uint32_t first = first_quad >> 6, end = (end_quad + 63u) >> 6;
     const uint32_t last = (end > first ? end : first + 1u) - 1u;
     return {first, last < groups ? last : groups - 1u, end_quad > first_quad ? last - first + 1u : 0u};
+}
+
+// k_lanes_gemv_few asks for 64 quads at a time from quad `from` (a multiple of four) on, four of them a lane: which four, of a cell
+// whose listed quads end at `end`.  Behind the last ones these are asked for again, also by a cell without any at a full list's end.
+LN_BOTH uint32_t ln_four_quads(uint32_t from, uint32_t lane, uint32_t end) {
+    const uint32_t at = (from >> 2) + (lane >> 2), last = (end ? end - 1u : 0u) >> 2;
+    return at < last ? at : last;
 }
 
 // Byte offset, in a row of `cells` cells of activations, of a listed element at position `pos` of segment `seg` (64 cells each), for rows

@@ -13,6 +13,7 @@ extern "C" void groups(uint32_t first, uint32_t end, uint32_t n, uint32_t *out) 
     const ixh::LnGroups g = ixh::ln_groups(first, end, n);
     out[0] = g.first; out[1] = g.last; out[2] = g.n;
 }
+extern "C" uint32_t four_quads(uint32_t from, uint32_t lane, uint32_t end) { return ixh::ln_four_quads(from, lane, end); }
 extern "C" int whole(uint64_t x, uint32_t in_f, int m, int64_t ldx) { return ixh::ln_whole_pieces(x, in_f, m, ldx); }
 extern "C" uint32_t column(uint32_t col, uint32_t in_f) { return ixh::ln_piece_column(col, in_f); }
 extern "C" uint32_t share(uint32_t n, uint32_t wave, uint32_t log_waves) { return ixh::ln_share(n, wave, log_waves); }
@@ -52,6 +53,24 @@ def test_requests_of_the_list_stay_in_it(bounds, total):
                 assert last == g_first + n - 1
             else:
                 assert n == 0
+
+
+@pytest.mark.parametrize("total", [0, 1, 3, 4, 63, 64, 65, 130, 192])
+def test_requests_of_a_cells_list_stay_in_the_list(bounds, total):
+    """Any part of a list of `total` quads as one cell's (also an empty one at its end), 64 quads at a time: no request goes behind the
+    list's last group, and each of the cell's quads is asked for by its own lanes."""
+    fours = 16 * max(-(-total // 64), 1)
+    for first in range(total + 1):
+        for end in range(first, total + 1):
+            asked, start = set(), first & ~3
+            while start == first & ~3 or start < end:
+                for lane in range(0, 64, 4):
+                    at = bounds.four_quads(start, lane, end)
+                    assert at < fours
+                    quad = start + lane
+                    asked |= {q for q in range(max(quad, first), min(quad + 4, end)) if q >> 2 == at}
+                start += 64
+            assert asked == set(range(first, end))
 
 
 @pytest.mark.parametrize("in_f", list(range(1, 34)) + [511, 512, 513, 1024, 1031])
