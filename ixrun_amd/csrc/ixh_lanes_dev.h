@@ -85,10 +85,9 @@ template <class P, int BITS, int OFF, bool FLOAT> __device__ __forceinline__ uin
     else return ((w >> (OFF - TO)) & P::kMask) + lut_lane;
 }
 
-// the sixteen dequantised pairs of a lane's `BITS` dwords; at 5 bits in the smaller table ARITH of the three whole pairs of a dword by
-// arithmetic (k_lanes_gemm with a block of weights a wave, whose waves all look up at the same time: two; 10240 x 5120 at 17 / 32 / 48
-// rows 23.7 / 24.4 / 26.8 us with one, 22.7 / 23.5 / 26.0 with two)
-template <int BITS, bool WIDE, int ARITH = 1, bool FLOAT = ln_float_shifts<LnPairs<BITS, WIDE>>>
+// the sixteen dequantised pairs of a lane's `BITS` dwords; at 5 bits in the smaller table one of the three whole pairs of a dword by
+// arithmetic
+template <int BITS, bool WIDE, bool FLOAT = ln_float_shifts<LnPairs<BITS, WIDE>>>
 __device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lut_lane, float scale, uint32_t (&o)[16]) {
     using P = LnPairs<BITS, WIDE>;
     if constexpr (BITS == 8) {
@@ -137,16 +136,11 @@ __device__ __forceinline__ void ln_decode(const uint32_t (&w)[BITS], uint32_t lu
                 const float lo = __uint_as_float(((w[d] >> 4) & 0x7C0000u) | 0x3F800000u);
                 const float hi = __uint_as_float(((w[d] >> 9) & 0x7C0000u) | 0x3F800000u);
                 o[PER * d + 2] = ln_pack(__fmaf_rn(lo, s32, off), __fmaf_rn(hi, s32, off));
-                if constexpr (ARITH > 1) {
-                    const float lo1 = __uint_as_float(((w[d] << 6) & 0x7C0000u) | 0x3F800000u);
-                    const float hi1 = __uint_as_float(((w[d] << 1) & 0x7C0000u) | 0x3F800000u);
-                    o[PER * d + 1] = ln_pack(__fmaf_rn(lo1, s32, off), __fmaf_rn(hi1, s32, off));
-                }
             }
         }
 #pragma unroll
         for (int p = 0; p < 16; ++p)
-            if (BITS != 5 || WIDE || p == 15 || p % 3 < 3 - ARITH)
+            if (BITS != 5 || WIDE || p == 15 || p % 3 < 2)
                 o[p] = *reinterpret_cast<const LN_LDS(uint32_t) *>((uintptr_t)(FLOAT ? a[p] : a[p] + lut_lane));
     }
 }

@@ -226,7 +226,7 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
         auto store = [&](uint32_t q) {  // stage q of the cell, to its half of the tile
             const uint32_t base = store_at + (q & 1u) * kLpTile;
             uint32_t o[16];
-            ln_decode<BITS, true, 1, FLOAT>(w[q % CODES], lut_lane, scale, o);
+            ln_decode<BITS, true, FLOAT>(w[q % CODES], lut_lane, scale, o);
 #pragma unroll
             for (uint32_t k = 0; k < 4; ++k)
                 *reinterpret_cast<LN_LDS(ln_u32x4) *>((uintptr_t)(base + ((k ^ q) << 10) + lane * 16u)) =
@@ -320,7 +320,7 @@ k_lanes_prompt(const uint32_t *__restrict__ plane, const ln_u32x4 *__restrict__ 
                         if (j == 0) {
                             if (b && b * PER % 4 == 0) piece(b * PER / 4 - 1);
                             uint32_t d[16];
-                            ln_decode<BITS, true, 1, FLOAT>(w[p % CODES], lut_lane, scale, d);
+                            ln_decode<BITS, true, FLOAT>(w[p % CODES], lut_lane, scale, d);
 #pragma unroll
                             for (uint32_t k = b * PER; k < b * PER + PER; ++k) o[k] = d[k];
                             __builtin_amdgcn_sched_barrier(0);

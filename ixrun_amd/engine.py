@@ -196,7 +196,7 @@ class StreamingLinear(nn.Module):
 
         MI355X, us from graphs, a layer without lanes (decode + library GEMM or, for tensors almost all level 1, ``ixh_gemm``)
         against this.  5 bits a weight (55 / 40 / 5 %) at 64 / 100 / 128 / 160 / 256 rows: 10240 x 5120 62 / 64 / 66 / 71 / 84
-        against 35 / 41 / 42 / 50 / 57, 17408 x 5120 90 / 94 / 94 / 101 / 115 against 55 / 65 / 70 / 75 / 85.  3 bits at 64 / 100 /
+        against 27 / 35 / 37 / 49 / 57, 17408 x 5120 90 / 94 / 94 / 101 / 115 against 42 / 55 / 61 / 75 / 85.  3 bits at 64 / 100 /
         200 / 256: 10240 x 5120 65 / 66 / 70 / 70 against 28 / 35 / 49 / 49, 17408 x 5120 96 / 101 / 111 / 115 against 46 / 53 / 76
         / 77.  8 bits, which have no list, at 64 / 100 / 160: 10240 x 5120 62 / 62 / 71 against 28 / 35 / 45, 17408 x 5120 102 /
         106 / 116 against 49 / 55 / 68, 4096 x 4096 30 / 31 / 39 against 17 / 23 / 24.  Below 2**24

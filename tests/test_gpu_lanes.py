@@ -272,6 +272,28 @@ def test_many_rows_of_larger_weights(oracle, dev, out_f, in_f, m):
     check(oracle, p, x, y)
 
 
+@pytest.mark.parametrize("scale", [2.0 ** -100, 1.5 * 2.0 ** 99, 2.0 ** 100, 1.75 * 2.0 ** 112])
+@pytest.mark.parametrize("kind", ["four", "real"])
+def test_many_rows_at_extreme_scales(oracle, dev, kind, scale):
+    """Multiples of the scale by up to 2^20 stand behind codes of five bits; from 2^100 on they would be infinities.  Every count of blocks of
+    16 activation rows."""
+    out_f, in_f = 260, 1032
+    v, scheme, _ = values(kind, out_f, in_f)
+    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
+    p["scale"] = torch.full_like(p["scale"], scale)
+    p, lanes = lay_out_values(p, out_f, in_f, dev)
+    for m in (17, 48, 64, 80, 96, 112, 128):
+        x = (activations(m, in_f, seed=m).float() * 2.0 ** -12).bfloat16()
+        y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
+        lanes.gemm(x.to(dev), y)
+        assert bool(y.isfinite().all())
+        # (a power of two takes the sums to where the oracle's squares are finite; it changes no rounding)
+        p_one = dict(p, scale=torch.full_like(p["scale"], scale * 2.0 ** -int(np.log2(scale))))
+        want = oracle.f32_to_bf16_bits(oracle.gemm_f64(oracle.decode_packed_bf16(p_one), bf16_bits(x)).astype(np.float32))
+        got = (y.double() * 2.0 ** -int(np.log2(scale))).cpu().numpy()
+        assert rel_l2(got, oracle.bf16_bits_to_f32(want)) <= 1e-3
+
+
 def test_prompts_of_a_layer_take_the_lanes_in_every_form(oracle, dev):
     """What goes to the fused decode+GEMM comes out as from the layer without lanes, whatever the activations' form; what it
     is not for (gradients, other types, more rows) still goes through the decode."""
