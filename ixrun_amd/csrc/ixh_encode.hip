@@ -72,7 +72,8 @@ __device__ __forceinline__ uint32_t enc_cut(int bits, float scale, float inv_sca
     return above == ~0ull ? 0u : (uint32_t)min(max(around + (int)__builtin_ctzll(above | 1ull << 63), 0), 0x7fff);
 }
 
-// Bound by HBM (a read of 178 MB: 37 us, 4.8 TB/s; more loads in flight or more workgroups change nothing).
+// Bound by HBM (a read of 178 MB: 37 us, 4.8 TB/s; more loads in flight or more workgroups change nothing); what is left
+// of a small weight's passes without loads in flight is 16 bytes a lane too (by single weights: 2^20 of them 4.3 -> 2.4 us).
 __global__ void __launch_bounds__(1024) k_enc_absmax(const uint16_t *__restrict__ w, uint32_t n, uint32_t *parts) {
     const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
     typedef uint16_t half2 __attribute__((ext_vector_type(2)));
@@ -92,6 +93,7 @@ __global__ void __launch_bounds__(1024) k_enc_absmax(const uint16_t *__restrict_
 #pragma unroll
         for (int k = 0; k < kEncAhead; ++k) take(q[k]);
     }
+    for (; aligned && base + 1024u * 8u <= n; base += stride) take(load8<true>(w, base + mine, n));
     for (; base < n; base += stride) take(load8<false>(w, base + mine, n));
     __shared__ uint32_t wave_m[16];
     uint32_t top = wave_max(max((uint32_t)m.x, (uint32_t)m.y));
