@@ -116,14 +116,17 @@ __global__ void __launch_bounds__(1024) k_enc_absmax(const uint16_t *__restrict_
 // four units.  Bound by its read, which the last-level cache serves in part: 5120 x 17408 in 28 us, 6.3 TB/s (35 when
 // every weight was quantised in fp32).
 constexpr uint32_t kCountUnits = 64;
+// Weights of no more units than make two such workgroups a CU have workgroups of 16, a turn a wave, which are over in one trip to memory (a
+// whole call, 64 / 16 units: 2048 x 2500 42.4 / 35.8 us, 3000 x 3000 47.2 / 40.8, 4096 x 4096 50.0 / 48.2, 4096 x 8192 68.7 / 73.2).
+constexpr uint32_t kCountFewUnits = 16, kCountFew = 32768;
 
-template <int L, bool kWhole>
+template <int L, bool kWhole, uint32_t UNITS>
 __device__ __forceinline__ void
 count_units(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, const uint32_t *__restrict__ parts,
             const EncLevels &lv, int32_t *table, uint32_t *sums, uint16_t *scale_out) {
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t u_first = blockIdx.x * kCountUnits + wave * (kCountUnits / kEncWaves);
-    constexpr int kTurns = kCountUnits / kEncWaves / 4;
+    const uint32_t u_first = blockIdx.x * UNITS + wave * (UNITS / kEncWaves);
+    constexpr int kTurns = UNITS / kEncWaves / 4;
     auto place = [&](int turn, int k) {
         return (uint64_t)(u_first + 4 * turn + (lane >> 4)) * kEncUnit + (lane & 15u) * 8u + 128u * k;
     };
@@ -196,15 +199,15 @@ count_units(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, const 
     }
 }
 
-template <int L>
+template <int L, uint32_t UNITS>
 __global__ void __launch_bounds__(kWave *kEncWaves)
 k_enc_count(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, const uint32_t *__restrict__ parts,
             EncLevels lv, int32_t *table, uint32_t *sums, uint16_t *scale_out) {
     const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
-    if (aligned && (uint64_t)(blockIdx.x + 1) * kCountUnits * kEncUnit <= n)
-        count_units<L, true>(w, n, n_units, parts, lv, table, sums, scale_out);
+    if (aligned && (uint64_t)(blockIdx.x + 1) * UNITS * kEncUnit <= n)
+        count_units<L, true, UNITS>(w, n, n_units, parts, lv, table, sums, scale_out);
     else
-        count_units<L, false>(w, n, n_units, parts, lv, table, sums, scale_out);
+        count_units<L, false, UNITS>(w, n, n_units, parts, lv, table, sums, scale_out);
 }
 
 // In place, per row: row[0] = 0, row[u + 1] = counts of units 0 .. u.  Each thread takes four consecutive entries; what
@@ -212,7 +215,7 @@ k_enc_count(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, const 
 // eight entries a thread, and sums from a kernel of their own: 14).
 struct __attribute__((packed, aligned(4))) Int4 { int32_t v[4]; };
 __global__ void __launch_bounds__(1024)
-k_enc_scan(int32_t *table, uint32_t n_units, const uint32_t *__restrict__ sums, uint32_t groups, int64_t *host_totals) {
+k_enc_scan(int32_t *table, uint32_t n_units, const uint32_t *__restrict__ sums, uint32_t groups, uint32_t group_units, int64_t *host_totals) {
     int32_t *row = table + (size_t)blockIdx.y * (n_units + 1);
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ uint32_t wave_s[16], wave_c[16];
@@ -228,7 +231,7 @@ k_enc_scan(int32_t *table, uint32_t n_units, const uint32_t *__restrict__ sums, 
     }
     uint32_t c = 0;
     const uint32_t *row_sums = sums + (size_t)blockIdx.y * groups;
-    for (uint32_t g = tid; g < blockIdx.x * (kScanTile / kCountUnits); g += 1024) c += row_sums[g];
+    for (uint32_t g = tid; g < blockIdx.x * (kScanTile / group_units); g += 1024) c += row_sums[g];
     c = wave_scan_inclusive(c);
     if (lane == 63) wave_c[wave] = c;
     const uint32_t mine = v[0] + v[1] + v[2] + v[3];
@@ -637,7 +640,11 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
 }
 
 // workspace: partial maxima (kEncParts), sums of k_enc_count's workgroups
-static uint32_t count_groups(uint64_t n) { return (uint32_t)((n + (uint64_t)kEncUnit * kCountUnits - 1) / ((uint64_t)kEncUnit * kCountUnits)); }
+static uint32_t group_units(uint64_t n) { return (n + kEncUnit - 1) / kEncUnit <= kCountFew ? kCountFewUnits : kCountUnits; }
+static uint32_t count_groups(uint64_t n) {
+    const uint64_t group = (uint64_t)kEncUnit * group_units(n);
+    return (uint32_t)((n + group - 1) / group);
+}
 
 size_t encode_workspace_bytes(uint64_t n, int n_levels) {
     return 4u * (kEncParts + (size_t)(n_levels - 1) * count_groups(n));
@@ -646,8 +653,12 @@ size_t encode_workspace_bytes(uint64_t n, int n_levels) {
 template <int L>
 static void scan_launch(const uint16_t *w, uint32_t n, uint32_t n_units, const EncLevels &lv, const uint32_t *parts,
                         uint16_t *scale, int32_t *table, uint32_t *sums, hipStream_t s) {
-    hipLaunchKernelGGL(k_enc_count<L>, dim3(count_groups(n)), dim3(kWave * kEncWaves), 0, s, w, n, n_units, parts, lv, table,
-                       sums, scale);
+    if (group_units(n) == kCountUnits)
+        hipLaunchKernelGGL((k_enc_count<L, kCountUnits>), dim3(count_groups(n)), dim3(kWave * kEncWaves), 0, s, w, n, n_units, parts, lv, table,
+                           sums, scale);
+    else
+        hipLaunchKernelGGL((k_enc_count<L, kCountFewUnits>), dim3(count_groups(n)), dim3(kWave * kEncWaves), 0, s, w, n, n_units, parts, lv,
+                           table, sums, scale);
 }
 
 int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *bits, uint16_t *scale, int32_t *table,
@@ -670,7 +681,7 @@ int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *b
         default: scan_launch<8>(w, n, n_units, lv, parts, scale, table, sums, s); break;
     }
     hipLaunchKernelGGL(k_enc_scan, dim3(tiles, n_levels - 1), dim3(1024), 0, s, table, n_units, sums, count_groups(n),
-                       host_totals);
+                       group_units(n), host_totals);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 

@@ -202,6 +202,15 @@ def test_encode_waves_of_more_than_a_span(oracle, dev, level_bits, waves, spans,
     check_against_oracle(oracle, dev, make_weight("calibrated_odd_scale", 1, n), level_bits)
 
 
+@pytest.mark.parametrize("n,top", [(3 * 8192 + 5, 8191), (3 * 8192 + 5, 3 * 8192 - 1), (3 * 8192 + 5, 3 * 8192 + 4), (16 * 512, 16 * 512 - 1),
+                                   (16 * 512 + 1, 16 * 512), (32768 * 512, 32768 * 512 - 1), (32768 * 512 + 1, 32768 * 512)])
+def test_encode_counts_by_groups_of_either_size(oracle, dev, n, top):
+    """The largest weight in a whole or in the ragged part of the search for it; units counted 16 and 64 to a workgroup."""
+    w = make_weight("calibrated_odd_scale", 1, n)
+    w[0, top] = -4 * w.abs().max()
+    check_against_oracle(oracle, dev, w, (3, 5, 8))
+
+
 SCAN = "ixh_encode_scan_counts"
 
 
