@@ -340,12 +340,12 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 }
 
 // How the work is cut: groups of 16 .. 128 activation rows, slices of the columns and groups of 16-row blocks, a workgroup
-// per CU. Of all such cuts the one with the shortest estimate, in half nanoseconds: 250 for each block of weights that a SIMD has in a
-// stage (its vector instructions), 120 for each 16 activation rows, 10 for each of these and block (operands read from LDS); the slices'
-// sums cost a launch and their way through memory.  Fitted to all cuts, timed, of 24 shapes from 256 x 4096 to 17408 x 5120 at 12 to 160
-// rows and 3, 5 and 8 bits: within 0.6 % of the shortest in the mean, 13 % at worst.  (An estimate that took a stage as 3000 to 3500
-// clocks whatever the blocks in it, right for two blocks a wave, is 2.1 % off in the mean: 4096 x 4096 (3 bits) at 128 rows 23.6 us
-// against 19.8, 8192 x 2048 24.3 against 19.2, 17408 x 5120 at 64 rows 42.3 against 37.2.)
+// per CU. Of all such cuts the one with the shortest estimate, in units of some half nanosecond: 250 for each block of weights that a SIMD has
+// in a stage (its vector instructions), 125 for each 16 activation rows, 3 for each of these and block (operands read from LDS), and no
+// less than the way of a stage's requests and activations takes with few blocks; the slices' sums cost a launch and their way through memory.
+// Fitted to all cuts, timed, of 52 shapes from 256 x 4096 to 17408 x 5120 at 9 to 160 rows and 3, 5 and 8 bits: within 0.55 % of the shortest
+// in the mean, 13 % at worst (1.2 and 33 without that least, which cut long rows so that a workgroup has few blocks and many cells: 2048 x 17408
+// at 16 rows 18.4 us against 14.3, 8192 x 2048 (5 bits) at 64 rows 18.9 against 16.2).
 struct LgPlan { uint32_t m_groups, mb, slices, groups; };
 static LgPlan lg_plan(const LanesDev &L, int m) {
     const uint32_t blocks = (L.n_tiles + 3u) / 4u, m_blocks = ((uint32_t)m + 15u) / 16u;
@@ -357,8 +357,8 @@ static LgPlan lg_plan(const LanesDev &L, int m) {
             const uint32_t groups = min(max(cus / s, 1u), blocks);
             const uint32_t share = (blocks + groups - 1u) / groups, rounds = (share + kLgBlocks - 1u) / kLgBlocks;
             const uint32_t at_once = (share + rounds - 1u) / rounds, cells = (L.n_cells + s - 1u) / s;
-            const uint64_t stage = 250u * ((at_once + 3u) / 4u) + 120u * mb + 10u * mb * at_once;
-            const uint64_t sums = s > 1 ? 1100u + (uint64_t)s * (uint32_t)m * blocks * 16u / 570u : 0u;
+            const uint64_t stage = max(250u * ((at_once + 3u) / 4u) + 125u * mb + 3u * mb * at_once, 400u + 115u * mb);
+            const uint64_t sums = s > 1 ? 1600u + (uint64_t)s * (uint32_t)m * blocks * 16u / 670u : 0u;
             const uint64_t cost = 4u * stage * rounds * cells + sums;
             if (cost < best_cost) { best_cost = cost; best = {m_groups, mb, s, groups}; }
         }
