@@ -395,15 +395,20 @@ static LrPlan lr_plan_of(const LanesDev &L, int m) {
     }
 }
 
-// Nine to sixteen rows of up to 20 * 2^20 weights: turning the activations round for the whole of a long slice, or starting up for
-// a single cell, takes longer than k_lanes_gemm's way, whose sixteen waves share a copy of 128 columns a stage.  us, this / that at
-// 16 rows, 5 bits: 512 rows x 512 columns 6.6 / 6.0, 512 x 1024 7.2 / 8.3, 512 x 2048 8.8 / 8.3, 2048 x 4096 10.4 / 9.4, 4096 x 4096
-// 12.3 / 11.4, 4288 x 4096 (a second block for some workgroups) 13.9 / 11.9, 8192 x 4096 14.7 / 15.6.  Three bits, whose pairs sit in LDS 32 times over here: 4096 x 2048 8.7 / 10.6, 2048 x 4096
-// 10.1 / 10.7, 4096 x 4096 11.5 / 10.5, 2048 x 8192 11.6 / 10.9, 4096 x 8192 13.8 / 14.5.
+// Nine to sixteen rows: turning the activations round for the whole of a long slice, or starting up for a single cell, takes longer than
+// k_lanes_gemm's way, whose sixteen waves share a copy of 128 columns a stage, up to 20 * 2^20 weights, and of long rows at 4, 5 and 8 bits
+// from 25 to 48 * 2^20; not of tall layers, of which a workgroup here has one slice.  us, this / that at 16 rows, 5 bits: 512 x 512
+// 6.6 / 5.7, 1024 x 1024 7.2 / 7.9, 512 x 2048 8.7 / 7.9, 2048 x 2048 8.8 / 9.0, 4096 x 2048 9.0 / 9.4, 1536 x 6144 13.1 / 10.1, 4096 x 4096
+// 12.0 / 11.1, 8192 x 2560 12.1 / 12.6, 4096 x 6144 13.9 / 14.8, 5120 x 5120 15.7 / 15.0, 6144 x 6144 18.0 / 17.0, 9216 x 5120 20.8 / 18.6, 8192 x
+// 4096 14.0 / 15.0, 17408 x 5120 28.6 / 30.1.  Three bits, whose pairs sit in LDS 32 times over here: 512 x 4096 8.6 / 8.5, 2560 x 2560 10.3 / 9.1,
+// 1536 x 6144 12.4 / 9.5, 4096 x 4096 10.4 / 9.6, 8192 x 2560 9.4 / 11.0, 3072 x 8192 12.4 / 12.1, 4096 x 6144 11.5 / 12.3, 6144 x 6144 14.6 / 14.8.
 static bool lr_gemm_wins(const LanesDev &L, int m) {
     const uint64_t n = (uint64_t)L.out_f * L.in_f;
-    if (m <= 8 || n > 20u << 20) return false;
-    return L.bits == 3 ? n > 9u << 20 && L.in_f > 2560u : L.in_f <= kLnCols || L.in_f >= 2048u;
+    if (m <= 8) return false;
+    if (L.bits != 3 && L.in_f <= kLnCols) return n <= 20u << 20;
+    if (L.out_f >= 2ull * L.in_f) return false;
+    if (L.bits == 3) return L.in_f >= 2560u && n > 4u << 20 && n <= 20u << 20;
+    return n <= 20u << 20 ? L.in_f >= 2048u : L.in_f >= 4608u && n >= 25u << 20 && n <= 48u << 20;
 }
 
 static size_t lr_bytes(const LanesDev &L, const LrPlan &p, int m) {

@@ -272,6 +272,17 @@ def test_many_rows_of_larger_weights(oracle, dev, out_f, in_f, m):
     check(oracle, p, x, y)
 
 
+@pytest.mark.parametrize("kind,out_f,in_f", [("rare", 1638, 2560), ("rare", 1639, 2560), ("real", 40, 2040), ("real", 40, 2048),
+                                             ("real", 4095, 2048), ("real", 4096, 2048), ("four", 5120, 5112), ("four", 5120, 5120)])
+def test_nine_to_sixteen_rows_either_way(oracle, dev, kind, out_f, in_f):
+    """Weights on both sides of the lines between the two kernels that take nine to sixteen rows; few blocks and many, one cell to ten a slice."""
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    for m in (9, 16):
+        x = activations(m, in_f, seed=m)
+        check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f, bias.to(dev)), bias)
+
+
 @pytest.mark.parametrize("scale", [2.0 ** -100, 1.5 * 2.0 ** 99, 2.0 ** 100, 1.75 * 2.0 ** 112])
 @pytest.mark.parametrize("kind", ["four", "real"])
 def test_many_rows_at_extreme_scales(oracle, dev, kind, scale):
