@@ -54,13 +54,21 @@ __device__ __forceinline__ void lg_decode5(const uint32_t (&w)[5], uint32_t lut_
     }
 }
 
+// n things to k parts, floor(i n / k) in front of part i, without a division in the kernel: four of them in front of the first request took
+// 0.5 us a launch (5 bits, 9 rows of 512 x 512 5.40 -> 4.78 us, 17 of 2048 x 2048 8.29 -> 7.83).  The first parts having one more
+// instead takes up to 6 % more (9216 x 5120 at 5 bits, 9 to 32 rows).  (Plain arguments: a structure's members are not in registers when the kernel starts.)
+struct LgSplit {
+    uint32_t share, more;  // a part's whole share, and the rest of it in 2^-32, rounded up: exact for up to 2^16 parts
+    LgSplit(uint32_t n, uint32_t k) : share(n / k), more((uint32_t)((((uint64_t)(n % k) << 32) + k - 1u) / k)) {}
+};
+__device__ __forceinline__ uint32_t lg_first(uint32_t i, uint32_t share, uint32_t more) { return i * share + __umulhi(i, more); }
+
 template <int BITS, int MB, int DEPTH>
 __global__ void __launch_bounds__(kLgBlocks *kWave)
-k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint32_t *__restrict__ exc_off,
-             const uint16_t *__restrict__ scale_at, uint32_t n_cells, uint32_t n_tiles, uint32_t slices, uint32_t groups,
-             const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, uint32_t in_f, uint32_t m_all, int64_t ldx,
-             uint32_t out_f, float *__restrict__ ws, bool ws_aligned, const uint16_t *__restrict__ bias, bool once,
-             uint16_t *__restrict__ y, int64_t ldy) {
+k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint16_t *__restrict__ scale_at, uint32_t c_share,
+             uint32_t c_more, uint32_t b_share, uint32_t b_more, uint32_t in_f, uint32_t ldx, uint32_t m_all, uint32_t most_at_once, uint32_t n_cells, uint32_t n_tiles,
+             const uint32_t *__restrict__ exc_off, const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, uint32_t out_f,
+             float *__restrict__ ws, bool ws_aligned, const uint16_t *__restrict__ bias, bool once, uint16_t *__restrict__ y, int64_t ldy) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lg_smem[];
     using P = LnPairs<BITS, false>;
     constexpr uint32_t kTile = kLgTileBytes;
@@ -68,13 +76,13 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)lg_smem;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, n = lane & 15u, kg = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const uint32_t slice = blockIdx.x % slices, group = blockIdx.x / slices % groups, row0 = blockIdx.x / slices / groups * (16u * MB);
+    const uint32_t slice = blockIdx.x, group = blockIdx.y, row0 = blockIdx.z * (16u * MB);
     const uint32_t m_last = m_all - 1u;
     const uint32_t n_blocks = (n_tiles + 3u) / 4u;
-    const uint32_t c0 = slice * n_cells / slices, c1 = (slice + 1u) * n_cells / slices, len = c1 - c0;
-    const uint32_t b0 = group * n_blocks / groups, b1 = (group + 1u) * n_blocks / groups;
-    const uint32_t rounds = (b1 - b0 + kLgBlocks - 1u) / kLgBlocks;
-    const uint32_t at_once = (b1 - b0 + rounds - 1u) / rounds;  // blocks of a round (the last one may have fewer)
+    const uint32_t c0 = lg_first(slice, c_share, c_more), c1 = lg_first(slice + 1u, c_share, c_more), len = c1 - c0;
+    const uint32_t b0 = lg_first(group, b_share, b_more), b1 = lg_first(group + 1u, b_share, b_more), own = b1 - b0;
+    // blocks of a round (the last one may have fewer)
+    const uint32_t rounds = (own + kLgBlocks - 1u) / kLgBlocks, at_once = rounds == 1u ? own : most_at_once;
     const uint32_t total = rounds * len;
     const uint32_t tile_at = smem + P::kLutBytes + wave * kTile;
     // (base registers that the compiler takes as they are, the rest in the accesses' offset fields)
@@ -89,7 +97,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     uint32_t x_row[XP];
 #pragma unroll
     for (uint32_t k = 0; k < XP; ++k)  // (the activations lie within 4 GB)
-        x_row[k] = min(row0 + ((tid + k * kThreads) >> 8) * 16u + n, m_last) * (uint32_t)ldx * 2u;
+        x_row[k] = min(row0 + ((tid + k * kThreads) >> 8) * 16u + n, m_last) * ldx * 2u;
     const uint32_t x_in = (tid >> 4 & 15u) * 16u, x_bytes = in_f * 2u;
     auto x_load = [&](uint32_t g) {
         Pieces r;
@@ -312,7 +320,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
             for (int b = 0; b < MB; ++b, r += 16u) {
                 if (BITS == 5) acc[b] *= big ? 0x1p32f : 1.0f;
                 if (mine && r < m_all) {
-                    if (slices > 1u) {
+                    if (c_share < n_cells) {
                         float *const to = ws + ((size_t)slice * m_all + r) * (n_blocks * 16u) + at;
                         if (ws_aligned) *reinterpret_cast<ln_f32x4 *>(to) = acc[b];
                         else
@@ -383,9 +391,11 @@ static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, in
     static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemm<BITS, MB, DEPTH>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
-    hipLaunchKernelGGL((k_lanes_gemm<BITS, MB, DEPTH>), dim3(p.slices * p.groups * p.m_groups), dim3(kLgBlocks * kWave), lds, s, L.plane, x,
-                       L.exc_off, L.scale, L.n_cells, L.n_tiles, p.slices, p.groups, L.exc_pos, L.exc_val, L.in_f, (uint32_t)m, ldx,
-                       L.out_f, ws, ((uintptr_t)ws & 15u) == 0, bias, once, y, ldy);
+    const uint32_t blocks = (L.n_tiles + 3u) / 4u, most = (blocks + p.groups - 1u) / p.groups, rounds = (most + kLgBlocks - 1u) / kLgBlocks;
+    const LgSplit c(L.n_cells, p.slices), b(blocks, p.groups);
+    hipLaunchKernelGGL((k_lanes_gemm<BITS, MB, DEPTH>), dim3(p.slices, p.groups, p.m_groups), dim3(kLgBlocks * kWave), lds, s, L.plane, x, L.scale,
+                       c.share, c.more, b.share, b.more, L.in_f, (uint32_t)ldx, (uint32_t)m, (most + rounds - 1u) / rounds, L.n_cells,
+                       L.n_tiles, L.exc_off, L.exc_pos, L.exc_val, L.out_f, ws, ((uintptr_t)ws & 15u) == 0, bias, once, y, ldy);
     if (p.slices > 1)
         return launch_lanes_reduce(ws, p.slices, m, L.out_f, (L.n_tiles + 3u) / 4u * 16u, bias, once, y, ldy, s);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
