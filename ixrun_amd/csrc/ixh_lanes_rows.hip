@@ -81,19 +81,25 @@ k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     // ---- asked for first: this wave's activations, its first units, the list's extent, the scale ----
     // a pair of columns a lane, all rows; pairs past the last column are those of the last
     struct Pairs { uint32_t v[MT]; };
+    // Rows' places in 32 bits (where pairs are asked for, they lie within 4 GB): with the rows' addresses in 64 a wave's first request was
+    // behind 240 instructions at 16 rows, 105 now (5120 x 17408, 3 bits, 16 rows 20.3 -> 19.8 us; 1024 x 1024, 5 bits 6.6 -> 6.3, eight rows 5.6 -> 5.5).
+    const uint32_t x_step = (uint32_t)ldx * 2u, x_last = (m - 1u) * x_step;
     auto x_load = [&](uint32_t task) {
         Pairs r;
         const uint32_t col = c0 * kLnCols + task * 128u + 2u * lane;
         if (x_pairs) {
-            const uint32_t at = min(col, in_f - 2u);
+            const uint32_t at = min(col, in_f - 2u) * 2u;
 #pragma unroll
-            for (uint32_t k = 0; k < MT; ++k) r.v[k] = *reinterpret_cast<const uint32_t *>(x + (int64_t)min(k, m - 1u) * ldx + at);
+            for (uint32_t k = 0; k < MT; ++k)
+                r.v[k] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(x) + (min(k * x_step, x_last) + at));
         } else {
             const uint32_t at = min(col, in_f - 1u), next = min(col + 1u, in_f - 1u);
             uint32_t hi[MT];
+            int64_t step = ldx;
+            asm volatile("" : "+s"(step));  // (rows' addresses are worked out here, not in front of the other way's requests)
 #pragma unroll
             for (uint32_t k = 0; k < MT; ++k) {
-                const uint16_t *const row = x + (int64_t)min(k, m - 1u) * ldx;
+                const uint16_t *const row = x + (int64_t)min(k, m - 1u) * step;
                 r.v[k] = row[at], hi[k] = row[next];
             }
 #pragma unroll
@@ -428,7 +434,7 @@ static int rows_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx,
     static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_rows<BITS, MT, WIDE>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLnLds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
-    const bool pairs = ((uintptr_t)x & 3u) == 0 && L.in_f % 2u == 0 && ldx % 2 == 0;
+    const bool pairs = ((uintptr_t)x & 3u) == 0 && L.in_f % 2u == 0 && ldx % 2 == 0 && ldx < 1ll << 27;
     const uint32_t blocks = (L.n_tiles + 3u) / 4u, log_waves = 31u - (uint32_t)__builtin_clz(p.waves);
     const uint32_t shape = (uint32_t)m | log_waves << 5 | (uint32_t)pairs << 8;
     hipLaunchKernelGGL((k_lanes_rows<BITS, MT, WIDE>), dim3(p.slices, p.groups), dim3(kWave * p.waves), p.lds, s, L.plane, x, L.exc_off,
