@@ -341,12 +341,14 @@ k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 }
 
 // How the work is cut: slices of the columns, workgroups of a slice, waves of a workgroup. Of a few cuts the one with the shortest
-// estimate, in clocks: 4000 to the first product and 400 for each wave that has to be there, 20 or 30 (up to 8 or 16 rows) for 128
-// columns of activations a wave turns round, then whichever is longer, 2500 or 2000 for a step of 16 x 256 weights in a wave or 130
-// in the CU; the slices' sums cost a launch and their way through memory.  Fitted to all cuts, timed, of 32 shapes from 256 x 4096 to
-// 17408 x 5120: within 0.3 % of the shortest in the mean, 8 % at worst.  (Without the waves' 400, and the slices dearer, layers of few
-// rows had one slice of sixteen waves where several of four fill the CUs: 960 x 3072 at 11 rows 11.0 us against 8.9, 256 x 4096
-// 11.9 against 8.7, 5120 x 17408 at 7 rows 18.0 against 16.0.)
+// estimate, in clocks: 4000 to the first product and 510 for each wave that has to be there, 22 or 29 (up to 8 or 16 rows) for 128
+// columns of activations a wave turns round, 28 or 56 for each cell of them that an XCD fetches, then whichever is longer, 2700 for a step of
+// 16 x 256 weights in a wave or 135 in the CU, and 16 for each block and cell where the longer slices are always the same XCDs'; the slices'
+// sums cost a launch and their way through memory.  Fitted to all cuts, timed, of 54 shapes from 512 x 512 to 17408 x 5120 and 20480 x 4096
+// at 8 and 16 rows and 3, 5 and 8 bits: within 1.0 % of the shortest in the mean, 9 % at worst (1.9 and 15 with 400 for a wave and without
+// the XCDs' terms: eight rows of 2048 x 11008, 5 bits, in eleven slices instead of eight 12.6 us against 11.3, 2048 x 6144 by sixteen waves
+// instead of eight 11.0 against 10.5).  (Without a cost of each wave, and the slices dearer, layers of few rows had one slice of sixteen waves
+// where several of four fill the CUs: 960 x 3072 at 11 rows 11.0 us against 8.9, 256 x 4096 11.9 against 8.7.)
 struct LrPlan { uint32_t slices, groups, waves, x_rows; size_t lds; };
 
 template <int BITS, int MT, bool WIDE>
@@ -360,6 +362,9 @@ static LrPlan lr_plan(const LanesDev &L) {
     for (uint32_t s = s_min; s <= min(L.n_cells, s_min + 15u); ++s) {
         // (16 rows more: the zeros that places without an element point at)
         const uint32_t cells = (L.n_cells + s - 1u) / s, x_rows = cells * kLnCols + 16u;
+        // workgroups go round the eight XCDs: slices that one of them has; the longer ones are always the same one's
+        const uint32_t xcd_slices = s / min(s & (0u - s), 8u);
+        const bool uneven = xcd_slices == 1u && L.n_cells % s != 0u;
         for (uint32_t waves = 16; waves >= 4; waves /= 2) {
             const size_t fixed = kLrXAt<BITS, WIDE> + (size_t)x_rows * 2u * MT + waves * kPart;
             if (fixed + kPart > kLnLds) continue;
@@ -372,9 +377,10 @@ static LrPlan lr_plan(const LanesDev &L) {
             const uint32_t per_cu = min((uint32_t)(kLnLds / lds), 16u / waves), rounds = (groups * s + cus * per_cu - 1u) / (cus * per_cu);
             const uint32_t steps = nb * cells * 2u, mine = (steps + waves - 1u) / waves;
             const uint32_t resident = min(per_cu, (groups * s + cus - 1u) / cus);
-            const uint64_t run = std::max<uint64_t>((uint64_t)mine * (MT == 8 ? 2500u : 2000u), (uint64_t)steps * resident * 130u);
-            const uint64_t sums = s > 1 ? (MT == 8 ? 4000u : 2000u) + (uint64_t)s * L.n_tiles * 4u * MT * 8u / 3400u : 0u;
-            const uint64_t cost = rounds * (4000u + 400u * waves + (uint64_t)cells * 64u / waves * (MT == 8 ? 20u : 30u) + run) + sums;
+            const uint64_t run = std::max<uint64_t>((uint64_t)mine * 2700u, (uint64_t)steps * resident * 135u);
+            const uint64_t sums = s > 1 ? (MT == 8 ? 4800u : 3300u) + (uint64_t)s * L.n_tiles * 4u * MT * 8u / 3300u : 0u;
+            const uint64_t turned = (uint64_t)cells * 64u / waves * (MT == 8 ? 22u : 29u) + (uint64_t)cells * xcd_slices * (MT == 8 ? 28u : 56u);
+            const uint64_t cost = rounds * (4000u + 510u * waves + turned + run + (uneven ? 16u * cells * nb : 0u)) + sums;
             if (cost < best_cost) { best_cost = cost; best = {s, groups, waves, x_rows, lds}; }
         }
     }
