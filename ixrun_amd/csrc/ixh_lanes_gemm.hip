@@ -8,7 +8,7 @@ namespace ixh {
 //
 // Bound: a stage's vector instructions (decode, listed elements), then LDS (operands read back, look-ups, stores), then the parts of a stage
 // that follow one another in a wave, while all waves meet at its end; the matrix unit is busy for 15 % of it.  10240 x 5120 at 55 / 40 /
-// 5 %, 100 rows: 34.6 us with the slices' sums (37.7 with two blocks of 16 weight rows a wave from 49 rows on, which halves the reads of
+// 5 %, 100 rows: 34.2 us with the slices' sums (37.7 with two blocks of 16 weight rows a wave from 49 rows on, which halves the reads of
 // activations, and half as many waves to fill in for one another: 64 rows 30.9 -> 27.3, 128 rows 40.6 -> 37.5; 74.3 for the decode to
 // memory and the library's GEMM).  Looking up the next stage's weights between the products of this one changes nothing, nor does the list
 // half a cell earlier; waves of their own for decode and products (eight and four, a stage of 64 columns) take 44; activations straight

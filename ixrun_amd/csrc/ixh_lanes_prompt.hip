@@ -61,7 +61,7 @@ k_lanes_xtile(const uint16_t *__restrict__ x, int64_t ldx, uint32_t m, uint32_t 
 // k_lanes_prompt<BITS, MI, NW>: 128 MI / NW activation rows by 128 weight rows a workgroup, over a run of the cells of a tile.
 //
 // Bound: the matrix unit and what stands between two stages.  5120 x 17408 at 512 rows (3 bits): 97 us a call; one after the other
-// under the profiler 86 to 96 for this kernel, 8 for the activations' reordering and 12 for adding the sums (63 MB read).  (Which blocks share
+// under the profiler 86 to 96 for this kernel, 8 for the activations' reordering and 11 for adding the sums (63 MB read).  (Which blocks share
 // an XCD's L2 matters little: all of an XCD on the same columns 2 to 4 % slower, on neighbouring runs up to 3 %.  Operands straight from
 // row-major activations: 126 instead of 88.)  The
 // products would take 58 at the rate of a large library product; decode into memory and that library's product took 126.  Clocks a stage
@@ -418,10 +418,10 @@ static uint32_t lp_part_size(const LpPlan &p) { return kLpWaves * p.mi * (8u / p
 
 // Above 128 rows and 3 * 2^23 weights.  Fewer rows do not hide the decode behind their products, and fewer weights leave a workgroup a
 // few cells, which the pipeline's start and the sums' way through memory outweigh.  us, k_lanes_gemm against this: 5120 x 17408
-// (3 bits) 49 / 50 at 128 rows, 71 / 55 at 144, 145 / 100 at 512; 5120 x 5120 28 / 30, 33 / 32, 63 / 53; 5120 x 4096 28 / 32 at 144
-// rows and 41 / 41 at 384; 4096 x 4096 (5 bits) 30 / 30 at 192 rows, 46 / 47 at 512; 2048 x 2048 29 / 36 at 512.  Planes of 4 and 8 bits at
-// 129 / 256 / 512 rows: 5120 x 5120 (4) 32 / 31, 39 / 35, 63 / 52, 17408 x 5120 (4) 79 / 60, 110 / 78, 200 / 115, 5120 x 5120 (8) 30 / 28,
-// 43 / 35, 66 / 52, 12288 x 6144 (8) 61 / 57, 85 / 73, 145 / 107.  The bounds keep offsets within 32 bits.
+// (3 bits) 50 / 53 at 128 rows, 61 / 52 at 144, 138 / 97 at 512; 5120 x 5120 25 / 28, 27 / 29, 56 / 48; 5120 x 4096 25 / 28 at 144
+// rows and 47 / 46 at 512; 4096 x 4096 (5 bits) 26 / 28 at 192 rows, 41 / 44 at 512; 2048 x 2048 23 / 35 at 512; at 129 / 256 / 512 rows:
+// 5120 x 5120 (5) 31 / 29, 37 / 35, 60 / 52, 17408 x 5120 (5) 80 / 65, 101 / 83, 196 / 120, 5120 x 5120 (8) 26 / 26,
+// 33 / 33, 55 / 51, 12288 x 6144 (8) 52 / 54, 68 / 69, 114 / 104.  The bounds keep offsets within 32 bits.
 bool lanes_prompt_wins(const LanesDev &L, int m) {
     return m > 128 && (uint64_t)L.out_f * L.in_f > 3u << 23 && (uint64_t)lp_tiles(L.n_tiles) * L.n_cells < 1u << 24 &&
            (uint64_t)L.n_cells * 16u * (((uint32_t)m + 15u) / 16u) * 1024u < 1ull << 31;
