@@ -50,14 +50,14 @@ _ENCODE = ("ixh_encode.hip", "ixh_dev.h")
 _OLD = ((), "measured-on-earlier-sources")  # figures kept for the record; reported as null
 MEASURED_TRAFFIC_BYTES = {
     # k_lanes_gemv; eight rows k_lanes_rows, sixteen with k_lanes_reduce
-    "down_proj_5120x17408_m1_student_t": (18536.6 * 2.0 * 1024 + 16.0 * 1024, _LANES, "70d5731cfa05d6b6"),
-    "down_proj_5120x17408_m1_calibrated": (40732.0 * 2.0 * 1024 + 16.0 * 1024, _LANES, "70d5731cfa05d6b6"),
-    "down_proj_5120x17408_m1_five_level_calibrated": (40732.0 * 2.0 * 1024 + 16.0 * 1024, _LANES, "70d5731cfa05d6b6"),
-    "gate_up_17408x5120_m8_calibrated": (36785.0 * 2.0 * 1024 + 272.0 * 1024, _LANES, "70d5731cfa05d6b6"),
-    "down_proj_5120x17408_m16_student_t": ((20853.0 + 1128.0) * 2.0 * 1024 + (2240.0 + 160.0) * 1024, _LANES, "70d5731cfa05d6b6"),
+    "down_proj_5120x17408_m1_student_t": (18520.8 * 2.0 * 1024 + 16.0 * 1024, _LANES, "60ab0395ea2043ab"),
+    "down_proj_5120x17408_m1_calibrated": (40731.8 * 2.0 * 1024 + 16.0 * 1024, _LANES, "60ab0395ea2043ab"),
+    "down_proj_5120x17408_m1_five_level_calibrated": (40731.8 * 2.0 * 1024 + 16.0 * 1024, _LANES, "60ab0395ea2043ab"),
+    "gate_up_17408x5120_m8_calibrated": (36781.3 * 2.0 * 1024 + 272.0 * 1024, _LANES, "60ab0395ea2043ab"),
+    "down_proj_5120x17408_m16_student_t": ((19432.0 + 974.0) * 2.0 * 1024 + (1920.0 + 160.0) * 1024, _LANES, "60ab0395ea2043ab"),
     # k_lanes_xtile, k_lanes_prompt and k_lanes_prompt_reduce
-    "prefill_5120x17408_m512_five_level": ((8714.5 + 57943.0 + 30743.5) * 2.0 * 1024 + (17408.0 + 66720.0 + 5126.5) * 1024,
-                                           _LANES, "70d5731cfa05d6b6"),
+    "prefill_5120x17408_m512_five_level": ((8715.6 + 57942.1 + 30734.5) * 2.0 * 1024 + (17408.0 + 66720.0 + 5122.2) * 1024,
+                                           _LANES, "60ab0395ea2043ab"),
     "down_proj_5120x17408_m1_student_t_packed": (23032.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "0d8ffbb8d311f48d"),
     "gate_up_17408x5120_m1_student_t_packed": (22935.9 * 2.0 * 1024 + 40.0 * 1024, _ROWS, "0d8ffbb8d311f48d"),
     "attn_proj_5120x5120_m1_student_t_packed": (7135.5 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "0d8ffbb8d311f48d"),
@@ -82,19 +82,19 @@ MEASURED_TRAFFIC_BYTES = {
     "decode_5120x17408_student_t": (23268.0 * 2.0 * 1024 + 179524.0 * 1024,) + _OLD,
     "decode_gs_5120x17408_student_t": (33559.0 * 2.0 * 1024 + 174080.0 * 1024,) + _OLD,
     # all kernels of one encode step together (absmax, count, scan, borders, pack)
-    "encode_5120x17408_student_t": ((87063.2 + 87104.3 + 780.9 + 659.2 + 89011.6) * 2.0 * 1024
-                                    + (8.0 + 2327.4 + 1362.7 + 309.2 + 46619.3) * 1024, _ENCODE, "f244d71e976cb685"),
-    "encode_5120x17408_calibrated": ((87063.1 + 87104.0 + 780.9 + 659.2 + 89092.8) * 2.0 * 1024
-                                     + (8.0 + 2318.4 + 1362.7 + 600.0 + 68672.5) * 1024, _ENCODE, "f244d71e976cb685"),
+    "encode_5120x17408_student_t": ((87063.5 + 87104.1 + 776.9 + 658.6 + 88982.6) * 2.0 * 1024
+                                    + (8.0 + 2314.2 + 1362.7 + 309.2 + 46625.1) * 1024, _ENCODE, "b65837a2706e3a15"),
+    "encode_5120x17408_calibrated": ((87063.5 + 87104.1 + 776.9 + 658.6 + 89071.9) * 2.0 * 1024
+                                     + (8.0 + 2320.2 + 1362.7 + 600.0 + 68700.9) * 1024, _ENCODE, "b65837a2706e3a15"),
 }
 
 # Wave-level instruction counts per launch of the dominant kernel (SQ_INSTS_VALU, SQ_INSTS_SALU, SQ_INSTS_LDS from one
 # rocprofv3 --pmc run of this script, mean over the launches), gated by the hash of the kernel's sources like the
 # traffic figures.  Reported per weight: vector and LDS instructions x 64 lanes / weights, scalar instructions / weights.
 MEASURED_INSTRUCTIONS = {
-    "down_proj_5120x17408_m1_student_t": ((3414116.0, 2201438.0, 819680.0), _LANES, "70d5731cfa05d6b6"),
-    "down_proj_5120x17408_m1_calibrated": ((4829187.0, 3166052.0, 918004.0), _LANES, "70d5731cfa05d6b6"),
-    "down_proj_5120x17408_m1_five_level_calibrated": ((4829187.0, 3166052.0, 918004.0), _LANES, "70d5731cfa05d6b6"),
+    "down_proj_5120x17408_m1_student_t": ((3414116.0, 2201438.0, 819680.0), _LANES, "60ab0395ea2043ab"),
+    "down_proj_5120x17408_m1_calibrated": ((4829187.0, 3166052.0, 918004.0), _LANES, "60ab0395ea2043ab"),
+    "down_proj_5120x17408_m1_five_level_calibrated": ((4829187.0, 3166052.0, 918004.0), _LANES, "60ab0395ea2043ab"),
     "down_proj_5120x17408_m1_student_t_packed": ((5734195.0, 4469166.0, 1360042.0), _ROWS, "0d8ffbb8d311f48d"),
     "gate_up_17408x5120_m1_student_t_packed": ((6030194.0, 4450915.0, 1414314.0), _ROWS, "0d8ffbb8d311f48d"),
     "attn_proj_5120x5120_m1_student_t_packed": ((3570752.0, 2281697.0, 593732.0), _ROWS, "0d8ffbb8d311f48d"),
