@@ -1,7 +1,10 @@
-// What a wave of k_lanes_gemv and k_lanes_gemv_few (ixh_lanes.hip) asks for ahead of knowing whether it needs it, and where the workgroups of
-// k_lanes_prompt (ixh_lanes_prompt.hip) leave their sums.  Plain C++, so that the ranges can be walked without a GPU.
+// What a wave of k_lanes_gemv and k_lanes_gemv_few (ixh_lanes.hip) asks for ahead of knowing whether it needs it, where the workgroups of
+// k_lanes_prompt (ixh_lanes_prompt.hip) leave their sums, and how the work of k_lanes_gemm (ixh_lanes_gemm.hip) is cut.  Plain C++, so that
+// the ranges can be walked without a GPU.
 #pragma once
 #include <stdint.h>
+
+#include <algorithm>
 
 #ifdef __HIPCC__
 #define LN_BOTH __host__ __device__ __forceinline__
@@ -75,6 +78,59 @@ LN_BOTH uint32_t lp_parts(uint32_t groups, uint32_t tiles) {
     if (tiles % groups == 0) return 0;
     if (groups % tiles == 0) return groups;
     return groups + (tiles < groups ? tiles : groups) - 1u;
+}
+
+// k_lanes_gemm: blocks of 16 weight rows that a workgroup has in work at a time, and the most blocks of 16 activation rows.
+constexpr uint32_t kLgBlocks = 16;
+constexpr uint32_t kLgMost = 8;
+
+// n things to k parts, floor(i n / k) in front of part i, without a division in the kernel: four of them in front of the first request took
+// 0.5 us a launch (5 bits, 9 rows of 512 x 512 5.40 -> 4.78 us, 17 of 2048 x 2048 8.29 -> 7.83).  The first parts having one more
+// instead takes up to 6 % more (9216 x 5120 at 5 bits, 9 to 32 rows).  (Plain arguments: a structure's members are not in registers when the kernel starts.)
+struct LgSplit {
+    uint32_t share, more;  // a part's whole share, and the rest of it in 2^-32, rounded up: exact for up to 2^16 parts
+    LgSplit(uint32_t n, uint32_t k) : share(n / k), more((uint32_t)((((uint64_t)(n % k) << 32) + k - 1u) / k)) {}
+};
+LN_BOTH uint32_t lg_first(uint32_t i, uint32_t share, uint32_t more) { return i * share + (uint32_t)((uint64_t)i * more >> 32); }
+
+// Rounds of a workgroup with `own` blocks, and the blocks of a round (the last one may have fewer).  `most_at_once`: those of the launch's
+// largest workgroups, whose rounds are even.  A workgroup of one block less has as many rounds, in which that is enough, or one round less: its
+// blocks are then whole rounds of kLgBlocks.
+LN_BOTH uint32_t lg_rounds(uint32_t own) { return (own + kLgBlocks - 1u) / kLgBlocks; }
+LN_BOTH uint32_t lg_at_once(uint32_t own, uint32_t most_at_once) {
+    return own % kLgBlocks == 0u ? kLgBlocks : own < kLgBlocks ? own : most_at_once;
+}
+LN_BOTH uint32_t lg_most_at_once(uint32_t blocks, uint32_t groups) {
+    const uint32_t most = (blocks + groups - 1u) / groups, rounds = lg_rounds(most);
+    return (most + rounds - 1u) / rounds;
+}
+
+// How the work is cut: groups of 16 .. 128 activation rows, slices of the columns and groups of 16-row blocks, a workgroup
+// per CU. Of all such cuts the one with the shortest estimate, in units of some half nanosecond: 250 for each block of weights that a SIMD has
+// in a stage (its vector instructions), 125 for each 16 activation rows, 3 for each of these and block (operands read from LDS), and no
+// less than the way of a stage's requests and activations takes with few blocks; the slices' sums cost a launch and their way through memory.
+// Fitted to all cuts, timed, of 52 shapes from 256 x 4096 to 17408 x 5120 at 9 to 160 rows and 3, 5 and 8 bits: within 0.55 % of the shortest
+// in the mean, 13 % at worst (1.2 and 33 without that least, which cut long rows so that a workgroup has few blocks and many cells: 2048 x 17408
+// at 16 rows 18.4 us against 14.3, 8192 x 2048 (5 bits) at 64 rows 18.9 against 16.2).
+struct LgPlan { uint32_t m_groups, mb, slices, groups; };
+inline LgPlan lg_plan(uint32_t n_tiles, uint32_t n_cells, int m, uint32_t all_cus) {
+    const uint32_t blocks = (n_tiles + 3u) / 4u, m_blocks = ((uint32_t)m + 15u) / 16u;
+    LgPlan best{};
+    uint64_t best_cost = ~0ull;
+    for (uint32_t m_groups = (m_blocks + kLgMost - 1u) / kLgMost; m_groups <= std::max((m_blocks + 1u) / 2u, 1u); ++m_groups) {
+        const uint32_t mb = (m_blocks + m_groups - 1u) / m_groups, cus = std::max(all_cus / m_groups, 1u);
+        for (uint32_t s = 1; s <= std::min(n_cells, cus); ++s) {
+            const uint32_t groups = std::min(std::max(cus / s, 1u), blocks);
+            const uint32_t share = (blocks + groups - 1u) / groups, rounds = lg_rounds(share);
+            const uint32_t at_once = (share + rounds - 1u) / rounds, cells = (n_cells + s - 1u) / s;
+            const uint64_t stage = std::max(250u * ((at_once + 3u) / 4u) + 125u * mb + 3u * mb * at_once, 400u + 115u * mb);
+            const uint64_t sums = s > 1 ? 1600u + (uint64_t)s * (uint32_t)m * blocks * 16u / 670u : 0u;
+            const uint64_t cost = 4u * stage * rounds * cells + sums;
+            if (cost < best_cost) { best_cost = cost; best = {m_groups, mb, s, groups}; }
+        }
+        if (m_groups * 2u > all_cus) break;
+    }
+    return best;
 }
 
 }  // namespace ixh

@@ -21,12 +21,10 @@ namespace ixh {
 // A workgroup owns a slice of the columns (whole cells) of a run of 16-row blocks, sixteen at most at a time; the slices' sums
 // meet in the workspace and launch_lanes_reduce adds them in slice order.
 // ---------------------------------------------------------------------------------------------------------------
-constexpr uint32_t kLgBlocks = 16;  // of 16 weight rows, in work at a time
 constexpr uint32_t kLgTile = 4096;
 constexpr uint32_t kLgTileBytes = kLgTile + 256u;  // and a dword a lane behind it, for what is not to be stored
 // where what the next stage could begin with between the products of this one takes more registers than there are
 template <int BITS, int MB> constexpr bool kLgTight = (BITS <= 4 && MB == 6) || (BITS == 5 && MB == 5);
-constexpr uint32_t kLgMost = 8;  // blocks of 16 activation rows
 
 __device__ __forceinline__ void lg_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -54,15 +52,6 @@ __device__ __forceinline__ void lg_decode5(const uint32_t (&w)[5], uint32_t lut_
     }
 }
 
-// n things to k parts, floor(i n / k) in front of part i, without a division in the kernel: four of them in front of the first request took
-// 0.5 us a launch (5 bits, 9 rows of 512 x 512 5.40 -> 4.78 us, 17 of 2048 x 2048 8.29 -> 7.83).  The first parts having one more
-// instead takes up to 6 % more (9216 x 5120 at 5 bits, 9 to 32 rows).  (Plain arguments: a structure's members are not in registers when the kernel starts.)
-struct LgSplit {
-    uint32_t share, more;  // a part's whole share, and the rest of it in 2^-32, rounded up: exact for up to 2^16 parts
-    LgSplit(uint32_t n, uint32_t k) : share(n / k), more((uint32_t)((((uint64_t)(n % k) << 32) + k - 1u) / k)) {}
-};
-__device__ __forceinline__ uint32_t lg_first(uint32_t i, uint32_t share, uint32_t more) { return i * share + __umulhi(i, more); }
-
 template <int BITS, int MB, int DEPTH>
 __global__ void __launch_bounds__(kLgBlocks *kWave)
 k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x, const uint16_t *__restrict__ scale_at, uint32_t c_share,
@@ -81,8 +70,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     const uint32_t n_blocks = (n_tiles + 3u) / 4u;
     const uint32_t c0 = lg_first(slice, c_share, c_more), c1 = lg_first(slice + 1u, c_share, c_more), len = c1 - c0;
     const uint32_t b0 = lg_first(group, b_share, b_more), b1 = lg_first(group + 1u, b_share, b_more), own = b1 - b0;
-    // blocks of a round (the last one may have fewer)
-    const uint32_t rounds = (own + kLgBlocks - 1u) / kLgBlocks, at_once = rounds == 1u ? own : most_at_once;
+    const uint32_t rounds = lg_rounds(own), at_once = lg_at_once(own, most_at_once);
     const uint32_t total = rounds * len;
     const uint32_t tile_at = smem + P::kLutBytes + wave * kTile;
     // (base registers that the compiler takes as they are, the rest in the accesses' offset fields)
@@ -347,40 +335,14 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     }
 }
 
-// How the work is cut: groups of 16 .. 128 activation rows, slices of the columns and groups of 16-row blocks, a workgroup
-// per CU. Of all such cuts the one with the shortest estimate, in units of some half nanosecond: 250 for each block of weights that a SIMD has
-// in a stage (its vector instructions), 125 for each 16 activation rows, 3 for each of these and block (operands read from LDS), and no
-// less than the way of a stage's requests and activations takes with few blocks; the slices' sums cost a launch and their way through memory.
-// Fitted to all cuts, timed, of 52 shapes from 256 x 4096 to 17408 x 5120 at 9 to 160 rows and 3, 5 and 8 bits: within 0.55 % of the shortest
-// in the mean, 13 % at worst (1.2 and 33 without that least, which cut long rows so that a workgroup has few blocks and many cells: 2048 x 17408
-// at 16 rows 18.4 us against 14.3, 8192 x 2048 (5 bits) at 64 rows 18.9 against 16.2).
-struct LgPlan { uint32_t m_groups, mb, slices, groups; };
-static LgPlan lg_plan(const LanesDev &L, int m) {
-    const uint32_t blocks = (L.n_tiles + 3u) / 4u, m_blocks = ((uint32_t)m + 15u) / 16u;
-    LgPlan best{};
-    uint64_t best_cost = ~0ull;
-    for (uint32_t m_groups = (m_blocks + kLgMost - 1u) / kLgMost; m_groups <= max((m_blocks + 1u) / 2u, 1u); ++m_groups) {
-        const uint32_t mb = (m_blocks + m_groups - 1u) / m_groups, cus = max(ln_cus() / m_groups, 1u);
-        for (uint32_t s = 1; s <= min(L.n_cells, cus); ++s) {
-            const uint32_t groups = min(max(cus / s, 1u), blocks);
-            const uint32_t share = (blocks + groups - 1u) / groups, rounds = (share + kLgBlocks - 1u) / kLgBlocks;
-            const uint32_t at_once = (share + rounds - 1u) / rounds, cells = (L.n_cells + s - 1u) / s;
-            const uint64_t stage = max(250u * ((at_once + 3u) / 4u) + 125u * mb + 3u * mb * at_once, 400u + 115u * mb);
-            const uint64_t sums = s > 1 ? 1600u + (uint64_t)s * (uint32_t)m * blocks * 16u / 670u : 0u;
-            const uint64_t cost = 4u * stage * rounds * cells + sums;
-            if (cost < best_cost) { best_cost = cost; best = {m_groups, mb, s, groups}; }
-        }
-        if (m_groups * 2u > ln_cus()) break;
-    }
-    return best;
-}
+static LgPlan lg_cut(const LanesDev &L, int m) { return lg_plan(L.n_tiles, L.n_cells, m, ln_cus()); }
 
 static size_t lg_bytes(const LanesDev &L, const LgPlan &p, int m) {
     return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * ((L.n_tiles + 3u) / 4u * 16u) * sizeof(float) : 0;
 }
 
 size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m) {
-    return lanes_prompt_wins(L, m) ? lanes_prompt_workspace_bytes(L, m) : lg_bytes(L, lg_plan(L, m), m);
+    return lanes_prompt_wins(L, m) ? lanes_prompt_workspace_bytes(L, m) : lg_bytes(L, lg_cut(L, m), m);
 }
 
 template <int BITS, int MB, int DEPTH>
@@ -391,10 +353,10 @@ static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, in
     static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemm<BITS, MB, DEPTH>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
     if (!raised) return IXH_ELAUNCH;
-    const uint32_t blocks = (L.n_tiles + 3u) / 4u, most = (blocks + p.groups - 1u) / p.groups, rounds = (most + kLgBlocks - 1u) / kLgBlocks;
+    const uint32_t blocks = (L.n_tiles + 3u) / 4u;
     const LgSplit c(L.n_cells, p.slices), b(blocks, p.groups);
     hipLaunchKernelGGL((k_lanes_gemm<BITS, MB, DEPTH>), dim3(p.slices, p.groups, p.m_groups), dim3(kLgBlocks * kWave), lds, s, L.plane, x, L.scale,
-                       c.share, c.more, b.share, b.more, L.in_f, (uint32_t)ldx, (uint32_t)m, (most + rounds - 1u) / rounds, L.n_cells,
+                       c.share, c.more, b.share, b.more, L.in_f, (uint32_t)ldx, (uint32_t)m, lg_most_at_once(blocks, p.groups), L.n_cells,
                        L.n_tiles, L.exc_off, L.exc_pos, L.exc_val, L.out_f, ws, ((uintptr_t)ws & 15u) == 0, bias, once, y, ldy);
     if (p.slices > 1)
         return launch_lanes_reduce(ws, p.slices, m, L.out_f, (L.n_tiles + 3u) / 4u * 16u, bias, once, y, ldy, s);
@@ -423,7 +385,7 @@ int launch_lanes_gemm(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, 
                       int64_t ldy, LnScratch &ws, hipStream_t s) {
     if (!lanes_gemm_aligned(L, x, m, ldx)) return IXH_EUNSUPPORTED;
     if (lanes_prompt_wins(L, m)) return launch_lanes_prompt(L, x, m, ldx, bias, y, ldy, ws, s);
-    const LgPlan p = lg_plan(L, m);
+    const LgPlan p = lg_cut(L, m);
     if (!ws.holds(lg_bytes(L, p, m))) return IXH_EWORKSPACE;
     if (m == 1) ldx = L.in_f;
     switch (L.bits) {

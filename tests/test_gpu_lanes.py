@@ -272,6 +272,29 @@ def test_many_rows_of_larger_weights(oracle, dev, out_f, in_f, m):
     check(oracle, p, x, y)
 
 
+def planned(bounds, dev, out_f, in_f, m):
+    """(groups of activation rows, blocks of 16 of them in a group, slices of the columns, groups of weight rows) of k_lanes_gemm."""
+    out = (C.c_uint32 * 4)()
+    bounds.plan(out_f, -(-in_f // 512), m, torch.cuda.get_device_properties(dev).multi_processor_count, out)
+    return tuple(out)
+
+
+@pytest.mark.parametrize("kind,out_f,in_f,m,most,least", [
+    ("real", 13616, 2560, 1, 17, 16), ("rare", 16400, 512, 512, 29, 28), ("real", 9808, 6656, 17, 33, 32),
+    ("rare", 9984, 6656, 17, 33, 32), ("four", 10048, 6656, 17, 34, 33)])
+def test_workgroups_of_several_rounds(bounds, dev, oracle, kind, out_f, in_f, m, most, least):
+    """More blocks of weight rows than a workgroup has waves, and one more for some than for others: also where these have a round less."""
+    groups, blocks = planned(bounds, dev, out_f, in_f, m)[3], -(-out_f // 16)
+    assert (-(-blocks // groups), blocks // groups) == (most, least) or torch.cuda.get_device_properties(dev).multi_processor_count != 256
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    x = activations(m, in_f, seed=m).to(dev)
+    weight = bits_to_bf16(oracle.decode_packed_bf16(p)).to(dev).reshape(out_f, in_f).float()
+    y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
+    lanes.gemm(x, y)
+    # (see test_many_rows_of_the_largest_weights)
+    assert rel_l2(y.float().cpu().numpy(), (x.float() @ weight.t()).bfloat16().float().cpu().numpy()) <= 1e-3
+
+
 @pytest.mark.parametrize("kind,out_f,in_f", [("rare", 1638, 2560), ("rare", 1639, 2560), ("real", 40, 2040), ("real", 40, 2048),
                                              ("real", 4095, 2048), ("real", 4096, 2048), ("four", 5120, 5112), ("four", 5120, 5120)])
 def test_nine_to_sixteen_rows_either_way(oracle, dev, kind, out_f, in_f):

@@ -1,41 +1,8 @@
 """What the lane kernels ask for ahead of need stays inside their buffers, and what the prompts' workgroups leave in memory has
 places of its own: the ranges of ``csrc/ixh_lanes_bounds.h`` walked on the host (the header is plain C++)."""
 import ctypes as C
-import os
-import subprocess
 
 import pytest
-
-CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ixrun_amd", "csrc")
-SOURCE = """
-#include "ixh_lanes_bounds.h"
-extern "C" void groups(uint32_t first, uint32_t end, uint32_t n, uint32_t *out) {
-    const ixh::LnGroups g = ixh::ln_groups(first, end, n);
-    out[0] = g.first; out[1] = g.last; out[2] = g.n;
-}
-extern "C" uint32_t four_quads(uint32_t from, uint32_t lane, uint32_t end) { return ixh::ln_four_quads(from, lane, end); }
-extern "C" int whole(uint64_t x, uint32_t in_f, int m, int64_t ldx) { return ixh::ln_whole_pieces(x, in_f, m, ldx); }
-extern "C" uint32_t column(uint32_t col, uint32_t in_f) { return ixh::ln_piece_column(col, in_f); }
-extern "C" uint32_t share(uint32_t n, uint32_t wave, uint32_t log_waves) { return ixh::ln_share(n, wave, log_waves); }
-extern "C" uint32_t listed_at(uint32_t pos, uint32_t value, int in_range, uint32_t seg, uint32_t cells) {
-    return ixh::ln_listed_at(pos, value, in_range, seg, cells);
-}
-extern "C" uint32_t begin(uint32_t g, uint32_t groups, uint32_t tiles, uint32_t cells) { return ixh::lp_begin(g, groups, tiles, cells); }
-extern "C" uint32_t group_of(uint32_t c, uint32_t groups, uint32_t tiles, uint32_t cells) { return ixh::lp_group_of(c, groups, tiles, cells); }
-extern "C" uint32_t part(uint32_t g, uint32_t tile, int begins, uint32_t groups, uint32_t tiles) { return ixh::lp_part(g, tile, begins, groups, tiles); }
-extern "C" uint32_t parts(uint32_t groups, uint32_t tiles) { return ixh::lp_parts(groups, tiles); }
-"""
-
-
-@pytest.fixture(scope="module")
-def bounds(tmp_path_factory):
-    d = tmp_path_factory.mktemp("bounds")
-    (d / "bounds.cpp").write_text(SOURCE)
-    subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", CSRC, str(d / "bounds.cpp"),
-                           "-o", str(d / "bounds.so")])
-    lib = C.CDLL(str(d / "bounds.so"))
-    lib.whole.argtypes = [C.c_uint64, C.c_uint32, C.c_int, C.c_int64]
-    return lib
 
 
 @pytest.mark.parametrize("total", [0, 1, 63, 64, 65, 127, 128, 129, 192])
@@ -141,6 +108,40 @@ def test_parts_of_shared_tiles_each_have_a_place(bounds, cells):
                 g0, g1 = (bounds.group_of(tile * cells + c, groups, tiles, cells) for c in (0, cells - 1))
                 begins = bounds.begin(g0, groups, tiles, cells) == tile * cells
                 assert own == ([] if g0 == g1 else [bounds.part(g0, tile, begins, groups, tiles)] + list(range(g0 + 1, g1 + 1)))
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3, 7, 8, 19, 32, 51, 64, 85, 128, 256])
+def test_blocks_of_a_workgroups_rounds_follow_one_another(bounds, groups):
+    """Every block of weight rows in work once, whatever a workgroup has more or less than the others: shares of all sizes up to five rounds."""
+    for blocks in [*range(groups, 5 * 16 * groups + groups, max(1, groups // 5)), *(k * groups + d for k in (16, 17, 32, 33, 48, 64) for d in (-1, 0, 1))]:
+        if blocks >= groups:
+            assert bounds.uncovered(blocks, groups) == 0, (blocks, groups)
+
+
+def test_parts_of_a_whole_are_those_of_a_division(bounds):
+    for n in [*range(1, 70), 136, 1088, 1089, 65535, 8388608]:
+        for k in [k for k in (*range(1, 40), 61, 85, 127, 128, 253, 256, 1021, 65521, 65536) if k <= n]:
+            for i in {0, 1, 2, k // 3, k // 2, k - 1, k}:
+                assert bounds.first(i, n, k) == i * n // k, (i, n, k)
+
+
+@pytest.mark.parametrize("cus", [256, 304, 64, 1])
+def test_cuts_of_prompts_take_everything(bounds, cus):
+    """Over the shapes and row counts that the kernel is given: slices and groups of at least a cell and a block, all activation rows in
+    groups of at most 128, every block in work once."""
+    out, seen = (C.c_uint32 * 4)(), set()
+    for out_f in (1, 16, 17, 260, 512, 1536, 2752, 4100, 5120, 8208, 8256, 9808, 10240, 13120, 13616, 16400, 16512, 16640, 17408, 40000, 70000):
+        for cells in (1, 2, 3, 5, 8, 10, 13, 16, 22, 34, 130):
+            if out_f * cells * 512 > 9e7 and out_f <= 17408 and cells <= 34:
+                continue
+            for m in (1, 9, 16, 17, 25, 33, 64, 65, 100, 128, 129, 160, 512, 1024, 4096):
+                bounds.plan(out_f, cells, m, cus, out)
+                m_groups, mb, slices, groups = out
+                blocks = -(-out_f // 16)
+                assert 1 <= slices <= cells and 1 <= groups <= blocks and 1 <= mb <= 8 and m_groups * mb * 16 >= m
+                if (blocks, groups) not in seen:
+                    seen.add((blocks, groups))
+                    assert bounds.uncovered(blocks, groups) == 0, (out_f, cells, m)
 
 
 def described(out_f, in_f, bits=3):
