@@ -230,8 +230,8 @@ int64_t ixh_lanes_plane_words(int64_t out_f, int64_t in_f, int32_t bits);
 int64_t ixh_lanes_cells(int64_t out_f, int64_t in_f);
 
 /*
- * Writing it, from the bf16 weights that ixh_decode makes of the packed tensor (out_f x in_f, dense; the integers come
- * back exactly).  ixh_lanes_pack writes the plane and the number of quads of every cell to `counts` (ixh_lanes_cells
+ * Writing it, from the bf16 weights that ixh_decode makes of the packed tensor (out_f x in_f, dense, all finite; the integers
+ * come back exactly).  ixh_lanes_pack writes the plane and the number of quads of every cell to `counts` (ixh_lanes_cells
  * entries); the caller turns those into exc_off (an exclusive running sum, the total behind the last), zeroes exc_val
  * and ixh_lanes_list fills both in, with positions of no effect where there is no element.  In both, `dst` names the buffers (written despite the const of its
  * fields; ixh_lanes_pack uses plane and scale only).

@@ -437,6 +437,12 @@ class LanePacked:
             return None
         return 4 * words + 4 * (cells + 1) + max(4 * sum(c for b, c in zip(level_bits, counts) if b > bits), 64 * 12)
 
+    @staticmethod
+    def holds(scale: torch.Tensor) -> bool:
+        """Whether all weights of this scale are finite in bf16: the layout is made from those, and an infinite one's integer is lost
+        (one synchronisation)."""
+        return abs(float(scale)) * 127 < 2.0 ** 128 - 2.0 ** 119  # (from there on the rounding goes to infinity)
+
     @property
     def nbytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self.tensors)

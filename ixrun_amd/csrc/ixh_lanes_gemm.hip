@@ -108,7 +108,8 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     };
 
     Pieces first = x_load(4u * c0);
-    // (5 bits: scales of 2^100 and more are taken as 2^-32 of them, so that their multiples are no infinities)
+    // (5 bits: scales of 2^100 and more are taken as 2^-32 of them, so that their multiples are no infinities.  The rounding is the same: a
+    // layout's weights are finite at the scale itself.)
     const float scale_full = bf16_bits_to_f32(*scale_at);
     const bool big = BITS == 5 && fabsf(scale_full) >= 0x1p100f;
     const float scale = big ? scale_full * 0x1p-32f : scale_full;

@@ -169,7 +169,7 @@ class StreamingLinear(nn.Module):
         self._lanes = None
         n_bytes = _lane_bytes(self.level_bits, self.out_features, self.in_features, self.counts)
         free, total = torch.cuda.mem_get_info(self._scale.device)
-        if not n_bytes or free - n_bytes - 2 * self.N < total // 4:
+        if not n_bytes or free - n_bytes - 2 * self.N < total // 4 or not _lib.LanePacked.holds(self._scale):
             for name in LANE_BUFFERS:
                 self.register_buffer(name, None, persistent=False)
             self._bind()
@@ -285,7 +285,13 @@ class StreamingLinear(nn.Module):
         if self._flat_table is not None:
             self._flat_table.copy_(self._dp.prefix_build(FUSED_TILE))
         if self._lanes is not None:  # a layer that was built without lanes stays without
-            self._refresh_lanes()
+            if _lib.LanePacked.holds(self._scale):
+                self._refresh_lanes()
+            else:
+                self._replaced_lanes.append(self._lanes)  # (see _refresh_lanes)
+                for name in LANE_BUFFERS:
+                    setattr(self, name, None)
+                self._bind()
         self._stale = False
 
     def _refresh_lanes(self):

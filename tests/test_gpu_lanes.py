@@ -328,6 +328,36 @@ def test_many_rows_at_extreme_scales(oracle, dev, kind, scale):
         assert rel_l2(got, oracle.bf16_bits_to_f32(want)) <= 1e-3
 
 
+@pytest.mark.parametrize("scale,lanes", [(2.0 ** 121, True), ((1 + 2.0 ** -7) * 2.0 ** 121, False), (float("inf"), False), (float("nan"), False)])
+def test_weights_that_round_to_infinities(oracle, dev, scale, lanes):
+    """The layout is made from the bf16 weights and has no place for an infinite one: such a layer (its largest weight is the largest bf16
+    value) has none, also when its state comes later, and its products have the infinities of its decode."""
+    from ixrun_amd.engine import StreamingLinear
+
+    out_f, in_f = 260, 2048
+    v = values("rare", out_f, in_f)[0]
+    v[5::1009] = 127 - 254 * (np.arange(v[5::1009].size) % 2)
+    p = packed_from_int8(v, out_f, in_f)
+    other = StreamingLinear(p, None)
+    assert other._lanes is not None
+    p = dict(p, scale=torch.full_like(p["scale"], scale))
+    layer = StreamingLinear(p, None)
+    other.load_state_dict(layer.state_dict())
+    weight = bits_to_bf16(oracle.decode_packed_bf16(p)).reshape(out_f, in_f).double()
+    assert bool(weight.isfinite().all()) == lanes
+    for each in (layer, other):
+        assert (each._lanes is not None) == lanes
+        each._set_shared_buf(torch.empty(out_f * in_f, dtype=torch.bfloat16, device=dev))
+        for m in (1, 2, 4, 8, 16, 17, 100):
+            x = (activations(m, in_f, seed=m).float() * 2.0 ** -20).bfloat16()
+            with torch.no_grad():
+                y = each(x.to(dev)).double().cpu()
+            want = x.double() @ weight.t()
+            assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y[y.isinf()], want[want.isinf()])
+            fine = want.isfinite()  # (the power of two takes the squares to where they are finite; it changes no rounding)
+            assert rel_l2(y[fine].numpy() * 2.0 ** -110, want[fine].bfloat16().double().numpy() * 2.0 ** -110) <= 1e-3 or not fine.any()
+
+
 def test_prompts_of_a_layer_take_the_lanes_in_every_form(oracle, dev):
     """What goes to the fused decode+GEMM comes out as from the layer without lanes, whatever the activations' form; what it
     is not for (gradients, other types, more rows) still goes through the decode."""
