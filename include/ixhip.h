@@ -283,6 +283,7 @@ size_t ixh_lanes_gemm_workspace_bytes(const IxhLanes *lanes, int32_t m);
  * struct's fields), the scale and the table written by ixh_encode_scan for the same w.
  * No write goes past the lengths given in dst.
  */
+/* Enough for smaller weights as well. */
 size_t ixh_encode_workspace_bytes(int64_t out_f, int64_t in_f, int32_t n_levels);
 
 int ixh_encode_scan(const uint16_t *w, int64_t out_f, int64_t in_f, int32_t n_levels, const int32_t *level_bits,

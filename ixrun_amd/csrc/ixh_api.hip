@@ -692,14 +692,15 @@ static int encode_scan(const uint16_t *w, int64_t out_f, int64_t in_f, int32_t n
     const uint64_t n = (uint64_t)out_f * (uint64_t)in_f;
     if (n >= (1ull << 31)) { set_error("out_f * in_f = %llu does not fit the 31-bit rank tables", (unsigned long long)n); return IXH_EINVAL; }
     if (!w || !scale || !prefix) { set_error("encode: w, scale or prefix is NULL"); return IXH_EINVAL; }
-    const size_t need = encode_workspace_bytes(n, n_levels);
+    const size_t need = encode_workspace_least(n, n_levels);
     if (!workspace || workspace_bytes < need) {
         set_error("workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
         return IXH_EWORKSPACE;
     }
     int bits[IXH_MAX_LEVELS];
     for (int i = 0; i < n_levels; ++i) bits[i] = level_bits[i];
-    rc = launch_encode_scan(w, (uint32_t)n, n_levels, bits, scale, prefix, workspace, host_counts, (hipStream_t)stream);
+    rc = launch_encode_scan(w, (uint32_t)n, n_levels, bits, scale, prefix, workspace, workspace_bytes, host_counts,
+                            (hipStream_t)stream);
     if (rc == IXH_ELAUNCH) set_error("encode_scan: launch failed");
     return rc;
 }

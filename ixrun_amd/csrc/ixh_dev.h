@@ -146,8 +146,9 @@ bool prefill_supports(const Dev &P, const uint16_t *x, int64_t ldx);
 int launch_prefill(const Dev &P, const int32_t *prefix, const uint16_t *x, uint32_t m_rows, int64_t ldx, uint16_t *y,
                    int64_t ldy, float *ws, hipStream_t s);
 size_t encode_workspace_bytes(uint64_t n, int n_levels);
+size_t encode_workspace_least(uint64_t n, int n_levels);
 int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *bits, uint16_t *scale, int32_t *table,
-                       void *workspace, int64_t *host_totals, hipStream_t s);
+                       void *workspace, size_t workspace_bytes, int64_t *host_totals, hipStream_t s);
 int launch_encode_pack(const uint16_t *w, const Dev &P, const int32_t *table, hipStream_t s);
 int launch_fill_u16(uint16_t *dst, uint32_t n, uint16_t value, hipStream_t s);
 void set_error(const char *fmt, ...);

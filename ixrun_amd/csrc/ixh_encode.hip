@@ -640,30 +640,35 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
 }
 
 // workspace: partial maxima (kEncParts), sums of k_enc_count's workgroups
-static uint32_t group_units(uint64_t n) { return (n + kEncUnit - 1) / kEncUnit <= kCountFew ? kCountFewUnits : kCountUnits; }
-static uint32_t count_groups(uint64_t n) {
-    const uint64_t group = (uint64_t)kEncUnit * group_units(n);
+static uint32_t count_groups(uint64_t n, uint32_t units) {
+    const uint64_t group = (uint64_t)kEncUnit * units;
     return (uint32_t)((n + group - 1) / group);
+}
+static size_t workspace_bytes_by(uint64_t n, int n_levels, uint32_t units) {
+    return 4u * (kEncParts + (size_t)(n_levels - 1) * count_groups(n, units));
 }
 
 size_t encode_workspace_bytes(uint64_t n, int n_levels) {
-    return 4u * (kEncParts + (size_t)(n_levels - 1) * count_groups(n));
+    return workspace_bytes_by(n, n_levels, (n + kEncUnit - 1) / kEncUnit <= kCountFew ? kCountFewUnits : kCountUnits);
 }
+// What a call does with: a small weight asks for more than a larger one may have (2^24 weights for 2048 sums a level, 2^25 for 1024), so
+// a scratch that is shared by weights of several sizes takes the small ones by larger workgroups.
+size_t encode_workspace_least(uint64_t n, int n_levels) { return workspace_bytes_by(n, n_levels, kCountUnits); }
 
 template <int L>
-static void scan_launch(const uint16_t *w, uint32_t n, uint32_t n_units, const EncLevels &lv, const uint32_t *parts,
+static void scan_launch(const uint16_t *w, uint32_t n, uint32_t n_units, uint32_t group_units, const EncLevels &lv, const uint32_t *parts,
                         uint16_t *scale, int32_t *table, uint32_t *sums, hipStream_t s) {
-    if (group_units(n) == kCountUnits)
-        hipLaunchKernelGGL((k_enc_count<L, kCountUnits>), dim3(count_groups(n)), dim3(kWave * kEncWaves), 0, s, w, n, n_units, parts, lv, table,
-                           sums, scale);
+    const dim3 grid(count_groups(n, group_units)), block(kWave * kEncWaves);
+    if (group_units == kCountUnits)
+        hipLaunchKernelGGL((k_enc_count<L, kCountUnits>), grid, block, 0, s, w, n, n_units, parts, lv, table, sums, scale);
     else
-        hipLaunchKernelGGL((k_enc_count<L, kCountFewUnits>), dim3(count_groups(n)), dim3(kWave * kEncWaves), 0, s, w, n, n_units, parts, lv,
-                           table, sums, scale);
+        hipLaunchKernelGGL((k_enc_count<L, kCountFewUnits>), grid, block, 0, s, w, n, n_units, parts, lv, table, sums, scale);
 }
 
 int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *bits, uint16_t *scale, int32_t *table,
-                       void *workspace, int64_t *host_totals, hipStream_t s) {
+                       void *workspace, size_t workspace_bytes, int64_t *host_totals, hipStream_t s) {
     const uint32_t n_units = (n + kEncUnit - 1) / kEncUnit;
+    const uint32_t group_units = n_units <= kCountFew && workspace_bytes >= encode_workspace_bytes(n, n_levels) ? kCountFewUnits : kCountUnits;
     const uint32_t tiles = max(1u, (n_units + kScanTile - 1) / kScanTile);
     uint32_t *parts = static_cast<uint32_t *>(workspace);
     uint32_t *sums = parts + kEncParts;
@@ -672,16 +677,16 @@ int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *b
     for (int i = 0; i < IXH_MAX_LEVELS; ++i) lv.bits[i] = i < n_levels ? bits[i] : 0;
     hipLaunchKernelGGL(k_enc_absmax, dim3(kEncParts), dim3(1024), 0, s, w, n, parts);
     switch (n_levels) {
-        case 2: scan_launch<2>(w, n, n_units, lv, parts, scale, table, sums, s); break;
-        case 3: scan_launch<3>(w, n, n_units, lv, parts, scale, table, sums, s); break;
-        case 4: scan_launch<4>(w, n, n_units, lv, parts, scale, table, sums, s); break;
-        case 5: scan_launch<5>(w, n, n_units, lv, parts, scale, table, sums, s); break;
-        case 6: scan_launch<6>(w, n, n_units, lv, parts, scale, table, sums, s); break;
-        case 7: scan_launch<7>(w, n, n_units, lv, parts, scale, table, sums, s); break;
-        default: scan_launch<8>(w, n, n_units, lv, parts, scale, table, sums, s); break;
+        case 2: scan_launch<2>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
+        case 3: scan_launch<3>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
+        case 4: scan_launch<4>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
+        case 5: scan_launch<5>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
+        case 6: scan_launch<6>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
+        case 7: scan_launch<7>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
+        default: scan_launch<8>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
     }
-    hipLaunchKernelGGL(k_enc_scan, dim3(tiles, n_levels - 1), dim3(1024), 0, s, table, n_units, sums, count_groups(n),
-                       group_units(n), host_totals);
+    hipLaunchKernelGGL(k_enc_scan, dim3(tiles, n_levels - 1), dim3(1024), 0, s, table, n_units, sums,
+                       count_groups(n, group_units), group_units, host_totals);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 

@@ -211,6 +211,28 @@ def test_encode_counts_by_groups_of_either_size(oracle, dev, n, top):
     check_against_oracle(oracle, dev, w, (3, 5, 8))
 
 
+@pytest.mark.parametrize("units,of_units", [(32768, 32769), (32768, 32768), (40, 64), (20000, 32769), (16, 16)])
+def test_encode_scratch_of_a_larger_weight(dev, units, of_units):
+    """A scratch that the size call names for one weight is enough for smaller ones, and nothing behind it is written."""
+    import ctypes as C
+
+    from ixrun_amd import _lib
+
+    L, levels = _lib.lib(), (3, 5, 8)
+    n = units * 512
+    w = make_weight("calibrated_odd_scale", 1, n).to(dev)
+    need = int(L.ixh_encode_workspace_bytes(1, of_units * 512, len(levels)))
+    ws = torch.full((need + 4096,), 0xA5, dtype=torch.uint8, device=dev)
+    scale = torch.zeros(1, dtype=torch.bfloat16, device=dev)
+    table = torch.empty(2 * (units + 1), dtype=torch.int32, device=dev)
+    bits = (C.c_int32 * len(levels))(*levels)
+    _lib.check(L.ixh_encode_scan(w.data_ptr(), 1, n, len(levels), bits, scale.data_ptr(), table.data_ptr(), ws.data_ptr(), need,
+                                 _lib.current_stream(dev)))
+    assert bool((ws[need:] == 0xA5).all())
+    packed, whole, _ = _lib.encode_device(w, levels)
+    assert torch.equal(table.view(2, -1), whole.view(2, -1))
+
+
 SCAN = "ixh_encode_scan_counts"
 
 
