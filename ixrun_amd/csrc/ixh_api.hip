@@ -623,7 +623,7 @@ size_t ixh_lanes_gemv_workspace_bytes(const IxhLanes *lanes, int32_t m) {
     // From five rows on, what any count up to 16 takes: a batch that grows makes no caller replace its buffer (a shared one that
     // captured graphs hold is kept for them beside the new one).
     if (m <= 4) return lanes_gemv_takes(d, m) ? 0 : lanes_rows_workspace_bytes(d, m);
-    return max(lanes_rows_workspace_bytes(d, m), max(lanes_rows_workspace_bytes(d, 8), lanes_rows_workspace_bytes(d, 16)));
+    return lanes_rows_workspace_most(d);
 }
 
 int ixh_lanes_gemv(const IxhLanes *lanes, const uint16_t *x, int64_t ldx, const uint16_t *bias, int32_t m, uint16_t *y,

@@ -79,7 +79,8 @@ int launch_lanes_list(const uint16_t *w, const LanesDev &L, uint16_t *pos, int8_
 bool lanes_gemv_takes(const LanesDev &L, int m);
 int launch_lanes_gemv(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y,
                       int64_t ldy, LnScratch &ws, hipStream_t s);
-size_t lanes_rows_workspace_bytes(const LanesDev &L, int m);
+size_t lanes_rows_workspace_bytes(const LanesDev &L, int m);  // in k_lanes_rows
+size_t lanes_rows_workspace_most(const LanesDev &L);           // of any count from five to sixteen, whichever kernel takes it
 int launch_lanes_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, uint16_t *y, int64_t ldy,
                       LnScratch &ws, hipStream_t s);
 // 17 and more rows (ixh_lanes_gemm.hip), the bias added before the one rounding (once) or after one, then rounded again;

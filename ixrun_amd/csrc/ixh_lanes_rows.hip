@@ -427,9 +427,14 @@ static size_t lr_bytes(const LanesDev &L, const LrPlan &p, int m) {
     return p.slices > 1 ? (size_t)p.slices * (uint32_t)m * L.n_tiles * 4u * sizeof(float) : 0;
 }
 
-size_t lanes_rows_workspace_bytes(const LanesDev &L, int m) {
-    const size_t sums = lr_bytes(L, lr_plan_of(L, m), m);
-    return lr_gemm_wins(L, m) ? max(sums, lanes_gemm_workspace_bytes(L, m)) : sums;
+size_t lanes_rows_workspace_bytes(const LanesDev &L, int m) { return lr_bytes(L, lr_plan_of(L, m), m); }
+
+// (k_lanes_gemm cuts the columns finer for fewer rows, and then takes more)
+size_t lanes_rows_workspace_most(const LanesDev &L) {
+    size_t most = max(lanes_rows_workspace_bytes(L, 8), lanes_rows_workspace_bytes(L, 16));
+    if (lr_gemm_wins(L, 16))
+        for (int m = 9; m <= 16; ++m) most = max(most, lanes_gemm_workspace_bytes(L, m));
+    return most;
 }
 
 template <int BITS, int MT, bool WIDE>

@@ -272,6 +272,26 @@ def test_many_rows_of_larger_weights(oracle, dev, out_f, in_f, m):
     check(oracle, p, x, y)
 
 
+@pytest.mark.parametrize("kind,out_f,in_f", [("real", 4347, 6032), ("real", 5120, 5120), ("rare", 1024, 8192), ("four", 1000, 4096)])
+def test_scratch_of_any_count_up_to_sixteen(oracle, dev, kind, out_f, in_f):
+    """What five rows ask for is enough for any count up to sixteen, whichever kernel takes it, and nothing behind it is written."""
+    from ixrun_amd import _lib
+
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    need = lanes.gemv_workspace_bytes(5)
+    assert all(lanes.gemv_workspace_bytes(m) == need for m in range(5, 17))
+    ws = torch.full((need + 4096,), 0xA5, dtype=torch.uint8, device=dev)
+    weight = bits_to_bf16(oracle.decode_packed_bf16(p)).to(dev).reshape(out_f, in_f).float()
+    for m in range(5, 17):
+        x = activations(m, in_f, seed=m).to(dev)
+        y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
+        _lib.check(_lib.lib().ixh_lanes_gemv(C.byref(lanes.struct), x.data_ptr(), in_f, None, m, y.data_ptr(), out_f, ws.data_ptr(), need,
+                                             _lib.current_stream(dev)))
+        # (see test_many_rows_of_the_largest_weights)
+        assert rel_l2(y.float().cpu().numpy(), (x.float() @ weight.t()).bfloat16().float().cpu().numpy()) <= 1e-3
+    assert bool((ws[need:] == 0xA5).all())
+
+
 def planned(bounds, dev, out_f, in_f, m):
     """(groups of activation rows, blocks of 16 of them in a group, slices of the columns, groups of weight rows) of k_lanes_gemm."""
     out = (C.c_uint32 * 4)()
