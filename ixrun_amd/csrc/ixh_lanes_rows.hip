@@ -408,19 +408,27 @@ static LrPlan lr_plan_of(const LanesDev &L, int m) {
 }
 
 // Nine to sixteen rows: turning the activations round for the whole of a long slice, or starting up for a single cell, takes longer than
-// k_lanes_gemm's way, whose sixteen waves share a copy of 128 columns a stage, up to 20 * 2^20 weights, and of long rows at 4, 5 and 8 bits
-// from 25 to 48 * 2^20; not of tall layers, of which a workgroup here has one slice.  us, this / that at 16 rows, 5 bits: 512 x 512
-// 6.6 / 5.7, 1024 x 1024 7.2 / 7.9, 512 x 2048 8.7 / 7.9, 2048 x 2048 8.8 / 9.0, 4096 x 2048 9.0 / 9.4, 1536 x 6144 13.1 / 10.1, 4096 x 4096
-// 12.0 / 11.1, 8192 x 2560 12.1 / 12.6, 4096 x 6144 13.9 / 14.8, 5120 x 5120 15.7 / 15.0, 6144 x 6144 18.0 / 17.0, 9216 x 5120 20.8 / 18.6, 8192 x
-// 4096 14.0 / 15.0, 17408 x 5120 28.6 / 30.1.  Three bits, whose pairs sit in LDS 32 times over here: 512 x 4096 8.6 / 8.5, 2560 x 2560 10.3 / 9.1,
-// 1536 x 6144 12.4 / 9.5, 4096 x 4096 10.4 / 9.6, 8192 x 2560 9.4 / 11.0, 3072 x 8192 12.4 / 12.1, 4096 x 6144 11.5 / 12.3, 6144 x 6144 14.6 / 14.8.
+// k_lanes_gemm's way, whose sixteen waves share a copy of 128 columns a stage, up to 20 * 2^20 weights, and of long rows from 25 * 2^20 to
+// 46 at 5 bits and 38 at 8; not of tall layers, of which a workgroup here has one slice.  us, this / that at 16 rows (nine and twelve
+// are within 4 % of that):
+//   5 bits   1024 x 1024 7.2 / 7.6, 2048 x 2048 8.8 / 8.7, 2560 x 2560 10.6 / 9.2, 2048 x 4096 10.4 / 9.7, 4096 x 2048 9.1 / 9.8, 1536 x 6144
+//            12.6 / 10.2, 4096 x 4096 12.0 / 11.6, 4096 x 5120 13.9 / 12.9, 3072 x 8192 15.5 / 14.0, 4096 x 6144 14.2 / 14.8, 5120 x 5120 15.8 /
+//            15.0, 4096 x 8192 15.9 / 16.0, 6144 x 6144 18.4 / 17.8, 6656 x 6656 20.9 / 19.0, 9216 x 5120 21.1 / 19.1, 4096 x 12288 20.1 / 20.8
+//   8 bits   2048 x 2048 7.1 / 7.4, 2048 x 4096 9.0 / 8.3, 1536 x 6144 10.4 / 8.8, 4096 x 4096 9.7 / 10.0, 4096 x 5120 11.1 / 10.8, 4096 x 6144
+//            11.7 / 11.9, 5120 x 5120 13.3 / 12.4, 2880 x 9536 13.4 / 13.1, 4096 x 8192 14.5 / 14.3, 6144 x 6144 15.5 / 15.6, 8192 x 5120 16.1 /
+//            16.5, 6656 x 6656 18.4 / 16.5, 4096 x 11008 16.7 / 17.3, 2560 x 17408 16.2 / 17.2
+//   4 bits   2048 x 2048 7.9 / 7.9, 2560 x 2560 9.0 / 8.6, 1536 x 6144 11.0 / 9.5, 4096 x 4096 10.2 / 10.8, 5120 x 5120 13.3 / 14.1, 6144 x 6144
+//            14.6 / 16.4, 4096 x 11008 15.4 / 18.2
+//   3 bits   (whose pairs sit in LDS 32 times over here) 2048 x 2048 7.6 / 7.5, 2560 x 2560 8.5 / 8.4, 2048 x 4096 9.1 / 8.4, 4096 x 2048 7.7 / 8.5,
+//            1536 x 6144 10.5 / 9.1, 2048 x 8192 10.1 / 9.9, 4096 x 4096 9.8 / 9.9, 4096 x 5120 10.9 / 11.3, 4096 x 6144 11.2 / 12.7
 static bool lr_gemm_wins(const LanesDev &L, int m) {
     const uint64_t n = (uint64_t)L.out_f * L.in_f;
     if (m <= 8) return false;
     if (L.bits != 3 && L.in_f <= kLnCols) return n <= 20u << 20;
     if (L.out_f >= 2ull * L.in_f) return false;
     if (L.bits == 3) return L.in_f >= 2560u && n > 4u << 20 && n <= 20u << 20;
-    return n <= 20u << 20 ? L.in_f >= 2048u : L.in_f >= 4608u && n >= 25u << 20 && n <= 48u << 20;
+    if (n <= 20u << 20) return L.in_f >= 2048u;
+    return L.bits != 4 && L.in_f >= 4608u && n >= 25u << 20 && n <= (L.bits == 5 ? 46u : 38u) << 20;
 }
 
 static size_t lr_bytes(const LanesDev &L, const LrPlan &p, int m) {

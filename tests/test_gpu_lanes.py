@@ -316,7 +316,9 @@ def test_workgroups_of_several_rounds(bounds, dev, oracle, kind, out_f, in_f, m,
 
 
 @pytest.mark.parametrize("kind,out_f,in_f", [("rare", 1638, 2560), ("rare", 1639, 2560), ("real", 40, 2040), ("real", 40, 2048),
-                                             ("real", 4095, 2048), ("real", 4096, 2048), ("four", 5120, 5112), ("four", 5120, 5120)])
+                                             ("real", 4095, 2048), ("real", 4096, 2048), ("four", 5120, 5112), ("four", 5120, 5120),
+                                             ("real", 5120, 5112), ("real", 5120, 5120), ("wide", 5120, 5112), ("wide", 5120, 5120),
+                                             ("real", 9420, 5120), ("real", 9421, 5120), ("wide", 7782, 5120), ("wide", 7783, 5120)])
 def test_nine_to_sixteen_rows_either_way(oracle, dev, kind, out_f, in_f):
     """Weights on both sides of the lines between the two kernels that take nine to sixteen rows; few blocks and many, one cell to ten a slice."""
     p, lanes = lay_out(kind, out_f, in_f, dev)
