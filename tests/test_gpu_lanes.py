@@ -179,6 +179,18 @@ def test_rows_at_the_edges_of_their_slices(oracle, dev, kind, out_f, in_f, m):
         assert torch.equal(y, product(lanes, x, out_f, in_f, bias.to(dev)))
 
 
+@pytest.mark.parametrize("ldx", [(1 << 27) - 2, (1 << 27) - 1, 1 << 27, (1 << 27) + 2])
+def test_rows_far_apart(oracle, dev, ldx):
+    """Strides on both sides of 2^27 elements, up to which pairs are asked for at places in 32 bits."""
+    out_f, in_f, m = 37, 3586, 16
+    p, lanes = lay_out("real", out_f, in_f, dev)
+    x = activations(m, in_f, seed=m)
+    far = torch.empty((m - 1) * ldx + in_f, dtype=torch.bfloat16, device=dev).as_strided((m, in_f), (ldx, 1))
+    far.copy_(x)
+    for n in (5, 8, 16):
+        check(oracle, p, x[:n], product(lanes, far[:n], out_f, in_f))
+
+
 @pytest.mark.parametrize("kind", ["four", "real"])
 @pytest.mark.parametrize("out_f,in_f", [(4131, 1500), (4131, 3080)])
 def test_both_tables_of_pairs(oracle, dev, kind, out_f, in_f):
@@ -264,7 +276,7 @@ def test_scratch_of_prompts_at_any_address(oracle, dev, kind, out_f, in_f):
 
 @pytest.mark.parametrize("out_f,in_f,m", [(4100, 520, 20), (4500, 1536, 130), (20, 33800, 40)])
 def test_many_rows_of_larger_weights(oracle, dev, out_f, in_f, m):
-    """Workgroups with several rounds of blocks, and slices of several cells."""
+    """Several blocks of weight rows a workgroup, and slices of several cells."""
     p, lanes = lay_out("real", out_f, in_f, dev)
     x = activations(m, in_f, seed=m)
     y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
@@ -328,26 +340,57 @@ def test_nine_to_sixteen_rows_either_way(oracle, dev, kind, out_f, in_f):
         check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f, bias.to(dev)), bias)
 
 
-@pytest.mark.parametrize("scale", [2.0 ** -100, 1.5 * 2.0 ** 99, 2.0 ** 100, 1.75 * 2.0 ** 112])
+# rows of activations that one workgroup takes, 16 a block: a shape whose cut leaves them together (33 slices, three or four blocks of weight
+# rows a workgroup and one less; the last cell and its last 128 columns incomplete)
+def shape_of_blocks(bounds, dev, m):
+    out_f, in_f = 205 if m <= 48 else 397, 16800
+    together = planned(bounds, dev, out_f, in_f, m)[1] == max(-(-m // 16), 1)
+    assert together or torch.cuda.get_device_properties(dev).multi_processor_count != 256
+    return out_f, in_f
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 48, 50, 64, 65, 79, 81, 96, 97, 112, 113, 127, 128])
+@pytest.mark.parametrize("kind", ["narrow", "rare", "four", "real", "full_row", "wide"])
+def test_each_count_of_blocks_of_activation_rows(bounds, oracle, dev, kind, m):
+    """Every form of the kernel, with whole and nearly empty last blocks."""
+    out_f, in_f = shape_of_blocks(bounds, dev, m)
+    p, lanes = lay_out(kind, out_f, in_f, dev)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16().to(dev) if m % 2 else None
+    x = activations(m, in_f + 8, seed=m).to(dev)[:, 8:]
+    weight = bits_to_bf16(oracle.decode_packed_bf16(p)).to(dev).reshape(out_f, in_f).double()
+    y = torch.full((2, m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
+    for t in y:
+        lanes.gemm(x, t, bias)
+    want = (x.double() @ weight.t() + (0 if bias is None else bias.double())).float().bfloat16()
+    # (see test_many_rows_of_the_largest_weights)
+    assert rel_l2(y[0].float().cpu().numpy(), want.float().cpu().numpy()) <= 1e-3
+    assert torch.equal(y[0], y[1])
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -100, 1.5 * 2.0 ** 99, 2.0 ** 100, 1.75 * 2.0 ** 112, 2.0 ** 120])
 @pytest.mark.parametrize("kind", ["four", "real"])
-def test_many_rows_at_extreme_scales(oracle, dev, kind, scale):
+def test_many_rows_at_extreme_scales(bounds, oracle, dev, kind, scale):
     """Multiples of the scale by up to 2^20 stand behind codes of five bits; from 2^100 on they would be infinities.  Every count of blocks of
-    16 activation rows."""
-    out_f, in_f = 260, 1032
-    v, scheme, _ = values(kind, out_f, in_f)
-    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
-    p["scale"] = torch.full_like(p["scale"], scale)
-    p, lanes = lay_out_values(p, out_f, in_f, dev)
-    for m in (17, 48, 64, 80, 96, 112, 128):
-        x = (activations(m, in_f, seed=m).float() * 2.0 ** -12).bfloat16()
-        y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
-        lanes.gemm(x.to(dev), y)
+    16 activation rows, and nine and 16 as a batch (rounded before the bias as well as after it)."""
+    down = 2.0 ** -int(np.log2(scale))  # (a power of two takes the sums to where their squares are finite; it changes no rounding)
+    for m in (9, 16, 17, 48, 64, 80, 96, 112, 128):
+        out_f, in_f = shape_of_blocks(bounds, dev, m)
+        v, scheme, _ = values(kind, out_f, in_f)
+        p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
+        p["scale"] = torch.full_like(p["scale"], scale)
+        p, lanes = lay_out_values(p, out_f, in_f, dev)
+        x = (activations(m, in_f, seed=m).float() * 2.0 ** -12).bfloat16().to(dev)
+        weight = bits_to_bf16(oracle.decode_packed_bf16(p)).to(dev).reshape(out_f, in_f).double()
+        want = (x.double() @ weight.t() * down).float().bfloat16()
+        if m <= 16:
+            bias = (want[0].double() / down).bfloat16()
+            y = product(lanes, x, out_f, in_f, bias)
+            want = (want.double() + bias.double() * down).float().bfloat16()
+        else:
+            y = torch.full((m, out_f), 7.0, dtype=torch.bfloat16, device=dev)
+            lanes.gemm(x, y)
         assert bool(y.isfinite().all())
-        # (a power of two takes the sums to where the oracle's squares are finite; it changes no rounding)
-        p_one = dict(p, scale=torch.full_like(p["scale"], scale * 2.0 ** -int(np.log2(scale))))
-        want = oracle.f32_to_bf16_bits(oracle.gemm_f64(oracle.decode_packed_bf16(p_one), bf16_bits(x)).astype(np.float32))
-        got = (y.double() * 2.0 ** -int(np.log2(scale))).cpu().numpy()
-        assert rel_l2(got, oracle.bf16_bits_to_f32(want)) <= 1e-3
+        assert rel_l2((y.double() * down).cpu().numpy(), want.double().cpu().numpy()) <= 1e-3
 
 
 @pytest.mark.parametrize("scale,lanes", [(2.0 ** 121, True), ((1 + 2.0 ** -7) * 2.0 ** 121, False), (float("inf"), False), (float("nan"), False)])
