@@ -38,8 +38,9 @@ __device__ __forceinline__ uint32_t ln_pack(float lo, float hi) {
 template <int BITS, bool WIDE> struct LnPairs {
     // log2: 32 copies of 64 entries never collide, nor do 16 of 256 or 1024 much (a look-up 4.0 clocks of the LDS, against 6.1 with 8
     // copies of 1024 and 6.9 with one; 2.2 without collisions).  WIDE, where LDS has the room: 17408 x 5120, 5 bits, one row
-    // 15.9 us with 8 copies and every third pair by arithmetic, 15.2 with 16.  k_lanes_gemm gains nothing from four (5 bits)
-    // or sixteen (4 bits) instead of two: 10240 x 5120, 100 rows, 5 bits 47.3 and 47.8 us.
+    // 15.9 us with 8 copies and every third pair by arithmetic, 15.2 with 16.  k_lanes_gemm with two / four (5 bits) or
+    // sixteen (4 bits): 10240 x 5120 at 17 / 64 / 100 rows, 5 bits 22.4 / 27.5 / 34.7 and 22.3 / 27.6 / 34.8 us, 4 bits 21.2 / 26.3 / 33.2 and 19.7 /
+    // 24.7 / 31.6, which is not taken yet.
     static constexpr int kCopies = BITS == 3 ? 5 : WIDE ? 4 : 1;
     static constexpr uint32_t kEntries = BITS == 8 ? 0u : 1u << (2 * BITS);
     static constexpr uint32_t kLutBytes = kEntries << (kCopies + 2);
@@ -73,7 +74,7 @@ template <int SH> __device__ __forceinline__ uint32_t ln_shift(uint32_t w) {
 }
 // Where copies of a table do not collide: 5120 x 17408 (3 bits), from graphs over copies beyond the last-level cache, at 1 / 8 / 16 / 64 rows
 // 12.2 / 16.3 / 19.5 / 35.6 us with shifts, 11.8 / 15.8 / 18.8 / 34.9 so (one layer over and over, one row: 10.5 and 9.9), 10240 x 5120 (5 bits) at 1 / 8 rows 11.1 / 16.3 and 10.8 / 15.5.  With two copies the look-ups are what a wave waits
-// for: 1536 x 3072 (4 bits) at 12 / 32 rows 8.3 / 9.1 with shifts, 8.5 / 9.3 so, 10240 x 5120 (5 bits) at 128 rows 41.0 and 41.7.
+// for: 1536 x 3072 (4 bits) at 12 / 32 rows 8.0 / 8.6 with shifts, 8.2 / 8.8 so, 10240 x 5120 (4 bits) at 100 rows 33.2 either way.
 template <class P> constexpr bool ln_float_shifts = P::kCopies > 1;
 // the address of the pair whose code begins at bit OFF of a dword (without FLOAT less lut_lane)
 template <class P, int BITS, int OFF, bool FLOAT> __device__ __forceinline__ uint32_t ln_pair_at(uint32_t w, uint32_t lut_lane) {

@@ -6,12 +6,14 @@ namespace ixh {
 // ---------------------------------------------------------------------------------------------------------------
 // k_lanes_gemm<BITS, MB, DEPTH>: up to 16 * MB activation rows at a time, MB <= 8; DEPTH activation operands in flight.
 //
-// Bound: a stage's vector instructions (decode, listed elements), then LDS (operands read back, look-ups, stores), then the parts of a stage
-// that follow one another in a wave, while all waves meet at its end; the matrix unit is busy for 15 % of it.  10240 x 5120 at 55 / 40 /
-// 5 %, 100 rows: 34.2 us with the slices' sums (37.7 with two blocks of 16 weight rows a wave from 49 rows on, which halves the reads of
-// activations, and half as many waves to fill in for one another: 64 rows 30.9 -> 27.3, 128 rows 40.6 -> 37.5; 74.3 for the decode to
-// memory and the library's GEMM).  Looking up the next stage's weights between the products of this one changes nothing, nor does the list
-// half a cell earlier; waves of their own for decode and products (eight and four, a stage of 64 columns) take 44; activations straight
+// Bound: a stage's parts (decode, listed elements, products), which follow one another in a wave while all waves meet at its end; no unit is
+// full.  10240 x 5120 at 55 / 40 / 5 %, 100 rows: vector instructions are in issue for 41 % of the time, LDS is busy for 42 (a fifth of
+// that with collisions), the matrix unit for 18; waves wait for 56 % of theirs.  34.7 us with the slices' sums (37.7 with two blocks of 16
+// weight rows a wave from 49 rows on, which halves the reads of activations, and half as many waves to fill in for one another: 64 rows
+// 30.9 -> 27.3, 128 rows 40.6 -> 37.5; 74.3 for the decode to memory and the library's GEMM); without the products and the operands
+// read for them 28.4, without the listed elements 30.1, without the decode 33.1, without the activations' copies 32.9.  Looking up the next
+// stage's weights between the products of this one changes nothing, nor does the list half a cell earlier; waves of their own for decode
+// and products (eight and four, a stage of 64 columns) take 44; activations straight
 // from the L2 as operands twice as long.  A wave takes 16 weight rows x 128 columns a stage: it decodes them to its own 4 KB of LDS in
 // operand order, stores the listed elements over their places and reads the operands back.  All waves of the workgroup are in the same
 // 128 columns, whose activations one copy in LDS serves (in operand order, two stages of it: the next one is fetched during the
@@ -31,9 +33,9 @@ __device__ __forceinline__ void lg_barrier() { asm volatile("s_waitcnt lgkmcnt(0
 // 5 bits: two of the three whole pairs of a dword by arithmetic, which evens out the LDS and the vector unit.  A code at bit P is, as the
 // bits of a float, a multiple of the smallest one: times 2^127 it is code * 2^(P - 22), and that times scale * 2^(22 - P) less 15 scale is
 // value * scale, all exact: an AND, a product and a multiply-add, each at the full rate, where a shift left, an AND-OR and a
-// multiply-add took 12 clocks instead of 7.  (us, all looked up / one of three / two, with two
-// blocks a wave from 49 rows on, 10240 x 5120 at 55 / 40 / 5 %: 32 rows 24.6 / - / 22.8, 64 rows 30.8 / 29.6 / 29.6, 100 rows 37.5 / 37.0 /
-// 36.7; 4096 x 4096, 100 rows 23.9 / 23.1 / 23.0.)
+// multiply-add took 12 clocks instead of 7.  (us, all looked up / one of three by arithmetic / two, 10240 x 5120 at 55 / 40 / 5 %: 17 rows
+// 23.9 / 23.1 / 22.4, 32 rows 24.6 / 23.6 / 23.0, 64 rows 29.7 / 28.5 / 27.5, 100 rows 36.1 / 35.1 / 34.7, 128 rows 39.6 / 39.0 / 37.8; 4096 x 4096,
+// 100 rows 21.1 / 20.7 / 20.5.)
 struct LgScale { float at2, at7, at12, at17, off; };
 __device__ __forceinline__ float lg_value(uint32_t field, float by, float off) { return __fmaf_rn(__uint_as_float(field) * 0x1p127f, by, off); }
 __device__ __forceinline__ void lg_decode5(const uint32_t (&w)[5], uint32_t lut_lane, const LgScale &k, uint32_t (&o)[16]) {
@@ -202,13 +204,13 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     for (uint32_t u = 0; u < total; ++u) {
         // ---- listed elements: value (high half), where it goes in the tile of its quarter (bits 0..11; the tile's block i
         // is at i ^ q, as the list has it), the quarter (bits 12..14; none of the four where there is no element) ----
-        // Rounds that no row has elements for are passed over (3 bits, 5120 x 17408 Student-t at 17 rows 28.8 -> 27.5 us, 5 bits at 5 %
-        // listed, 10240 x 5120 at 40 rows 28.5 -> 27.7).
+        // Rounds that no row has elements for are passed over (us, taken / passed over: 3 bits, 0.3 % listed, 5120 x 17408 at 17 rows 28.1 /
+        // 26.5; 5 bits, 5 % listed, 10240 x 5120 at 17 / 64 / 100 / 128 rows 22.1 / 27.3 / 35.6 / 39.7 and 22.4 / 27.5 / 34.7 / 37.8).
         uint32_t put[4 * ROUNDS];
         const uint32_t cell_bits = (now.c % kLnSegCells << 10) * 0x10001u;
         // A round's stores in each quarter that any lane has elements of, without branches around them: a lane's elements of other
-        // quarters go behind the tile.  (5 bits at 5 % listed, 10240 x 5120 at 17 / 64 / 100 / 128 rows 24.5 / 32.2 / 39.0 / 41.5 -> 23.6 /
-        // 30.5 / 37.6 / 40.2, with two blocks a wave.)
+        // quarters go behind the tile.  (A branch a store / so: 5 bits at 5 % listed, 10240 x 5120 at 17 / 64 / 100 / 128 rows 22.8 / 36.3 /
+        // 36.7 / 41.3 and 22.4 / 27.5 / 34.7 / 37.8 us; 3 bits, 5120 x 17408 at 17 rows 29.5 and 26.5.)
         uint32_t in_q[ROUNDS];  // bit q: the lane has elements of quarter q in the round
 #pragma unroll
         for (uint32_t r = 0; r < ROUNDS; ++r) {

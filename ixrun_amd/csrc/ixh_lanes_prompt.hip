@@ -421,7 +421,8 @@ static uint32_t lp_part_size(const LpPlan &p) { return kLpWaves * p.mi * (8u / p
 // (3 bits) 50 / 53 at 128 rows, 61 / 52 at 144, 138 / 97 at 512; 5120 x 5120 25 / 28, 27 / 29, 56 / 48; 5120 x 4096 25 / 28 at 144
 // rows and 47 / 46 at 512; 4096 x 4096 (5 bits) 26 / 28 at 192 rows, 41 / 44 at 512; 2048 x 2048 23 / 35 at 512; at 129 / 256 / 512 rows:
 // 5120 x 5120 (5) 31 / 29, 37 / 35, 60 / 52, 17408 x 5120 (5) 80 / 65, 101 / 83, 196 / 120, 5120 x 5120 (8) 26 / 26,
-// 33 / 33, 55 / 51, 12288 x 6144 (8) 52 / 54, 68 / 69, 114 / 104.  The bounds keep offsets within 32 bits.
+// 33 / 33, 55 / 51, 12288 x 6144 (8) 52 / 54, 68 / 69, 114 / 104.  (The line is that of a k_lanes_gemm that took 10 to 20 % longer; it is now up to
+// 7 % the faster one on this side of it, up to some 192 rows of 2^25 weights and 256 at 8 bits.)  The bounds keep offsets within 32 bits.
 bool lanes_prompt_wins(const LanesDev &L, int m) {
     return m > 128 && (uint64_t)L.out_f * L.in_f > 3u << 23 && (uint64_t)lp_tiles(L.n_tiles) * L.n_cells < 1u << 24 &&
            (uint64_t)L.n_cells * 16u * (((uint32_t)m + 15u) / 16u) * 1024u < 1ull << 31;

@@ -347,7 +347,8 @@ k_lanes_rows(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
 // sums cost a launch and their way through memory.  Fitted to all cuts, timed, of 54 shapes from 512 x 512 to 17408 x 5120 and 20480 x 4096
 // at 8 and 16 rows and 3, 5 and 8 bits: within 1.0 % of the shortest in the mean, 9 % at worst (1.9 and 15 with 400 for a wave and without
 // the XCDs' terms: eight rows of 2048 x 11008, 5 bits, in eleven slices instead of eight 12.6 us against 11.3, 2048 x 6144 by sixteen waves
-// instead of eight 11.0 against 10.5).  (Without a cost of each wave, and the slices dearer, layers of few rows had one slice of sixteen waves
+// instead of eight 11.0 against 10.5; where this one errs: 1760 x 12320, 5 bits, at 16 rows 15.4 us against 14.3 by that, 5024 x 9472, 3 bits, at
+// eight 13.2 against 12.4, 2880 x 13728, 8 bits, at eight 15.1 against 14.6).  (Without a cost of each wave, and the slices dearer, layers of few rows had one slice of sixteen waves
 // where several of four fill the CUs: 960 x 3072 at 11 rows 11.0 us against 8.9, 256 x 4096 11.9 against 8.7.)
 struct LrPlan { uint32_t slices, groups, waves, x_rows; size_t lds; };
 

@@ -199,7 +199,9 @@ class StreamingLinear(nn.Module):
         against 27 / 35 / 37 / 49 / 57, 17408 x 5120 90 / 94 / 94 / 101 / 115 against 42 / 55 / 61 / 75 / 85.  3 bits at 64 / 100 /
         200 / 256: 10240 x 5120 65 / 66 / 70 / 70 against 28 / 35 / 49 / 49, 17408 x 5120 96 / 101 / 111 / 115 against 46 / 53 / 76
         / 77.  8 bits, which have no list, at 64 / 100 / 160: 10240 x 5120 62 / 62 / 71 against 28 / 35 / 45, 17408 x 5120 102 /
-        106 / 116 against 49 / 55 / 68, 4096 x 4096 30 / 31 / 39 against 17 / 23 / 24.  Below 2**24
+        106 / 116 against 49 / 55 / 68, 4096 x 4096 30 / 31 / 39 against 17 / 23 / 24.  (From 2**24 to 3 * 2**23 weights the lanes
+        win further now than the line has it: at 192 / 256 / 384 / 512 rows 4096 x 4096 (5 bits) 43 / 34 / 37 / 41 against 27 / 30 / 36 / 42,
+        4608 x 5120 (8 bits) 52 / 62 / 49 / 56 against 28 / 31 / 48 / 56, 5120 x 4096 (3 bits) 40 / 47 / 37 / 42 against 29 / 32 / 37 / 47.)  Below 2**24
         weights the decode, the GEMM and the host's way through both weigh more: 12000 x 768 at 256 rows 35 against 29, 2048 x 2048
         23 against 21 (eager: 31 against 20), and up to 2**20 weights 15 against 14 at 512 rows (eager 31 against 13).  Layers of at
         most 2**18 weights keep decoding into their buffer (12 us at 100 rows; the lanes took 8), which callers see there.  Rows of
