@@ -6,7 +6,8 @@
 // of its time on ranks: prefix sums over bitmap words, windows at bit offsets that depend on them, a splice or a
 // gather per element (7 to 16 vector instructions a weight).  Here a weight is `bits` wide (3, 4, 5 or 8) and sits in
 // the registers of the lane that multiplies it as soon as it is loaded; the few elements whose value does not fit go
-// to a list.  The values are the same integers: nothing is rounded on the way.
+// to a list.  The values are the same integers: nothing is rounded on the way.  (They are taken from the bf16 weights, so a tensor whose scale
+// makes some of these infinite has no lane layout.)
 //
 //   cell      4 weight rows x 512 columns = 2048 weights, 64 lanes x `bits` dwords.  Cell (t, c) holds rows 4 t ..
 //             4 t + 3 and columns 512 c ..; cells are stored row quads first: index t * n_cells + c.
