@@ -38,9 +38,7 @@ __device__ __forceinline__ uint32_t ln_pack(float lo, float hi) {
 template <int BITS, bool WIDE> struct LnPairs {
     // log2: 32 copies of 64 entries never collide, nor do 16 of 256 or 1024 much (a look-up 4.0 clocks of the LDS, against 6.1 with 8
     // copies of 1024 and 6.9 with one; 2.2 without collisions).  WIDE, where LDS has the room: 17408 x 5120, 5 bits, one row
-    // 15.9 us with 8 copies and every third pair by arithmetic, 15.2 with 16.  k_lanes_gemm with two / four (5 bits) or
-    // sixteen (4 bits): 10240 x 5120 at 17 / 64 / 100 rows, 5 bits 22.4 / 27.5 / 34.7 and 22.3 / 27.6 / 34.8 us, 4 bits 21.2 / 26.3 / 33.2 and 19.7 /
-    // 24.7 / 31.6, which is not taken yet.
+    // 15.9 us with 8 copies and every third pair by arithmetic, 15.2 with 16.  k_lanes_gemm: see kLgWide.
     static constexpr int kCopies = BITS == 3 ? 5 : WIDE ? 4 : 1;
     static constexpr uint32_t kEntries = BITS == 8 ? 0u : 1u << (2 * BITS);
     static constexpr uint32_t kLutBytes = kEntries << (kCopies + 2);

@@ -23,6 +23,11 @@ namespace ixh {
 // A workgroup owns a slice of the columns (whole cells) of a run of 16-row blocks, sixteen at most at a time; the slices' sums
 // meet in the workspace and launch_lanes_reduce adds them in slice order.
 // ---------------------------------------------------------------------------------------------------------------
+// Sixteen copies of the pair table at 4 bits, whose pairs are all looked up and whose 16 KB LDS holds beside 128 activation rows: two / sixteen, us from
+// graphs, 10240 x 5120 at 17 / 64 / 100 / 128 rows 21.9 / 27.3 / 34.2 / 36.6 and 20.5 / 25.5 / 32.3 / 34.9, 17408 x 5120 at 80 46.5 / 43.4, 2048 x 2048 at 16 /
+// 100 7.5 / 12.1 and 7.4 / 11.5, 320 x 2048 at 20 7.2 / 7.0, 30 such calls 0.957 in the mean and none more than before. At 5 bits, where two of three pairs are worked
+// out, four copies gain nothing (10240 x 5120 at 17 / 64 / 100 rows 22.4 / 27.5 / 34.7 and 22.3 / 27.6 / 34.8), and 64 KB are not there.
+template <int BITS> constexpr bool kLgWide = BITS == 4;
 constexpr uint32_t kLgTile = 4096;
 constexpr uint32_t kLgTileBytes = kLgTile + 256u;  // and a dword a lane behind it, for what is not to be stored
 // where what the next stage could begin with between the products of this one takes more registers than there are
@@ -61,7 +66,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
              const uint32_t *__restrict__ exc_off, const uint16_t *__restrict__ exc_pos, const int8_t *__restrict__ exc_val, uint32_t out_f,
              float *__restrict__ ws, bool ws_aligned, const uint16_t *__restrict__ bias, bool once, uint16_t *__restrict__ y, int64_t ldy) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lg_smem[];
-    using P = LnPairs<BITS, false>;
+    using P = LnPairs<BITS, kLgWide<BITS>>;
     constexpr uint32_t kTile = kLgTileBytes;
     constexpr uint32_t kThreads = kLgBlocks * kWave;
     const uint32_t smem = (uint32_t)(uintptr_t)(LN_LDS(uint8_t) *)lg_smem;
@@ -117,7 +122,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     const float scale = big ? scale_full * 0x1p-32f : scale_full;
 
     if (wave >= at_once) {  // no block: this wave's part of the copies only
-        ln_build_lut<BITS, false>(smem, scale, tid, kThreads);
+        ln_build_lut<BITS, kLgWide<BITS>>(smem, scale, tid, kThreads);
         x_store(first, 4u * c0, 0);
         lg_barrier();
         uint32_t c = c0;
@@ -192,7 +197,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
     for (uint32_t q = 0; q < 2; ++q) codes(from, c0, q);
     Quads list = quads(e_now);
     Extent e_next = extent(next);
-    ln_build_lut<BITS, false>(smem, scale, tid, kThreads);
+    ln_build_lut<BITS, kLgWide<BITS>>(smem, scale, tid, kThreads);
     x_store(first, 4u * c0, 0);
     lg_barrier();
     const LgScale scales{scale * 0x1p20f, scale * 0x1p15f, scale * 0x1p10f, scale * 0x1p5f, -15.0f * scale};
@@ -248,7 +253,7 @@ k_lanes_gemm(const uint32_t *__restrict__ plane, const uint16_t *__restrict__ x,
             Pieces x_next = x_load(g_next);
             uint32_t o[16];
             if constexpr (BITS == 5) lg_decode5(w[q & 1u], lut_lane, scales, o);
-            else ln_decode<BITS, false>(w[q & 1u], lut_lane, scale, o);
+            else ln_decode<BITS, kLgWide<BITS>>(w[q & 1u], lut_lane, scale, o);
             codes(q < 2 ? from : from_next, q < 2 ? now.c : next.c, q ^ 2u);
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i)
@@ -351,7 +356,7 @@ size_t lanes_gemm_workspace_bytes(const LanesDev &L, int m) {
 template <int BITS, int MB, int DEPTH>
 static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, int m, int64_t ldx, const uint16_t *bias, bool once,
                        uint16_t *y, int64_t ldy, float *ws, hipStream_t s) {
-    constexpr size_t lds = LnPairs<BITS, false>::kLutBytes + kLgBlocks * kLgTileBytes + 2u * MB * 4096u;
+    constexpr size_t lds = LnPairs<BITS, kLgWide<BITS>>::kLutBytes + kLgBlocks * kLgTileBytes + 2u * MB * 4096u;
     static_assert(lds <= kLnLds, "LDS of a CU");
     static const bool raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_lanes_gemm<BITS, MB, DEPTH>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
