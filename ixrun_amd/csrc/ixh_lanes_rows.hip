@@ -390,13 +390,16 @@ static LrPlan lr_plan(const LanesDev &L) {
 
 // The larger pair table up to eight rows (LDS has the room beside their activations) and from some cells a CU on: below, what it
 // saves is less than its 64 KB take to write (5 bits, 8 rows, larger / smaller: 512 x 512 5.9 / 5.2 us, 2000 x 2048 with 8 cells a CU
-// 6.9 / 6.6, 4000 x 3072 with 24 8.9 / 8.6, 2000 x 8192 with 32 11.1 / 11.8, 5000 x 5120 with 50 12.7 / 12.8).
+// 6.9 / 6.6, 4000 x 3072 with 24 8.9 / 8.6, 2000 x 8192 with 32 11.1 / 11.8, 5000 x 5120 with 50 12.7 / 12.8).  At 4 bits,
+// where it is 16 KB, up to sixteen rows (smaller / larger at 16: 17408 x 5120 24.0 / 21.9, 5120 x 17408 24.2 / 22.2, 10240 x 5120 18.4 / 16.9,
+// 5120 x 5120 with 50 cells a CU 14.1 / 13.3, 4096 x 4096 with 32 10.6 / 10.6, 8192 x 1024 with 16 7.3 / 7.3, 1024 x 1024 6.7 / 6.8).
 template <int BITS> static bool lr_wide(const LanesDev &L, int m) {
-    return (BITS == 4 || BITS == 5) && m <= 8 && (uint64_t)L.n_tiles * L.n_cells > 24u * ln_cus();
+    const uint64_t cells = (uint64_t)L.n_tiles * L.n_cells;
+    return m <= 8 ? (BITS == 4 || BITS == 5) && cells > 24u * ln_cus() : BITS == 4 && cells > 32u * ln_cus();
 }
 
 template <int BITS> static LrPlan lr_plan_rows(const LanesDev &L, int m) {
-    if (lr_wide<BITS>(L, m)) return lr_plan<BITS, 8, true>(L);
+    if (lr_wide<BITS>(L, m)) return m <= 8 ? lr_plan<BITS, 8, true>(L) : lr_plan<BITS, 16, true>(L);
     return m <= 8 ? lr_plan<BITS, 8, false>(L) : lr_plan<BITS, 16, false>(L);
 }
 static LrPlan lr_plan_of(const LanesDev &L, int m) {
@@ -468,7 +471,8 @@ int launch_lanes_rows(const LanesDev &L, const uint16_t *x, int m, int64_t ldx, 
                       LnScratch &ws, hipStream_t s) {
     if (lr_gemm_wins(L, m) && lanes_gemm_aligned(L, x, m, ldx)) return launch_lanes_gemm(L, x, m, ldx, bias, false, y, ldy, ws, s);
 #define LR_ROWS(B)                                                                                                              \
-    (lr_wide<B>(L, m) ? rows_launch<B, 8, (B == 4 || B == 5)>(L, x, m, ldx, bias, y, ldy, ws, s)                                 \
+    (lr_wide<B>(L, m) ? m <= 8 ? rows_launch<B, 8, (B == 4 || B == 5)>(L, x, m, ldx, bias, y, ldy, ws, s)                        \
+                               : rows_launch<B, 16, B == 4>(L, x, m, ldx, bias, y, ldy, ws, s)                                   \
      : m <= 8         ? rows_launch<B, 8, false>(L, x, m, ldx, bias, y, ldy, ws, s)                                              \
                       : rows_launch<B, 16, false>(L, x, m, ldx, bias, y, ldy, ws, s))
     switch (L.bits) {

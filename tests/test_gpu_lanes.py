@@ -111,6 +111,14 @@ def test_long_rows_and_many_rows(oracle, dev, kind, out_f, in_f):
         check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
 
 
+@pytest.mark.parametrize("out_f,in_f,m", [(32801, 25, 9), (32801, 25, 16), (16501, 1030, 9), (16501, 1030, 16)])
+def test_four_bits_by_the_larger_table(oracle, dev, out_f, in_f, m):
+    """Nine to sixteen rows of more than 32 cells a CU: sixteen copies of the pair table beside the activations."""
+    p, lanes = lay_out("four", out_f, in_f, dev)
+    x = activations(m, in_f, seed=m)
+    check(oracle, p, x, product(lanes, x.to(dev), out_f, in_f))
+
+
 @pytest.mark.parametrize("at", [5, 32767, 32768, 33799])
 @pytest.mark.parametrize("listed", [1, 16, 17, 33])
 def test_list_of_one_segment_of_long_rows(oracle, dev, at, listed):
