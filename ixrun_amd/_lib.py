@@ -80,6 +80,12 @@ def host():
     return _native
 
 
+def is_current(device) -> bool:
+    """Whether a device, or its name, is the current GPU."""
+    device = torch.device(device)
+    return device.type == "cuda" and device.index in (None, torch.cuda.current_device())
+
+
 class IxhError(RuntimeError):
     """A call into libixhip returned a negative code."""
 

@@ -21,7 +21,7 @@ TORCH="$($PYTHON -c 'import os, importlib.util as u; print(os.path.dirname(u.fin
 PYINC="$($PYTHON -c 'import sysconfig; print(sysconfig.get_paths()["include"])')"
 g++ -O2 -std=c++17 -fPIC -shared -fvisibility=hidden -Wall -Wno-unknown-pragmas -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 \
     -I"$PYINC" -isystem "$TORCH/include" -isystem "$TORCH/include/torch/csrc/api/include" -isystem /opt/rocm/include \
-    ixh_host.cpp -o ../_host.so -L"$TORCH/lib" -lc10 -lc10_hip -ltorch_cpu -ltorch_python &
+    ixh_host.cpp -o ../_host.so -L"$TORCH/lib" -lc10 -lc10_hip -ltorch_cpu -ltorch_hip -ltorch_python &
 HOST_PID=$!
 OBJS=""
 for s in $SRCS; do OBJS="$OBJS build/${s%.hip}.o"; done

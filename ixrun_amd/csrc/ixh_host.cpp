@@ -1,18 +1,27 @@
 // ixrun_amd._host: the host side of the calls whose kernels are shorter than Python's bookkeeping around them.
 //
 // A forward of one token spends 5 us on the GPU; checked, allocated and launched from Python through ctypes it took the
-// host 8.  The same steps here: see the figures at each function.  Everything that is not the common case (other types,
+// host 8.  The same steps here: see the figures at each function.  (Whole calls with the caller's own Python around them, with memory
+// allocated through the dispatcher, plain calls found out in Python and the decoders' and the encoder's Python under a no_grad of its own / now: 1536 x
+// 1536, one row 7.0 / 6.8 us; 1024 x 1024 at 40 rows 11.4 / 10.5; decode of 1408 x 672 9.3 / 6.5, with group scales of 640 x 1024 9.6 / 7.2; encode of
+// 448 x 1024 39.3 / 36.2, of 2048 x 2500 40.0 / 37.3.)  Everything that is not the common case (other types,
 // other devices, views, a scratch that has to grow, errors) is left to the caller: a function returns None and has done
 // nothing, and the Python code behind it goes on.
 #include <Python.h>
 #include <structmember.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/core/Tensor.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/empty.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <vector>
 
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/ixhip.h"
@@ -21,6 +30,24 @@ namespace {
 
 using LanesGemv = decltype(&ixh_lanes_gemv);
 constexpr int kMaxRows = 16;
+
+// What this thread has on that looks at what goes through the dispatcher: modes, transforms, tracing.
+c10::DispatchKeySet watching() { return c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set; }
+
+// Memory on the GPU, as at::empty gives it, which takes 0.3 us longer.
+at::Tensor fresh(at::IntArrayRef size, at::ScalarType type, int64_t device) {
+    const c10::Device on(c10::kCUDA, (c10::DeviceIndex)device);
+    if (watching().empty()) return at::Tensor(at::detail::empty_cuda(size, type, on, std::nullopt));
+    return at::empty(size, at::TensorOptions().device(on).dtype(type));
+}
+
+// Whether a product of `x`, an exact tensor, that is not torch's own is what the caller gets from F.linear: engine._plain_call, which takes 0.4 us.
+bool plain_call(const at::Tensor &x) {
+    return !(x.requires_grad() && c10::GradMode::is_enabled()) && !torch::autograd::ForwardADLevel::try_get_by_idx(0) &&
+           !at::impl::torch_function_mode_enabled() &&
+           !watching().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::FuncTorchDynamicLayerBackMode})) &&
+           (!at::autocast::is_autocast_enabled(at::kCUDA) || at::autocast::get_autocast_dtype(at::kCUDA) == at::kBFloat16);
+}
 
 // The fused forward of one layer over its lane layout: an object called with the activations.
 struct Forward {
@@ -40,7 +67,6 @@ struct Forward {
     PyObject *workspaces;  // dict: device -> scratch tensor
     PyObject *device_key;
     PyObject *check;       // raises for a negative code
-    PyObject *plain;       // whether a call with these activations is a plain one
 };
 
 // A token of a layer of 2.4 M weights: 5 us of host time a call (8 us from Python).
@@ -55,13 +81,7 @@ PyObject *forward_call(PyObject *self_, PyObject *const *args, size_t nargsf, Py
         Py_RETURN_NONE;
     const int64_t rows = x.numel() / self->in_f;
     if (rows < 1 || rows > kMaxRows) Py_RETURN_NONE;
-    if (rows > self->any_rows) {
-        PyObject *r = PyObject_CallOneArg(self->plain, args[0]);
-        const int yes = r ? PyObject_IsTrue(r) : -1;
-        Py_XDECREF(r);
-        if (yes < 0) return nullptr;
-        if (!yes) Py_RETURN_NONE;
-    }
+    if (rows > self->any_rows && !plain_call(x)) Py_RETURN_NONE;
     const size_t need = self->workspace_bytes[rows];
     void *scratch = nullptr;
     if (need) {
@@ -81,7 +101,7 @@ PyObject *forward_call(PyObject *self_, PyObject *const *args, size_t nargsf, Py
     int rc;
     {
         pybind11::gil_scoped_release without_gil;
-        y = at::empty(shape, x.options());
+        y = fresh(shape, at::kBFloat16, self->device);
         rc = self->gemv(self->lanes, static_cast<const uint16_t *>(x.const_data_ptr()), self->in_f, self->bias, (int32_t)rows,
                         static_cast<uint16_t *>(y.data_ptr()), self->out_f, scratch, need,
                         c10::hip::getCurrentHIPStream((c10::DeviceIndex)self->device).stream());
@@ -109,20 +129,16 @@ PyObject *forward_many(PyObject *self_, PyObject *arg) {
         Py_RETURN_NONE;
     const int64_t rows = x.numel() / self->in_f;
     if (rows <= kMaxRows || rows > self->many_rows || (reinterpret_cast<uintptr_t>(x.const_data_ptr()) & 15u) != 0) Py_RETURN_NONE;
-    PyObject *plain = PyObject_CallOneArg(self->plain, arg);
-    const int yes = plain ? PyObject_IsTrue(plain) : -1;
-    Py_XDECREF(plain);
-    if (yes < 0) return nullptr;
-    if (!yes) Py_RETURN_NONE;
+    if (!plain_call(x)) Py_RETURN_NONE;
     c10::SmallVector<int64_t, 4> shape(x.sizes().begin(), x.sizes().end());
     shape.back() = self->out_f;
     at::Tensor y, sums;
     int rc;
     try {
         pybind11::gil_scoped_release without_gil;
-        y = at::empty(shape, x.options());
+        y = fresh(shape, at::kBFloat16, self->device);
         const size_t need = self->gemm_workspace_bytes(self->lanes, (int32_t)rows);
-        if (need) sums = at::empty({(int64_t)need}, x.options().dtype(at::kByte));
+        if (need) sums = fresh({(int64_t)need}, at::kByte, self->device);
         rc = self->gemm(self->lanes, static_cast<const uint16_t *>(x.const_data_ptr()), self->in_f, self->bias, (int32_t)rows,
                         static_cast<uint16_t *>(y.data_ptr()), self->out_f, need ? sums.data_ptr() : nullptr, need,
                         c10::hip::getCurrentHIPStream((c10::DeviceIndex)self->device).stream());
@@ -138,16 +154,16 @@ PyObject *forward_many(PyObject *self_, PyObject *arg) {
     END_HANDLE_TH_ERRORS
 }
 
-// Forward(gemv, lanes, bias, in_f, out_f, device, workspace_bytes, owner, workspaces, device_key, check, plain, gemm,
+// Forward(gemv, lanes, bias, in_f, out_f, device, workspace_bytes, owner, workspaces, device_key, check, gemm,
 // gemm_workspace_bytes); addresses as ints.  any_rows and many_rows are 0 until they are set.
 int forward_init(PyObject *self_, PyObject *args, PyObject *) {
     Forward *self = reinterpret_cast<Forward *>(self_);
     unsigned long long gemv, lanes, bias, gemm, gemm_workspace_bytes;
     long long in_f, out_f;
     long device;
-    PyObject *bytes, *owner, *workspaces, *key, *check, *plain;
-    if (!PyArg_ParseTuple(args, "KKKLLlO!OO!OOOKK", &gemv, &lanes, &bias, &in_f, &out_f, &device, &PyTuple_Type, &bytes, &owner,
-                          &PyDict_Type, &workspaces, &key, &check, &plain, &gemm, &gemm_workspace_bytes))
+    PyObject *bytes, *owner, *workspaces, *key, *check;
+    if (!PyArg_ParseTuple(args, "KKKLLlO!OO!OOKK", &gemv, &lanes, &bias, &in_f, &out_f, &device, &PyTuple_Type, &bytes, &owner,
+                          &PyDict_Type, &workspaces, &key, &check, &gemm, &gemm_workspace_bytes))
         return -1;
     if (!gemv || !lanes || !gemm || !gemm_workspace_bytes || in_f < 1 || out_f < 1 || PyTuple_GET_SIZE(bytes) != kMaxRows + 1) {
         PyErr_SetString(PyExc_ValueError, "Forward: malformed arguments");
@@ -166,9 +182,9 @@ int forward_init(PyObject *self_, PyObject *args, PyObject *) {
     self->in_f = in_f;
     self->out_f = out_f;
     self->device = device;
-    PyObject **slots[] = {&self->owner, &self->workspaces, &self->device_key, &self->check, &self->plain};
-    PyObject *values[] = {owner, workspaces, key, check, plain};
-    for (int i = 0; i < 5; ++i) {
+    PyObject **slots[] = {&self->owner, &self->workspaces, &self->device_key, &self->check};
+    PyObject *values[] = {owner, workspaces, key, check};
+    for (int i = 0; i < 4; ++i) {
         Py_INCREF(values[i]);
         Py_XSETREF(*slots[i], values[i]);
     }
@@ -193,7 +209,6 @@ int forward_traverse(PyObject *self_, visitproc visit, void *arg) {
     Py_VISIT(self->workspaces);
     Py_VISIT(self->device_key);
     Py_VISIT(self->check);
-    Py_VISIT(self->plain);
     return 0;
 }
 
@@ -204,7 +219,6 @@ int forward_clear(PyObject *self_) {
     Py_CLEAR(self->workspaces);
     Py_CLEAR(self->device_key);
     Py_CLEAR(self->check);
-    Py_CLEAR(self->plain);
     return 0;
 }
 
@@ -317,7 +331,7 @@ bool describe(PyObject *level_bits, long long out_f, long long in_f, PyObject *b
 // decode(level_bits, out_f, in_f, bitmaps, streams, scale, table, group_scales, group_size): the bf16 weight, by units of
 // 512; without a rank table small (3,5,8) tensors do without and for others one is built, with group scales (fp16, in place of `scale`) they are used.  Of tensors on the
 // current device.
-// 2048 x 2048 with a table: 9 us of host time (17 from Python).
+// 2048 x 2048 with a table: 6 us of host time (17 from Python).
 PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
     constexpr int64_t kUnit = 512;
@@ -347,9 +361,8 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     int rc = 0;
     {
         pybind11::gil_scoped_release without_gil;
-        const auto options = at::TensorOptions().device(c10::Device(c10::kCUDA, (c10::DeviceIndex)device));
         ixh_stream_t stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
-        w = at::empty({out_f, in_f}, options.dtype(at::kBFloat16));
+        w = fresh({out_f, in_f}, at::kBFloat16, device);
         uint16_t *out = static_cast<uint16_t *>(w.data_ptr());
         const uint16_t *of_groups = scales ? static_cast<const uint16_t *>(scales->const_data_ptr()) : nullptr;
         const bool ranked = given || !library.decode_unranked_takes(&p, of_groups, group, out);
@@ -357,7 +370,7 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
             rc = library.decode_unranked(&p, of_groups, group, out, stream);
         } else if (!given) {
             const size_t bytes = library.prefix_workspace_bytes(n, kUnit, p.n_levels);
-            table = at::empty({rows * entries + (int64_t)bytes / 4}, options.dtype(at::kInt));  // and the scratch
+            table = fresh({rows * entries + (int64_t)bytes / 4}, at::kInt, device);  // and the scratch
             int32_t *ranks = static_cast<int32_t *>(table.data_ptr());
             rc = library.prefix_build(&p, kUnit, ranks, ranks + rows * entries, bytes, stream);
         }
@@ -425,14 +438,13 @@ PyObject *encode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     int rc;
     {
         pybind11::gil_scoped_release without_gil;
-        const auto options = at::TensorOptions().device(c10::Device(c10::kCUDA, (c10::DeviceIndex)device));
         ixh_stream_t stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
         const uint16_t *src = static_cast<const uint16_t *>(w->const_data_ptr());
-        scratch = at::empty({(int64_t)bytes}, options.dtype(at::kByte));
-        scale = at::empty({1}, options.dtype(at::kBFloat16));
-        table = at::empty({levels - 1, entries}, options.dtype(at::kInt));
+        scratch = fresh({(int64_t)bytes}, at::kByte, device);
+        scale = fresh({1}, at::kBFloat16, device);
+        table = fresh({levels - 1, entries}, at::kInt, device);
         arrived = at::empty({levels - 1}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-        bitmaps[0] = at::empty({(n + 31) / 32}, options.dtype(at::kInt));
+        bitmaps[0] = fresh({(n + 31) / 32}, at::kInt, device);
         int32_t *ranks = static_cast<int32_t *>(table.data_ptr());
         int64_t *host = static_cast<int64_t *>(arrived.data_ptr());
         rc = library.encode_scan(src, out_f, in_f, levels, p.level_bits, static_cast<uint16_t *>(scale.data_ptr()), ranks,
@@ -442,8 +454,8 @@ PyObject *encode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
             int64_t left = n;
             for (int i = 0; i < levels - 1; ++i) {
                 counts[i] = host[i];
-                if (i > 0) bitmaps[i] = at::empty({(left + 31) / 32}, options.dtype(at::kInt));
-                streams[i] = at::empty({(counts[i] * p.level_bits[i] + 31) / 32}, options.dtype(at::kInt));
+                if (i > 0) bitmaps[i] = fresh({(left + 31) / 32}, at::kInt, device);
+                streams[i] = fresh({(counts[i] * p.level_bits[i] + 31) / 32}, at::kInt, device);
                 p.bitmap_words[i] = (uint64_t)bitmaps[i].numel();
                 p.stream_words[i] = (uint64_t)streams[i].numel();
                 p.bitmaps[i] = bitmaps[i].numel() ? static_cast<const uint32_t *>(bitmaps[i].data_ptr()) : nullptr;
@@ -451,7 +463,7 @@ PyObject *encode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
                 left -= counts[i];
             }
             counts[levels - 1] = left;
-            streams[levels - 1] = at::empty({left}, options.dtype(at::kByte));
+            streams[levels - 1] = fresh({left}, at::kByte, device);
             p.last_bytes = (uint64_t)left;
             p.last = left ? static_cast<const uint8_t *>(streams[levels - 1].data_ptr()) : nullptr;
             p.scale = static_cast<const uint16_t *>(scale.data_ptr());

@@ -252,7 +252,7 @@ class StreamingLinear(nn.Module):
                 ctypes.cast(self._gemv_fn, ctypes.c_void_p).value, ctypes.addressof(self._lanes.struct), self._bias_ptr or 0,
                 self.in_features, self.out_features, dev.index,
                 (0,) + tuple(self._lanes.gemv_workspace_bytes(n) for n in range(1, MAX_FUSED_ROWS + 1)),
-                (self._lanes, self._bias), _workspaces, dev, _lib.check, _plain_call,
+                (self._lanes, self._bias), _workspaces, dev, _lib.check,
                 *(ctypes.cast(f, ctypes.c_void_p).value
                   for f in (_lib.lib().ixh_lanes_gemm, _lib.lib().ixh_lanes_gemm_workspace_bytes)))
             # (what _lanes_gemm_wins allows for a count of rows, it allows for fewer)

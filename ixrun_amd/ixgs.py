@@ -16,6 +16,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _lib
 from .bitpack import pack_bits_stream, unpack_bits_stream
 
 __all__ = ["GROUP_SIZE", "SCALE_DIVISOR", "int8gs_quantize", "decode_weight_scatter", "decode_weight_triton",
@@ -103,8 +104,6 @@ def has_triton() -> bool:
     built HIP library."""
     if not torch.cuda.is_available():
         return False
-    from . import _lib
-
     try:
         _lib.lib()
     except RuntimeError:
@@ -112,22 +111,24 @@ def has_triton() -> bool:
     return True
 
 
-@torch.no_grad()
 def decode_weight_triton(packed: dict, device=None, dtype=torch.bfloat16) -> torch.Tensor:
     """Device decode (``ixgs/kernels.py:121-142``) through ``ixh_decode_gs``.  Needs the GPU and the library;
     there is no fallback inside this function."""
-    from . import _lib
-
-    assert torch.cuda.is_available(), "the device decoder needs the GPU"
-    device = torch.device(device) if device is not None else torch.device("cuda")
-    n = packed["N"]
-    if n and n == packed["out_f"] * packed["in_f"] and device.type == "cuda" and device.index in (None, torch.cuda.current_device()):
+    n, scales = packed["N"], packed["group_scales"]
+    if n and n == packed["out_f"] * packed["in_f"] and scales.is_cuda and (device is None or _lib.is_current(device)):
         # in one native call, where every tensor is on the device already
         w = _lib.host().decode((3, 5, 8), packed["out_f"], packed["in_f"], [packed["b1"], packed["b2"]],
-                               [packed["l1"], packed["l2"], packed["l3"]], None, None, packed["group_scales"],
-                               packed["group_size"])
+                               [packed["l1"], packed["l2"], packed["l3"]], None, None, scales, packed["group_size"])
         if w is not None:
             return w if dtype is torch.bfloat16 else w.to(dtype)
+    return _decode_moved(packed, device, dtype)
+
+
+@torch.no_grad()
+def _decode_moved(packed: dict, device, dtype) -> torch.Tensor:
+    """``decode_weight_triton`` of tensors that are anywhere."""
+    assert torch.cuda.is_available(), "the device decoder needs the GPU"
+    device = torch.device(device) if device is not None else torch.device("cuda")
     mv = lambda t: t.to(device).contiguous()
     dp = _lib.DevicePacked((3, 5, 8), packed["out_f"], packed["in_f"], [mv(packed["b1"]), mv(packed["b2"])],
                            [mv(packed["l1"]), mv(packed["l2"]), mv(packed["l3"])], None)

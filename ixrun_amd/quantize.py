@@ -91,7 +91,6 @@ def int8x_quantize(weight: torch.Tensor, level_bits: tuple = DEFAULT_LEVELS) -> 
     }
 
 
-@torch.no_grad()
 def int8x_quantize_device(weight: torch.Tensor, level_bits: tuple = DEFAULT_LEVELS) -> dict:
     """``int8x_quantize`` for a bf16 weight that lives on the GPU, done by the library's encoder kernels.
 

@@ -44,7 +44,6 @@ def precompute_block_offsets(packed: dict, blk: int = TRITON_BLOCK, device=None)
     return b1, b2
 
 
-@torch.no_grad()
 def decode_weight_triton(packed: dict, device=None, dtype=torch.bfloat16) -> torch.Tensor:
     """Decode a packed dict to a ``[out_f, in_f]`` weight on the GPU.
 
@@ -55,17 +54,22 @@ def decode_weight_triton(packed: dict, device=None, dtype=torch.bfloat16) -> tor
     the CPU decoder to call by name (``Int8XLinear`` does so in a process that has no GPU at all, as the
     reference's does at ``ixrun/linear.py:84-86``).
     """
+    n, scale = packed["N"], packed["scale"]
+    if n and n == packed["out_f"] * packed["in_f"] and scale.is_cuda and (device is None or _lib.is_current(device)):
+        # in one native call, where every tensor is on the device already
+        w = _lib.host().decode(packed["level_bits"], packed["out_f"], packed["in_f"], packed["bitmaps"], packed["streams"],
+                               scale, packed.get("table512"), None, 0)
+        if w is not None:
+            return w if dtype is torch.bfloat16 else w.to(dtype)
     if not torch.cuda.is_available():
         raise RuntimeError("decode_weight_triton runs the HIP kernel and needs the GPU; "
                            "decode_weight_scatter is the CPU decoder")
-    device = torch.device(device) if device is not None else torch.device("cuda")
-    n = packed["N"]
-    if n and n == packed["out_f"] * packed["in_f"] and device.type == "cuda" and device.index in (None, torch.cuda.current_device()):
-        # in one native call, where every tensor is on the device already
-        w = _lib.host().decode(packed["level_bits"], packed["out_f"], packed["in_f"], packed["bitmaps"], packed["streams"],
-                               packed["scale"], packed.get("table512"), None, 0)
-        if w is not None:
-            return w if dtype is torch.bfloat16 else w.to(dtype)
+    return _decode_moved(packed, torch.device(device) if device is not None else torch.device("cuda"), dtype)
+
+
+@torch.no_grad()
+def _decode_moved(packed: dict, device, dtype) -> torch.Tensor:
+    """``decode_weight_triton`` of tensors that are anywhere."""
     dp = _lib.DevicePacked.from_dict(packed, device)
     out = torch.empty(packed["N"], dtype=torch.bfloat16, device=device)
     if packed["N"]:

@@ -227,3 +227,41 @@ def test_two_fused_calls_for_17_to_32_rows(oracle, monkeypatch, rows, buffered, 
             assert calls == [16, rows - 16] and not bool((buf != 9.0).any())
         else:
             assert calls == [] and bool((buf != 9.0).any()) == buffered
+
+
+@pytest.mark.parametrize("rows", [1, 12, 40])
+@pytest.mark.parametrize("lanes_only", [True, False])
+def test_outputs_are_allocated_where_a_mode_sees_it(rows, lanes_only):
+    """A call's own memory goes past the dispatcher in a plain call, and through it under a mode; the results are the same, also in
+    inference mode and with fresh memory filled."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from ixrun_amd.engine import StreamingLinear
+    from ixrun_amd.quantize import int8x_quantize_device
+
+    class Seen(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.ops = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    layer = StreamingLinear(int8x_quantize_device(outlier_weight(768, 1024, seed=3).cuda(), (3, 5, 8)))
+    if not lanes_only:
+        layer._set_shared_buf(torch.empty(768 * 1024, dtype=torch.bfloat16, device="cuda"))
+    x = torch.randn(rows, 1024, device="cuda").bfloat16()
+    with torch.no_grad():
+        y = layer(x)
+        with Seen() as seen:
+            assert torch.equal(layer(x), y)
+    assert any("empty" in op for op in seen.ops)
+    with torch.inference_mode():
+        again = layer(x)
+        assert again.is_inference() and torch.equal(again, y)
+    torch.use_deterministic_algorithms(True, warn_only=True)
+    try:
+        assert torch.equal(layer(x), y)
+    finally:
+        torch.use_deterministic_algorithms(False)
