@@ -557,10 +557,10 @@ int launch_decode_rows358(const Dev &P, const int32_t *prefix, uint16_t *o16, hi
     if (lds > 160 * 1024) return IXH_EUNSUPPORTED;
     const uint32_t flags = ((uintptr_t)P.last & 3u) == 0 ? 1u : 0u;
     if (P.n_levels == 3 && P.bits[1] == 5)
-        hipLaunchKernelGGL(k_decode358_rows<false>, dim3(groups), dim3(kDrWaves * kWave), lds, s, P, prefix, n_quads, quads,
+        IXH_LAUNCH(k_decode358_rows<false>, dim3(groups), dim3(kDrWaves * kWave), lds, s, P, prefix, n_quads, quads,
                            flags, o16);
     else
-        hipLaunchKernelGGL(k_decode358_rows<true>, dim3(groups), dim3(kDrWaves * kWave), lds, s, P, prefix, n_quads, quads,
+        IXH_LAUNCH(k_decode358_rows<true>, dim3(groups), dim3(kDrWaves * kWave), lds, s, P, prefix, n_quads, quads,
                            flags, o16);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }

@@ -1050,10 +1050,10 @@ int launch_decode_dense358(const Dev &P, const int32_t *prefix, uint16_t *o16, G
     }();
     const uint32_t blocks = min(resident, (n_spans + kDnWaves - 1) / kDnWaves);
     if (gs.fp16)
-        hipLaunchKernelGGL(k_decode358_dense<true>, dim3(blocks), dim3(kWave * kDnWaves), 0, s, P, prefix, n_units, n_spans, o16,
+        IXH_LAUNCH(k_decode358_dense<true>, dim3(blocks), dim3(kWave * kDnWaves), 0, s, P, prefix, n_units, n_spans, o16,
                            gs.fp16, (uint32_t)__builtin_ctz(gs.group));
     else
-        hipLaunchKernelGGL(k_decode358_dense<false>, dim3(blocks), dim3(kWave * kDnWaves), 0, s, P, prefix, n_units, n_spans, o16,
+        IXH_LAUNCH(k_decode358_dense<false>, dim3(blocks), dim3(kWave * kDnWaves), 0, s, P, prefix, n_units, n_spans, o16,
                            (const uint16_t *)nullptr, 0u);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
@@ -1062,9 +1062,9 @@ int launch_decode_counted358(const Dev &P, uint16_t *o16, GroupScales gs, hipStr
     const uint32_t n_spans = (P.n + kDnSpan - 1) / kDnSpan, per_wg = (n_spans + 255u) / 256u;
     const dim3 grid((n_spans + per_wg - 1u) / per_wg), block(kWave * kDnCountedWaves);
     if (gs.fp16)
-        hipLaunchKernelGGL(k_decode358_counted<true>, grid, block, 0, s, P, n_spans, per_wg, o16, gs.fp16, (uint32_t)__builtin_ctz(gs.group));
+        IXH_LAUNCH(k_decode358_counted<true>, grid, block, 0, s, P, n_spans, per_wg, o16, gs.fp16, (uint32_t)__builtin_ctz(gs.group));
     else
-        hipLaunchKernelGGL(k_decode358_counted<false>, grid, block, 0, s, P, n_spans, per_wg, o16, (const uint16_t *)nullptr, 0u);
+        IXH_LAUNCH(k_decode358_counted<false>, grid, block, 0, s, P, n_spans, per_wg, o16, (const uint16_t *)nullptr, 0u);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 

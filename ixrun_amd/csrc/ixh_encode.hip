@@ -660,9 +660,9 @@ static void scan_launch(const uint16_t *w, uint32_t n, uint32_t n_units, uint32_
                         uint16_t *scale, int32_t *table, uint32_t *sums, hipStream_t s) {
     const dim3 grid(count_groups(n, group_units)), block(kWave * kEncWaves);
     if (group_units == kCountUnits)
-        hipLaunchKernelGGL((k_enc_count<L, kCountUnits>), grid, block, 0, s, w, n, n_units, parts, lv, table, sums, scale);
+        IXH_LAUNCH((k_enc_count<L, kCountUnits>), grid, block, 0, s, w, n, n_units, parts, lv, table, sums, scale);
     else
-        hipLaunchKernelGGL((k_enc_count<L, kCountFewUnits>), grid, block, 0, s, w, n, n_units, parts, lv, table, sums, scale);
+        IXH_LAUNCH((k_enc_count<L, kCountFewUnits>), grid, block, 0, s, w, n, n_units, parts, lv, table, sums, scale);
 }
 
 int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *bits, uint16_t *scale, int32_t *table,
@@ -675,7 +675,7 @@ int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *b
     EncLevels lv;
     lv.n_levels = n_levels;
     for (int i = 0; i < IXH_MAX_LEVELS; ++i) lv.bits[i] = i < n_levels ? bits[i] : 0;
-    hipLaunchKernelGGL(k_enc_absmax, dim3(kEncParts), dim3(1024), 0, s, w, n, parts);
+    IXH_LAUNCH(k_enc_absmax, dim3(kEncParts), dim3(1024), 0, s, w, n, parts);
     switch (n_levels) {
         case 2: scan_launch<2>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
         case 3: scan_launch<3>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
@@ -685,7 +685,7 @@ int launch_encode_scan(const uint16_t *w, uint32_t n, int n_levels, const int *b
         case 7: scan_launch<7>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
         default: scan_launch<8>(w, n, n_units, group_units, lv, parts, scale, table, sums, s); break;
     }
-    hipLaunchKernelGGL(k_enc_scan, dim3(tiles, n_levels - 1), dim3(1024), 0, s, table, n_units, sums,
+    IXH_LAUNCH(k_enc_scan, dim3(tiles, n_levels - 1), dim3(1024), 0, s, table, n_units, sums,
                        count_groups(n, group_units), group_units, host_totals);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
@@ -701,9 +701,9 @@ static void pack_launch(const uint16_t *w, uint32_t n, uint32_t n_units, const u
     }();
     const uint32_t spans = (n_units + kEncSpanUnits - 1) / kEncSpanUnits, waves = min(spans, at_once);
     const EncShare share{waves, waves ? spans / waves : 0u, waves ? spans % waves : 0u};
-    hipLaunchKernelGGL(k_enc_borders<L>, dim3((share.waves + 256u) / 256u), dim3(256), 0, s, lv, table, n, n_units, share, out);
+    IXH_LAUNCH(k_enc_borders<L>, dim3((share.waves + 256u) / 256u), dim3(256), 0, s, lv, table, n, n_units, share, out);
     if (n_units == 0) return;
-    hipLaunchKernelGGL(k_enc_pack<L>, dim3((share.waves + kEncWaves - 1) / kEncWaves), dim3(kWave * kEncWaves), 0, s, w, n, n_units,
+    IXH_LAUNCH(k_enc_pack<L>, dim3((share.waves + kEncWaves - 1) / kEncWaves), dim3(kWave * kEncWaves), 0, s, w, n, n_units,
                        share, scale, lv, table, out);
 }
 

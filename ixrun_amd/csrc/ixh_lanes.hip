@@ -543,7 +543,7 @@ k_lanes_reduce(const float *__restrict__ ws, uint32_t slices, int m, uint32_t ou
 
 int launch_lanes_reduce(const float *ws, uint32_t slices, int m, uint32_t out_f, uint32_t ws_ld, const uint16_t *bias, bool once,
                         uint16_t *y, int64_t ldy, hipStream_t s) {
-    hipLaunchKernelGGL(k_lanes_reduce, dim3((out_f + 255u) / 256u, m), dim3(256), 0, s, ws, slices, m, out_f, ws_ld, bias, once,
+    IXH_LAUNCH(k_lanes_reduce, dim3((out_f + 255u) / 256u, m), dim3(256), 0, s, ws, slices, m, out_f, ws_ld, bias, once,
                        y, ldy);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
@@ -705,7 +705,7 @@ static int lanes_gemv_few_launch(const LanesDev &L, uint32_t tiles, uint32_t wav
     const bool aligned = ln_whole_pieces((uintptr_t)x, L.in_f, m, ldx);
     const uint32_t shape = L.n_cells | tiles << 8 | (uint32_t)__builtin_ctz(waves) << 16 | (uint32_t)aligned << 19 | (uint32_t)(m - 1) << 20;
     // (a cell / n_cells as a product with 2^16 / n_cells, rounded up: exact for the 32 cells that there are at most)
-    hipLaunchKernelGGL((k_lanes_gemv_few<BITS, MT, N>), dim3((L.n_tiles + tiles - 1u) / tiles), dim3(kWave * waves), lds, s, L.plane, x, L.exc_off,
+    IXH_LAUNCH((k_lanes_gemv_few<BITS, MT, N>), dim3((L.n_tiles + tiles - 1u) / tiles), dim3(kWave * waves), lds, s, L.plane, x, L.exc_off,
                        L.scale, bias, shape, 65536u / L.n_cells + 1u, L.out_f, L.in_f, L.exc_pos, L.exc_val, ldx, y, ldy);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
@@ -749,7 +749,7 @@ static int lanes_gemv_launch(const LanesDev &L, const uint16_t *x, int m, int64_
     // quotients by best_tiles as products with 2^32 / best_tiles, rounded up: exact for the cells of a workgroup, n_cells * best_tiles,
     // while these times best_tiles are below 2^32; each has 16 bytes of LDS
     const uint32_t inv_tiles = best_tiles == 1 ? 0u : (uint32_t)(((1ull << 32) + best_tiles - 1u) / best_tiles);
-    hipLaunchKernelGGL(kernel, dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave << log_waves),
+    IXH_LAUNCH(kernel, dim3((L.n_tiles + best_tiles - 1) / best_tiles), dim3(kWave << log_waves),
                        (lv_lds<BITS, MT, WIDE, BY_WAVE>(L, best_tiles, 1u << log_waves)), s, L.plane, x, L.exc_off, L.scale, shape, L.n_tiles, best_tiles, L.in_f,
                        inv_tiles, L.list_groups, L.exc_pos, L.exc_val, ldx, bias, y, ldy, L.out_f);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;

@@ -363,7 +363,7 @@ static int gemm_launch(const LanesDev &L, const LgPlan &p, const uint16_t *x, in
     if (!raised) return IXH_ELAUNCH;
     const uint32_t blocks = (L.n_tiles + 3u) / 4u;
     const LgSplit c(L.n_cells, p.slices), b(blocks, p.groups);
-    hipLaunchKernelGGL((k_lanes_gemm<BITS, MB, DEPTH>), dim3(p.slices, p.groups, p.m_groups), dim3(kLgBlocks * kWave), lds, s, L.plane, x, L.scale,
+    IXH_LAUNCH((k_lanes_gemm<BITS, MB, DEPTH>), dim3(p.slices, p.groups, p.m_groups), dim3(kLgBlocks * kWave), lds, s, L.plane, x, L.scale,
                        c.share, c.more, b.share, b.more, L.in_f, (uint32_t)ldx, (uint32_t)m, lg_most_at_once(blocks, p.groups), L.n_cells,
                        L.n_tiles, L.exc_off, L.exc_pos, L.exc_val, L.out_f, ws, ((uintptr_t)ws & 15u) == 0, bias, once, y, ldy);
     if (p.slices > 1)

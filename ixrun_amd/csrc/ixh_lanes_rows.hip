@@ -460,7 +460,7 @@ static int rows_launch(const LanesDev &L, const uint16_t *x, int m, int64_t ldx,
     const bool pairs = ((uintptr_t)x & 3u) == 0 && L.in_f % 2u == 0 && ldx % 2 == 0 && ldx < 1ll << 27;
     const uint32_t blocks = (L.n_tiles + 3u) / 4u, log_waves = 31u - (uint32_t)__builtin_clz(p.waves);
     const uint32_t shape = (uint32_t)m | log_waves << 5 | (uint32_t)pairs << 8;
-    hipLaunchKernelGGL((k_lanes_rows<BITS, MT, WIDE>), dim3(p.slices, p.groups), dim3(kWave * p.waves), p.lds, s, L.plane, x, L.exc_off,
+    IXH_LAUNCH((k_lanes_rows<BITS, MT, WIDE>), dim3(p.slices, p.groups), dim3(kWave * p.waves), p.lds, s, L.plane, x, L.exc_off,
                        L.scale, L.n_cells, L.n_tiles, L.in_f, shape, (L.n_cells / p.slices) << 20 | L.n_cells % p.slices,
                        (blocks / p.groups) << 24 | blocks % p.groups, L.exc_pos, L.exc_val, ldx, L.out_f, p.x_rows, ws.at, bias, y, ldy);
     if (p.slices > 1) return launch_lanes_reduce(ws.at, p.slices, m, L.out_f, L.n_tiles * 4u, bias, false, y, ldy, s);
