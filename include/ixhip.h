@@ -144,6 +144,14 @@ int ixh_decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, i
                         ixh_stream_t stream);
 
 /*
+ * The same, and the larger of these tensors have their bitmaps counted by a launch of its own in front: `workspace` of
+ * ixh_decode_unranked_workspace_bytes (0: one launch, no workspace), 4-byte aligned.
+ */
+size_t ixh_decode_unranked_workspace_bytes(const IxhPacked *packed);
+int ixh_decode_unranked_ws(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, uint16_t *out_bf16,
+                           void *workspace, size_t workspace_bytes, ixh_stream_t stream);
+
+/*
  * Fused decode + GEMV / skinny GEMM:
  *   y[m, r] = bf16( sum_k f32(x[m, k]) * f32(bf16(f32(v[r, k]) * f32(scale))) ),
  * fp32 accumulation, m < M <= 16; x is bf16 [M, ldx], y is bf16 [M, ldy].

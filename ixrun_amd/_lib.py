@@ -74,8 +74,8 @@ def host():
         L = lib()
         _host.bind(*(C.cast(f, C.c_void_p).value for f in (
             L.ixh_prefix_entries, L.ixh_prefix_workspace_bytes, L.ixh_prefix_build_ws, L.ixh_decode, L.ixh_decode_gs,
-            L.ixh_decode_unranked_takes, L.ixh_decode_unranked, L.ixh_encode_workspace_bytes, L.ixh_encode_scan_counts,
-            L.ixh_encode_wait, L.ixh_encode_pack)), check)
+            L.ixh_decode_unranked_takes, L.ixh_decode_unranked_workspace_bytes, L.ixh_decode_unranked_ws, L.ixh_encode_workspace_bytes,
+            L.ixh_encode_scan_counts, L.ixh_encode_wait, L.ixh_encode_pack)), check)
         _native = _host
     return _native
 
@@ -102,7 +102,8 @@ EXPORTS = (
     "ixh_prefix_workspace_bytes", "ixh_decode",
     "ixh_gemv", "ixh_gemv_workspace_bytes", "ixh_gemv_noalloc", "ixh_gemm", "ixh_gemm_workspace_bytes",
     "ixh_encode_workspace_bytes", "ixh_encode_scan", "ixh_encode_scan_counts", "ixh_encode_wait", "ixh_encode_pack",
-    "ixh_decode_gs", "ixh_decode_unranked", "ixh_decode_unranked_takes",
+    "ixh_decode_gs", "ixh_decode_unranked", "ixh_decode_unranked_takes", "ixh_decode_unranked_workspace_bytes",
+    "ixh_decode_unranked_ws",
     "ixh_lanes_plane_words", "ixh_lanes_cells", "ixh_lanes_pack", "ixh_lanes_list", "ixh_lanes_gemv",
     "ixh_lanes_gemv_workspace_bytes", "ixh_lanes_gemm", "ixh_lanes_gemm_workspace_bytes",
 )
@@ -138,6 +139,10 @@ def lib() -> C.CDLL:
                                     C.c_void_p]
         L.ixh_decode_unranked.restype = C.c_int
         L.ixh_decode_unranked.argtypes = [C.POINTER(IxhPacked), C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p]
+        L.ixh_decode_unranked_workspace_bytes.restype = C.c_size_t
+        L.ixh_decode_unranked_workspace_bytes.argtypes = [C.POINTER(IxhPacked)]
+        L.ixh_decode_unranked_ws.restype = C.c_int
+        L.ixh_decode_unranked_ws.argtypes = [C.POINTER(IxhPacked), C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]
         L.ixh_decode_unranked_takes.restype = C.c_int
         L.ixh_decode_unranked_takes.argtypes = [C.POINTER(IxhPacked), C.c_void_p, C.c_int64, C.c_void_p]
         L.ixh_gemv.restype = C.c_int

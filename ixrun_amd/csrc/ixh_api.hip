@@ -261,8 +261,8 @@ int ixh_decode_unranked_takes(const IxhPacked *packed, const uint16_t *group_sca
     return packed && !unranked_refuses(*packed, group_scales, group_size, out_bf16);
 }
 
-int ixh_decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, uint16_t *out_bf16,
-                        ixh_stream_t stream) {
+static int decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, uint16_t *out_bf16, uint32_t *runs,
+                           ixh_stream_t stream) {
     Dev d;
     int rc = to_dev(packed, &d, group_scales == nullptr);
     if (rc) return rc;
@@ -274,9 +274,29 @@ int ixh_decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, i
         set_error("decode_unranked: %s", why);
         return IXH_EUNSUPPORTED;
     }
-    rc = launch_decode_counted358(d, out_bf16, gs, (hipStream_t)stream);
+    rc = launch_decode_counted358(d, out_bf16, gs, runs, (hipStream_t)stream);
     if (rc == IXH_ELAUNCH) set_error("decode_unranked: launch failed");
     return rc;
+}
+
+int ixh_decode_unranked(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, uint16_t *out_bf16,
+                        ixh_stream_t stream) {
+    return decode_unranked(packed, group_scales, group_size, out_bf16, nullptr, stream);
+}
+
+size_t ixh_decode_unranked_workspace_bytes(const IxhPacked *packed) {
+    return packed && packed->out_f > 0 && packed->in_f > 0 && packed->out_f <= kDnCountedMost / packed->in_f
+               ? decode_counted358_workspace_bytes((uint64_t)(packed->out_f * packed->in_f)) : 0;
+}
+
+int ixh_decode_unranked_ws(const IxhPacked *packed, const uint16_t *group_scales, int64_t group_size, uint16_t *out_bf16,
+                           void *workspace, size_t workspace_bytes, ixh_stream_t stream) {
+    const size_t need = ixh_decode_unranked_workspace_bytes(packed);
+    if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 3u) != 0)) {
+        set_error("decode_unranked: a 4-byte aligned workspace of %zu bytes needed, %zu given", need, workspace ? workspace_bytes : (size_t)0);
+        return IXH_EWORKSPACE;
+    }
+    return decode_unranked(packed, group_scales, group_size, out_bf16, need ? static_cast<uint32_t *>(workspace) : nullptr, stream);
 }
 
 static int gemv_checks(const Dev &d, int64_t chunk, int32_t m) {

@@ -657,14 +657,14 @@ k_decode358_dense(Dev P, const int32_t *__restrict__ prefix, uint32_t n_units, u
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// The same without a rank table, for tensors of up to 2^22 weights: a workgroup counts the bitmaps in front of its spans itself, at
-// most eight spans, one a wave.  Bound by the latency of its chain (bitmap 0 up to the spans, bitmap 1 up to there, the spans' codes); at
-// 2^22 weights a workgroup reads up to 512 KB of bitmap 0, from the caches, which takes nearly as long as the table's two launches.  The
-// rule ends there, with a span a wave in 256 workgroups; above it neither was timed.  us from a graph, table / without, with group scales: 256 x
-// 512 9.8 / 5.9, 512 x 1024 10.2 / 6.9, 1024 x 1024 10.6 / 7.2, 1400 x 1500 11.4 / 9.0, 2048 x 2048 12.7 / 11.8 to 12.9; of tensors with a
-// scale of their own, almost all in the first level (k_decode358_rows with the table) / at 55 / 40 / 5 %: 256 x 512 10.2 / 6.1 and 10.2 / 6.1, 1024 x
-// 1024 11.3 / 7.4 and 11.3 / 7.4, 1400 x 1500 12.1 / 9.5 and 12.3 / 9.8, 2048 x 2048 14.6 / 12.7 and 14.8 / 13.7; called one by one, where three
-// launches take the host as long, 16 / 8 to 9 up to 1400 x 1500 and 16 / 11.4 to 12.1 at 2048 x 2048.
+// The same without a rank table, for tensors of up to 2^22 weights: a workgroup finds the ranks of its spans, at most eight, one a wave, itself.
+// Bound by the latency of its chain (bitmap 0 up to the spans, bitmap 1 up to there, the spans' codes).  Up to 2^21 weights it counts all that
+// lies in front of them, from the caches, 64 bytes a clock and CU; above (RUNS) a launch in front has counted both bitmaps by runs of 128 words, each
+// in the order of its own bits, so that one does not wait for the other, and a workgroup adds those and counts a run's rest.  The rule ends at 2^22, with a span a wave in 256
+// workgroups; above it neither was timed.  us, from a graph / called one by one, with group scales, in one launch and with RUNS: 1024 x 1024 7.4 / 7.3 and 7.8 /
+// 9.6, 1400 x 1500 9.3 / 9.4 and 8.8 / 9.4, 1600 x 1600 10.3 / 10.3 and 8.9 / 9.0, 1792 x 1792 11.0 / 10.7 and 9.3 / 9.0, 2048 x 2048 13.3 / 12.9 and 9.9 / 9.9; without,
+// 55 / 40 / 5 % 1400 x 1500 9.0 / 8.8 and 8.7 / 9.5, 2048 x 2048 13.4 / 12.8 and 9.5 / 9.5.  From a graph with a table built first, which takes three launches: 256 x
+// 512 9.8, 1024 x 1024 10.6, 2048 x 2048 12.7 with group scales, 14.6 to 14.8 without.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kDnCountedWaves = 16, kDnCountedSpans = 8;
 static_assert(kDnCountedMost == 256u * kDnCountedSpans * kDnSpan, "up to 256 workgroups");
@@ -674,10 +674,22 @@ struct DnOneSpan {
     __device__ __forceinline__ bool first_span(DnSpan &sp) const { sp = span; return true; }
     __device__ __forceinline__ bool next(const DnSpan &, DnSpan &) const { return false; }
 };
-template <bool GS>
+// RUNS: how many bits are set in each run of 128 words of either bitmap is there already (k_count_runs).
+constexpr uint32_t kDnRunWords = 128, kDnRuns = kDnCountedMost / 32u / kDnRunWords;
+static_assert(kDnRuns <= kWave * kDnCountedWaves, "a run a thread");
+__global__ void __launch_bounds__(256)
+k_count_runs(const uint32_t *__restrict__ b1, uint32_t words1, const uint32_t *__restrict__ b2, uint32_t words2, uint32_t *__restrict__ runs) {
+    const uint32_t lane = threadIdx.x & 63u, run = blockIdx.x * 4u + (threadIdx.x >> 6), words = blockIdx.y ? words2 : words1;
+    const __amdgpu_buffer_rsrc_t bitmap = __builtin_amdgcn_make_buffer_rsrc((void *)(blockIdx.y ? b2 : b1), 0, (int)(words * 4u), 0x00020000);
+    const d_u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(bitmap, (int)(run * (kDnRunWords * 4u) + lane * 8u), 0, 0);
+    const uint32_t c = wave_scan_inclusive((uint32_t)(__popc(w[0]) + __popc(w[1])));
+    if (lane == 63u && run < kDnRuns) runs[blockIdx.y * kDnRuns + run] = c;  // (nothing behind a bitmap's end)
+}
+
+template <bool GS, bool RUNS>
 __global__ void __launch_bounds__(kWave *kDnCountedWaves)
 k_decode358_counted(Dev P, uint32_t n_spans, uint32_t spans_per_wg, uint16_t *__restrict__ out,
-                    const uint16_t *__restrict__ group_scales, uint32_t group_shift) {
+                    const uint16_t *__restrict__ group_scales, uint32_t group_shift, const uint32_t *__restrict__ runs) {
     __shared__ __attribute__((aligned(16))) uint32_t lut[kDnLutBytes / 4];
     __shared__ __attribute__((aligned(16))) uint16_t wc_all[kDnCountedSpans][kDnSlots];
     __shared__ uint32_t front[2][kDnCountedWaves], inside[2][kDnCountedWaves];  // bits in front of the workgroup, of a wave's span
@@ -692,8 +704,14 @@ k_decode358_counted(Dev P, uint32_t n_spans, uint32_t spans_per_wg, uint16_t *__
     };
     const __amdgpu_buffer_rsrc_t b1 = rsrc_of(P.bm[0], P.bm_words[0]), b2 = rsrc_of(P.bm[1], P.bm_words[1]);
     // set bits in the first `quads` runs of four words, a thread's part of them
-    auto count = [&](const __amdgpu_buffer_rsrc_t &bitmap, uint32_t quads) {
+    auto count = [&](const __amdgpu_buffer_rsrc_t &bitmap, uint32_t quads, uint32_t level) {
         uint32_t c = 0;
+        if constexpr (RUNS) {  // whole runs, and the quads behind them
+            const uint32_t whole = quads / (kDnRunWords / 4u), q = whole * (kDnRunWords / 4u) + tid;
+            const d_u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(bitmap, (int)(q < quads ? q * 16u : 0x7FFFFFF0u), 0, 0);
+            if (tid < whole) c = runs[level * kDnRuns + tid];
+            return c + __popc(w[0]) + __popc(w[1]) + __popc(w[2]) + __popc(w[3]);
+        }
         for (uint32_t q = tid; q < quads; q += kThreads * kAhead) {
             d_u32x4 w[kAhead];
 #pragma unroll
@@ -714,7 +732,7 @@ k_decode358_counted(Dev P, uint32_t n_spans, uint32_t spans_per_wg, uint16_t *__
     };
 
     uint32_t w1 = 32 * lane < n_el ? __builtin_amdgcn_raw_buffer_load_b32(b1, (int)((p0 >> 5) * 4u + lane * 4u), 0, 0) : 0u;
-    uint32_t c = count(b1, s0 * (kDnSpan / 128u));
+    uint32_t c = count(b1, s0 * (kDnSpan / 128u), 0u);
     const float scale = GS ? 1.0f : bf16_bits_to_f32(*P.scale);
     for (uint32_t e = tid; e < 64 * 32; e += kThreads) {
         const uint32_t idx = e >> 5;
@@ -732,7 +750,7 @@ k_decode358_counted(Dev P, uint32_t n_spans, uint32_t spans_per_wg, uint16_t *__
     uint32_t ahead = s0 * kDnSpan;
 #pragma unroll
     for (uint32_t k = 0; k < kDnCountedWaves; ++k) ahead -= front[0][k];
-    c = count(b2, ahead >> 7);
+    c = count(b2, ahead >> 7, 1u);
     if (tid < 4u) {  // the run of four words that the workgroup's first bit lies in
         const uint32_t word = (ahead >> 7) * 4u + tid, bits = ahead > word * 32u ? min(ahead - word * 32u, 32u) : 0u;
         c += __popc(__builtin_amdgcn_raw_buffer_load_b32(b2, (int)(word * 4u), 0, 0) & (uint32_t)(0xFFFFFFFFull >> (32u - bits)));
@@ -1058,13 +1076,24 @@ int launch_decode_dense358(const Dev &P, const int32_t *prefix, uint16_t *o16, G
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 
-int launch_decode_counted358(const Dev &P, uint16_t *o16, GroupScales gs, hipStream_t s) {
+size_t decode_counted358_workspace_bytes(uint64_t n) { return n > kDnCountedAlone ? 2u * kDnRuns * sizeof(uint32_t) : 0; }
+
+int launch_decode_counted358(const Dev &P, uint16_t *o16, GroupScales gs, uint32_t *runs, hipStream_t s) {
     const uint32_t n_spans = (P.n + kDnSpan - 1) / kDnSpan, per_wg = (n_spans + 255u) / 256u;
     const dim3 grid((n_spans + per_wg - 1u) / per_wg), block(kWave * kDnCountedWaves);
-    if (gs.fp16)
-        IXH_LAUNCH(k_decode358_counted<true>, grid, block, 0, s, P, n_spans, per_wg, o16, gs.fp16, (uint32_t)__builtin_ctz(gs.group));
+    const uint32_t shift = gs.fp16 ? (uint32_t)__builtin_ctz(gs.group) : 0u;
+    if (runs) {
+        const uint32_t words1 = min(P.bm_words[0], kDnCountedMost / 32u), words2 = min(P.bm_words[1], kDnCountedMost / 32u);
+        IXH_LAUNCH(k_count_runs, dim3((P.n / 32u + 4u * kDnRunWords) / (4u * kDnRunWords), 2u), dim3(256), 0, s, P.bm[0], words1, P.bm[1], words2, runs);
+    }
+    if (gs.fp16 && runs)
+        IXH_LAUNCH((k_decode358_counted<true, true>), grid, block, 0, s, P, n_spans, per_wg, o16, gs.fp16, shift, runs);
+    else if (gs.fp16)
+        IXH_LAUNCH((k_decode358_counted<true, false>), grid, block, 0, s, P, n_spans, per_wg, o16, gs.fp16, shift, runs);
+    else if (runs)
+        IXH_LAUNCH((k_decode358_counted<false, true>), grid, block, 0, s, P, n_spans, per_wg, o16, gs.fp16, shift, runs);
     else
-        IXH_LAUNCH(k_decode358_counted<false>, grid, block, 0, s, P, n_spans, per_wg, o16, (const uint16_t *)nullptr, 0u);
+        IXH_LAUNCH((k_decode358_counted<false, false>), grid, block, 0, s, P, n_spans, per_wg, o16, gs.fp16, shift, runs);
     return hipGetLastError() == hipSuccess ? IXH_OK : IXH_ELAUNCH;
 }
 

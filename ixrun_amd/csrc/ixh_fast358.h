@@ -52,7 +52,9 @@ bool decode_dense358_supports(const Dev &P, uint32_t chunk, const int8_t *o8, co
 int launch_decode_dense358(const Dev &P, const int32_t *prefix, uint16_t *o16, GroupScales gs, hipStream_t s);
 // the same without a rank table, up to kDnCountedMost weights
 constexpr uint32_t kDnCountedMost = 1u << 22;
-int launch_decode_counted358(const Dev &P, uint16_t *o16, GroupScales gs, hipStream_t s);
+constexpr uint32_t kDnCountedAlone = 1u << 21;  // in one launch: see k_decode358_counted
+size_t decode_counted358_workspace_bytes(uint64_t n);  // of a launch that counts first, 0 up to kDnCountedAlone
+int launch_decode_counted358(const Dev &P, uint16_t *o16, GroupScales gs, uint32_t *runs, hipStream_t s);  // runs: that, or NULL
 int launch_reduce_chunks(const float *ws, uint32_t n_chunks, int m, uint32_t out_f, uint16_t *y, int64_t ldy,
                          hipStream_t s);
 

@@ -236,7 +236,8 @@ struct Library {
     decltype(&ixh_decode) decode;
     decltype(&ixh_decode_gs) decode_gs;
     decltype(&ixh_decode_unranked_takes) decode_unranked_takes;
-    decltype(&ixh_decode_unranked) decode_unranked;
+    decltype(&ixh_decode_unranked_workspace_bytes) decode_unranked_workspace_bytes;
+    decltype(&ixh_decode_unranked_ws) decode_unranked;
     decltype(&ixh_encode_workspace_bytes) encode_workspace_bytes;
     decltype(&ixh_encode_scan_counts) encode_scan;
     decltype(&ixh_encode_wait) encode_wait;
@@ -257,22 +258,23 @@ bool checked(int rc) {
     return r != nullptr;
 }
 
-// bind(prefix_entries, prefix_workspace_bytes, prefix_build_ws, decode, decode_gs, decode_unranked_takes, decode_unranked,
-// encode_workspace_bytes, encode_scan_counts, encode_wait, encode_pack, check): addresses, and what raises for a negative code
+// bind(prefix_entries, prefix_workspace_bytes, prefix_build_ws, decode, decode_gs, decode_unranked_takes, decode_unranked_workspace_bytes,
+// decode_unranked_ws, encode_workspace_bytes, encode_scan_counts, encode_wait, encode_pack, check): addresses, and what raises for a negative code
 PyObject *bind(PyObject *, PyObject *args) {
-    PyObject *f[11], *check;
-    if (!PyArg_ParseTuple(args, "OOOOOOOOOOOO", &f[0], &f[1], &f[2], &f[3], &f[4], &f[5], &f[6], &f[7], &f[8], &f[9], &f[10], &check)) return nullptr;
+    PyObject *f[12], *check;
+    if (!PyArg_ParseTuple(args, "OOOOOOOOOOOOO", &f[0], &f[1], &f[2], &f[3], &f[4], &f[5], &f[6], &f[7], &f[8], &f[9], &f[10], &f[11], &check)) return nullptr;
     entry(library.prefix_entries, f[0]);
     entry(library.prefix_workspace_bytes, f[1]);
     entry(library.prefix_build, f[2]);
     entry(library.decode, f[3]);
     entry(library.decode_gs, f[4]);
     entry(library.decode_unranked_takes, f[5]);
-    entry(library.decode_unranked, f[6]);
-    entry(library.encode_workspace_bytes, f[7]);
-    entry(library.encode_scan, f[8]);
-    entry(library.encode_wait, f[9]);
-    entry(library.encode_pack, f[10]);
+    entry(library.decode_unranked_workspace_bytes, f[6]);
+    entry(library.decode_unranked, f[7]);
+    entry(library.encode_workspace_bytes, f[8]);
+    entry(library.encode_scan, f[9]);
+    entry(library.encode_wait, f[10]);
+    entry(library.encode_pack, f[11]);
     if (PyErr_Occurred()) return nullptr;
     Py_INCREF(check);
     Py_XSETREF(library.check, check);
@@ -367,7 +369,9 @@ PyObject *decode(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
         const uint16_t *of_groups = scales ? static_cast<const uint16_t *>(scales->const_data_ptr()) : nullptr;
         const bool ranked = given || !library.decode_unranked_takes(&p, of_groups, group, out);
         if (!ranked) {
-            rc = library.decode_unranked(&p, of_groups, group, out, stream);
+            const size_t bytes = library.decode_unranked_workspace_bytes(&p);
+            if (bytes) table = fresh({(int64_t)bytes / 4}, at::kInt, device);
+            rc = library.decode_unranked(&p, of_groups, group, out, bytes ? table.data_ptr() : nullptr, bytes, stream);
         } else if (!given) {
             const size_t bytes = library.prefix_workspace_bytes(n, kUnit, p.n_levels);
             table = fresh({rows * entries + (int64_t)bytes / 4}, at::kInt, device);  // and the scratch

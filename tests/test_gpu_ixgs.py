@@ -133,6 +133,42 @@ def test_per_tensor_decode_without_a_table(oracle, dev, kind, shape):
     assert np.array_equal(bf16_bits(decode_weight_triton(p)).reshape(-1), want)
 
 
+@pytest.mark.parametrize("mix", ["tier1", "tier3", "all"])
+@pytest.mark.parametrize("n", [(1 << 21) + 1, 256 * 5 * 2048 - 31, 256 * 5 * 2048, 256 * 7 * 2048 + 4096 + 33, (1 << 22) - 127, 1 << 22])
+def test_bitmaps_counted_by_a_launch_of_their_own(oracle, dev, n, mix):
+    """Workgroups that begin within a run of counted words and at one; either bitmap whole and next to empty; one launch gives the same."""
+    from ixrun_amd import _lib
+    import ctypes as C
+
+    rng = np.random.default_rng(n)
+    q = {"tier1": rng.integers(-3, 5, size=n), "tier3": rng.choice([-127, -16, 17, 128], size=n), "all": rng.integers(-20, 21, size=n)}[mix].astype(np.int16)
+    q[n // 2] = 9
+    scales = (rng.random(-(-n // 64)).astype(np.float32) * 0.01 + 1e-4).astype(np.float16).view(np.uint16)
+    p = on_device(packed_from_ints(oracle, q, scales, 1, n, 64), dev)
+    dp = _lib.DevicePacked((3, 5, 8), 1, n, [p["b1"], p["b2"]], [p["l1"], p["l2"], p["l3"]], None)
+    need = _lib.lib().ixh_decode_unranked_workspace_bytes(C.byref(dp.struct))
+    assert need > 0
+    out, one = (torch.full((n + 8,), 7.0, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    ws = torch.full((need + 64,), 0xA5, dtype=torch.uint8, device=dev)
+    call = lambda ws_ptr, given: _lib.lib().ixh_decode_unranked_ws(C.byref(dp.struct), p["group_scales"].data_ptr(), 64, out.data_ptr(), ws_ptr, given,
+                                                                   _lib.current_stream(dev))
+    assert call(None, need) == call(ws.data_ptr(), need - 1) == call(ws.data_ptr() + 2, need) == -4
+    for _ in range(2):
+        _lib.check(call(ws.data_ptr(), need))
+    _lib.check(_lib.lib().ixh_decode_unranked(C.byref(dp.struct), p["group_scales"].data_ptr(), 64, one.data_ptr(), _lib.current_stream(dev)))
+    assert np.array_equal(bf16_bits(out)[:n], oracle.gs_dequant_bf16(q, scales, 64)) and bool((out[n:] == 7.0).all())
+    assert torch.equal(out, one) and bool((ws[need:] == 0xA5).all())
+
+
+def test_small_tensors_are_counted_in_one_launch(dev):
+    from ixrun_amd import _lib
+    import ctypes as C
+
+    for out_f, in_f, counted in ((1 << 10, 1 << 11, 0), (1 << 11, 1 << 11, 1), ((1 << 11) + 1, 1 << 11, 0)):
+        s = _lib.IxhPacked(n_levels=3, out_f=out_f, in_f=in_f)
+        assert (_lib.lib().ixh_decode_unranked_workspace_bytes(C.byref(s)) > 0) == bool(counted)
+
+
 @pytest.mark.parametrize("levels,shape", [((3, 4, 5, 6, 8), (33, 1000)), ((3, 5, 8), (2049, 2048))])
 def test_a_decode_that_succeeds_leaves_no_error(oracle, dev, levels, shape):
     """Tensors that need a table are not first refused without one."""
