@@ -199,11 +199,18 @@ class StreamingLinear(nn.Module):
         against 27 / 35 / 37 / 49 / 57, 17408 x 5120 90 / 94 / 94 / 101 / 115 against 42 / 55 / 61 / 75 / 85.  3 bits at 64 / 100 /
         200 / 256: 10240 x 5120 65 / 66 / 70 / 70 against 28 / 35 / 49 / 49, 17408 x 5120 96 / 101 / 111 / 115 against 46 / 53 / 76
         / 77.  8 bits, which have no list, at 64 / 100 / 160: 10240 x 5120 62 / 62 / 71 against 28 / 35 / 45, 17408 x 5120 102 /
-        106 / 116 against 49 / 55 / 68, 4096 x 4096 30 / 31 / 39 against 17 / 23 / 24.  (From 2**24 to 3 * 2**23 weights the lanes
-        win further now than the line has it: at 192 / 256 / 384 / 512 rows 4096 x 4096 (5 bits) 43 / 34 / 37 / 41 against 27 / 30 / 36 / 42,
-        4608 x 5120 (8 bits) 52 / 62 / 49 / 56 against 28 / 31 / 48 / 56, 5120 x 4096 (3 bits) 40 / 47 / 37 / 42 against 29 / 32 / 37 / 47.)  Below 2**24
+        106 / 116 against 49 / 55 / 68, 4096 x 4096 30 / 31 / 39 against 17 / 23 / 24.  From 2**24 to 3 * 2**23 weights the lanes win
+        to 256 rows (at 240 / 256: 6144 x 4096, 5 bits, 41 / 53 against 34 / 35, 5120 x 4608, 3 bits, 39 / 54 against 32 / 35, 8192 x
+        2560, 8 bits, 36 / 44 against 28 / 28, 24576 x 1024, 5 bits, 39 / 38 against 38 / 36; at worst, a tenth of 4 bits listed, 42
+        against 43) and no further: 4096 x 4096, 5 bits, at 384 / 512 rows 37 / 41 against 36 / 42.  Below 2**24
         weights the decode, the GEMM and the host's way through both weigh more: 12000 x 768 at 256 rows 35 against 29, 2048 x 2048
-        23 against 21 (eager: 31 against 20), and up to 2**20 weights 15 against 14 at 512 rows (eager 31 against 13).  Layers of at
+        23 against 21 (eager: 31 against 20).  Up to 2**23 weights that holds to 512 rows where the list is short, a quad of listed
+        elements to 48 weights or fewer (5 % of a layer's), and the rows are not so many and short that the library's product is next
+        to free, at 264 / 512 rows: 2048 x 4096, 4 bits, 35 / 37 against 24 / 30, 1024 x 8192 39 / 39 against 22 / 30, 8192 x 1024,
+        5 bits, 27 / 28 against 22 / 27, 2048 x 1024 15 / 17 against 12 / 15 (eager 31 / 30 against 12 / 14); with a tenth
+        listed 2048 x 2048, 4 bits, 24 / 28 against 22 / 38, and 16384 x 256, 3 bits, 18 / 20 against 21 / 30.  Up to 2**20 weights it
+        holds to 1024 rows whatever the list: at 640 / 1024 1024 x 1024, 5 bits, 15 / 15 against 13 / 14 (eager 32 / 31 against 12 /
+        14), 512 x 2048, 4 bits, a tenth listed, 20 / 21 against 17 / 19; 1024 x 4096, 3 bits, 28 against 30 there.  Layers of at
         most 2**18 weights keep decoding into their buffer (12 us at 100 rows; the lanes took 8), which callers see there.  Rows of
         up to 256 columns: 16384 x 256 at 80 / 100 rows 17 / 17 against 13 / 15 (eager 32 / 31 against 11 / 14).
 
@@ -217,10 +224,10 @@ class StreamingLinear(nn.Module):
         (8 bits) 67 / 85 / 90 against 40 / 53 / 78, 5120 x 17408 (8 bits) 199 / 249 / 217 against 56 / 72 / 105; at 1024 rows
         12288 x 6144 161 against 160 (4 bits) and 165 against 159 (8 bits)."""
         n = self.N
-        return (self._lanes is not None and self._gemv_flags == 0 and self.in_features % 8 == 0 and n > 1 << 18
-                and rows * self.in_features < 1 << 31
-                and (rows <= 160 or (rows <= 224 and self._lanes.bits <= 4) or (rows <= 256 and n < 1 << 24)
-                     or (rows <= 512 and (n <= 1 << 20 or n > 3 << 23)) or (rows <= 1024 and n > 1 << 26)))
+        if self._lanes is None or self._gemv_flags or self.in_features % 8 or n <= 1 << 18 or rows * self.in_features >= 1 << 31:
+            return False
+        light = n <= 1 << 23 and self.out_features <= 8192 and 48 * self._lanes.struct.n_quads <= n
+        return rows <= 256 or (rows <= 512 and (light or n > 3 << 23)) or (rows <= 1024 and (n <= 1 << 20 or n > 1 << 26))
 
     def _bind(self):
         n_levels = len(self.level_bits)
@@ -256,7 +263,7 @@ class StreamingLinear(nn.Module):
                 *(ctypes.cast(f, ctypes.c_void_p).value
                   for f in (_lib.lib().ixh_lanes_gemm, _lib.lib().ixh_lanes_gemm_workspace_bytes)))
             # (what _lanes_gemm_wins allows for a count of rows, it allows for fewer)
-            self._native.many_rows = max((rows for rows in (160, 224, 256, 512, 1024) if self._lanes_gemm_wins(rows)), default=0)
+            self._native.many_rows = max((rows for rows in (256, 512, 1024) if self._lanes_gemm_wins(rows)), default=0)
         self._forget_plans()
 
     def _apply(self, fn, recurse=True):

@@ -621,6 +621,34 @@ def test_prompts_from_native_code(dev, kind):
     assert bool(layer._w_buf.any())
 
 
+@pytest.mark.parametrize("kind,out_f,in_f,most", [
+    ("real", 1020, 1024, 1024), ("listed", 1023, 1024, 1024), ("real", 1030, 1024, 512), ("listed", 1030, 1024, 256), ("rare", 8192, 1024, 512),
+    ("rare", 8193, 520, 256), ("four", 4099, 2048, 256), ("four", 4099, 4096, 256), ("wide", 6001, 4192, 256),
+    ("wide", 6004, 4192, 512)])
+def test_how_many_rows_the_lanes_serve(dev, kind, out_f, in_f, most):
+    """The last prompt that goes to the lanes, on both sides of each bound (weights, listed elements, rows of weights): there and
+    one row further the layer's result is the decoded weight's product, whichever way it goes."""
+    from ixrun_amd.engine import StreamingLinear
+
+    v, scheme, _ = values("four" if kind == "listed" else kind, out_f, in_f)
+    if kind == "listed":
+        v[::11] = 100
+    p = packed_from_int8(v, out_f, in_f, level_bits=scheme)
+    bias = (torch.randn(out_f, generator=torch.Generator().manual_seed(1)) * 0.5).bfloat16()
+    layer = StreamingLinear(p, bias=bias)
+    assert layer._native.many_rows == most
+    wide = activations(most + 1, in_f, seed=4).to(dev)
+    layer._set_shared_buf(torch.zeros(p["N"], dtype=torch.bfloat16, device=dev))
+    weight = layer._decode().float()
+    for rows in (most - 15, most, most + 1):
+        x = wide[:rows]
+        y = layer(x)
+        assert (layer._native.many(x) is not None) == (rows <= most)
+        # one rounding to bf16 of sums whose fp32 errors are far below it, and the same of the general path's
+        assert rel_l2(y.float().cpu().numpy(), (x.float() @ weight.t() + bias.to(dev).float()).bfloat16().float().cpu().numpy()) <= 1e-3
+        assert rel_l2(y.float().cpu().numpy(), layer._decode_and_multiply(x).float().cpu().numpy()) <= 2e-3
+
+
 @pytest.mark.parametrize("kind,out_f,in_f", [("rare", 24600, 1032), ("real", 8200, 3080)])
 def test_large_prompts_of_a_layer(oracle, dev, kind, out_f, in_f):
     """Prompts of a layer large enough for tiles of 128 weight rows, with a bias: from native code, from Python, as views, and
