@@ -279,14 +279,21 @@ __device__ __forceinline__ void wave_lds_sync() {
 //
 // A wave takes spans of four units, 2048 elements, 32 consecutive ones a lane, so one prefix sum over the lanes serves them
 // all and a lane's membership bits are a whole word of bitmap 0.  Every element goes to LDS as one byte, value + 128: those
-// of the level to its dense run, the others to a second one, in order; the next level splits that second run the same
+// of the level to the dense run, the others to what waits for the next level, in order; that level splits its run the same
 // way, 16 bytes a lane.  A dense run starts in LDS where its first code falls in the stream's groups of 32 codes, so a
 // lane turns 32 bytes into `bits` whole words of the stream at once.  Only the groups (and bitmap words) that a wave
 // shares with its neighbours are OR-ed into memory; k_enc_borders clears those beforehand.
 // (Before, a wave packed 512 elements with an LDS atomic per code and a flush per stream: 279 us.)
 // ---------------------------------------------------------------------------------------------------------------
 constexpr uint32_t kEncSpan = 2048, kEncSpanUnits = kEncSpan / kEncUnit;
-constexpr uint32_t kEncBuf = kEncSpan + 256;  // two runs with their margins
+constexpr uint32_t kEncBuf = kEncSpan + 256;  // a dense run, and one behind it, with their margins
+constexpr uint32_t kEncHeld = kEncSpan + 96;  // what waits for its level, with its margins
+// Elements behind the second level are few in a span, and a level's turn (a scan, comparisons, a store) takes as long for 100 as for 1024: from
+// four levels on they wait in LDS, a run a level, until the next would not fit, over the spans of a wave (5120 x 17408, whole calls: levels
+// 3, 4, 5, 6, 8 at 55 / 13 / 27 / 0.7 / 4 % 196 -> 177 us, the launch 108 -> 86; Student-t weights, nearly all in the first, 165 -> 141;
+// four levels 167 -> 161 and 150 -> 132, seven 269 -> 252 and 207 -> 163).  Three levels are bound by memory as much as by issue (139 -> 143
+// and 133 -> 137): there the second has its turn each span.  Eight would leave two waves a SIMD room in LDS (315 -> 354).
+template <int L> constexpr bool kEncHold = L > 3 && L < 8;
 constexpr uint32_t dense_at = 32u;            // where a dense run's groups start in it
 
 // Spans per wave: a wave that goes on hands its unfinished groups to its next span in registers, and only its first and last
@@ -456,49 +463,83 @@ template <int L>
 __global__ void __launch_bounds__(kWave *kEncWaves, L <= 3 ? 5 : 4)
 k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShare share,
            const uint16_t *__restrict__ scale_in, EncLevels lv, const int32_t *__restrict__ table, EncOut out) {
-    __shared__ __attribute__((aligned(32))) uint8_t bufs[kEncWaves][2][kEncBuf];
+    constexpr int kBufs = kEncHold<L> || L < 4 ? L - 2 : 2;  // of elements on their way to the next level
+    __shared__ __attribute__((aligned(32))) uint8_t bufs[kEncWaves][kEncBuf + kBufs * kEncHeld];
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t mine = blockIdx.x * kEncWaves + wave;
     if (mine >= share.waves) return;
     const uint32_t u_first = share.first_unit(mine, n_units), u_end = share.first_unit(mine + 1u, n_units);
+    if (u_first >= u_end) return;
     const EncRanks ranks{table, n_units + 1, n};
     const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
     const float scale = bf16_bits_to_f32(*scale_in), inv_scale = __fdiv_rn(1.0f, scale);
     const float cut0 = bf16_bits_to_f32(enc_cut(lv.bits[0], scale, inv_scale, lane));
-    // r0, space[i]: ranks and bitmap index at the span's start; g_*, w_*: the groups and bitmap words shared with the
-    // neighbouring waves; carry, bm_carry: what the span before left of an unfinished group and bitmap word
-    uint32_t r0[L - 1], g_first[L - 1], g_last[L - 1], carry[L - 1], w_first[L - 1], w_last[L - 1], bm_carry[L - 1];
+    uint8_t *const dense = bufs[wave];
+    // elements that wait for level i, 1 .. L - 2
+    auto held = [&](int i) { return dense + kEncBuf + (kEncHold<L> ? i - 1 : (i - 1) & 1) * kEncHeld; };
+    // r0: codes of the level so far; space, count: what waits for it, index of the first in its bitmap and how many; r1[i][j]: codes of
+    // level j up to where those of level i end (one row, where none waits); g_*, w_*: the groups and bitmap words shared with the
+    // neighbouring waves; carry, bm_carry: what was left of an unfinished group and bitmap word
+    uint32_t r0[L - 1], space[L - 1], count[L - 1], r1[L - 1][L - 1], g_first[L - 1], g_last[L - 1], carry[L - 1], w_first[L - 1], w_last[L - 1],
+        bm_carry[L - 1];
+    bool done[L - 1];  // the level has had all of the wave's elements
 #pragma unroll
     for (int i = 0; i < L - 1; ++i) {
         r0[i] = ranks.rank(i, u_first);
+        space[i] = ranks.space(i, u_first);
+        count[i] = 0u;
         g_first[i] = r0[i] / 32u;
         g_last[i] = ranks.rank(i, u_end) / 32u;
-        w_first[i] = ranks.space(i, u_first) / 32u;
+        w_first[i] = space[i] / 32u;
         w_last[i] = ranks.space(i, u_end) / 32u;
         carry[i] = 128u - (uint32_t)threshold_of(lv.bits[i]);
         bm_carry[i] = 0u;
+        done[i] = false;
+#pragma unroll
+        for (int j = 0; j < L - 1; ++j) r1[i][j] = 0u;
     }
     // a span's weights and the ranks at its end are asked for while the span before is packed
-    uint32_t d[16], r1_next[L - 1];
+    uint32_t d[16], r1_next[L - 1], after;  // (after: the first level's at the end of the span behind that)
     auto ask = [&](uint32_t u) {
         const uint32_t e = u * kEncUnit, to = min(u + kEncSpanUnits, n_units);
         load32(w, e + lane * 32u, n, aligned && (uint64_t)e + kEncSpan <= n, d);
 #pragma unroll
         for (int i = 0; i < L - 1; ++i) r1_next[i] = ranks.rank(i, to);
+        after = kEncHold<L> ? ranks.rank(0, min(to + kEncSpanUnits, n_units)) : 0u;
     };
     ask(u_first);
-    for (uint32_t u0 = u_first; u0 < u_end; u0 += kEncSpanUnits) {
+    // In front of a dense run: the codes of its unfinished group; behind it code 0.  Around what waits for a level: value 0, a member of
+    // every level.
+    auto margins = [&](uint8_t *b, uint32_t first, uint32_t n_run, uint32_t front, uint32_t back) {
+        const uint32_t off = first & 31u;
+        if (lane < 32u) {
+            if (lane < off) b[lane] = (uint8_t)front;
+            b[off + n_run + lane] = (uint8_t)back;
+        }
+    };
+    // a level's dense run of n_i codes to its stream, the unfinished group kept or, at the wave's end, stored
+    auto store_level = [&](int i, uint32_t n_i, bool final) {
+        const uint32_t to = r0[i] + n_i, whole = to / 32u - r0[i] / 32u;
+        enc_store_run_of((uint32_t)lv.bits[i], dense + dense_at, r0[i] / 32u, final ? (to + 31u) / 32u - r0[i] / 32u : whole,
+                         g_first[i], g_last[i], out.st[i], out.st_words[i], lane);
+        carry[i] = dense[dense_at + whole * 32u + (lane & 31u)];
+        r0[i] = to;
+    };
+    // the last level: one byte, value + 127, per element left over (quantize.py:84-86)
+    auto store_last = [&](const uint8_t *run, uint32_t first, uint32_t n_run) {
+        for (uint32_t k = lane; k < n_run; k += kWave)
+            if (first + k < out.last_bytes) out.last[first + k] = (uint8_t)(max((int)run[k], 1) - 1);
+    };
+    uint32_t u0 = u_first;
+    for (;;) {
+        // ---- a span: quantise ----
         const uint32_t u1 = min(u0 + kEncSpanUnits, n_units);
         const bool final = u1 == u_end;
         const uint32_t e0 = u0 * kEncUnit, e1 = min(e0 + kEncSpan, n);
-        uint32_t r1[L - 1];
-#pragma unroll
-        for (int i = 0; i < L - 1; ++i) r1[i] = r1_next[i];
-        uint32_t left = e1 - e0;  // (the counts below come from the caller's table: held to the span)
-
-        // ---- quantise ----
         const uint32_t p = e0 + lane * 32u;
+        // (counts come from the caller's table: held to what there is)
+        const uint32_t n_0 = min(r1_next[0] - r0[0], e1 - e0), left = e1 - e0 - n_0, then = after;
         uint32_t member = 0;
         float v[32];
 #pragma unroll
@@ -510,20 +551,18 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
         member = __brev(member);  // bit t: element t is in the first level
         if (p < e1 && p / 32u < out.bm_words[0]) out.bm[0][p / 32u] = member;
 
-        // ---- first level: codes to the dense run in buffer 0, the rest behind it (what lies past the last element
-        // follows them and is overwritten by the margin) ----
-        uint8_t *buf = bufs[wave][0], *other = bufs[wave][1];
+        // ---- first level: codes to the dense run, the rest to what waits for the second or, in two levels, behind it (what lies past the
+        // last element follows them and is overwritten by the margin) ----
         const uint32_t cnt = (uint32_t)__popc(member);
         const uint32_t before = wave_scan_inclusive(cnt) - cnt;
-        uint32_t n_i = min(r1[0] - r0[0], left);
-        r1[0] = r0[0] + n_i;
-        left -= n_i;
-        uint32_t rest = ((dense_at + 31u + (r0[0] & 31u) + n_i) & ~31u) + 32u;  // the other run's start
-        uint32_t space0 = e0 - r0[0], space1 = space0 + left;                   // its elements' indexes in the next bitmap
+        const uint32_t next = e0 - r0[0];
+        constexpr int k = L > 2 ? 1 : 0;
+        if (!kEncHold<L> && k > 0) space[k] = next, count[k] = 0u;
+        uint8_t *const rest = k > 0 ? held(k) + (space[k] & 31u) + count[k] : dense + ((dense_at + 31u + (r0[0] & 31u) + n_0) & ~31u) + 32u;
         {
             const uint32_t low = (uint32_t)__popc(member & 0xffffu);
-            const uint32_t to1 = lds_address(buf) + dense_at + (r0[0] & 31u) + before;
-            const uint32_t to0 = lds_address(buf) + rest + (space0 & 31u) + lane * 32u - before;
+            const uint32_t to1 = lds_address(dense) + dense_at + (r0[0] & 31u) + before;
+            const uint32_t to0 = lds_address(rest) + lane * 32u - before;
             EncPut put{to1 | (to1 + low) << 16, to0 | (to0 + 16u - low) << 16, ~member};
             // 1.5 * 2^23 rounds half to even and leaves the integer in the low bits; the 3072 comes off with the same sum, which is
             // exact up to its rounding
@@ -531,111 +570,122 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
 #pragma unroll
             for (int t = 0; t < 16; ++t) put.two(t, byte(t), byte(16 + t));
         }
-        // In front of a dense run: the codes of its unfinished group; behind it code 0.  Around the other run: value 0, a
-        // member of every level.
-        auto margins = [&](uint8_t *b, uint32_t at, uint32_t first, uint32_t count, uint32_t front, uint32_t back) {
-            const uint32_t off = first & 31u;
-            if (lane < 32u) {
-                if (lane < off) b[at + lane] = (uint8_t)front;
-                b[at + off + count + lane] = (uint8_t)back;
-            }
-        };
-        // a level's run to its stream, the unfinished group kept for the next span or, at the wave's end, stored
-        auto store_level = [&](int i, const uint8_t *b) {
-            const uint32_t whole = r1[i] / 32u - r0[i] / 32u;
-            enc_store_run_of((uint32_t)lv.bits[i], b + dense_at, r0[i] / 32u, final ? (r1[i] + 31u) / 32u - r0[i] / 32u : whole,
-                             g_first[i], g_last[i], out.st[i], out.st_words[i], lane);
-            carry[i] = b[dense_at + whole * 32u + (lane & 31u)];
-        };
-        if (!final) ask(u1);
-        margins(buf, dense_at, r0[0], n_i, carry[0], 128u - (uint32_t)threshold_of(lv.bits[0]));
-        margins(buf, rest, space0, left, 128u, 128u);
-        wave_lds_sync();
-        store_level(0, buf);
-
-        // ---- the other levels, 16 elements a lane and turn; margin elements pass as members in front of the first and
-        // behind the last code, where the run's own margins overwrite them ----
+        if constexpr (L > 2) {
+            // (by a true table there are no more than a span: so a level that has had its turn has room for any other's)
+            count[1] = kEncHold<L> ? min(count[1] + left, kEncSpan) : left;
 #pragma unroll
-        for (int i = 1; i < L - 1; ++i) {
-            if (space1 == space0 && !final) {  // nothing came this far: what is unfinished stays so
-                r1[i] = r0[i];
-                continue;
-            }
-            const uint32_t off = space0 & 31u, end = off + (space1 - space0);
-            const uint32_t thr = (uint32_t)threshold_of(lv.bits[i]);
-            n_i = min(r1[i] - r0[i], left);
-            r1[i] = r0[i] + n_i;
-            left -= n_i;
-            const uint32_t rest_i = ((dense_at + 31u + (r0[i] & 31u) + n_i) & ~31u) + 32u;
-            const uint32_t next0 = space0 - r0[i], next1 = next0 + left;
-            uint32_t base1 = dense_at + (r0[i] & 31u) - off, base0 = rest_i + (next0 & 31u);
-            uint32_t unfinished = 0;
-            for (uint32_t s = 0; s < end; s += 1024u) {
-                const uint32_t at = s + 16u * lane;
-                uint32_t bits = 0, n_here = 0, x[4] = {0, 0, 0, 0}, m[4] = {0, 0, 0, 0};
-                if (at < end) {
-                    const uint4 q = *reinterpret_cast<const uint4 *>(buf + rest + at);
-                    x[0] = q.x; x[1] = q.y; x[2] = q.z; x[3] = q.w;
-                    n_here = 16u;
-                    // four bytes at a time: bit 7 of m set where 128 - threshold <= byte <= 128 + threshold
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const uint32_t low = x[k] & 0x7f7f7f7fu;
-                        m[k] = ((low + thr * 0x01010101u) | x[k]) & ~((low + (127u - thr) * 0x01010101u) & x[k]) & 0x80808080u;
-                    }
-                    bits = (__builtin_amdgcn_udot4(m[1], 0x80402010u, __builtin_amdgcn_udot4(m[0], 0x08040201u, 0u, false), false) >> 7) |
-                           (__builtin_amdgcn_udot4(m[3], 0x80402010u, __builtin_amdgcn_udot4(m[2], 0x08040201u, 0u, false), false) >> 7 << 8);
-                }
-                const uint32_t c1 = (uint32_t)__popc(bits), c0 = n_here - c1;
-                const uint32_t incl = wave_scan_inclusive(c1 | (c0 << 16));
-                if (at < end) {
-                    const uint32_t low = (uint32_t)__popc(bits & 0xffu);
-                    uint32_t to1 = lds_address(other) + base1 + (incl & 0xffffu) - c1, to0 = lds_address(other) + base0 + (incl >> 16) - c0;
-                    EncPut put{to1 | (to1 + low) << 16, to0 | (to0 + 8u - low) << 16, ~((bits & 0xffu) | bits >> 8 << 16)};
-#pragma unroll
-                    for (int t = 0; t < 8; ++t)
-                        put.two(t, (uint8_t)(x[t / 4] >> (8 * (t & 3))), (uint8_t)(x[2 + t / 4] >> (8 * (t & 3))));
-                }
-                const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-                base1 += total & 0xffffu;
-                base0 += total >> 16;
-                // bitmap i: the bits of this lane's elements that are the span's, two lanes to a word
-                uint32_t mine = at < end ? bits : 0u;
-                if (at < off) mine &= off - at < 16u ? ~0u << (off - at) : 0u;
-                if (at + 16u > end) mine &= at < end ? (1u << (end - at)) - 1u : 0u;
-                uint32_t word = (mine & 0xffffu) | ((uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0xB1, 0xf, 0xf, true) << 16);
-                if (at == 0) word |= bm_carry[i];
-                const uint32_t wi = space0 / 32u + (at >> 5);
-                const bool last_word = at >= (end & ~31u);
-                if ((end & ~31u) - s < 1024u)
-                    unfinished = (uint32_t)__builtin_amdgcn_readlane((int)word, (int)(((end & ~31u) - s) >> 4));
-                if ((lane & 1u) == 0 && at < end && wi < out.bm_words[i] && (final || !last_word)) {
-                    if (wi == w_first[i] || wi == w_last[i]) {
-                        if (word) atomicOr(&out.bm[i][wi], word);
-                    } else {
-                        out.bm[i][wi] = word;
-                    }
-                }
-            }
-            bm_carry[i] = unfinished;
-            margins(other, dense_at, r0[i], n_i, carry[i], 128u - (uint32_t)threshold_of(lv.bits[i]));
-            margins(other, rest_i, next0, left, 128u, 128u);
-            wave_lds_sync();
-            store_level(i, other);
-            uint8_t *const swap = buf;
-            buf = other;
-            other = swap;
-            rest = rest_i;
-            space0 = next0;
-            space1 = next1;
+            for (int j = 1; j < L - 1; ++j) r1[1][j] = r1_next[j];
         }
-        // ---- last level: one byte, value + 127, per element left over (quantize.py:84-86) ----
-        for (uint32_t k = lane; k < space1 - space0; k += kWave)
-            if (space0 + k < out.last_bytes)
-                out.last[space0 + k] = (uint8_t)(max((int)buf[rest + (space0 & 31u) + k], 1) - 1);
-#pragma unroll
-        for (int i = 0; i < L - 1; ++i) r0[i] = r1[i];
+        if (!final) ask(u1);
+        margins(dense + dense_at, r0[0], n_0, carry[0], 128u - (uint32_t)threshold_of(lv.bits[0]));
+        if (L > 2 && !kEncHold<L>) margins(held(1), space[k], count[k], 128u, 128u);
         wave_lds_sync();
+        store_level(0, n_0, final);
+        if constexpr (L == 2) store_last(rest, next, left);
+        done[0] = final;
+        wave_lds_sync();
+
+        // ---- the levels behind the first: one has its turn where it has no room for what comes next, and at the wave's end; the next one
+        // before it where that has none for what it will pass on ----
+        for (bool again = true; again;) {
+            again = false;
+            bool now = false;
+            if constexpr (kEncHold<L>) now = !final && count[1] > min(then - r0[0], kEncSpan);  // + (kEncSpan - those of the first level) > kEncSpan
+            else if constexpr (L > 2) now = count[1] != 0u;
+            if (!now && !final) break;  // (past all of it, which lies behind the span's code: an only span's wave runs straight on)
+            // 16 elements a lane and turn; margin elements pass as members in front of the first and behind the last code, where the run's own
+            // margins overwrite them
+#pragma unroll
+            for (int i = 1; i < L - 1; ++i) {
+                const bool all = kEncHold<L> ? done[i - 1] : final, turn = kEncHold<L> ? now || (all && !done[i]) : all || count[i] != 0u;
+                now = false;
+                if (!turn) continue;
+                const uint32_t n_i = min(r1[kEncHold<L> ? i : 1][i] - r0[i], count[i]), left = count[i] - n_i;
+                if (kEncHold<L> && i < L - 2 && count[i < L - 2 ? i + 1 : i] + left > kEncSpan) {
+                    now = again = true;
+                    continue;
+                }
+                const uint32_t off = space[i] & 31u, end = off + count[i];
+                const uint32_t thr = (uint32_t)threshold_of(lv.bits[i]);
+                const uint32_t next = space[i] - r0[i];  // index of the first element that goes on
+                const int k = i < L - 2 ? i + 1 : i;       // the level it goes to
+                if (!kEncHold<L> && k > i) space[k] = next, count[k] = 0u;  // (as they are: but not kept in registers)
+                uint8_t *const from = held(i);
+                uint8_t *const rest = k > i ? held(k) + (space[k] & 31u) + count[k]
+                                            : dense + ((dense_at + 31u + (r0[i] & 31u) + n_i) & ~31u) + 32u;
+                if (kEncHold<L>) {
+                    margins(from, space[i], count[i], 128u, 128u);
+                    wave_lds_sync();
+                }
+                uint32_t base1 = dense_at + (r0[i] & 31u) - off, base0 = 0;
+                uint32_t unfinished = 0;
+                for (uint32_t s = 0; s < end; s += 1024u) {
+                    const uint32_t at = s + 16u * lane;
+                    uint32_t bits = 0, n_here = 0, x[4] = {0, 0, 0, 0}, m[4] = {0, 0, 0, 0};
+                    if (at < end) {
+                        const uint4 q = *reinterpret_cast<const uint4 *>(from + at);
+                        x[0] = q.x; x[1] = q.y; x[2] = q.z; x[3] = q.w;
+                        n_here = 16u;
+                        // four bytes at a time: bit 7 of m set where 128 - threshold <= byte <= 128 + threshold
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const uint32_t low = x[k] & 0x7f7f7f7fu;
+                            m[k] = ((low + thr * 0x01010101u) | x[k]) & ~((low + (127u - thr) * 0x01010101u) & x[k]) & 0x80808080u;
+                        }
+                        bits = (__builtin_amdgcn_udot4(m[1], 0x80402010u, __builtin_amdgcn_udot4(m[0], 0x08040201u, 0u, false), false) >> 7) |
+                               (__builtin_amdgcn_udot4(m[3], 0x80402010u, __builtin_amdgcn_udot4(m[2], 0x08040201u, 0u, false), false) >> 7 << 8);
+                    }
+                    const uint32_t c1 = (uint32_t)__popc(bits), c0 = n_here - c1;
+                    const uint32_t incl = wave_scan_inclusive(c1 | (c0 << 16));
+                    if (at < end) {
+                        const uint32_t low = (uint32_t)__popc(bits & 0xffu);
+                        uint32_t to1 = lds_address(dense) + base1 + (incl & 0xffffu) - c1, to0 = lds_address(rest) + base0 + (incl >> 16) - c0;
+                        EncPut put{to1 | (to1 + low) << 16, to0 | (to0 + 8u - low) << 16, ~((bits & 0xffu) | bits >> 8 << 16)};
+#pragma unroll
+                        for (int t = 0; t < 8; ++t)
+                            put.two(t, (uint8_t)(x[t / 4] >> (8 * (t & 3))), (uint8_t)(x[2 + t / 4] >> (8 * (t & 3))));
+                    }
+                    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+                    base1 += total & 0xffffu;
+                    base0 += total >> 16;
+                    // bitmap i: the bits of this lane's elements that are the wave's, two lanes to a word
+                    uint32_t mine = at < end ? bits : 0u;
+                    if (at < off) mine &= off - at < 16u ? ~0u << (off - at) : 0u;
+                    if (at + 16u > end) mine &= at < end ? (1u << (end - at)) - 1u : 0u;
+                    uint32_t word = (mine & 0xffffu) | ((uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0xB1, 0xf, 0xf, true) << 16);
+                    if (at == 0) word |= bm_carry[i];
+                    const uint32_t wi = space[i] / 32u + (at >> 5);
+                    const bool last_word = at >= (end & ~31u);
+                    if ((end & ~31u) - s < 1024u)
+                        unfinished = (uint32_t)__builtin_amdgcn_readlane((int)word, (int)(((end & ~31u) - s) >> 4));
+                    if ((lane & 1u) == 0 && at < end && wi < out.bm_words[i] && (all || !last_word)) {
+                        if (wi == w_first[i] || wi == w_last[i]) {
+                            if (word) atomicOr(&out.bm[i][wi], word);
+                        } else {
+                            out.bm[i][wi] = word;
+                        }
+                    }
+                }
+                bm_carry[i] = unfinished;
+                if (k > i) {
+                    count[k] += left;
+#pragma unroll
+                    for (int j = k; j < L - 1; ++j)
+                        if (kEncHold<L>) r1[k][j] = r1[i][j];
+                    if (!kEncHold<L>) margins(held(k), space[k], count[k], 128u, 128u);
+                }
+                margins(dense + dense_at, r0[i], n_i, carry[i], 128u - thr);
+                wave_lds_sync();
+                store_level(i, n_i, all);
+                if (k == i) store_last(rest, next, left);
+                space[i] += count[i];
+                count[i] = 0u;
+                if (kEncHold<L>) done[i] = all;
+                wave_lds_sync();
+            }
+        }
+        if (final) break;
+        u0 = u1;
     }
 }
 

@@ -202,6 +202,24 @@ def test_encode_waves_of_more_than_a_span(oracle, dev, level_bits, waves, spans,
     check_against_oracle(oracle, dev, make_weight("calibrated_odd_scale", 1, n), level_bits)
 
 
+@pytest.mark.parametrize("level_bits,waves", [((3, 5, 8), 20), ((3, 4, 6, 8), 20), ((3, 4, 5, 6, 8), 16), ((2, 3, 4, 5, 6, 7, 8), 12),
+                                              ((1, 2, 3, 4, 5, 6, 7, 8), 20)])
+def test_encode_elements_that_wait_for_their_level(oracle, dev, level_bits, waves):
+    """Waves of five and six spans whose elements go to the levels by turns: spans of one level, of two, of all, so that what waits for a
+    level is nothing, a few, as much as fits or more than the next has room for."""
+    n = 5 * waves * torch.cuda.get_device_properties(dev).multi_processor_count * 2048 + 4099
+    rng = np.random.default_rng(len(level_bits))
+    top = np.array([0] + [(1 << (b - 1)) - 1 for b in level_bits])
+    spans = n // 2048 + 1
+    low, high = rng.integers(0, len(level_bits), size=(2, spans))
+    low, high = np.where(rng.random(spans) < 0.2, 0, np.minimum(low, high)), np.maximum(low, high)
+    level = (low[:, None] + rng.integers(0, 1 << 16, size=(spans, 2048), dtype=np.uint16) % (high - low + 1)[:, None]).reshape(-1)[:n]
+    size = top[level] + 1 + rng.integers(0, 1 << 16, size=n, dtype=np.uint16) % (top[level + 1] - top[level]).clip(1)
+    v = np.where(rng.integers(0, 2, size=n, dtype=np.int8) == 1, size, -size).clip(-127, 127)
+    v[n // 2] = 127
+    check_against_oracle(oracle, dev, torch.from_numpy(v.astype(np.float32) * 2.0 ** -9).bfloat16().reshape(1, n), level_bits)
+
+
 @pytest.mark.parametrize("n,top", [(3 * 8192 + 5, 8191), (3 * 8192 + 5, 3 * 8192 - 1), (3 * 8192 + 5, 3 * 8192 + 4), (16 * 512, 16 * 512 - 1),
                                    (16 * 512 + 1, 16 * 512), (32768 * 512, 32768 * 512 - 1), (32768 * 512 + 1, 32768 * 512)])
 def test_encode_counts_by_groups_of_either_size(oracle, dev, n, top):
