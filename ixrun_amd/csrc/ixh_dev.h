@@ -18,20 +18,33 @@ constexpr int kWave = 64;
 // A launch of a kernel whose arguments are laid out here, as the kernel's argument block has them: 2.5 us of host time for 17 arguments where
 // hipLaunchKernelGGL, which hands over each by itself and looks the kernel up, takes 2.75 (calls that the host bounds, GGL / so: one row of 512 x 512 6.79 /
 // 6.60 us, two launches of 1024 x 1024 at 40 rows 10.55 / 10.20, the five of an encode of 448 x 1024 37.2 / 35.0).
+// The function is that of the current device, and a stream may be another's: then, and where a look-up fails, the launch is by symbol, which the
+// runtime resolves for the stream (its error is taken back: the caller asks for the launch's).
 struct LaunchHandle {
     static constexpr int kDevices = 16;
     std::atomic<hipFunction_t> of[kDevices]{};
-    hipFunction_t get(const void *kernel) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || dev >= kDevices) return nullptr;
-        hipFunction_t f = of[dev].load(std::memory_order_acquire);
-        if (!f && hipGetFuncBySymbol(&f, kernel) == hipSuccess) of[dev].store(f, std::memory_order_release);
-        return f;
+    hipFunction_t get(const void *kernel, hipStream_t s) {
+        int dev = 0, at = 0;
+        const bool own = s && s != hipStreamLegacy && s != hipStreamPerThread;  // (those are the current device's)
+        hipError_t e = hipGetDevice(&dev);
+        if (e == hipSuccess && own) e = hipStreamGetDevice(s, &at);
+        if (e == hipSuccess) {
+            if ((own && at != dev) || dev >= kDevices) return nullptr;
+            hipFunction_t f = of[dev].load(std::memory_order_acquire);
+            if (f) return f;
+            e = hipGetFuncBySymbol(&f, kernel);
+            if (e == hipSuccess) {
+                of[dev].store(f, std::memory_order_release);
+                return f;
+            }
+        }
+        (void)hipGetLastError();
+        return nullptr;
     }
 };
 template <class... P>
 inline void launch_packed(LaunchHandle &handle, void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t s, std::common_type_t<P>... args) {
-    const hipFunction_t f = handle.get(reinterpret_cast<const void *>(kernel));
+    const hipFunction_t f = handle.get(reinterpret_cast<const void *>(kernel), s);
     if (!f) {
         hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);
         return;
