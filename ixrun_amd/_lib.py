@@ -479,7 +479,8 @@ class LanePacked:
             first = cls(dp.out_f, dp.in_f, (plane, exc_off, none, none.to(torch.int8)), dp.tensors[-1])
             check(L.ixh_lanes_pack(w.data_ptr(), C.byref(first.struct), quads.data_ptr(), stream))
             torch.cumsum(quads, 0, dtype=torch.int32, out=exc_off[1:])
-            n_quads = max(int(exc_off[-1]), 1)
+            listed_quads = int(exc_off[-1])
+            n_quads = max(listed_quads, 1)
             if into is not None and into.bits == first.bits and n_quads <= into.struct.n_quads:
                 whole = into
                 for kept, t in zip(whole.tensors, (plane, exc_off)):
@@ -493,6 +494,7 @@ class LanePacked:
                 whole = cls(dp.out_f, dp.in_f, (plane, exc_off, torch.empty(4 * n_quads, dtype=torch.int16, device=dev),
                                                 torch.zeros(4 * n_quads, dtype=torch.int8, device=dev)), dp.tensors[-1])
             check(L.ixh_lanes_list(w.data_ptr(), C.byref(whole.struct), stream))
+        whole.listed_quads = listed_quads  # (struct.n_quads: what the list has memory for)
         return whole
 
     def gemv_workspace_bytes(self, m: int) -> int:

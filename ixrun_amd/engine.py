@@ -175,6 +175,7 @@ class StreamingLinear(nn.Module):
             self._bind()
             return
         lanes = _lib.LanePacked.build(self._dp, *self._decode_table(), self.counts)
+        self._listed_quads = lanes.listed_quads
         for name, t in zip(LANE_BUFFERS, lanes.tensors):
             self.register_buffer(name, t, persistent=False)
         self._bind()
@@ -204,8 +205,8 @@ class StreamingLinear(nn.Module):
         2560, 8 bits, 36 / 44 against 28 / 28, 24576 x 1024, 5 bits, 39 / 38 against 38 / 36; at worst, a tenth of 4 bits listed, 42
         against 43) and no further: 4096 x 4096, 5 bits, at 384 / 512 rows 37 / 41 against 36 / 42.  Below 2**24
         weights the decode, the GEMM and the host's way through both weigh more: 12000 x 768 at 256 rows 35 against 29, 2048 x 2048
-        23 against 21 (eager: 31 against 20).  Up to 2**23 weights that holds to 512 rows where the list is short, a quad of listed
-        elements to 48 weights or fewer (5 % of a layer's), and the rows are not so many and short that the library's product is next
+        23 against 21 (eager: 31 against 20).  Up to 2**23 weights that holds to 512 rows where the list is short, one quad of listed
+        elements or fewer to 50 weights (5 % of a layer's), and the rows are not so many and short that the library's product is next
         to free, at 264 / 512 rows: 2048 x 4096, 4 bits, 35 / 37 against 24 / 30, 1024 x 8192 39 / 39 against 22 / 30, 8192 x 1024,
         5 bits, 27 / 28 against 22 / 27, 2048 x 1024 15 / 17 against 12 / 15 (eager 31 / 30 against 12 / 14); with a tenth
         listed 2048 x 2048, 4 bits, 24 / 28 against 22 / 38, and 16384 x 256, 3 bits, 18 / 20 against 21 / 30.  Up to 2**20 weights it
@@ -226,7 +227,7 @@ class StreamingLinear(nn.Module):
         n = self.N
         if self._lanes is None or self._gemv_flags or self.in_features % 8 or n <= 1 << 18 or rows * self.in_features >= 1 << 31:
             return False
-        light = n <= 1 << 23 and self.out_features <= 8192 and 48 * self._lanes.struct.n_quads <= n
+        light = n <= 1 << 23 and self.out_features <= 8192 and 50 * self._listed_quads <= n
         return rows <= 256 or (rows <= 512 and (light or n > 3 << 23)) or (rows <= 1024 and (n <= 1 << 20 or n > 1 << 26))
 
     def _bind(self):
@@ -262,8 +263,6 @@ class StreamingLinear(nn.Module):
                 (self._lanes, self._bias), _workspaces, dev, _lib.check,
                 *(ctypes.cast(f, ctypes.c_void_p).value
                   for f in (_lib.lib().ixh_lanes_gemm, _lib.lib().ixh_lanes_gemm_workspace_bytes)))
-            # (what _lanes_gemm_wins allows for a count of rows, it allows for fewer)
-            self._native.many_rows = max((rows for rows in (256, 512, 1024) if self._lanes_gemm_wins(rows)), default=0)
         self._forget_plans()
 
     def _apply(self, fn, recurse=True):
@@ -308,11 +307,14 @@ class StreamingLinear(nn.Module):
         streams.  Where the new list does not fit into the old one's memory the layout is replaced as a whole and the old one
         stays alive: such a graph goes on serving the old weights and has to be captured again."""
         lanes = _lib.LanePacked.build(self._dp, *self._decode_table(), self.counts, into=self._lanes)
+        self._listed_quads = lanes.listed_quads
         if lanes is not self._lanes:
             self._replaced_lanes.append(self._lanes)
             for name, t in zip(LANE_BUFFERS, lanes.tensors):
                 setattr(self, name, t)
             self._bind()
+        else:
+            self._forget_plans()
 
     def _set_shared_buf(self, w_buf):
         self._w_buf = w_buf
@@ -320,8 +322,10 @@ class StreamingLinear(nn.Module):
 
     def _forget_plans(self):
         self._plans = {}
-        if self._native is not None:  # rows up to which calls that are not plain go to the lanes too: see _fused_plan
-            self._native.any_rows = self._packed_rows()
+        if self._native is not None:
+            self._native.any_rows = self._packed_rows()  # rows up to which calls that are not plain go to the lanes too: see _fused_plan
+            # (what _lanes_gemm_wins allows for a count of rows, it allows for fewer)
+            self._native.many_rows = max((rows for rows in (256, 512, 1024) if self._lanes_gemm_wins(rows)), default=0)
 
     def _decode_table(self):
         """The rank table and unit of a decode of the whole weight."""

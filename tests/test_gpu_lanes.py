@@ -649,6 +649,37 @@ def test_how_many_rows_the_lanes_serve(dev, kind, out_f, in_f, most):
         assert rel_l2(y.float().cpu().numpy(), layer._decode_and_multiply(x).float().cpu().numpy()) <= 2e-3
 
 
+@pytest.mark.parametrize("first", ["short", "long"])
+def test_prompts_go_by_the_list_that_is_loaded(dev, first):
+    """Which prompts the lanes serve follows from the elements listed now, not from the memory that an earlier list of the layer left: a
+    layer that has loaded a state goes the way of a new one of it."""
+    from ixrun_amd.engine import StreamingLinear
+
+    out_f, in_f, listed = 2048, 1024, 43
+    lists = {}
+    for kind in ("short", "long"):  # equal level counts: the elements of a quad's four rows, or four times as many of one of them
+        v = values("four", out_f, in_f)[0].reshape(out_f, in_f)
+        v[v == 100] = 6
+        if kind == "short":
+            v[:, : 16 * listed : 16] = 100
+        else:
+            v[::4, : 16 * listed : 4] = 100
+        lists[kind] = packed_from_int8(v.reshape(-1), out_f, in_f, level_bits=(4, 8))
+    assert lists["short"]["counts"] == lists["long"]["counts"]
+    fresh = {kind: StreamingLinear(p) for kind, p in lists.items()}
+    layer = StreamingLinear(lists[first])
+    buf = torch.zeros(out_f * in_f, dtype=torch.bfloat16, device=dev)
+    for each in (layer, *fresh.values()):
+        each._set_shared_buf(buf)
+    x = activations(512, in_f, seed=3).to(dev)
+    for kind in ("long", "short", "long", "short", "short"):
+        layer.load_state_dict(fresh[kind].state_dict())
+        assert layer._native.many_rows == fresh[kind]._native.many_rows == {"short": 512, "long": 256}[kind]
+        for rows in (256, 257, 512):
+            assert layer._lanes_gemm_wins(rows) == fresh[kind]._lanes_gemm_wins(rows) == (rows <= layer._native.many_rows)
+            assert torch.equal(layer(x[:rows]), fresh[kind](x[:rows]))
+
+
 @pytest.mark.parametrize("kind,out_f,in_f", [("rare", 24600, 1032), ("real", 8200, 3080)])
 def test_large_prompts_of_a_layer(oracle, dev, kind, out_f, in_f):
     """Prompts of a layer large enough for tiles of 128 weight rows, with a bias: from native code, from Python, as views, and
