@@ -9,7 +9,8 @@
  *   - every pointer inside IxhPacked and every buffer argument is a DEVICE
  *     pointer owned by the caller; the library never allocates, frees, copies
  *     to the host or synchronises, so every call may be stream-captured;
- *   - all work is enqueued on the given stream (0 = the null stream);
+ *   - all work is enqueued on the given stream (0 = the null stream, which is
+ *     the current device's: the tensors' device has to be current then);
  *   - return value: IXH_OK (0) or a negative IXH_E* code; ixh_last_error()
  *     gives the calling thread's last message.  Nothing throws or aborts;
  *   - lengths of every stream are passed and respected: no kernel reads past

@@ -5,7 +5,7 @@
 // allocated through the dispatcher, plain calls found out in Python and the decoders' and the encoder's Python under a no_grad of its own / now: 1536 x
 // 1536, one row 7.0 / 6.8 us; 1024 x 1024 at 40 rows 11.4 / 10.5; decode of 1408 x 672 9.3 / 6.5, with group scales of 640 x 1024 9.6 / 7.2; encode of
 // 448 x 1024 39.3 / 36.2, of 2048 x 2500 40.0 / 37.3.)  Everything that is not the common case (other types,
-// other devices, views, a scratch that has to grow, errors) is left to the caller: a function returns None and has done
+// other devices than the current one, views, a scratch that has to grow, errors) is left to the caller: a function returns None and has done
 // nothing, and the Python code behind it goes on.
 #include <Python.h>
 #include <structmember.h>
@@ -77,7 +77,7 @@ PyObject *forward_call(PyObject *self_, PyObject *const *args, size_t nargsf, Py
         Py_RETURN_NONE;
     const at::Tensor &x = THPVariable_Unpack(args[0]);
     if (!x.is_cuda() || x.scalar_type() != at::kBFloat16 || x.dim() < 1 || x.size(-1) != self->in_f || x.get_device() != self->device ||
-        !x.is_contiguous())
+        !x.is_contiguous() || c10::hip::current_device() != self->device)
         Py_RETURN_NONE;
     const int64_t rows = x.numel() / self->in_f;
     if (rows < 1 || rows > kMaxRows) Py_RETURN_NONE;

@@ -265,3 +265,47 @@ def test_outputs_are_allocated_where_a_mode_sees_it(rows, lanes_only):
         assert torch.equal(layer(x), y)
     finally:
         torch.use_deterministic_algorithms(False)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 40, 600])
+@pytest.mark.parametrize("lanes", [True, False])
+def test_a_forward_runs_with_its_device_current(monkeypatch, rows, lanes):
+    """The null stream is the current device's: a call of a layer whose device is not current makes it so for the launches.  (One GPU: what
+    the layer asks for the current device says another one until the layer's is entered.)"""
+    from ixrun_amd import _lib, engine
+    from ixrun_amd.quantize import int8x_quantize_device
+
+    layer = engine.StreamingLinear(int8x_quantize_device(outlier_weight(768, 1024, seed=3).cuda(), (3, 5, 8)), lanes=lanes)
+    layer._set_shared_buf(torch.empty(768 * 1024, dtype=torch.bfloat16, device="cuda"))
+    layer._native = None  # (which asks the runtime itself, and leaves such calls to Python)
+    x = torch.randn(rows, 1024, device="cuda").bfloat16()
+    want = layer(x)
+    entered, launches = [], []
+
+    class Device:
+        def __init__(self, device):
+            self.device = torch.device(device)
+
+        def __enter__(self):
+            entered.append(self.device.index)
+
+        def __exit__(self, *exc):
+            entered.pop()
+
+    class Lib:
+        def __getattr__(self, name):
+            if "bytes" not in name and "entries" not in name:
+                launches.append(list(entered))
+            return getattr(_lib._lib, name)
+
+    def gemv(*args, fn=layer._gemv_fn):
+        launches.append(list(entered))
+        return fn(*args)
+
+    layer._gemv_fn = gemv
+    monkeypatch.setattr(_lib, "lib", Lib)
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(engine, "_current_device", lambda: entered[-1] if entered else x.get_device() + 1, raising=False)
+    y = layer(x)
+    assert torch.equal(y, want) and launches and not entered
+    assert all(at and at[0] == x.get_device() for at in launches)
