@@ -7,6 +7,7 @@ loading or the call raises.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import os
 
@@ -225,6 +226,18 @@ def current_stream(device) -> C.c_void_p:
     return C.c_void_p(_raw_stream(device.index if device.index is not None else torch.cuda.current_device()))
 
 
+try:
+    _current_device = torch._C._cuda_getDevice
+except AttributeError:  # a CPU-only torch build
+    _current_device = torch.cuda.current_device
+_nothing = contextlib.nullcontext()
+
+
+def on_device(device):
+    """For the launches of a call: the null stream is the current device's, so that a tensor's device has to be current."""
+    return _nothing if device.index in (None, _current_device()) else torch.cuda.device(device)
+
+
 def _require_cuda(t: torch.Tensor, what: str) -> None:
     if not t.is_cuda:
         raise RuntimeError(f"{what} must live on the GPU (got {t.device}); the HIP path has no CPU fallback")
@@ -293,8 +306,9 @@ class DevicePacked:
         table = torch.empty((len(self.level_bits) - 1, entries), dtype=torch.int32, device=self.device)
         ws = torch.empty(lib().ixh_prefix_workspace_bytes(self.N, int(chunk), len(self.level_bits)), dtype=torch.uint8,
                          device=self.device)
-        check(lib().ixh_prefix_build_ws(C.byref(self.struct), int(chunk), table.data_ptr(), ws.data_ptr(), ws.numel(),
-                                        current_stream(self.device)))
+        with on_device(self.device):
+            check(lib().ixh_prefix_build_ws(C.byref(self.struct), int(chunk), table.data_ptr(), ws.data_ptr(), ws.numel(),
+                                            current_stream(self.device)))
         return table
 
     def decode(self, table: torch.Tensor, chunk: int, out_i8=None, out_bf16=None) -> None:
@@ -303,10 +317,11 @@ class DevicePacked:
                 _require_cuda(t, "decode output")
                 if t.dtype != dt or t.numel() < self.N:
                     raise ValueError(f"decode output must be {dt} with at least {self.N} elements")
-        check(lib().ixh_decode(
-            C.byref(self.struct), table.data_ptr(), int(chunk),
-            out_i8.data_ptr() if out_i8 is not None else None,
-            out_bf16.data_ptr() if out_bf16 is not None else None, current_stream(self.device)))
+        with on_device(self.device):
+            check(lib().ixh_decode(
+                C.byref(self.struct), table.data_ptr(), int(chunk),
+                out_i8.data_ptr() if out_i8 is not None else None,
+                out_bf16.data_ptr() if out_bf16 is not None else None, current_stream(self.device)))
 
     def decode_gs(self, table: torch.Tensor, chunk: int, group_scales: torch.Tensor, group_size: int,
                   out_bf16: torch.Tensor) -> None:
@@ -318,8 +333,9 @@ class DevicePacked:
             raise ValueError(f"group_scales must be fp16 with at least {n_groups} elements")
         if out_bf16.dtype != torch.bfloat16 or out_bf16.numel() < self.N:
             raise ValueError(f"decode output must be bf16 with at least {self.N} elements")
-        check(lib().ixh_decode_gs(C.byref(self.struct), table.data_ptr(), int(chunk), group_scales.data_ptr(),
-                                  int(group_size), out_bf16.data_ptr(), current_stream(self.device)))
+        with on_device(self.device):
+            check(lib().ixh_decode_gs(C.byref(self.struct), table.data_ptr(), int(chunk), group_scales.data_ptr(),
+                                      int(group_size), out_bf16.data_ptr(), current_stream(self.device)))
 
     def gemv_workspace_bytes(self, chunk: int, m: int, flags: int = 0) -> int:
         return int(lib().ixh_gemv_workspace_bytes(C.byref(self.struct), int(chunk), int(m), int(flags)))
@@ -369,13 +385,14 @@ class DevicePacked:
     def gemv(self, table, chunk, x, y=None, y32=None, workspace=None, flags=0) -> None:
         """x bf16 [M, in_f] (row stride x.stride(0)); y bf16 [M, out_f] or y32 fp32 (atomic mode)."""
         x2, m, ldx, ldy = self._gemv_operands(table, chunk, x, y, y32, workspace)
-        check(lib().ixh_gemv(
-            C.byref(self.struct), table.data_ptr(), int(chunk), x2.data_ptr(), m, ldx,
-            y.data_ptr() if y is not None else None, ldy,
-            y32.data_ptr() if y32 is not None else None,
-            workspace.data_ptr() if workspace is not None else None,
-            workspace.numel() * workspace.element_size() if workspace is not None else 0,
-            int(flags), current_stream(self.device)))
+        with on_device(self.device):
+            check(lib().ixh_gemv(
+                C.byref(self.struct), table.data_ptr(), int(chunk), x2.data_ptr(), m, ldx,
+                y.data_ptr() if y is not None else None, ldy,
+                y32.data_ptr() if y32 is not None else None,
+                workspace.data_ptr() if workspace is not None else None,
+                workspace.numel() * workspace.element_size() if workspace is not None else 0,
+                int(flags), current_stream(self.device)))
 
     def gemv_noalloc(self, table, chunk, x, y, flags=0) -> None:
         """``gemv`` through the entry point that allocates nothing: partial sums go to the library's own buffer
@@ -404,12 +421,13 @@ class DevicePacked:
             raise ValueError("x and y rows must be contiguous")
         m = x2.shape[0]
         y2 = y.reshape(m, self.out_f)
-        check(lib().ixh_gemm(
-            C.byref(self.struct), table512.data_ptr(), x2.data_ptr(), m,
-            x2.stride(0) if m > 1 else self.in_f, y2.data_ptr(), y2.stride(0) if m > 1 else self.out_f,
-            workspace.data_ptr() if workspace is not None else None,
-            workspace.numel() * workspace.element_size() if workspace is not None else 0,
-            current_stream(self.device)))
+        with on_device(self.device):
+            check(lib().ixh_gemm(
+                C.byref(self.struct), table512.data_ptr(), x2.data_ptr(), m,
+                x2.stride(0) if m > 1 else self.in_f, y2.data_ptr(), y2.stride(0) if m > 1 else self.out_f,
+                workspace.data_ptr() if workspace is not None else None,
+                workspace.numel() * workspace.element_size() if workspace is not None else 0,
+                current_stream(self.device)))
 
 
 LANE_BITS = (3, 4, 5, 8)

@@ -309,3 +309,51 @@ def test_a_forward_runs_with_its_device_current(monkeypatch, rows, lanes):
     y = layer(x)
     assert torch.equal(y, want) and launches and not entered
     assert all(at and at[0] == x.get_device() for at in launches)
+
+
+def test_packed_tensors_calls_run_with_their_device_current(monkeypatch):
+    """Tables, decodes and products called on a packed tensor itself, whose device is not the current one (as above)."""
+    from ixrun_amd import _lib
+    from ixrun_amd.quantize import int8x_quantize_device
+
+    packed = int8x_quantize_device(outlier_weight(512, 1024, seed=3).cuda(), (3, 5, 8))
+    dp, n = packed["device_packed"], 512 * 1024
+    x = torch.randn(32, 1024, device="cuda").bfloat16()
+    scales = torch.full((n // 64,), 0.01, dtype=torch.float16, device="cuda")
+    entered, launches = [], []
+
+    class Device:
+        def __init__(self, device):
+            self.device = torch.device(device)
+
+        def __enter__(self):
+            entered.append(self.device.index)
+
+        def __exit__(self, *exc):
+            entered.pop()
+
+    class Lib:
+        def __getattr__(self, name):
+            if "bytes" not in name and "entries" not in name:
+                launches.append(list(entered))
+            return getattr(_lib._lib, name)
+
+    def calls():
+        table = dp.prefix_build(512)
+        w, v, g = (torch.empty(n, dtype=t, device="cuda") for t in (torch.bfloat16, torch.int8, torch.bfloat16))
+        y, ym = (torch.empty(rows, 512, dtype=torch.bfloat16, device="cuda") for rows in (4, 32))
+        ws = torch.empty(max(dp.gemv_workspace_bytes(512, 4), dp.gemm_workspace_bytes(32), 4), dtype=torch.uint8, device="cuda")
+        dp.decode(table, 512, out_bf16=w)
+        dp.decode(table, 512, out_i8=v)
+        dp.decode_gs(table, 512, scales, 64, g)
+        dp.gemv(table, 512, x[:4], y=y, workspace=ws)
+        dp.gemv_noalloc(table, 512, x[:4], y)
+        dp.gemm(table, x, ym, ws)
+        return table, w, v, g, y, ym
+
+    want = calls()
+    monkeypatch.setattr(_lib, "lib", Lib)
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(_lib, "_current_device", lambda: entered[-1] if entered else x.get_device() + 1, raising=False)
+    assert all(torch.equal(a, b) for a, b in zip(calls(), want))
+    assert len(launches) == 7 and not entered and all(at and at[0] == x.get_device() for at in launches)
