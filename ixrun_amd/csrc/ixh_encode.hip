@@ -465,6 +465,7 @@ k_enc_pack(const uint16_t *__restrict__ w, uint32_t n, uint32_t n_units, EncShar
            const uint16_t *__restrict__ scale_in, EncLevels lv, const int32_t *__restrict__ table, EncOut out) {
     constexpr int kBufs = kEncHold<L> || L < 4 ? L - 2 : 2;  // of elements on their way to the next level
     __shared__ __attribute__((aligned(32))) uint8_t bufs[kEncWaves][kEncBuf + kBufs * kEncHeld];
+    static_assert(sizeof bufs <= 1u << 16, "EncPut holds LDS addresses in the halves of a word");
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t mine = blockIdx.x * kEncWaves + wave;
