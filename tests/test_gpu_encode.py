@@ -220,6 +220,10 @@ def test_encode_elements_that_wait_for_their_level(oracle, dev, level_bits, wave
     check_against_oracle(oracle, dev, torch.from_numpy(v.astype(np.float32) * 2.0 ** -9).bfloat16().reshape(1, n), level_bits)
 
 
+def test_encode_elements_that_wait_for_their_level_of_six(oracle, dev):
+    test_encode_elements_that_wait_for_their_level(oracle, dev, (3, 4, 5, 6, 7, 8), 12)
+
+
 @pytest.mark.parametrize("n,top", [(3 * 8192 + 5, 8191), (3 * 8192 + 5, 3 * 8192 - 1), (3 * 8192 + 5, 3 * 8192 + 4), (16 * 512, 16 * 512 - 1),
                                    (16 * 512 + 1, 16 * 512), (32768 * 512, 32768 * 512 - 1), (32768 * 512 + 1, 32768 * 512)])
 def test_encode_counts_by_groups_of_either_size(oracle, dev, n, top):
