@@ -288,9 +288,10 @@ __device__ __forceinline__ void wave_lds_sync() {
 constexpr uint32_t kEncSpan = 2048, kEncSpanUnits = kEncSpan / kEncUnit;
 constexpr uint32_t kEncBuf = kEncSpan + 256;  // a dense run, and one behind it, with their margins
 constexpr uint32_t kEncHeld = kEncSpan + 96;  // what waits for its level, with its margins
-// Elements behind the second level are few in a span, and a level's turn (a scan, comparisons, a store) takes as long for 100 as for 1024: from
-// four levels on they wait in LDS, a run a level, until the next would not fit, over the spans of a wave (5120 x 17408, whole calls: levels
-// 3, 4, 5, 6, 8 at 55 / 13 / 27 / 0.7 / 4 % 196 -> 177 us, the launch 108 -> 86; Student-t weights, nearly all in the first, 165 -> 141;
+// A level's turn (a scan, comparisons, a store) takes as long for 100 elements as for 1024.  From four levels on what is not of the first waits in
+// LDS for the second level, and so on to the last but one, a run a level, over the spans of a wave until what comes next would not fit: of levels 3,
+// 4, 5, 6, 8 at 55 / 13 / 27 / 0.7 / 4 % a span leaves 920 elements to the second, 660 to the third, 96 to the fourth, so that these have their turns every other
+// span, every third and once in twenty (5120 x 17408, whole calls: 196 -> 177 us, the launch 108 -> 86; Student-t weights, nearly all in the first, 165 -> 141;
 // four levels 167 -> 161 and 150 -> 132, seven 269 -> 252 and 207 -> 163).  Three levels are bound by memory as much as by issue (139 -> 143
 // and 133 -> 137): there the second has its turn each span.  Eight would leave two waves a SIMD room in LDS (315 -> 354).
 template <int L> constexpr bool kEncHold = L > 3 && L < 8;

@@ -391,8 +391,9 @@ static LrPlan lr_plan(const LanesDev &L) {
 // The larger pair table up to eight rows (LDS has the room beside their activations) and from some cells a CU on: below, what it
 // saves is less than its 64 KB take to write (5 bits, 8 rows, larger / smaller: 512 x 512 5.9 / 5.2 us, 2000 x 2048 with 8 cells a CU
 // 6.9 / 6.6, 4000 x 3072 with 24 8.9 / 8.6, 2000 x 8192 with 32 11.1 / 11.8, 5000 x 5120 with 50 12.7 / 12.8).  At 4 bits,
-// where it is 16 KB, up to sixteen rows (smaller / larger at 16: 17408 x 5120 24.0 / 21.9, 5120 x 17408 24.2 / 22.2, 10240 x 5120 18.4 / 16.9,
-// 5120 x 5120 with 50 cells a CU 14.1 / 13.3, 4096 x 4096 with 32 10.6 / 10.6, 8192 x 1024 with 16 7.3 / 7.3, 1024 x 1024 6.7 / 6.8).
+// where it is 16 KB, up to sixteen rows (smaller / larger at 16, 1.5 % of the weights listed: 17408 x 5120 22.6 / 20.4, 5120 x 17408 22.6 / 19.8,
+// 10240 x 5120 17.1 / 15.9, 5120 x 5120 with 50 cells a CU 13.9 / 13.1; 5 % listed 26.5 / 24.7, 26.7 / 24.1, 20.0 / 18.9, 15.5 / 14.8; 4096 x 4096 with
+// 32 10.6 / 10.6, 8192 x 1024 with 16 7.3 / 7.3, 1024 x 1024 6.7 / 6.8.  lr_plan's costs were fitted without this form.)
 template <int BITS> static bool lr_wide(const LanesDev &L, int m) {
     const uint64_t cells = (uint64_t)L.n_tiles * L.n_cells;
     return m <= 8 ? (BITS == 4 || BITS == 5) && cells > 24u * ln_cus() : BITS == 4 && cells > 32u * ln_cus();
@@ -414,15 +415,17 @@ static LrPlan lr_plan_of(const LanesDev &L, int m) {
 // Nine to sixteen rows: turning the activations round for the whole of a long slice, or starting up for a single cell, takes longer than
 // k_lanes_gemm's way, whose sixteen waves share a copy of 128 columns a stage, up to 20 * 2^20 weights, and of long rows from 25 * 2^20 to
 // 46 at 5 bits and 38 at 8; not of tall layers, of which a workgroup here has one slice.  us, this / that at 16 rows (nine and twelve
-// are within 4 % of that):
+// are within 4 % of that where nothing else is said):
 //   5 bits   1024 x 1024 7.2 / 7.6, 2048 x 2048 8.8 / 8.7, 2560 x 2560 10.6 / 9.2, 2048 x 4096 10.4 / 9.7, 4096 x 2048 9.1 / 9.8, 1536 x 6144
 //            12.6 / 10.2, 4096 x 4096 12.0 / 11.6, 4096 x 5120 13.9 / 12.9, 3072 x 8192 15.5 / 14.0, 4096 x 6144 14.2 / 14.8, 5120 x 5120 15.8 /
 //            15.0, 4096 x 8192 15.9 / 16.0, 6144 x 6144 18.4 / 17.8, 6656 x 6656 20.9 / 19.0, 9216 x 5120 21.1 / 19.1, 4096 x 12288 20.1 / 20.8
 //   8 bits   2048 x 2048 7.1 / 7.4, 2048 x 4096 9.0 / 8.3, 1536 x 6144 10.4 / 8.8, 4096 x 4096 9.7 / 10.0, 4096 x 5120 11.1 / 10.8, 4096 x 6144
 //            11.7 / 11.9, 5120 x 5120 13.3 / 12.4, 2880 x 9536 13.4 / 13.1, 4096 x 8192 14.5 / 14.3, 6144 x 6144 15.5 / 15.6, 8192 x 5120 16.1 /
 //            16.5, 6656 x 6656 18.4 / 16.5, 4096 x 11008 16.7 / 17.3, 2560 x 17408 16.2 / 17.2
-//   4 bits   2048 x 2048 7.9 / 7.9, 2560 x 2560 9.0 / 8.6, 1536 x 6144 11.0 / 9.5, 4096 x 4096 10.2 / 10.8, 5120 x 5120 13.3 / 14.1, 6144 x 6144
-//            14.6 / 16.4, 4096 x 11008 15.4 / 18.2
+//   4 bits   (1.5 % listed) 2048 x 2048 7.8 / 7.3, 2560 x 2560 9.2 / 8.0, 1536 x 6144 10.7 / 8.6, 4096 x 4096 10.4 / 9.4, 4096 x 5120 11.3 / 11.2,
+//            3072 x 8192 12.4 / 11.8, 4096 x 6144 11.4 / 12.4, 5120 x 5120 12.7 / 12.6, 6144 x 6144 13.4 / 14.4, 4096 x 11008 14.3 / 16.1, 10240 x
+//            5120 15.2 / 17.4; with 5 % listed 9 to 18 % more either way, the same side ahead; at nine rows 5120 x 5120 12.7 / 11.5, 3072 x 8192 12.2 /
+//            10.8.  (Between 20 and 25 * 2^20 that way would be ahead where rows are long.)
 //   3 bits   (whose pairs sit in LDS 32 times over here) 2048 x 2048 7.6 / 7.5, 2560 x 2560 8.5 / 8.4, 2048 x 4096 9.1 / 8.4, 4096 x 2048 7.7 / 8.5,
 //            1536 x 6144 10.5 / 9.1, 2048 x 8192 10.1 / 9.9, 4096 x 4096 9.8 / 9.9, 4096 x 5120 10.9 / 11.3, 4096 x 6144 11.2 / 12.7
 static bool lr_gemm_wins(const LanesDev &L, int m) {

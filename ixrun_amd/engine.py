@@ -2,7 +2,7 @@
 
 ``StreamingLinear`` keeps a layer's packed streams resident on the GPU and
 serves every forward from them: up to 16 activation rows go through the fused
-decode+GEMV kernel (the bf16 weight never reaches memory), prompts of up to 160
+decode+GEMV kernel (the bf16 weight never reaches memory), prompts of up to 256
 to 1024 rows through a fused decode+GEMM, larger ones are decoded into a shared
 bf16 buffer and multiplied with ``F.linear``.
 ``GraphLinear`` / ``Int8XEngine`` follow the reference's ``ixrun/engine.py``
