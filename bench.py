@@ -50,55 +50,55 @@ _ENCODE = ("ixh_encode.hip", "ixh_dev.h")
 _OLD = ((), "measured-on-earlier-sources")  # figures kept for the record; reported as null
 MEASURED_TRAFFIC_BYTES = {
     # k_lanes_gemv; eight rows k_lanes_rows, sixteen with k_lanes_reduce
-    "down_proj_5120x17408_m1_student_t": (18527.8 * 2.0 * 1024 + 16.0 * 1024, _LANES, "58f0e28d2101b827"),
-    "down_proj_5120x17408_m1_calibrated": (40731.7 * 2.0 * 1024 + 16.0 * 1024, _LANES, "58f0e28d2101b827"),
-    "down_proj_5120x17408_m1_five_level_calibrated": (40731.9 * 2.0 * 1024 + 16.0 * 1024, _LANES, "58f0e28d2101b827"),
-    "gate_up_17408x5120_m8_calibrated": (36775.9 * 2.0 * 1024 + 272.0 * 1024, _LANES, "58f0e28d2101b827"),
-    "down_proj_5120x17408_m16_student_t": ((19440.6 + 974.0) * 2.0 * 1024 + (1920.0 + 160.0) * 1024, _LANES, "58f0e28d2101b827"),
+    "down_proj_5120x17408_m1_student_t": (18521.0 * 2.0 * 1024 + 16.0 * 1024, _LANES, "e5dd4cabcbebf53f"),
+    "down_proj_5120x17408_m1_calibrated": (40732.0 * 2.0 * 1024 + 16.0 * 1024, _LANES, "e5dd4cabcbebf53f"),
+    "down_proj_5120x17408_m1_five_level_calibrated": (40731.8 * 2.0 * 1024 + 16.0 * 1024, _LANES, "e5dd4cabcbebf53f"),
+    "gate_up_17408x5120_m8_calibrated": (36774.0 * 2.0 * 1024 + 272.0 * 1024, _LANES, "e5dd4cabcbebf53f"),
+    "down_proj_5120x17408_m16_student_t": ((19440.5 + 974.0) * 2.0 * 1024 + (1920.0 + 160.0) * 1024, _LANES, "e5dd4cabcbebf53f"),
     # k_lanes_xtile, k_lanes_prompt and k_lanes_prompt_reduce
-    "prefill_5120x17408_m512_five_level": ((8715.8 + 57947.2 + 30739.5) * 2.0 * 1024 + (17408.0 + 66720.0 + 5122.4) * 1024,
-                                           _LANES, "58f0e28d2101b827"),
-    "down_proj_5120x17408_m1_student_t_packed": (23031.8 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "1fdd69999d604da2"),
-    "gate_up_17408x5120_m1_student_t_packed": (22935.7 * 2.0 * 1024 + 40.0 * 1024, _ROWS, "1fdd69999d604da2"),
-    "attn_proj_5120x5120_m1_student_t_packed": (7135.4 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "1fdd69999d604da2"),
-    "down_proj_5120x17408_m1_calibrated_packed": (33837.4 * 2.0 * 1024 + 40.0 * 1024, _DENSE, "e61b807eff8d0496"),
-    "down_proj_5120x17408_m1_five_level_calibrated_packed": (49695.3 * 2.0 * 1024 + 1327.4 * 1024, _DENSE5, "c90fda40702b4752"),
-    "gate_up_17408x5120_m4_student_t_packed": (28711.3 * 2.0 * 1024 + 160.0 * 1024, _TILES, "3bdb0448e558c413"),
-    "gate_up_17408x5120_m16_student_t_packed": (26660.4 * 2.0 * 1024 + 640.0 * 1024, _TILES, "3bdb0448e558c413"),
-    "attn_proj_5120x5120_m16_student_t_packed": (8657.2 * 2.0 * 1024 + 640.0 * 1024, _TILES, "3bdb0448e558c413"),
-    "down_proj_5120x17408_m16_student_t_packed": (27677.1 * 2.0 * 1024 + 960.0 * 1024, _TILES, "3bdb0448e558c413"),
-    "decode_5120x17408_calibrated": (37277.2 * 2.0 * 1024 + 174080.0 * 1024, _DENSE, "e61b807eff8d0496"),
-    "decode_5120x17408_five_level_calibrated": (49530.0 * 2.0 * 1024 + 174080.0 * 1024, _DENSE5, "c90fda40702b4752"),
+    "prefill_5120x17408_m512_five_level": ((8715.5 + 57939.8 + 30739.5) * 2.0 * 1024 + (17408.0 + 66720.0 + 5122.2) * 1024,
+                                           _LANES, "e5dd4cabcbebf53f"),
+    "down_proj_5120x17408_m1_student_t_packed": (23032.0 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "9c5848bbce659441"),
+    "gate_up_17408x5120_m1_student_t_packed": (22935.9 * 2.0 * 1024 + 40.0 * 1024, _ROWS, "9c5848bbce659441"),
+    "attn_proj_5120x5120_m1_student_t_packed": (7135.5 * 2.0 * 1024 + 16.0 * 1024, _ROWS, "9c5848bbce659441"),
+    "down_proj_5120x17408_m1_calibrated_packed": (33834.1 * 2.0 * 1024 + 40.0 * 1024, _DENSE, "1f7c6b74b169a3de"),
+    "down_proj_5120x17408_m1_five_level_calibrated_packed": (49695.3 * 2.0 * 1024 + 1328.6 * 1024, _DENSE5, "5b2d5307061aed1f"),
+    "gate_up_17408x5120_m4_student_t_packed": (28703.1 * 2.0 * 1024 + 160.0 * 1024, _TILES, "e4518543e34fde14"),
+    "gate_up_17408x5120_m16_student_t_packed": (26653.6 * 2.0 * 1024 + 640.0 * 1024, _TILES, "e4518543e34fde14"),
+    "attn_proj_5120x5120_m16_student_t_packed": (8657.2 * 2.0 * 1024 + 640.0 * 1024, _TILES, "e4518543e34fde14"),
+    "down_proj_5120x17408_m16_student_t_packed": (27677.9 * 2.0 * 1024 + 960.0 * 1024, _TILES, "e4518543e34fde14"),
+    "decode_5120x17408_calibrated": (37277.5 * 2.0 * 1024 + 174080.0 * 1024, _DENSE, "1f7c6b74b169a3de"),
+    "decode_5120x17408_five_level_calibrated": (49520.2 * 2.0 * 1024 + 174080.0 * 1024, _DENSE5, "5b2d5307061aed1f"),
     "prefill_5120x5120_m512_five_level_packed": (50297.9 * 2.0 * 1024 + 30720.0 * 1024,) + _OLD,
     # the three kernels of a step: k_prefill_xtile + k_prefill358 + k_prefill358_reduce
-    "prefill_5120x17408_m512_five_level_packed": ((8715.5 + 68467.8 + 30733.5) * 2.0 * 1024 + (17408.0 + 61606.2 + 5120.0) * 1024,
-                                                  _PREFILL, "7b413e1dcc6999fa"),
+    "prefill_5120x17408_m512_five_level_packed": ((8715.5 + 68458.8 + 30733.5) * 2.0 * 1024 + (17408.0 + 61606.2 + 5120.0) * 1024,
+                                                  _PREFILL, "f1cc2dd9dabb8793"),
     # k_decode358_rows<true> (x 2.0 / x 1.0 as above) + the operands and outputs of the library GEMM that
     # torch.cuda.tunable picked (bf16 weight, X, Y: its FETCH_SIZE, 158,001, is weighted for other request sizes than
     # our kernels' and fixes its reads only between 162 and 324 MB)
-    "prefill_5120x17408_m512_five_level_unfused": (23101.5 * 2.0 * 1024 + 179850.5 * 1024
+    "prefill_5120x17408_m512_five_level_unfused": (23095.2 * 2.0 * 1024 + 179839.1 * 1024
                                                    + 2.0 * (5120 * 17408 + 512 * 17408 + 512 * 5120),
-                                                   _DECODE_ROWS, "8c155b8acfa278a1"),
+                                                   _DECODE_ROWS, "e0bcc82ebf5cc40a"),
     "decode_5120x17408_student_t": (23268.0 * 2.0 * 1024 + 179524.0 * 1024,) + _OLD,
     "decode_gs_5120x17408_student_t": (33559.0 * 2.0 * 1024 + 174080.0 * 1024,) + _OLD,
     # all kernels of one encode step together (absmax, count, scan, borders, pack)
-    "encode_5120x17408_student_t": ((87063.5 + 87104.3 + 776.9 + 653.1 + 88991.4) * 2.0 * 1024
-                                    + (8.0 + 2322.2 + 1362.7 + 309.2 + 46629.7) * 1024, _ENCODE, "289d251e29fbd323"),
-    "encode_5120x17408_calibrated": ((87063.5 + 87104.1 + 776.9 + 653.1 + 89078.6) * 2.0 * 1024
-                                     + (8.0 + 2328.5 + 1362.7 + 600.0 + 68676.1) * 1024, _ENCODE, "289d251e29fbd323"),
+    "encode_5120x17408_student_t": ((87063.5 + 87104.3 + 776.9 + 653.2 + 88980.9) * 2.0 * 1024
+                                    + (8.0 + 2325.3 + 1362.7 + 309.2 + 46625.4) * 1024, _ENCODE, "8cc564571df8446d"),
+    "encode_5120x17408_calibrated": ((87063.5 + 87104.1 + 776.9 + 653.1 + 89068.9) * 2.0 * 1024
+                                     + (8.0 + 2324.3 + 1362.7 + 600.0 + 68682.4) * 1024, _ENCODE, "8cc564571df8446d"),
 }
 
 # Wave-level instruction counts per launch of the dominant kernel (SQ_INSTS_VALU, SQ_INSTS_SALU, SQ_INSTS_LDS from one
 # rocprofv3 --pmc run of this script, mean over the launches), gated by the hash of the kernel's sources like the
 # traffic figures.  Reported per weight: vector and LDS instructions x 64 lanes / weights, scalar instructions / weights.
 MEASURED_INSTRUCTIONS = {
-    "down_proj_5120x17408_m1_student_t": ((3414116.0, 2201438.0, 819680.0), _LANES, "58f0e28d2101b827"),
-    "down_proj_5120x17408_m1_calibrated": ((4829187.0, 3166052.0, 918004.0), _LANES, "58f0e28d2101b827"),
-    "down_proj_5120x17408_m1_five_level_calibrated": ((4829187.0, 3166052.0, 918004.0), _LANES, "58f0e28d2101b827"),
-    "down_proj_5120x17408_m1_student_t_packed": ((5734195.0, 4469166.0, 1360042.0), _ROWS, "1fdd69999d604da2"),
-    "gate_up_17408x5120_m1_student_t_packed": ((6030194.0, 4450915.0, 1414314.0), _ROWS, "1fdd69999d604da2"),
-    "attn_proj_5120x5120_m1_student_t_packed": ((3570752.0, 2281697.0, 593732.0), _ROWS, "1fdd69999d604da2"),
-    "down_proj_5120x17408_m1_level1_only_packed": ((4881551.0, 4104235.0, 1254926.0), _ROWS, "1fdd69999d604da2"),
+    "down_proj_5120x17408_m1_student_t": ((3414116.0, 2201438.0, 819680.0), _LANES, "e5dd4cabcbebf53f"),
+    "down_proj_5120x17408_m1_calibrated": ((4829187.0, 3166052.0, 918004.0), _LANES, "e5dd4cabcbebf53f"),
+    "down_proj_5120x17408_m1_five_level_calibrated": ((4829187.0, 3166052.0, 918004.0), _LANES, "e5dd4cabcbebf53f"),
+    "down_proj_5120x17408_m1_student_t_packed": ((5734195.0, 4469166.0, 1360042.0), _ROWS, "9c5848bbce659441"),
+    "gate_up_17408x5120_m1_student_t_packed": ((6030194.0, 4450915.0, 1414314.0), _ROWS, "9c5848bbce659441"),
+    "attn_proj_5120x5120_m1_student_t_packed": ((3570752.0, 2281697.0, 593732.0), _ROWS, "9c5848bbce659441"),
+    "down_proj_5120x17408_m1_level1_only_packed": ((4881551.0, 4104235.0, 1254926.0), _ROWS, "9c5848bbce659441"),
 }
 
 WORKLOADS = {
